@@ -148,7 +148,9 @@ def _gen(dev, seed):
 
 
 def _hybrid_tensors(cfg, mod, dev, seed):
-    """Checkpoint-named random weights in bfloat16, scaled like the designs' own random weights."""
+    """Checkpoint-named random weights in bfloat16, scaled like the designs' own random weights.  The keys of the recurrent
+    layers lean towards their queries: a sequence's first read-out, (k . q) v scaled to unit size, would otherwise be a
+    random sign times its value, which no two programs share."""
     g, out = _gen(dev, seed), {}
     for name, shape in mod.tensor_shapes(cfg).items():
         leaf = name.rsplit(".", 1)[-1]
@@ -160,6 +162,9 @@ def _hybrid_tensors(cfg, mod, dev, seed):
             t += 2.0 if name.endswith(("a2.b", "f.b")) else 0.0
         else:
             t = torch.randn(shape, generator=g, device=dev) * (0.5 if leaf == "conv" else shape[1] ** -0.5)
+            q = out.get(name[:-1] + "q")
+            if leaf == "k" and q.shape == t.shape:
+                t = 0.6 * q.float() + 0.8 * t
         out[name] = t.to(torch.bfloat16)
     return out
 
