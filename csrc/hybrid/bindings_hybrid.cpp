@@ -19,7 +19,7 @@ void launch_hy_layer_norm(const void*, bool, float*, const float*, void*, bool, 
 void launch_hy_rowdot(const void*, const void*, const float*, float*, int, int, int, bool, hipStream_t);
 void launch_hy_act(void*, int64_t, int, bool, hipStream_t);
 void launch_hy_mlstm_scan(const void*, int, const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*,
-                          float*, float*, float*, float*, float*, int, int, int, int, float, bool, hipStream_t);
+                          float*, float*, float*, int, int, int, int, int, float, int, bool, hipStream_t);
 void launch_hy_mlstm_out(const float*, const void*, int, int, const float*, void*, int, int, int, float, bool,
                          hipStream_t);
 void launch_hy_latent_prep(void*, int64_t, const void*, int64_t, const int32_t*, const int32_t*, const int32_t*, int,
@@ -77,7 +77,7 @@ void launch_hy_delta_prep(const void*, int, const float*, const float*, float*, 
                           float, bool, hipStream_t);
 bool launch_hy_linear_scan(const void*, int, int, int, int, const float*, const float*, float, const float*, bool, bool,
                            const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*, int, int, int, int,
-                           int, int, const float*, bool, hipStream_t);
+                           int, int, const float*, int, bool, hipStream_t);
 void launch_hy_moe_route_topk(const void*, const void*, const float*, float*, int32_t*, float*, int, int, int, int, bool,
                               hipStream_t);
 void launch_hy_moe_glu_grouped(const uint16_t*, const int32_t*, const float*, const uint16_t*, const uint16_t*, uint16_t*,
@@ -174,8 +174,12 @@ void hy_act(Tensor& x, int64_t kind) {
     chronos::launch_hy_act(x.data_ptr(), x.numel(), (int)kind, f32(x), stream());
 }
 
+// the most new tokens of any of B sequences with T in all (a launch-shape hint): max_q, or where the caller did not say
+// (0) what it is if the others bring one each
+static int longest(int64_t T, int64_t B, int64_t max_q) { return (int)(max_q > 0 ? max_q : T - B + 1); }
+
 Tensor hy_mlstm_scan(const Tensor& proj, const Tensor& gate_pre, const Tensor& q_start, const Tensor& pos0,
-                     const Tensor& slots, Tensor& S, Tensor& n, Tensor& m, int64_t H, int64_t D, int64_t Dv, double cap) {
+                     const Tensor& slots, Tensor& S, Tensor& n, Tensor& m, int64_t H, int64_t D, int64_t Dv, double cap, int64_t max_q) {
     c10::hip::HIPGuardMasqueradingAsCUDA g(proj.device());
     need(is_act(proj) && proj.dim() == 2 && proj.is_contiguous(), "mlstm_scan: proj [T, C]");
     need(proj.size(1) >= 2 * H * D + H * Dv, "mlstm_scan: proj narrower than q | k | v");
@@ -191,13 +195,11 @@ Tensor hy_mlstm_scan(const Tensor& proj, const Tensor& gate_pre, const Tensor& q
     need(m.dim() == 2 && m.size(0) == S.size(0) && m.size(1) == H, "mlstm_scan: m [NS, H]");
     need(D >= 1 && D <= 512 && H >= 1 && Dv >= 1, "mlstm_scan: 1 <= D <= 512");
     auto o = at::empty({T, H, Dv}, proj.options().dtype(at::kFloat));
-    auto scratch = at::empty({3, T, H}, proj.options().dtype(at::kFloat));
-    float* sp = scratch.data_ptr<float>();
+    auto scratch = at::empty({3 * T * H + B * H * D}, proj.options().dtype(at::kFloat));
     chronos::launch_hy_mlstm_scan(proj.data_ptr(), (int)proj.size(1), gate_pre.data_ptr<float>(),
                                   q_start.data_ptr<int32_t>(), pos0.data_ptr<int32_t>(), slots.data_ptr<int32_t>(),
-                                  S.data_ptr<float>(), n.data_ptr<float>(), m.data_ptr<float>(), sp, sp + T * H,
-                                  sp + 2 * T * H, o.data_ptr<float>(), (int)B, (int)H, (int)D, (int)Dv, (float)cap,
-                                  f32(proj), stream());
+                                  S.data_ptr<float>(), n.data_ptr<float>(), m.data_ptr<float>(), scratch.data_ptr<float>(),
+                                  o.data_ptr<float>(), (int)T, (int)B, (int)H, (int)D, (int)Dv, (float)cap, longest(T, B, max_q), f32(proj), stream());
     return o;
 }
 
@@ -714,7 +716,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> hy_delta_prep(const Tensor& y, const 
 Tensor hy_linear_scan(const Tensor& proj, int64_t q_off, int64_t k_off, int64_t v_off, const c10::optional<Tensor>& qscale,
                       const c10::optional<Tensor>& kscale, double q_mul, const Tensor& decay,
                       const c10::optional<Tensor>& beta, const Tensor& q_start, const Tensor& pos0, const Tensor& slots,
-                      Tensor& S, int64_t HK, int64_t H, int64_t D, int64_t Dv, const c10::optional<Tensor>& vscale) {
+                      Tensor& S, int64_t HK, int64_t H, int64_t D, int64_t Dv, const c10::optional<Tensor>& vscale, int64_t max_q) {
     c10::hip::HIPGuardMasqueradingAsCUDA g(proj.device());
     need(is_act(proj) && proj.dim() == 2 && proj.is_contiguous(), "linear_scan: proj [T, C]");
     const int64_t T = proj.size(0), C = proj.size(1), B = slots.numel();
@@ -739,7 +741,7 @@ Tensor hy_linear_scan(const Tensor& proj, int64_t q_off, int64_t k_off, int64_t 
         kscale ? kscale->data_ptr<float>() : nullptr, (float)q_mul, decay.data_ptr<float>(), chd, fixed,
         beta ? beta->data_ptr<float>() : nullptr, q_start.data_ptr<int32_t>(), pos0.data_ptr<int32_t>(),
         slots.data_ptr<int32_t>(), S.data_ptr<float>(), o.data_ptr<float>(), (int)T, (int)B, (int)HK, (int)H, (int)D, (int)Dv,
-        vscale ? vscale->data_ptr<float>() : nullptr, f32(proj), stream());
+        vscale ? vscale->data_ptr<float>() : nullptr, longest(T, B, max_q), f32(proj), stream());
     TORCH_CHECK(ok, "chronos hybrid op: linear_scan keeps a state column in registers, D <= 256 (got ", D, ")");
     return o;
 }
@@ -1027,7 +1029,7 @@ TORCH_LIBRARY_FRAGMENT(chronos, m) {
     m.def("hy_rowdot(Tensor h, Tensor w, Tensor? bias) -> Tensor");
     m.def("hy_act(Tensor(a!) x, int kind) -> ()");
     m.def("hy_mlstm_scan(Tensor proj, Tensor gate_pre, Tensor q_start, Tensor pos0, Tensor slots, Tensor(a!) S, "
-          "Tensor(b!) n, Tensor(c!) m, int H, int D, int Dv, float cap) -> Tensor");
+          "Tensor(b!) n, Tensor(c!) m, int H, int D, int Dv, float cap, int max_q=0) -> Tensor");
     m.def("hy_mlstm_out(Tensor o, Tensor proj, int g_off, Tensor w, float eps, bool out_f32) -> Tensor");
     m.def("hy_latent_prep(Tensor(a!) q, Tensor? dkv, Tensor pos, Tensor tok_seq, Tensor block_table, Tensor? w_norm, "
           "float eps, Tensor? cos_sin, int dims, int rank, Tensor(b!) cache, Tensor(c!)? qa=None, "
@@ -1072,7 +1074,7 @@ TORCH_LIBRARY_FRAGMENT(chronos, m) {
     m.def("hy_delta_prep(Tensor y, Tensor ab, Tensor a_log, int HK, int H, int D, float q_mul) -> (Tensor, Tensor, Tensor, Tensor)");
     m.def("hy_linear_scan(Tensor proj, int q_off, int k_off, int v_off, Tensor? qscale, Tensor? kscale, float q_mul, "
           "Tensor decay, Tensor? beta, Tensor q_start, Tensor pos0, Tensor slots, Tensor(a!) S, int HK, int H, int D, "
-          "int Dv, Tensor? vscale) -> Tensor");
+          "int Dv, Tensor? vscale, int max_q=0) -> Tensor");
     m.def("hy_moe_route_topk(Tensor h, Tensor w, Tensor bias, int top) -> (Tensor, Tensor)");
     m.def("hy_add_rms_norm(Tensor y, Tensor(a!) x, Tensor? w_out, float eps, bool out_f32, Tensor? y2, Tensor? gate2, "
           "Tensor? w_y, bool emit) -> Tensor");

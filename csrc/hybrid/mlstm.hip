@@ -8,7 +8,8 @@
 //   S_t = a_t S_{t-1} + b_t k_t v_t^T              n_t = a_t n_{t-1} + b_t k_t
 //   o_t = S_t^T q_t / (max(|n_t . q_t|, exp(-m_t)) + 1e-6),   q_t scaled by D^-1/2
 //
-// Three launches:
+// Token by token, in three launches (launches whose longest range has 16 tokens and more take chunk_scan.hip's form in
+// place of the first two):
 //   gate_scan    one wave per (sequence, head): the scalar recurrences a_t, b_t and the denominators (n lives in the
 //                wave's lanes); sequential in t but only O(D) work per token;
 //   state_scan   one workgroup per (sequence, head, 64 value columns): S in registers (lane = column, the D rows
@@ -402,11 +403,20 @@ static void mlstm_scan_t(const T* proj, int ldp, const float* gate_pre, const in
 #undef HY_SCAN
 }
 
-// D <= 512.  a, b, den: float [T, H] scratch.
+bool hy_chunk_scan_ok(const void*, int, int, int, int, int, int, int);
+void launch_hy_chunk_mlstm(const uint16_t*, int, const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*,
+                           float*, float*, float*, int, int, int, int, int, float, hipStream_t);
+
+// D <= 512.  scratch: 3 T H + B H D floats.  longest: the most tokens that any sequence brings (or an upper bound of it).
 void launch_hy_mlstm_scan(const void* proj, int ldp, const float* gate_pre, const int32_t* q_start, const int32_t* pos0,
-                          const int32_t* slots, float* S, float* n, float* m, float* a, float* b, float* den, float* o,
-                          int B, int H, int D, int Dv, float cap, bool f32, hipStream_t s) {
+                          const int32_t* slots, float* S, float* n, float* m, float* scratch, float* o, int T, int B, int H, int D,
+                          int Dv, float cap, int longest, bool f32, hipStream_t s) {
     if (B == 0) return;
+    if (!f32 && hy_chunk_scan_ok(proj, ldp, 0, H * D, 2 * H * D, D, Dv, longest)) {
+        launch_hy_chunk_mlstm((const uint16_t*)proj, ldp, gate_pre, q_start, pos0, slots, S, n, m, scratch, o, T, B, H, D, Dv, cap, s);
+        return;
+    }
+    float *a = scratch, *b = a + (int64_t)T * H, *den = b + (int64_t)T * H;
     if (f32) mlstm_scan_t<float>((const float*)proj, ldp, gate_pre, q_start, pos0, slots, S, n, m, a, b, den, o, B, H, D, Dv, cap, s);
     else mlstm_scan_t<uint16_t>((const uint16_t*)proj, ldp, gate_pre, q_start, pos0, slots, S, n, m, a, b, den, o, B, H, D, Dv, cap, s);
 }

@@ -942,7 +942,7 @@ def mix_retention(model, li, spec: RetentionSpec, w: dict, h, meta: StepMeta, ca
     proj = hops.matmul(h, w["w_proj"])          # q | k | v | g
     hops.rotate_qk(proj, 0, H * D, H, H, D, spec.rope_dims, model.rope.get(li), meta.pos, 1.0, D ** -0.5)
     o = hops.linear_scan(proj, 0, H * D, 2 * H * D, None, None, 1.0, w["decay"], None, meta.q_start, meta.pos0,
-                         meta.slots, cache.S[li], H, H, D, Dv)
+                         meta.slots, cache.S[li], H, H, D, Dv, max_q=meta.max_q)
     return hops.matmul(hops.head_norm_gate(o, proj, 2 * H * D + H * Dv, w["ones"], model.cfg.norm_eps, True,
                                            model.act_dtype), w["w_o"])
 
@@ -972,7 +972,7 @@ def mix_mamba2(model, li: int, spec: Mamba2Spec, w: dict, h, meta: StepMeta, cac
     decay, dt = hops.ssm_prep(dt_pre, w["a_log"])
     # state rows = B, read by C, written with dt x: S <- decay S + B (dt x)^T, o = S^T C
     o = hops.linear_scan(xbc, inner + GN, inner, 0, None, None, 1.0, decay, None, meta.q_start, meta.pos0, meta.slots,
-                         cache.S[li], G, H, N, P, dt)
+                         cache.S[li], G, H, N, P, dt, meta.max_q)
     y = hops.gated_group_norm(o, xbc, 0, w["skip"], proj, 0, w["norm"], spec.norm_groups, model.cfg.norm_eps,
                               model.act_dtype)
     return hops.matmul(y, w["w_o"])
@@ -997,7 +997,7 @@ def mix_delta_rule(model, li: int, spec: DeltaRuleSpec, w: dict, h, meta: StepMe
     y = hops.short_conv(proj, w["taps"], meta.tok_seq, meta.q_start, meta.pos0, meta.slots, cache.hist[li], True)
     qscale, kscale, decay, beta = hops.delta_prep(y, ab, w["a_log"], HK, H, D, D ** -0.5)
     o = hops.linear_scan(y, 0, HK * D, 2 * HK * D, qscale, kscale, 1.0, decay, beta, meta.q_start, meta.pos0,
-                         meta.slots, cache.S[li], HK, H, D, Dv)
+                         meta.slots, cache.S[li], HK, H, D, Dv, max_q=meta.max_q)
     return hops.matmul(hops.head_norm_gate(o, proj, C, w["norm"], model.cfg.norm_eps, True, model.act_dtype), w["w_o"])
 
 
@@ -1007,7 +1007,7 @@ def mix_gla(model, li: int, spec: GLASpec, w: dict, h, meta: StepMeta, cache: Hy
     z = torch.addmm(w["b_a2"], hops.rowdot(h, w["w_a1"]), w["w_a2t"])  # float32 decay logits [T, H D]
     decay = hops.decay_pow(z, 1.0 / spec.tau)
     o = hops.linear_scan(proj, 0, H * D, 2 * H * D, None, None, D ** -0.5, decay, None, meta.q_start, meta.pos0,
-                         meta.slots, cache.S[li], H, H, D, Dv)
+                         meta.slots, cache.S[li], H, H, D, Dv, max_q=meta.max_q)
     o = hops.head_norm_gate(o, proj, 2 * H * D + H * Dv, w["norm"], model.cfg.norm_eps, True, model.act_dtype)
     return _with_gate(hops.matmul(o, w["w_o"]), proj, w)
 

@@ -1,0 +1,101 @@
+"""The chunked forms of the linear-state recurrences (csrc/hybrid/chunk_scan.hip) against the token-by-token recurrence in
+float64, at the edges of a chunk (64 tokens) and of its 16-token tiles, with ranges that continue a state, with decays of 0
+and 1, and with column counts off the 64-column slabs.
+
+Tolerance: inputs are exact in both (bfloat16 and float32); what differs is float32 rounding, 2^-24 per operation, of
+sums over at most 129 tokens and 256 state rows and of one exponential per token.  Errors of independent roundings grow with the
+square root of their number: sqrt(129 * 256) * 2^-24 = 1.1e-5 at the very worst alignment of the result's cancellation,
+2e-6 over a whole result's norm."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+LENS, STARTS, SLOTS = [1, 64, 129, 0, 17, 63, 65, 16], [0, 5, 0, 3, 9, 0, 2, 7], [2, 0, 4, 1, 3, 7, 5, 8]
+
+
+def _setup(seed, T, C, H, D, Dv):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
+    qs = [0]
+    for n in LENS:
+        qs.append(qs[-1] + n)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    return g, rnd, qs, (i32(qs), i32(STARTS), i32(SLOTS))
+
+
+def _rel(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+@pytest.mark.parametrize("HK,H,D,Dv,form", [(2, 4, 32, 40, "token"), (1, 2, 64, 64, "token"), (2, 2, 128, 72, "head"),
+                                            (1, 3, 256, 128, "token"), (4, 4, 128, 128, "head")])
+def test_plain(HK, H, D, Dv, form):
+    from chronos.ops import hybrid as hops
+
+    T = sum(LENS)
+    C = 2 * HK * D + H * Dv + 16
+    g, rnd, qs, ranges = _setup(H * D + Dv, T, C, H, D, Dv)
+    proj = rnd(T, C).bfloat16()
+    if form == "head":
+        decay, vs = 1 - torch.rand(H, device=DEV, generator=g) ** 4, None
+        decay[0] = 1.0
+    else:
+        decay, vs = torch.exp(-2 * torch.rand(T, H, device=DEV, generator=g)), torch.rand(T, H, device=DEV, generator=g)
+        decay[3::50], decay[9::31], decay[11::37] = 0.0, 1e-30, 1.0
+    qsc, ksc = torch.rand(T, HK, device=DEV, generator=g), torch.rand(T, HK, device=DEV, generator=g)
+    S = rnd(9, H, D, Dv) * 0.3
+    S0 = S.clone()
+    o = hops.linear_scan(proj, 8, 8 + HK * D, 8 + 2 * HK * D, qsc, ksc, 1.0, decay, None, *ranges, S, HK, H, D, Dv, vs)
+    p = proj.double()
+    q = (p[:, 8:8 + HK * D].view(T, HK, D) * qsc.double()[..., None]).repeat_interleave(H // HK, 1)
+    k = (p[:, 8 + HK * D:8 + 2 * HK * D].view(T, HK, D) * ksc.double()[..., None]).repeat_interleave(H // HK, 1)
+    v = p[:, 8 + 2 * HK * D:8 + 2 * HK * D + H * Dv].view(T, H, Dv) * (vs.double()[..., None] if vs is not None else 1.0)
+    dec = decay.double().expand(T, H)
+    want, Sw = torch.empty(T, H, Dv, dtype=torch.double, device=DEV), S0.double()
+    for b, n in enumerate(LENS):
+        s = torch.zeros(H, D, Dv, dtype=torch.double, device=DEV) if STARTS[b] == 0 else Sw[SLOTS[b]]
+        for t in range(qs[b], qs[b] + n):
+            s = dec[t][:, None, None] * s + k[t][:, :, None] * v[t][:, None]
+            want[t] = (q[t][:, None] @ s)[:, 0]
+        if n:
+            Sw[SLOTS[b]] = s
+    assert _rel(o, want) < 2e-6 and _rel(S, Sw) < 2e-6
+    assert torch.equal(S[1], S0[1]) and torch.equal(S[6], S0[6]), "slots without tokens must stay untouched"
+
+
+@pytest.mark.parametrize("H,D,Dv,gate", [(2, 32, 24, 1.0), (1, 64, 128, 6.0), (3, 128, 72, 1.0), (2, 256, 64, 4.0)])
+def test_mlstm(H, D, Dv, gate):
+    from chronos.ops import hybrid as hops
+
+    T, cap = sum(LENS), 9.0
+    C = 2 * H * D + 2 * H * Dv
+    g, rnd, qs, ranges = _setup(H * D + Dv, T, C, H, D, Dv)
+    proj, gp = rnd(T, C).bfloat16(), rnd(T, 2 * H) * gate
+    gp[:, H:] += 2.0
+    S, n, m = rnd(9, H, D, Dv) * 0.3, rnd(9, H, D) * 0.5, rnd(9, H)
+    S0, n0, m0 = S.clone(), n.clone(), m.clone()
+    o = hops.mlstm_scan(proj, gp, *ranges, S, n, m, H, D, Dv, cap, max(LENS))
+    p, gd = proj.double(), gp.double()
+    ig = cap * torch.tanh(gd[:, :H] / cap)
+    fg = torch.nn.functional.logsigmoid(cap * torch.tanh(gd[:, H:] / cap))
+    num, den = torch.empty(T, H, Dv, dtype=torch.double, device=DEV), torch.empty(T, H, dtype=torch.double, device=DEV)
+    Sw, nw, mw = S0.double(), n0.double(), m0.double()
+    for b, cnt in enumerate(LENS):
+        s, nn, mm = (Sw[SLOTS[b]], nw[SLOTS[b]], mw[SLOTS[b]]) if STARTS[b] else (Sw[0] * 0, nw[0] * 0, mw[0] * 0)
+        for t in range(qs[b], qs[b] + cnt):
+            q, k = p[t, :H * D].view(H, D) * D ** -0.5, p[t, H * D:2 * H * D].view(H, D)
+            v = p[t, 2 * H * D:2 * H * D + H * Dv].view(H, Dv)
+            mn = torch.maximum(fg[t] + mm, ig[t])
+            a, w, mm = torch.exp(fg[t] + mm - mn), torch.exp(ig[t] - mn), mn
+            s = a[:, None, None] * s + (w[:, None] * k)[:, :, None] * v[:, None]
+            nn = a[:, None] * nn + w[:, None] * k
+            num[t] = (q[:, None] @ s)[:, 0]
+            den[t] = torch.maximum((nn * q).sum(-1).abs(), torch.exp(-mm)) + 1e-6
+        if cnt:
+            Sw[SLOTS[b]], nw[SLOTS[b]], mw[SLOTS[b]] = s, nn, mm
+    # a denominator that nearly cancels magnifies its own rounding: compare the read-out before the division
+    assert _rel(o * den[..., None].float(), num) < 1e-5
+    assert _rel(S, Sw) < 2e-6 and _rel(n, nw) < 2e-6 and _rel(m, mw) < 1e-6
+    for t, t0 in ((S, S0), (n, n0), (m, m0)):
+        assert torch.equal(t[1], t0[1]) and torch.equal(t[6], t0[6]), "slots without tokens must stay untouched"
