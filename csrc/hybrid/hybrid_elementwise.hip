@@ -126,6 +126,87 @@ __global__ void __launch_bounds__(256) rowdot_kernel(const T* __restrict__ h, co
     }
 }
 
+// The same on the matrix cores, for bfloat16 rows of whole 64-element steps (products of bfloat16 pairs are exact in
+// float32, and so are their sums' roundings: the precision of the kernel above).  A workgroup takes 16 TT tokens and 16 NT
+// output rows and splits d over its NWV waves, 64 elements at a time, straight from memory into operands; the waves' sums
+// meet in LDS.  Bound by reading h once (26 us for 8192 x 4096 by 64 rows, 2.6 TB/s; the kernel above reads every token's row
+// from LDS once per output row: 268 us).  Errors against float64 are the same: chains of four matrix products.
+template <int TT, int NT, int NWV>
+__global__ void __launch_bounds__(64 * NWV) rowdot_mfma_kernel(const uint16_t* __restrict__ h, const uint16_t* __restrict__ w,
+                                                               const float* __restrict__ bias, float* __restrict__ out, int rows,
+                                                               int d, int n) {
+    __shared__ f32x4 red[NWV][TT * NT][64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, ln = lane & 15, g = lane >> 4;
+    const int64_t t0 = (int64_t)blockIdx.x * 16 * TT;
+    const int n0 = blockIdx.y * 16 * NT;
+    const uint16_t *hp[TT], *wp[NT];   // rows past the end repeat the last one and are not stored
+#pragma unroll
+    for (int i = 0; i < TT; ++i) hp[i] = h + min(t0 + 16 * i + ln, (int64_t)rows - 1) * d + 8 * g;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) wp[j] = w + (int64_t)min(n0 + 16 * j + ln, n - 1) * d + 8 * g;
+    f32x4 sum[TT][NT];
+#pragma unroll
+    for (int i = 0; i < TT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int P = TT * NT == 1 ? 4 : 2;   // 64-element steps in flight
+    for (int k0 = wv * 64; k0 < d; k0 += P * NWV * 64) {
+        bf16x8 a[2 * P][TT], b[2 * P][NT];
+#pragma unroll
+        for (int u = 0; u < 2 * P; ++u) {
+            const int k = k0 + (u >> 1) * NWV * 64 + (u & 1) * 32;
+            if (k < d) {
+#pragma unroll
+                for (int i = 0; i < TT; ++i) a[u][i] = *reinterpret_cast<const bf16x8*>(hp[i] + k);
+#pragma unroll
+                for (int j = 0; j < NT; ++j) b[u][j] = *reinterpret_cast<const bf16x8*>(wp[j] + k);
+            } else {
+#pragma unroll
+                for (int i = 0; i < TT; ++i) a[u][i] = bf16x8{};
+#pragma unroll
+                for (int j = 0; j < NT; ++j) b[u][j] = bf16x8{};
+            }
+        }
+        // chains of four products at most, added up apart: the longer a chain, the more roundings at the size of its sum
+#pragma unroll
+        for (int i = 0; i < TT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                f32x4 acc[P / 2];
+#pragma unroll
+                for (int q = 0; q < P / 2; ++q) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int u = 0; u < 2 * P; ++u) acc[u / 4] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][i], b[u][j], acc[u / 4], 0, 0, 0);
+#pragma unroll
+                for (int q = 1; q < P / 2; ++q) acc[0] += acc[q];
+                sum[i][j] += acc[0];
+            }
+    }
+#pragma unroll
+    for (int i = 0; i < TT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) red[wv][i * NT + j][lane] = sum[i][j];
+    __syncthreads();
+    for (int p = wv; p < TT * NT; p += NWV) {   // element r of a tile: token 4 g + r, output row ln
+        f32x4 part[NWV];
+#pragma unroll
+        for (int u = 0; u < NWV; ++u) part[u] = red[u][p][lane];
+#pragma unroll
+        for (int o = NWV / 2; o > 0; o >>= 1)
+#pragma unroll
+            for (int u = 0; u < o; ++u) part[u] += part[u + o];
+        const f32x4 v = part[0];
+        const int r = n0 + 16 * (p % NT) + ln;
+        const int64_t t = t0 + 16 * (p / NT) + 4 * g;
+        if (r < n) {
+            const float bv = bias != nullptr ? bias[r] : 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (t + e < rows) out[(t + e) * n + r] = v[e] + bv;
+        }
+    }
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256) act_kernel(T* __restrict__ x, int64_t n, int kind) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -181,9 +262,30 @@ static void rowdot_t(const T* h, const T* w, const float* bias, float* out, int 
 #undef HY_RD
 }
 
+// Few tokens: 16 output rows per workgroup and d over 16 waves, so that a decode row's chain is short and its workgroups are
+// many; more: up to 64 output rows, and two tiles of tokens where that leaves a workgroup per CU, to read w less often.
+template <int TT, int NT, int NWV>
+static void rowdot_mfma(const uint16_t* h, const uint16_t* w, const float* bias, float* out, int rows, int d, int n, hipStream_t s) {
+    const dim3 grid((rows + 16 * TT - 1) / (16 * TT), (n + 16 * NT - 1) / (16 * NT));
+    hy::rowdot_mfma_kernel<TT, NT, NWV><<<grid, 64 * NWV, 0, s>>>(h, w, bias, out, rows, d, n);
+}
+
 void launch_hy_rowdot(const void* h, const void* w, const float* bias, float* out, int T, int d, int n, bool f32,
                       hipStream_t s) {
     if (T == 0 || n == 0) return;
+    // (us, vector ALUs / matrix cores: 16 tokens of 1024 by 8 rows 5.1 / 3.5, of 2048 by 200 rows 7.5 / 5.7, of 4096 by 64 rows
+    // 6.8 / 9.0; 200 tokens of 4096 by 64 rows 8.2 / 9.2; 1 token of it 9.8 / 6.1, 1024 tokens 28 / 20, 8192 tokens 268 / 26:
+    // a workgroup's 16 tokens share one CU's loads, which a few tokens of long rows would rather spread)
+    const bool spread = d > 2048 && T >= 2 && T <= 256;
+    if (!f32 && d % 64 == 0 && !spread && (((uintptr_t)h | (uintptr_t)w) & 15) == 0) {
+        const uint16_t *hb = (const uint16_t*)h, *wb = (const uint16_t*)w;
+        if (T <= 512) rowdot_mfma<1, 1, 16>(hb, wb, bias, out, T, d, n, s);
+        else if (n <= 16) rowdot_mfma<1, 1, 8>(hb, wb, bias, out, T, d, n, s);
+        else if (n <= 32) rowdot_mfma<1, 2, 8>(hb, wb, bias, out, T, d, n, s);
+        else if (T < 4096) rowdot_mfma<1, 4, 8>(hb, wb, bias, out, T, d, n, s);
+        else rowdot_mfma<2, 4, 8>(hb, wb, bias, out, T, d, n, s);
+        return;
+    }
     if (f32) rowdot_t<float>((const float*)h, (const float*)w, bias, out, T, d, n, s);
     else rowdot_t<uint16_t>((const uint16_t*)h, (const uint16_t*)w, bias, out, T, d, n, s);
 }

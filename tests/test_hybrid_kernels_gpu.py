@@ -235,3 +235,18 @@ def test_latent_attention_long_context_few_rows(dt, H, R, rank):
     o = hops.latent_attention(qa, cache, wide, q_start, pos, gate, 0.2, rank, dt, max(lens))
     o2 = ref.latent_attention(qa, cache, wide, q_start, pos, gate, 0.2, rank, dt)
     _close(o, o2, _tol(dt, 2e-5, 1e-2))
+
+
+@pytest.mark.parametrize("T", [1, 2, 15, 16, 17, 257, 513, 2049, 4097])
+@pytest.mark.parametrize("d,n", [(64, 1), (128, 16), (192, 17), (1088, 33), (2048, 200), (4160, 64)])
+def test_rowdot_at_tile_edges(T, d, n):
+    """Rows, output rows and 64-element steps at and off the matrix-core tiles, against float64.  A float32 sum of d products
+    rounds d times at most: sqrt(d) 2^-24 of the sum of their sizes, in norm well below 1e-6 of the result's."""
+    from chronos.ops import hybrid as hops
+
+    g = _gen(T + d + n)
+    h, w, b = _rand(g, T, d, dtype=torch.bfloat16), _rand(g, n, d, dtype=torch.bfloat16), _rand(g, n)
+    want = h.double() @ w.double().t() + b.double()
+    assert float((hops.rowdot(h, w, b).double() - want).norm() / want.norm()) < 1e-6
+    want -= b.double()
+    assert float((hops.rowdot(h, w).double() - want).norm() / want.norm()) < 1e-6
