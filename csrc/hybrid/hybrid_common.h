@@ -25,6 +25,40 @@ __device__ __forceinline__ float sigmoidf_(float z) { return 1.f / (1.f + expf(-
 // log(sigmoid(z)) without overflow on either side
 __device__ __forceinline__ float logsigmoidf_(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }
 
+// The same for values that end up in activation type T: for bfloat16 through the hardware's exponential and reciprocal (one
+// or two units of float32's last place, 2^-15 of bfloat16's)
+template <typename T> __device__ __forceinline__ float sigmoid_act(float z) {
+    if constexpr (sizeof(T) == 4) return sigmoidf_(z);
+    else return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.44269504088896340736f * z));
+}
+
+// 8 neighbouring activations, 16-byte aligned for bfloat16
+__device__ __forceinline__ void ld8(const uint16_t* p, float (&v)[8]) {
+    const uint4 r = *reinterpret_cast<const uint4*>(p);
+    const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        v[2 * i] = __uint_as_float(w[i] << 16);
+        v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    }
+}
+__device__ __forceinline__ void st8(uint16_t* p, const float (&v)[8]) {
+    u16x8 o;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[i] = f2bf(v[i]);
+    *reinterpret_cast<u16x8*>(p) = o;
+}
+// 8 neighbouring floats, 16-byte aligned
+__device__ __forceinline__ void ld8f(const float* p, float (&v)[8]) {
+    const f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { v[i] = a[i]; v[4 + i] = b[i]; }
+}
+__device__ __forceinline__ void st8f(float* p, const float (&v)[8]) {
+    *reinterpret_cast<f32x4*>(p) = f32x4{v[0], v[1], v[2], v[3]};
+    *reinterpret_cast<f32x4*>(p + 4) = f32x4{v[4], v[5], v[6], v[7]};
+}
+
 // Transposing LDS read (gfx950): the 16 lanes of a lane group name the 8-byte pieces of a 4 x 16 matrix of 16-bit
 // elements, row by row (lane l: row l / 4, columns 4 (l % 4) ..), and lane l receives column l, its 4 rows in order.
 // Rows may lie anywhere.  A row-major tile thus serves as either operand of a matrix product.
@@ -66,6 +100,9 @@ __device__ __forceinline__ float act_apply(float z, int kind) {
     }
     return 0.5f * z * (1.f + erff(z * 0.70710678118654752440f));
 }
+
+// host: every pointer (nullptr too) on a 16-byte boundary
+template <typename... P> inline bool aligned16(P... p) { return ((reinterpret_cast<uintptr_t>(p) | ...) & 15) == 0; }
 
 }  // namespace hy
 }  // namespace chronos

@@ -106,12 +106,12 @@ __global__ void __launch_bounds__(256) glu_kernel(const T* __restrict__ gu, int6
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const float a = fminf(gv[k], limit), u = fminf(fmaxf(uv[k], -limit), limit);
-            o[k] = a * sigmoidf_(slope * a) * (u + shift);
+            o[k] = a * sigmoid_act<T>(slope * a) * (u + shift);
         }
         st4<T>(y + r * ldy + c, o);
     } else {
         const float a = fminf(ld<T>(g), limit), u = fminf(fmaxf(ld<T>(g + F), -limit), limit);
-        st<T>(y + r * ldy + c, a * sigmoidf_(slope * a) * (u + shift));
+        st<T>(y + r * ldy + c, a * sigmoid_act<T>(slope * a) * (u + shift));
     }
 }
 

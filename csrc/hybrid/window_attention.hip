@@ -114,6 +114,98 @@ __global__ void __launch_bounds__(256) window_prep_kernel(
     }
 }
 
+// The same for bfloat16 heads of 8 LPH columns (LPH lanes per head, 8 columns each) and rotations in steps of 8 pairs: a
+// column's partner in the rotation sits half / 8 lanes away.  One workgroup per token; lanes past the query and key heads
+// take 8 columns of values.  Every column moves once, 16 bytes at a time: 8192 tokens of 32 + 8 + 8 heads of 128 in 58 us,
+// 219 us column by column through LDS.
+__global__ void __launch_bounds__(256) window_prep_vec_kernel(
+        uint16_t* __restrict__ qkv, int ldq, int H, int G, int LPH, int Dv, const uint16_t* __restrict__ v_first,
+        const float* __restrict__ lam, const int32_t* __restrict__ pos, const int32_t* __restrict__ tok_seq,
+        const int32_t* __restrict__ block_table, int max_blocks, const float* __restrict__ q_norm,
+        const float* __restrict__ k_norm, float eps, const float* __restrict__ cos_sin, int dims, uint16_t* __restrict__ kc,
+        uint16_t* __restrict__ vc, int BS, uint16_t* __restrict__ v_out, int v_off, const float* __restrict__ v_cos_sin,
+        const float* __restrict__ q_temp) {
+    const int64_t t = blockIdx.x;
+    const int lane = threadIdx.x & 63, D = 8 * LPH;
+    const int p = pos[t];
+    const int64_t slot = (int64_t)block_table[(int64_t)tok_seq[t] * max_blocks + p / BS] * BS + p % BS;
+    uint16_t* const base = qkv + t * ldq;
+    const int nqk = (H + G) * LPH, nv = G * Dv / (v_cos_sin != nullptr ? 16 : 8);
+    for (int it = threadIdx.x; it < nqk + nv; it += 256) {
+        if (it < nqk) {
+            const int j = it / LPH, cl = it % LPH, c = cl * 8;   // head, lane of the head
+            const bool isq = j < H;
+            const float* nw = isq ? q_norm : k_norm;
+            if (nw == nullptr && dims == 0 && isq && q_temp == nullptr) continue;   // plain queries stay as they are
+            float v[8];
+            ld8(base + (int64_t)j * D + c, v);
+            if (nw != nullptr) {
+                float ss = 0.f, wf[8];
+                ld8f(nw + c, wf);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+                for (int k = 1; k < LPH; k <<= 1) ss += __shfl_xor(ss, k, 64);
+                const float inv = 1.f / sqrtf(ss / (float)D + eps);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = v[e] * inv * wf[e];
+            }
+            if (dims != 0) {
+                const int half = dims / 2, hl = half / 8;
+                const bool lo = cl < hl, hi = !lo && cl < 2 * hl;
+                float o[8], cs[8], sn[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[e] = __shfl(v[e], lo ? lane + hl : hi ? lane - hl : lane, 64);
+                if (lo || hi) {
+                    const float* tab = cos_sin + (int64_t)p * dims + (lo ? c : c - half);
+                    ld8f(tab, cs);
+                    ld8f(tab + half, sn);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[e] = lo ? v[e] * cs[e] - o[e] * sn[e] : v[e] * cs[e] + o[e] * sn[e];
+                }
+            }
+            if (isq && q_temp != nullptr) {
+                const float f = q_temp[p];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] *= f;
+            }
+            st8(isq ? base + (int64_t)j * D + c : kc + (slot * G + (j - H)) * D + c, v);
+            continue;
+        }
+        const float l = v_first != nullptr ? lam[0] : 0.f;
+        auto value = [&](int i, float (&v)[8]) {   // columns i .. i + 7; the value as projected goes to v_out
+            const uint16_t* src = base + v_off + i;
+            ld8(src, v);
+            if (v_out != nullptr) *reinterpret_cast<uint4*>(v_out + t * G * Dv + i) = *reinterpret_cast<const uint4*>(src);
+            if (v_first != nullptr) {
+                float f[8];
+                ld8(v_first + t * G * Dv + i, f);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = (1.f - l) * v[e] + l * f[e];
+            }
+        };
+        float u[8];
+        if (v_cos_sin == nullptr) {
+            const int i = (it - nqk) * 8;
+            value(i, u);
+            st8(vc + slot * G * Dv + i, u);
+        } else {   // columns m and m + Dv / 2 of a head turn by p * f_m
+            const int vh = Dv / 2, i = (it - nqk) * 8, m = i % vh, a = i / vh * Dv + m;
+            float w[8], cs[8], sn[8], x[8], y[8];
+            value(a, u);
+            value(a + vh, w);
+            ld8f(v_cos_sin + (int64_t)p * Dv + m, cs);
+            ld8f(v_cos_sin + (int64_t)p * Dv + vh + m, sn);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                x[e] = u[e] * cs[e] - w[e] * sn[e];
+                y[e] = w[e] * cs[e] + u[e] * sn[e];
+            }
+            st8(vc + slot * G * Dv + a, x);
+            st8(vc + slot * G * Dv + a + vh, y);
+        }
+    }
+}
+
 // grid (blocks per sequence at most, B): workgroup = one block of `pool` positions that the step completes.
 template <typename T>
 __global__ void __launch_bounds__(256) pool_blocks_kernel(const T* __restrict__ kc, const T* __restrict__ vc,
@@ -374,6 +466,14 @@ void launch_hy_window_prep(void* qkv, int ld, int H, int G, int D, int Dv, const
     if (T == 0) return;
     const int bytes = 4 * D * 4;
     if (v_off < 0) v_off = (H + G) * D;
+    // (values in front of column H D would be read while the queries there are rewritten, in another order than the general kernel's)
+    const int lph = D / 8;
+    if (!f32 && ks == nullptr && D % 8 == 0 && (lph & (lph - 1)) == 0 && lph <= 64 && dims % 16 == 0 && Dv % 8 == 0 &&
+        (v_cos_sin == nullptr || Dv % 16 == 0) && v_off >= H * D && ((ld | v_off) & 7) == 0 &&
+        hy::aligned16(qkv, v_first, q_norm, k_norm, cos_sin, kc, vc, v_out, v_cos_sin)) {
+        hy::window_prep_vec_kernel<<<T, 256, 0, s>>>((uint16_t*)qkv, ld, H, G, lph, Dv, (const uint16_t*)v_first, lam, pos, tok_seq, block_table, max_blocks, q_norm, k_norm, eps, cos_sin, dims, (uint16_t*)kc, (uint16_t*)vc, BS, (uint16_t*)v_out, v_off, v_cos_sin, q_temp);
+        return;
+    }
     if (f32) hy::window_prep_kernel<float><<<T, 256, bytes, s>>>((float*)qkv, ld, H, G, D, Dv, (const float*)v_first, lam, pos, tok_seq, block_table, max_blocks, q_norm, k_norm, eps, cos_sin, dims, (float*)kc, (float*)vc, BS, (float*)v_out, v_off, v_cos_sin, q_temp, ks);
     else hy::window_prep_kernel<uint16_t><<<T, 256, bytes, s>>>((uint16_t*)qkv, ld, H, G, D, Dv, (const uint16_t*)v_first, lam, pos, tok_seq, block_table, max_blocks, q_norm, k_norm, eps, cos_sin, dims, (uint16_t*)kc, (uint16_t*)vc, BS, (uint16_t*)v_out, v_off, v_cos_sin, q_temp, ks);
 }

@@ -1,0 +1,117 @@
+"""The 16-bytes-per-lane forms of the row kernels (csrc/hybrid) at the sizes where they start, end and fall back, against the
+PyTorch references.  Outputs are bfloat16 (2^-8 of the value between neighbours; the largest value's rounding plus that of a
+float32 sum in another order: 1.2e-2 of the largest magnitude at most, as in the other kernel tests) or float32 (2e-5)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+BF = torch.bfloat16
+
+
+def _g(seed):
+    return torch.Generator(device=DEV).manual_seed(seed)
+
+
+def _rand(g, *shape, dtype=torch.float32, scale=1.0):
+    return (torch.randn(*shape, device=DEV, generator=g) * scale).to(dtype)
+
+
+def _close(a, b, tol):
+    a, b = a.float(), b.float()
+    assert float((a - b).abs().max()) <= tol * (float(b.abs().max()) + 1e-6)
+
+
+def _i32(v):
+    return torch.tensor(v, dtype=torch.int32, device=DEV)
+
+
+@pytest.mark.parametrize("rows", [1, 5, 64])
+@pytest.mark.parametrize("d", [8, 520, 1024, 1032, 2048, 2056, 4096, 8192, 8200, 100])
+def test_add_layer_norm(rows, d):
+    from chronos.ops import hybrid as hops, hybrid_ref as ref
+
+    g = _g(rows + d)
+    y, x, w = _rand(g, rows, d, dtype=BF, scale=3.0), _rand(g, rows, d), _rand(g, d)
+    x2 = x.clone()
+    h, h2 = hops.add_layer_norm(y, x, w, 1e-5, BF), ref.add_layer_norm(y, x2, w, 1e-5, BF)
+    _close(x, x2, 2e-5)
+    _close(h, h2, 1.2e-2)
+
+
+@pytest.mark.parametrize("n", [8, 2048, 2056, 4100, 7])
+@pytest.mark.parametrize("kind", [0, 1])
+def test_act(n, kind):
+    from chronos.ops import hybrid as hops, hybrid_ref as ref
+
+    x = _rand(_g(n), 3, n, dtype=BF, scale=3.0)
+    x[0, 0], x[-1, -1] = 50.0, -50.0
+    _close(hops.act_inplace(x.clone(), kind), ref.act_inplace(x.clone(), kind), 1.2e-2)
+
+
+@pytest.mark.parametrize("H,Dv,off", [(3, 32, 8), (2, 64, 0), (5, 128, 16), (2, 256, 8), (1, 512, 8), (2, 96, 8), (3, 128, 3)])
+@pytest.mark.parametrize("silu", [True, False])
+def test_head_norm_gate(H, Dv, off, silu):
+    from chronos.ops import hybrid as hops, hybrid_ref as ref
+
+    g = _g(H * Dv + off)
+    o, src, w = _rand(g, 13, H, Dv), _rand(g, 13, off + H * Dv + 8, dtype=BF, scale=4.0), _rand(g, H * Dv)
+    src[0, off], src[1, off] = 200.0, -200.0
+    _close(hops.head_norm_gate(o, src, off, w, 1e-6, silu, BF), ref.head_norm_gate(o, src, off, w, 1e-6, silu, BF), 1.2e-2)
+
+
+@pytest.mark.parametrize("C,K,off", [(8, 2, 0), (264, 3, 8), (2056, 4, 16), (4096, 4, 8), (64, 5, 8), (64, 4, 4)])
+@pytest.mark.parametrize("many", [False, True])
+def test_short_conv(C, K, off, many):
+    """``many``: enough tokens for eight per thread; ranges start and end inside and on the edges of those blocks."""
+    from chronos.ops import hybrid as hops, hybrid_ref as ref
+
+    lens = [2, 1, 8, 0, 1, 13, 3, 700, 1400, 8] if many else [1, 3, 0, 9]
+    g = _g(C + K)
+    starts = [(0, 5, 2, 7, 1, 0, 3, 9, 0, 4)[i] for i in range(len(lens))]
+    slots = list(range(len(lens)))[::-1]
+    qs = [0]
+    for n in lens:
+        qs.append(qs[-1] + n)
+    seq = _i32([b for b, n in enumerate(lens) for _ in range(n)])
+    x, w, bias = _rand(g, qs[-1], C + off + 8, dtype=BF), _rand(g, C, K, scale=0.5), _rand(g, C)
+    hist = _rand(g, len(lens) + 1, K - 1, C, dtype=BF)
+    hist2 = hist.clone()
+    for b, silu in ((bias, True), (None, False)):
+        y = hops.short_conv(x, w, seq, _i32(qs), _i32(starts), _i32(slots), hist, silu, b, off)
+        y2 = ref.short_conv(x, w, _i32(qs), _i32(starts), _i32(slots), hist2, silu, b, off)
+        _close(y, y2, 8e-3)
+        assert torch.equal(hist, hist2)
+
+
+@pytest.mark.parametrize("H,G,D,Dv,dims,norm,v_rot,v_k", [
+    (8, 2, 128, 128, 64, True, False, False), (4, 1, 64, 64, 64, True, True, False), (3, 3, 128, 128, 16, False, False, True),
+    (2, 1, 256, 64, 0, False, False, False), (2, 2, 512, 32, 256, True, True, False), (4, 2, 8, 8, 0, True, False, False),
+    (6, 2, 32, 48, 32, True, True, False), (2, 1, 128, 128, 8, True, False, False), (2, 1, 96, 96, 32, True, False, False)])
+@pytest.mark.parametrize("mix", [False, True])
+def test_window_prep(H, G, D, Dv, dims, norm, v_rot, v_k, mix):
+    from chronos.models.hybrid import rope_cos_sin
+    from chronos.ops import hybrid as hops, hybrid_ref as ref
+
+    g = _g(H * D + Dv + dims)
+    T, NB, bs = 9, 7, 16
+    off = H * D if v_k else -1
+    width = max((H + G) * D + G * Dv, 0) + 8
+    qkv = _rand(g, T, width, dtype=BF)
+    pos, seq = _i32([0, 1, 2, 30, 31, 32, 5, 6, 47]), _i32([0, 0, 0, 1, 1, 1, 2, 2, 1])
+    bt = _i32([[1, 0, 0], [2, 3, 4], [5, 6, 0]])
+    kc, vc = _rand(g, NB, bs, G, D, dtype=BF), _rand(g, NB, bs, G, Dv, dtype=BF)
+    kc2, vc2 = kc.clone(), vc.clone()
+    qn, kn = (_rand(g, D) + 1, _rand(g, D) + 1) if norm else (None, None)
+    vf, lam = (_rand(g, T, G * Dv, dtype=BF), _rand(g, 1)) if mix else (None, None)
+    cs = rope_cos_sin(1e4, dims, 64, DEV) if dims else None
+    vcs = rope_cos_sin(1e4, Dv, 64, DEV) if v_rot else None
+    temp = torch.rand(64, device=DEV, generator=g) if mix else None
+    a, b = qkv.clone(), qkv.clone()
+    v1 = hops.window_prep(a, H, G, D, Dv, vf, lam, pos, seq, bt, qn, kn, 1e-6, cs, dims, kc, vc, not mix, off, vcs, temp)
+    v2 = ref.window_prep(b, H, G, D, Dv, vf, lam, pos, seq, bt, qn, kn, 1e-6, cs, dims, kc2, vc2, not mix, off, vcs, temp)
+    for x, y in ((a, b), (kc, kc2), (vc, vc2)):
+        _close(x, y, 1.2e-2)
+    assert torch.equal(a[:, H * D:], qkv[:, H * D:]), "only queries are rewritten"
+    if not mix:
+        assert torch.equal(v1, v2)
