@@ -40,7 +40,9 @@ void launch_hy_moe_route(const void*, const void*, const float*, float*, int32_t
                          hipStream_t);
 void launch_hy_moe_ffn_token(const void*, const int32_t*, const float*, const void*, const void*, void*, int, int, int,
                              int, int, int, bool, hipStream_t);
-int hy_moe_max_tiles(int, int);
+int hy_moe_tile(int, int, int, int, int);
+int hy_moe_max_tiles(int, int, int);
+int64_t hy_moe_meta_ints(int, int, int);
 void launch_hy_moe_grouped(const uint16_t*, const int32_t*, const float*, const uint16_t*, const uint16_t*, uint16_t*,
                            int32_t*, uint16_t*, uint16_t*, int, int, int, int, int, int, hipStream_t);
 void launch_hy_rms_norm(const void*, float*, const float*, void*, bool, int, int, float, float, hipStream_t);
@@ -400,10 +402,12 @@ Tensor hy_moe_ffn(const Tensor& h, const Tensor& idx, const Tensor& wt, const Te
     // float32, or widths off the 128 grid: the token-parallel kernel
     if (!f32(h) && d % 128 == 0 && F % 128 == 0 && E <= 256 && T > 0) {
         const int top = (int)idx.size(1), items = (int)T * top;
-        const int maxTiles = chronos::hy_moe_max_tiles(items, (int)E);
-        auto meta = at::empty({1 + (int64_t)maxTiles + (int64_t)maxTiles * 128 + items}, h.options().dtype(at::kInt));
-        auto z = at::empty({(int64_t)maxTiles * 128, F}, h.options());
-        auto yrows = at::empty({(int64_t)maxTiles * 128, d}, h.options());
+        const int tile = chronos::hy_moe_tile(items, (int)E, (int)d, (int)F, (int)F);
+        const int maxTiles = chronos::hy_moe_max_tiles(items, (int)E, tile);
+        const int64_t rows = (int64_t)maxTiles * tile;
+        auto meta = at::empty({chronos::hy_moe_meta_ints(items, (int)E, tile)}, h.options().dtype(at::kInt));
+        auto z = at::empty({rows, F}, h.options());
+        auto yrows = at::empty({rows, d}, h.options());
         chronos::launch_hy_moe_grouped((const uint16_t*)h.data_ptr(), idx.data_ptr<int32_t>(), wt.data_ptr<float>(),
                                        (const uint16_t*)w_up.data_ptr(), (const uint16_t*)w_down.data_ptr(),
                                        (uint16_t*)out.data_ptr(), meta.data_ptr<int32_t>(), (uint16_t*)z.data_ptr(),
@@ -773,15 +777,18 @@ Tensor hy_moe_glu_ffn(const Tensor& h, const Tensor& idx, const Tensor& wt, cons
     i32(idx, "moe_glu_ffn: idx"); flt(wt, "moe_glu_ffn: weights");
     need(idx.dim() == 2 && idx.size(0) == T && wt.sizes() == idx.sizes(), "moe_glu_ffn: idx / weights [T, top]");
     auto out = at::empty_like(h);
-    // bfloat16 with tile-sized widths and more than a few tokens: the grouped MFMA GEMMs over the tile-ordered copy
-    // of the gate / up rows; otherwise the token-parallel kernel (which reads either row order)
+    // bfloat16 with tile-sized widths: the grouped MFMA GEMMs over the tile-ordered copy of the gate / up rows, for a single
+    // token too (32 experts of 4096 by 1536, 1 and 16 tokens: 49 and 220 us; the token-parallel kernel, a workgroup per token,
+    // 85 and 126 ms); otherwise the token-parallel kernel (which reads either row order)
     need(!tiled || (!f32(h) && d % 128 == 0 && F % 128 == 0), "moe_glu_ffn: the tile order is for bfloat16 experts with d and F on the 128 grid");
-    if (tiled && E <= 256 && T * idx.size(1) >= 4 * E) {
+    if (tiled && E <= 256 && T > 0) {
         const int top = (int)idx.size(1), items = (int)T * top;
-        const int maxTiles = chronos::hy_moe_max_tiles(items, (int)E);
-        auto meta = at::empty({1 + (int64_t)maxTiles + (int64_t)maxTiles * 128 + items}, h.options().dtype(at::kInt));
-        auto z = at::empty({(int64_t)maxTiles * 128, F}, h.options());
-        auto yrows = at::empty({(int64_t)maxTiles * 128, d}, h.options());
+        const int tile = chronos::hy_moe_tile(items, (int)E, (int)d, (int)F, 2 * (int)F);
+        const int maxTiles = chronos::hy_moe_max_tiles(items, (int)E, tile);
+        const int64_t rows = (int64_t)maxTiles * tile;
+        auto meta = at::empty({chronos::hy_moe_meta_ints(items, (int)E, tile)}, h.options().dtype(at::kInt));
+        auto z = at::empty({rows, F}, h.options());
+        auto yrows = at::empty({rows, d}, h.options());
         chronos::launch_hy_moe_glu_grouped((const uint16_t*)h.data_ptr(), idx.data_ptr<int32_t>(), wt.data_ptr<float>(),
                                            (const uint16_t*)w_gu.data_ptr(), (const uint16_t*)w_down.data_ptr(),
                                            (uint16_t*)out.data_ptr(), meta.data_ptr<int32_t>(), (uint16_t*)z.data_ptr(),

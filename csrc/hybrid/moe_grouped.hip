@@ -1,10 +1,10 @@
 // moe_grouped.hip — the experts of a mixture-of-experts layer as two grouped MFMA GEMMs (bfloat16), for any number of
-// tokens: every expert's weights are streamed once per 128 of its tokens, never once per token.
+// tokens: every expert's weights are streamed once per tile of its tokens, never once per token.
 //
-//   align     one workgroup: counts the (token, choice) items of every expert with weights, gives each expert a run
-//             of whole 128-row tiles in a sorted row space, and writes row -> item (or -1 for padding), item -> row
+//   align     (count and place kernels) counts the (token, choice) items of every expert with weights, gives each expert a
+//             run of whole tiles in a sorted row space, and writes row -> item (or -1 for padding), item -> row
 //             and the tile -> expert table.  Everything stays on the device: the GEMM grids are sized for the worst
-//             case (items / 128 + experts tiles) and surplus workgroups leave at once, so the host never learns the
+//             case (items / tile + experts tiles) and surplus workgroups leave at once, so the host never learns the
 //             routing and the step captures into a graph.
 //   up GEMM   Z[row, :] = act(h[token(row), :] W_up[e]^T): the x operand's rows are GATHERED by token through the
 //             per-lane LDS-DMA source addresses; activation in the epilogue.
@@ -16,8 +16,8 @@
 // time (moe_glu_row_order) so that every 128-row tile holds 64 gate rows and their 64 up rows in the accumulator
 // positions of the same lane; the epilogue combines them and writes 64 columns of Z [rows, F] per tile.
 //
-// The tile loop is the 128 x 128 x 64 LDS-DMA ring of csrc/kernels/gemm.hip (4 waves as 2 x 2, 16x16x32 bf16 MFMAs,
-// XOR-swizzled images, one barrier per k-step with a counted vmcnt).  Needs d % 128 == 0 and F % 128 == 0.
+// The tile loop is an LDS-DMA ring (16x16x32 bf16 MFMAs, XOR-swizzled images, one barrier per k-step with a counted vmcnt) at
+// three tile sizes, below.  Needs d % 128 == 0 and F % 128 == 0.
 #include "hybrid_common.h"
 
 namespace chronos {
@@ -26,88 +26,201 @@ namespace hy {
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef __attribute__((address_space(1))) void* gbl_ptr_t;
 
-constexpr int GBM = 128, GBN = 128, GBK = 64, GSTAGES = 3;
-constexpr int kImg = 128 * GBK * 2;
+// A tile: TM rows (tokens) by TN weight rows, k taken 64 at a time (whole 128-byte lines: rows of half lines reach a CU at a
+// third of the rate) through a ring of ST stages; waves as 2 (weight rows) x WX (tokens).
+//   256 x 256, two stages (128 KB), 8 waves of 128 x 64 outputs (moe_gemm256_kernel): experts with many tokens; half the bytes
+//    per product of
+//   128 x 128, two stages (64 KB: two workgroups per CU, one multiplies while the other waits), 4 waves of 64 x 64
+//    32 x 128, four stages (80 KB: two workgroups per CU, the weights of three k-steps in flight in each): few tokens
+template <int TM> struct Tile {
+    static constexpr int TN = 128, ST = TM == 32 ? 4 : 2, WX = 2, WAVES = 4;
+    static constexpr int W = TN * 128, X = TM * 128;                                     // bytes of the two images of a stage
+    static constexpr int WP = W / 1024 / WAVES, XP = X / 1024 / WAVES;                   // 1 KiB pieces per wave and stage
+    static constexpr int NS = TN / 32, NM = TM / 16 / WX;                                // 16-row blocks per wave
+    static constexpr int lds = ST * (W + X);
+};
 
 template <int N>
 __device__ __forceinline__ void wait_vm() {
     __builtin_amdgcn_s_waitcnt((N & 0xF) | (0x7 << 4) | (0xF << 8) | ((N >> 4) << 14));
 }
+constexpr int kActGlu = 2;
+
+// 16-byte piece c of image row r lies at c ^ (r & 7): 16 rows at the same c fall on different banks
 __device__ __forceinline__ bf16x8 frag(const unsigned char* img, int row, int chunk) {
     return *reinterpret_cast<const bf16x8*>(img + row * 128 + ((chunk ^ (row & 7)) << 4));
 }
 
-// meta layout (int32): [0] tiles used | [1 .. 1+maxTiles) tile -> expert | then row -> item [maxTiles * 128] |
-// then item -> row [items]
-__global__ void __launch_bounds__(1024) moe_align_kernel(const int32_t* __restrict__ idx, int items, int E, int maxTiles,
+// meta layout (int32): [0] tiles used | [1 .. 1+maxTiles) tile -> expert | then row -> item [maxTiles * TM] |
+// then item -> row [items] | then items per workgroup and expert [workgroups, E]
+constexpr int kAlignItems = 2048;   // items per workgroup
+
+// Ranks of items [lo, hi) within their experts, into rank_of (-1: nobody's item), and the experts' counts into cnt (LDS).
+// The lanes of a wave with the same expert find each other by the bits of its number (one ballot per bit) and the first of them
+// moves the expert's counter for all: one LDS atomic per wave and expert.
+__device__ __forceinline__ void moe_rank(const int32_t* __restrict__ idx, int lo, int hi, int E, int* cnt, int32_t* __restrict__ rank_of) {
+    const int lane = threadIdx.x & 63;
+    for (int e = threadIdx.x; e < E; e += blockDim.x) cnt[e] = 0;
+    __syncthreads();
+    int bits = 0;
+    while ((1 << bits) < E) ++bits;
+    for (int i0 = lo + threadIdx.x - lane; i0 < hi; i0 += blockDim.x) {   // (whole waves: the ballots take all lanes)
+        const int i = i0 + lane, e = i < hi ? idx[i] : -1;
+        const bool ok = e >= 0 && e < E;
+        unsigned long long same = __ballot(ok);
+        for (int k = 0; k < bits; ++k) {
+            const unsigned long long one = __ballot((e >> k) & 1);
+            same &= ((e >> k) & 1) ? one : ~one;
+        }
+        const int first = ok ? __ffsll(same) - 1 : lane, rank = __popcll(same & ((1ull << lane) - 1));
+        int base = 0;
+        if (ok && lane == first) base = atomicAdd(&cnt[e], __popcll(same));
+        base = __shfl(base, first, 64);
+        if (i < hi) rank_of[i] = ok ? base + rank : -1;
+    }
+    __syncthreads();
+}
+
+__global__ void __launch_bounds__(1024) moe_count_kernel(const int32_t* __restrict__ idx, int items, int E, int32_t* __restrict__ counts,
+                                                         int32_t* __restrict__ item_row) {
+    __shared__ int cnt[256];
+    const int lo = blockIdx.x * kAlignItems;
+    moe_rank(idx, lo, min(lo + kAlignItems, items), E, cnt, item_row);
+    for (int e = threadIdx.x; e < E; e += blockDim.x) counts[blockIdx.x * E + e] = cnt[e];
+}
+
+// Gives every expert a run of whole tiles and every item its row.  One workgroup ranks its items itself; of several each places
+// the items that it counted in moe_count_kernel (32768 items: 10 us in two launches of 16 workgroups; one workgroup took 38).
+// Which row of its expert's run an item takes does not matter: every row is computed on its own and found again through
+// item -> row, so the result is the same for any order.
+__global__ void __launch_bounds__(1024) moe_place_kernel(const int32_t* __restrict__ idx, int items, int E, int TM, int maxTiles,
                                                          int32_t* __restrict__ meta) {
-    __shared__ int cnt[256], start[257], fill[256];
+    __shared__ int cnt[256], before[256], start[257];
     int32_t* tile_e = meta + 1;
     int32_t* row_item = tile_e + maxTiles;
-    int32_t* item_row = row_item + maxTiles * GBM;
-    for (int e = threadIdx.x; e < E; e += blockDim.x) { cnt[e] = 0; fill[e] = 0; }
-    __syncthreads();
-    for (int i = threadIdx.x; i < items; i += blockDim.x) {
-        const int e = idx[i];
-        if (e >= 0 && e < E) atomicAdd(&cnt[e], 1);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int t = 0;
-        for (int e = 0; e < E; ++e) {
-            start[e] = t;
-            const int n = (cnt[e] + GBM - 1) / GBM;
-            for (int j = 0; j < n; ++j) tile_e[t + j] = e;
-            t += n;
+    int32_t* item_row = row_item + maxTiles * TM;
+    const int32_t* counts = item_row + items;
+    const int tid = threadIdx.x, wg = blockIdx.x, nwg = gridDim.x;
+    const int lo = wg * kAlignItems, hi = nwg == 1 ? items : min(lo + kAlignItems, items);
+    if (nwg == 1) {
+        moe_rank(idx, lo, hi, E, cnt, item_row);
+        if (tid < E) before[tid] = 0;
+    } else if (tid < E) {
+        int sum = 0, mine = 0;
+        for (int g = 0; g < nwg; ++g) {
+            if (g == wg) mine = sum;
+            sum += counts[g * E + tid];
         }
-        start[E] = t;
-        meta[0] = t;
+        cnt[tid] = sum;
+        before[tid] = mine;
     }
     __syncthreads();
-    const int used = start[E];
-    for (int i = threadIdx.x; i < used * GBM; i += blockDim.x) row_item[i] = -1;
+    if (tid < 64) {   // first tile of every expert: a running sum over the experts, four per lane
+        int n[4], sum = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            n[j] = 4 * tid + j < E ? (cnt[4 * tid + j] + TM - 1) / TM : 0;
+            sum += n[j];
+        }
+        int to = sum;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int v = __shfl_up(to, o, 64);
+            if (tid >= o) to += v;
+        }
+        int at = to - sum;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            start[4 * tid + j] = at;
+            at += n[j];
+        }
+        if (tid == 63) {
+            start[256] = at;
+            if (wg == 0) meta[0] = at;
+        }
+    }
     __syncthreads();
-    // which row of its expert's run an item takes does not matter: every row is computed on its own and found again
-    // through item -> row, so the result is the same for any order
-    for (int i = threadIdx.x; i < items; i += blockDim.x) {
-        const int e = idx[i];
-        if (e >= 0 && e < E) {
-            const int r = start[e] * GBM + atomicAdd(&fill[e], 1);
+    for (int e = wg; e < E; e += nwg) {   // an expert's tiles, and the rows behind its last item
+        for (int j = start[e] + tid; j < start[e + 1]; j += blockDim.x) tile_e[j] = e;
+        for (int r = start[e] * TM + cnt[e] + tid; r < start[e + 1] * TM; r += blockDim.x) row_item[r] = -1;
+    }
+    for (int i = lo + tid; i < hi; i += blockDim.x) {
+        const int e = idx[i], k = item_row[i];
+        if (k >= 0) {
+            const int r = start[e] * TM + before[e] + k;
             row_item[r] = i;
             item_row[i] = r;
         }
     }
-    for (int i = threadIdx.x; i < items; i += blockDim.x) {
-        const int e = idx[i];
-        if (e < 0 || e >= E) item_row[i] = -1;
+}
+
+// The wave's outputs: NS x NM accumulator tiles of 16 weight rows by 16 tokens, from weight row n0 and token row m0 on.  Lane l
+// holds D[n = 4 (l >> 4) + i][m = l & 15] of each = y[m][n .. n + 3].
+template <int ACT, int NS, int NM>
+__device__ __forceinline__ void moe_store(const f32x4 (&acc)[NS][NM], uint16_t* __restrict__ y, const int32_t* __restrict__ row_item,
+                                          int m0, int n0, int N, int lane, float limit, float slope, float shift) {
+#pragma unroll
+    for (int t = 0; t < NM; ++t) {
+        const int m = m0 + 16 * t + (lane & 15);
+        if (row_item[m] < 0) continue;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            const int row = n0 + 16 * s;   // first weight row of the block
+            if (row >= N) break;           // (the last tile of a 256-row launch may be half)
+            u16x4 o;
+            if constexpr (ACT == kActGlu) {
+                // every 64 rows: blocks 0 and 1 are gate rows, 2 and 3 the up rows of the same outputs
+                if (s & 2) continue;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float a = fminf(bf2f(f2bf(acc[s][t][i])), limit);
+                    const float u = fminf(fmaxf(bf2f(f2bf(acc[s | 2][t][i])), -limit), limit);
+                    o[i] = f2bf(a * sigmoid_act<uint16_t>(slope * a) * (u + shift));
+                }
+                const int n = (row >> 6) * 32 + (row & 31) + 4 * (lane >> 4);
+                *reinterpret_cast<u16x4*>(y + (int64_t)m * (N / 2) + n) = o;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    float v = acc[s][t][i];
+                    if constexpr (ACT >= 0) v = act_apply(bf2f(f2bf(v)), ACT);
+                    o[i] = f2bf(v);
+                }
+                *reinterpret_cast<u16x4*>(y + (int64_t)m * N + row + 4 * (lane >> 4)) = o;
+            }
+        }
     }
 }
 
-// y[row, n] = sum_k x[src(row), k] * w[e][n, k]; GATHER: src(row) = row_item[row] / top (rows of h), else row.
-// ACT >= 0: activation of that kind in the epilogue.  ACT == kActGlu: w holds N = 2F permuted gate / up rows, y is
-// [rows, N / 2], and (limit, slope, shift) are the gated unit's constants.
-constexpr int kActGlu = 2;
-template <bool GATHER, int ACT>
-__global__ void __launch_bounds__(256) moe_gemm_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
-                                                       uint16_t* __restrict__ y, const int32_t* __restrict__ meta,
-                                                       int maxTiles, int top, int N, int K, float limit, float slope,
-                                                       float shift) {
+// The tiles there are go to the XCDs in contiguous runs (their L2s then share rows of x and w); a launch of small tiles is
+// bound by the weights' bytes and spreads them over all.
+template <int TM, bool GATHER, int ACT>
+__global__ void __launch_bounds__(256, 2) moe_gemm_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
+                                                          uint16_t* __restrict__ y, const int32_t* __restrict__ meta,
+                                                          int maxTiles, int top, int N, int K, float limit, float slope,
+                                                          float shift) {
+    using C = Tile<TM>;
+    constexpr int ST = C::ST, BK = 64;
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-    const int nt = N / GBN;
-    const int tile = blockIdx.x / nt, tn = blockIdx.x % nt;
-    if (tile >= meta[0]) return;
+    const int nt = N / C::TN, used = meta[0];
+    if ((int)blockIdx.x >= used * nt) return;
+    const int id = TM == 128 ? xcd_remap(blockIdx.x, used * nt) : (int)blockIdx.x;
+    const int tile = id / nt, tn = id - tile * nt;
     const int e = meta[1 + tile];
     const int32_t* row_item = meta + 1 + maxTiles;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int m0 = tile * GBM;
+    const int m0 = tile * TM;
     const uint16_t* we = w + (int64_t)e * N * K;
-    const uint16_t* wsrc[4];
-    const uint16_t* xsrc[4];
+    const uint16_t* wsrc[C::WP];
+    const uint16_t* xsrc[C::XP];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int r = 32 * wave + 8 * i + (lane >> 3);
-        const int c = (lane & 7) ^ (r & 7);
-        wsrc[i] = we + (int64_t)(tn * GBN + r) * K + c * 8;
+    for (int i = 0; i < C::WP; ++i) {
+        const int r = 8 * (C::WP * wave + i) + (lane >> 3), c = (lane & 7) ^ (r & 7);
+        wsrc[i] = we + (int64_t)(tn * C::TN + r) * K + c * 8;
+    }
+#pragma unroll
+    for (int i = 0; i < C::XP; ++i) {
+        const int r = 8 * (C::XP * wave + i) + (lane >> 3), c = (lane & 7) ^ (r & 7);
         int64_t xr = m0 + r;
         if constexpr (GATHER) {
             const int it = row_item[m0 + r];
@@ -116,95 +229,162 @@ __global__ void __launch_bounds__(256) moe_gemm_kernel(const uint16_t* __restric
         xsrc[i] = x + xr * K + c * 8;
     }
     auto issue = [&](int kt) {
-        unsigned char* st = smem + (kt % GSTAGES) * 2 * kImg;
-        const int koff = kt * GBK;
+        unsigned char* st = smem + (kt % ST) * (C::W + C::X);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            __builtin_amdgcn_global_load_lds((gbl_ptr_t)(wsrc[i] + koff), (lds_ptr_t)(st + (4 * wave + i) * 1024), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds((gbl_ptr_t)(xsrc[i] + koff), (lds_ptr_t)(st + kImg + (4 * wave + i) * 1024), 16, 0, 0);
-        }
+        for (int i = 0; i < C::WP; ++i)
+            __builtin_amdgcn_global_load_lds((gbl_ptr_t)(wsrc[i] + kt * BK), (lds_ptr_t)(st + (C::WP * wave + i) * 1024), 16, 0, 0);
+#pragma unroll
+        for (int i = 0; i < C::XP; ++i)
+            __builtin_amdgcn_global_load_lds((gbl_ptr_t)(xsrc[i] + kt * BK), (lds_ptr_t)(st + C::W + (C::XP * wave + i) * 1024), 16, 0, 0);
     };
-    const int wn = wave >> 1, wm = wave & 1;
-    f32x4 acc[4][4];
+    const int wn = wave / C::WX, wm = wave % C::WX;
+    f32x4 acc[C::NS][C::NM];
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
+    for (int s = 0; s < C::NS; ++s)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) acc[s][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int KT = K / GBK;
+        for (int t = 0; t < C::NM; ++t) acc[s][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int KT = K / BK;
 #pragma unroll
-    for (int p = 0; p < GSTAGES - 1; ++p)
+    for (int p = 0; p < ST - 1; ++p)
         if (p < KT) issue(p);
     for (int kt = 0; kt < KT; ++kt) {
-        if (kt + GSTAGES - 2 < KT) wait_vm<8 * (GSTAGES - 2)>();
+        if (kt + ST - 2 < KT) wait_vm<(C::WP + C::XP) * (ST - 2)>();
         else wait_vm<0>();
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if (kt + GSTAGES - 1 < KT) issue(kt + GSTAGES - 1);
-        const unsigned char* wimg = smem + (kt % GSTAGES) * 2 * kImg;
-        const unsigned char* ximg = wimg + kImg;
+        if (kt + ST - 1 < KT) issue(kt + ST - 1);
+        const unsigned char* wimg = smem + (kt % ST) * (C::W + C::X);
+        const unsigned char* ximg = wimg + C::W;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int h = 0; h < BK / 32; ++h) {
             const int chunk = h * 4 + (lane >> 4);
-            bf16x8 a[4], b[4];
+            bf16x8 a[C::NS], b[C::NM];
 #pragma unroll
-            for (int s = 0; s < 4; ++s) a[s] = frag(wimg, 64 * wn + 16 * s + (lane & 15), chunk);
+            for (int t = 0; t < C::NM; ++t) b[t] = frag(ximg, 16 * (C::NM * wm + t) + (lane & 15), chunk);
 #pragma unroll
-            for (int t = 0; t < 4; ++t) b[t] = frag(ximg, 64 * wm + 16 * t + (lane & 15), chunk);
+            for (int s = 0; s < C::NS; ++s) a[s] = frag(wimg, C::TN / 2 * wn + 16 * s + (lane & 15), chunk);
 #pragma unroll
-            for (int s = 0; s < 4; ++s)
+            for (int s = 0; s < C::NS; ++s)
 #pragma unroll
-                for (int t = 0; t < 4; ++t)
+                for (int t = 0; t < C::NM; ++t)
                     acc[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], b[t], acc[s][t], 0, 0, 0);
         }
     }
-    // lane holds D[n = 4 * (lane >> 4) + i][m = lane & 15] of each 16 x 16 tile = y[m][n .. n + 3]
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        const int m = m0 + 64 * wm + 16 * t + (lane & 15);
-        if (row_item[m] < 0) continue;
-        if constexpr (ACT == kActGlu) {
-            // tile-local rows 64 wn + 16 s + j: s = 0, 1 are gate rows, s = 2, 3 the up rows of the same outputs
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                u16x4 o;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float a = fminf(bf2f(f2bf(acc[s][t][i])), limit);
-                    const float u = fminf(fmaxf(bf2f(f2bf(acc[s + 2][t][i])), -limit), limit);
-                    o[i] = f2bf(a * sigmoidf_(slope * a) * (u + shift));
-                }
-                const int n = tn * 64 + 32 * wn + 16 * s + 4 * (lane >> 4);
-                *reinterpret_cast<u16x4*>(y + (int64_t)m * (N / 2) + n) = o;
-            }
-            continue;
-        }
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            u16x4 o;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float v = acc[s][t][i];
-                if constexpr (ACT >= 0 && ACT != kActGlu) v = act_apply(bf2f(f2bf(v)), ACT);
-                o[i] = f2bf(v);
-            }
-            const int n = tn * GBN + 64 * wn + 16 * s + 4 * (lane >> 4);
-            *reinterpret_cast<u16x4*>(y + (int64_t)m * N + n) = o;
-        }
-    }
+    moe_store<ACT, C::NS, C::NM>(acc, y, row_item, m0 + 16 * C::NM * wm, tn * C::TN + C::TN / 2 * wn, N, lane, limit, slope, shift);
 }
 
+// The 256 x 256 tile (x and one expert's weights below 4 and 2 GiB; weight rows past the end read as zeros).  Two sets of operands in registers: while
+// one half of a k-step (32 deep) is multiplied the other half's fragments are read from LDS, so that neither the LDS nor
+// the matrix cores wait for the other; one barrier per k-step, in its middle, behind which the buffer that everybody has read is
+// refilled for the step after next.
+template <bool GATHER, int ACT>
+__global__ void __launch_bounds__(512, 1) moe_gemm256_kernel(const uint16_t* __restrict__ x, uint32_t xbytes,
+                                                             const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
+                                                             const int32_t* __restrict__ meta, int maxTiles, int top, int N,
+                                                             int K, float limit, float slope, float shift) {
+    constexpr int IMG = 256 * 128, STAGE = 2 * IMG;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+    const int nt = (N + 255) / 256, used = meta[0];
+    if ((int)blockIdx.x >= used * nt) return;
+    const int id = xcd_remap(blockIdx.x, used * nt);
+    const int tile = id / nt, tn = id - tile * nt;
+    const int e = meta[1 + tile];
+    const int32_t* row_item = meta + 1 + maxTiles;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int m0 = tile * 256;
+    // wave w stages image rows 32 w .. 32 w + 31 of both operands in four pieces of 8 rows
+    const int pr = lane >> 3, pc = (lane & 7) ^ pr;
+    const uint32_t wvoff = (uint32_t)(pr * K + pc * 8) * 2;
+    const int wsoff = (tn * 256 + 32 * wave) * K * 2;
+    uint32_t xvoff[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t xr = m0 + 32 * wave + 8 * i + pr;
+        if constexpr (GATHER) {
+            const int it = row_item[xr];
+            xr = it < 0 ? 0 : it / top;  // padding rows read token 0 and are never stored
+        }
+        xvoff[i] = (xr * (uint32_t)K + pc * 8) * 2;
+    }
+    const uint16_t* we = w + (int64_t)e * N * K;
+    const uint32_t lds0 = lds_offset(smem);
+    auto dma_w = [&](int kt, int i) {
+        dma_1k_buf(we, (uint32_t)N * K * 2, lds0 + (kt & 1) * STAGE + (4 * wave + i) * 1024, wvoff, wsoff + (i * 8 * K + kt * 64) * 2);
+    };
+    auto dma_x = [&](int kt, int i) {
+        dma_1k_buf(x, xbytes, lds0 + (kt & 1) * STAGE + IMG + (4 * wave + i) * 1024, xvoff[i], kt * 128);
+    };
+    const int wn = wave >> 2, wm = wave & 3;
+    const int ln = lane & 15, g = lane >> 4;
+    const unsigned char* const wimg = smem + (128 * wn + ln) * 128;   // (16-row blocks: the swizzle depends on ln only)
+    const unsigned char* const ximg = smem + IMG + (64 * wm + ln) * 128;
+    const int ch[2] = {(g ^ (ln & 7)) * 16, ((4 + g) ^ (ln & 7)) * 16};
+    bf16x8 a[2][8], b[2][4];
+    auto ldw = [&](int st, int h, int s) { a[h][s] = *reinterpret_cast<const bf16x8*>(wimg + st * STAGE + s * 2048 + ch[h]); };
+    auto ldx = [&](int st, int h, int t) { b[h][t] = *reinterpret_cast<const bf16x8*>(ximg + st * STAGE + t * 2048 + ch[h]); };
+    f32x4 acc[8][4];
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[s][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int KT = K / 64;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { dma_w(kt, i); dma_x(kt, i); }
+    wait_vm<8>();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int t = 0; t < 4; ++t) ldx(0, 0, t);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) ldw(0, 0, s);
+    for (int kt = 0; kt < KT; ++kt) {
+        const int st = kt & 1;
+        // first half of the step; the second half's fragments on their way
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            if (s < 4) ldx(st, 1, s);
+            ldw(st, 1, s);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0][s], b[0][t], acc[s][t], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // this wave's pieces of the next step have landed and its reads of this one are done; behind the barrier: everybody's
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const bool more = kt + 2 < KT;
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            if (more && s < 4) { dma_w(kt + 2, s); dma_x(kt + 2, s); }
+            // (the last step reads the other buffer once more, for nothing)
+            if (s < 4) ldx(st ^ 1, 0, s);
+            ldw(st ^ 1, 0, s);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1][s], b[1][t], acc[s][t], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    moe_store<ACT, 8, 4>(acc, y, row_item, m0 + 64 * wm, tn * 256 + 128 * wn, N, lane, limit, slope, shift);
+}
+
+// An index of E and above is an identity expert (its output is the token itself) where the experts' layer has such
+// (identity), else, like a negative one, nobody's: it adds nothing.
 __global__ void __launch_bounds__(256) moe_combine_kernel(const uint16_t* __restrict__ h, const uint16_t* __restrict__ yrows,
                                                           const int32_t* __restrict__ idx, const float* __restrict__ wt,
                                                           const int32_t* __restrict__ item_row, uint16_t* __restrict__ out,
-                                                          int d, int top, int E) {
+                                                          int d, int top, int E, int identity) {
     const int64_t t = blockIdx.x;
     for (int c = threadIdx.x * 8; c < d; c += 256 * 8) {
         float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         for (int k = 0; k < top; ++k) {
-            const int e = idx[t * top + k];
+            const int e = idx[t * top + k], r = item_row[t * top + k];
             const float g = wt[t * top + k];
-            const uint16_t* src = e >= E ? h + t * d + c : yrows + (int64_t)item_row[t * top + k] * d + c;
+            if (r < 0 && !(identity && e >= E)) continue;
+            const uint16_t* src = r < 0 ? h + t * d + c : yrows + (int64_t)r * d + c;
             const u16x8 v = *reinterpret_cast<const u16x8*>(src);
 #pragma unroll
             for (int j = 0; j < 8; ++j) acc[j] += g * bf2f(v[j]);
@@ -218,47 +398,86 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(const uint16_t* __rest
 
 }  // namespace hy
 
-int hy_moe_max_tiles(int items, int E) { return (items + hy::GBM - 1) / hy::GBM + E; }
+// Rows per tile.  32 where experts see at most 16 tokens on average, so that a tile's padding rows cost little and the launch
+// streams weights with more of them in flight; 256 where there are enough tiles of that size for whole rounds on the CUs
+// (256 tokens per expert and 512 tiles); else 128.  up: rows of an expert's first matrix.  Measured on gated experts, us at
+// 32 / 128 / 256 rows: 16 experts of 2048 by 1024 with 64 tokens (4 experts each) 47 / 55 / 80, 200 tokens 52 / 58 / 83, 512 tokens
+// 84 / 69 / 87, 2048 tokens 251 / 156 / 175, 8192 tokens 874 / 546 / 485; 32 experts of 4096 by 1536 with 8192 tokens 2563 / 1653 / 1387;
+// 8 experts of 1024 by 512 with 8192 tokens (2 each) 144 / 101 / 118.  (At 200 tokens of 2048, 50 items per expert, 32 rows still
+// win by a tenth; at 128 per expert they lose by a fifth: the line lies lower because a skewed choice fills more tiles.)
+int hy_moe_tile(int items, int E, int d, int F, int up) {
+    const int64_t G4 = (int64_t)1 << 32, rows = (int64_t)items + 256 * E;
+    const bool fits = rows * (d > F ? d : F) * 2 < G4 && (int64_t)up * d * 2 < G4 / 2;   // 32-bit offsets
+    const int64_t big = (int64_t)(items / 256) * (up < d ? up : d) / 256;
+    return items <= 16 * E ? 32 : items < 256 * E || big < 512 || !fits ? 128 : 256;
+}
+int hy_moe_max_tiles(int items, int E, int tm) {
+    const int n = items / tm + E;   // an expert's last tile may hold a single item
+    return n < items ? n : items;
+}
+static int moe_align_wgs(int items) { return items <= 2 * hy::kAlignItems ? 1 : (items + hy::kAlignItems - 1) / hy::kAlignItems; }
+int64_t hy_moe_meta_ints(int items, int E, int tm) {
+    const int64_t n = hy_moe_max_tiles(items, E, tm);
+    return 1 + n + n * tm + items + (int64_t)moe_align_wgs(items) * E;
+}
 
-// meta: int32 [1 + maxTiles + maxTiles * 128 + items]; z: bf16 [maxTiles * 128, F]; yrows: bf16 [maxTiles * 128, d].
+template <int TM, bool GATHER, int ACT>
+static void moe_gemm(const uint16_t* x, int64_t rows, const uint16_t* w, uint16_t* y, const int32_t* meta, int maxTiles, int top, int N, int K,
+                     float limit, float slope, float shift, hipStream_t s) {
+    if constexpr (TM == 256) {
+        const auto kern = hy::moe_gemm256_kernel<GATHER, ACT>;
+        constexpr int lds = 4 * 256 * 128;
+        static const hipError_t once = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        (void)once;
+        kern<<<maxTiles * ((N + 255) / 256), 512, lds, s>>>(x, (uint32_t)(rows * K * 2), w, y, meta, maxTiles, top, N, K, limit, slope, shift);
+    } else {
+        const auto kern = hy::moe_gemm_kernel<TM, GATHER, ACT>;
+        constexpr int lds = hy::Tile<TM>::lds;
+        static const hipError_t once = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        (void)once;
+        kern<<<maxTiles * (N / hy::Tile<TM>::TN), 256, lds, s>>>(x, w, y, meta, maxTiles, top, N, K, limit, slope, shift);
+    }
+}
+
+// meta: int32 [hy_moe_meta_ints]; z: bf16 [maxTiles * tile, F]; yrows: bf16 [maxTiles * tile, d]
+// (tile: hy_moe_tile).  ACT kActGlu: w_up holds 2F rows in the tile order of moe_glu_row_order.
+template <int TM, int ACT>
+static void moe_grouped(const uint16_t* h, const int32_t* idx, const float* wt, const uint16_t* w_up, const uint16_t* w_down,
+                        uint16_t* out, int32_t* meta, uint16_t* z, uint16_t* yrows, int T, int d, int F, int E, int top,
+                        float limit, float slope, float shift, hipStream_t s) {
+    const int items = T * top, maxTiles = hy_moe_max_tiles(items, E, TM);
+    const int nwg = moe_align_wgs(items);
+    int32_t* item_row = meta + 1 + maxTiles + maxTiles * TM;
+    if (nwg > 1) hy::moe_count_kernel<<<nwg, 1024, 0, s>>>(idx, items, E, item_row + items, item_row);
+    hy::moe_place_kernel<<<nwg, 1024, 0, s>>>(idx, items, E, TM, maxTiles, meta);
+    moe_gemm<TM, true, ACT>(h, T, w_up, z, meta, maxTiles, top, ACT == hy::kActGlu ? 2 * F : F, d, limit, slope, shift, s);
+    moe_gemm<TM, false, -1>(z, (int64_t)maxTiles * TM, w_down, yrows, meta, maxTiles, top, d, F, 0.f, 0.f, 0.f, s);
+    hy::moe_combine_kernel<<<T, 256, 0, s>>>(h, yrows, idx, wt, item_row, out, d, top, E, ACT != hy::kActGlu);
+}
+
 void launch_hy_moe_grouped(const uint16_t* h, const int32_t* idx, const float* wt, const uint16_t* w_up,
                            const uint16_t* w_down, uint16_t* out, int32_t* meta, uint16_t* z, uint16_t* yrows, int T,
                            int d, int F, int E, int top, int act, hipStream_t s) {
-    if (T == 0) return;
-    const int items = T * top, maxTiles = hy_moe_max_tiles(items, E);
-    hy::moe_align_kernel<<<1, 1024, 0, s>>>(idx, items, E, maxTiles, meta);
-    const int lds = hy::GSTAGES * 2 * hy::kImg;
-    static bool attr = false;
-    if (!attr) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(hy::moe_gemm_kernel<true, 0>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(hy::moe_gemm_kernel<true, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(hy::moe_gemm_kernel<false, -1>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        attr = true;
-    }
-    if (act == 0) hy::moe_gemm_kernel<true, 0><<<maxTiles * (F / hy::GBN), 256, lds, s>>>(h, w_up, z, meta, maxTiles, top, F, d, 0.f, 0.f, 0.f);
-    else hy::moe_gemm_kernel<true, 1><<<maxTiles * (F / hy::GBN), 256, lds, s>>>(h, w_up, z, meta, maxTiles, top, F, d, 0.f, 0.f, 0.f);
-    hy::moe_gemm_kernel<false, -1><<<maxTiles * (d / hy::GBN), 256, lds, s>>>(z, w_down, yrows, meta, maxTiles, top, d, F, 0.f, 0.f, 0.f);
-    hy::moe_combine_kernel<<<T, 256, 0, s>>>(h, yrows, idx, wt, meta + 1 + maxTiles + maxTiles * hy::GBM, out, d, top, E);
+    if (T == 0 || top == 0) return;
+    const int tm = hy_moe_tile(T * top, E, d, F, F);
+#define HY_MOE(TM, ACT) moe_grouped<TM, ACT>(h, idx, wt, w_up, w_down, out, meta, z, yrows, T, d, F, E, top, 0.f, 0.f, 0.f, s)
+    if (act == 0) { if (tm == 32) HY_MOE(32, 0); else if (tm == 128) HY_MOE(128, 0); else HY_MOE(256, 0); }
+    else { if (tm == 32) HY_MOE(32, 1); else if (tm == 128) HY_MOE(128, 1); else HY_MOE(256, 1); }
+#undef HY_MOE
 }
 
-// Gated experts.  w_gu: bf16 [E, 2F, d] in the tile order of moe_glu_row_order; z: bf16 [maxTiles * 128, F];
-// needs d % 128 == 0 and F % 128 == 0 (the down GEMM's k-steps and the up GEMM's 64-output tiles).
+// Gated experts.  w_gu: bf16 [E, 2F, d] in the tile order of moe_glu_row_order; needs d % 128 == 0 and F % 128 == 0 (the down
+// GEMM's k-steps and the up GEMM's 64-output tiles).
 void launch_hy_moe_glu_grouped(const uint16_t* h, const int32_t* idx, const float* wt, const uint16_t* w_gu,
                                const uint16_t* w_down, uint16_t* out, int32_t* meta, uint16_t* z, uint16_t* yrows, int T,
                                int d, int F, int E, int top, float limit, float slope, float shift, hipStream_t s) {
-    if (T == 0) return;
-    const int items = T * top, maxTiles = hy_moe_max_tiles(items, E);
-    hy::moe_align_kernel<<<1, 1024, 0, s>>>(idx, items, E, maxTiles, meta);
-    const int lds = hy::GSTAGES * 2 * hy::kImg;
-    static bool attr = false;
-    if (!attr) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(hy::moe_gemm_kernel<true, hy::kActGlu>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(hy::moe_gemm_kernel<false, -1>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        attr = true;
-    }
-    hy::moe_gemm_kernel<true, hy::kActGlu><<<maxTiles * (2 * F / hy::GBN), 256, lds, s>>>(h, w_gu, z, meta, maxTiles, top, 2 * F, d, limit, slope, shift);
-    hy::moe_gemm_kernel<false, -1><<<maxTiles * (d / hy::GBN), 256, lds, s>>>(z, w_down, yrows, meta, maxTiles, top, d, F, 0.f, 0.f, 0.f);
-    hy::moe_combine_kernel<<<T, 256, 0, s>>>(h, yrows, idx, wt, meta + 1 + maxTiles + maxTiles * hy::GBM, out, d, top, E);
+    if (T == 0 || top == 0) return;
+    const int tm = hy_moe_tile(T * top, E, d, F, 2 * F);
+#define HY_MOE(TM) moe_grouped<TM, hy::kActGlu>(h, idx, wt, w_gu, w_down, out, meta, z, yrows, T, d, F, E, top, limit, slope, shift, s)
+    if (tm == 32) HY_MOE(32);
+    else if (tm == 128) HY_MOE(128);
+    else HY_MOE(256);
+#undef HY_MOE
 }
 
 }  // namespace chronos
