@@ -5,24 +5,34 @@
 //     o_t = r_t ( e^L_t S^T q_t + sum_(s <= t) e^(L_t - L_s) w_s (k_s . q_t) v_s )
 //     S  <- e^L_C S + sum_s k_s (e^(L_C - L_s) w_s v_s)^T
 //
-// which are the sums of the token-by-token form in another order.  Precision: q, k and v are bfloat16, everything else
-// stays float32.  A float32 operand of a matrix product (the state, the weights of a chunk's tokens, the scaled values)
-// enters as three bfloat16 terms cut off its 24-bit mantissa — exactly that number, so a product costs three matrix
-// instructions and loses nothing — and all products accumulate in float32.  L is summed in float64: differences of sums
-// over strong decays keep their digits.
+// which are the sums of the token-by-token form in another order.  With the delta rule a token writes u_s = beta_s (v_s - what
+// the state before it reads at k_s) in place of v_s; with A[t, s] = beta_t e^(L_t - L_s) w_t w_s (k_t . k_s) below the
+// diagonal (w: the scale of k), (I + A) u = beta (v - e^L w S^T k), solved 16 rows at a time with the diagonal tiles' inverses.
+//
+// Precision: q, k and v are bfloat16, everything else stays float32.  A float32 operand of a matrix product (the state, the
+// weights of a chunk's tokens, the scaled values) enters as three bfloat16 terms whose sum is exactly that number, so a
+// product costs three matrix instructions and loses nothing (two float32 operands: six of the nine products of terms, the
+// rest is below 2^-26), and all products accumulate in float32.  L is summed in float64: differences of sums over strong
+// decays keep their digits.  Terms by truncation cost 3% less time, but leave the errors one-sided and larger (the state
+// after the state-space form: 4.8e-8 of its norm off the float64 recurrence; nearest terms 3.9e-8; token by token 4.2e-8).
+// The delta rule's solve carries what its sums round off along: the state is 5.7e-8 off (token by token 5.8e-8; without,
+// 6.1e-8, and 9.3e-8 with the products added to the sum one by one).
 //
 // A workgroup is NW waves and serves 16 NW value columns of one (sequence, head); a wave keeps all D rows of its 16 columns
 // of S in accumulators, which are in the operand layout of the read-out's product as they stand.  A chunk's q, k, v rows
 // come by DMA into one of two LDS buffers while the chunk before is computed; 16-byte pieces are permuted within a row by a
 // function of the row, so that neither the row-wise reads nor the transposing ones meet in a bank.  The waves share the
-// 64 x 64 weights (ten 16 x 16 tiles on and below the diagonal) through LDS.
+// 64 x 64 weights (ten 16 x 16 tiles on and below the diagonal) through LDS; the delta rule's tiles lie beside.
 //
-// What bounds it: the chain of a sequence's chunks, one wave per SIMD: about 1300 vector instructions (the cutting into
-// terms, the exponentials) and 114 matrix instructions per chunk and wave at D = 128, and two barriers, 7 us a chunk.
-// Measured, 4 sequences of 2048 tokens, token by token -> this: retention, 8 heads of 128 x 128: 797 -> 233 us; 32 heads:
-// 857 -> 243; state-space form, 128 heads of 128 x 64: 1101 -> 527; mlstm, 4 heads of 128 x 256: 1987 -> 301, 4 heads of
-// 256 x 512: 3058 -> 462, 8 heads: 3228 -> 472.  One and two waves per workgroup: 436 and 302 us where four take 233.
+// What bounds it: the chain of a sequence's chunks, one wave per SIMD: vector instructions (the cutting into terms, the
+// exponentials) and 114 matrix instructions (delta: 162) per chunk and wave at D = 128, and two barriers, 5 us a chunk (delta: 10).
+// Measured, 4 sequences of 2048 tokens, token by token -> this: retention, 8 heads of 128 x 128: 797 -> 171 us; 32 heads:
+// 857 -> 192; state-space form, 128 heads of 128 x 64: 1058 -> 445; mlstm, 4 heads of 128 x 256: 1987 -> 220, 4 heads of
+// 256 x 512: 3050 -> 303; delta rule, 32 heads of 128 x 128: 959 -> 389.  One and two waves per workgroup: 436 and 302 us
+// where four took 233 (of 171, before addresses, weights and stores lost their branches).
 #include "hybrid_common.h"
+
+#include <type_traits>
 
 namespace chronos {
 namespace hy {
@@ -34,29 +44,26 @@ __device__ __forceinline__ f32x4 mfma_16x16x32(bf16x8 a, bf16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// x = h + m + l exactly: the upper, middle and lower 8 bits of the mantissa
+// x = h + m + l exactly: each term the bfloat16 nearest to what is left (the second remainder has 8 bits at most)
 struct Terms {
     bf16x8 h, m, l;
 };
 __device__ __forceinline__ Terms split3(const float (&x)[8]) {
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    u32x4 t[3];
+    Terms t;
     float a[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) a[i] = x[i];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t u = __float_as_uint(a[2 * i]), v = __float_as_uint(a[2 * i + 1]);
-            t[k][i] = __builtin_amdgcn_perm(v, u, 0x07060302);   // (upper half of v) << 16 | upper half of u
-            if (k < 2) {
-                a[2 * i] -= __uint_as_float(u & 0xffff0000u);
-                a[2 * i + 1] -= __uint_as_float(v & 0xffff0000u);
-            }
-        }
+    for (int i = 0; i < 8; ++i) {
+        t.h[i] = (__bf16)x[i];
+        a[i] = x[i] - (float)t.h[i];
     }
-    return {__builtin_bit_cast(bf16x8, t[0]), __builtin_bit_cast(bf16x8, t[1]), __builtin_bit_cast(bf16x8, t[2])};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        t.m[i] = (__bf16)a[i];
+        a[i] -= (float)t.m[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) t.l[i] = (__bf16)a[i];
+    return t;
 }
 __device__ __forceinline__ bf16x8 join8(bf16x4 a, bf16x4 b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
 
@@ -67,7 +74,7 @@ __device__ __forceinline__ float exp_d(double x) {
 }
 
 // Where piece c (16 bytes) of row r of a tile with CPR pieces per row lies: c ^ spread<CPR>(r).  16 rows at the same c, and
-// 4 rows at 4 neighbouring c, fall on different banks.
+// 4 rows at 4 neighbouring c, fall on different banks.  Depends on r % 16 only.
 template <int CPR> __device__ __forceinline__ int spread(int r) {
     if constexpr (CPR >= 16) return ((r & 3) << 2) | ((r >> 2) & 3);
     else if constexpr (CPR == 8) return ((r & 2) << 1) | ((r >> 2) & 3);
@@ -75,22 +82,34 @@ template <int CPR> __device__ __forceinline__ int spread(int r) {
     else return 0;
 }
 
-// 64 rows of CPR pieces from src (rows ld elements apart, last: the last row there is, n: real pieces per row) into LDS:
-// piece j of CPR, one per 64 lanes.
-template <int CPR> __device__ __forceinline__ void dma_tile(const uint16_t* src, int64_t ld, int last, int n, int j, uint32_t lds,
-                                                            int lane) {
-    const int i = j * 64 + lane, row = i / CPR, c = (i % CPR) ^ spread<CPR>(row);
-    dma_1k(src + min(row, last) * ld + min(c, n - 1) * 8, __builtin_amdgcn_readfirstlane(lds + j * 1024));
+// Running sum over the wave's lanes (lane l: the sum of lanes 0 .. l): within rows of 16 lanes, then from row to row.
+__device__ __forceinline__ double lanes_running_sum(double x) {
+    auto from = [](double v, auto ctrl, auto rows) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, v);
+        const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, decltype(ctrl)::value, decltype(rows)::value, 0xf, true);
+        const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), decltype(ctrl)::value, decltype(rows)::value, 0xf, true);
+        return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+    };
+    using std::integral_constant;
+    constexpr integral_constant<int, 0xf> all{};
+    x += from(x, integral_constant<int, 0x111>{}, all);                              // one lane to the right
+    x += from(x, integral_constant<int, 0x112>{}, all);
+    x += from(x, integral_constant<int, 0x114>{}, all);
+    x += from(x, integral_constant<int, 0x118>{}, all);
+    x += from(x, integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});    // lane 15 of rows 0, 2 to rows 1, 3
+    x += from(x, integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});    // lane 31 to rows 2 and 3
+    return x;
 }
 
-enum { kScanPlain = 0, kScanMlstm = 1 };
+enum { kScanPlain = 0, kScanMlstm = 1, kScanDelta = 2 };
 
-// What the two forms read per token: plain: decay (one per token and head, or dts = 0: per head), qscale, kscale, vscale
-// (any of the three may be absent); mlstm: the log decays, log write factors and e^-m of mlstm_gates_kernel.
+// What the forms read per token: plain: decay (one per token and head, or dts = 0: per head), qscale, kscale, vscale
+// (any of the three may be absent); delta: the same without vscale, and beta; mlstm: the log decays, log write factors and
+// e^-m of mlstm_gates_kernel.
 struct ChunkScan {
     const uint16_t* proj;
     int ldp, q_off, k_off, v_off;
-    const float *qscale, *kscale, *vscale, *decay;
+    const float *qscale, *kscale, *vscale, *decay, *beta;
     int dts;
     float q_mul;
     const float *la, *lb, *em;
@@ -100,24 +119,49 @@ struct ChunkScan {
     int B, HK, H, Dv;
 };
 
-template <int D> constexpr int chunk_scan_lds() {
-    constexpr int NW = kCW;
-    return 2 * kCH * (2 * D + 16 * NW) * 2 + 10 * 1024 + NW * (kCH * 16) + 10 * 16 * 4 + NW * kCH * 4;
+// LDS (bytes): two buffers of q | k | v | weight tiles [10][64 lanes] x 16 (delta: and the solve's tiles [10], the inverses of
+// the diagonal ones [4]) | every wave's own copy of the scalars (L in float64, w, c; delta: beta, beta k-scale, and that times
+// e^L) | mlstm: the weight tiles' sums over s [10][16] and the waves' parts of n . q [NW][64]
+template <int D, int MODE> struct ChunkLds {
+    static constexpr int Q = kCH * D * 2, V = kCH * kCW * 32, BUF = 2 * Q + V;
+    static constexpr int PT = 2 * BUF, AT = PT + 10 * 1024, TT = AT + (MODE == kScanDelta ? 10 * 1024 : 0);
+    static constexpr int OWN = TT + (MODE == kScanDelta ? 4 * 1024 : 0), OWN_SIZE = kCH * (MODE == kScanDelta ? 28 : 16);
+    static constexpr int SUM = OWN + kCW * OWN_SIZE, SIZE = SUM + (MODE == kScanMlstm ? 640 + kCW * 256 : 0);
+};
+
+// a * b of two float32 operands in matrix layout (4 elements per lane, k = 4 g + e), as the six leading products of their terms:
+// the other three are below 2^-24 of the result.  The two halves of a 32-deep instruction hold two of the six.
+struct Terms4 {
+    bf16x4 h, m, l;
+};
+__device__ __forceinline__ Terms4 split3(const f32x4& x) {
+    const float v[8] = {x[0], x[1], x[2], x[3], 0.f, 0.f, 0.f, 0.f};
+    const Terms t = split3(v);
+    return {__builtin_shufflevector(t.h, t.h, 0, 1, 2, 3), __builtin_shufflevector(t.m, t.m, 0, 1, 2, 3), __builtin_shufflevector(t.l, t.l, 0, 1, 2, 3)};
 }
+__device__ __forceinline__ f32x4 mul_low(const Terms4& a, const Terms4& b, f32x4 c) {
+    c = mfma_16x16x32(join8(a.m, a.h), join8(b.m, b.l), c);
+    return mfma_16x16x32(join8(a.h, a.l), join8(b.m, b.h), c);
+}
+__device__ __forceinline__ f32x4 mul_high(const Terms4& a, const Terms4& b, f32x4 c) { return mfma_16x16x32(join8(a.h, a.m), join8(b.h, b.h), c); }
 
 template <int D, int MODE>
-__global__ void __launch_bounds__(64 * kCW, 1) chunk_scan_kernel(const ChunkScan a) {
+__global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) chunk_scan_kernel(const ChunkScan a) {
+    using M = ChunkLds<D, MODE>;
+    constexpr bool DELTA = MODE == kScanDelta, MLSTM = MODE == kScanMlstm;
     constexpr int NW = kCW, CPR = D / 8, VC = 2 * NW, KK = D / 32;   // 16-byte pieces per row of q and k, of v; 32-row steps of the state
-    constexpr int QB = kCH * D * 2, VB = kCH * VC * 16, BUF = 2 * QB + VB;
     extern __shared__ __attribute__((aligned(1024))) unsigned char cs_smem[];
-    f32x4* const pt = reinterpret_cast<f32x4*>(cs_smem + 2 * BUF);                 // weight tiles, [10][64 lanes]
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, ln = lane & 15, g = lane >> 4;
-    unsigned char* const own = cs_smem + 2 * BUF + 10 * 1024 + wv * (kCH * 16);     // the wave's own copy of the scalars
+    f32x4* const pt = reinterpret_cast<f32x4*>(cs_smem + M::PT);
+    f32x4* const at = reinterpret_cast<f32x4*>(cs_smem + M::AT);
+    f32x4* const tt = reinterpret_cast<f32x4*>(cs_smem + M::TT);
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = lane & 15, g = lane >> 4;
+    unsigned char* const own = cs_smem + M::OWN + wv * M::OWN_SIZE;
     double* const Ls = reinterpret_cast<double*>(own);
     float* const ws = reinterpret_cast<float*>(own + kCH * 8);
     float* const cs = ws + kCH;
-    float* const psum = reinterpret_cast<float*>(cs_smem + 2 * BUF + 10 * 1024 + NW * (kCH * 16));   // [10][16]
-    float* const nq = psum + 160;                                                                    // [NW][64]
+    float *const bs = cs + kCH, *const bk = bs + kCH, *const be = bk + kCH;            // delta
+    float* const psum = reinterpret_cast<float*>(cs_smem + M::SUM);                    // mlstm
+    float* const nq = psum + 160;
     // groups of workgroups that share q and k rows go to one XCD (workgroup i runs on XCD i % 8)
     const int nslab = (a.Dv + 16 * NW - 1) / (16 * NW), id = blockIdx.x >> 3;
     const int group = (id / nslab) * 8 + (blockIdx.x & 7), slab = id % nslab;
@@ -137,9 +181,9 @@ __global__ void __launch_bounds__(64 * kCW, 1) chunk_scan_kernel(const ChunkScan
 #pragma unroll
         for (int r = 0; r < 4; ++r) S[i][r] = !fresh && live ? Sp[(int64_t)((i >> 1) * 32 + 8 * g + 4 * (i & 1) + r) * a.Dv] : 0.f;
     // mlstm: the normaliser n likewise, the 32-row steps dealt to the waves (every column of the accumulator the same)
-    constexpr int NO = MODE == kScanMlstm ? (KK + NW - 1) / NW : 1;
+    constexpr int NO = MLSTM ? (KK + NW - 1) / NW : 1;
     f32x4 nst[2 * NO];
-    if constexpr (MODE == kScanMlstm) {
+    if constexpr (MLSTM) {
 #pragma unroll
         for (int i = 0; i < 2 * NO; ++i)
 #pragma unroll
@@ -153,32 +197,46 @@ __global__ void __launch_bounds__(64 * kCW, 1) chunk_scan_kernel(const ChunkScan
     const uint16_t* const vp = a.proj + a.v_off + (int64_t)hd * a.Dv + c0;
     const int vn = min(VC, (a.Dv - c0) / 8);
     const uint32_t lds0 = lds_offset(cs_smem);
+    // A chunk's rows into buffer `buf`: pieces wv, wv + NW, .. of each operand, 64 / CPR rows each.  Rows past the last token
+    // repeat it (their weights are 0), columns past Dv the last ones (not stored).
     auto fetch = [&](int tb, int buf) {
-        const int64_t at = (int64_t)tb * a.ldp;
         const int last = t1 - 1 - tb;
-        const uint32_t dst = lds0 + buf * BUF;
-        for (int j = wv; j < 2 * CPR + VC; j += NW) {
-            if (j < CPR) dma_tile<CPR>(qp + at, a.ldp, last, CPR, j, dst, lane);
-            else if (j < 2 * CPR) dma_tile<CPR>(kp + at, a.ldp, last, CPR, j - CPR, dst + QB, lane);
-            else dma_tile<VC>(vp + at, a.ldp, last, vn, j - 2 * CPR, dst + 2 * QB, lane);
+        const uint32_t dst = lds0 + buf * M::BUF;
+        const uint16_t *const q = qp + (int64_t)tb * a.ldp, *const k = kp + (int64_t)tb * a.ldp, *const v = vp + (int64_t)tb * a.ldp;
+#pragma unroll
+        for (int u = 0; u < (CPR + NW - 1) / NW; ++u) {
+            const int j = wv + NW * u, i = j * 64 + lane, row = i / CPR, c = (i % CPR) ^ spread<CPR>(row);
+            if (CPR % NW == 0 || j < CPR) {
+                const int64_t at = (int64_t)min(row, last) * a.ldp + c * 8;
+                dma_1k(q + at, __builtin_amdgcn_readfirstlane(dst + j * 1024));
+                dma_1k(k + at, __builtin_amdgcn_readfirstlane(dst + M::Q + j * 1024));
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < VC / NW; ++u) {
+            const int j = wv + NW * u, i = j * 64 + lane, row = i / VC, c = (i % VC) ^ spread<VC>(row);
+            dma_1k(v + (int64_t)min(row, last) * a.ldp + min(c, vn - 1) * 8, __builtin_amdgcn_readfirstlane(dst + 2 * M::Q + j * 1024));
         }
     };
     // the scalars of token tb + lane, as loaded; past the range: nothing decays, nothing is written
-    float sd = 1.f, sw = 0.f, sr = 0.f;
-    const float fixed = MODE == kScanPlain && a.dts == 0 ? a.decay[hd] : 1.f;
+    float sd = 1.f, sw = 0.f, sr = 0.f, sb = 0.f;
+    const float fixed = !MLSTM && a.dts == 0 ? a.decay[hd] : 1.f;
     auto scalars = [&](int tb) {
         const int64_t t = min(tb + lane, t1 - 1);
-        if constexpr (MODE == kScanMlstm) {
+        if constexpr (MLSTM) {
             sd = a.la[t * a.H + hd];
             sw = a.lb[t * a.H + hd];
             sr = a.em[t * a.H + hd];
         } else {
             sd = a.dts != 0 ? a.decay[t * a.dts + hd] : fixed;
             sw = a.kscale != nullptr ? a.kscale[t * a.HK + hk] : 1.f;
-            if (a.vscale != nullptr) sw *= a.vscale[t * a.H + hd];
+            if (!DELTA && a.vscale != nullptr) sw *= a.vscale[t * a.H + hd];
             sr = a.qscale != nullptr ? a.qscale[t * a.HK + hk] : a.q_mul;
+            if constexpr (DELTA) sb = a.beta[t * a.H + hd];
         }
     };
+    // stores of the read-out: past the chunk's last token and past Dv the descriptor's range drops them
+    const uint32_t orow = (uint32_t)a.H * a.Dv * 4, ocol = live ? (uint32_t)col * 4 : 0x80000000u;
     fetch(t0, 0);
     scalars(t0);
     for (int tb = t0, buf = 0; tb < t1; tb += kCH, buf ^= 1) {
@@ -188,70 +246,125 @@ __global__ void __launch_bounds__(64 * kCW, 1) chunk_scan_kernel(const ChunkScan
         const bool valid = lane < nt;
         double L = 0.0;
         float w = 0.f;
-        const float rd = sr;
+        float rd = sr, gC = 1.f;   // gC: the sign of the product of the chunk's decays
         if (valid) {
-            if constexpr (MODE == kScanMlstm) {
+            if constexpr (MLSTM) {
                 L = sd;
                 w = expf(sw);
             } else {
-                const float lg = logf(sd);
+                const float lg = logf(fabsf(sd));
                 L = lg < -110.f ? -110.f : lg;   // e^-110 is 0 in float32, as a decay of 0 is
                 w = sw;
             }
         }
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const double up = __shfl_up(L, o, 64);
-            if (lane >= o) L += up;
+        if constexpr (!MLSTM) {   // the sign of a product of decays up to t goes with what t writes and reads
+            const uint64_t neg = __ballot(valid && sd < 0.f);
+            if (__popcll(neg & (~0ull >> (63 - lane))) & 1) {
+                w = -w;
+                rd = -rd;
+            }
+            if (__popcll(neg) & 1) gC = -1.f;
         }
-        const double LC = __shfl(L, 63, 64);
+        L = lanes_running_sum(L);
+        const double LC = __builtin_bit_cast(double, (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(__builtin_bit_cast(uint64_t, L) >> 32), 63) << 32 |
+                                                         (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)__builtin_bit_cast(uint64_t, L), 63));
+        const float eL = exp_d(L);
         Ls[lane] = L;
         ws[lane] = w;
-        cs[lane] = exp_d(LC - L) * w;
-        __builtin_amdgcn_wave_barrier();
+        cs[lane] = gC * exp_d(LC - L) * w;
+        if constexpr (DELTA) {
+            const float bt = valid ? sb : 0.f;
+            bs[lane] = bt;
+            bk[lane] = bt * w;
+            be[lane] = bt * w * eL;
+        }
         __syncthreads();   // this chunk's rows are in LDS; nobody reads the other buffer or the last chunk's weights any more
         if (tb + kCH < t1) {
             fetch(tb + kCH, buf ^ 1);
             scalars(tb + kCH);
         }
-        const unsigned char* const qb = cs_smem + buf * BUF;
-        const unsigned char* const kb = qb + QB;
-        const unsigned char* const vb = kb + QB;
+        const unsigned char* const qb = cs_smem + buf * M::BUF;
+        const unsigned char* const kb = qb + M::Q;
+        const unsigned char* const vb = kb + M::Q;
         // rows 16 i + ln of q or k, columns 32 kk + 8 g ..: either operand of a product over columns
+        const int sp = spread<CPR>(ln);
         auto row8 = [&](const unsigned char* base, int i, int kk) {
-            const int r = 16 * i + ln;
-            return *reinterpret_cast<const bf16x8*>(base + r * (D * 2) + (((kk * 4 + g) ^ spread<CPR>(r)) * 16));
+            return *reinterpret_cast<const bf16x8*>(base + (16 * i + ln) * (D * 2) + (((kk * 4 + g) ^ sp) * 16));
         };
         // k rows 32 p + 4 g + (0..3), 32 p + 16 + 4 g + (0..3), column 32 kk + 8 (ln / 4) + 4 h + ln % 4: the update's left operand
+        const int r4 = 4 * g + (ln >> 2), sp4 = spread<CPR>(r4);
         auto kcol8 = [&](int p, int kk, int h) {
-            const int r = 32 * p + 4 * g + (ln >> 2), c = ((kk * 4 + (ln & 3)) ^ spread<CPR>(r)) * 16 + h * 8;
-            return join8(lds_read_tr4(kb + r * (D * 2) + c), lds_read_tr4(kb + (r + 16) * (D * 2) + c));   // (spread: period 16)
+            const unsigned char* at = kb + (32 * p + r4) * (D * 2) + ((kk * 4 + (ln & 3)) ^ sp4) * 16 + h * 8;
+            return join8(lds_read_tr4(at), lds_read_tr4(at + 16 * (D * 2)));
         };
-        // ---- weights: tile p = (i, j) holds rows s = 16 j.. (4 g + r) and columns t = 16 i.. (ln)
-        for (int p = wv; p < 10; p += NW) {
-            const int i = p < 1 ? 0 : p < 3 ? 1 : p < 6 ? 2 : 3, j = p - i * (i + 1) / 2;
-            if (16 * i >= nt) continue;
+        // ---- weights: tile (i, j) holds rows s = 16 j.. (4 g + r) and columns t = 16 i.. (ln)
+        auto product = [&](const unsigned char* tbase, int i, int j) {
+            bf16x8 x[KK], y[KK];
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) { x[kk] = row8(kb, j, kk); y[kk] = row8(tbase, i, kk); }
             f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-            for (int kk = 0; kk < KK; ++kk) acc[kk & 1] = mfma_16x16x32(row8(kb, j, kk), row8(qb, i, kk), acc[kk & 1]);
+            for (int kk = 0; kk < KK; ++kk) acc[kk & 1] = mfma_16x16x32(x[kk], y[kk], acc[kk & 1]);
+            f32x4 v = acc[0];
+            if (KK > 1) v += acc[1];
+            // times e^(L_t - L_s) w_s, for s <= t
             const int t = 16 * i + ln;
             const double Lt = Ls[t];
-            f32x4 v;
-            float sum = 0.f;
+            const f32x4 wsv = *reinterpret_cast<const f32x4*>(ws + 16 * j + 4 * g);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int s = 16 * j + 4 * g + r;
-                v[r] = s <= t ? (acc[0][r] + acc[1][r]) * (ws[s] * exp_d(Lt - Ls[s])) : 0.f;
-                sum += v[r];
+                v[r] = s <= t ? v[r] * (wsv[r] * exp_d(Lt - Ls[s])) : 0.f;
             }
+            return v;
+        };
+        const int nrow = (nt + 15) / 16;   // 16-token rows of tiles that hold tokens
+        for (int p = wv; p < 10; p += NW) {
+            const int i = p < 1 ? 0 : p < 3 ? 1 : p < 6 ? 2 : 3, j = p - i * (i + 1) / 2;
+            if (i >= nrow) continue;
+            const f32x4 v = product(qb, i, j);
             pt[p * 64 + lane] = v;
-            if constexpr (MODE == kScanMlstm) {
+            if constexpr (MLSTM) {
+                float sum = (v[0] + v[1]) + (v[2] + v[3]);
                 sum += __shfl_xor(sum, 16, 64);
                 sum += __shfl_xor(sum, 32, 64);
                 if (g == 0) psum[p * 16 + ln] = sum;
             }
         }
-        if constexpr (MODE == kScanMlstm) {   // n . q of the state before the chunk, this wave's rows
+        if constexpr (DELTA) {
+            // -A, A[t, s] = beta_t k-scale_t k-scale_s e^(L_t - L_s) (k_t . k_s) for s < t: wave w the tiles of column w below the
+            // diagonal, and the diagonal one's (I + A)^-1 by forward substitution, lane n column n
+            for (int i = wv; i < nrow; ++i) {
+                const int p = i * (i + 1) / 2 + wv, t = 16 * i + ln;
+                f32x4 v = product(kb, i, wv);
+                const float f = -bk[t];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = 16 * wv + 4 * g + r < t ? v[r] * f : 0.f;
+                at[p * 64 + lane] = v;
+                if (i == wv) {
+                    __builtin_amdgcn_wave_barrier();   // the wave's own writes
+                    float x[16];
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        float acc[4] = {r == ln ? 1.f : 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int q = 0; q < (r + 3) / 4; ++q) {
+                            const f32x4 row = at[p * 64 + q * 16 + r];   // -A[r][4 q ..]
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                                if (4 * q + e < r) acc[e] += row[e] * x[4 * q + e];
+                        }
+                        x[r] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+                    }
+                    float* out = reinterpret_cast<float*>(tt + wv * 64);   // operand layout: lane (t, g) holds columns 4 g ..
+                    if (g == 0) {
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) out[((ln >> 2) * 16 + r) * 4 + (ln & 3)] = r == ln ? 0.f : x[r];   // less the identity
+                    }
+                }
+            }
+        }
+        if constexpr (MLSTM) {   // n . q of the state before the chunk, this wave's rows
             f32x4 acc[4] = {};
 #pragma unroll
             for (int u = 0; u < NO; ++u) {
@@ -260,11 +373,15 @@ __global__ void __launch_bounds__(64 * kCW, 1) chunk_scan_kernel(const ChunkScan
                     const float x[8] = {nst[2 * u][0], nst[2 * u][1], nst[2 * u][2], nst[2 * u][3],
                                         nst[2 * u + 1][0], nst[2 * u + 1][1], nst[2 * u + 1][2], nst[2 * u + 1][3]};
                     const Terms n = split3(x);
+                    bf16x8 q[4];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const bf16x8 q = row8(qb, i, kk);
-                        acc[i] = mfma_16x16x32(q, n.h, mfma_16x16x32(q, n.m, mfma_16x16x32(q, n.l, acc[i])));
-                    }
+                    for (int i = 0; i < 4; ++i) q[i] = row8(qb, i, kk);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[i] = mfma_16x16x32(q[i], n.l, acc[i]);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[i] = mfma_16x16x32(q[i], n.m, acc[i]);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[i] = mfma_16x16x32(q[i], n.h, acc[i]);
                 }
             }
             if (ln == 0) {
@@ -273,9 +390,8 @@ __global__ void __launch_bounds__(64 * kCW, 1) chunk_scan_kernel(const ChunkScan
             }
         }
         __syncthreads();   // the weights are there
-        const float eL = exp_d(L);
         float fr = rd;
-        if constexpr (MODE == kScanMlstm) {
+        if constexpr (MLSTM) {
             const int i = lane >> 4, p0 = i * (i + 1) / 2;
             float intra = 0.f, inter = 0.f;
             for (int j = 0; j <= i; ++j) intra += psum[(p0 + j) * 16 + ln];
@@ -283,86 +399,160 @@ __global__ void __launch_bounds__(64 * kCW, 1) chunk_scan_kernel(const ChunkScan
             for (int u = 0; u < NW; ++u) inter += nq[u * kCH + lane];
             fr = a.q_mul / (fmaxf(fabsf((intra + eL * inter) * a.q_mul), rd) + 1e-6f);
         }
-        // ---- read-out: state before the chunk, then the chunk's own tokens
-        Terms st[KK];
+        const float eC = gC * exp_d(LC);
+        // ---- read-out and the state after the chunk, NI rows of tiles
+        auto rest = [&](auto ni) {
+            constexpr int NI = decltype(ni)::value;
+            bf16x8 v[NI / 2];   // v rows 32 p + 4 g + (0..3), 32 p + 16 + 4 g + (0..3) of this lane's column
 #pragma unroll
-        for (int kk = 0; kk < KK; ++kk) {
-            const float x[8] = {S[2 * kk][0], S[2 * kk][1], S[2 * kk][2], S[2 * kk][3],
-                                S[2 * kk + 1][0], S[2 * kk + 1][1], S[2 * kk + 1][2], S[2 * kk + 1][3]};
-            st[kk] = split3(x);
-        }
-        bf16x8 v[2];   // v rows 32 p + 4 g + (0..3), 32 p + 16 + 4 g + (0..3) of this lane's column
+            for (int p = 0; p < NI / 2; ++p) {
+                const unsigned char* at = vb + (32 * p + r4) * (VC * 16) + ((wv * 2 + ((ln & 3) >> 1)) ^ spread<VC>(r4)) * 16 + (ln & 1) * 8;
+                v[p] = join8(lds_read_tr4(at), lds_read_tr4(at + 16 * (VC * 16)));
+            }
+            // the state before the chunk times q (delta: and k), a 32-row step of it at a time
+            f32x4 oq[NI], ok[NI];
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
-            const int r = 32 * p + 4 * g + (ln >> 2), c = ((wv * 2 + ((ln & 3) >> 1)) ^ spread<VC>(r)) * 16 + (ln & 1) * 8;
-            v[p] = join8(lds_read_tr4(vb + r * (VC * 16) + c), lds_read_tr4(vb + (r + 16) * (VC * 16) + c));
-        }
+            for (int i = 0; i < NI; ++i) oq[i] = ok[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            if (16 * i < nt) {
-                f32x4 ah = {0.f, 0.f, 0.f, 0.f}, am = ah, al = ah;
+            for (int kk = 0; kk < KK; ++kk) {
+                bf16x8 q[NI], k[NI];
 #pragma unroll
-                for (int kk = 0; kk < KK; ++kk) {
-                    const bf16x8 q = row8(qb, i, kk);
-                    ah = mfma_16x16x32(q, st[kk].h, ah);
-                    am = mfma_16x16x32(q, st[kk].m, am);
-                    al = mfma_16x16x32(q, st[kk].l, al);
+                for (int i = 0; i < NI; ++i) {
+                    q[i] = row8(qb, i, kk);
+                    if constexpr (DELTA) k[i] = row8(kb, i, kk);
                 }
-                f32x4 acc;
+                const float x[8] = {S[2 * kk][0], S[2 * kk][1], S[2 * kk][2], S[2 * kk][3],
+                                    S[2 * kk + 1][0], S[2 * kk + 1][1], S[2 * kk + 1][2], S[2 * kk + 1][3]};
+                const Terms st = split3(x);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) acc[r] = (ah[r] + (am[r] + al[r])) * __shfl(eL, 16 * i + 4 * g + r, 64);
+                for (int c = 0; c < 3; ++c) {
+                    const bf16x8 term = c == 0 ? st.l : c == 1 ? st.m : st.h;
 #pragma unroll
-                for (int p = 0; p <= i / 2; ++p) {
-                    const f32x4 x0 = pt[(i * (i + 1) / 2 + 2 * p) * 64 + lane];
-                    f32x4 x1 = {0.f, 0.f, 0.f, 0.f};
-                    if (2 * p + 1 <= i) x1 = pt[(i * (i + 1) / 2 + 2 * p + 1) * 64 + lane];
-                    const float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
-                    const Terms w3 = split3(x);
-                    acc = mfma_16x16x32(w3.h, v[p], mfma_16x16x32(w3.m, v[p], mfma_16x16x32(w3.l, v[p], acc)));
-                }
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int t = 16 * i + 4 * g + r;
-                    const float f = __shfl(fr, t, 64);
-                    if (t < nt && live) a.o[((int64_t)(tb + t) * a.H + hd) * a.Dv + col] = acc[r] * f;
+                    for (int i = 0; i < NI; ++i) {
+                        oq[i] = mfma_16x16x32(q[i], term, oq[i]);
+                        if constexpr (DELTA) ok[i] = mfma_16x16x32(k[i], term, ok[i]);
+                    }
                 }
             }
-        }
-        // ---- the state after the chunk
-        const float eC = exp_d(LC);
+            float el[NI][4], fo[NI][4];
 #pragma unroll
-        for (int i = 0; i < 2 * KK; ++i) S[i] *= eC;
-        if constexpr (MODE == kScanMlstm) {
+            for (int i = 0; i < NI; ++i)
 #pragma unroll
-            for (int i = 0; i < 2 * NO; ++i) nst[i] *= eC;
-        }
+                for (int r = 0; r < 4; ++r) {
+                    el[i][r] = __shfl(eL, 16 * i + 4 * g + r, 64);
+                    fo[i][r] = __shfl(fr, 16 * i + 4 * g + r, 64);
+                    oq[i][r] *= el[i][r];
+                }
+            f32x4 U[NI];   // what the chunk's tokens write, before the scales
+            if constexpr (DELTA) {
+                // (I + A) U = beta (v - e^L k-scale S^T k), 16 rows at a time
+                Terms4 ut[NI];
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
-            if (32 * p >= nt) break;
-            const f32x4 f0 = *reinterpret_cast<const f32x4*>(cs + 32 * p + 4 * g);
-            const f32x4 f1 = *reinterpret_cast<const f32x4*>(cs + 32 * p + 16 + 4 * g);
-            const float f[8] = {f0[0], f0[1], f0[2], f0[3], f1[0], f1[1], f1[2], f1[3]};
-            float x[8];
+                for (int i = 0; i < NI; ++i) {
+                    const f32x4 b0 = *reinterpret_cast<const f32x4*>(bs + 16 * i + 4 * g), b1 = *reinterpret_cast<const f32x4*>(be + 16 * i + 4 * g);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = f[e] * (float)v[p][e];
-            const Terms u = split3(x);
-            Terms un;
-            if constexpr (MODE == kScanMlstm) un = split3(f);
+                    for (int r = 0; r < 4; ++r) {
+                        const float p = b1[r] * ok[i][r];
+                        U[i][r] = b0[r] * (float)v[i / 2][4 * (i & 1) + r] - p;
+                        ok[i][r] = -__builtin_fmaf(b1[r], ok[i][r], -p);   // what rounding p and the sum below took, for the last sum
+                    }
+                }
 #pragma unroll
-            for (int kk = 0; kk < KK; ++kk)
+                for (int i = 0; i < NI; ++i) {
+                    if (i > 0 && i >= nrow) {   // (rows without tokens: nothing)
+                        ut[i] = split3(U[i]);
+                        continue;
+                    }
+// the small products first, and all of them before they meet the sum: one rounding at its size
+                    if (i > 0) {
+                        Terms4 w[NI];
+                        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const bf16x8 kc = kcol8(p, kk, h);
-                    f32x4& s = S[2 * kk + h];
-                    s = mfma_16x16x32(kc, u.h, mfma_16x16x32(kc, u.m, mfma_16x16x32(kc, u.l, s)));
-                    if constexpr (MODE == kScanMlstm) {
-                        if (kk % NW == wv) {
-                            f32x4& nn = nst[2 * (kk / NW) + h];
-                            nn = mfma_16x16x32(kc, un.h, mfma_16x16x32(kc, un.m, mfma_16x16x32(kc, un.l, nn)));
+                        for (int j = 0; j < i; ++j) acc = mul_low(w[j] = split3(at[(i * (i + 1) / 2 + j) * 64 + lane]), ut[j], acc);
+#pragma unroll
+                        for (int j = 0; j < i; ++j) acc = mul_high(w[j], ut[j], acc);
+                        const f32x4 sum = U[i] + acc, part = sum - U[i];
+                        ok[i] += (U[i] - (sum - part)) + (acc - part);
+                        U[i] = sum;
+                    }
+                    const Terms4 w = split3(tt[i * 64 + lane]), u = split3(U[i]);
+                    U[i] += mul_high(w, u, mul_low(w, u, ok[i]));
+                    ut[i] = split3(U[i]);
+                }
+#pragma unroll
+                for (int i = 0; i < NI; ++i) {
+                    if (i > 0 && i >= nrow) continue;
+                    Terms4 w[NI];
+                    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int j = 0; j <= i; ++j) acc = mul_low(w[j] = split3(pt[(i * (i + 1) / 2 + j) * 64 + lane]), ut[j], acc);
+#pragma unroll
+                    for (int j = 0; j <= i; ++j) acc = mul_high(w[j], ut[j], acc);
+                    oq[i] += acc;
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < NI; ++i)
+#pragma unroll
+                    for (int p = 0; p <= i / 2; ++p) {
+                        const f32x4 x0 = pt[(i * (i + 1) / 2 + 2 * p) * 64 + lane];
+                        f32x4 x1 = {0.f, 0.f, 0.f, 0.f};
+                        if (2 * p + 1 <= i) x1 = pt[(i * (i + 1) / 2 + 2 * p + 1) * 64 + lane];
+                        const float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+                        const Terms w3 = split3(x);
+                        oq[i] = mfma_16x16x32(w3.h, v[p], mfma_16x16x32(w3.m, v[p], mfma_16x16x32(w3.l, v[p], oq[i])));
+                    }
+            }
+            const auto ord = __builtin_amdgcn_make_buffer_rsrc(a.o + ((int64_t)tb * a.H + hd) * a.Dv, (short)0, (int)(nt * orow), 0x00020000);
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(oq[i][r] * fo[i][r]), ord, ocol + (16 * i + 4 * g + r) * orow, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 2 * KK; ++i) S[i] *= eC;
+            if constexpr (MLSTM) {
+#pragma unroll
+                for (int i = 0; i < 2 * NO; ++i) nst[i] *= eC;
+            }
+#pragma unroll
+            for (int p = 0; p < NI / 2; ++p) {
+                const f32x4 f0 = *reinterpret_cast<const f32x4*>(cs + 32 * p + 4 * g);
+                const f32x4 f1 = *reinterpret_cast<const f32x4*>(cs + 32 * p + 16 + 4 * g);
+                const float f[8] = {f0[0], f0[1], f0[2], f0[3], f1[0], f1[1], f1[2], f1[3]};
+                float x[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = f[e] * (DELTA ? U[2 * p + (e >> 2)][e & 3] : (float)v[p][e]);
+                const Terms u = split3(x);
+                Terms un;
+                if constexpr (MLSTM) un = split3(f);
+#pragma unroll
+                for (int k2 = 0; k2 < KK; k2 += 2) {   // four tiles of the state at a time
+                    constexpr int NT = KK > 1 ? 4 : 2;
+                    bf16x8 kc[NT];
+#pragma unroll
+                    for (int y = 0; y < NT; ++y) kc[y] = kcol8(p, k2 + (y >> 1), y & 1);
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        const bf16x8 term = c == 0 ? u.l : c == 1 ? u.m : u.h;
+#pragma unroll
+                        for (int y = 0; y < NT; ++y) S[2 * k2 + y] = mfma_16x16x32(kc[y], term, S[2 * k2 + y]);
+                    }
+                    if constexpr (MLSTM) {
+#pragma unroll
+                        for (int y = 0; y < NT; ++y) {
+                            const int kk = k2 + (y >> 1);
+                            if (kk % NW == wv) {
+                                f32x4& nn = nst[2 * (kk / NW) + (y & 1)];
+                                nn = mfma_16x16x32(kc[y], un.h, mfma_16x16x32(kc[y], un.m, mfma_16x16x32(kc[y], un.l, nn)));
+                            }
                         }
                     }
                 }
-        }
+            }
+        };
+        if (nt > 32) rest(std::integral_constant<int, 4>{});
+        else rest(std::integral_constant<int, 2>{});
     }
     if (live) {
 #pragma unroll
@@ -370,7 +560,7 @@ __global__ void __launch_bounds__(64 * kCW, 1) chunk_scan_kernel(const ChunkScan
 #pragma unroll
             for (int r = 0; r < 4; ++r) Sp[(int64_t)((i >> 1) * 32 + 8 * g + 4 * (i & 1) + r) * a.Dv] = S[i][r];
     }
-    if constexpr (MODE == kScanMlstm) {
+    if constexpr (MLSTM) {
         if (slab == 0 && ln == 0) {
 #pragma unroll
             for (int i = 0; i < 2 * NO; ++i)
@@ -442,16 +632,17 @@ __global__ void __launch_bounds__(256) mlstm_gates_kernel(const float* __restric
 // When the chunked form serves a launch: bfloat16 rows of q, k and v on 16-byte boundaries, a state of 32, 64, 128 or 256
 // rows, and a sequence with at least 16 new tokens (longest: the most that any sequence brings).  A chunk costs the same
 // whether it is full or not, the token-by-token kernels cost per token: 32 sequences of n tokens take (token by token /
-// chunked, us) 9.9 / 16.5 at n = 4, 11.7 / 16.4 at 8, 15.9 / 16.1 at 16, 71.5 / 39.3 at 117 (8 heads of 128 x 128, fixed
-// decays), and 50 / 68, 61 / 67, 85 / 67, 444 / 144 (mlstm, 4 heads of 256 x 512).
-bool hy_chunk_scan_ok(const void* proj, int ldp, int q_off, int k_off, int v_off, int D, int Dv, int longest) {
-    return longest >= 16 && (D == 32 || D == 64 || D == 128 || D == 256) && Dv % 8 == 0 && ((uintptr_t)proj & 15) == 0 &&
-           ((ldp | q_off | k_off | v_off) & 7) == 0;
+// chunked, us) 10.7 / 15.5 at n = 4, 12.5 / 15.6 at 8, 17.1 / 15.4 at 16, 71 / 33 at 117 (8 heads of 128 x 128, fixed decays),
+// 50 / 68, 61 / 67, 87 / 56, 443 / 105 (mlstm, 4 heads of 256 x 512), and with the delta rule (16 heads of
+// 128 x 128) 35 / 38 at 16, 57 / 44 at 32, 179 / 111 at 117.  The delta rule's tiles leave no room for D = 256.
+bool hy_chunk_scan_ok(const void* proj, int ldp, int q_off, int k_off, int v_off, int D, int Dv, int longest, bool delta) {
+    return longest >= (delta ? 32 : 16) && (D == 32 || D == 64 || D == 128 || (D == 256 && !delta)) && Dv % 8 == 0 && ((uintptr_t)proj & 15) == 0 &&
+           ((ldp | q_off | k_off | v_off) & 7) == 0 && ldp < 1 << 23;   // (64 rows of o, no wider than proj's, within 2^31 bytes)
 }
 
 template <int D, int MODE>
 static void chunk_scan_run(const hy::ChunkScan& a, hipStream_t s) {
-    constexpr int lds = hy::chunk_scan_lds<D>();
+    constexpr int lds = hy::ChunkLds<D, MODE>::SIZE;
     static_assert(lds <= 160 * 1024, "LDS of one workgroup");
     const auto kern = hy::chunk_scan_kernel<D, MODE>;
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -464,17 +655,19 @@ static void chunk_scan_d(int D, const hy::ChunkScan& a, hipStream_t s) {
     if (D == 32) chunk_scan_run<32, MODE>(a, s);
     else if (D == 64) chunk_scan_run<64, MODE>(a, s);
     else if (D == 128) chunk_scan_run<128, MODE>(a, s);
-    else chunk_scan_run<256, MODE>(a, s);
+    else if constexpr (MODE != hy::kScanDelta) chunk_scan_run<256, MODE>(a, s);   // (delta: its tiles do not fit the LDS beside)
 }
 
-// One decay per head and token (dts = H) or per head (dts = 0), no delta correction; see launch_hy_linear_scan.
+// One decay per head and token (dts = H) or per head (dts = 0), with beta the delta correction (D <= 128); see
+// launch_hy_linear_scan.
 void launch_hy_chunk_scan(const uint16_t* proj, int ldp, int q_off, int k_off, int v_off, const float* qscale, const float* kscale,
-                          float q_mul, const float* decay, int dts, const int32_t* q_start, const int32_t* pos0,
-                          const int32_t* slots, float* S, float* o, int B, int HK, int H, int D, int Dv, const float* vscale,
+                          float q_mul, const float* decay, int dts, const float* beta, const int32_t* q_start,
+                          const int32_t* pos0, const int32_t* slots, float* S, float* o, int B, int HK, int H, int D, int Dv, const float* vscale,
                           hipStream_t s) {
-    hy::ChunkScan a{proj, ldp, q_off, k_off, v_off, qscale, kscale, vscale, decay, dts, q_mul, nullptr, nullptr, nullptr,
+    hy::ChunkScan a{proj, ldp, q_off, k_off, v_off, qscale, kscale, vscale, decay, beta, dts, q_mul, nullptr, nullptr, nullptr,
                     q_start, pos0, slots, nullptr, S, nullptr, o, B, HK, H, Dv};
-    chunk_scan_d<hy::kScanPlain>(D, a, s);
+    if (beta != nullptr) chunk_scan_d<hy::kScanDelta>(D, a, s);
+    else chunk_scan_d<hy::kScanPlain>(D, a, s);
 }
 
 // scratch: 3 T H + B H D floats
@@ -484,7 +677,7 @@ void launch_hy_chunk_mlstm(const uint16_t* proj, int ldp, const float* gate_pre,
     const int64_t th = (int64_t)T * H;
     float *la = scratch, *lb = la + th, *em = lb + th, *n0 = em + th;
     hy::mlstm_gates_kernel<<<dim3(B, H), 256, 0, s>>>(gate_pre, q_start, pos0, slots, n, m, n0, la, lb, em, H, D, cap);
-    hy::ChunkScan a{proj, ldp, 0, H * D, 2 * H * D, nullptr, nullptr, nullptr, nullptr, H, 1.f / sqrtf((float)D), la, lb, em,
+    hy::ChunkScan a{proj, ldp, 0, H * D, 2 * H * D, nullptr, nullptr, nullptr, nullptr, nullptr, H, 1.f / sqrtf((float)D), la, lb, em,
                     q_start, pos0, slots, n0, S, n, o, B, H, H, Dv};
     chunk_scan_d<hy::kScanMlstm>(D, a, s);
 }

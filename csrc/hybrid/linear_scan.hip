@@ -414,9 +414,9 @@ __global__ void __launch_bounds__(256) linear_scan_kernel(
 
 }  // namespace hy
 
-bool hy_chunk_scan_ok(const void*, int, int, int, int, int, int, int);
+bool hy_chunk_scan_ok(const void*, int, int, int, int, int, int, int, bool);
 void launch_hy_chunk_scan(const uint16_t*, int, int, int, int, const float*, const float*, float, const float*, int,
-                          const int32_t*, const int32_t*, const int32_t*, float*, float*, int, int, int, int, int, const float*,
+                          const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*, int, int, int, int, int, const float*,
                           hipStream_t);
 
 // x points at the first convolved column of the first row (rows ldx apart); bias may be nullptr
@@ -510,8 +510,8 @@ bool launch_hy_linear_scan(const void* proj, int ldp, int q_off, int k_off, int 
     if (B == 0) return true;
     const bool pipe = T > B;   // some sequence brings more than one token
     const bool delta = beta != nullptr;
-    if (!delta && !chd && !f32 && hy_chunk_scan_ok(proj, ldp, q_off, k_off, v_off, D, Dv, longest)) {
-        launch_hy_chunk_scan((const uint16_t*)proj, ldp, q_off, k_off, v_off, qscale, kscale, q_mul, decay, fixed ? 0 : H,
+    if (!chd && !f32 && hy_chunk_scan_ok(proj, ldp, q_off, k_off, v_off, D, Dv, longest, delta)) {
+        launch_hy_chunk_scan((const uint16_t*)proj, ldp, q_off, k_off, v_off, qscale, kscale, q_mul, decay, fixed ? 0 : H, beta,
                              q_start, pos0, slots, S, o, B, HK, H, D, Dv, vscale, s);
         return true;
     }

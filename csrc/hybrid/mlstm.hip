@@ -431,7 +431,7 @@ static void mlstm_scan_t(const T* proj, int ldp, const float* gate_pre, const in
 #undef HY_SCAN
 }
 
-bool hy_chunk_scan_ok(const void*, int, int, int, int, int, int, int);
+bool hy_chunk_scan_ok(const void*, int, int, int, int, int, int, int, bool);
 void launch_hy_chunk_mlstm(const uint16_t*, int, const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*,
                            float*, float*, float*, int, int, int, int, int, float, hipStream_t);
 
@@ -440,7 +440,7 @@ void launch_hy_mlstm_scan(const void* proj, int ldp, const float* gate_pre, cons
                           const int32_t* slots, float* S, float* n, float* m, float* scratch, float* o, int T, int B, int H, int D,
                           int Dv, float cap, int longest, bool f32, hipStream_t s) {
     if (B == 0) return;
-    if (!f32 && hy_chunk_scan_ok(proj, ldp, 0, H * D, 2 * H * D, D, Dv, longest)) {
+    if (!f32 && hy_chunk_scan_ok(proj, ldp, 0, H * D, 2 * H * D, D, Dv, longest, false)) {
         launch_hy_chunk_mlstm((const uint16_t*)proj, ldp, gate_pre, q_start, pos0, slots, S, n, m, scratch, o, T, B, H, D, Dv, cap, s);
         return;
     }

@@ -1,6 +1,6 @@
 """The chunked forms of the linear-state recurrences (csrc/hybrid/chunk_scan.hip) against the token-by-token recurrence in
 float64, at the edges of a chunk (64 tokens) and of its 16-token tiles, with ranges that continue a state, with decays of 0
-and 1, and with column counts off the 64-column slabs.
+and 1, negative ones and ones above 1, and with column counts off the 64-column slabs.
 
 Tolerance: inputs are exact in both (bfloat16 and float32); what differs is float32 rounding, 2^-24 per operation, of
 sums over at most 129 tokens and 256 state rows and of one exponential per token.  Errors of independent roundings grow with the
@@ -42,7 +42,7 @@ def test_plain(HK, H, D, Dv, form):
         decay[0] = 1.0
     else:
         decay, vs = torch.exp(-2 * torch.rand(T, H, device=DEV, generator=g)), torch.rand(T, H, device=DEV, generator=g)
-        decay[3::50], decay[9::31], decay[11::37] = 0.0, 1e-30, 1.0
+        decay[3::50], decay[9::31], decay[11::37], decay[20::29], decay[23::61] = 0.0, 1e-30, 1.0, -0.8, 1.4
     qsc, ksc = torch.rand(T, HK, device=DEV, generator=g), torch.rand(T, HK, device=DEV, generator=g)
     S = rnd(9, H, D, Dv) * 0.3
     S0 = S.clone()
@@ -57,6 +57,52 @@ def test_plain(HK, H, D, Dv, form):
         s = torch.zeros(H, D, Dv, dtype=torch.double, device=DEV) if STARTS[b] == 0 else Sw[SLOTS[b]]
         for t in range(qs[b], qs[b] + n):
             s = dec[t][:, None, None] * s + k[t][:, :, None] * v[t][:, None]
+            want[t] = (q[t][:, None] @ s)[:, 0]
+        if n:
+            Sw[SLOTS[b]] = s
+    assert _rel(o, want) < 2e-6 and _rel(S, Sw) < 2e-6
+    assert torch.equal(S[1], S0[1]) and torch.equal(S[6], S0[6]), "slots without tokens must stay untouched"
+
+
+@pytest.mark.parametrize("HK,H,D,Dv,form", [(2, 4, 32, 40, "token"), (2, 2, 64, 64, "head"), (2, 4, 128, 72, "token"), (1, 3, 128, 128, "same")])
+def test_delta(HK, H, D, Dv, form):
+    """The delta rule's 16-row solves: keys of length 1, in "same" all nearly one direction with betas near 1 (every token undoes
+    most of the last one's write, the system is as far from the identity as it gets)."""
+    from chronos.ops import hybrid as hops
+
+    T = sum(LENS)
+    C = 2 * HK * D + H * Dv + 16
+    g, rnd, qs, ranges = _setup(H * D + Dv, T, C, H, D, Dv)
+    proj = rnd(T, C)
+    if form == "same":
+        proj[:, 8 + HK * D:8 + 2 * HK * D] = 3 * rnd(HK * D) + 0.1 * proj[:, 8 + HK * D:8 + 2 * HK * D]
+    proj = proj.bfloat16()
+    beta = torch.rand(T, H, device=DEV, generator=g)
+    if form == "same":
+        beta = 1 - 0.05 * beta
+    beta[5::23] = 0.0
+    if form == "head":
+        decay = 1 - torch.rand(H, device=DEV, generator=g) ** 4
+        decay[0] = 1.0
+    else:
+        decay = torch.exp(-0.3 * torch.rand(T, H, device=DEV, generator=g))
+        decay[3::50], decay[9::31], decay[11::37], decay[20::29], decay[23::61] = 0.0, 1e-30, 1.0, -0.8, 1.4
+    p = proj.double()
+    q, k = p[:, 8:8 + HK * D].view(T, HK, D), p[:, 8 + HK * D:8 + 2 * HK * D].view(T, HK, D)
+    qsc, ksc = (1 / q.norm(dim=-1)).float(), (1 / k.norm(dim=-1)).float()
+    S = rnd(9, H, D, Dv) * 0.3
+    S0 = S.clone()
+    o = hops.linear_scan(proj, 8, 8 + HK * D, 8 + 2 * HK * D, qsc, ksc, 1.0, decay, beta, *ranges, S, HK, H, D, Dv, max_q=max(LENS))
+    q = (q * qsc.double()[..., None]).repeat_interleave(H // HK, 1)
+    k = (k * ksc.double()[..., None]).repeat_interleave(H // HK, 1)
+    v, dec, bt = p[:, 8 + 2 * HK * D:8 + 2 * HK * D + H * Dv].view(T, H, Dv), decay.double().expand(T, H), beta.double()
+    want, Sw = torch.empty(T, H, Dv, dtype=torch.double, device=DEV), S0.double()
+    for b, n in enumerate(LENS):
+        s = torch.zeros(H, D, Dv, dtype=torch.double, device=DEV) if STARTS[b] == 0 else Sw[SLOTS[b]]
+        for t in range(qs[b], qs[b] + n):
+            s = dec[t][:, None, None] * s
+            u = bt[t][:, None] * (v[t] - (k[t][:, None] @ s)[:, 0])
+            s = s + k[t][:, :, None] * u[:, None]
             want[t] = (q[t][:, None] @ s)[:, 0]
         if n:
             Sw[SLOTS[b]] = s
