@@ -52,7 +52,9 @@ bool launch_gemm_lg_f8(int cfg, bool swiglu, const PPArgs& a, hipStream_t st);
 // skinny-M family (csrc/kernels/gemm_skinny.hip, M <= 16 * MT): same PPArgs / epilogues; the workgroup owns 16 * RT
 // W rows (swiglu: 8 * RT gate + 8 * RT up), ws holds [groups * splitk, 64 * RT * MT] f32x4 slabs, cnt one ticket per
 // group, kResid partials are [M, N / (16 * RT)]; K % (64 * NW * splitk) == 0
-constexpr int kSkinnyConfigs = 12;
+constexpr int kSkinnyConfigs = 16;
+constexpr int kSkinnyUneven = 12;  // from this config on: plain epilogue only, K any multiple of 64 (the shares of slices
+                                  // and waves differ by a unit), the split's sums in a second launch instead of tickets
 int gemm_skinny_rt(int cfg);
 int gemm_skinny_mt(int cfg);
 int gemm_skinny_nw(int cfg);  // waves per workgroup

@@ -623,10 +623,10 @@ std::tuple<Tensor, Tensor> gemm_skinny(const Tensor& x, const Tensor& w, int64_t
     CHK(cfg >= 0 && cfg < chronos::kSkinnyConfigs, "gemm_skinny: cfg");
     CHK(mode >= 0 && mode <= 2, "gemm_skinny: mode");
     const int RT = chronos::gemm_skinny_rt((int)cfg), MT = chronos::gemm_skinny_mt((int)cfg);
-    const int NW = chronos::gemm_skinny_nw((int)cfg);
-    CHK(M >= 1 && M <= 16 * MT, "gemm_skinny: M must be in [1, 16 * MT] of the config");
-    CHK(splitk >= 1 && K % (64 * NW * splitk) == 0 && K <= (1 << 20) && N * K < (1LL << 40),
-        "gemm_skinny: K % (64 * NW * splitk) == 0");
+    const bool uneven = cfg >= chronos::kSkinnyUneven;
+    CHK(splitk >= 1 && K % (uneven ? 64 : 64 * chronos::gemm_skinny_nw((int)cfg) * splitk) == 0 && (!uneven || splitk <= 64) &&
+            K <= (1 << 20) && N * K < (1LL << 40),
+        "gemm_skinny: K % (64 * NW * splitk) == 0 (uneven configs: K % 64 == 0)");
     CHK(mode == 1 ? RT % 2 == 0 && (N / 2) % (8 * RT) == 0 && N % 2 == 0 : N % (16 * RT) == 0,
         "gemm_skinny: N % (16 RT) (swiglu: F % (8 RT), RT even)");
     CHK(mode != 2 || !part_in.has_value(), "gemm_skinny: resid mode has no norm prologue");
@@ -660,9 +660,9 @@ std::tuple<Tensor, Tensor> gemm_skinny(const Tensor& x, const Tensor& w, int64_t
     const int64_t groups = mode == 1 ? (N / 2) / (8 * RT) : N / (16 * RT);
     Tensor ws;
     if (splitk > 1) {
-        ws = at::empty({groups * splitk * 64 * RT * MT * 4}, x.options().dtype(at::kFloat));
+        ws = at::empty({uneven ? splitk * M * N : groups * splitk * 64 * RT * MT * 4}, x.options().dtype(at::kFloat));
         a.ws = ws.data_ptr<float>();
-        a.cnt = split_tickets(x, groups);
+        if (!uneven) a.cnt = split_tickets(x, groups);
     }
     CHK(chronos::launch_gemm_skinny((int)cfg, (int)mode, part_in.has_value(), a, cur_stream()), "gemm_skinny: launch");
     return {y, part_out};

@@ -55,9 +55,9 @@ __global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a) {
     const int G = MODE == kSwiglu ? a.F / (8 * RT) : a.N / (16 * RT);
     const int task = xcd_remap(blockIdx.x, G * S);
     const int g = task / S, s = task - g * S;
-    const int KS = K / S;
-    const int NU = KS / (64 * NW);  // 64-k units per wave
-    const int kbase = s * KS + wave * 64 + 8 * (lane >> 4);
+    const int unit0 = K / 64 * s / S;  // the slice's 64-k units (slices and waves differ by one where they do not divide; may be 0)
+    const int NU = (K / 64 * (s + 1) / S - unit0 + NW - 1 - __builtin_amdgcn_readfirstlane(wave)) / NW;  // of this wave
+    const int kbase = unit0 * 64 + wave * 64 + 8 * (lane >> 4);
 
     const bf16x8* wp[RT];
 #pragma unroll
@@ -87,7 +87,7 @@ __global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a) {
     if constexpr (XL) {
 #pragma unroll
         for (int i = 0; i < 2 * MT; ++i)
-            xl[i] = reinterpret_cast<const bf16x8*>(a.x + (int64_t)min(8 * i + (lane >> 3), M - 1) * K + s * KS +
+            xl[i] = reinterpret_cast<const bf16x8*>(a.x + (int64_t)min(8 * i + (lane >> 3), M - 1) * K + unit0 * 64 +
                                                     wave * 64 + 8 * (lane & 7));
     }
     unsigned char* xs = smem + wave * (MT * 2048);  // XL: this wave's x tile, 16 MT rows x 128 B
@@ -217,6 +217,16 @@ __global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a) {
             }
     }
 
+    if (MODE == kPlain && !NORMP && S > 1 && a.cnt == nullptr) {  // the slice's sums [S, M, N]: skinny_sum_kernel adds them
+        if (active) {
+#pragma unroll
+            for (int j = 0; j < VP; ++j) {
+                const int v = tid + NT * j, r = v / CPR, c = v % CPR;
+                if (r < M) *reinterpret_cast<f32x4*>(a.ws + ((int64_t)s * M + r) * a.N + g * 16 * RT + 4 * c) = val[j][0];
+            }
+        }
+        return;
+    }
     if (S > 1) {  // split-K: slab per task in output-unit order, ticket per row group, last arriver sums in order
         // fence-free hand-off (chronos_hip.h st_wt / ld_wt): write-through slab stores, one lane's ticket after every
         // wave drained its stores, sc1 slab loads by the last arriver — an agent release + acquire pair per workgroup
@@ -301,6 +311,18 @@ __global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a) {
     }
 }
 
+// y = the sum over S slices of 4 outputs per thread, in slice order
+__global__ void __launch_bounds__(256) skinny_sum_kernel(const float* __restrict__ ws, uint16_t* __restrict__ y, int64_t n, int S) {
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i >= n) return;
+    f32x4 v = *reinterpret_cast<const f32x4*>(ws + i);
+    for (int s = 1; s < S; ++s) v += *reinterpret_cast<const f32x4*>(ws + s * n + i);
+    u16x4 o;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) o[k] = f2bf(v[k]);
+    *reinterpret_cast<u16x4*>(y + i) = o;
+}
+
 template <int RT, int MT, int D, int NW, int MODE, bool NORMP>
 void launch_cfg(const PPArgs& a, hipStream_t st) {
     constexpr int UNITS = RT * MT * 64;
@@ -314,10 +336,16 @@ void launch_cfg(const PPArgs& a, hipStream_t st) {
     }
     const int G = MODE == kSwiglu ? a.F / (8 * RT) : a.N / (16 * RT);
     hipLaunchKernelGGL(kern, dim3(G * a.splitk), dim3(64 * NW), lds, st, a);
+    if (a.splitk > 1 && a.cnt == nullptr) {
+        const int64_t n = (int64_t)a.M * a.N;
+        skinny_sum_kernel<<<(unsigned)((n / 4 + 255) / 256), 256, 0, st>>>(a.ws, a.y, n, a.splitk);
+    }
 }
 
 // configs {RT (W tiles of 16 rows per workgroup), MT (x tiles: M <= 16 MT), D (ring depth in 64-k units), NW (waves
-// splitting K inside the workgroup; K % (64 NW splitk) == 0)}
+// splitting K inside the workgroup; K % (64 NW splitk) == 0, from kSkinnyUneven on K % 64 == 0: the shares then differ by a unit.  At a few MB of weights what bounds a launch is latency, so these run 8 short waves: 2048 x 2048 with 16 rows 6.0 us (the
+// library 11.0), 1024 x 2816 with one row 5.7 (8.6).  Their split across workgroups writes [split, M, N] sums that a second launch adds
+// up: 2.0-2.3 us, as much as tickets cost, with nothing kept between calls)}
 #define SK_CONFIGS(X)  \
     X(0, 1, 1, 4, 16)  \
     X(1, 2, 1, 4, 8)   \
@@ -330,7 +358,11 @@ void launch_cfg(const PPArgs& a, hipStream_t st) {
     X(8, 1, 2, 4, 16)  \
     X(9, 1, 4, 2, 16)  \
     X(10, 2, 4, 2, 8)  \
-    X(11, 1, 1, 4, 8)
+    X(11, 1, 1, 4, 8)  \
+    X(12, 1, 2, 4, 8)  \
+    X(13, 1, 4, 2, 8)  \
+    X(14, 1, 1, 4, 8)  \
+    X(15, 2, 1, 4, 8)
 
 template <int MODE, bool NORMP>
 bool launch_mode(int cfg, const PPArgs& a, hipStream_t st) {
@@ -338,6 +370,7 @@ bool launch_mode(int cfg, const PPArgs& a, hipStream_t st) {
 #define SK_CASE(ID, RT_, MT_, D_, NW_)                                     \
     case ID:                                                               \
         if constexpr (MODE == kSwiglu && RT_ % 2) return false;            \
+        else if constexpr (ID >= kSkinnyUneven && (MODE != kPlain || NORMP)) return false; \
         else {                                                             \
             launch_cfg<RT_, MT_, D_, NW_, MODE, NORMP>(a, st);             \
             return true;                                                   \

@@ -12,8 +12,9 @@ Routing is by measured shape:
   with the kernel, tile config and split-K of the measured plan (``gemm_plan.json``: per (N, K, epilogue) the best
   by M range, from ``scripts/tune_gemm_pp.py`` on one MI355X, random operands, cold weights; plan cfg >= 100 is
   skinny config cfg - 100);
+* shapes that the plan does not list: up to 64 rows ``few_rows_plan``, where its measured range says that it wins;
 * hipBLASLt (torch.matmul) only where the plan records that the library wins by more than 3 % (the "plain library
-  GEMM" rule), or for shapes the kernel does not take (K % 64, N % 4).  CHRONOS_PP=lib|own|auto forces a side.
+  GEMM" rule), for unlisted shapes outside that range, or for shapes the kernel does not take (K % 64, N % 4).  CHRONOS_PP=lib|own|auto forces a side.
 """
 from __future__ import annotations
 
@@ -64,6 +65,18 @@ SK_BASE = 100
 _SK = {0: (1, 1, 16), 1: (2, 1, 8), 2: (4, 1, 4), 3: (2, 2, 8), 4: (4, 2, 4), 5: (2, 4, 4), 6: (4, 4, 4),
        7: (2, 8, 4), 8: (1, 2, 16), 9: (1, 4, 16), 10: (2, 4, 8), 11: (1, 1, 8)}
 SKINNY_MAX_M = 128
+# Configs that take any K % 64 (gemm_skinny.hip kSkinnyUneven): (W rows per workgroup, x rows, waves splitting K)
+_UNEVEN = {112: (16, 32, 8), 113: (16, 64, 8), 114: (16, 16, 8), 115: (32, 16, 8)}
+# Few rows, plain epilogue, shapes that the plan does not list: per largest M the configs that won somewhere on a grid of
+# N = 512 .. 32768 by K = 512 .. 14336, and what a launch of each takes in us, fitted on that grid (cold weights; rms error 5 %):
+# constant, split-K's second launch, per 64-deep step of a wave, per MB of weights, per 256 workgroups, per such step of each
+# further round of 256 workgroups, per 100 MB of x that all workgroups read together.  The pick is within 1 % of the best config on average.
+_FEW = ((16, {114: (2.4, 2.0, 0.77, 0.016, 0.23, 0.69, 3.4), 115: (2.2, 2.1, 1.4, 0.0082, 0.57, 1.3, 5.1),
+              72: (2.2, 0.0, 0.16, 0.07, 1.2, 0.24, 8.3), 75: (1.7, 0.0, 0.28, 0.1, 1.4, 0.0, 10.0)}),
+        (32, {112: (2.3, 2.1, 1.1, 0.0, 0.67, 0.9, 1.0), 72: (2.1, 0.0, 0.18, 0.052, 1.5, 0.22, 8.7),
+              75: (1.8, 0.0, 0.29, 0.085, 1.7, 0.0, 12.0)}),
+        (64, {113: (2.4, 2.3, 1.5, 0.0, 0.9, 1.0, 0.75), 72: (2.2, 0.0, 0.16, 0.0, 1.3, 0.19, 5.1),
+              38: (3.0, 0.0, 0.31, 0.0, 0.54, 0.0, 35.0), 39: (2.4, 0.0, 0.21, 0.0, 1.2, 0.22, 14.0)}))
 _plan_cache: dict = {}
 _plan_table: Optional[dict] = None
 _qplan_table: Optional[dict] = None
@@ -188,6 +201,52 @@ def pp_plan(m: int, n: int, k: int, mode: int = PP_PLAIN) -> Optional[tuple[int,
             out = None
     _plan_cache[key] = out
     return out
+
+
+def few_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
+    """(config, split-K) of the hand-written GEMM for few rows of a shape that no plan lists, or None (the GEMV or the
+    library).  Where it wins, measured on the grid of _FEW, us, GEMV or library -> this:
+    one row: K < 2048, where the GEMV's waves have one step each (5632 x 1024: 7.3 -> 5.7; 32768 x 512: 22 -> 9.7; at K = 2048 the
+    two are level), and K % 512, which the GEMV does not take (1024 x 2816: 8.6 -> 5.7): no slower at any of 41 shapes;
+    2 .. 64 rows: weights up to 12.5 M elements, from 33 rows on up to 7 M or K <= 2048 (2048 x 2048, 16 rows: 11.0 -> 6.0; 64 rows:
+    11.7 -> 8.1): 1.3 .. 1.6 times as fast on average, 4 of 590 slower by more than 3 %, the worst by 6 %; 48 shapes off the grid: 1.7 times,
+none slower.  More weights than that stream from
+    memory at the library's rate too (8192 x 8192, 16 rows: 30.5, 31.1 here), except that it keeps half the chip idle for wide
+    outputs of up to 48 rows (22016 x 2048, 16 rows: 44 -> 21)."""
+    key = (m, n, k, -1)
+    hit = _plan_cache.get(key, False)
+    if hit is not False:
+        return hit
+    nk, out = n * k, None
+    if m == 1:
+        ok = (k < 2048 or k % 512 != 0) and nk <= 100_000_000
+    else:
+        ok = GEMV_MAX_M < m <= 64 and (nk <= 12_500_000 and (m <= 32 or k <= 2048 or nk <= 7_000_000) or
+                                       m <= 48 and n >= 12288 and nk <= (40_000_000 if n < 16384 else 100_000_000))
+    if ok and k % 64 == 0 and n % 16 == 0 and PP_MODE == "auto" and (n, k, PP_PLAIN) not in _plan_file():
+        best = None
+        for cfg, c in next(models for most, models in _FEW if m <= most).items():
+            bn, bm, nw = _UNEVEN.get(cfg) or (_PP_BN[cfg], _PP_BM[cfg], 1)
+            for sk in (1, 2, 4, 8) if cfg in _UNEVEN else (1,):
+                groups = -(-n // bn) * -(-m // bm) * sk
+                if cfg in _UNEVEN and n % bn or k < 64 * sk or (sk > 1 and groups > 1024):
+                    continue
+                steps = k / (64 * sk * nw)
+                t = (c[0] + c[1] * (sk > 1) + c[2] * steps + c[3] * nk * 2e-6 + c[4] * groups / 256
+                     + c[5] * (-(-groups // 256) - 1) * steps + c[6] * m * k * groups * 2e-8)
+                if best is None or t < best:
+                    best, out = t, (cfg, sk)
+    _plan_cache[key] = out
+    return out
+
+
+def _plain_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Operands that the kernels take as they lie, and nothing that has to see the product (gradients, transforms)."""
+    return (type(x) is torch.Tensor and x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16 and w.dim() == 2
+            and w.shape[1] == x.shape[-1] and w.device == x.device
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
+            and not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0
+            and x.is_contiguous() and w.is_contiguous() and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 
 
 def pp_gemm(x: torch.Tensor, w: torch.Tensor, mode: int, plan: tuple[int, int], resid=None, part=None,
@@ -395,12 +454,13 @@ def linear(x, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tens
     if x.is_cuda:
         m, k = x.numel() // x.shape[-1], x.shape[-1]
         n = w.shape[0]
-        if gemv_ok(m, n, k):
+        few = few_rows_plan(m, n, k) if out is None and 0 < m <= 64 and _plain_rows(x, w) else None
+        if few is None and gemv_ok(m, n, k):
             return _gemv(x, w)
         for pred, fn in _custom:
             if pred(m, n, k):
                 return fn(x, w)
-        plan = pp_plan(m, n, k, PP_PLAIN) if out is None else None
+        plan = (few or pp_plan(m, n, k, PP_PLAIN)) if out is None else None
         if plan is not None:
             y, _ = pp_gemm(x, w, PP_PLAIN, plan)
             return y.view(*x.shape[:-1], n)
