@@ -23,8 +23,12 @@ void launch_hy_mlstm_scan(const void*, int, const float*, const int32_t*, const 
 void launch_hy_mlstm_out(const float*, const void*, int, int, const float*, void*, int, int, int, float, bool,
                          hipStream_t);
 void launch_hy_latent_prep(void*, int64_t, const void*, int64_t, const int32_t*, const int32_t*, const int32_t*, int,
-                           const float*, float, const float*, int, bool, int, int, int, int, void*, int, void*, int, bool,
+                           const float*, float, const float*, int, bool, int, int, int, int, void*, int, void*, void*, void*, int, bool,
                            hipStream_t);
+bool hy_latent_expanded_ok(int, int, int);
+void launch_hy_latent_expanded(const uint16_t*, int64_t, const uint16_t*, const uint16_t*, int64_t, const int32_t*, const float*,
+                               const uint16_t*, int64_t, const float*, uint16_t*, int64_t, int, int, int, int, int, float, int,
+                               int, hipStream_t);
 void launch_hy_head_matmul(const void*, int64_t, int64_t, const void*, void*, int64_t, int64_t, const void*, int64_t, int,
                            int, int, int, bool, hipStream_t);
 void launch_hy_dyn_tanh(const float*, const float*, void*, int, int, bool, hipStream_t);
@@ -221,7 +225,7 @@ Tensor hy_mlstm_out(const Tensor& o, const Tensor& proj, int64_t g_off, const Te
 void hy_latent_prep(Tensor& q, const c10::optional<Tensor>& dkv, const Tensor& pos, const Tensor& tok_seq,
                     const Tensor& block_table, const c10::optional<Tensor>& w_norm, double eps,
                     const c10::optional<Tensor>& cos_sin, int64_t dims, int64_t rank, Tensor& cache, c10::optional<Tensor> qa,
-                    bool interleaved) {
+                    bool interleaved, c10::optional<Tensor> lat, c10::optional<Tensor> kr) {
     c10::hip::HIPGuardMasqueradingAsCUDA g(q.device());
     same_act(q, cache, "latent_prep: the cache holds the activation dtype");
     need(q.dim() == 3 && cache.dim() == 3 && cache.is_contiguous(), "latent_prep: layouts");
@@ -248,12 +252,19 @@ void hy_latent_prep(Tensor& q, const c10::optional<Tensor>& dkv, const Tensor& p
         same_act(q, *qa, "latent_prep: qa in the activation dtype");
         need(qa->is_contiguous() && qa->dim() == 3 && qa->size(0) == T && qa->size(1) == H && qa->size(2) == DK, "latent_prep: qa [T, H, rank + R]");
     }
+    need(lat.has_value() == kr.has_value() && (!lat || dkv), "latent_prep: copies of own rows, both parts");
+    if (lat) {
+        same_act(q, *lat, "latent_prep: copies in the activation dtype");
+        same_act(q, *kr, "latent_prep: copies in the activation dtype");
+        need(lat->is_contiguous() && lat->dim() == 2 && lat->size(0) == T && lat->size(1) == rank && kr->is_contiguous() &&
+             kr->dim() == 2 && kr->size(0) == T && kr->size(1) == R, "latent_prep: copies [T, rank] and [T, R]");
+    }
     chronos::launch_hy_latent_prep(q.data_ptr(), q.stride(0), dkv ? dkv->data_ptr() : nullptr, dkv ? dkv->stride(0) : 0,
                                    pos.data_ptr<int32_t>(), tok_seq.data_ptr<int32_t>(), block_table.data_ptr<int32_t>(),
                                    (int)block_table.size(1), dkv ? w_norm->data_ptr<float>() : nullptr, (float)eps,
                                    cos_sin ? cos_sin->data_ptr<float>() : nullptr, (int)dims, interleaved, (int)rank, (int)R,
-                                   (int)H, (int)D, cache.data_ptr(), (int)cache.size(1), qa ? qa->data_ptr() : nullptr, (int)T,
-                                   f32(q), stream());
+                                   (int)H, (int)D, cache.data_ptr(), (int)cache.size(1), qa ? qa->data_ptr() : nullptr,
+                                   lat ? lat->data_ptr() : nullptr, kr ? kr->data_ptr() : nullptr, (int)T, f32(q), stream());
 }
 
 // the first gate column of row 0 of a [T, C] activation tensor, after checking that columns off .. off + n exist
@@ -368,6 +379,35 @@ Tensor hy_latent_attention(const Tensor& qa, const Tensor& cache, const Tensor& 
     TORCH_CHECK(ok, "chronos hybrid op: latent_attention has no launch geometry for heads=", H, " row width=", DK,
                 " rank=", rank, " (rank <= 512; 16 keys and 4 query rows must fit the LDS)");
     return out;
+}
+
+// Attention of sequences whose positions are 0, 1, ..: q [T, H, D + R] rows (rotated part last), kv [T, H, D + Dv], kr [T, R] rows
+void hy_latent_expanded(const Tensor& q, const Tensor& kv, const Tensor& kr, const Tensor& q_start, const c10::optional<Tensor>& gate,
+                        const c10::optional<Tensor>& gate_src, int64_t g_off, const c10::optional<Tensor>& sink, Tensor& out,
+                        double scale, int64_t max_q, int64_t window) {
+    c10::hip::HIPGuardMasqueradingAsCUDA g(q.device());
+    for (const Tensor* t : {&kv, &kr, static_cast<const Tensor*>(&out)}) same_act(q, *t, "latent_expanded: one activation dtype");
+    need(!f32(q) && q.dim() == 3 && kv.dim() == 3 && kr.dim() == 2 && out.dim() == 3 && kv.is_contiguous(), "latent_expanded: bfloat16 layouts");
+    const int64_t T = q.size(0), H = q.size(1), R = kr.size(1), D = q.size(2) - R, Dv = out.size(2);
+    need(kv.size(0) == T && kv.size(1) == H && kv.size(2) == D + Dv && kr.size(0) == T && out.size(0) == T && out.size(1) == H, "latent_expanded: shapes");
+    need(std::max({D, R, Dv}) <= 1024 && chronos::hy_latent_expanded_ok((int)D, (int)R, (int)Dv), "latent_expanded: D % 8, R % 8, D + R <= 192, Dv % 16, Dv <= 128");
+    need(q.stride(2) == 1 && q.stride(1) == D + R && q.stride(0) % 8 == 0 && q.stride(0) >= H * (D + R) && (R == 0 || (kr.stride(1) == 1 && kr.stride(0) % 8 == 0 && kr.stride(0) >= R)) &&
+         out.stride(2) == 1 && out.stride(1) == Dv && out.stride(0) % 4 == 0 && out.stride(0) >= H * Dv, "latent_expanded: rows");
+    need((reinterpret_cast<uintptr_t>(q.data_ptr()) | reinterpret_cast<uintptr_t>(kv.data_ptr()) | reinterpret_cast<uintptr_t>(kr.data_ptr())) % 16 == 0 &&
+         reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0, "latent_expanded: alignment");
+    need(scale > 0 && window >= 0 && max_q >= 0 && max_q <= T, "latent_expanded: scale > 0, window, max_q");
+    i32(q_start, "latent_expanded: q_start");
+    const int64_t B = q_start.numel() - 1;
+    need(B * H < (1LL << 31) && (max_q + 127) / 128 <= 65535, "latent_expanded: launch");
+    if (gate) { flt(*gate, "latent_expanded: float32 gate"); need(gate->numel() == T * H, "latent_expanded: gate [T, H]"); }
+    if (sink) { flt(*sink, "latent_expanded: float32 sinks"); need(sink->numel() == H, "latent_expanded: sink [H]"); }
+    const void* gp = gate_cols(q, gate_src, g_off, T, H * Dv, "latent_expanded: gate columns");
+    if (T == 0 || B <= 0) return;
+    auto p = [](const Tensor& t) { return static_cast<const uint16_t*>(t.data_ptr()); };
+    chronos::launch_hy_latent_expanded(p(q), q.stride(0), p(kv), p(kr), kr.stride(0), q_start.data_ptr<int32_t>(),
+                                       gate ? gate->data_ptr<float>() : nullptr, static_cast<const uint16_t*>(gp), gate_src ? gate_src->stride(0) : 0,
+                                       sink ? sink->data_ptr<float>() : nullptr, static_cast<uint16_t*>(out.data_ptr()), out.stride(0), (int)B, (int)H,
+                                       (int)D, (int)R, (int)Dv, (float)scale, (int)window, (int)max_q, stream());
 }
 
 std::tuple<Tensor, Tensor> hy_moe_route(const Tensor& h, const Tensor& w, const Tensor& corr, int64_t top) {
@@ -1040,7 +1080,12 @@ TORCH_LIBRARY_FRAGMENT(chronos, m) {
     m.def("hy_mlstm_out(Tensor o, Tensor proj, int g_off, Tensor w, float eps, bool out_f32) -> Tensor");
     m.def("hy_latent_prep(Tensor(a!) q, Tensor? dkv, Tensor pos, Tensor tok_seq, Tensor block_table, Tensor? w_norm, "
           "float eps, Tensor? cos_sin, int dims, int rank, Tensor(b!) cache, Tensor(c!)? qa=None, "
-          "bool interleaved=False) -> ()");
+          "bool interleaved=False, Tensor(d!)? lat=None, Tensor(e!)? kr=None) -> ()");
+    m.def("hy_latent_expanded(Tensor q, Tensor kv, Tensor kr, Tensor q_start, Tensor? gate, Tensor? gate_src, int g_off, "
+          "Tensor? sink, Tensor(a!) out, float scale, int max_q, int window=0) -> ()");
+    m.def("hy_latent_expanded_ok(int D, int R, int Dv) -> bool", [](int64_t D, int64_t R, int64_t Dv) {
+        return std::max({D, R, Dv}) <= 1024 && chronos::hy_latent_expanded_ok((int)D, (int)R, (int)Dv) && chronos::hy_latent_use_mfma(false, 16, 16);
+    });
     m.def("hy_head_matmul(Tensor a, Tensor w, Tensor(a!) out, Tensor? gate_src, int g_off) -> ()");
     m.def("hy_dyn_tanh(Tensor x, Tensor wba, bool out_f32) -> Tensor");
     m.def("hy_gated_join(Tensor y, Tensor(a!) x, Tensor? gate_src, int g_off, Tensor? gate_b, float mult, Tensor? wba, "
@@ -1110,6 +1155,7 @@ TORCH_LIBRARY_IMPL(chronos, CUDA, m) {
     m.impl("hy_dyn_tanh", &hy_dyn_tanh);
     m.impl("hy_gated_join", &hy_gated_join);
     m.impl("hy_poly_norm", &hy_poly_norm);
+    m.impl("hy_latent_expanded", &hy_latent_expanded);
     m.impl("hy_latent_attention", &hy_latent_attention);
     m.impl("hy_moe_route", &hy_moe_route);
     m.impl("hy_moe_ffn", &hy_moe_ffn);

@@ -1,7 +1,7 @@
 // latent_attention.hip — attention over a paged cache that holds ONE row per token: a low-rank latent (kv_rank
 // columns, RMS-normed) followed by a rotated key part (R columns) shared by all heads.
 //
-// Keys and values are never materialised.  The caller carries each head's query into the latent space
+// Keys and values are not materialised.  The caller carries each head's query into the latent space
 // (q_u W_uk), so the score of head h against token j is  qa[h] . row_j  with qa = [q_u W_uk | rotated q_r], and the
 // attention output is a weighted sum of the rows' latent columns, which the caller brings back through W_uv.  All
 // heads therefore share the same key/value rows: one pass over the cache serves every head (a multi-query layout with
@@ -11,7 +11,8 @@
 //                     every head's rotated query columns (cos / sin from a float table made in double precision; pairs
 //                     are columns i and i + dims / 2, or 2i and 2i + 1), cache write at the token's page and slot.  The
 //                     projections' rows may be wider than what is read of them, and the rotated query columns go in
-//                     place or straight to their columns of the latent query.
+//                     place or straight to their columns of the latent query.  Optionally the cached rows also go to two
+//                     arrays in token order (for latent_expanded.hip, which whole long prompts take).
 //   latent_attention  one workgroup per (sequence, block of up to 64 (token, head) rows): the rows are split
 //                     over 4 waves; 64-key tiles of the cache are staged in LDS; lanes are keys for the scores
 //                     (float accumulation, causal mask by each row's own position, online softmax in float) and
@@ -31,7 +32,8 @@ __global__ void __launch_bounds__(256) latent_prep_kernel(
         T* q, int64_t ldq, const T* __restrict__ dkv, int64_t ldkv, const int32_t* __restrict__ pos,
         const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ block_table, int max_blocks,
         const float* __restrict__ w_norm, float eps, const float* __restrict__ cos_sin, int dims, int inter, int rank,
-        int R, int H, int D, T* __restrict__ cache, int BS, T* __restrict__ qa) {
+        int R, int H, int D, T* __restrict__ cache, int BS, T* __restrict__ qa, T* __restrict__ lat,
+        T* __restrict__ kr) {
     __shared__ float red[16];
     const int64_t t = blockIdx.x;
     const int p = pos[t];
@@ -47,7 +49,10 @@ __global__ void __launch_bounds__(256) latent_prep_kernel(
             ss += v * v;
         }
         const float inv = 1.f / sqrtf(block_sum(ss, red) / (float)rank + eps);
-        for (int i = threadIdx.x; i < rank; i += 256) st<T>(crow + i, ld<T>(drow + i) * inv * w_norm[i]);
+        for (int i = threadIdx.x; i < rank; i += 256) {
+            st<T>(crow + i, ld<T>(drow + i) * inv * w_norm[i]);
+            if (lat != nullptr) lat[t * rank + i] = crow[i];
+        }
     }
     const int half = dims / 2;
     const float* cs = cos_sin + (int64_t)p * dims;
@@ -62,11 +67,18 @@ __global__ void __launch_bounds__(256) latent_prep_kernel(
         const float u = ld<T>(src + lo), v = ld<T>(src + hi), c = cs[k], s = cs[half + k];
         st<T>(dst + lo, u * c - v * s);
         st<T>(dst + hi, v * c + u * s);
+        if (kr != nullptr && row == 0) {
+            kr[t * R + lo] = dst[lo];
+            kr[t * R + hi] = dst[hi];
+        }
     }
     const int rest = R - dims;
     for (int i = threadIdx.x + (own ? 0 : rest); i < (qa != nullptr ? H + 1 : 1) * rest; i += 256) {
         const int row = i / rest, k = dims + i % rest;
-        if (row == 0) crow[rank + k] = drow[rank + k];
+        if (row == 0) {
+            crow[rank + k] = drow[rank + k];
+            if (kr != nullptr) kr[t * R + k] = drow[rank + k];
+        }
         else qa[(t * H + row - 1) * DK + rank + k] = q[t * ldq + (int64_t)(row - 1) * (D + R) + D + k];
     }
 }
@@ -232,14 +244,15 @@ __global__ void __launch_bounds__(256) latent_attention_kernel(
 
 }  // namespace hy
 
-// ldq, ldkv: row strides of q and dkv in elements.  qa == nullptr: queries are rotated in place.
+// ldq, ldkv: row strides of q and dkv in elements.  qa == nullptr: queries are rotated in place.  lat,
+// kr (may be nullptr): [T, rank] and [T, R], copies of the cached rows' parts.
 void launch_hy_latent_prep(void* q, int64_t ldq, const void* dkv, int64_t ldkv, const int32_t* pos, const int32_t* tok_seq,
                            const int32_t* bt, int max_blocks, const float* w_norm, float eps, const float* cos_sin, int dims,
-                           bool inter, int rank, int R, int H, int D, void* cache, int BS, void* qa, int T, bool f32,
+                           bool inter, int rank, int R, int H, int D, void* cache, int BS, void* qa, void* lat, void* kr, int T, bool f32,
                            hipStream_t s) {
     if (T == 0) return;
-    if (f32) hy::latent_prep_kernel<float><<<T, 256, 0, s>>>((float*)q, ldq, (const float*)dkv, ldkv, pos, tok_seq, bt, max_blocks, w_norm, eps, cos_sin, dims, inter, rank, R, H, D, (float*)cache, BS, (float*)qa);
-    else hy::latent_prep_kernel<uint16_t><<<T, 256, 0, s>>>((uint16_t*)q, ldq, (const uint16_t*)dkv, ldkv, pos, tok_seq, bt, max_blocks, w_norm, eps, cos_sin, dims, inter, rank, R, H, D, (uint16_t*)cache, BS, (uint16_t*)qa);
+    if (f32) hy::latent_prep_kernel<float><<<T, 256, 0, s>>>((float*)q, ldq, (const float*)dkv, ldkv, pos, tok_seq, bt, max_blocks, w_norm, eps, cos_sin, dims, inter, rank, R, H, D, (float*)cache, BS, (float*)qa, (float*)lat, (float*)kr);
+    else hy::latent_prep_kernel<uint16_t><<<T, 256, 0, s>>>((uint16_t*)q, ldq, (const uint16_t*)dkv, ldkv, pos, tok_seq, bt, max_blocks, w_norm, eps, cos_sin, dims, inter, rank, R, H, D, (uint16_t*)cache, BS, (uint16_t*)qa, (uint16_t*)lat, (uint16_t*)kr);
 }
 
 // Launch geometry of latent_attention for these sizes: RBLK (token, head) rows per workgroup (<= 64), KT keys per

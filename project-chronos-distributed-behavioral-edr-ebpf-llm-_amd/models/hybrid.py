@@ -604,12 +604,16 @@ def pack_latent(spec: LatentAttentionSpec, t: dict, device, act_dtype) -> dict:
     """t: q (or dq, dq.norm, uq), dkv, dkv.norm (not with kv_from), uk, uv, g, sink, o.  q | dkv (| g with a gate per
     output column) are one projection, with a query latent dq | dkv are; per-head
     gate rows are a few-row float32-output projection.  The per-head up-projections are kept as [H, rank, D] and
-    [H, Dv, rank]: keys are never materialised (the query is carried into the latent space instead) and the value
-    up-projection is applied to the attention's latent-space output."""
+    [H, Dv, rank]: over cached latents keys are not materialised (the query is carried into the latent space instead) and the
+    value up-projection is applied to the attention's latent-space output."""
     a = lambda x: x.to(device=device, dtype=act_dtype).contiguous()  # noqa: E731
     f = lambda x: x.to(device=device, dtype=torch.float32).contiguous()  # noqa: E731
     out = dict(w_uk=a(t["uk"].view(spec.heads, spec.dim, spec.kv_rank).transpose(1, 2)),
                w_uv=a(t["uv"].view(spec.heads, spec.vdim, spec.kv_rank)))
+    if out["w_uv"].is_cuda and act_dtype == torch.bfloat16 and spec.kv_from is None and not spec.two_term and spec.scale > 0 and \
+            spec.kv_rank % 8 == 0 and hops.latent_expanded_ok(spec.dim, spec.rot_dim, spec.vdim):
+        # whole prompts: every head's keys and values in one product of the latents
+        out["w_kv"] = torch.cat([out["w_uk"].transpose(1, 2), out["w_uv"]], 1).reshape(-1, spec.kv_rank)
     rows = [t["dq"] if spec.q_rank else t["q"]]
     if spec.q_rank:
         out.update(dq_norm=f(t["dq.norm"]), w_uq=a(t["uq"]))
@@ -838,6 +842,7 @@ class StepMeta:
     last_idx: torch.Tensor
     max_q: int
     shared: dict = field(default_factory=dict)  # what one layer of a step leaves for later layers of the same step
+    fresh: bool = False         # every sequence starts at position 0: its keys are all among the step's tokens
 
 
 def mix_mlstm(model, li: int, spec: MLSTMSpec, w: dict, h, meta: StepMeta, cache: HybridCache):
@@ -875,6 +880,13 @@ def _wide_out(w: dict, proj, n: int):
     return wide, wide[:, :n]
 
 
+# Least tokens x heads x longest sequence for which a prompt's keys and values are written out: below, a step is bound by its
+# launches and the form through the latents has fewer.  Whole steps of 4 layers, two of them latent attention, us, through the
+# latents / written out: 0.7 M (8 heads, 300 tokens) 608 / 640; 1.8 M (8 heads, 16 x 100) 613 / 640; 2.9 M (32 heads, 300) 1314 / 1221;
+# 7 M (32 heads, 16 x 100) 3018 / 2845; 130 M (8 heads, 4000) 1895 / 1710; 500 M (32 heads, 4000) 8040 / 6765.
+EXPAND_MIN = 1 << 21
+
+
 def mix_latent_attention(model, li: int, spec: LatentAttentionSpec, w: dict, h, meta: StepMeta, cache: HybridCache):
     T = h.shape[0]
     H, D, R, rank = spec.heads, spec.dim, spec.rot_dim, spec.kv_rank
@@ -887,6 +899,17 @@ def mix_latent_attention(model, li: int, spec: LatentAttentionSpec, w: dict, h, 
     q = q.view(T, H, D + R)
     gate = hops.rowdot(h, w["w_g"]) if spec.gate and not spec.gate_wide else None
     own = spec.kv_from is None
+    wide, ov = _wide_out(w, proj, H * spec.vdim)
+    if meta.fresh and "w_kv" in w and T * H * meta.max_q >= EXPAND_MIN and q.stride(0) % 8 == 0 and (ov is None or ov.stride(0) % 4 == 0):
+        # All keys are among this step's tokens: written out per head they cost what carrying the queries into the latent
+        # space and the output back costs, and attention takes D + R + Dv products per score, not 2 rank + R.
+        lat, kr = (torch.empty(T, n, device=h.device, dtype=h.dtype) for n in (rank, R))
+        hops.latent_prep(q, proj[:, nq:nq + nkv], meta.pos, meta.tok_seq, meta.block_table, w["dkv_norm"], eps, model.rope.get(li),
+                         spec.rope_dims, rank, cache.lat[li], None, spec.rope_interleaved, lat, kr)
+        kv = hops.matmul(lat, w["w_kv"]).view(T, H, D + spec.vdim)
+        ov = hops.latent_expanded(q, kv, kr, meta.q_start, gate, proj if spec.gate and spec.gate_wide else None, nq + nkv,
+                                  w.get("sink"), spec.scale, meta.max_q, spec.window, None if ov is None else ov.view(T, H, spec.vdim))
+        return _with_gate(hops.matmul(ov.view(T, H * spec.vdim) if wide is None else wide, w["w_o"]), proj, w)
     # the query goes into the latent space (q_u W_uk per head), so a key is the cached row itself; the output
     # comes back through W_uv per head
     qa = torch.empty(T, H, rank + R, device=h.device, dtype=h.dtype)
@@ -895,7 +918,6 @@ def mix_latent_attention(model, li: int, spec: LatentAttentionSpec, w: dict, h, 
     hops.head_matmul(q[:, :, :D], w["w_uk"], qa[:, :, :rank])
     oa = hops.latent_attention(qa, cache.lat[li], meta.block_table, meta.q_start, meta.pos, gate, spec.scale, rank,
                                model.act_dtype, meta.max_q, spec.window, spec.two_term, w.get("sink"))
-    wide, ov = _wide_out(w, proj, H * spec.vdim)
     ov = hops.head_matmul(oa, w["w_uv"], None if ov is None else ov.view(T, H, spec.vdim),
                           proj if spec.gate and spec.gate_wide else None, nq + nkv if own else nq)
     return _with_gate(hops.matmul(ov.view(T, H * spec.vdim) if wide is None else wide, w["w_o"]), proj, w)
@@ -1181,10 +1203,13 @@ class HybridDecoder:
         last = torch.tensor([q - 1 for q in qs[1:]] if want is None else list(want), dtype=torch.int64)
         dv = lambda t: h2d(t, self.device)  # noqa: E731
         mq = max((len(c) for c in chunks), default=0)
-        return StepBatch(dv(it(ids)), dv(it(pos)), dv(it(tok_seq)), dv(bt), dv(it(qs)),
-                         dv(it([s0 + len(t) for t, s0 in zip(chunks, starts)])), dv(last),
-                         dv(torch.zeros(max(1, len(chunks)), 2, dtype=torch.int32)), len(chunks), nqt, 1,
-                         slots=dv(it(list(slots))), max_q=mq)
+        sb = StepBatch(dv(it(ids)), dv(it(pos)), dv(it(tok_seq)), dv(bt), dv(it(qs)),
+                       dv(it([s0 + len(t) for t, s0 in zip(chunks, starts)])), dv(last),
+                       dv(torch.zeros(max(1, len(chunks)), 2, dtype=torch.int32)), len(chunks), nqt, 1,
+                       slots=dv(it(list(slots))), max_q=mq)
+        if not any(starts) and not sb.pos.is_inference():   # (inference tensors do not count their changes)
+            sb.fresh = (sb.pos, sb.pos._version, sb.q_start, sb.q_start._version)
+        return sb
 
     def _meta(self, sb: StepBatch) -> StepMeta:
         def one(p: StepBatch) -> StepMeta:
@@ -1193,8 +1218,10 @@ class HybridDecoder:
             if p.tiles is None:  # decode rows: token i is sequence i
                 return StepMeta(p.ids, p.pos, p.tok_seq, p.block_table, p.q_start, p.pos, p.slots, p.last_idx, 1)
             pos0 = p.pos.index_select(0, p.q_start[:-1].long().clamp(max=max(0, p.pos.numel() - 1)))
+            f = p.fresh
+            fresh = f is not None and f[0] is p.pos and f[2] is p.q_start and f[1] == p.pos._version and f[3] == p.q_start._version
             return StepMeta(p.ids, p.pos, p.tok_seq, p.block_table, p.q_start, pos0, p.slots, p.last_idx,
-                            p.max_q or p.ids.numel())
+                            p.max_q or p.ids.numel(), fresh=fresh)
 
         m = one(sb)
         if sb.dec is None:

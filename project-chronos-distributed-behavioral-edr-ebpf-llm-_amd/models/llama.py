@@ -499,6 +499,9 @@ class StepBatch:
     # the most tokens any sequence brings in this step (a launch-shape hint)
     slots: Optional[torch.Tensor] = None
     max_q: int = 0
+    # set by the builder of a prefill step whose sequences all start at position 0: (pos, its version, q_start, its version) as
+    # built; counts only while the batch still holds these tensors as they were (models/hybrid.py)
+    fresh: Optional[tuple] = None
 
 
 # decode-form attention for tiny chunks over long contexts (StepBatch.rows_dec): at least this much context (the

@@ -110,15 +110,19 @@ def mlstm_out(o, proj, g_off: int, norm_w, eps: float, act_dtype):
 
 
 def latent_prep(q, dkv, pos, tok_seq, block_table, w_norm, eps: float, cos_sin, dims: int, rank: int, cache, qa=None,
-                interleaved: bool = False) -> None:
-    """``qa``: where the rotated query columns go (its last R columns per head; default: in place); ``interleaved``:
+                interleaved: bool = False, lat=None, kr=None) -> None:
+    """``lat`` [T, rank] and ``kr`` [T, R]: also get the cached rows' two parts.  ``qa``: where the rotated query columns go (its last R columns per head; default: in place); ``interleaved``:
     neighbouring columns form the rotated pairs.  q and dkv may be column ranges of one wider projection; dkv None: the
     cache is another layer's and only the queries are rotated."""
     if _gpu(q):
         _k().hy_latent_prep(q, dkv, pos, tok_seq, block_table, w_norm, eps, cos_sin if dims else None, dims, rank, cache,
-                            qa, interleaved)
+                            qa, interleaved, lat, kr)
     else:
         ref.latent_prep(q, dkv, pos, tok_seq, block_table, w_norm, eps, cos_sin, dims, rank, cache, qa, interleaved)
+        if lat is not None:
+            rows = cache[block_table[tok_seq.long(), (pos // cache.shape[1]).long()].long(), (pos % cache.shape[1]).long()]
+            lat.copy_(rows[:, :rank])
+            kr.copy_(rows[:, rank:])
 
 
 def head_matmul(a, w, out=None, gate_src=None, g_off: int = -1):
@@ -140,6 +144,20 @@ def latent_attention(qa, cache, block_table, q_start, pos, gate, scale: float, r
     if _gpu(qa):
         return _k().hy_latent_attention(qa, cache, block_table, q_start, pos, gate, scale, rank, max_q, window, two_term, sink)
     return ref.latent_attention(qa, cache, block_table, q_start, pos, gate, scale, rank, act_dtype, window, sink)
+
+
+def latent_expanded_ok(D: int, R: int, Dv: int) -> bool:
+    return _k().hy_latent_expanded_ok(D, R, Dv)
+
+
+def latent_expanded(q, kv, kr, q_start, gate, gate_src, g_off: int, sink, scale: float, max_q: int, window: int = 0, out=None):
+    """Latent attention of sequences that all start at position 0, keys and values written out: q [T, H, D + R] rotated, kv
+    [T, H, D + Dv], kr [T, R] the shared rotated keys (q, kr and ``out`` [T, H, Dv] may be column ranges of wider rows); ``gate``,
+    ``sink`` as in latent_attention, ``gate_src`` columns as in head_matmul.  On the GPU only (bfloat16)."""
+    if out is None:
+        out = torch.empty(*q.shape[:2], kv.shape[2] - q.shape[2] + kr.shape[1], device=q.device, dtype=q.dtype)
+    _k().hy_latent_expanded(q, kv, kr, q_start, gate, gate_src, g_off, sink, out, scale, max_q, window)
+    return out
 
 
 def moe_route(h, w_router, correction, top: int):
