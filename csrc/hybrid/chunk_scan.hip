@@ -30,7 +30,7 @@
 // 857 -> 192; state-space form, 128 heads of 128 x 64: 1058 -> 445; mlstm, 4 heads of 128 x 256: 1987 -> 220, 4 heads of
 // 256 x 512: 3050 -> 303; delta rule, 32 heads of 128 x 128: 959 -> 389.  One and two waves per workgroup: 436 and 302 us
 // where four took 233 (of 171, before addresses, weights and stores lost their branches).
-#include "hybrid_common.h"
+#include "chunk_common.h"
 
 #include <type_traits>
 
@@ -40,46 +40,10 @@ namespace hy {
 constexpr int kCH = 64;   // tokens per chunk
 constexpr int kCW = 4;    // waves per workgroup (NW above)
 
-__device__ __forceinline__ f32x4 mfma_16x16x32(bf16x8 a, bf16x8 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
-// x = h + m + l exactly: each term the bfloat16 nearest to what is left (the second remainder has 8 bits at most)
-struct Terms {
-    bf16x8 h, m, l;
-};
-__device__ __forceinline__ Terms split3(const float (&x)[8]) {
-    Terms t;
-    float a[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        t.h[i] = (__bf16)x[i];
-        a[i] = x[i] - (float)t.h[i];
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        t.m[i] = (__bf16)a[i];
-        a[i] -= (float)t.m[i];
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) t.l[i] = (__bf16)a[i];
-    return t;
-}
-__device__ __forceinline__ bf16x8 join8(bf16x4 a, bf16x4 b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
-
 // e^x with x's digits beyond float32 kept
 __device__ __forceinline__ float exp_d(double x) {
     const float h = (float)x, e = expf(h);
     return e + e * (float)(x - h);
-}
-
-// Where piece c (16 bytes) of row r of a tile with CPR pieces per row lies: c ^ spread<CPR>(r).  16 rows at the same c, and
-// 4 rows at 4 neighbouring c, fall on different banks.  Depends on r % 16 only.
-template <int CPR> __device__ __forceinline__ int spread(int r) {
-    if constexpr (CPR >= 16) return ((r & 3) << 2) | ((r >> 2) & 3);
-    else if constexpr (CPR == 8) return ((r & 2) << 1) | ((r >> 2) & 3);
-    else if constexpr (CPR == 4) return (r >> 2) & 3;
-    else return 0;
 }
 
 // Running sum over the wave's lanes (lane l: the sum of lanes 0 .. l): within rows of 16 lanes, then from row to row.
@@ -128,22 +92,6 @@ template <int D, int MODE> struct ChunkLds {
     static constexpr int OWN = TT + (MODE == kScanDelta ? 4 * 1024 : 0), OWN_SIZE = kCH * (MODE == kScanDelta ? 28 : 16);
     static constexpr int SUM = OWN + kCW * OWN_SIZE, SIZE = SUM + (MODE == kScanMlstm ? 640 + kCW * 256 : 0);
 };
-
-// a * b of two float32 operands in matrix layout (4 elements per lane, k = 4 g + e), as the six leading products of their terms:
-// the other three are below 2^-24 of the result.  The two halves of a 32-deep instruction hold two of the six.
-struct Terms4 {
-    bf16x4 h, m, l;
-};
-__device__ __forceinline__ Terms4 split3(const f32x4& x) {
-    const float v[8] = {x[0], x[1], x[2], x[3], 0.f, 0.f, 0.f, 0.f};
-    const Terms t = split3(v);
-    return {__builtin_shufflevector(t.h, t.h, 0, 1, 2, 3), __builtin_shufflevector(t.m, t.m, 0, 1, 2, 3), __builtin_shufflevector(t.l, t.l, 0, 1, 2, 3)};
-}
-__device__ __forceinline__ f32x4 mul_low(const Terms4& a, const Terms4& b, f32x4 c) {
-    c = mfma_16x16x32(join8(a.m, a.h), join8(b.m, b.l), c);
-    return mfma_16x16x32(join8(a.h, a.l), join8(b.m, b.h), c);
-}
-__device__ __forceinline__ f32x4 mul_high(const Terms4& a, const Terms4& b, f32x4 c) { return mfma_16x16x32(join8(a.h, a.m), join8(b.h, b.h), c); }
 
 template <int D, int MODE>
 __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) chunk_scan_kernel(const ChunkScan a) {

@@ -15,7 +15,8 @@
 //                 with two 2-step cross-lane sums (S^T k and S^T q over the four row groups).  decay is one number per
 //                 head or one per state row.  The same kernel
 //                 serves prompt portions of any length and decode rows (a range of one token); a range that starts at
-//                 position 0 starts from the zero state, so a reused slot needs no clearing.
+//                 position 0 starts from the zero state, so a reused slot needs no clearing.  Prompt portions whose rows
+//                 allow it take chunk_scan.hip (one decay per head) or gla_scan.hip (one per state row).
 #include "hybrid_common.h"
 
 namespace chronos {
@@ -419,6 +420,10 @@ void launch_hy_chunk_scan(const uint16_t*, int, int, int, int, const float*, con
                           const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*, int, int, int, int, int, const float*,
                           hipStream_t);
 
+bool hy_gla_scan_ok(const void*, const void*, int, int, int, int, int, int, int);
+void launch_hy_gla_scan(const uint16_t*, int, int, int, int, const float*, const float*, float, const float*, const int32_t*,
+                        const int32_t*, const int32_t*, float*, float*, int, int, int, int, int, const float*, hipStream_t);
+
 // x points at the first convolved column of the first row (rows ldx apart); bias may be nullptr
 void launch_hy_conv_hist(const void* x, int ldx, const int32_t* q_start, const int32_t* pos0, const int32_t* slots,
                          void* hist, int B, int C, int K, bool f32, hipStream_t s) {
@@ -510,6 +515,11 @@ bool launch_hy_linear_scan(const void* proj, int ldp, int q_off, int k_off, int 
     if (B == 0) return true;
     const bool pipe = T > B;   // some sequence brings more than one token
     const bool delta = beta != nullptr;
+    if (chd && !delta && !f32 && hy_gla_scan_ok(proj, decay, ldp, q_off, k_off, v_off, D, Dv, longest)) {
+        launch_hy_gla_scan((const uint16_t*)proj, ldp, q_off, k_off, v_off, qscale, kscale, q_mul, decay, q_start, pos0, slots, S, o,
+                           B, HK, H, D, Dv, vscale, s);
+        return true;
+    }
     if (!chd && !f32 && hy_chunk_scan_ok(proj, ldp, q_off, k_off, v_off, D, Dv, longest, delta)) {
         launch_hy_chunk_scan((const uint16_t*)proj, ldp, q_off, k_off, v_off, qscale, kscale, q_mul, decay, fixed ? 0 : H, beta,
                              q_start, pos0, slots, S, o, B, HK, H, D, Dv, vscale, s);

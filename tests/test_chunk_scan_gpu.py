@@ -64,6 +64,39 @@ def test_plain(HK, H, D, Dv, form):
     assert torch.equal(S[1], S0[1]) and torch.equal(S[6], S0[6]), "slots without tokens must stay untouched"
 
 
+@pytest.mark.parametrize("HK,H,D,Dv,scales", [(2, 4, 32, 40, True), (1, 2, 64, 64, False), (3, 3, 128, 72, True), (2, 2, 256, 128, False)])
+def test_rows(HK, H, D, Dv, scales):
+    """One decay per state row (csrc/hybrid/gla_scan.hip, 16 tokens at a time, chunks whose products of decays leave the range token by
+    token: the first sequences have some of both, the last two none)."""
+    from chronos.ops import hybrid as hops
+
+    T = sum(LENS)
+    C = 2 * HK * D + H * Dv + 16
+    g, rnd, qs, ranges = _setup(H * D + Dv, T, C, H, D, Dv)
+    proj = rnd(T, C).bfloat16()
+    rand = lambda *s: torch.rand(*s, device=DEV, generator=g)  # noqa: E731
+    decay = rand(T, H, D) ** (1 / 8)
+    decay[3:200:50], decay[9:200:31], decay[11::37], decay[20::29], decay[23::61, :, ::3] = 0.0, 1e-30, 1.0, -0.8, 1.4
+    qsc, ksc, vs = (rand(T, HK), rand(T, HK), rand(T, H)) if scales else (None, None, None)
+    S = rnd(9, H, D, Dv) * 0.3
+    S0 = S.clone()
+    o = hops.linear_scan(proj, 8, 8 + HK * D, 8 + 2 * HK * D, qsc, ksc, 0.7, decay, None, *ranges, S, HK, H, D, Dv, vs, max(LENS))
+    p, one = proj.double(), torch.ones(T, 1, dtype=torch.double, device=DEV)
+    q = (p[:, 8:8 + HK * D].view(T, HK, D) * (qsc.double()[..., None] if scales else 0.7)).repeat_interleave(H // HK, 1)
+    k = (p[:, 8 + HK * D:8 + 2 * HK * D].view(T, HK, D) * (ksc.double() if scales else one)[..., None]).repeat_interleave(H // HK, 1)
+    v = p[:, 8 + 2 * HK * D:8 + 2 * HK * D + H * Dv].view(T, H, Dv) * (vs.double() if scales else one)[..., None]
+    want, Sw = torch.empty(T, H, Dv, dtype=torch.double, device=DEV), S0.double()
+    for b, n in enumerate(LENS):
+        s = torch.zeros(H, D, Dv, dtype=torch.double, device=DEV) if STARTS[b] == 0 else Sw[SLOTS[b]]
+        for t in range(qs[b], qs[b] + n):
+            s = decay[t].double()[..., None] * s + k[t][:, :, None] * v[t][:, None]
+            want[t] = (q[t][:, None] @ s)[:, 0]
+        if n:
+            Sw[SLOTS[b]] = s
+    assert _rel(o, want) < 2e-6 and _rel(S, Sw) < 2e-6
+    assert torch.equal(S[1], S0[1]) and torch.equal(S[6], S0[6]), "slots without tokens must stay untouched"
+
+
 @pytest.mark.parametrize("HK,H,D,Dv,form", [(2, 4, 32, 40, "token"), (2, 2, 64, 64, "head"), (2, 4, 128, 72, "token"), (1, 3, 128, 128, "same")])
 def test_delta(HK, H, D, Dv, form):
     """The delta rule's 16-row solves: keys of length 1, in "same" all nearly one direction with betas near 1 (every token undoes
