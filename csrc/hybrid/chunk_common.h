@@ -14,21 +14,15 @@ struct Terms {
     bf16x8 h, m, l;
 };
 __device__ __forceinline__ Terms split3(const float (&x)[8]) {
-    Terms t;
-    float a[8];
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    u32x4 t[3];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        t.h[i] = (__bf16)x[i];
-        a[i] = x[i] - (float)t.h[i];
+    for (int i = 0; i < 4; ++i) {
+        float a = x[2 * i], b = x[2 * i + 1];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) t[k][i] = round_pair(a, b);
     }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        t.m[i] = (__bf16)a[i];
-        a[i] -= (float)t.m[i];
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) t.l[i] = (__bf16)a[i];
-    return t;
+    return {__builtin_bit_cast(bf16x8, t[0]), __builtin_bit_cast(bf16x8, t[1]), __builtin_bit_cast(bf16x8, t[2])};
 }
 __device__ __forceinline__ bf16x8 join8(bf16x4 a, bf16x4 b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
 

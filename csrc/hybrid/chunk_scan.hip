@@ -27,8 +27,8 @@
 // What bounds it: the chain of a sequence's chunks, one wave per SIMD: vector instructions (the cutting into terms, the
 // exponentials) and 114 matrix instructions (delta: 162) per chunk and wave at D = 128, and two barriers, 5 us a chunk (delta: 10).
 // Measured, 4 sequences of 2048 tokens, token by token -> this: retention, 8 heads of 128 x 128: 797 -> 171 us; 32 heads:
-// 857 -> 192; state-space form, 128 heads of 128 x 64: 1058 -> 445; mlstm, 4 heads of 128 x 256: 1987 -> 220, 4 heads of
-// 256 x 512: 3050 -> 303; delta rule, 32 heads of 128 x 128: 959 -> 389.  One and two waves per workgroup: 436 and 302 us
+// 857 -> 192; state-space form, 128 heads of 128 x 64: 1058 -> 434; mlstm, 4 heads of 128 x 256: 1987 -> 220, 4 heads of
+// 256 x 512: 3050 -> 291; delta rule, 32 heads of 128 x 128: 959 -> 366.  One and two waves per workgroup: 436 and 302 us
 // where four took 233 (of 171, before addresses, weights and stores lost their branches).
 #include "chunk_common.h"
 

@@ -14,10 +14,10 @@
 // F q, half w k / F (two rows of 8 tokens each), shared through LDS as terms, and each wave reads out and updates its columns.
 //
 // What bounds it: the chain of a sequence's chunks, one wave per SIMD: about 600 vector and 66 matrix instructions a chunk and wave at
-// D = 128, two barriers and the LDS reads between them, 3.1 us.  Measured, 4 sequences of 2048 tokens, 16 heads of 128 x 256: token by
-// token 988 us, this 448; one of 4000, 8 heads: 1684 and 771.  P on the vector ALUs from running products: 648 us, and the same
+// D = 128, two barriers and the LDS reads between them, 2.8 us.  Measured, 4 sequences of 2048 tokens, 16 heads of 128 x 256: token by
+// token 988 us, this 403; one of 4000, 8 heads: 1684 and 697.  P on the vector ALUs from running products: 648 us, and the same
 // with F in float32: state 9.6e-8 of its norm off the float64 recurrence (token by token 8.7e-8, this 7.8e-8); with the stores of a
-// chunk waited for by the next: 482 us.
+// chunk waited for by the next: 482 us, with that 448, and the terms rounded in pairs 403.
 #include "chunk_common.h"
 
 #include <type_traits>
@@ -161,12 +161,7 @@ __global__ void __launch_bounds__(256, 1) gla_scan_kernel(const GlaScan a) {
         auto put = [&](int base, int t, int rp, float x, float y) {   // the terms of rows 2 rp, 2 rp + 1 of token t
             unsigned char* at = gs_smem + base + t * (D * 2) + (((rp >> 2) ^ spread<CPR>(t)) * 16) + (rp & 3) * 4;
 #pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const __bf16 u = (__bf16)x, v = (__bf16)y;
-                *reinterpret_cast<uint32_t*>(at + k * M::Q) = (uint32_t)__builtin_bit_cast(uint16_t, v) << 16 | __builtin_bit_cast(uint16_t, u);
-                x -= (float)u;
-                y -= (float)v;
-            }
+            for (int k = 0; k < 3; ++k) *reinterpret_cast<uint32_t*>(at + k * M::Q) = round_pair(x, y);
         };
         const bool keys = tid >= 128;   // (wave-uniform)
         const uint16_t* const src = keys ? ks : qs;
@@ -311,7 +306,7 @@ __global__ void __launch_bounds__(256, 1) gla_scan_kernel(const GlaScan a) {
 
 // When this form serves a launch: bfloat16 rows of q, k, v and rows of decays on 16-byte boundaries, a state of 32, 64, 128 or 256
 // rows, and a sequence of at least 4 new tokens (longest: the most that any sequence brings): 21 sequences of n tokens, 4 heads of
-// 128 x 256, token by token / here, us: 9.2 / 9.8 at n = 2, 10.9 / 10.1 at 4, 14.0 / 10.3 at 8, 21 / 10.3 at 16, 109 / 43 at 117.
+// 128 x 256, token by token / here, us: 9.2 / 9.8 at n = 2, 10.9 / 9.8 at 4, 14.0 / 9.8 at 8, 21 / 9.9 at 16, 109 / 39 at 117.
 bool hy_gla_scan_ok(const void* proj, const void* decay, int ldp, int q_off, int k_off, int v_off, int D, int Dv, int longest) {
     return longest >= 4 && (D == 32 || D == 64 || D == 128 || D == 256) && Dv % 8 == 0 && hy::aligned16(proj, decay) &&
            ((ldp | q_off | k_off | v_off) & 7) == 0 && ldp < 1 << 23;

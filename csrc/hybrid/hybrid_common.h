@@ -100,6 +100,17 @@ template <int CPR> __device__ __forceinline__ void dma_rows(const uint16_t* src,
     dma_1k(src + (int64_t)rows[row] * width + min(ch, n - 1) * 8, __builtin_amdgcn_readfirstlane(lds + j * 1024));
 }
 
+// bfloat16 of a (lower half) and b, and what the rounding leaves of them.  Taken apart as a word: the compiler would convert each a second
+// time, alone, to have it back as a float.
+__device__ __forceinline__ uint32_t round_pair(float& a, float& b) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
+    a -= __uint_as_float(u << 16);
+    b -= __uint_as_float(u & 0xffff0000u);
+    return u;
+}
+
 constexpr int kActRelu2 = 0, kActGelu = 1;
 __device__ __forceinline__ float act_apply(float z, int kind) {
     if (kind == kActRelu2) {

@@ -25,6 +25,9 @@
 // merge the float partials in a second kernel.
 // With unit keys (SH: a key is the cached value times a float factor) the one image serves both products, and a score is
 // multiplied by its key's factor.
+// Blocks of late rows see the most keys: they start first (in full causal attention over 4 x 2048 tokens, 8 heads of 128, 122 us with the
+// blocks in order, 89 so).  Two sets of 16 rows per wave halve the LDS reads and win nothing (50 us where one set takes 48, window 512):
+// what bounds a tile is the vector instructions of its softmax, 160 per wave and 17 exponentials, beside 48 matrix instructions.
 // With chunk > 0 a row also hides the keys below its own chunk of positions (key >= floor(pos / chunk) * chunk).
 // Sizes: D % 8 == 0, Dv % 16 == 0, D <= 256, Dv <= 256.  Everything else takes the general kernel.
 #include <algorithm>
@@ -53,11 +56,15 @@ __global__ void __launch_bounds__(64 * NW) window_attention_mfma_kernel(
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     constexpr int KT = WKT, RPB = 16 * NW / KS;
     const int R = H / G;
-    const int b = blockIdx.x, kvh = blockIdx.z;
+    // blockIdx.x: sequence and key/value head; blockIdx.y: row block and split, later blocks (which see more keys) first.  Where two
+    // workgroups per CU hold the whole launch its second half runs the other way, so that a CU gets a long walk and a short one.
+    const int b = blockIdx.x / G, kvh = blockIdx.x % G;
     const int t0 = q_start[b], t1 = q_start[b + 1];
     const int rows_total = (t1 - t0) * R;
-    const int split = blockIdx.y % nsplit;   // key tiles are dealt round-robin to the nsplit workgroups of a row block
-    const int rb0 = blockIdx.y / nsplit * RPB;
+    const int ny = gridDim.y, y0 = blockIdx.y, half = ny / 2;
+    const int y = gridDim.x * ny <= 512 && y0 >= ny - half ? y0 - (ny - half) : ny - 1 - y0;
+    const int split = y % nsplit;   // key tiles are dealt round-robin to the nsplit workgroups of a row block
+    const int rb0 = y / nsplit * RPB;
     if (rb0 >= rows_total) return;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, g4 = lane >> 4, qi = lane & 15;
     const int nct = Dv / 16;
@@ -234,13 +241,15 @@ __global__ void __launch_bounds__(64 * NW) window_attention_mfma_kernel(
         }
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
-            bf16x8 pf, pl;
+            typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+            u32x4 whi, wlo;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float w = S[2 * u + (e >> 2)][e & 3];
-                pf[e] = (__bf16)w;
-                pl[e] = (__bf16)(w - (float)pf[e]);
+            for (int e = 0; e < 4; ++e) {
+                float w0 = S[2 * u + (e >> 1)][2 * (e & 1)], w1 = S[2 * u + (e >> 1)][2 * (e & 1) + 1];
+                whi[e] = round_pair(w0, w1);
+                wlo[e] = round_pair(w0, w1);
             }
+            const bf16x8 pf = __builtin_bit_cast(bf16x8, whi), pl = __builtin_bit_cast(bf16x8, wlo);
 #pragma unroll
             for (int c = 0; c < NCT; ++c) {
                 const bf16x4 lo = lds_read_tr4(vt + 32 * u * vrs + c * 32);
@@ -420,7 +429,7 @@ static void wa_mfma_launch(const uint16_t* qkv, int ldq, const uint16_t* kc, con
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
         set_bytes = bytes;
     }
-    const dim3 grid(B, (max_q * (H / G) + 16 * NW / KS - 1) / (16 * NW / KS) * nsplit, G);
+    const dim3 grid(B * G, (max_q * (H / G) + 16 * NW / KS - 1) / (16 * NW / KS) * nsplit);
     kern<<<grid, 64 * NW, bytes, s>>>(qkv, ldq, kc, vc, bt, max_blocks, q_start, pos, sink, gate, out, H, G, D, Dv, BS, scale,
                                       window, keep, chunk, nsplit, part_o, part_ml, pool, EP, kp, vp, vcs, g_off, ks, ldo);
 }
@@ -429,7 +438,10 @@ bool hy_window_mfma_ok(int ldq, int D, int Dv) { return !(D % 8 || Dv % 16 || D 
 
 // Splits of a row block's key tiles over workgroups (merged by a combine kernel) for launches that would leave most
 // of the chip idle — decode rows, a lone short portion: enough workgroups to cover the CUs twice (four times for few
-// rows with unit keys, whose workgroups need half the LDS), at least 2 key tiles per split, at most 16.  The tile count
+// rows with unit keys, whose workgroups need half the LDS), at least 2 key tiles per split, at most 16.  Prompt portions (more than 64
+// rows) write and read far more partials than decode rows: 3 tiles, and 8 from half a workgroup per CU on (us, 8 heads, 2 of keys, splits of
+// 2 tiles / none: 1 x 700 tokens, 44 workgroups 22 / 30; 1 x 300, 20 workgroups 15.5 / 17.6; 8 x 117, 64 workgroups of 3 tiles 16.4 / 11.1;
+// 21 x 117, 168 workgroups 26 / 12; 8 x 300, 160 workgroups 32 / 19).  The tile count
 // follows from sizes the host knows (the window, or the block table's width when there is none).  1 for float32 and
 // sizes the matrix-core kernel does not serve.
 int hy_window_nsplit(bool f32, int ldq, int B, int max_q, int H, int G, int D, int Dv, int window, int keep, int chunk,
@@ -444,7 +456,7 @@ int hy_window_nsplit(bool f32, int ldq, int B, int max_q, int H, int G, int D, i
     const int tiles = span / hy::WKT + 1 + (window > 0 ? (std::min(keep, max_ctx) + hy::WKT - 1) / hy::WKT : 0) +
                       (window > 0 && pool > 0 ? (max_ctx / pool + hy::WKT - 1) / hy::WKT : 0);
     int want = (enough + wgs - 1) / wgs;
-    want = std::min(want, std::min(16, tiles / 2));
+    want = std::min(want, std::min(16, tiles / (rows <= 64 ? 2 : wgs < 128 ? 3 : 8)));
     return want < 1 ? 1 : want;
 }
 
