@@ -16,7 +16,7 @@
 //                 head or one per state row.  The same kernel
 //                 serves prompt portions of any length and decode rows (a range of one token); a range that starts at
 //                 position 0 starts from the zero state, so a reused slot needs no clearing.  Prompt portions whose rows
-//                 allow it take chunk_scan.hip (one decay per head) or gla_scan.hip (one per state row).
+//                 allow it take chunk_scan.hip (one decay per head) or gla_scan.hip (one per state row), decode rows state_step.hip.
 #include "hybrid_common.h"
 
 namespace chronos {
@@ -424,6 +424,11 @@ bool hy_gla_scan_ok(const void*, const void*, int, int, int, int, int, int, int)
 void launch_hy_gla_scan(const uint16_t*, int, int, int, int, const float*, const float*, float, const float*, const int32_t*,
                         const int32_t*, const int32_t*, float*, float*, int, int, int, int, int, const float*, hipStream_t);
 
+bool hy_state_step_ok(const void*, const void*, const void*, int, int, int, int, int);
+void launch_hy_state_step(const uint16_t*, int, int, int, int, const float*, const float*, float, const float*, bool, int,
+                          const float*, const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*, int, int, int,
+                          int, int, const float*, hipStream_t);
+
 // x points at the first convolved column of the first row (rows ldx apart); bias may be nullptr
 void launch_hy_conv_hist(const void* x, int ldx, const int32_t* q_start, const int32_t* pos0, const int32_t* slots,
                          void* hist, int B, int C, int K, bool f32, hipStream_t s) {
@@ -515,6 +520,11 @@ bool launch_hy_linear_scan(const void* proj, int ldp, int q_off, int k_off, int 
     if (B == 0) return true;
     const bool pipe = T > B;   // some sequence brings more than one token
     const bool delta = beta != nullptr;
+    if (!f32 && hy_state_step_ok(proj, S, o, ldp, v_off, D, Dv, longest)) {
+        launch_hy_state_step((const uint16_t*)proj, ldp, q_off, k_off, v_off, qscale, kscale, q_mul, decay, chd, fixed ? 0 : H, beta, nullptr,
+                             q_start, pos0, slots, S, o, B, HK, H, D, Dv, vscale, s);
+        return true;
+    }
     if (chd && !delta && !f32 && hy_gla_scan_ok(proj, decay, ldp, q_off, k_off, v_off, D, Dv, longest)) {
         launch_hy_gla_scan((const uint16_t*)proj, ldp, q_off, k_off, v_off, qscale, kscale, q_mul, decay, q_start, pos0, slots, S, o,
                            B, HK, H, D, Dv, vscale, s);

@@ -8,7 +8,7 @@
 //   S_t = a_t S_{t-1} + b_t k_t v_t^T              n_t = a_t n_{t-1} + b_t k_t
 //   o_t = S_t^T q_t / (max(|n_t . q_t|, exp(-m_t)) + 1e-6),   q_t scaled by D^-1/2
 //
-// Token by token, in three launches (launches whose longest range has 16 tokens and more take chunk_scan.hip's form in
+// Token by token, in three launches (decode rows take state_step.hip for the state, launches whose longest range has 16 tokens and more chunk_scan.hip's form in
 // place of the first two):
 //   gate_scan    one wave per (sequence, head): the scalar recurrences a_t, b_t and the denominators (n lives in the
 //                wave's lanes); sequential in t but only O(D) work per token;
@@ -403,10 +403,15 @@ __global__ void __launch_bounds__(256) mlstm_out_vec_kernel(const float* __restr
 
 }  // namespace hy
 
+bool hy_state_step_ok(const void*, const void*, const void*, int, int, int, int, int);
+void launch_hy_state_step(const uint16_t*, int, int, int, int, const float*, const float*, float, const float*, bool, int,
+                          const float*, const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*, int, int, int,
+                          int, int, const float*, hipStream_t);
+
 template <typename T>
 static void mlstm_scan_t(const T* proj, int ldp, const float* gate_pre, const int32_t* q_start, const int32_t* pos0,
                          const int32_t* slots, float* S, float* n, float* m, float* a, float* b, float* den, float* o,
-                         int B, int H, int D, int Dv, float cap, hipStream_t s) {
+                         int B, int H, int D, int Dv, float cap, int longest, hipStream_t s) {
     // tokens per gate-scan block: as many (<= 64) as keep the staged k and q rows within 40 KB
     int TG = 64;
     while (TG > 1 && (size_t)TG * 2 * D * sizeof(T) > 40 * 1024) TG >>= 1;
@@ -414,6 +419,12 @@ static void mlstm_scan_t(const T* proj, int ldp, const float* gate_pre, const in
     const int gvec = ldp % gev == 0 && D % gev == 0;  // q and k rows start and end on 16-byte boundaries
     hy::mlstm_gate_scan_kernel<T><<<dim3(B, H), 256, (size_t)TG * 2 * D * sizeof(T) + 5 * 64 * 4 + 64 * 65 * 4, s>>>(
         proj, ldp, gate_pre, q_start, pos0, slots, n, m, a, b, den, H, D, cap, TG, gvec);
+    if constexpr (sizeof(T) == 2)
+        if (hy_state_step_ok(proj, S, o, ldp, 2 * H * D, D, Dv, longest)) {
+            launch_hy_state_step(proj, ldp, 0, H * D, 2 * H * D, nullptr, nullptr, 1.f / sqrtf((float)D), a, false, H, nullptr, den, q_start, pos0,
+                                 slots, S, o, B, H, H, D, Dv, b, s);
+            return;
+        }
     const dim3 grid(B, H, (Dv + 63) / 64);
     // rows of q, k, v on 16-byte boundaries: the vector-load kernel with the next stage prefetched (its LDS stays
     // within the static 64 KB up to D = 256); anything else: the plain one
@@ -445,8 +456,8 @@ void launch_hy_mlstm_scan(const void* proj, int ldp, const float* gate_pre, cons
         return;
     }
     float *a = scratch, *b = a + (int64_t)T * H, *den = b + (int64_t)T * H;
-    if (f32) mlstm_scan_t<float>((const float*)proj, ldp, gate_pre, q_start, pos0, slots, S, n, m, a, b, den, o, B, H, D, Dv, cap, s);
-    else mlstm_scan_t<uint16_t>((const uint16_t*)proj, ldp, gate_pre, q_start, pos0, slots, S, n, m, a, b, den, o, B, H, D, Dv, cap, s);
+    if (f32) mlstm_scan_t<float>((const float*)proj, ldp, gate_pre, q_start, pos0, slots, S, n, m, a, b, den, o, B, H, D, Dv, cap, longest, s);
+    else mlstm_scan_t<uint16_t>((const uint16_t*)proj, ldp, gate_pre, q_start, pos0, slots, S, n, m, a, b, den, o, B, H, D, Dv, cap, longest, s);
 }
 
 // silu_gate: the gate columns pass SiLU instead of the sigmoid (the read-out of the linear-state mixers)

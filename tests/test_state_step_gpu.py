@@ -1,0 +1,74 @@
+"""One token per sequence of the recurrences (csrc/hybrid/state_step.hip): every form against one step in float64, sequences without a token,
+fresh ones, columns off the lanes' tiles.
+
+Tolerance: float32 rounding, 2^-24 per operation, of sums over at most 256 rows: 2^-24 sqrt(256) = 1e-6 of the result's norm, taken twice."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+COUNT, STARTS, SLOTS = [1, 0, 1, 1, 1], [0, 3, 9, 1, 4], [2, 5, 0, 4, 1]
+
+
+@pytest.mark.parametrize("form", ["fixed", "token", "rows", "delta", "delta_rows", "mlstm"])
+@pytest.mark.parametrize("HK,H,D,Dv", [(2, 4, 32, 40), (2, 2, 64, 64), (1, 3, 128, 72), (4, 4, 128, 256), (2, 2, 256, 516)])
+def test_step(form, HK, H, D, Dv):
+    from chronos.ops import hybrid as hops
+
+    if form == "mlstm":
+        HK = H
+    T = sum(COUNT)
+    g = torch.Generator(device=DEV).manual_seed(H * D + Dv)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
+    rand = lambda *s: torch.rand(*s, device=DEV, generator=g)  # noqa: E731
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    qs = [0]
+    for n in COUNT:
+        qs.append(qs[-1] + n)
+    proj = rnd(T, 2 * HK * D + H * Dv + 12).bfloat16()
+    S = rnd(7, H, D, Dv)
+    S0, p = S.clone(), proj.double()
+    q, k = (p[:, i * HK * D:(i + 1) * HK * D].view(T, HK, D) for i in (0, 1))
+    v = p[:, 2 * HK * D:2 * HK * D + H * Dv].view(T, H, Dv)
+    ranges = (i32(qs), i32(STARTS), i32(SLOTS))
+    beta = vs = None
+    if form == "mlstm":
+        n, m, gp = rnd(7, H, D), rnd(7, H), rnd(T, 2 * H)
+        n0, m0 = n.double(), m.double()
+        o = hops.mlstm_scan(proj, gp, *ranges, S, n, m, H, D, Dv, 9.0, 1)
+        ig, fg = 9 * torch.tanh(gp[:, :H].double() / 9), torch.nn.functional.logsigmoid(9 * torch.tanh(gp[:, H:].double() / 9))
+    else:
+        delta = form.startswith("delta")
+        dec = rand(H) if form == "fixed" else rand(T, H, D) if form.endswith("rows") else rand(T, H)
+        qsc, ksc = (rand(T, HK), rand(T, HK)) if form != "fixed" else (None, None)
+        beta = rand(T, H) if delta else None
+        vs = rand(T, H) if form == "token" else None
+        o = hops.linear_scan(proj, 0, HK * D, 2 * HK * D, qsc, ksc, 0.3, dec, beta, *ranges, S, HK, H, D, Dv, vs, 1)
+        q = q * (qsc.double()[..., None] if qsc is not None else 0.3)
+        k = k * (ksc.double()[..., None] if ksc is not None else 1.0)
+        d = dec.double().expand(T, H) if dec.dim() < 3 else dec.double()
+    q, k = q.repeat_interleave(H // HK, 1), k.repeat_interleave(H // HK, 1)
+    want, Sw = torch.empty(T, H, Dv, dtype=torch.double, device=DEV), S0.double()
+    for b, cnt in enumerate(COUNT):
+        if not cnt:
+            continue
+        t, sl, keep = qs[b], SLOTS[b], float(STARTS[b] > 0)
+        s = Sw[sl] * keep
+        if form == "mlstm":
+            mn = torch.maximum(fg[t] + m0[sl] * keep, ig[t])
+            a, w = torch.exp(fg[t] + m0[sl] * keep - mn), torch.exp(ig[t] - mn)
+            s = a[:, None, None] * s + (w[:, None] * k[t])[:, :, None] * v[t][:, None]
+            nn = a[:, None] * n0[sl] * keep + w[:, None] * k[t]
+            qt = q[t] * D ** -0.5
+            want[t] = (qt[:, None] @ s)[:, 0] / (torch.maximum((nn * qt).sum(-1).abs(), torch.exp(-mn)) + 1e-6)[:, None]
+        else:
+            s = d[t].view(H, -1, 1) * s
+            u = v[t] * (vs[t].double()[:, None] if vs is not None else 1.0)
+            if beta is not None:
+                u = beta[t].double()[:, None] * (u - (k[t][:, None] @ s)[:, 0])
+            s = s + k[t][:, :, None] * u[:, None]
+            want[t] = (q[t][:, None] @ s)[:, 0]
+        Sw[sl] = s
+    assert float((o.double() - want).norm() / want.norm()) < 2e-6
+    assert float((S.double() - Sw).norm() / Sw.norm()) < 2e-6
+    assert torch.equal(S[3], S0[3]) and torch.equal(S[5], S0[5]) and torch.equal(S[6], S0[6])
