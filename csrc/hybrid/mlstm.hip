@@ -8,8 +8,8 @@
 //   S_t = a_t S_{t-1} + b_t k_t v_t^T              n_t = a_t n_{t-1} + b_t k_t
 //   o_t = S_t^T q_t / (max(|n_t . q_t|, exp(-m_t)) + 1e-6),   q_t scaled by D^-1/2
 //
-// Token by token, in three launches (decode rows take state_step.hip for the state, launches whose longest range has 16 tokens and more chunk_scan.hip's form in
-// place of the first two):
+// Token by token, in three launches (decode rows take state_step.hip in place of the second, launches whose longest range has 16
+// tokens and more chunk_scan.hip's form in place of the first two):
 //   gate_scan    one wave per (sequence, head): the scalar recurrences a_t, b_t and the denominators (n lives in the
 //                wave's lanes); sequential in t but only O(D) work per token;
 //   state_scan   one workgroup per (sequence, head, 64 value columns): S in registers (lane = column, the D rows

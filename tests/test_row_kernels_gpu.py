@@ -115,3 +115,33 @@ def test_window_prep(H, G, D, Dv, dims, norm, v_rot, v_k, mix):
     assert torch.equal(a[:, H * D:], qkv[:, H * D:]), "only queries are rewritten"
     if not mix:
         assert torch.equal(v1, v2)
+
+
+@pytest.mark.parametrize("T,F,pad", [(1, 8, 0), (3, 2056, 0), (5, 2064, 8), (4, 12, 0), (2, 2048, 4)])
+def test_glu(T, F, pad):
+    """16 bytes per lane and what does not allow it (F % 8, rows off 16 bytes).  Tolerance: the result's rounding to bfloat16, half a last
+    place or 2^-8 of the value, and the hardware's sigmoid, 1e-6."""
+    from chronos.ops import hybrid as hops
+
+    g = torch.Generator(device=DEV).manual_seed(F)
+    gu = (torch.randn(T, 2 * F + pad, device=DEV, generator=g) * 4).bfloat16()
+    y = torch.empty(T, F + pad, device=DEV, dtype=torch.bfloat16)
+    hops.glu_cols(gu, 0, F, 7.0, 1.702, 1.0, y[:, :F])
+    a, u = gu[:, :F].double().clamp(max=7.0), gu[:, F:2 * F].double().clamp(-7.0, 7.0)
+    want = a * torch.sigmoid(1.702 * a) * (u + 1.0)
+    assert ((y[:, :F].double() - want).abs() <= want.abs() * (2 ** -8 + 1e-5) + 1e-6).all()
+
+
+@pytest.mark.parametrize("n,p", [(4, 1 / 16), (4099, 1 / 16), (4096, 1 / 8), (4096, 1.0), (4096, 2.5)])
+def test_decay_pow(n, p):
+    """Both forms, at the ends of the range: a few float32 roundings of p log sigmoid(z) (2^-24 of up to 7 p) and of the result."""
+    from chronos.ops import hybrid as hops
+
+    g = torch.Generator(device=DEV).manual_seed(n)
+    z = torch.randn(n, device=DEV, generator=g) * 4
+    z[:4] = torch.tensor([float("inf"), -float("inf"), 100.0, 0.0], device=DEV)
+    want = torch.exp(p * torch.nn.functional.logsigmoid(z.double()))
+    got = hops.decay_pow(z.clone(), p)
+    assert ((got.double() - want).abs() <= want * (2 ** -22 + 2 ** -20 * p)).all()
+    nan = torch.full((4,), float("nan"), device=DEV)
+    assert hops.decay_pow(nan, p).isnan().all()
