@@ -19,7 +19,9 @@ void launch_hy_layer_norm(const void*, bool, float*, const float*, void*, bool, 
 void launch_hy_rowdot(const void*, const void*, const float*, float*, int, int, int, bool, hipStream_t);
 void launch_hy_act(void*, int64_t, int, bool, hipStream_t);
 void launch_hy_mlstm_scan(const void*, int, const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*,
-                          float*, float*, float*, int, int, int, int, int, float, int, bool, hipStream_t);
+                          float*, float*, float*, int, int, int, int, int, float, int, int, bool, hipStream_t);
+int hy_chunk_segments(int, int, int, int, int);
+int64_t hy_chunk_segment_floats(int, int, int, int, int);
 void launch_hy_mlstm_out(const float*, const void*, int, int, const float*, void*, int, int, int, float, bool,
                          hipStream_t);
 void launch_hy_latent_prep(void*, int64_t, const void*, int64_t, const int32_t*, const int32_t*, const int32_t*, int,
@@ -83,7 +85,7 @@ void launch_hy_delta_prep(const void*, int, const float*, const float*, float*, 
                           float, bool, hipStream_t);
 bool launch_hy_linear_scan(const void*, int, int, int, int, const float*, const float*, float, const float*, bool, bool,
                            const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*, int, int, int, int,
-                           int, int, const float*, int, bool, hipStream_t);
+                           int, int, const float*, int, int, float*, bool, hipStream_t);
 void launch_hy_moe_route_topk(const void*, const void*, const float*, float*, int32_t*, float*, int, int, int, int, bool,
                               hipStream_t);
 void launch_hy_moe_glu_grouped(const uint16_t*, const int32_t*, const float*, const uint16_t*, const uint16_t*, uint16_t*,
@@ -201,11 +203,13 @@ Tensor hy_mlstm_scan(const Tensor& proj, const Tensor& gate_pre, const Tensor& q
     need(m.dim() == 2 && m.size(0) == S.size(0) && m.size(1) == H, "mlstm_scan: m [NS, H]");
     need(D >= 1 && D <= 512 && H >= 1 && Dv >= 1, "mlstm_scan: 1 <= D <= 512");
     auto o = at::empty({T, H, Dv}, proj.options().dtype(at::kFloat));
-    auto scratch = at::empty({3 * T * H + B * H * D}, proj.options().dtype(at::kFloat));
+    const int mq = longest(T, B, max_q), segs = f32(proj) ? 1 : chronos::hy_chunk_segments((int)B, (int)H, (int)D, (int)Dv, mq);
+    auto scratch = at::empty({3 * T * H + B * H * D + chronos::hy_chunk_segment_floats((int)B, (int)H, (int)D, (int)Dv, segs)},
+                             proj.options().dtype(at::kFloat));
     chronos::launch_hy_mlstm_scan(proj.data_ptr(), (int)proj.size(1), gate_pre.data_ptr<float>(),
                                   q_start.data_ptr<int32_t>(), pos0.data_ptr<int32_t>(), slots.data_ptr<int32_t>(),
                                   S.data_ptr<float>(), n.data_ptr<float>(), m.data_ptr<float>(), scratch.data_ptr<float>(),
-                                  o.data_ptr<float>(), (int)T, (int)B, (int)H, (int)D, (int)Dv, (float)cap, longest(T, B, max_q), f32(proj), stream());
+                                  o.data_ptr<float>(), (int)T, (int)B, (int)H, (int)D, (int)Dv, (float)cap, mq, segs, f32(proj), stream());
     return o;
 }
 
@@ -780,12 +784,15 @@ Tensor hy_linear_scan(const Tensor& proj, int64_t q_off, int64_t k_off, int64_t 
     need(S.dim() == 4 && S.size(1) == H && S.size(2) == D && S.size(3) == Dv, "linear_scan: S [NS, H, D, Dv]");
     auto o = at::empty({T, H, Dv}, proj.options().dtype(at::kFloat));
     if (T == 0) return o;
+    const int mq = longest(T, B, max_q), segs = f32(proj) || chd || beta ? 1 : chronos::hy_chunk_segments((int)B, (int)H, (int)D, (int)Dv, mq);
+    Tensor seg;
+    if (segs > 1) seg = at::empty({chronos::hy_chunk_segment_floats((int)B, (int)H, (int)D, (int)Dv, segs)}, S.options());
     const bool ok = chronos::launch_hy_linear_scan(
         proj.data_ptr(), (int)C, (int)q_off, (int)k_off, (int)v_off, qscale ? qscale->data_ptr<float>() : nullptr,
         kscale ? kscale->data_ptr<float>() : nullptr, (float)q_mul, decay.data_ptr<float>(), chd, fixed,
         beta ? beta->data_ptr<float>() : nullptr, q_start.data_ptr<int32_t>(), pos0.data_ptr<int32_t>(),
         slots.data_ptr<int32_t>(), S.data_ptr<float>(), o.data_ptr<float>(), (int)T, (int)B, (int)HK, (int)H, (int)D, (int)Dv,
-        vscale ? vscale->data_ptr<float>() : nullptr, longest(T, B, max_q), f32(proj), stream());
+        vscale ? vscale->data_ptr<float>() : nullptr, mq, segs, segs > 1 ? seg.data_ptr<float>() : nullptr, f32(proj), stream());
     TORCH_CHECK(ok, "chronos hybrid op: linear_scan keeps a state column in registers, D <= 256 (got ", D, ")");
     return o;
 }

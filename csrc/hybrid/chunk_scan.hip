@@ -26,12 +26,14 @@
 //
 // What bounds it: the chain of a sequence's chunks, one wave per SIMD: vector instructions (the cutting into terms, the
 // exponentials) and 114 matrix instructions (delta: 162) per chunk and wave at D = 128, and two barriers, 5 us a chunk (delta: 10).
-// Measured, 4 sequences of 2048 tokens, token by token -> this: retention, 8 heads of 128 x 128: 797 -> 171 us; 32 heads:
-// 857 -> 192; state-space form, 128 heads of 128 x 64: 1058 -> 434; mlstm, 4 heads of 128 x 256: 1987 -> 220, 4 heads of
-// 256 x 512: 3050 -> 291; delta rule, 32 heads of 128 x 128: 959 -> 366.  One and two waves per workgroup: 436 and 302 us
-// where four took 233 (of 171, before addresses, weights and stores lost their branches).
+// Measured, 4 sequences of 2048 tokens, token by token -> this: retention, 8 heads of 128 x 128: 797 -> 168 us, in four
+// segments 68; 32 heads: 857 -> 177; state-space form, 128 heads of 128 x 64: 1058 -> 434; mlstm, 4 heads of 128 x 256: 1987
+// -> 220, in four segments 97, 4 heads of 256 x 512: 3050 -> 299, in two 220; delta rule, 32 heads of 128 x 128: 959 -> 366.
+// One and two waves per workgroup: 436 and 302 us where four took 233 (of 171, before addresses, weights and stores lost
+// their branches).
 #include "chunk_common.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace chronos {
@@ -81,6 +83,10 @@ struct ChunkScan {
     const float* n0;   // [B, H, D]: the normaliser before the step (workgroups of one (sequence, head) start at any time)
     float *S, *n, *o;
     int B, HK, H, Dv;
+    // more than one segment per sequence: states before it [B, H, D, Dv], then of each segment but the last; mlstm: normalisers and all:
+    // products of decays of each segment but the last, [segs - 1, B, H, ..]
+    int segs;
+    float *seg_s, *seg_n, *seg_d;
 };
 
 // LDS (bytes): two buffers of q | k | v | weight tiles [10][64 lanes] x 16 (delta: and the solve's tiles [10], the inverses of
@@ -93,7 +99,8 @@ template <int D, int MODE> struct ChunkLds {
     static constexpr int SUM = OWN + kCW * OWN_SIZE, SIZE = SUM + (MODE == kScanMlstm ? 640 + kCW * 256 : 0);
 };
 
-template <int D, int MODE>
+// STATE: the first pass over segments, which only carries the state on (each from 0, the first from the sequence's state)
+template <int D, int MODE, bool STATE>
 __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) chunk_scan_kernel(const ChunkScan a) {
     using M = ChunkLds<D, MODE>;
     constexpr bool DELTA = MODE == kScanDelta, MLSTM = MODE == kScanMlstm;
@@ -110,13 +117,17 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
     float *const bs = cs + kCH, *const bk = bs + kCH, *const be = bk + kCH;            // delta
     float* const psum = reinterpret_cast<float*>(cs_smem + M::SUM);                    // mlstm
     float* const nq = psum + 160;
-    // groups of workgroups that share q and k rows go to one XCD (workgroup i runs on XCD i % 8)
-    const int nslab = (a.Dv + 16 * NW - 1) / (16 * NW), id = blockIdx.x >> 3;
-    const int group = (id / nslab) * 8 + (blockIdx.x & 7), slab = id % nslab;
+    // groups of workgroups that share q and k rows go to one XCD (workgroup i runs on XCD i % 8), the next segment's behind them: less
+    // than 8 groups leave XCDs free
+    const int nslab = (a.Dv + 16 * NW - 1) / (16 * NW), id = blockIdx.x >> 3, seg = blockIdx.y;
+    const int group = (id / nslab) * 8 + ((blockIdx.x - seg * a.B * a.H) & 7), slab = id % nslab;
     if (group >= a.B * a.H) return;
     const int b = group / a.H, hd = group % a.H, hk = hd / (a.H / a.HK);
-    const int t0 = a.q_start[b], t1 = a.q_start[b + 1];
-    if (t1 <= t0) return;
+    const int s0 = a.q_start[b], t1 = a.q_start[b + 1];
+    if (t1 <= s0) return;
+    const int chunks = (t1 - s0 + kCH - 1) / kCH;
+    const int t0 = s0 + chunks * seg / a.segs * kCH, te = min(t1, s0 + chunks * (seg + 1) / a.segs * kCH);   // this segment's tokens
+    const int64_t cells = (int64_t)a.B * a.H;
     const int c0 = slab * 16 * NW, col = c0 + wv * 16 + ln;
     const bool live = col < a.Dv;
     const int64_t srow = (int64_t)a.slots[b] * a.H + hd;
@@ -124,22 +135,57 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
     const bool fresh = a.pos0[b] == 0;
     // S[2 kk + h], element r of lane group g: row 32 kk + 8 g + 4 h + r (what the read-out's product takes from that lane)
     f32x4 S[2 * KK];
-#pragma unroll
-    for (int i = 0; i < 2 * KK; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) S[i][r] = !fresh && live ? Sp[(int64_t)((i >> 1) * 32 + 8 * g + 4 * (i & 1) + r) * a.Dv] : 0.f;
-    // mlstm: the normaliser n likewise, the 32-row steps dealt to the waves (every column of the accumulator the same)
+    auto row_of = [&](int i, int r) { return (i >> 1) * 32 + 8 * g + 4 * (i & 1) + r; };
+    // element r of S[i] of a state at `at` (this lane's column of its first row)
+    auto take = [&](const float* at, int i, int r) { return live ? at[(int64_t)row_of(i, r) * a.Dv] : 0.f; };
+    // the normaliser n likewise, the 32-row steps dealt to the waves (every column of the accumulator the same)
     constexpr int NO = MLSTM ? (KK + NW - 1) / NW : 1;
     f32x4 nst[2 * NO];
-    if constexpr (MLSTM) {
+    auto n_row = [&](int i, int r) {
+        const int kk = wv + NW * (i >> 1);
+        return kk < KK ? kk * 32 + 8 * g + 4 * (i & 1) + r : -1;
+    };
+    float* const seg0 = a.segs > 1 ? a.seg_s + (int64_t)group * D * a.Dv + col : nullptr;   // the state before the step, kept by the first pass
+    const bool first = seg == 0, from0 = fresh || (STATE && !first);
+    {
+        const float* const at = STATE || a.segs == 1 ? Sp : first ? seg0 : seg0 + cells * D * a.Dv;
 #pragma unroll
-        for (int i = 0; i < 2 * NO; ++i)
+        for (int i = 0; i < 2 * KK; ++i)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int kk = wv + NW * (i >> 1);
-                nst[i][r] = kk < KK ? a.n0[(int64_t)group * D + kk * 32 + 8 * g + 4 * (i & 1) + r] : 0.f;
-            }
+            for (int r = 0; r < 4; ++r) S[i][r] = from0 && (STATE || first) ? 0.f : take(at, i, r);
+        if (STATE && first && !fresh && live) {
+#pragma unroll
+            for (int i = 0; i < 2 * KK; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) seg0[(int64_t)row_of(i, r) * a.Dv] = S[i][r];
+        }
+        if constexpr (MLSTM) {
+            const float* const nat = STATE || first ? a.n0 + (int64_t)group * D : a.seg_n + (int64_t)group * D;
+#pragma unroll
+            for (int i = 0; i < 2 * NO; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) nst[i][r] = (STATE && !first) || n_row(i, r) < 0 ? 0.f : nat[n_row(i, r)];
+        }
     }
+    if constexpr (!STATE && !DELTA) {
+        for (int j = 1; j < seg; ++j) {   // over the segments between: S <- (product of decays) S + what they write
+            const float d = a.seg_d[cells * j + group];
+            const float* const at = seg0 + cells * (j + 1) * D * a.Dv;
+#pragma unroll
+            for (int i = 0; i < 2 * KK; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) S[i][r] = d * S[i][r] + take(at, i, r);
+            if constexpr (MLSTM) {
+#pragma unroll
+                for (int i = 0; i < 2 * NO; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (n_row(i, r) >= 0) nst[i][r] = d * nst[i][r] + a.seg_n[(cells * j + group) * D + n_row(i, r)];
+            }
+        }
+    }
+    double Lseg = 0.0;   // STATE: the sum of the segment's log decays, and the sign of their product
+    float gseg = 1.f;
     const uint16_t* const qp = a.proj + a.q_off + (int64_t)hk * D;
     const uint16_t* const kp = a.proj + a.k_off + (int64_t)hk * D;
     const uint16_t* const vp = a.proj + a.v_off + (int64_t)hd * a.Dv + c0;
@@ -156,7 +202,7 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
             const int j = wv + NW * u, i = j * 64 + lane, row = i / CPR, c = (i % CPR) ^ spread<CPR>(row);
             if (CPR % NW == 0 || j < CPR) {
                 const int64_t at = (int64_t)min(row, last) * a.ldp + c * 8;
-                dma_1k(q + at, __builtin_amdgcn_readfirstlane(dst + j * 1024));
+                if (!STATE) dma_1k(q + at, __builtin_amdgcn_readfirstlane(dst + j * 1024));
                 dma_1k(k + at, __builtin_amdgcn_readfirstlane(dst + M::Q + j * 1024));
             }
         }
@@ -185,10 +231,12 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
     };
     // stores of the read-out: past the chunk's last token and past Dv the descriptor's range drops them
     const uint32_t orow = (uint32_t)a.H * a.Dv * 4, ocol = live ? (uint32_t)col * 4 : 0x80000000u;
-    fetch(t0, 0);
-    scalars(t0);
-    for (int tb = t0, buf = 0; tb < t1; tb += kCH, buf ^= 1) {
-        const int nt = min(kCH, t1 - tb);
+    if (t0 < te) {
+        fetch(t0, 0);
+        scalars(t0);
+    }
+    for (int tb = t0, buf = 0; tb < te; tb += kCH, buf ^= 1) {
+        const int nt = min(kCH, te - tb);
         dma_wait();
         // ---- the chunk's scalars (before the next chunk's DMA is issued: what waits for them would wait for that, too)
         const bool valid = lane < nt;
@@ -216,6 +264,10 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
         L = lanes_running_sum(L);
         const double LC = __builtin_bit_cast(double, (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(__builtin_bit_cast(uint64_t, L) >> 32), 63) << 32 |
                                                          (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)__builtin_bit_cast(uint64_t, L), 63));
+        if constexpr (STATE) {
+            Lseg += LC;
+            gseg *= gC;
+        }
         const float eL = exp_d(L);
         Ls[lane] = L;
         ws[lane] = w;
@@ -227,7 +279,7 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
             be[lane] = bt * w * eL;
         }
         __syncthreads();   // this chunk's rows are in LDS; nobody reads the other buffer or the last chunk's weights any more
-        if (tb + kCH < t1) {
+        if (tb + kCH < te) {
             fetch(tb + kCH, buf ^ 1);
             scalars(tb + kCH);
         }
@@ -267,7 +319,7 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
             return v;
         };
         const int nrow = (nt + 15) / 16;   // 16-token rows of tiles that hold tokens
-        for (int p = wv; p < 10; p += NW) {
+        for (int p = STATE ? 10 : wv; p < 10; p += NW) {
             const int i = p < 1 ? 0 : p < 3 ? 1 : p < 6 ? 2 : 3, j = p - i * (i + 1) / 2;
             if (i >= nrow) continue;
             const f32x4 v = product(qb, i, j);
@@ -312,7 +364,7 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
                 }
             }
         }
-        if constexpr (MLSTM) {   // n . q of the state before the chunk, this wave's rows
+        if constexpr (MLSTM && !STATE) {   // n . q of the state before the chunk, this wave's rows
             f32x4 acc[4] = {};
 #pragma unroll
             for (int u = 0; u < NO; ++u) {
@@ -337,9 +389,9 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
                 for (int i = 0; i < 4; ++i) *reinterpret_cast<f32x4*>(nq + wv * kCH + 16 * i + 4 * g) = acc[i];
             }
         }
-        __syncthreads();   // the weights are there
+        if constexpr (!STATE) __syncthreads();   // the weights are there
         float fr = rd;
-        if constexpr (MLSTM) {
+        if constexpr (MLSTM && !STATE) {
             const int i = lane >> 4, p0 = i * (i + 1) / 2;
             float intra = 0.f, inter = 0.f;
             for (int j = 0; j <= i; ++j) intra += psum[(p0 + j) * 16 + ln];
@@ -357,6 +409,8 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
                 const unsigned char* at = vb + (32 * p + r4) * (VC * 16) + ((wv * 2 + ((ln & 3) >> 1)) ^ spread<VC>(r4)) * 16 + (ln & 1) * 8;
                 v[p] = join8(lds_read_tr4(at), lds_read_tr4(at + 16 * (VC * 16)));
             }
+            f32x4 U[NI];   // delta: what the chunk's tokens write, before the scales
+            if constexpr (!STATE) {
             // the state before the chunk times q (delta: and k), a 32-row step of it at a time
             f32x4 oq[NI], ok[NI];
 #pragma unroll
@@ -391,7 +445,6 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
                     fo[i][r] = __shfl(fr, 16 * i + 4 * g + r, 64);
                     oq[i][r] *= el[i][r];
                 }
-            f32x4 U[NI];   // what the chunk's tokens write, before the scales
             if constexpr (DELTA) {
                 // (I + A) U = beta (v - e^L k-scale S^T k), 16 rows at a time
                 Terms4 ut[NI];
@@ -457,6 +510,7 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(oq[i][r] * fo[i][r]), ord, ocol + (16 * i + 4 * g + r) * orow, 0, 0);
+            }
 #pragma unroll
             for (int i = 0; i < 2 * KK; ++i) S[i] *= eC;
             if constexpr (MLSTM) {
@@ -502,23 +556,26 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
         if (nt > 32) rest(std::integral_constant<int, 4>{});
         else rest(std::integral_constant<int, 2>{});
     }
+    if (!STATE && seg != a.segs - 1) return;
+    float* const dst = STATE ? seg0 + cells * (seg + 1) * D * a.Dv : Sp;
     if (live) {
 #pragma unroll
         for (int i = 0; i < 2 * KK; ++i)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) Sp[(int64_t)((i >> 1) * 32 + 8 * g + 4 * (i & 1) + r) * a.Dv] = S[i][r];
+            for (int r = 0; r < 4; ++r) dst[(int64_t)row_of(i, r) * a.Dv] = S[i][r];
     }
+    if (slab != 0) return;
     if constexpr (MLSTM) {
-        if (slab == 0 && ln == 0) {
+        float* const nd = STATE ? a.seg_n + (cells * seg + group) * D : a.n + srow * D;
+        if (ln == 0) {
 #pragma unroll
             for (int i = 0; i < 2 * NO; ++i)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int kk = wv + NW * (i >> 1);
-                    if (kk < KK) a.n[srow * D + kk * 32 + 8 * g + 4 * (i & 1) + r] = nst[i][r];
-                }
+                for (int r = 0; r < 4; ++r)
+                    if (n_row(i, r) >= 0) nd[n_row(i, r)] = nst[i][r];
         }
     }
+    if (STATE && threadIdx.x == 0) a.seg_d[cells * seg + group] = gseg * exp_d(Lseg);
 }
 
 // The scalar recurrences of mlstm.hip for a whole prompt portion: m_t = max(f_t + m_(t-1), i_t) is a prefix of the pairs
@@ -588,14 +645,44 @@ bool hy_chunk_scan_ok(const void* proj, int ldp, int q_off, int k_off, int v_off
            ((ldp | q_off | k_off | v_off) & 7) == 0 && ldp < 1 << 23;   // (64 rows of o, no wider than proj's, within 2^31 bytes)
 }
 
-template <int D, int MODE>
-static void chunk_scan_run(const hy::ChunkScan& a, hipStream_t s) {
+template <int D, int MODE, bool STATE>
+static void chunk_scan_pass(const hy::ChunkScan& a, int segs, hipStream_t s) {
     constexpr int lds = hy::ChunkLds<D, MODE>::SIZE;
     static_assert(lds <= 160 * 1024, "LDS of one workgroup");
-    const auto kern = hy::chunk_scan_kernel<D, MODE>;
+    const auto kern = hy::chunk_scan_kernel<D, MODE, STATE>;
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     const int nslab = (a.Dv + 16 * hy::kCW - 1) / (16 * hy::kCW);
-    kern<<<(a.B * a.H + 7) / 8 * 8 * nslab, 64 * hy::kCW, lds, s>>>(a);
+    kern<<<dim3((a.B * a.H + 7) / 8 * 8 * nslab, segs), 64 * hy::kCW, lds, s>>>(a);
+}
+template <int D, int MODE>
+static void chunk_scan_run(const hy::ChunkScan& a, hipStream_t s) {
+    if constexpr (MODE != hy::kScanDelta)
+        if (a.segs > 1) chunk_scan_pass<D, MODE, true>(a, a.segs - 1, s);
+    chunk_scan_pass<D, MODE, false>(a, a.segs, s);
+}
+
+// Segments that a sequence's chunks are dealt to: launches that leave half of the CUs or more without a workgroup carry the states over
+// segments of at least 4 chunks first (half a chunk's work) and take all of them side by side then.  Not with the delta rule, whose step
+// from state to state is a matrix.  Measured, one pass -> segments: retention, 8 heads of 128 x 128, 4 sequences of 512 tokens (two
+// segments) 45 -> 26 us, one of 512 (two) 45 -> 35, 4096 (16) 332 -> 51; mlstm, 4 heads of 256 x 512, one of 512 (two) 79 -> 64, 4096
+// (eight) 577 -> 152, of 32768 4701 -> 1009; state-space form, 128 heads of 128 x 64, one of 512 (two) 52 -> 43.  At most four segments:
+// 118 and 232 us for the two of 4096.
+int hy_chunk_segments(int B, int H, int D, int Dv, int longest) {
+    if (D != 32 && D != 64 && D != 128 && D != 256) return 1;
+    const int64_t wgs = (int64_t)B * H * ((Dv + 63) / 64);
+    const int64_t segs = std::min<int64_t>({wgs > 0 ? 256 / wgs : 1, (longest + 63) / 64 / 4, 16});
+    return segs > 1 ? (int)segs : 1;
+}
+// floats of scratch: the states before the step and of all segments but the last; normalisers and products of decays of those
+int64_t hy_chunk_segment_floats(int B, int H, int D, int Dv, int segs) {
+    return segs > 1 ? (int64_t)B * H * ((int64_t)segs * D * Dv + (segs - 1) * (int64_t)(D + 1)) : 0;
+}
+static void chunk_scan_scratch(hy::ChunkScan& a, int D, int segs, float* seg) {
+    a.segs = segs;
+    const int64_t cells = (int64_t)a.B * a.H;
+    a.seg_s = seg;
+    a.seg_n = seg + cells * segs * D * a.Dv;
+    a.seg_d = a.seg_n + cells * (segs - 1) * D;
 }
 
 template <int MODE>
@@ -611,22 +698,24 @@ static void chunk_scan_d(int D, const hy::ChunkScan& a, hipStream_t s) {
 void launch_hy_chunk_scan(const uint16_t* proj, int ldp, int q_off, int k_off, int v_off, const float* qscale, const float* kscale,
                           float q_mul, const float* decay, int dts, const float* beta, const int32_t* q_start,
                           const int32_t* pos0, const int32_t* slots, float* S, float* o, int B, int HK, int H, int D, int Dv, const float* vscale,
-                          hipStream_t s) {
+                          int segs, float* seg, hipStream_t s) {
     hy::ChunkScan a{proj, ldp, q_off, k_off, v_off, qscale, kscale, vscale, decay, beta, dts, q_mul, nullptr, nullptr, nullptr,
-                    q_start, pos0, slots, nullptr, S, nullptr, o, B, HK, H, Dv};
+                    q_start, pos0, slots, nullptr, S, nullptr, o, B, HK, H, Dv, 1, nullptr, nullptr, nullptr};
+    if (beta == nullptr && segs > 1) chunk_scan_scratch(a, D, segs, seg);
     if (beta != nullptr) chunk_scan_d<hy::kScanDelta>(D, a, s);
     else chunk_scan_d<hy::kScanPlain>(D, a, s);
 }
 
-// scratch: 3 T H + B H D floats
+// segs: hy_chunk_segments (1: none).  scratch: 3 T H + B H D + hy_chunk_segment_floats floats
 void launch_hy_chunk_mlstm(const uint16_t* proj, int ldp, const float* gate_pre, const int32_t* q_start, const int32_t* pos0,
                            const int32_t* slots, float* S, float* n, float* m, float* scratch, float* o, int T, int B, int H,
-                           int D, int Dv, float cap, hipStream_t s) {
+                           int D, int Dv, float cap, int segs, hipStream_t s) {
     const int64_t th = (int64_t)T * H;
     float *la = scratch, *lb = la + th, *em = lb + th, *n0 = em + th;
     hy::mlstm_gates_kernel<<<dim3(B, H), 256, 0, s>>>(gate_pre, q_start, pos0, slots, n, m, n0, la, lb, em, H, D, cap);
     hy::ChunkScan a{proj, ldp, 0, H * D, 2 * H * D, nullptr, nullptr, nullptr, nullptr, nullptr, H, 1.f / sqrtf((float)D), la, lb, em,
-                    q_start, pos0, slots, n0, S, n, o, B, H, H, Dv};
+                    q_start, pos0, slots, n0, S, n, o, B, H, H, Dv, 1, nullptr, nullptr, nullptr};
+    if (segs > 1) chunk_scan_scratch(a, D, segs, n0 + (int64_t)B * H * D);
     chunk_scan_d<hy::kScanMlstm>(D, a, s);
 }
 

@@ -418,7 +418,7 @@ __global__ void __launch_bounds__(256) linear_scan_kernel(
 bool hy_chunk_scan_ok(const void*, int, int, int, int, int, int, int, bool);
 void launch_hy_chunk_scan(const uint16_t*, int, int, int, int, const float*, const float*, float, const float*, int,
                           const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*, int, int, int, int, int, const float*,
-                          hipStream_t);
+                          int, float*, hipStream_t);
 
 bool hy_gla_scan_ok(const void*, const void*, int, int, int, int, int, int, int);
 void launch_hy_gla_scan(const uint16_t*, int, int, int, int, const float*, const float*, float, const float*, const int32_t*,
@@ -511,12 +511,12 @@ static bool linear_scan_d(bool pipe, const T* proj, int ldp, int q_off, int k_of
 // delta: beta != nullptr.  vscale (float [T, H], may be nullptr; without delta only): a factor on the written value.
 // chd: decay holds one number per state row ([T, H, D]) instead of one per head ([T, H]).
 // fixed (not with chd): decay holds one number per head for all tokens ([H]).
-// longest: the most tokens that any sequence brings (or an upper bound of it).
+// longest: the most tokens that any sequence brings (or an upper bound of it).  segs, seg: hy_chunk_segments and its scratch.
 // Returns false when D has no instantiation (D > 256).
 bool launch_hy_linear_scan(const void* proj, int ldp, int q_off, int k_off, int v_off, const float* qscale,
                            const float* kscale, float q_mul, const float* decay, bool chd, bool fixed, const float* beta,
                            const int32_t* q_start, const int32_t* pos0, const int32_t* slots, float* S, float* o, int T,
-                           int B, int HK, int H, int D, int Dv, const float* vscale, int longest, bool f32, hipStream_t s) {
+                           int B, int HK, int H, int D, int Dv, const float* vscale, int longest, int segs, float* seg, bool f32, hipStream_t s) {
     if (B == 0) return true;
     const bool pipe = T > B;   // some sequence brings more than one token
     const bool delta = beta != nullptr;
@@ -532,7 +532,7 @@ bool launch_hy_linear_scan(const void* proj, int ldp, int q_off, int k_off, int 
     }
     if (!chd && !f32 && hy_chunk_scan_ok(proj, ldp, q_off, k_off, v_off, D, Dv, longest, delta)) {
         launch_hy_chunk_scan((const uint16_t*)proj, ldp, q_off, k_off, v_off, qscale, kscale, q_mul, decay, fixed ? 0 : H, beta,
-                             q_start, pos0, slots, S, o, B, HK, H, D, Dv, vscale, s);
+                             q_start, pos0, slots, S, o, B, HK, H, D, Dv, vscale, segs, seg, s);
         return true;
     }
     const int dts = fixed ? 0 : H;

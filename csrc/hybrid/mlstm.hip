@@ -444,15 +444,15 @@ static void mlstm_scan_t(const T* proj, int ldp, const float* gate_pre, const in
 
 bool hy_chunk_scan_ok(const void*, int, int, int, int, int, int, int, bool);
 void launch_hy_chunk_mlstm(const uint16_t*, int, const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*,
-                           float*, float*, float*, int, int, int, int, int, float, hipStream_t);
+                           float*, float*, float*, int, int, int, int, int, float, int, hipStream_t);
 
-// D <= 512.  scratch: 3 T H + B H D floats.  longest: the most tokens that any sequence brings (or an upper bound of it).
+// D <= 512.  segs: hy_chunk_segments.  scratch: 3 T H + B H D + hy_chunk_segment_floats floats.  longest: the most tokens that any sequence brings (or an upper bound of it).
 void launch_hy_mlstm_scan(const void* proj, int ldp, const float* gate_pre, const int32_t* q_start, const int32_t* pos0,
                           const int32_t* slots, float* S, float* n, float* m, float* scratch, float* o, int T, int B, int H, int D,
-                          int Dv, float cap, int longest, bool f32, hipStream_t s) {
+                          int Dv, float cap, int longest, int segs, bool f32, hipStream_t s) {
     if (B == 0) return;
     if (!f32 && hy_chunk_scan_ok(proj, ldp, 0, H * D, 2 * H * D, D, Dv, longest, false)) {
-        launch_hy_chunk_mlstm((const uint16_t*)proj, ldp, gate_pre, q_start, pos0, slots, S, n, m, scratch, o, T, B, H, D, Dv, cap, s);
+        launch_hy_chunk_mlstm((const uint16_t*)proj, ldp, gate_pre, q_start, pos0, slots, S, n, m, scratch, o, T, B, H, D, Dv, cap, segs, s);
         return;
     }
     float *a = scratch, *b = a + (int64_t)T * H, *den = b + (int64_t)T * H;

@@ -178,3 +178,45 @@ def test_mlstm(H, D, Dv, gate):
     assert _rel(S, Sw) < 2e-6 and _rel(n, nw) < 2e-6 and _rel(m, mw) < 1e-6
     for t, t0 in ((S, S0), (n, n0), (m, m0)):
         assert torch.equal(t[1], t0[1]) and torch.equal(t[6], t0[6]), "slots without tokens must stay untouched"
+
+
+@pytest.mark.parametrize("lens,starts", [([1100, 40, 0, 513, 1023], [0, 3, 5, 9, 0]), ([2500], [7])])
+@pytest.mark.parametrize("form", ["token", "mlstm"])
+def test_segments(lens, starts, form):
+    """Few, long sequences: their chunks are dealt to segments (1100 tokens: four of 18 chunks; 2500: ten of 40), whose states
+    are carried first; against the same sequences in launches too wide for segments."""
+    from chronos.ops import hybrid as hops
+
+    H, D, Dv, T = 2, 64, 72, sum(lens)
+    reps = 40   # copies of the sequences that fill the chip: no segments
+    g = torch.Generator(device=DEV).manual_seed(T)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    proj, gp = rnd(T, 2 * H * D + 2 * H * Dv).bfloat16(), rnd(T, 2 * H)
+    gp[:, H:] += 3.0
+    dec = torch.exp(-0.2 * torch.rand(T, H, device=DEV, generator=g))
+    dec[7::90], dec[11::400] = -0.9, 1.2
+    B = len(lens)
+    S0, n0, m0 = rnd(B, H, D, Dv) * 0.3, rnd(B, H, D) * 0.5, rnd(B, H)
+
+    def run(r):
+        qs = [0]
+        for n in lens * r:
+            qs.append(qs[-1] + n)
+        rg = (i32(qs), i32(starts * r), torch.arange(B * r, device=DEV).int())
+        S, n, m = (t.repeat(r, *[1] * (t.dim() - 1)) for t in (S0, n0, m0))
+        if form == "mlstm":
+            o = hops.mlstm_scan(proj.repeat(r, 1), gp.repeat(r, 1), *rg, S, n, m, H, D, Dv, 9.0, max(lens))
+        else:
+            o = hops.linear_scan(proj.repeat(r, 1), 0, H * D, 2 * H * D, None, None, 0.3, dec.repeat(r, 1), None, *rg, S, H, H, D, Dv,
+                                 None, max(lens))
+        return o[:T], S[:B], n[:B], m[:B]
+
+    a, w = run(1), run(reps)
+    for x, y in zip(a[1:], w[1:]):
+        assert _rel(x, y.double()) < 2e-6
+    if form == "mlstm":   # (the read-out is divided by a sum that may nearly cancel: as in test_mlstm, before the division)
+        near = (a[0] - w[0]).abs() > 1e-4 * w[0].abs().clamp_min(float(w[0].abs().mean()))
+        assert float(near.float().mean()) < 1e-3
+    else:
+        assert _rel(a[0], w[0].double()) < 2e-6
