@@ -20,7 +20,7 @@ void launch_hy_rowdot(const void*, const void*, const float*, float*, int, int, 
 void launch_hy_act(void*, int64_t, int, bool, hipStream_t);
 void launch_hy_mlstm_scan(const void*, int, const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*,
                           float*, float*, float*, int, int, int, int, int, float, int, int, bool, hipStream_t);
-int hy_chunk_segments(int, int, int, int, int);
+int hy_chunk_segments(int, int, int, int, int, int);
 int64_t hy_chunk_segment_floats(int, int, int, int, int);
 void launch_hy_mlstm_out(const float*, const void*, int, int, const float*, void*, int, int, int, float, bool,
                          hipStream_t);
@@ -203,7 +203,7 @@ Tensor hy_mlstm_scan(const Tensor& proj, const Tensor& gate_pre, const Tensor& q
     need(m.dim() == 2 && m.size(0) == S.size(0) && m.size(1) == H, "mlstm_scan: m [NS, H]");
     need(D >= 1 && D <= 512 && H >= 1 && Dv >= 1, "mlstm_scan: 1 <= D <= 512");
     auto o = at::empty({T, H, Dv}, proj.options().dtype(at::kFloat));
-    const int mq = longest(T, B, max_q), segs = f32(proj) ? 1 : chronos::hy_chunk_segments((int)B, (int)H, (int)D, (int)Dv, mq);
+    const int mq = longest(T, B, max_q), segs = f32(proj) ? 1 : chronos::hy_chunk_segments((int)B, (int)H, (int)D, (int)Dv, mq, 256);
     auto scratch = at::empty({3 * T * H + B * H * D + chronos::hy_chunk_segment_floats((int)B, (int)H, (int)D, (int)Dv, segs)},
                              proj.options().dtype(at::kFloat));
     chronos::launch_hy_mlstm_scan(proj.data_ptr(), (int)proj.size(1), gate_pre.data_ptr<float>(),
@@ -784,7 +784,7 @@ Tensor hy_linear_scan(const Tensor& proj, int64_t q_off, int64_t k_off, int64_t 
     need(S.dim() == 4 && S.size(1) == H && S.size(2) == D && S.size(3) == Dv, "linear_scan: S [NS, H, D, Dv]");
     auto o = at::empty({T, H, Dv}, proj.options().dtype(at::kFloat));
     if (T == 0) return o;
-    const int mq = longest(T, B, max_q), segs = f32(proj) || chd || beta ? 1 : chronos::hy_chunk_segments((int)B, (int)H, (int)D, (int)Dv, mq);
+    const int mq = longest(T, B, max_q), segs = f32(proj) || beta ? 1 : chronos::hy_chunk_segments((int)B, (int)H, (int)D, (int)Dv, mq, chd ? 128 : 256);
     Tensor seg;
     if (segs > 1) seg = at::empty({chronos::hy_chunk_segment_floats((int)B, (int)H, (int)D, (int)Dv, segs)}, S.options());
     const bool ok = chronos::launch_hy_linear_scan(

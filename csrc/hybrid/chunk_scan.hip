@@ -661,16 +661,19 @@ static void chunk_scan_run(const hy::ChunkScan& a, hipStream_t s) {
     chunk_scan_pass<D, MODE, false>(a, a.segs, s);
 }
 
-// Segments that a sequence's chunks are dealt to: launches that leave half of the CUs or more without a workgroup carry the states over
-// segments of at least 4 chunks first (half a chunk's work) and take all of them side by side then.  Not with the delta rule, whose step
-// from state to state is a matrix.  Measured, one pass -> segments: retention, 8 heads of 128 x 128, 4 sequences of 512 tokens (two
+// Segments that a sequence's chunks are dealt to, here and in gla_scan.hip: launches that leave half of the CUs or more without a
+// workgroup carry the states over segments of at least `least` tokens first (half a chunk's work) and take all of them side by side
+// then.  Not with the delta rule, whose step from state to state is a matrix.  256 tokens here (four chunks), 128 in gla_scan.hip (eight,
+// slower ones).  Measured, one pass -> segments: retention, 8 heads of 128 x 128, 4 sequences of 512 tokens (two
 // segments) 45 -> 26 us, one of 512 (two) 45 -> 35, 4096 (16) 332 -> 51; mlstm, 4 heads of 256 x 512, one of 512 (two) 79 -> 64, 4096
 // (eight) 577 -> 152, of 32768 4701 -> 1009; state-space form, 128 heads of 128 x 64, one of 512 (two) 52 -> 43.  At most four segments:
-// 118 and 232 us for the two of 4096.
-int hy_chunk_segments(int B, int H, int D, int Dv, int longest) {
+// 118 and 232 us for the two of 4096.  One decay per row, heads of 128 x 256: 16 heads, 2 sequences of 256 tokens (two segments) 50 -> 48
+// us, one of 2048 (four) 360 -> 167; 4 heads, 4 of 256 (two) 49 -> 30, one of 256 (two) 48 -> 46, of 512 (four) 92 -> 49, of 2048 (16)
+// 359 -> 77.
+int hy_chunk_segments(int B, int H, int D, int Dv, int longest, int least) {
     if (D != 32 && D != 64 && D != 128 && D != 256) return 1;
     const int64_t wgs = (int64_t)B * H * ((Dv + 63) / 64);
-    const int64_t segs = std::min<int64_t>({wgs > 0 ? 256 / wgs : 1, (longest + 63) / 64 / 4, 16});
+    const int64_t segs = std::min<int64_t>({wgs > 0 ? 256 / wgs : 1, (longest + 63) / least, 16});
     return segs > 1 ? (int)segs : 1;
 }
 // floats of scratch: the states before the step and of all segments but the last; normalisers and products of decays of those

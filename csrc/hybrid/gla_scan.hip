@@ -15,7 +15,7 @@
 //
 // What bounds it: the chain of a sequence's chunks, one wave per SIMD: about 600 vector and 66 matrix instructions a chunk and wave at
 // D = 128, two barriers and the LDS reads between them, 2.8 us.  Measured, 4 sequences of 2048 tokens, 16 heads of 128 x 256: token by
-// token 988 us, this 403; one of 4000, 8 heads: 1684 and 697.  P on the vector ALUs from running products: 648 us, and the same
+// token 988 us, this 403; one of 4000, 8 heads: 1684 and 694, in eight segments 173.  P on the vector ALUs from running products: 648 us, and the same
 // with F in float32: state 9.6e-8 of its norm off the float64 recurrence (token by token 8.7e-8, this 7.8e-8); with the stores of a
 // chunk waited for by the next: 482 us, with that 448, and the terms rounded in pairs 403.
 #include "chunk_common.h"
@@ -33,6 +33,10 @@ struct GlaScan {
     const int32_t *q_start, *pos0, *slots;
     float *S, *o;
     int B, HK, H, Dv;
+    // segments of a sequence side by side (1: none), as in chunk_scan.hip: the state before the step and, of each segment but the last,
+    // what it writes, [segs, B, H, D, Dv]; products of its decays [segs - 1, B, H, D]
+    int segs;
+    float *seg_s, *seg_d;
 };
 
 constexpr int kGC = 16;   // tokens per chunk
@@ -50,7 +54,8 @@ template <int D> struct GlaLds {
     static constexpr int TQ = 2 * BUF, TK = TQ + 3 * Q, F = TK + 3 * Q, SC = F + D * 4, BAD = SC + 4 * kGC * 4, SIZE = BAD + 16;
 };
 
-template <int D>
+// STATE: the first pass over segments, which only carries the state on (each from 0, the first from the sequence's state)
+template <int D, bool STATE>
 __global__ void __launch_bounds__(256, 1) gla_scan_kernel(const GlaScan a) {
     using M = GlaLds<D>;
     constexpr int CPR = D / 8, KK = D / 32;   // 16-byte pieces per row of q and k; 32-row steps
@@ -59,22 +64,50 @@ __global__ void __launch_bounds__(256, 1) gla_scan_kernel(const GlaScan a) {
     float* const sc = reinterpret_cast<float*>(gs_smem + M::SC);
     int* const bad = reinterpret_cast<int*>(gs_smem + M::BAD);
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), ln = lane & 15, g = lane >> 4;
-    // groups of workgroups that share q, k and decay rows go to one XCD (workgroup i runs on XCD i % 8)
-    const int nslab = (a.Dv + 63) / 64, id = blockIdx.x >> 3, group = (id / nslab) * 8 + (blockIdx.x & 7), slab = id % nslab;
+    // groups of workgroups that share q, k and decay rows go to one XCD (workgroup i runs on XCD i % 8), the next segment's behind them
+    const int nslab = (a.Dv + 63) / 64, id = blockIdx.x >> 3, seg = blockIdx.y, slab = id % nslab;
+    const int group = (id / nslab) * 8 + ((blockIdx.x - seg * a.B * a.H) & 7);
     if (group >= a.B * a.H) return;
     const int b = group / a.H, hd = group % a.H, hk = hd / (a.H / a.HK);
-    const int t0 = a.q_start[b], t1 = a.q_start[b + 1];
-    if (t1 <= t0) return;
+    const int s0 = a.q_start[b], t1 = a.q_start[b + 1];
+    if (t1 <= s0) return;
+    const int chunks = (t1 - s0 + kGC - 1) / kGC;
+    const int t0 = s0 + chunks * seg / a.segs * kGC, te = min(t1, s0 + chunks * (seg + 1) / a.segs * kGC);   // this segment's tokens
+    const int64_t cells = (int64_t)a.B * a.H;
     const int c0 = slab * 64, col = c0 + wv * 16 + ln;
     const bool live = col < a.Dv;
     float* const Sp = a.S + ((int64_t)a.slots[b] * a.H + hd) * D * a.Dv + col;
     const bool fresh = a.pos0[b] == 0;
     // S[2 kk + h], element r of lane group g: row 32 kk + 8 g + 4 h + r (what the read-out's product takes from that lane)
     f32x4 S[2 * KK];
+    auto row_of = [&](int i, int r) { return (i >> 1) * 32 + 8 * g + 4 * (i & 1) + r; };
+    float* const seg0 = a.segs > 1 ? a.seg_s + (int64_t)group * D * a.Dv + col : nullptr;   // the state before the step, kept by the first pass
+    {
+        const bool first = seg == 0, zero = !live || (STATE ? !first || fresh : first && fresh);
+        const float* const at = STATE || a.segs == 1 ? Sp : first ? seg0 : seg0 + cells * D * a.Dv;
 #pragma unroll
-    for (int i = 0; i < 2 * KK; ++i)
+        for (int i = 0; i < 2 * KK; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) S[i][r] = !fresh && live ? Sp[(int64_t)((i >> 1) * 32 + 8 * g + 4 * (i & 1) + r) * a.Dv] : 0.f;
+            for (int r = 0; r < 4; ++r) S[i][r] = zero ? 0.f : at[(int64_t)row_of(i, r) * a.Dv];
+        if (STATE && first && !zero) {
+#pragma unroll
+            for (int i = 0; i < 2 * KK; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) seg0[(int64_t)row_of(i, r) * a.Dv] = S[i][r];
+        }
+    }
+    if constexpr (!STATE) {
+        for (int j = 1; j < seg; ++j) {   // over the segments between: S <- (products of decays) S + what they write
+            const float *const at = seg0 + cells * (j + 1) * D * a.Dv, *const d = a.seg_d + (cells * j + group) * D;
+#pragma unroll
+            for (int i = 0; i < 2 * KK; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) S[i][r] = d[row_of(i, r)] * S[i][r] + (live ? at[(int64_t)row_of(i, r) * a.Dv] : 0.f);
+        }
+    }
+    double dx[(D + 127) / 128], dy[(D + 127) / 128];   // STATE: the products of the segment's decays so far (rows as F q below)
+#pragma unroll
+    for (int it = 0; it < (D + 127) / 128; ++it) dx[it] = dy[it] = 1.0;
     const uint16_t* const qp = a.proj + a.q_off + (int64_t)hk * D;
     const uint16_t* const kp = a.proj + a.k_off + (int64_t)hk * D;
     const uint16_t* const vp = a.proj + a.v_off + (int64_t)hd * a.Dv + c0;
@@ -123,19 +156,21 @@ __global__ void __launch_bounds__(256, 1) gla_scan_kernel(const GlaScan a) {
     };
     const uint32_t orow = (uint32_t)a.H * a.Dv * 4, ocol = live ? (uint32_t)col * 4 : 0x80000000u;
     if (tid < 3) bad[tid] = 0;
-    fetch(t0, 0);
-    scalars(t0);
+    if (t0 < te) {
+        fetch(t0, 0);
+        scalars(t0);
+    }
     received(sw);
     received(sr);
-    for (int tb = t0, buf = 0, turn = 0; tb < t1; tb += kGC, buf ^= 1, turn = turn == 2 ? 0 : turn + 1) {
-        const int nt = min(kGC, t1 - tb);
+    for (int tb = t0, buf = 0, turn = 0; tb < te; tb += kGC, buf ^= 1, turn = turn == 2 ? 0 : turn + 1) {
+        const int nt = min(kGC, te - tb);
         unsigned char* const raw = gs_smem + buf * M::BUF;
         const uint16_t* const qs = reinterpret_cast<const uint16_t*>(raw);
         const uint16_t* const ks = reinterpret_cast<const uint16_t*>(raw + M::Q);
         float* const ds = reinterpret_cast<float*>(raw + M::DEC);
         float* const ws = sc + buf * 2 * kGC;
         // (each earlier chunk issued 4 stores or 16 after this chunk's pieces)
-        if (tb == t0) dma_wait();
+        if (STATE || tb == t0) dma_wait();
         else dma_wait_before_stores<4>();
         if (tid < kGC) {
             ws[tid] = tid < nt ? sw : 0.f;
@@ -146,7 +181,7 @@ __global__ void __launch_bounds__(256, 1) gla_scan_kernel(const GlaScan a) {
             for (int i = nt * D + tid; i < kGC * D; i += 256) ds[i] = 1.f;
             __syncthreads();
         }
-        if (tb + kGC < t1) {
+        if (tb + kGC < te) {
             fetch(tb + kGC, buf ^ 1);
             scalars(tb + kGC);
         }
@@ -220,6 +255,10 @@ __global__ void __launch_bounds__(256, 1) gla_scan_kernel(const GlaScan a) {
                 if (!keys && half) {
                     fs[2 * rp] = x[7];
                     fs[2 * rp + 1] = y[7];
+                    if constexpr (STATE) {
+                        dx[it] *= X;
+                        dy[it] *= Y;
+                    }
                 }
             }
         }
@@ -245,43 +284,45 @@ __global__ void __launch_bounds__(256, 1) gla_scan_kernel(const GlaScan a) {
                 float x = acc[0] + acc[1];
                 x += __shfl_xor(x, 16, 64);
                 x += __shfl_xor(x, 32, 64);
-                if (g == 0) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x * ws[kGC + t]), ord, ocol + t * orow, 0, 0);
+                if (!STATE && g == 0) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x * ws[kGC + t]), ord, ocol + t * orow, 0, 0);
             }
             continue;
-        }
-        // ---- read-out: o = (F q)^T S, and P with rows s = 4 g + r and columns t = ln (as its product with v takes it)
-        const int sp = spread<CPR>(ln);
-        f32x4 small = {0.f, 0.f, 0.f, 0.f}, big = small, psmall = small, pbig = small;
-#pragma unroll
-        for (int kk = 0; kk < KK; ++kk) {
-            const unsigned char* at = gs_smem + M::TQ + ln * (D * 2) + ((kk * 4 + g) ^ sp) * 16;
-            auto term = [&](int base) { return *reinterpret_cast<const bf16x8*>(at + base); };
-            const bf16x8 qh = term(0), qm = term(M::Q), ql = term(2 * M::Q), kh = term(3 * M::Q), km = term(4 * M::Q), kl = term(5 * M::Q);
-            psmall = mfma_16x16x32(kl, qh, psmall);
-            psmall = mfma_16x16x32(km, qm, psmall);
-            psmall = mfma_16x16x32(kh, ql, psmall);
-            psmall = mfma_16x16x32(km, qh, psmall);
-            psmall = mfma_16x16x32(kh, qm, psmall);
-            pbig = mfma_16x16x32(kh, qh, pbig);
-            small = mfma_16x16x32(ql, st[kk].h, small);
-            small = mfma_16x16x32(qm, st[kk].m, small);
-            small = mfma_16x16x32(qh, st[kk].l, small);
-            small = mfma_16x16x32(qm, st[kk].h, small);
-            small = mfma_16x16x32(qh, st[kk].m, small);
-            big = mfma_16x16x32(qh, st[kk].h, big);
         }
         const bf16x4 v4 = lds_read_tr4(raw + M::V + (4 * g + (ln >> 2)) * 128 + wv * 32 + (ln & 3) * 8);   // tokens 4 g ..
         const bf16x8 vv = join8(v4, v4);
         const bf16x4 none = {};
-        f32x4 P = psmall + pbig;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) P[r] = 4 * g + r <= ln ? P[r] : 0.f;
-        const Terms4 pt = split3(P);
-        small = mfma_16x16x32(join8(pt.l, none), vv, small);
-        big = mfma_16x16x32(join8(pt.h, pt.m), vv, big);
-#pragma unroll
-        for (int r = 0; r < 4; ++r)   // (past the last token and past Dv the descriptor's range drops the store)
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((small[r] + big[r]) * fr[r]), ord, ocol + (4 * g + r) * orow, 0, 0);
+        if constexpr (!STATE) {
+            // ---- read-out: o = (F q)^T S, and P with rows s = 4 g + r and columns t = ln (as its product with v takes it)
+            const int sp = spread<CPR>(ln);
+            f32x4 small = {0.f, 0.f, 0.f, 0.f}, big = small, psmall = small, pbig = small;
+    #pragma unroll
+            for (int kk = 0; kk < KK; ++kk) {
+                const unsigned char* at = gs_smem + M::TQ + ln * (D * 2) + ((kk * 4 + g) ^ sp) * 16;
+                auto term = [&](int base) { return *reinterpret_cast<const bf16x8*>(at + base); };
+                const bf16x8 qh = term(0), qm = term(M::Q), ql = term(2 * M::Q), kh = term(3 * M::Q), km = term(4 * M::Q), kl = term(5 * M::Q);
+                psmall = mfma_16x16x32(kl, qh, psmall);
+                psmall = mfma_16x16x32(km, qm, psmall);
+                psmall = mfma_16x16x32(kh, ql, psmall);
+                psmall = mfma_16x16x32(km, qh, psmall);
+                psmall = mfma_16x16x32(kh, qm, psmall);
+                pbig = mfma_16x16x32(kh, qh, pbig);
+                small = mfma_16x16x32(ql, st[kk].h, small);
+                small = mfma_16x16x32(qm, st[kk].m, small);
+                small = mfma_16x16x32(qh, st[kk].l, small);
+                small = mfma_16x16x32(qm, st[kk].h, small);
+                small = mfma_16x16x32(qh, st[kk].m, small);
+                big = mfma_16x16x32(qh, st[kk].h, big);
+            }
+            f32x4 P = psmall + pbig;
+    #pragma unroll
+            for (int r = 0; r < 4; ++r) P[r] = 4 * g + r <= ln ? P[r] : 0.f;
+            const Terms4 pt = split3(P);
+            small = mfma_16x16x32(join8(pt.l, none), vv, small);
+            big = mfma_16x16x32(join8(pt.h, pt.m), vv, big);
+    #pragma unroll
+            for (int r = 0; r < 4; ++r)   // (past the last token and past Dv the descriptor's range drops the store)
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((small[r] + big[r]) * fr[r]), ord, ocol + (4 * g + r) * orow, 0, 0);
+        }
         // ---- the state after the chunk
         const int r4 = 4 * g + (ln >> 2), sp4 = spread<CPR>(r4);
 #pragma unroll
@@ -294,11 +335,24 @@ __global__ void __launch_bounds__(256, 1) gla_scan_kernel(const GlaScan a) {
             S[i] *= *reinterpret_cast<const f32x4*>(fs + kk * 32 + 8 * g + 4 * h);
         }
     }
+    if (!STATE && seg != a.segs - 1) return;
     if (live) {
+        float* const out = STATE ? seg0 + cells * (seg + 1) * D * a.Dv : Sp;
 #pragma unroll
         for (int i = 0; i < 2 * KK; ++i)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) Sp[(int64_t)((i >> 1) * 32 + 8 * g + 4 * (i & 1) + r) * a.Dv] = S[i][r];
+            for (int r = 0; r < 4; ++r) out[(int64_t)row_of(i, r) * a.Dv] = S[i][r];
+    }
+    if constexpr (STATE) {
+#pragma unroll
+        for (int it = 0; it < (D + 127) / 128; ++it) {
+            const int i = (tid & 127) + 128 * it, rp = i % (D / 2);
+            if (tid < 128 && (D % 128 == 0 || i < D) && i / (D / 2) == 1) {   // (every slab the same)
+                float* const d = a.seg_d + (cells * seg + group) * D + 2 * rp;
+                d[0] = (float)dx[it];
+                d[1] = (float)dy[it];
+            }
+        }
     }
 }
 
@@ -312,20 +366,27 @@ bool hy_gla_scan_ok(const void* proj, const void* decay, int ldp, int q_off, int
            ((ldp | q_off | k_off | v_off) & 7) == 0 && ldp < 1 << 23;
 }
 
-template <int D>
-static void gla_scan_run(const hy::GlaScan& a, hipStream_t s) {
+template <int D, bool STATE>
+static void gla_scan_pass(const hy::GlaScan& a, int segs, hipStream_t s) {
     constexpr int lds = hy::GlaLds<D>::SIZE;
     static_assert(lds <= 160 * 1024, "LDS of one workgroup");
-    static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(hy::gla_scan_kernel<D>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    const auto kern = hy::gla_scan_kernel<D, STATE>;
+    static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     (void)set;
     const int groups = (a.B * a.H + 7) / 8 * 8;
-    hy::gla_scan_kernel<D><<<groups * ((a.Dv + 63) / 64), 256, lds, s>>>(a);
+    kern<<<dim3(groups * ((a.Dv + 63) / 64), segs), 256, lds, s>>>(a);
+}
+template <int D>
+static void gla_scan_run(const hy::GlaScan& a, hipStream_t s) {
+    if (a.segs > 1) gla_scan_pass<D, true>(a, a.segs - 1, s);
+    gla_scan_pass<D, false>(a, a.segs, s);
 }
 
 void launch_hy_gla_scan(const uint16_t* proj, int ldp, int q_off, int k_off, int v_off, const float* qscale, const float* kscale,
                         float q_mul, const float* decay, const int32_t* q_start, const int32_t* pos0, const int32_t* slots,
-                        float* S, float* o, int B, int HK, int H, int D, int Dv, const float* vscale, hipStream_t s) {
-    const hy::GlaScan a{proj, ldp, q_off, k_off, v_off, qscale, kscale, vscale, decay, q_mul, q_start, pos0, slots, S, o, B, HK, H, Dv};
+                        float* S, float* o, int B, int HK, int H, int D, int Dv, const float* vscale, int segs, float* seg, hipStream_t s) {
+    const hy::GlaScan a{proj, ldp, q_off, k_off, v_off, qscale, kscale, vscale, decay, q_mul, q_start, pos0, slots, S, o, B, HK, H, Dv,
+                        segs, seg, segs > 1 ? seg + (int64_t)segs * B * H * D * Dv : nullptr};
     if (D == 32) gla_scan_run<32>(a, s);
     else if (D == 64) gla_scan_run<64>(a, s);
     else if (D == 128) gla_scan_run<128>(a, s);

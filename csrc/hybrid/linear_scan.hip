@@ -422,7 +422,7 @@ void launch_hy_chunk_scan(const uint16_t*, int, int, int, int, const float*, con
 
 bool hy_gla_scan_ok(const void*, const void*, int, int, int, int, int, int, int);
 void launch_hy_gla_scan(const uint16_t*, int, int, int, int, const float*, const float*, float, const float*, const int32_t*,
-                        const int32_t*, const int32_t*, float*, float*, int, int, int, int, int, const float*, hipStream_t);
+                        const int32_t*, const int32_t*, float*, float*, int, int, int, int, int, const float*, int, float*, hipStream_t);
 
 bool hy_state_step_ok(const void*, const void*, const void*, int, int, int, int, int);
 void launch_hy_state_step(const uint16_t*, int, int, int, int, const float*, const float*, float, const float*, bool, int,
@@ -527,7 +527,7 @@ bool launch_hy_linear_scan(const void* proj, int ldp, int q_off, int k_off, int 
     }
     if (chd && !delta && !f32 && hy_gla_scan_ok(proj, decay, ldp, q_off, k_off, v_off, D, Dv, longest)) {
         launch_hy_gla_scan((const uint16_t*)proj, ldp, q_off, k_off, v_off, qscale, kscale, q_mul, decay, q_start, pos0, slots, S, o,
-                           B, HK, H, D, Dv, vscale, s);
+                           B, HK, H, D, Dv, vscale, segs, seg, s);
         return true;
     }
     if (!chd && !f32 && hy_chunk_scan_ok(proj, ldp, q_off, k_off, v_off, D, Dv, longest, delta)) {

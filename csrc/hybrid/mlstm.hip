@@ -446,7 +446,8 @@ bool hy_chunk_scan_ok(const void*, int, int, int, int, int, int, int, bool);
 void launch_hy_chunk_mlstm(const uint16_t*, int, const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*,
                            float*, float*, float*, int, int, int, int, int, float, int, hipStream_t);
 
-// D <= 512.  segs: hy_chunk_segments.  scratch: 3 T H + B H D + hy_chunk_segment_floats floats.  longest: the most tokens that any sequence brings (or an upper bound of it).
+// D <= 512.  segs: hy_chunk_segments.  scratch: 3 T H + B H D + hy_chunk_segment_floats floats.  longest: the most tokens that any
+// sequence brings (or an upper bound of it).
 void launch_hy_mlstm_scan(const void* proj, int ldp, const float* gate_pre, const int32_t* q_start, const int32_t* pos0,
                           const int32_t* slots, float* S, float* n, float* m, float* scratch, float* o, int T, int B, int H, int D,
                           int Dv, float cap, int longest, int segs, bool f32, hipStream_t s) {

@@ -181,13 +181,13 @@ def test_mlstm(H, D, Dv, gate):
 
 
 @pytest.mark.parametrize("lens,starts", [([1100, 40, 0, 513, 1023], [0, 3, 5, 9, 0]), ([2500], [7])])
-@pytest.mark.parametrize("form", ["token", "mlstm"])
-def test_segments(lens, starts, form):
-    """Few, long sequences: their chunks are dealt to segments (1100 tokens: four of 18 chunks; 2500: ten of 40), whose states
-    are carried first; against the same sequences in launches too wide for segments."""
+@pytest.mark.parametrize("form,D", [("token", 64), ("mlstm", 64), ("rows", 32), ("rows", 64), ("rows", 128), ("rows", 256)])
+def test_segments(lens, starts, form, D):
+    """Few, long sequences: their chunks are dealt to segments (1100 tokens: four of 18 chunks; 2500: ten of 40; one
+    decay per row: nine of 69 and 16 of 157), whose states are carried first; against the same sequences in launches too wide for segments."""
     from chronos.ops import hybrid as hops
 
-    H, D, Dv, T = 2, 64, 72, sum(lens)
+    H, Dv, T = 2, 72, sum(lens)
     reps = 40   # copies of the sequences that fill the chip: no segments
     g = torch.Generator(device=DEV).manual_seed(T)
     rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
@@ -196,6 +196,9 @@ def test_segments(lens, starts, form):
     gp[:, H:] += 3.0
     dec = torch.exp(-0.2 * torch.rand(T, H, device=DEV, generator=g))
     dec[7::90], dec[11::400] = -0.9, 1.2
+    if form == "rows":
+        dec = torch.rand(T, H, D, device=DEV, generator=g) ** (1 / 16)
+        dec[300:420:40], dec[7::90], dec[11::400], dec[23::610, :, ::3] = 0.0, -0.9, 1.2, 1e-30
     B = len(lens)
     S0, n0, m0 = rnd(B, H, D, Dv) * 0.3, rnd(B, H, D) * 0.5, rnd(B, H)
 
@@ -208,7 +211,7 @@ def test_segments(lens, starts, form):
         if form == "mlstm":
             o = hops.mlstm_scan(proj.repeat(r, 1), gp.repeat(r, 1), *rg, S, n, m, H, D, Dv, 9.0, max(lens))
         else:
-            o = hops.linear_scan(proj.repeat(r, 1), 0, H * D, 2 * H * D, None, None, 0.3, dec.repeat(r, 1), None, *rg, S, H, H, D, Dv,
+            o = hops.linear_scan(proj.repeat(r, 1), 0, H * D, 2 * H * D, None, None, 0.3, dec.repeat(r, *[1] * (dec.dim() - 1)), None, *rg, S, H, H, D, Dv,
                                  None, max(lens))
         return o[:T], S[:B], n[:B], m[:B]
 
