@@ -623,6 +623,7 @@ std::tuple<Tensor, Tensor> gemm_skinny(const Tensor& x, const Tensor& w, int64_t
     CHK(cfg >= 0 && cfg < chronos::kSkinnyConfigs, "gemm_skinny: cfg");
     CHK(mode >= 0 && mode <= 2, "gemm_skinny: mode");
     const int RT = chronos::gemm_skinny_rt((int)cfg), MT = chronos::gemm_skinny_mt((int)cfg);
+    CHK(M >= 1 && M <= 16 * MT, "gemm_skinny: M must be in [1, 16 * MT] of the config");
     const bool uneven = cfg >= chronos::kSkinnyUneven;
     CHK(splitk >= 1 && K % (uneven ? 64 : 64 * chronos::gemm_skinny_nw((int)cfg) * splitk) == 0 && (!uneven || splitk <= 64) &&
             K <= (1 << 20) && N * K < (1LL << 40),

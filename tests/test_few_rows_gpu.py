@@ -44,7 +44,8 @@ def test_uneven(cfg, splitk):
     for rows in (1, m - 1, m):
         _check(torch.ops.chronos.gemm_skinny(x[:rows], w, 0, cfg, splitk, None, None, 1e-5)[0], x[:rows], w)
     for bad in (lambda: torch.ops.chronos.gemm_skinny(x, w[:, :k - 8].contiguous(), 0, cfg, splitk, None, None, 1e-5),
-                lambda: torch.ops.chronos.gemm_skinny(x, w, 1, cfg, splitk, None, None, 1e-5)):
+                lambda: torch.ops.chronos.gemm_skinny(x, w, 1, cfg, splitk, None, None, 1e-5),
+                lambda: torch.ops.chronos.gemm_skinny(torch.cat([x, x[:1]]), w, 0, cfg, splitk, None, None, 1e-5)):
         with pytest.raises(RuntimeError):
             bad()
 

@@ -144,9 +144,22 @@ def test_rejects_bad_shapes():
     g = torch.Generator(device=DEV).manual_seed(2)
     x = _rand((20, 512), g)
     w = _rand((256, 512), g)
-    with pytest.raises(RuntimeError):
-        _sk(x, w, 0, 0, 1)  # M = 20 > 16 MT for cfg 0
+    with pytest.raises(RuntimeError, match="M must be"):
+        _sk(_rand((20, 1024), g), _rand((256, 1024), g), 0, 0, 1)  # M = 20 > 16 MT for cfg 0
     with pytest.raises(RuntimeError):
         _sk(x[:8], w, 0, 0, 1)  # K % (64 * 16)
     with pytest.raises(RuntimeError):
         _sk(x[:8], w, 1, 0, 1)  # swiglu needs RT even
+
+
+@pytest.mark.parametrize("cfg", sorted(CFGS))
+@pytest.mark.parametrize("mode,splitk", [(0, 1), (0, 2), (2, 1)])
+def test_rejects_too_many_rows(cfg, mode, splitk):
+    """A row more than the config's tiles hold, all else in order (the kernel would leave it unwritten), and no row at all."""
+    mt = CFGS[cfg][1]
+    g = torch.Generator(device=DEV).manual_seed(5)
+    w = _rand((256, 2048), g)
+    for m in (0, 16 * mt + 1):
+        with pytest.raises(RuntimeError, match="M must be"):
+            _sk(_rand((m, 2048), g), w, mode, cfg, splitk, _rand((m, 256), g) if mode == 2 else None)
+    assert _sk(_rand((16 * mt, 2048), g), w, mode, cfg, splitk, _rand((16 * mt, 256), g) if mode == 2 else None)[0].shape == (16 * mt, 256)
