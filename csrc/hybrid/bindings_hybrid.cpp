@@ -9,6 +9,7 @@
 #include <torch/library.h>
 
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <cstdint>
 #include <tuple>
 
@@ -182,9 +183,9 @@ void hy_act(Tensor& x, int64_t kind) {
     chronos::launch_hy_act(x.data_ptr(), x.numel(), (int)kind, f32(x), stream());
 }
 
-// the most new tokens of any of B sequences with T in all (a launch-shape hint): max_q, or where the caller did not say
-// (0) what it is if the others bring one each
-static int longest(int64_t T, int64_t B, int64_t max_q) { return (int)(max_q > 0 ? max_q : T - B + 1); }
+// the most new tokens of any of B sequences with T in all: max_q, or where the caller did not say (0) what it is if the others
+// bring one each.  A hint for the choice of kernel only: each of them takes ranges of any length.
+static int longest(int64_t T, int64_t B, int64_t max_q) { return (int)(max_q > 0 ? std::min(max_q, T) : std::max<int64_t>(T - B + 1, 1)); }
 
 Tensor hy_mlstm_scan(const Tensor& proj, const Tensor& gate_pre, const Tensor& q_start, const Tensor& pos0,
                      const Tensor& slots, Tensor& S, Tensor& n, Tensor& m, int64_t H, int64_t D, int64_t Dv, double cap, int64_t max_q) {

@@ -511,7 +511,8 @@ static bool linear_scan_d(bool pipe, const T* proj, int ldp, int q_off, int k_of
 // delta: beta != nullptr.  vscale (float [T, H], may be nullptr; without delta only): a factor on the written value.
 // chd: decay holds one number per state row ([T, H, D]) instead of one per head ([T, H]).
 // fixed (not with chd): decay holds one number per head for all tokens ([H]).
-// longest: the most tokens that any sequence brings (or an upper bound of it).  segs, seg: hy_chunk_segments and its scratch.
+// longest: the most tokens that any sequence brings, as far as the caller knows (it only picks the kernel).
+// segs, seg: hy_chunk_segments and its scratch.
 // Returns false when D has no instantiation (D > 256).
 bool launch_hy_linear_scan(const void* proj, int ldp, int q_off, int k_off, int v_off, const float* qscale,
                            const float* kscale, float q_mul, const float* decay, bool chd, bool fixed, const float* beta,

@@ -447,7 +447,7 @@ void launch_hy_chunk_mlstm(const uint16_t*, int, const float*, const int32_t*, c
                            float*, float*, float*, int, int, int, int, int, float, int, hipStream_t);
 
 // D <= 512.  segs: hy_chunk_segments.  scratch: 3 T H + B H D + hy_chunk_segment_floats floats.  longest: the most tokens that any
-// sequence brings (or an upper bound of it).
+// sequence brings, as far as the caller knows (it only picks the kernel).
 void launch_hy_mlstm_scan(const void* proj, int ldp, const float* gate_pre, const int32_t* q_start, const int32_t* pos0,
                           const int32_t* slots, float* S, float* n, float* m, float* scratch, float* o, int T, int B, int H, int D,
                           int Dv, float cap, int longest, int segs, bool f32, hipStream_t s) {

@@ -1,5 +1,5 @@
-// state_step.hip — one token per sequence of the recurrences of linear_scan.hip and mlstm.hip (decode): the state is read once,
-// stepped and written once, bfloat16 rows.
+// state_step.hip — the recurrences of linear_scan.hip and mlstm.hip for one token per sequence (decode): the state is read once,
+// stepped and written once, bfloat16 rows.  A longer range is walked token by token, so the launch's hint need not be true.
 //
 //     plain:   S <- d S + k (w v),  o = r q^T S          d: one decay per head (fixed or per token) or per state row
 //     delta:   u = beta (v - w k^T (d S)),  S <- d S + k (w u),  o = r q^T S
@@ -36,8 +36,8 @@ __global__ void __launch_bounds__(D >= 128 ? 2 * D : 256) state_step_kernel(cons
     __shared__ float qs[D], ks[D], ds[ROWS ? D : 1];
     __shared__ __attribute__((aligned(16))) f32x4 part[NW][CL];
     const int b = blockIdx.x, hd = blockIdx.y, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int t = a.q_start[b];
-    if (a.q_start[b + 1] <= t) return;
+    const int t0 = a.q_start[b], t1 = a.q_start[b + 1];
+    if (t1 <= t0) return;
     const int cl = lane % CL, rl = lane / CL, col = (blockIdx.z * CL + cl) * 4, hk = hd / (a.H / a.HK);
     const bool live = col < a.Dv, fresh = a.pos0[b] == 0;
     const int row0 = wv * (NI * RI) + rl;                            // this lane's rows: row0 + RI i
@@ -46,24 +46,6 @@ __global__ void __launch_bounds__(D >= 128 ? 2 * D : 256) state_step_kernel(cons
 #pragma unroll
     for (int i = 0; i < NI; ++i)
         S[i] = live && !fresh ? *reinterpret_cast<const f32x4*>(Sp + (int64_t)(RI * i) * a.Dv) : f32x4{0.f, 0.f, 0.f, 0.f};
-    const uint16_t* const p = a.proj + (int64_t)t * a.ldp;
-    for (int r = threadIdx.x; r < D; r += NT) {
-        qs[r] = bf2f(p[a.q_off + hk * D + r]);
-        ks[r] = bf2f(p[a.k_off + hk * D + r]);
-        if constexpr (ROWS) ds[r] = a.decay[((int64_t)t * a.H + hd) * D + r];
-    }
-    const float g = ROWS ? 1.f : a.decay[(int64_t)t * a.dts + hd];
-    float w = a.kscale != nullptr ? a.kscale[(int64_t)t * a.HK + hk] : 1.f;
-    if (a.vscale != nullptr) w *= a.vscale[(int64_t)t * a.H + hd];
-    float r = a.qscale != nullptr ? a.qscale[(int64_t)t * a.HK + hk] : a.q_mul;
-    if (a.den != nullptr) r /= a.den[(int64_t)t * a.H + hd];
-    const float bt = DELTA ? a.beta[(int64_t)t * a.H + hd] : 1.f;
-    f32x4 u = {0.f, 0.f, 0.f, 0.f};
-    if (live) {
-        const u16x4 v = *reinterpret_cast<const u16x4*>(p + a.v_off + (int64_t)hd * a.Dv + col);
-        u = f32x4{bf2f(v[0]), bf2f(v[1]), bf2f(v[2]), bf2f(v[3])};
-    }
-    __syncthreads();
     auto total = [&](f32x4 x) {   // the sum over all rows of this lane's columns, in every lane
 #pragma unroll
         for (int o = CL; o < 64; o <<= 1)
@@ -76,33 +58,55 @@ __global__ void __launch_bounds__(D >= 128 ? 2 * D : 256) state_step_kernel(cons
         for (int i = 1; i < NW; ++i) x += part[i][cl];
         return x;
     };
+    auto step = [&](int t) {
+        const uint16_t* const p = a.proj + (int64_t)t * a.ldp;
+        for (int r = threadIdx.x; r < D; r += NT) {
+            qs[r] = bf2f(p[a.q_off + hk * D + r]);
+            ks[r] = bf2f(p[a.k_off + hk * D + r]);
+            if constexpr (ROWS) ds[r] = a.decay[((int64_t)t * a.H + hd) * D + r];
+        }
+        const float g = ROWS ? 1.f : a.decay[(int64_t)t * a.dts + hd];
+        float w = a.kscale != nullptr ? a.kscale[(int64_t)t * a.HK + hk] : 1.f;
+        if (a.vscale != nullptr) w *= a.vscale[(int64_t)t * a.H + hd];
+        float r = a.qscale != nullptr ? a.qscale[(int64_t)t * a.HK + hk] : a.q_mul;
+        if (a.den != nullptr) r /= a.den[(int64_t)t * a.H + hd];
+        const float bt = DELTA ? a.beta[(int64_t)t * a.H + hd] : 1.f;
+        f32x4 u = {0.f, 0.f, 0.f, 0.f};
+        if (live) {
+            const u16x4 v = *reinterpret_cast<const u16x4*>(p + a.v_off + (int64_t)hd * a.Dv + col);
+            u = f32x4{bf2f(v[0]), bf2f(v[1]), bf2f(v[2]), bf2f(v[3])};
+        }
+        __syncthreads();
 #pragma unroll
-    for (int i = 0; i < NI; ++i) S[i] *= ROWS ? ds[row0 + RI * i] : g;
-    if constexpr (DELTA) {
-        f32x4 x = {0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < NI; ++i) S[i] *= ROWS ? ds[row0 + RI * i] : g;
+        if constexpr (DELTA) {
+            f32x4 x = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < NI; ++i) x += S[i] * ks[row0 + RI * i];
-        u = (u - total(x) * w) * bt;
-        __syncthreads();   // part is read
-    }
-    u *= w;
-    f32x4 x[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+            for (int i = 0; i < NI; ++i) x += S[i] * ks[row0 + RI * i];
+            u = (u - total(x) * w) * bt;
+            __syncthreads();   // part is read
+        }
+        u *= w;
+        f32x4 x[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-        S[i] += u * ks[row0 + RI * i];
-        x[i & 1] += S[i] * qs[row0 + RI * i];
-    }
-    if (live)
+        for (int i = 0; i < NI; ++i) {
+            S[i] += u * ks[row0 + RI * i];
+            x[i & 1] += S[i] * qs[row0 + RI * i];
+        }
+        if (live && t + 1 == t1)
 #pragma unroll
-        for (int i = 0; i < NI; ++i) *reinterpret_cast<f32x4*>(Sp + (int64_t)(RI * i) * a.Dv) = S[i];
-    const f32x4 y = total(x[0] + x[1]) * r;
-    if (wv == 0 && rl == 0 && live) *reinterpret_cast<f32x4*>(a.o + ((int64_t)t * a.H + hd) * a.Dv + col) = y;
+            for (int i = 0; i < NI; ++i) *reinterpret_cast<f32x4*>(Sp + (int64_t)(RI * i) * a.Dv) = S[i];
+        const f32x4 y = total(x[0] + x[1]) * r;
+        if (wv == 0 && rl == 0 && live) *reinterpret_cast<f32x4*>(a.o + ((int64_t)t * a.H + hd) * a.Dv + col) = y;
+    };
+    step(t0);   // (apart from the loop: in front of one the compiler waits for the whole state)
+    for (int t = t0 + 1; t < t1; ++t) step(t);   // ranges longer than the launch was told
 }
 
 }  // namespace hy
 
-// bfloat16 rows, one token per sequence at most (longest: the most that any sequence brings), a state of 32, 64, 128 or 256 rows of a
-// multiple of 4 columns, v on 8-byte and the state and o on 16-byte boundaries
+// bfloat16 rows, one token per sequence (longest: the most that any sequence brings, as far as the caller knows), a state of 32, 64,
+// 128 or 256 rows of a multiple of 4 columns, v on 8-byte and the state and o on 16-byte boundaries
 bool hy_state_step_ok(const void* proj, const void* S, const void* o, int ldp, int v_off, int D, int Dv, int longest) {
     return longest == 1 && (D == 32 || D == 64 || D == 128 || D == 256) && Dv % 4 == 0 && (reinterpret_cast<uintptr_t>(proj) & 7) == 0 &&
            ((ldp | v_off) & 3) == 0 && hy::aligned16(S, o);

@@ -97,7 +97,8 @@ def act_inplace(x, kind: int):
 
 
 def mlstm_scan(proj, gate_pre, q_start, pos0, slots, S, n, m, H: int, D: int, Dv: int, cap: float, max_q: int = 0):
-    """``max_q``: the most tokens any sequence brings in this step (a launch-shape hint; 0 = unknown)."""
+    """``max_q``: the most tokens any sequence brings in this step (picks the kernel, any value gives the same
+    results up to rounding; 0 = unknown)."""
     if _gpu(proj):
         return _k().hy_mlstm_scan(proj, gate_pre, q_start, pos0, slots, S, n, m, H, D, Dv, cap, max_q)
     return ref.mlstm_scan(proj, gate_pre, q_start, pos0, slots, S, n, m, H, D, Dv, cap)
@@ -267,7 +268,8 @@ def decay_pow(z, inv_tau: float):
 
 def linear_scan(proj, q_off: int, k_off: int, v_off: int, qscale, kscale, q_mul: float, decay, beta, q_start, pos0,
                 slots, S, HK: int, H: int, D: int, Dv: int, vscale=None, max_q: int = 0):
-    """``max_q``: the most tokens any sequence brings in this step (a launch-shape hint; 0 = unknown)."""
+    """``max_q``: the most tokens any sequence brings in this step (picks the kernel, any value gives the same
+    results up to rounding; 0 = unknown)."""
     if _gpu(proj):
         return _k().hy_linear_scan(proj, q_off, k_off, v_off, qscale, kscale, q_mul, decay, beta, q_start, pos0, slots,
                                    S, HK, H, D, Dv, vscale, max_q)

@@ -72,3 +72,34 @@ def test_step(form, HK, H, D, Dv):
     assert float((o.double() - want).norm() / want.norm()) < 2e-6
     assert float((S.double() - Sw).norm() / Sw.norm()) < 2e-6
     assert torch.equal(S[3], S0[3]) and torch.equal(S[5], S0[5]) and torch.equal(S[6], S0[6])
+
+
+@pytest.mark.parametrize("count", [[3, 0, 0], [0, 2, 0, 1], [2, 5, 0]])
+@pytest.mark.parametrize("max_q", [0, 1])
+@pytest.mark.parametrize("form", ["fixed", "token", "rows", "delta", "mlstm"])
+def test_longer_ranges(form, max_q, count):
+    """Ranges of several tokens where the launch takes one per sequence for the longest: beside empty ones when nobody says (T <= B),
+    or with a hint of 1.  Against the plain recurrence of hybrid_ref in float32."""
+    from chronos.ops import hybrid as hops
+
+    H, D, Dv, T = 2, 64, 72, sum(count)
+    g = torch.Generator().manual_seed(T)
+    rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32)  # noqa: E731
+    qs = [sum(count[:i]) for i in range(len(count) + 1)]
+    args = [rnd(T, 2 * H * D + H * Dv + 16).bfloat16(), *(i32(x) for x in (qs, [4, 0, 7, 2][:len(count)], [1, 3, 0, 4][:len(count)])), rnd(5, H, D, Dv)]
+    n, m, gp = rnd(5, H, D), rnd(5, H), rnd(T, 2 * H)
+    dec = torch.rand(H, generator=g) if form == "fixed" else torch.rand(T, H, D, generator=g) if form == "rows" else torch.rand(T, H, generator=g)
+    beta = torch.rand(T, H, generator=g) if form == "delta" else None
+
+    def run(dev):
+        proj, q, p0, sl, S = (t.to(dev, copy=True) for t in args)
+        if form == "mlstm":
+            st = [S, n.to(dev, copy=True), m.to(dev, copy=True)]
+            return hops.mlstm_scan(proj, gp.to(dev), q, p0, sl, *st, H, D, Dv, 9.0, max_q), *st
+        o = hops.linear_scan(proj, 0, H * D, 2 * H * D, None, None, 0.3, dec.to(dev), None if beta is None else beta.to(dev), q, p0, sl, S,
+                             H, H, D, Dv, None, max_q)
+        return o, S
+
+    for got, want in zip(run(DEV), run("cpu")):   # both sides round
+        assert float((got.cpu() - want).norm() / want.norm()) < 4e-6
