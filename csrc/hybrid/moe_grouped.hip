@@ -455,10 +455,16 @@ static void moe_grouped(const uint16_t* h, const int32_t* idx, const float* wt, 
     hy::moe_combine_kernel<<<T, 256, 0, s>>>(h, yrows, idx, wt, item_row, out, d, top, E, ACT != hy::kActGlu);
 }
 
+// no expert chosen: the sum of nothing
+static void moe_no_choice(const uint16_t* h, uint16_t* out, int T, int d, hipStream_t s) {
+    hy::moe_combine_kernel<<<T, 256, 0, s>>>(h, nullptr, nullptr, nullptr, nullptr, out, d, 0, 0, 0);
+}
+
 void launch_hy_moe_grouped(const uint16_t* h, const int32_t* idx, const float* wt, const uint16_t* w_up,
                            const uint16_t* w_down, uint16_t* out, int32_t* meta, uint16_t* z, uint16_t* yrows, int T,
                            int d, int F, int E, int top, int act, hipStream_t s) {
-    if (T == 0 || top == 0) return;
+    if (T == 0) return;
+    if (top == 0) return moe_no_choice(h, out, T, d, s);
     const int tm = hy_moe_tile(T * top, E, d, F, F);
 #define HY_MOE(TM, ACT) moe_grouped<TM, ACT>(h, idx, wt, w_up, w_down, out, meta, z, yrows, T, d, F, E, top, 0.f, 0.f, 0.f, s)
     if (act == 0) { if (tm == 32) HY_MOE(32, 0); else if (tm == 128) HY_MOE(128, 0); else HY_MOE(256, 0); }
@@ -471,7 +477,8 @@ void launch_hy_moe_grouped(const uint16_t* h, const int32_t* idx, const float* w
 void launch_hy_moe_glu_grouped(const uint16_t* h, const int32_t* idx, const float* wt, const uint16_t* w_gu,
                                const uint16_t* w_down, uint16_t* out, int32_t* meta, uint16_t* z, uint16_t* yrows, int T,
                                int d, int F, int E, int top, float limit, float slope, float shift, hipStream_t s) {
-    if (T == 0 || top == 0) return;
+    if (T == 0) return;
+    if (top == 0) return moe_no_choice(h, out, T, d, s);
     const int tm = hy_moe_tile(T * top, E, d, F, 2 * F);
 #define HY_MOE(TM) moe_grouped<TM, hy::kActGlu>(h, idx, wt, w_gu, w_down, out, meta, z, yrows, T, d, F, E, top, limit, slope, shift, s)
     if (tm == 32) HY_MOE(32);

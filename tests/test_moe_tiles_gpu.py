@@ -51,6 +51,23 @@ def test_experts(T, d, F, E, top, kind):
     _close(hops.moe_glu_ffn(h, idx, wt, tiled, wd, 2.0, 1.702, 1.0, BF, True), ref.moe_glu_ffn(h, idx, wt, wgu, wd, 2.0, 1.702, 1.0, BF))
 
 
+@pytest.mark.parametrize("T", [1, 37, 3000])
+def test_no_choice(T):
+    """idx [T, 0]: the sum of no experts is zero, whatever the result's memory held."""
+    from chronos.ops import hybrid as hops
+
+    d, F, E = 256, 128, 4
+    h = torch.randn(T, d, device=DEV).to(BF)
+    idx, wt = torch.empty(T, 0, device=DEV, dtype=torch.int32), torch.empty(T, 0, device=DEV)
+    wu, wgu, wd = (torch.randn(E, *s, device=DEV).to(BF) for s in ((F, d), (2 * F, d), (d, F)))
+    for call in (lambda: hops.moe_ffn(h, idx, wt, wu, wd, 0, BF), lambda: hops.moe_ffn(h, idx, wt, wu, wd, 1, BF),
+                 lambda: hops.moe_glu_ffn(h, idx, wt, wgu, wd, 2.0, 1.702, 1.0, BF, True),
+                 lambda: hops.moe_glu_ffn(h, idx, wt, wgu, wd, 2.0, 1.702, 1.0, BF)):
+        held = torch.full((T, d), float("nan"), device=DEV, dtype=BF)   # the block that the result is likely to get
+        del held
+        assert torch.equal(call(), torch.zeros_like(h))
+
+
 def test_experts_in_a_graph():
     """Several replays with new choices in between: the routing is only known on the device."""
     from chronos.ops import hybrid as hops
