@@ -78,7 +78,8 @@ __device__ __forceinline__ f32x4 mfma_16x16x16(bf16x4 a, bf16x4 b, f32x4 c) {
 __device__ __forceinline__ void dma_1k(const void* src, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds) : "memory");
 }
-// The same through a buffer descriptor: byte voff + soff of a buffer of `bytes` bytes (past its end: zeros)
+// The same through a buffer descriptor: byte voff + soff of a buffer of `bytes` bytes, which must lie inside (the range check may leave
+// out soff)
 __device__ __forceinline__ void dma_1k_buf(const void* base, uint32_t bytes, uint32_t lds, uint32_t voff, int soff) {
     typedef int i32x4 __attribute__((ext_vector_type(4)));
     const uint64_t b = (uint64_t)base;

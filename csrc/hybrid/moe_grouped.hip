@@ -19,6 +19,7 @@
 // The tile loop is an LDS-DMA ring (16x16x32 bf16 MFMAs, XOR-swizzled images, one barrier per k-step with a counted vmcnt) at
 // three tile sizes, below.  Needs d % 128 == 0 and F % 128 == 0.
 #include "hybrid_common.h"
+#include "moe_tile.h"
 
 namespace chronos {
 namespace hy {
@@ -274,7 +275,7 @@ __global__ void __launch_bounds__(256, 2) moe_gemm_kernel(const uint16_t* __rest
     moe_store<ACT, C::NS, C::NM>(acc, y, row_item, m0 + 16 * C::NM * wm, tn * C::TN + C::TN / 2 * wn, N, lane, limit, slope, shift);
 }
 
-// The 256 x 256 tile (x and one expert's weights below 4 and 2 GiB; weight rows past the end read as zeros).  Two sets of operands in registers: while
+// The 256 x 256 tile (x and one expert's weights below 4 and 2 GiB; weight rows past the end repeat the last one).  Two sets of operands in registers: while
 // one half of a k-step (32 deep) is multiplied the other half's fragments are read from LDS, so that neither the LDS nor
 // the matrix cores wait for the other; one barrier per k-step, in its middle, behind which the buffer that everybody has read is
 // refilled for the step after next.
@@ -295,11 +296,10 @@ __global__ void __launch_bounds__(512, 1) moe_gemm256_kernel(const uint16_t* __r
     const int m0 = tile * 256;
     // wave w stages image rows 32 w .. 32 w + 31 of both operands in four pieces of 8 rows
     const int pr = lane >> 3, pc = (lane & 7) ^ pr;
-    const uint32_t wvoff = (uint32_t)(pr * K + pc * 8) * 2;
-    const int wsoff = (tn * 256 + 32 * wave) * K * 2;
-    uint32_t xvoff[4];
+    uint32_t wvoff[4], xvoff[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
+        wvoff[i] = moe_weight_offset(tn, wave, i, lane, N, K);
         uint32_t xr = m0 + 32 * wave + 8 * i + pr;
         if constexpr (GATHER) {
             const int it = row_item[xr];
@@ -310,7 +310,7 @@ __global__ void __launch_bounds__(512, 1) moe_gemm256_kernel(const uint16_t* __r
     const uint16_t* we = w + (int64_t)e * N * K;
     const uint32_t lds0 = lds_offset(smem);
     auto dma_w = [&](int kt, int i) {
-        dma_1k_buf(we, (uint32_t)N * K * 2, lds0 + (kt & 1) * STAGE + (4 * wave + i) * 1024, wvoff, wsoff + (i * 8 * K + kt * 64) * 2);
+        dma_1k_buf(we, (uint32_t)N * K * 2, lds0 + (kt & 1) * STAGE + (4 * wave + i) * 1024, wvoff[i], kt * 128);
     };
     auto dma_x = [&](int kt, int i) {
         dma_1k_buf(x, xbytes, lds0 + (kt & 1) * STAGE + IMG + (4 * wave + i) * 1024, xvoff[i], kt * 128);
