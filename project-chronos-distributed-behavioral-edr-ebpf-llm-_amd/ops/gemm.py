@@ -205,14 +205,14 @@ def pp_plan(m: int, n: int, k: int, mode: int = PP_PLAIN) -> Optional[tuple[int,
 
 def few_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     """(config, split-K) of the hand-written GEMM for few rows of a shape that no plan lists, or None (the GEMV or the
-    library).  Where it wins, measured on the grid of _FEW, us, GEMV or library -> this:
+    library): of shapes that the kernels take (rows of w in 16s, at least one; K in 64s up to 2^20).  Where it wins, measured on the
+    grid of _FEW, us, GEMV or library -> this:
     one row: K < 2048, where the GEMV's waves have one step each (5632 x 1024: 7.3 -> 5.7; 32768 x 512: 22 -> 9.7; at K = 2048 the
     two are level), and K % 512, which the GEMV does not take (1024 x 2816: 8.6 -> 5.7): no slower at any of 41 shapes;
     2 .. 64 rows: weights up to 12.5 M elements, from 33 rows on up to 7 M or K <= 2048 (2048 x 2048, 16 rows: 11.0 -> 6.0; 64 rows:
-    11.7 -> 8.1): 1.3 .. 1.6 times as fast on average, 4 of 590 slower by more than 3 %, the worst by 6 %; 48 shapes off the grid: 1.7 times,
-none slower.  More weights than that stream from
-    memory at the library's rate too (8192 x 8192, 16 rows: 30.5, 31.1 here), except that it keeps half the chip idle for wide
-    outputs of up to 48 rows (22016 x 2048, 16 rows: 44 -> 21)."""
+    11.7 -> 8.1): 1.3 .. 1.6 times as fast on average, 4 of 590 slower by more than 3 %, the worst by 6 %; 48 shapes off the grid: 1.7
+    times, none slower.  More weights than that stream from memory at the library's rate too (8192 x 8192, 16 rows: 30.5, 31.1 here),
+    except that it keeps half the chip idle for wide outputs of up to 48 rows (22016 x 2048, 16 rows: 44 -> 21)."""
     key = (m, n, k, -1)
     hit = _plan_cache.get(key, False)
     if hit is not False:
@@ -223,7 +223,7 @@ none slower.  More weights than that stream from
     else:
         ok = GEMV_MAX_M < m <= 64 and (nk <= 12_500_000 and (m <= 32 or k <= 2048 or nk <= 7_000_000) or
                                        m <= 48 and n >= 12288 and nk <= (40_000_000 if n < 16384 else 100_000_000))
-    if ok and k % 64 == 0 and n % 16 == 0 and PP_MODE == "auto" and (n, k, PP_PLAIN) not in _plan_file():
+    if ok and n > 0 and n % 16 == 0 and k % 64 == 0 and k <= 1 << 20 and PP_MODE == "auto" and (n, k, PP_PLAIN) not in _plan_file():
         best = None
         for cfg, c in next(models for most, models in _FEW if m <= most).items():
             bn, bm, nw = _UNEVEN.get(cfg) or (_PP_BN[cfg], _PP_BM[cfg], 1)

@@ -75,3 +75,13 @@ def test_fp8_qplan(monkeypatch):
     monkeypatch.setattr(ops, "_QGEMM", "auto")
     assert ops._qown(512, 28672, 4096, True) is False
     assert ops._qown(3, 4096, 4096, False) is True  # unmeasured: the round-1 rule (GEMV at M <= 4)
+
+
+@pytest.mark.parametrize("m", [1, 2, 33, 64])
+def test_few_rows_of_shapes_that_the_kernels_refuse(monkeypatch, m):
+    """No output column, a K beyond 2^20, sizes off the kernels' steps: the library, which takes them all."""
+    monkeypatch.setattr(G, "_plan_cache", {})
+    monkeypatch.setattr(G, "PP_MODE", "auto")
+    for n, k in [(0, 512), (0, 1024), (0, 2048), (16, (1 << 20) + 64), (24, 1024), (1024, 1000), (1024, 0)]:
+        assert G.few_rows_plan(m, n, k) is None, (n, k)
+    assert G.few_rows_plan(m, 1024, 576) is not None
