@@ -241,8 +241,9 @@ def few_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
 
 
 def _plain_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Operands that the kernels take as they lie, and nothing that has to see the product (gradients, transforms)."""
-    return (type(x) is torch.Tensor and x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16 and w.dim() == 2
+    """Operands that the kernels take as they lie, and nothing that has to see the product (gradients, transforms,
+    autocast, subclasses)."""
+    return (type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter) and not torch.is_autocast_enabled("cuda") and x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16 and w.dim() == 2
             and w.shape[1] == x.shape[-1] and w.device == x.device
             and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
             and not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0

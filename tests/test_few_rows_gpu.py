@@ -69,3 +69,21 @@ def test_other_operands():
     assert xg.grad is not None and xg.grad.shape == xg.shape
     ys = torch.vmap(lambda r: ops.linear(r, w))(big[:8, :1024].contiguous())
     _check(ys, big[:8, :1024], w)
+
+
+@pytest.mark.parametrize("m", [2, 16, 64])
+def test_autocast_and_subclasses(m):
+    """Products that somebody has to see: under autocast they take its type, of a subclass they come back as one."""
+    from chronos import ops
+    from chronos.ops import gemm as G
+
+    class Marked(torch.Tensor):
+        pass
+
+    x, w = (torch.randn(s, device=DEV).bfloat16() for s in ((m, 1024), (1024, 1024)))
+    assert G.few_rows_plan(m, 1024, 1024) is not None
+    with torch.autocast("cuda", torch.float16):
+        y = ops.linear(x, w)
+        assert y.dtype == torch.float16 and torch.equal(y, torch.matmul(x, w.t()))
+    assert ops.linear(x, w).dtype == torch.bfloat16
+    assert type(ops.linear(x, w.as_subclass(Marked))) is Marked
