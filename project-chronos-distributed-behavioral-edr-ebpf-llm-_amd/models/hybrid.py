@@ -842,7 +842,8 @@ class StepMeta:
     last_idx: torch.Tensor
     max_q: int
     shared: dict = field(default_factory=dict)  # what one layer of a step leaves for later layers of the same step
-    fresh: bool = False         # every sequence starts at position 0: its keys are all among the step's tokens
+    # every sequence starts at position 0, whenever these launches run: its keys are all among the step's tokens
+    fresh: bool = False
 
 
 def mix_mlstm(model, li: int, spec: MLSTMSpec, w: dict, h, meta: StepMeta, cache: HybridCache):
@@ -1220,6 +1221,8 @@ class HybridDecoder:
             pos0 = p.pos.index_select(0, p.q_start[:-1].long().clamp(max=max(0, p.pos.numel() - 1)))
             f = p.fresh
             fresh = f is not None and f[0] is p.pos and f[2] is p.q_start and f[1] == p.pos._version and f[3] == p.q_start._version
+            # a graph's replays read whatever positions its tensors hold then
+            fresh = fresh and not (p.pos.is_cuda and torch.cuda.is_current_stream_capturing())
             return StepMeta(p.ids, p.pos, p.tok_seq, p.block_table, p.q_start, pos0, p.slots, p.last_idx,
                             p.max_q or p.ids.numel(), fresh=fresh)
 

@@ -109,3 +109,47 @@ def test_prompt_step(rank):
     assert torch.equal(out[1][0], out[2][0])
     assert torch.equal(out[0][1][0], out[1][1][0])
     assert float((out[0][0] - out[1][0]).norm() / out[1][0].norm()) < 0.03
+
+
+def test_captured_step(monkeypatch):
+    """A prompt step captured while its sequences start at position 0 and replayed after its positions have moved on: the graph must read
+    the cached latents, as the same step run eagerly does."""
+    from chronos.models import hybrid, zokunex
+    from chronos.utils import design_bench as db
+
+    monkeypatch.setattr(hybrid, "EXPAND_MIN", 0)
+    c = db.zokunex_config(dict(db.SIZES["1k"], a=(8, 64, 32, 64, 128)))
+    for layer in c["layers"]:
+        layer["mlp"] = c["layers"][0]["mlp"]
+    cfg = zokunex.config_from_dict(c, name="z", max_position=1024)
+    m = hybrid.HybridDecoder(cfg, zokunex.pack_weights(cfg, zokunex.random_tensors(cfg, 0), torch.device(DEV), torch.bfloat16),
+                             torch.device(DEV), 1024, torch.bfloat16)
+    g = torch.Generator().manual_seed(6)
+    tokens = lambda lens: [torch.randint(0, cfg.vocab_size, (n,), generator=g).tolist() for n in lens]  # noqa: E731
+    lens, bts = [70, 1, 33], [list(range(1 + 10 * b, 11 + 10 * b)) for b in range(3)]
+    step = lambda ids, starts: m.prefill_batch(ids, starts, bts, [0, 1, 2])  # noqa: E731
+    ids = tokens(lens)
+    with torch.no_grad():
+        cache, sb = m.make_cache(31, 16, 3), step(ids, [0, 0, 0])
+        assert sb.fresh is not None
+        m.forward(sb, cache)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = m.forward(sb, cache)
+        for starts in ([32, 16, 48], [0, 0, 0], [16, 80, 1]):
+            prefix, own = tokens(starts), m.make_cache(31, 16, 3)
+            some = [b for b in range(3) if starts[b]]
+            for to in (cache, own):
+                if some:
+                    m.forward(m.prefill_batch([prefix[b] for b in some], [0] * len(some), [bts[b] for b in some], some), to)
+            now = step(ids, starts)
+            want = m.forward(now, own)
+            for name in ("pos", "ctx_len"):
+                getattr(sb, name).copy_(getattr(now, name))
+            graph.replay()
+            torch.cuda.synchronize()
+            if some:
+                assert torch.equal(y, want), starts
+            else:   # (run eagerly it takes the other form; tolerance as above)
+                assert float((y - want).norm() / want.norm()) < 0.03
