@@ -400,7 +400,8 @@ void hy_latent_expanded(const Tensor& q, const Tensor& kv, const Tensor& kr, con
          out.stride(2) == 1 && out.stride(1) == Dv && out.stride(0) % 4 == 0 && out.stride(0) >= H * Dv, "latent_expanded: rows");
     need((reinterpret_cast<uintptr_t>(q.data_ptr()) | reinterpret_cast<uintptr_t>(kv.data_ptr()) | reinterpret_cast<uintptr_t>(kr.data_ptr())) % 16 == 0 &&
          reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0, "latent_expanded: alignment");
-    need(scale > 0 && window >= 0 && max_q >= 0 && max_q <= T, "latent_expanded: scale > 0, window, max_q");
+    need(scale > 0 && window >= 0 && max_q >= 0, "latent_expanded: scale > 0, window, max_q");
+    max_q = std::min(max_q, T);   // (a hint may be too large)
     i32(q_start, "latent_expanded: q_start");
     const int64_t B = q_start.numel() - 1;
     need(B * H < (1LL << 31) && (max_q + 127) / 128 <= 65535, "latent_expanded: launch");

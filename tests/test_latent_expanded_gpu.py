@@ -57,6 +57,16 @@ def test_kernel(H, D, R, Dv, lens, extra):
         assert float((o[sl].double() - want).norm() / want.norm()) < 2 ** -8, (b, n)
 
 
+def test_longest_beyond_the_tokens():
+    """``max_q`` sizes the launch: more than there are tokens is no error."""
+    from chronos.ops import hybrid as hops
+
+    q, kv, kr = torch.randn(40, 2, 96, device=DEV).bfloat16(), torch.randn(40, 2, 128, device=DEV).bfloat16(), torch.randn(40, 32, device=DEV).bfloat16()
+    qs = torch.tensor([0, 33, 40], dtype=torch.int32, device=DEV)
+    a, b = (hops.latent_expanded(q, kv, kr, qs, None, None, -1, None, 0.1, most) for most in (33, 1 << 20))
+    assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("rank", [256, 64])
 def test_prompt_step(rank):
     """The same latents in the first layer's cache, logits within the two forms' rounding (of different intermediates to bfloat16, 2^-9 each
