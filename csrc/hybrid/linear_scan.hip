@@ -61,9 +61,9 @@ __global__ void __launch_bounds__(256) short_conv_vec_kernel(const uint16_t* __r
                                                              const int32_t* __restrict__ slots,
                                                              const uint16_t* __restrict__ hist, uint16_t* __restrict__ y, int T,
                                                              int C, int TK, int silu, const float* __restrict__ bias) {
-    const int c = (blockIdx.x * 256 + threadIdx.x) * 8;
+    const int gx = (C / 8 + 255) / 256, c = (blockIdx.x % gx * 256 + threadIdx.x) * 8;   // workgroups of the same tokens side by side
     if (c >= C) return;
-    const int tb = blockIdx.y * TK, te = min(tb + TK, T);
+    const int tb = blockIdx.x / gx * TK, te = min(tb + TK, T);
     float wf[8][K], bv[8], in[K][8];   // in[i]: the input K - 1 - i tokens back
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -445,7 +445,7 @@ void launch_hy_short_conv(const void* x, int ldx, const float* w, const float* b
     if (!f32 && K >= 2 && K <= 4 && C % 8 == 0 && ldx % 8 == 0 && hy::aligned16(x, hist, y)) {
         // 8 tokens per thread where that leaves a workgroup per CU, else one
         const int gx = (C / 8 + 255) / 256, tk = (int64_t)gx * ((T + 7) / 8) >= 256 ? 8 : 1;
-        const dim3 grid(gx, (T + tk - 1) / tk);
+        const unsigned grid = (unsigned)gx * ((T + tk - 1) / tk);   // (one axis: the second ends at 65535 blocks)
 #define HY_CONV(KK) hy::short_conv_vec_kernel<KK><<<grid, 256, 0, s>>>((const uint16_t*)x, ldx, w, tok_seq, q_start, pos0, slots, (const uint16_t*)hist, (uint16_t*)y, T, C, tk, silu, bias)
         if (K == 2) HY_CONV(2);
         else if (K == 3) HY_CONV(3);

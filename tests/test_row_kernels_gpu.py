@@ -84,6 +84,19 @@ def test_short_conv(C, K, off, many):
         assert torch.equal(hist, hist2)
 
 
+def test_short_conv_of_many_tokens():
+    """More blocks of eight tokens than a second grid axis holds."""
+    from chronos.ops import hybrid as hops, hybrid_ref as ref
+
+    C, K, lens = 8, 3, [8 * 65535 + 1, 20]
+    T, g = sum(lens), _g(1)
+    x, w = _rand(g, T, C, dtype=BF), _rand(g, C, K)
+    seq = torch.arange(2, device=DEV, dtype=torch.int32).repeat_interleave(torch.tensor(lens, device=DEV))
+    qs, zero, slots, hist = _i32([0, lens[0], T]), _i32([0, 0]), _i32([0, 1]), torch.zeros(2, K - 1, C, device=DEV, dtype=BF)
+    y = hops.short_conv(x, w, seq, qs, zero, slots, hist.clone(), True, None, 0)
+    _close(y, ref.short_conv(x, w, qs, zero, slots, hist.clone(), True, None, 0), 8e-3)
+
+
 @pytest.mark.parametrize("H,G,D,Dv,dims,norm,v_rot,v_k", [
     (8, 2, 128, 128, 64, True, False, False), (4, 1, 64, 64, 64, True, True, False), (3, 3, 128, 128, 16, False, False, True),
     (2, 1, 256, 64, 0, False, False, False), (2, 2, 512, 32, 256, True, True, False), (4, 2, 8, 8, 0, True, False, False),
