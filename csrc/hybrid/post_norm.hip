@@ -115,7 +115,7 @@ __global__ void __launch_bounds__(256) glu_kernel(const T* __restrict__ gu, int6
     }
 }
 
-// 16 bytes per lane: 8192 x 2 x 11008, 540 MB: 127 us at 8 bytes per lane, 117 so; 2457 x 2 x 2816: 10.6 and 7.6
+// 16 bytes per lane: 8192 x 2 x 11008, 540 MB: 127 us at 8 bytes per lane, 120 so; 2457 x 2 x 2816: 10.6 and 9.1
 __global__ void __launch_bounds__(256) glu_vec_kernel(const uint16_t* __restrict__ gu, int64_t ldg, uint16_t* __restrict__ y, int64_t ldy,
                                                       int F, float limit, float slope, float shift) {
     const int64_t r = blockIdx.x;

@@ -158,3 +158,25 @@ def test_decay_pow(n, p):
     assert ((got.double() - want).abs() <= want * (2 ** -22 + 2 ** -20 * p)).all()
     nan = torch.full((4,), float("nan"), device=DEV)
     assert hops.decay_pow(nan, p).isnan().all()
+
+
+def test_gated_unit_sigmoid():
+    """a sigmoid(slope a), every bfloat16 a from -60 to 30 and 150 slopes, against float64.  A float32 result off by n units of its last
+    place rounds to another bfloat16 than the exact one in n / 32768 of the cases at most (bfloat16 keeps 16 bits less): with the 4 units
+    that the sigmoid and two products may be off, 1.3e-4 of them.  No result is further off than the rounding to bfloat16 (2^-8), where the
+    sigmoid is below float32's normal numbers neither (slope a down to -88.2)."""
+    from chronos.ops import hybrid as hops
+
+    a = torch.arange(-32768, 32768, dtype=torch.int32, device=DEV).to(torch.int16).view(BF)
+    a = a[(a >= -60) & (a <= 30) & (a.abs() > 2 ** -10)]
+    a = a[:a.numel() // 8 * 8].view(1, -1)
+    gu, wrong, total = torch.cat([a, torch.zeros_like(a)], 1), 0, 0
+    for i in range(150):
+        slope = float(torch.tensor(0.5 + 0.97 * i / 149, dtype=torch.float32))
+        z = (a.float() * slope).double()
+        y, want = hops.glu(gu, 1e30, slope, 1.0, BF), (a.double() * torch.sigmoid(z))
+        wrong += int((y != want.to(BF)).sum())
+        total += a.numel()
+        assert float(((y.double() - want).abs() - want.abs() * 2 ** -7.9).max()) <= 0
+    assert total > 400_000 and wrong <= 1.3e-4 * total, (wrong, total)
+
