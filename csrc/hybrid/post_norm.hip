@@ -132,18 +132,20 @@ __global__ void __launch_bounds__(256) glu_vec_kernel(const uint16_t* __restrict
     st8(y + r * ldy + c, g);
 }
 
-// p <= 1/8: log2 sigmoid(z) = min(z, 0) log2 e - log2(1 + 2^(-|z| log2 e)) through the hardware's exp2 and log2, whose absolute error of 1e-7
-// times p is a small part of a last place of the result (rms 2.1e-8 off at p = 1/16, as with the library functions; at p = 1 9.0e-8 and
-// 7.7e-8); 16 bytes per lane.  8192 x 2048 values: 67 us with the library functions, which bound it, 20 so.
+// p <= 1/16: log sigmoid(z) = min(z, 0) - log(1 + e^-|z|) with the second part through the hardware's exp2 and log2, whose absolute error of
+// 1e-7 times p is a small part of a last place of the result; the outer exponential is the library's.  Largest error and root mean square in
+// units of the result's last place at p = 1/16, this and the library throughout: z in -100 .. -20 0.83, 0.300 both; -20 .. -6 1.14, 0.344 and
+// 1.08, 0.343; -0.1 .. 0.1 0.67, 0.292 and 0.64, 0.291 (at p = 1/8 0.90, 0.315 and 0.89, 0.308, hence the line).  Through exp2 to the end the
+// rounding of z p log2 e shows: 4.2, 1.33 at z < -40.  16 bytes per lane.  8192 x 2048 values: 67 us with the library, which bounds it, 20 so.
 __global__ void __launch_bounds__(256) decay_pow_vec_kernel(f32x4* __restrict__ z, int64_t n4, float p) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n4) return;
-    constexpr float kLog2e = 1.4426950408889634f;
+    constexpr float kLog2e = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
     f32x4 v = z[i];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const float t = __builtin_amdgcn_exp2f(-fabsf(v[e]) * kLog2e);
-        v[e] = __builtin_amdgcn_exp2f(p * (fminf(v[e], 0.f) * kLog2e - __builtin_amdgcn_logf(1.f + t)));
+        v[e] = expf(p * __builtin_fmaf(-kLn2, __builtin_amdgcn_logf(1.f + t), fminf(v[e], 0.f)));
     }
     z[i] = v;
 }
@@ -197,7 +199,7 @@ void launch_hy_glu(const void* gu, int64_t ldg, void* y, int64_t ldy, int64_t ro
 
 void launch_hy_decay_pow(float* z, int64_t n, float p, hipStream_t s) {
     if (n == 0) return;
-    if (p > 0.f && p <= 0.125f && n % 4 == 0 && hy::aligned16(z)) {
+    if (p > 0.f && p <= 0.0625f && n % 4 == 0 && hy::aligned16(z)) {
         hy::decay_pow_vec_kernel<<<(unsigned)((n / 4 + 255) / 256), 256, 0, s>>>(reinterpret_cast<f32x4*>(z), n / 4, p);
         return;
     }

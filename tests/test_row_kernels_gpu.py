@@ -180,3 +180,16 @@ def test_gated_unit_sigmoid():
         assert float(((y.double() - want).abs() - want.abs() * 2 ** -7.9).max()) <= 0
     assert total > 400_000 and wrong <= 1.3e-4 * total, (wrong, total)
 
+@pytest.mark.parametrize("tau", [16.0, 20.0, 64.0])
+@pytest.mark.parametrize("lo,hi", [(-100.0, -20.0), (-20.0, -4.0), (-4.0, 4.0), (4.0, 60.0)])
+def test_decay_pow_error(tau, lo, hi):
+    """Relative error of sigmoid(z)^(1 / tau) as a float32.  The logarithm and its product with 1 / tau round once each, 2^-24 of at most
+    100 / tau, which the exponential turns into a relative error; the exponential itself and the result: 2 units, 2^-23."""
+    from chronos.ops import hybrid as hops
+
+    z = (torch.rand(1 << 16, device=DEV, generator=_g(int(tau))) * (hi - lo) + lo).view(16, -1)
+    p = float(torch.tensor(1 / tau, dtype=torch.float32))
+    want = torch.exp(torch.nn.functional.logsigmoid(z.double()) * p)
+    rel = ((hops.decay_pow(z.clone(), p).double() - want) / want).abs().max()
+    size = max(-lo, 0.7) / tau
+    assert float(rel) <= 2 ** -23 + (0 if tau in (16.0, 64.0) and hi <= -4 else size * 2 ** -23)
