@@ -18,6 +18,10 @@
 // The delta rule's solve carries what its sums round off along: the state is 5.7e-8 off (token by token 5.8e-8; without,
 // 6.1e-8, and 9.3e-8 with the products added to the sum one by one).
 //
+// Where something is infinite or NaN, or overflows on the way, a weight of 0 above the diagonal times a later token's value would reach
+// back to earlier tokens, and a number without three finite terms would turn to NaN: a wave that has met such a thing in its read-outs
+// or its state takes the sequence's tokens again at the end, one by one, from the state before them.
+//
 // A workgroup is NW waves and serves 16 NW value columns of one (sequence, head); a wave keeps all D rows of its 16 columns
 // of S in accumulators, which are in the operand layout of the read-out's product as they stand.  A chunk's q, k, v rows
 // come by DMA into one of two LDS buffers while the chunk before is computed; 16-byte pieces are permuted within a row by a
@@ -46,6 +50,13 @@ constexpr int kCW = 4;    // waves per workgroup (NW above)
 __device__ __forceinline__ float exp_d(double x) {
     const float h = (float)x, e = expf(h);
     return e + e * (float)(x - h);
+}
+
+// acc, or NaN where one of x is infinite or NaN
+__device__ __forceinline__ float not_finite(const f32x4& x, float acc) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc = __builtin_fmaf(x[r], 0.f, acc);
+    return acc;
 }
 
 // Running sum over the wave's lanes (lane l: the sum of lanes 0 .. l): within rows of 16 lanes, then from row to row.
@@ -186,6 +197,7 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
     }
     double Lseg = 0.0;   // STATE: the sum of the segment's log decays, and the sign of their product
     float gseg = 1.f;
+    float odd = 0.f;     // NaN once something was not finite
     const uint16_t* const qp = a.proj + a.q_off + (int64_t)hk * D;
     const uint16_t* const kp = a.proj + a.k_off + (int64_t)hk * D;
     const uint16_t* const vp = a.proj + a.v_off + (int64_t)hd * a.Dv + c0;
@@ -397,6 +409,7 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
             for (int j = 0; j <= i; ++j) intra += psum[(p0 + j) * 16 + ln];
 #pragma unroll
             for (int u = 0; u < NW; ++u) inter += nq[u * kCH + lane];
+            odd = __builtin_fmaf(inter, 0.f, odd);
             fr = a.q_mul / (fmaxf(fabsf((intra + eL * inter) * a.q_mul), rd) + 1e-6f);
         }
         const float eC = gC * exp_d(LC);
@@ -504,6 +517,11 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
                         oq[i] = mfma_16x16x32(w3.h, v[p], mfma_16x16x32(w3.m, v[p], mfma_16x16x32(w3.l, v[p], oq[i])));
                     }
             }
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {   // (rows without tokens hold what was in LDS)
+                const float met = not_finite(oq[i], odd);
+                odd = i == 0 || i < nrow ? met : odd;
+            }
             const auto ord = __builtin_amdgcn_make_buffer_rsrc(a.o + ((int64_t)tb * a.H + hd) * a.Dv, (short)0, (int)(nt * orow), 0x00020000);
 #pragma unroll
             for (int i = 0; i < NI; ++i)
@@ -556,6 +574,81 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
         if (nt > 32) rest(std::integral_constant<int, 4>{});
         else rest(std::integral_constant<int, 2>{});
     }
+    bool again = false;
+    float nl[(D + 63) / 64] = {};   // mlstm: rows lane, lane + 64 .. of the normaliser
+    if constexpr (!STATE) {         // (a segment's state that is not finite shows in the next one's)
+#pragma unroll
+        for (int i = 0; i < 2 * KK; ++i) odd = not_finite(S[i], odd);
+        again = __builtin_amdgcn_ballot_w64(odd != odd) != 0;   // (wave-uniform)
+    }
+    if (again) {   // from the sequence's first token
+        dma_wait();   // what the chunks stored is there before the same places are written
+#pragma unroll
+        for (int i = 0; i < 2 * KK; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S[i][r] = fresh ? 0.f : take(a.segs == 1 ? Sp : seg0, i, r);
+        if constexpr (MLSTM) {
+#pragma unroll
+            for (int j = 0; j < (D + 63) / 64; ++j) nl[j] = a.n0[(int64_t)group * D + min(lane + 64 * j, D - 1)];
+        }
+        auto over_rows = [](float x) {   // lanes of the same column hold a quarter of the rows each
+            x += __shfl_xor(x, 16, 64);
+            return x + __shfl_xor(x, 32, 64);
+        };
+        for (int64_t t = s0; t < te; ++t) {
+            float d, w, rr = a.q_mul;
+            if constexpr (MLSTM) {
+                d = expf(a.la[t * a.H + hd]);
+                w = expf(a.lb[t * a.H + hd]);
+            } else {
+                d = a.dts != 0 ? a.decay[t * a.dts + hd] : fixed;
+                w = a.kscale != nullptr ? a.kscale[t * a.HK + hk] : 1.f;
+                if (!DELTA && a.vscale != nullptr) w *= a.vscale[t * a.H + hd];
+                if (a.qscale != nullptr) rr = a.qscale[t * a.HK + hk];
+            }
+            const uint16_t *const q = qp + t * a.ldp, *const k = kp + t * a.ldp;
+            if constexpr (MLSTM) {
+                float x = 0.f;
+#pragma unroll
+                for (int j = 0; j < (D + 63) / 64; ++j)
+                    if (lane + 64 * j < D) {
+                        nl[j] = d * nl[j] + bf2f(k[lane + 64 * j]) * w;
+                        x += nl[j] * bf2f(q[lane + 64 * j]);
+                    }
+                rr = a.q_mul / (fmaxf(fabsf(wave_sum(x) * a.q_mul), a.em[t * a.H + hd]) + 1e-6f);
+            }
+#pragma unroll
+            for (int i = 0; i < 2 * KK; ++i) S[i] *= d;
+            float u = live ? bf2f(vp[t * a.ldp + wv * 16 + ln]) : 0.f;
+            if constexpr (DELTA) {
+                float x = 0.f;
+#pragma unroll
+                for (int kk = 0; kk < KK; ++kk) {
+                    float kf[8];
+                    ld8(k + 32 * kk + 8 * g, kf);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) x += S[2 * kk + (e >> 2)][e & 3] * kf[e];
+                }
+                u = (u - over_rows(x) * w) * a.beta[t * a.H + hd];
+            }
+            u *= w;
+            float y = 0.f;
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) {
+                float kf[8], qf[8];
+                ld8(k + 32 * kk + 8 * g, kf);
+                ld8(q + 32 * kk + 8 * g, qf);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    f32x4& s = S[2 * kk + (e >> 2)];
+                    s[e & 3] += kf[e] * u;
+                    y += s[e & 3] * qf[e];
+                }
+            }
+            y = over_rows(y) * rr;
+            if (t >= t0 && g == 0 && live) a.o[(t * a.H + hd) * a.Dv + col] = y;
+        }
+    }
     if (!STATE && seg != a.segs - 1) return;
     float* const dst = STATE ? seg0 + cells * (seg + 1) * D * a.Dv : Sp;
     if (live) {
@@ -567,7 +660,13 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
     if (slab != 0) return;
     if constexpr (MLSTM) {
         float* const nd = STATE ? a.seg_n + (cells * seg + group) * D : a.n + srow * D;
-        if (ln == 0) {
+        if (again) {
+#pragma unroll
+            for (int j = 0; j < (D + 63) / 64; ++j) {
+                const int row = lane + 64 * j;
+                if (row < D && (row / 32) % NW == wv) nd[row] = nl[j];
+            }
+        } else if (ln == 0) {
 #pragma unroll
             for (int i = 0; i < 2 * NO; ++i)
 #pragma unroll

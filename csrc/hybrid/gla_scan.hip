@@ -5,7 +5,9 @@
 //     o_t = r_t ( (F_t q_t)^T S + sum_(s <= t) P[t, s] v_s ),   P[t, s] = (F_t q_t) . (w_s k_s / F_s)
 //     S  <- F_16 (S + sum_s (w_s k_s / F_s) v_s^T)
 //
-// A chunk in which some |F_t| leaves [2^-40, 2^40] (a decay of 0, say) is taken token by token instead, by the same waves.
+// A chunk in which some |F_t| leaves [2^-40, 2^40] (a decay of 0, say) is taken token by token instead, by the same waves; so is one with
+// infinities, NaN or numbers beyond 2^25 among k, w and v, or whose read-out is not finite: a weight of 0 above the diagonal times a
+// later token's infinite value would reach back, and an infinity has no terms.
 // Precision: as chunk_scan.hip, all but q, k, v is float32; a float32 operand of a matrix product enters as three bfloat16 terms
 // whose sum it is, two of them as the six leading of the nine products of terms.
 //
@@ -40,6 +42,11 @@ struct GlaScan {
 };
 
 constexpr int kGC = 16;   // tokens per chunk
+constexpr uint16_t kBig = 0x4c00;   // 2^25 as bfloat16: sums of products of three such and 2^40 stay finite
+
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+// the larger magnitudes of two and of a pair of bfloat16, as bits
+__device__ __forceinline__ u16x2 max_bits(u16x2 m, uint32_t pair) { return __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, pair & 0x7fff7fffu)); }
 
 // Waits for the wave's DMA pieces when `STORES` of its stores (all that it issued after them) may still be under way: memory
 // instructions of a wave complete in the order of issue, and a store takes as long as a chunk's arithmetic.
@@ -48,7 +55,7 @@ template <int STORES> __device__ __forceinline__ void dma_wait_before_stores() {
 __device__ __forceinline__ void received(float& a) { asm volatile("" : "+v"(a)); }
 
 // LDS (bytes): two buffers of q | k | decays (float) | v (64 columns), rows as they lie | F q and w k / F, three terms each | F_16 |
-// the factors w and r of two chunks | whether a chunk's F are in range, for three chunks
+// the factors w and r of two chunks | whether a chunk goes token by token, for three chunks, and whether the segment starts at the sequence's
 template <int D> struct GlaLds {
     static constexpr int Q = kGC * D * 2, DEC = 2 * Q, V = DEC + kGC * D * 4, BUF = V + kGC * 128;
     static constexpr int TQ = 2 * BUF, TK = TQ + 3 * Q, F = TK + 3 * Q, SC = F + D * 4, BAD = SC + 4 * kGC * 4, SIZE = BAD + 16;
@@ -72,7 +79,7 @@ __global__ void __launch_bounds__(256, 1) gla_scan_kernel(const GlaScan a) {
     const int s0 = a.q_start[b], t1 = a.q_start[b + 1];
     if (t1 <= s0) return;
     const int chunks = (t1 - s0 + kGC - 1) / kGC;
-    const int t0 = s0 + chunks * seg / a.segs * kGC, te = min(t1, s0 + chunks * (seg + 1) / a.segs * kGC);   // this segment's tokens
+    const int own = s0 + chunks * seg / a.segs * kGC, te = min(t1, s0 + chunks * (seg + 1) / a.segs * kGC);   // this segment's tokens
     const int64_t cells = (int64_t)a.B * a.H;
     const int c0 = slab * 64, col = c0 + wv * 16 + ln;
     const bool live = col < a.Dv;
@@ -105,6 +112,24 @@ __global__ void __launch_bounds__(256, 1) gla_scan_kernel(const GlaScan a) {
                 for (int r = 0; r < 4; ++r) S[i][r] = d[row_of(i, r)] * S[i][r] + (live ? at[(int64_t)row_of(i, r) * a.Dv] : 0.f);
         }
     }
+    int t0 = own;
+    if (tid < 4) bad[tid] = 0;
+    if constexpr (!STATE)
+        if (seg != 0) {   // products of decays cannot carry on a state that is not finite: then from the sequence's first token
+            f32x4 odd = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 2 * KK; ++i) odd += S[i] * 0.f;
+            __syncthreads();
+            if (!(odd[0] + odd[1] + odd[2] + odd[3] == 0.f)) bad[3] = 1;
+            __syncthreads();
+            if (bad[3] != 0) {
+                t0 = s0;
+#pragma unroll
+                for (int i = 0; i < 2 * KK; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) S[i][r] = live && !fresh ? seg0[(int64_t)row_of(i, r) * a.Dv] : 0.f;
+            }
+        }
     double dx[(D + 127) / 128], dy[(D + 127) / 128];   // STATE: the products of the segment's decays so far (rows as F q below)
 #pragma unroll
     for (int it = 0; it < (D + 127) / 128; ++it) dx[it] = dy[it] = 1.0;
@@ -155,7 +180,6 @@ __global__ void __launch_bounds__(256, 1) gla_scan_kernel(const GlaScan a) {
         sr = a.qscale != nullptr ? a.qscale[t * a.HK + hk] : a.q_mul;
     };
     const uint32_t orow = (uint32_t)a.H * a.Dv * 4, ocol = live ? (uint32_t)col * 4 : 0x80000000u;
-    if (tid < 3) bad[tid] = 0;
     if (t0 < te) {
         fetch(t0, 0);
         scalars(t0);
@@ -175,6 +199,7 @@ __global__ void __launch_bounds__(256, 1) gla_scan_kernel(const GlaScan a) {
         if (tid < kGC) {
             ws[tid] = tid < nt ? sw : 0.f;
             ws[kGC + tid] = sr;
+            if (!(fabsf(sw) < 0x1p25f)) bad[turn] = 1;
         }
         __syncthreads();   // the rows are there; nobody reads the other buffer or the last chunk's products any more
         if (nt < kGC) {    // tokens past the range decay nothing
@@ -233,12 +258,16 @@ __global__ void __launch_bounds__(256, 1) gla_scan_kernel(const GlaScan a) {
                 }
                 if (keys) {
                     float lo = 1.f, hi = 1.f;
+                    u16x2 big = {0, 0};   // (largest magnitudes as bits: a NaN is above all)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) big = max_bits(big, q[e]);
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
                         lo = fminf(lo, fminf(fabsf(x[e]), fabsf(y[e])));
                         hi = fmaxf(hi, fmaxf(fabsf(x[e]), fabsf(y[e])));
                     }
-                    if (!(lo >= 0x1p-40f) || !(hi <= 0x1p40f) || X != X || Y != Y) bad[turn] = 1;   // (fminf and fmaxf drop a NaN, X and Y keep it)
+                    // (fminf and fmaxf drop a NaN, X and Y keep it)
+                    if (!(lo >= 0x1p-40f) || !(hi <= 0x1p40f) || X != X || Y != Y || big[0] >= kBig || big[1] >= kBig) bad[turn] = 1;
                     auto inverse = [](float v) {   // to half a last place in the range that counts
                         const float r = __builtin_amdgcn_rcpf(v);
                         return __builtin_fmaf(__builtin_fmaf(-v, r, 1.f), r, r);
@@ -267,8 +296,46 @@ __global__ void __launch_bounds__(256, 1) gla_scan_kernel(const GlaScan a) {
         received(sw);
         received(sr);
         const f32x4 fr = *reinterpret_cast<const f32x4*>(ws + kGC + 4 * g);
-        const auto ord = __builtin_amdgcn_make_buffer_rsrc(a.o + ((int64_t)tb * a.H + hd) * a.Dv, (short)0, (int)(nt * orow), 0x00020000);
-        if (bad[turn] != 0) {   // token by token
+        const auto ord = __builtin_amdgcn_make_buffer_rsrc(a.o + ((int64_t)tb * a.H + hd) * a.Dv, (short)0, tb < own ? 0 : (int)(nt * orow), 0x00020000);
+        const bf16x4 v4 = lds_read_tr4(raw + M::V + (4 * g + (ln >> 2)) * 128 + wv * 32 + (ln & 3) * 8);   // tokens 4 g ..
+        const bf16x8 vv = join8(v4, v4);
+        const bf16x4 none = {};
+        const uint2 vw = __builtin_bit_cast(uint2, v4);
+        const u16x2 vbig = max_bits(max_bits(u16x2{0, 0}, vw.x), vw.y);
+        bool apart = __builtin_amdgcn_ballot_w64(bad[turn] != 0 || (!STATE && (vbig[0] >= kBig || vbig[1] >= kBig))) != 0;   // (wave-uniform)
+        f32x4 o = {0.f, 0.f, 0.f, 0.f};
+        if (!STATE && !apart) {
+            // ---- read-out: o = (F q)^T S, and P with rows s = 4 g + r and columns t = ln (as its product with v takes it)
+            const int sp = spread<CPR>(ln);
+            f32x4 small = {0.f, 0.f, 0.f, 0.f}, big = small, psmall = small, pbig = small;
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) {
+                const unsigned char* at = gs_smem + M::TQ + ln * (D * 2) + ((kk * 4 + g) ^ sp) * 16;
+                auto term = [&](int base) { return *reinterpret_cast<const bf16x8*>(at + base); };
+                const bf16x8 qh = term(0), qm = term(M::Q), ql = term(2 * M::Q), kh = term(3 * M::Q), km = term(4 * M::Q), kl = term(5 * M::Q);
+                psmall = mfma_16x16x32(kl, qh, psmall);
+                psmall = mfma_16x16x32(km, qm, psmall);
+                psmall = mfma_16x16x32(kh, ql, psmall);
+                psmall = mfma_16x16x32(km, qh, psmall);
+                psmall = mfma_16x16x32(kh, qm, psmall);
+                pbig = mfma_16x16x32(kh, qh, pbig);
+                small = mfma_16x16x32(ql, st[kk].h, small);
+                small = mfma_16x16x32(qm, st[kk].m, small);
+                small = mfma_16x16x32(qh, st[kk].l, small);
+                small = mfma_16x16x32(qm, st[kk].h, small);
+                small = mfma_16x16x32(qh, st[kk].m, small);
+                big = mfma_16x16x32(qh, st[kk].h, big);
+            }
+            f32x4 P = psmall + pbig;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) P[r] = 4 * g + r <= ln ? P[r] : 0.f;
+            const Terms4 pt = split3(P);
+            small = mfma_16x16x32(join8(pt.l, none), vv, small);
+            big = mfma_16x16x32(join8(pt.h, pt.m), vv, big);
+            o = small + big;
+            apart = __builtin_amdgcn_ballot_w64(!(__builtin_fmaf(o[0], 0.f, o[1] * 0.f) + __builtin_fmaf(o[2], 0.f, o[3] * 0.f) == 0.f)) != 0;
+        }
+        if (apart) {   // token by token
             const uint16_t* const vs = reinterpret_cast<const uint16_t*>(raw + M::V) + wv * 16 + ln;
             for (int t = 0; t < nt; ++t) {
                 const float u = bf2f(vs[t * 64]) * ws[t];
@@ -288,40 +355,10 @@ __global__ void __launch_bounds__(256, 1) gla_scan_kernel(const GlaScan a) {
             }
             continue;
         }
-        const bf16x4 v4 = lds_read_tr4(raw + M::V + (4 * g + (ln >> 2)) * 128 + wv * 32 + (ln & 3) * 8);   // tokens 4 g ..
-        const bf16x8 vv = join8(v4, v4);
-        const bf16x4 none = {};
         if constexpr (!STATE) {
-            // ---- read-out: o = (F q)^T S, and P with rows s = 4 g + r and columns t = ln (as its product with v takes it)
-            const int sp = spread<CPR>(ln);
-            f32x4 small = {0.f, 0.f, 0.f, 0.f}, big = small, psmall = small, pbig = small;
-    #pragma unroll
-            for (int kk = 0; kk < KK; ++kk) {
-                const unsigned char* at = gs_smem + M::TQ + ln * (D * 2) + ((kk * 4 + g) ^ sp) * 16;
-                auto term = [&](int base) { return *reinterpret_cast<const bf16x8*>(at + base); };
-                const bf16x8 qh = term(0), qm = term(M::Q), ql = term(2 * M::Q), kh = term(3 * M::Q), km = term(4 * M::Q), kl = term(5 * M::Q);
-                psmall = mfma_16x16x32(kl, qh, psmall);
-                psmall = mfma_16x16x32(km, qm, psmall);
-                psmall = mfma_16x16x32(kh, ql, psmall);
-                psmall = mfma_16x16x32(km, qh, psmall);
-                psmall = mfma_16x16x32(kh, qm, psmall);
-                pbig = mfma_16x16x32(kh, qh, pbig);
-                small = mfma_16x16x32(ql, st[kk].h, small);
-                small = mfma_16x16x32(qm, st[kk].m, small);
-                small = mfma_16x16x32(qh, st[kk].l, small);
-                small = mfma_16x16x32(qm, st[kk].h, small);
-                small = mfma_16x16x32(qh, st[kk].m, small);
-                big = mfma_16x16x32(qh, st[kk].h, big);
-            }
-            f32x4 P = psmall + pbig;
-    #pragma unroll
-            for (int r = 0; r < 4; ++r) P[r] = 4 * g + r <= ln ? P[r] : 0.f;
-            const Terms4 pt = split3(P);
-            small = mfma_16x16x32(join8(pt.l, none), vv, small);
-            big = mfma_16x16x32(join8(pt.h, pt.m), vv, big);
-    #pragma unroll
+#pragma unroll
             for (int r = 0; r < 4; ++r)   // (past the last token and past Dv the descriptor's range drops the store)
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((small[r] + big[r]) * fr[r]), ord, ocol + (4 * g + r) * orow, 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[r] * fr[r]), ord, ocol + (4 * g + r) * orow, 0, 0);
         }
         // ---- the state after the chunk
         const int r4 = 4 * g + (ln >> 2), sp4 = spread<CPR>(r4);
