@@ -22,6 +22,8 @@ void launch_hy_act(void*, int64_t, int, bool, hipStream_t);
 void launch_hy_mlstm_scan(const void*, int, const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*,
                           float*, float*, float*, int, int, int, int, int, float, int, int, bool, hipStream_t);
 int hy_chunk_segments(int, int, int, int, int, int);
+bool hy_chunk_scan_pays(int, int, int, int, int, int, int);
+bool hy_gla_scan_pays(int, int, int);
 int64_t hy_chunk_segment_floats(int, int, int, int, int);
 void launch_hy_mlstm_out(const float*, const void*, int, int, const float*, void*, int, int, int, float, bool,
                          hipStream_t);
@@ -1095,6 +1097,13 @@ TORCH_LIBRARY_FRAGMENT(chronos, m) {
     m.def("hy_latent_expanded_ok(int D, int R, int Dv) -> bool", [](int64_t D, int64_t R, int64_t Dv) {
         return std::max({D, R, Dv}) <= 1024 && chronos::hy_latent_expanded_ok((int)D, (int)R, (int)Dv) && chronos::hy_latent_use_mfma(false, 16, 16);
     });
+    // forms: 0 one decay per head and token, 1 mlstm, 2 delta rule, 3 one decay per state row
+    m.def("hy_chunk_scan_pays(int form, int T, int B, int H, int D, int Dv, int longest) -> bool",
+          [](int64_t form, int64_t T, int64_t B, int64_t H, int64_t D, int64_t Dv, int64_t longest) {
+              need(form >= 0 && form <= 3 && T >= longest && longest >= 1 && B >= 1, "chunk_scan_pays: a form, 1 <= longest <= T");
+              return form == 3 ? chronos::hy_gla_scan_pays((int)T, (int)B, (int)longest)
+                               : chronos::hy_chunk_scan_pays((int)form, (int)T, (int)B, (int)H, (int)D, (int)Dv, (int)longest);
+          });
     m.def("hy_head_matmul(Tensor a, Tensor w, Tensor(a!) out, Tensor? gate_src, int g_off) -> ()");
     m.def("hy_dyn_tanh(Tensor x, Tensor wba, bool out_f32) -> Tensor");
     m.def("hy_gated_join(Tensor y, Tensor(a!) x, Tensor? gate_src, int g_off, Tensor? gate_b, float mult, Tensor? wba, "

@@ -38,6 +38,7 @@
 #include "chunk_common.h"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace chronos {
@@ -77,8 +78,6 @@ __device__ __forceinline__ double lanes_running_sum(double x) {
     x += from(x, integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});    // lane 31 to rows 2 and 3
     return x;
 }
-
-enum { kScanPlain = 0, kScanMlstm = 1, kScanDelta = 2 };
 
 // What the forms read per token: plain: decay (one per token and head, or dts = 0: per head), qscale, kscale, vscale
 // (any of the three may be absent); delta: the same without vscale, and beta; mlstm: the log decays, log write factors and
@@ -733,15 +732,39 @@ __global__ void __launch_bounds__(256) mlstm_gates_kernel(const float* __restric
 
 }  // namespace hy
 
+int hy_chunk_segments(int B, int H, int D, int Dv, int longest, int least);
+
+// Whether a launch takes less time in chunks than token by token.  A chunk costs the same whether it is full or not: a range of one token
+// costs a workgroup 6 to 10 us per slab, token by token little more than its state's bytes, so that a short prompt beside many decode
+// rows is faster there: retention, 8 heads of 128 x 128, us in chunks / token by token: 16 tokens beside 256 decode rows 118 / 50, 117 beside
+// 256 115 / 95, 117 beside 64 35 / 64, 2048 beside 256 176 / 957; delta rule, 32 heads: 40 beside 64 142 / 65, 117 beside 256 550 / 296, 2048
+// beside 256 622 / 1214.  Alone, 32 sequences of n tokens: 15.5 / 10.7 at n = 4, 15.4 / 17.1 at 16, 33 / 71 at 117.  The times are
+// modelled: the chain of the longest range (in segments side by side, which walk it 1.6 times) or the chunks of all over 256 CUs, the chain
+// of tokens or all tokens, and the states' megabytes; fitted per form on 2639 launches of 14 shapes (rms 0.13 .. 0.15 of a time;
+// profiles/recurrence_forms.json).  Chunked where that is 0.8 of the other at most: 2 of the 2639 are then slower than token by token by more
+// than 3% (by 6), always chunked 445 (by up to 140); 2% on average off the better of the two.
+bool hy_chunk_scan_pays(int mode, int T, int B, int H, int D, int Dv, int longest) {
+    struct Cost {
+        double c0, chain, work, t0, step, steps, mb;
+    };
+    constexpr Cost costs[3] = {{4.7, 5.7, 6.5, 2.8, 0.465, 0.277, 0.175}, {10.3, 7.1, 7.7, 9.1, 1.0, 0.54, 0.295}, {6.5, 11.4, 9.8, 4.3, 0.475, 0.52, 0.18}};
+    const Cost& c = costs[mode];
+    const int segs = mode == hy::kScanDelta ? 1 : hy_chunk_segments(B, H, D, Dv, longest, 256), most = (longest + 63) / 64;
+    const double slabs = (double)H * ((Dv + 63) / 64), size = std::sqrt(D / 128.0);
+    const double chunks = most + std::max(B - 1.0, (T - longest) / 64.0 + (B - 1) / 2.0);
+    const double chunked = c.c0 + std::max(c.chain * most / segs * (segs > 1 ? 1.6 : 1.0), c.work * slabs * chunks / 256) * size;
+    const double token = c.t0 + std::max(c.step * longest * size, c.steps * T * slabs * D / 128 / 256) + c.mb * B * H * D * Dv * 8e-6;
+    return chunked <= 0.8 * token;
+}
+
 // When the chunked form serves a launch: bfloat16 rows of q, k and v on 16-byte boundaries, a state of 32, 64, 128 or 256
-// rows, and a sequence with at least 16 new tokens (longest: the most that any sequence brings).  A chunk costs the same
-// whether it is full or not, the token-by-token kernels cost per token: 32 sequences of n tokens take (token by token /
-// chunked, us) 10.7 / 15.5 at n = 4, 12.5 / 15.6 at 8, 17.1 / 15.4 at 16, 71 / 33 at 117 (8 heads of 128 x 128, fixed decays),
-// 50 / 68, 61 / 67, 87 / 56, 443 / 105 (mlstm, 4 heads of 256 x 512), and with the delta rule (16 heads of
-// 128 x 128) 35 / 38 at 16, 57 / 44 at 32, 179 / 111 at 117.  The delta rule's tiles leave no room for D = 256.
-bool hy_chunk_scan_ok(const void* proj, int ldp, int q_off, int k_off, int v_off, int D, int Dv, int longest, bool delta) {
+// rows, a sequence with at least 16 new tokens, with the delta rule 32 (longest: the most that any sequence brings), and a launch that
+// gains (above).  The delta rule's tiles leave no room for D = 256.
+bool hy_chunk_scan_ok(const void* proj, int ldp, int q_off, int k_off, int v_off, int T, int B, int H, int D, int Dv, int longest, int mode) {
+    const bool delta = mode == hy::kScanDelta;
     return longest >= (delta ? 32 : 16) && (D == 32 || D == 64 || D == 128 || (D == 256 && !delta)) && Dv % 8 == 0 && ((uintptr_t)proj & 15) == 0 &&
-           ((ldp | q_off | k_off | v_off) & 7) == 0 && ldp < 1 << 23;   // (64 rows of o, no wider than proj's, within 2^31 bytes)
+           ((ldp | q_off | k_off | v_off) & 7) == 0 && ldp < 1 << 23 &&   // (64 rows of o, no wider than proj's, within 2^31 bytes)
+           hy_chunk_scan_pays(mode, T, B, H, D, Dv, longest);
 }
 
 template <int D, int MODE, bool STATE>

@@ -395,11 +395,17 @@ __global__ void __launch_bounds__(256, 1) gla_scan_kernel(const GlaScan a) {
 
 }  // namespace hy
 
+// Whether a launch takes less time in chunks than token by token: ranges of 8 tokens on average, or one of 24.  A chunk costs the same
+// whether it is full or not: 21 sequences of n tokens, 4 heads of 128 x 256, token by token / here, us: 9.2 / 9.8 at n = 2, 10.9 / 9.8 at 4, 14.0 / 9.8
+// at 8, 21 / 9.9 at 16, 109 / 39 at 117; one of n beside 64 ranges of one token: 19.7 / 25.8 at 4, 25.2 / 26.0 at 16, beside 256 63.8 / 74.3 at 16,
+// 68.6 / 73.6 at 24.  Of 905 launches of 4 shapes (profiles/recurrence_forms.json) 2 lose by more than 3% (the worst by 8); from 4 tokens for the longest
+// on 66 did (by up to 45).
+bool hy_gla_scan_pays(int T, int B, int longest) { return longest >= 24 || (longest >= 4 && T >= 8 * (int64_t)B); }
+
 // When this form serves a launch: bfloat16 rows of q, k, v and rows of decays on 16-byte boundaries, a state of 32, 64, 128 or 256
-// rows, and a sequence of at least 4 new tokens (longest: the most that any sequence brings): 21 sequences of n tokens, 4 heads of
-// 128 x 256, token by token / here, us: 9.2 / 9.8 at n = 2, 10.9 / 9.8 at 4, 14.0 / 9.8 at 8, 21 / 9.9 at 16, 109 / 39 at 117.
-bool hy_gla_scan_ok(const void* proj, const void* decay, int ldp, int q_off, int k_off, int v_off, int D, int Dv, int longest) {
-    return longest >= 4 && (D == 32 || D == 64 || D == 128 || D == 256) && Dv % 8 == 0 && hy::aligned16(proj, decay) &&
+// rows, and a launch that gains (longest: the most new tokens that any sequence brings).
+bool hy_gla_scan_ok(const void* proj, const void* decay, int ldp, int q_off, int k_off, int v_off, int T, int B, int D, int Dv, int longest) {
+    return hy_gla_scan_pays(T, B, longest) && (D == 32 || D == 64 || D == 128 || D == 256) && Dv % 8 == 0 && hy::aligned16(proj, decay) &&
            ((ldp | q_off | k_off | v_off) & 7) == 0 && ldp < 1 << 23;
 }
 

@@ -122,6 +122,9 @@ __device__ __forceinline__ uint32_t round_pair(float& a, float& b) {
     return u;
 }
 
+// forms of the recurrences with one decay per head and token (chunk_scan.hip)
+enum { kScanPlain = 0, kScanMlstm = 1, kScanDelta = 2 };
+
 constexpr int kActRelu2 = 0, kActGelu = 1;
 __device__ __forceinline__ float act_apply(float z, int kind) {
     if (kind == kActRelu2) {

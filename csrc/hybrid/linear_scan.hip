@@ -415,12 +415,12 @@ __global__ void __launch_bounds__(256) linear_scan_kernel(
 
 }  // namespace hy
 
-bool hy_chunk_scan_ok(const void*, int, int, int, int, int, int, int, bool);
+bool hy_chunk_scan_ok(const void*, int, int, int, int, int, int, int, int, int, int, int);
 void launch_hy_chunk_scan(const uint16_t*, int, int, int, int, const float*, const float*, float, const float*, int,
                           const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*, int, int, int, int, int, const float*,
                           int, float*, hipStream_t);
 
-bool hy_gla_scan_ok(const void*, const void*, int, int, int, int, int, int, int);
+bool hy_gla_scan_ok(const void*, const void*, int, int, int, int, int, int, int, int, int);
 void launch_hy_gla_scan(const uint16_t*, int, int, int, int, const float*, const float*, float, const float*, const int32_t*,
                         const int32_t*, const int32_t*, float*, float*, int, int, int, int, int, const float*, int, float*, hipStream_t);
 
@@ -526,12 +526,12 @@ bool launch_hy_linear_scan(const void* proj, int ldp, int q_off, int k_off, int 
                              q_start, pos0, slots, S, o, B, HK, H, D, Dv, vscale, s);
         return true;
     }
-    if (chd && !delta && !f32 && hy_gla_scan_ok(proj, decay, ldp, q_off, k_off, v_off, D, Dv, longest)) {
+    if (chd && !delta && !f32 && hy_gla_scan_ok(proj, decay, ldp, q_off, k_off, v_off, T, B, D, Dv, longest)) {
         launch_hy_gla_scan((const uint16_t*)proj, ldp, q_off, k_off, v_off, qscale, kscale, q_mul, decay, q_start, pos0, slots, S, o,
                            B, HK, H, D, Dv, vscale, segs, seg, s);
         return true;
     }
-    if (!chd && !f32 && hy_chunk_scan_ok(proj, ldp, q_off, k_off, v_off, D, Dv, longest, delta)) {
+    if (!chd && !f32 && hy_chunk_scan_ok(proj, ldp, q_off, k_off, v_off, T, B, H, D, Dv, longest, delta ? hy::kScanDelta : hy::kScanPlain)) {
         launch_hy_chunk_scan((const uint16_t*)proj, ldp, q_off, k_off, v_off, qscale, kscale, q_mul, decay, fixed ? 0 : H, beta,
                              q_start, pos0, slots, S, o, B, HK, H, D, Dv, vscale, segs, seg, s);
         return true;

@@ -442,7 +442,7 @@ static void mlstm_scan_t(const T* proj, int ldp, const float* gate_pre, const in
 #undef HY_SCAN
 }
 
-bool hy_chunk_scan_ok(const void*, int, int, int, int, int, int, int, bool);
+bool hy_chunk_scan_ok(const void*, int, int, int, int, int, int, int, int, int, int, int);
 void launch_hy_chunk_mlstm(const uint16_t*, int, const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*,
                            float*, float*, float*, int, int, int, int, int, float, int, hipStream_t);
 
@@ -452,7 +452,7 @@ void launch_hy_mlstm_scan(const void* proj, int ldp, const float* gate_pre, cons
                           const int32_t* slots, float* S, float* n, float* m, float* scratch, float* o, int T, int B, int H, int D,
                           int Dv, float cap, int longest, int segs, bool f32, hipStream_t s) {
     if (B == 0) return;
-    if (!f32 && hy_chunk_scan_ok(proj, ldp, 0, H * D, 2 * H * D, D, Dv, longest, false)) {
+    if (!f32 && hy_chunk_scan_ok(proj, ldp, 0, H * D, 2 * H * D, T, B, H, D, Dv, longest, hy::kScanMlstm)) {
         launch_hy_chunk_mlstm((const uint16_t*)proj, ldp, gate_pre, q_start, pos0, slots, S, n, m, scratch, o, T, B, H, D, Dv, cap, segs, s);
         return;
     }
