@@ -56,16 +56,17 @@ __global__ void __launch_bounds__(64 * NW) window_attention_mfma_kernel(
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     constexpr int KT = WKT, RPB = 16 * NW / KS;
     const int R = H / G;
-    // blockIdx.x: sequence and key/value head; blockIdx.y: row block and split, later blocks (which see more keys) first.  Where two
-    // workgroups per CU hold the whole launch its second half runs the other way, so that a CU gets a long walk and a short one.
+    // blockIdx.x: sequence and key/value head; blockIdx.y: row block and split, a sequence's later blocks (which see more keys) first, so that
+    // a decode row, its sequence's last, starts with the prompts' last ones.  Where two workgroups per CU hold the whole launch the
+    // second half of a sequence's runs the other way, so that a CU gets a long walk and a short one.
     const int b = blockIdx.x / G, kvh = blockIdx.x % G;
     const int t0 = q_start[b], t1 = q_start[b + 1];
     const int rows_total = (t1 - t0) * R;
-    const int ny = gridDim.y, y0 = blockIdx.y, half = ny / 2;
-    const int y = gridDim.x * ny <= 512 && y0 >= ny - half ? y0 - (ny - half) : ny - 1 - y0;
+    const int ny = (rows_total + RPB - 1) / RPB * nsplit, y0 = blockIdx.y, half = ny / 2;
+    if (y0 >= ny) return;
+    const int y = gridDim.x * gridDim.y <= 512 && y0 >= ny - half ? y0 - (ny - half) : ny - 1 - y0;
     const int split = y % nsplit;   // key tiles are dealt round-robin to the nsplit workgroups of a row block
     const int rb0 = y / nsplit * RPB;
-    if (rb0 >= rows_total) return;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, g4 = lane >> 4, qi = lane & 15;
     const int nct = Dv / 16;
     constexpr int KCH = NS * 4 + 1, krs = KCH * 16;                     // key row in LDS: 16-byte chunks, bytes

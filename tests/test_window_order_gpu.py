@@ -32,3 +32,32 @@ def test_order(B, T, window, keep):
         s = torch.matmul(q.transpose(0, 1), k.permute(1, 2, 0)) * D ** -0.5
         want = torch.matmul(torch.softmax(s.masked_fill_(hide, float("-inf")), -1), v.transpose(0, 1)).transpose(0, 1)
         assert float((o[b].float() - want).norm() / want.norm()) < 2 ** -8, b
+
+
+@pytest.mark.parametrize("lens,past", [([900, 1, 65, 0, 1, 300], [0, 700, 0, 5, 40, 100]), ([130] + [1] * 9, [16] + [200] * 9),
+                                       ([33, 700, 2] * 8, [0, 64, 300] * 8), ([17, 1, 1], [480, 1, 333])])
+@pytest.mark.parametrize("window,keep", [(0, 0), (100, 3)])
+def test_order_of_unequal_sequences(lens, past, window, keep):
+    """Prompts beside decode rows: every sequence's blocks are its own number, in its own order, with and without splits of the keys."""
+    from chronos.ops import hybrid as hops
+
+    H, G, D, BS = 8, 2, 64, 16
+    B, T, g = len(lens), sum(lens), torch.Generator(device=DEV).manual_seed(sum(lens))
+    qkv, per = torch.randn(T, (H + 2 * G) * D, device=DEV, generator=g).bfloat16(), max((n + c + BS - 1) // BS for n, c in zip(lens, past))
+    kc, vc = (torch.randn(B * per + 1, BS, G, D, device=DEV, generator=g).bfloat16() for _ in range(2))
+    bt = (1 + torch.randperm(B * per, device=DEV, generator=g)).int().view(B, per)
+    qs = [sum(lens[:b]) for b in range(B + 1)]
+    pos = torch.cat([torch.arange(c, c + n) for n, c in zip(lens, past)]).int().to(DEV)
+    o = hops.window_attention(qkv, kc, vc, bt, torch.tensor(qs).int().to(DEV), pos, None, None, D ** -0.5, window, keep, H, torch.bfloat16, max(lens)).view(T, H, D)
+    for b, (n, c) in enumerate(zip(lens, past)):
+        if n == 0:
+            continue
+        k, v = (x[bt[b].long()].reshape(-1, G, D)[:c + n].float().repeat_interleave(H // G, 1) for x in (kc, vc))
+        q = qkv[qs[b]:qs[b + 1], :H * D].float().view(n, H, D)
+        i, p = torch.arange(c + n, device=DEV)[None], torch.arange(c, c + n, device=DEV)[:, None]
+        hide = i > p
+        if window:
+            hide = hide | ((i <= p - window) & (i >= keep))
+        s = torch.matmul(q.transpose(0, 1), k.permute(1, 2, 0).contiguous()) * D ** -0.5
+        want = torch.matmul(torch.softmax(s.masked_fill_(hide, float("-inf")), -1), v.transpose(0, 1).contiguous()).transpose(0, 1)
+        assert float((o[qs[b]:qs[b + 1]].float() - want).norm() / want.norm()) < 2 ** -8, b
