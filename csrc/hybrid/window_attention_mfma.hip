@@ -440,12 +440,14 @@ bool hy_window_mfma_ok(int ldq, int D, int Dv) { return !(D % 8 || Dv % 16 || D 
 // Splits of a row block's key tiles over workgroups (merged by a combine kernel) for launches that would leave most
 // of the chip idle — decode rows, a lone short portion: enough workgroups to cover the CUs twice (four times for few
 // rows with unit keys, whose workgroups need half the LDS), at least 2 key tiles per split, at most 16.  Prompt portions (more than 64
-// rows) write and read far more partials than decode rows: 3 tiles, and 8 from half a workgroup per CU on (us, 8 heads, 2 of keys, splits of
-// 2 tiles / none: 1 x 700 tokens, 44 workgroups 22 / 30; 1 x 300, 20 workgroups 15.5 / 17.6; 8 x 117, 64 workgroups of 3 tiles 16.4 / 11.1;
-// 21 x 117, 168 workgroups 26 / 12; 8 x 300, 160 workgroups 32 / 19).  The tile count
+// rows) write and read far more partials than decode rows: only where a walk's tiles weigh more than all rows' partials, 1000 (token, head)
+// rows a tile, all of the step's tokens counted and not its longest portion's, which a mixed step's decode rows do not have.  us, split /
+// not: 8 heads, 2 of keys, 8 x 300 tokens (19200 rows, 5 tiles) 32 / 19, 21 x 117 (3) 26 / 12, 1 x 700 (5600, 11) 22 / 30; 300 tokens beside 8 decode
+// rows, window 512 (2464, 14) 23 / 35; 32 heads, 40 beside 8 (1536, 10) 20 / 35.  Of 985 launches where it decides, 1% on average off the better
+// of the two (always 6.5%, by the longest portion 3.8%).  The tile count
 // follows from sizes the host knows (the window, or the block table's width when there is none).  1 for float32 and
 // sizes the matrix-core kernel does not serve.
-int hy_window_nsplit(bool f32, int ldq, int B, int max_q, int H, int G, int D, int Dv, int window, int keep, int chunk,
+int hy_window_nsplit(bool f32, int ldq, int T, int B, int max_q, int H, int G, int D, int Dv, int window, int keep, int chunk,
                      int max_ctx, int pool, bool unit) {
     if (f32 || !hy_window_mfma_ok(ldq, D, Dv) || B <= 0) return 1;
     const int rows = max_q * (H / G);
@@ -457,7 +459,7 @@ int hy_window_nsplit(bool f32, int ldq, int B, int max_q, int H, int G, int D, i
     const int tiles = span / hy::WKT + 1 + (window > 0 ? (std::min(keep, max_ctx) + hy::WKT - 1) / hy::WKT : 0) +
                       (window > 0 && pool > 0 ? (max_ctx / pool + hy::WKT - 1) / hy::WKT : 0);
     int want = (enough + wgs - 1) / wgs;
-    want = std::min(want, std::min(16, tiles / (rows <= 64 ? 2 : wgs < 128 ? 3 : 8)));
+    want = std::min(want, std::min(16, rows <= 64 || (int64_t)T * H <= 1000LL * tiles ? tiles / 2 : 1));
     return want < 1 ? 1 : want;
 }
 
