@@ -62,11 +62,10 @@ __global__ void __launch_bounds__(64 * NW) window_attention_mfma_kernel(
     const int b = blockIdx.x / G, kvh = blockIdx.x % G;
     const int t0 = q_start[b], t1 = q_start[b + 1];
     const int rows_total = (t1 - t0) * R;
-    const int ny = (rows_total + RPB - 1) / RPB * nsplit, y0 = blockIdx.y, half = ny / 2;
-    if (y0 >= ny) return;
-    const int y = gridDim.x * gridDim.y <= 512 && y0 >= ny - half ? y0 - (ny - half) : ny - 1 - y0;
-    const int split = y % nsplit;   // key tiles are dealt round-robin to the nsplit workgroups of a row block
-    const int rb0 = y / nsplit * RPB;
+    const int nb = (rows_total + RPB - 1) / RPB, y0 = blockIdx.y / nsplit, half = nb / 2;
+    if (y0 >= nb) return;
+    const int split = blockIdx.y % nsplit;   // key tiles are dealt round-robin to the nsplit workgroups of a row block: the first have most
+    const int rb0 = (gridDim.x * gridDim.y <= 512 && y0 >= nb - half ? y0 - (nb - half) : nb - 1 - y0) * RPB;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, g4 = lane >> 4, qi = lane & 15;
     const int nct = Dv / 16;
     constexpr int KCH = NS * 4 + 1, krs = KCH * 16;                     // key row in LDS: 16-byte chunks, bytes
