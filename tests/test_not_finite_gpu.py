@@ -26,6 +26,8 @@ def _run(form, H, HK, D, Dv, lens, what, at, value, starts=(0, 3), seed=0):
     from chronos.ops import hybrid as hops
 
     T, g = sum(lens), torch.Generator().manual_seed(seed + D + Dv)
+    hops.load()
+    assert torch.ops.chronos.hy_chunk_scan_pays({"mlstm": 1, "delta": 2, "rows": 3}.get(form, 0), T, len(lens), H, D, Dv, max(lens))   # in chunks
     rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
     rand = lambda *s: torch.rand(*s, generator=g)  # noqa: E731
     i32 = lambda v: torch.tensor(v, dtype=torch.int32)  # noqa: E731

@@ -103,3 +103,62 @@ def test_longer_ranges(form, max_q, count):
 
     for got, want in zip(run(DEV), run("cpu")):   # both sides round
         assert float((got.cpu() - want).norm() / want.norm()) < 4e-6
+
+
+@pytest.mark.parametrize("form", ["fixed", "token", "rows", "delta", "delta_rows", "mlstm"])
+@pytest.mark.parametrize("HK,H,D,Dv", [(2, 4, 32, 100), (4, 4, 256, 128), (2, 4, 64, 264), (4, 4, 128, 132), (2, 4, 256, 512)])
+def test_many_rows(form, HK, H, D, Dv):
+    """Launches with a workgroup for every CU: 32 and 64 lanes to a row of the state (columns in 128s and 256s), two of 66 sequences empty.
+    Every sequence is one step, all of them at once in float64; tolerance as above."""
+    from chronos.ops import hybrid as hops
+
+    if form == "mlstm":
+        HK = H
+    B, g = 66, torch.Generator(device=DEV).manual_seed(D + Dv)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
+    rand = lambda *s: torch.rand(*s, device=DEV, generator=g)  # noqa: E731
+    count = torch.ones(B, dtype=torch.int64)
+    count[[5, 60]] = 0
+    T, rep = int(count.sum()), H // HK
+    assert T * H * ((Dv + 255) // 256) >= 256
+    qs = torch.cat([torch.zeros(1, dtype=torch.int64), count.cumsum(0)]).int().to(DEV)
+    start, slots = torch.arange(B, device=DEV).int() % 3, torch.randperm(B + 2, device=DEV, generator=g)[:B].int()
+    live = count.bool().to(DEV)
+    sl, keep = slots[live].long(), (start[live] > 0).double()[:, None]
+    proj, S = rnd(T, 2 * HK * D + H * Dv + 12).bfloat16(), rnd(B + 2, H, D, Dv)
+    S0, p = S.clone(), proj.double()
+    q, k = (p[:, i * HK * D:(i + 1) * HK * D].view(T, HK, D) for i in (0, 1))
+    v = p[:, 2 * HK * D:2 * HK * D + H * Dv].view(T, H, Dv)
+    s = S0[sl].double() * keep[..., None, None]
+    if form == "mlstm":
+        n, m, gp = rnd(B + 2, H, D), rnd(B + 2, H), rnd(T, 2 * H)
+        n0, m0 = n[sl].double() * keep[..., None], m[sl].double() * keep
+        o = hops.mlstm_scan(proj, gp, qs, start, slots, S, n, m, H, D, Dv, 9.0, 1)
+        ig, fg = 9 * torch.tanh(gp[:, :H].double() / 9), torch.nn.functional.logsigmoid(9 * torch.tanh(gp[:, H:].double() / 9))
+        mn = torch.maximum(fg + m0, ig)
+        a, w = torch.exp(fg + m0 - mn), torch.exp(ig - mn)
+        s = a[..., None, None] * s + (w[..., None] * k)[..., None] * v[:, :, None]
+        nn = a[..., None] * n0 + w[..., None] * k
+        den = torch.maximum((nn * q * D ** -0.5).sum(-1).abs(), torch.exp(-mn)) + 1e-6
+        # (before the division: a denominator that nearly cancels magnifies its own rounding)
+        got, want = o.double() * den[..., None], (q[:, :, None] @ s)[:, :, 0] * D ** -0.5
+        assert float((n[sl].double() - nn).norm() / nn.norm()) < 2e-6 and float((m[sl].double() - mn).norm() / mn.norm()) < 2e-6
+    else:
+        delta = form.startswith("delta")
+        dec = rand(H) if form == "fixed" else rand(T, H, D) if form.endswith("rows") else rand(T, H)
+        qsc, ksc = (rand(T, HK), rand(T, HK)) if form != "fixed" else (None, None)
+        beta, vs = rand(T, H) if delta else None, rand(T, H) if form == "token" else None
+        o = hops.linear_scan(proj, 0, HK * D, 2 * HK * D, qsc, ksc, 0.3, dec, beta, qs, start, slots, S, HK, H, D, Dv, vs, 1)
+        q = (q * (qsc.double()[..., None] if qsc is not None else 0.3)).repeat_interleave(rep, 1)
+        k = (k * (ksc.double()[..., None] if ksc is not None else 1.0)).repeat_interleave(rep, 1)
+        s = (dec.double().expand(T, H) if dec.dim() < 3 else dec.double()).reshape(T, H, -1, 1) * s
+        u = v * (vs.double()[..., None] if vs is not None else 1.0)
+        if delta:
+            u = beta.double()[..., None] * (u - (k[:, :, None] @ s)[:, :, 0])
+        s = s + k[..., None] * u[:, :, None]
+        got, want = o.double(), (q[:, :, None] @ s)[:, :, 0]
+    assert float((got - want).norm() / want.norm()) < (1e-5 if form == "mlstm" else 2e-6)
+    assert float((S[sl].double() - s).norm() / s.norm()) < 2e-6
+    rest = torch.ones(B + 2, dtype=torch.bool, device=DEV)
+    rest[sl] = False
+    assert torch.equal(S[rest], S0[rest])
