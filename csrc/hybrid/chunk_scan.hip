@@ -31,8 +31,8 @@
 // What bounds it: the chain of a sequence's chunks, one wave per SIMD: vector instructions (the cutting into terms, the
 // exponentials) and 114 matrix instructions (delta: 162) per chunk and wave at D = 128, and two barriers, 5 us a chunk (delta: 10).
 // Measured, 4 sequences of 2048 tokens, token by token -> this: retention, 8 heads of 128 x 128: 797 -> 168 us, in four
-// segments 68; 32 heads: 857 -> 177; state-space form, 128 heads of 128 x 64: 1058 -> 434; mlstm, 4 heads of 128 x 256: 1987
-// -> 220, in four segments 97, 4 heads of 256 x 512: 3050 -> 299, in two 220; delta rule, 32 heads of 128 x 128: 959 -> 366.
+// segments 73; 32 heads: 857 -> 182; state-space form, 128 heads of 128 x 64: 1058 -> 442; mlstm, 4 heads of 128 x 256: 1987
+// -> 220, in four segments 95, 4 heads of 256 x 512: 3050 -> 299, in two 213; delta rule, 32 heads of 128 x 128: 959 -> 352.
 // One and two waves per workgroup: 436 and 302 us where four took 233 (of 171, before addresses, weights and stores lost
 // their branches).
 #include "chunk_common.h"
@@ -476,7 +476,7 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
                         ut[i] = split3(U[i]);
                         continue;
                     }
-// the small products first, and all of them before they meet the sum: one rounding at its size
+                    // the small products first, and all of them before they meet the sum: one rounding at its size
                     if (i > 0) {
                         Terms4 w[NI];
                         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -784,8 +784,9 @@ static void chunk_scan_run(const hy::ChunkScan& a, hipStream_t s) {
 }
 
 // Segments that a sequence's chunks are dealt to, here and in gla_scan.hip: launches that leave half of the CUs or more without a
-// workgroup carry the states over segments of at least `least` tokens first (half a chunk's work) and take all of them side by side
-// then.  Not with the delta rule, whose step from state to state is a matrix.  256 tokens here (four chunks), 128 in gla_scan.hip (eight,
+// workgroup carry the states over segments first (half a chunk's work) and take all of them side by side then: of at least `least`
+// tokens in the longest sequence, counted up to a chunk (449 tokens: two of 224 for 256), of less or none in the others.  Not with the
+// delta rule, whose step from state to state is a matrix.  256 tokens here (four chunks), 128 in gla_scan.hip (eight,
 // slower ones).  Measured, one pass -> segments: retention, 8 heads of 128 x 128, 4 sequences of 512 tokens (two
 // segments) 45 -> 26 us, one of 512 (two) 45 -> 35, 4096 (16) 332 -> 51; mlstm, 4 heads of 256 x 512, one of 512 (two) 79 -> 64, 4096
 // (eight) 577 -> 152, of 32768 4701 -> 1009; state-space form, 128 heads of 128 x 64, one of 512 (two) 52 -> 43.  At most four segments:

@@ -17,9 +17,9 @@
 //
 // What bounds it: the chain of a sequence's chunks, one wave per SIMD: about 600 vector and 66 matrix instructions a chunk and wave at
 // D = 128, two barriers and the LDS reads between them, 2.8 us.  Measured, 4 sequences of 2048 tokens, 16 heads of 128 x 256: token by
-// token 988 us, this 403; one of 4000, 8 heads: 1684 and 694, in eight segments 173.  P on the vector ALUs from running products: 648 us, and the same
+// token 988 us, this 375; one of 4000, 8 heads: 1684 and 694, in eight segments 172.  P on the vector ALUs from running products: 648 us, and the same
 // with F in float32: state 9.6e-8 of its norm off the float64 recurrence (token by token 8.7e-8, this 7.8e-8); with the stores of a
-// chunk waited for by the next: 482 us, with that 448, and the terms rounded in pairs 403.
+// chunk waited for by the next: 482 us, with that 448, and the terms rounded in pairs 403 (382 as measured for the 375).
 #include "chunk_common.h"
 
 #include <type_traits>

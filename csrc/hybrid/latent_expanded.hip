@@ -12,11 +12,18 @@
 //     weights are the sum's right operand as they stand, the values are read by transposing LDS reads.  Each key and value
 //     operand serves the wave's two sets of 16 rows: with one set per wave the LDS reads take twice the matrix cores' time;
 //   * masks only where a tile reaches past a row's own position (or a window's edge); waves skip tiles they do not see.
-// Workgroups of one (sequence, head) run on one XCD (blockIdx.x is the pair) and so share its L2; the longest walks start first.
+// blockIdx.x is the (sequence, head): where their number is a multiple of 8 the workgroups of one run on one XCD and share its L2, else they
+// are dealt over the XCDs; the longest walks start first.
 //
 // What bounds it: per tile and wave 80 matrix instructions of 16 cycles (D + R = 192, Dv = 128) beside about 1000 cycles of
 // softmax on the vector ALUs, two waves per SIMD.  Measured, 4 sequences of 2048 tokens, 16 heads of 128 + 64 and 128, rank 512: through
 // the latents 557 us and 121 for the two products around it; this 136 (640 TFLOP/s) and 47 for the product in front.
+//
+// Precision: through the latents the query in latent space and the weighted latents are rounded to bfloat16, here the keys and the values;
+// weights and result in both.  Error of a layer's output against float64, of its norm, prompts of 117 to 2048 tokens, through the latents / here:
+// scores of deviation 1 0.00271 .. 0.00292 / 0.00266 .. 0.00283, a third of it 0.00256 .. 0.00277 / 0.00255 .. 0.00276, three times 0.00318 .. 0.00354
+// / 0.00323 .. 0.00368 (rounded values no longer average out over the keys).  Logits of whole prompt steps, 15 of 1872 to 8192 tokens:
+// 0.00962 and 0.00951 on average, the smaller one here in 9.
 #include "hybrid_common.h"
 
 namespace chronos {

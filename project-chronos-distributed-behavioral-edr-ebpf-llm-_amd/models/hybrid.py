@@ -612,7 +612,8 @@ def pack_latent(spec: LatentAttentionSpec, t: dict, device, act_dtype) -> dict:
                w_uv=a(t["uv"].view(spec.heads, spec.vdim, spec.kv_rank)))
     if out["w_uv"].is_cuda and act_dtype == torch.bfloat16 and spec.kv_from is None and not spec.two_term and spec.scale > 0 and \
             spec.kv_rank % 8 == 0 and hops.latent_expanded_ok(spec.dim, spec.rot_dim, spec.vdim):
-        # whole prompts: every head's keys and values in one product of the latents
+        # whole prompts: every head's keys and values in one product of the latents (the up-projections a second time, 2 heads (dim + vdim) rank
+        # bytes: 4 MB a layer for 16 heads of 128 + 128 and rank 512)
         out["w_kv"] = torch.cat([out["w_uk"].transpose(1, 2), out["w_uv"]], 1).reshape(-1, spec.kv_rank)
     rows = [t["dq"] if spec.q_rank else t["q"]]
     if spec.q_rank:
