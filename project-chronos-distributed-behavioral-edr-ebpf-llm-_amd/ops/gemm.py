@@ -71,6 +71,7 @@ _UNEVEN = {112: (16, 32, 8), 113: (16, 64, 8), 114: (16, 16, 8), 115: (32, 16, 8
 # N = 512 .. 32768 by K = 512 .. 14336, and what a launch of each takes in us, fitted on that grid (cold weights; rms error 5 %):
 # constant, split-K's second launch, per 64-deep step of a wave, per MB of weights, per 256 workgroups, per such step of each
 # further round of 256 workgroups, per 100 MB of x that all workgroups read together.  The pick is within 1 % of the best config on average.
+# profiles/few_rows_gemm.json: 68 of the shapes, every one measured with the library, the best config and the pick.
 _FEW = ((16, {114: (2.4, 2.0, 0.77, 0.016, 0.23, 0.69, 3.4), 115: (2.2, 2.1, 1.4, 0.0082, 0.57, 1.3, 5.1),
               72: (2.2, 0.0, 0.16, 0.07, 1.2, 0.24, 8.3), 75: (1.7, 0.0, 0.28, 0.1, 1.4, 0.0, 10.0)}),
         (32, {112: (2.3, 2.1, 1.1, 0.0, 0.67, 0.9, 1.0), 72: (2.1, 0.0, 0.18, 0.052, 1.5, 0.22, 8.7),
