@@ -214,6 +214,8 @@ def few_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     11.7 -> 8.1): 1.3 .. 1.6 times as fast on average, 4 of 590 slower by more than 3 %, the worst by 6 %; 48 shapes off the grid: 1.7
     times, none slower.  More weights than that stream from memory at the library's rate too (8192 x 8192, 16 rows: 30.5, 31.1 here),
     except that it keeps half the chip idle for wide outputs of up to 48 rows (22016 x 2048, 16 rows: 44 -> 21)."""
+    if 1 < m <= GEMV_MAX_M or PP_MODE != "auto":   # (programs set both while they run: nothing of them in the cache)
+        return None
     key = (m, n, k, -1)
     hit = _plan_cache.get(key, False)
     if hit is not False:
@@ -222,9 +224,9 @@ def few_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     if m == 1:
         ok = (k < 2048 or k % 512 != 0) and nk <= 100_000_000
     else:
-        ok = GEMV_MAX_M < m <= 64 and (nk <= 12_500_000 and (m <= 32 or k <= 2048 or nk <= 7_000_000) or
+        ok = m <= 64 and (nk <= 12_500_000 and (m <= 32 or k <= 2048 or nk <= 7_000_000) or
                                        m <= 48 and n >= 12288 and nk <= (40_000_000 if n < 16384 else 100_000_000))
-    if ok and n > 0 and n % 16 == 0 and k % 64 == 0 and k <= 1 << 20 and PP_MODE == "auto" and (n, k, PP_PLAIN) not in _plan_file():
+    if ok and n > 0 and n % 16 == 0 and k % 64 == 0 and k <= 1 << 20 and (n, k, PP_PLAIN) not in _plan_file():
         best = None
         for cfg, c in next(models for most, models in _FEW if m <= most).items():
             bn, bm, nw = _UNEVEN.get(cfg) or (_PP_BN[cfg], _PP_BM[cfg], 1)

@@ -85,3 +85,19 @@ def test_few_rows_of_shapes_that_the_kernels_refuse(monkeypatch, m):
     for n, k in [(0, 512), (0, 1024), (0, 2048), (16, (1 << 20) + 64), (24, 1024), (1024, 1000), (1024, 0)]:
         assert G.few_rows_plan(m, n, k) is None, (n, k)
     assert G.few_rows_plan(m, 1024, 576) is not None
+
+
+def test_few_rows_follow_the_switches(monkeypatch):
+    """GEMV_MAX_M and PP_MODE count at every call: a plan made under one setting does not outlive it."""
+    monkeypatch.setattr(G, "_plan_cache", {})
+    monkeypatch.setattr(G, "PP_MODE", "auto")
+    monkeypatch.setattr(G, "GEMV_MAX_M", 1)
+    first = G.few_rows_plan(2, 1024, 1024)
+    assert first is not None
+    monkeypatch.setattr(G, "GEMV_MAX_M", 2)
+    assert G.few_rows_plan(2, 1024, 1024) is None and G.few_rows_plan(2, 2048, 1024) is None
+    monkeypatch.setattr(G, "GEMV_MAX_M", 1)
+    assert G.few_rows_plan(2, 1024, 1024) == first and G.few_rows_plan(2, 2048, 1024) is not None
+    for mode in ("lib", "own"):
+        monkeypatch.setattr(G, "PP_MODE", mode)
+        assert G.few_rows_plan(2, 1024, 1024) is None and G.few_rows_plan(1, 1024, 1024) is None
