@@ -30,7 +30,7 @@
 //
 // What bounds it: the chain of a sequence's chunks, one wave per SIMD: vector instructions (the cutting into terms, the
 // exponentials) and 114 matrix instructions (delta: 162) per chunk and wave at D = 128, and two barriers, 5 us a chunk (delta: 10).
-// Measured, 4 sequences of 2048 tokens, token by token -> this: retention, 8 heads of 128 x 128: 797 -> 168 us, in four
+// Measured, 4 sequences of 2048 tokens, token by token -> this: retention, 8 heads of 128 x 128: 797 -> 177 us, in four
 // segments 73; 32 heads: 857 -> 182; state-space form, 128 heads of 128 x 64: 1058 -> 442; mlstm, 4 heads of 128 x 256: 1987
 // -> 220, in four segments 95, 4 heads of 256 x 512: 3050 -> 299, in two 213; delta rule, 32 heads of 128 x 128: 959 -> 352.
 // One and two waves per workgroup: 436 and 302 us where four took 233 (of 171, before addresses, weights and stores lost
@@ -787,12 +787,12 @@ static void chunk_scan_run(const hy::ChunkScan& a, hipStream_t s) {
 // workgroup carry the states over segments first (half a chunk's work) and take all of them side by side then: of at least `least`
 // tokens in the longest sequence, counted up to a chunk (449 tokens: two of 224 for 256), of less or none in the others.  Not with the
 // delta rule, whose step from state to state is a matrix.  256 tokens here (four chunks), 128 in gla_scan.hip (eight,
-// slower ones).  Measured, one pass -> segments: retention, 8 heads of 128 x 128, 4 sequences of 512 tokens (two
-// segments) 45 -> 26 us, one of 512 (two) 45 -> 35, 4096 (16) 332 -> 51; mlstm, 4 heads of 256 x 512, one of 512 (two) 79 -> 64, 4096
-// (eight) 577 -> 152, of 32768 4701 -> 1009; state-space form, 128 heads of 128 x 64, one of 512 (two) 52 -> 43.  At most four segments:
-// 118 and 232 us for the two of 4096.  One decay per row, heads of 128 x 256: 16 heads, 2 sequences of 256 tokens (two segments) 50 -> 48
-// us, one of 2048 (four) 360 -> 167; 4 heads, 4 of 256 (two) 49 -> 30, one of 256 (two) 48 -> 46, of 512 (four) 92 -> 49, of 2048 (16)
-// 359 -> 77.
+// slower ones).  Measured, one pass -> segments (profiles/prompt_form_rules.json, 82 launches, one of them slower, by 1 %): retention, 8 heads of
+// 128 x 128, 4 sequences of 512 tokens (two segments) 48 -> 39 us, one of 512 (two) 47 -> 36, 4096 (16) 346 -> 57; mlstm, 4 heads of
+// 256 x 512, one of 512 (two) 81 -> 67, 4096 (eight) 579 -> 157, of 32768 4701 -> 1009; state-space form, 128 heads of 128 x 64, one of
+// 512 (two) 50 -> 43.  At most four segments: 118 and 232 us for the two of 4096.  One decay per row, heads of 128 x 256: 16 heads, 2
+// sequences of 256 tokens (two segments) 52 both, one of 2048 (four) 371 -> 174; 4 heads, 4 of 256 (two) 51 -> 50, of 512 (four) 96 -> 55,
+// one of 512 (four) 96 -> 51, of 2048 (16) 369 -> 79.
 int hy_chunk_segments(int B, int H, int D, int Dv, int longest, int least) {
     if (D != 32 && D != 64 && D != 128 && D != 256) return 1;
     const int64_t wgs = (int64_t)B * H * ((Dv + 63) / 64);

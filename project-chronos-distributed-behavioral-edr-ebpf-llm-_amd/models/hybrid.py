@@ -886,6 +886,8 @@ def _wide_out(w: dict, proj, n: int):
 # launches and the form through the latents has fewer.  Whole steps of 4 layers, two of them latent attention, us, through the
 # latents / written out: 0.7 M (8 heads, 300 tokens) 608 / 640; 1.8 M (8 heads, 16 x 100) 613 / 640; 2.9 M (32 heads, 300) 1314 / 1221;
 # 7 M (32 heads, 16 x 100) 3018 / 2845; 130 M (8 heads, 4000) 1895 / 1710; 500 M (32 heads, 4000) 8040 / 6765.
+# Between 2 and 10 M, 8 heads of 64 are up to 3 % slower written out where their step is still bound by launches (one prompt of 700:
+# 677 / 694) and up to 3 % faster where it is not (32 x 100: 785 / 761); 16 heads of 128 are 5 to 10 % faster (profiles/prompt_form_rules.json).
 EXPAND_MIN = 1 << 21
 
 

@@ -180,6 +180,7 @@ def test_gated_unit_sigmoid():
         assert float(((y.double() - want).abs() - want.abs() * 2 ** -7.9).max()) <= 0
     assert total > 400_000 and wrong <= 1.3e-4 * total, (wrong, total)
 
+
 @pytest.mark.parametrize("tau", [16.0, 20.0, 64.0])
 @pytest.mark.parametrize("lo,hi", [(-100.0, -20.0), (-20.0, -4.0), (-4.0, 4.0), (4.0, 60.0)])
 def test_decay_pow_error(tau, lo, hi):
