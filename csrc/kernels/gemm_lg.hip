@@ -84,26 +84,33 @@ __device__ __forceinline__ void lg_dma16(const void* base, int bytes, unsigned c
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)dst, 16, voff, soff, 0, 0);
 }
 
-// The same piece as inline asm (VAR 2): M0 = the LDS destination, written in the same statement that reads it
-// (cdna_hip_programming.md §5.7).  No VGPR destination; completion is counted by the kernel's own vmcnt waits.
+// The same piece as inline asm (VAR 2): M0 = the LDS destination, written in the same statement that reads it, with the one
+// wait state a scalar write of M0 needs before an LDS-DMA.  No VGPR destination; completion is counted by the kernel's own
+// vmcnt waits.
 typedef int lg_i32x4 __attribute__((ext_vector_type(4)));
-template <bool NOP = true>
-__device__ __forceinline__ void lg_dma16_asm(const void* base, int bytes, uint32_t lds, uint32_t voff, int soff) {
+__device__ __forceinline__ lg_i32x4 lg_rsrc(const void* base, int bytes) {
     const uint64_t b = (uint64_t)base;
-    const lg_i32x4 r = {(int)(uint32_t)b, (int)(uint32_t)(b >> 32), bytes, 0x00020000};
-    if constexpr (NOP)
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %3 offen lds"
-                     ::"v"(voff), "s"(r), "s"(lds), "s"(soff) : "memory");
-    else  // (hipBLASLt's gfx950 code issues the LDS-DMA right after its M0 write)
-        asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, %3 offen lds"
-                     ::"v"(voff), "s"(r), "s"(lds), "s"(soff) : "memory");
+    return lg_i32x4{(int)(uint32_t)b, (int)(uint32_t)(b >> 32), bytes, 0x00020000};
+}
+__device__ __forceinline__ void lg_dma16_asm(const void* base, int bytes, uint32_t lds, uint32_t voff, int soff) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %3 offen lds"
+                 ::"v"(voff), "s"(lg_rsrc(base, bytes)), "s"(lds), "s"(soff) : "memory");
+}
+// HB: the two halves of a piece, with an MFMA between them for the wait state.  One wave per SIMD has issue slots for three
+// instructions beside a 16-cycle MFMA: a third one per piece measured 80 of a slab's 2300 cycles.
+template <int OFF>
+__device__ __forceinline__ void lg_dma_dst(uint32_t lds) {
+    asm volatile("s_add_u32 m0, %0, %1" ::"s"(lds), "n"(OFF) : "memory", "scc");
+}
+__device__ __forceinline__ void lg_dma_go(const void* base, int bytes, uint32_t voff, int soff) {
+    asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(lg_rsrc(base, bytes)), "s"(soff) : "memory");
 }
 
 // HB: image row of W fragment block s relative to block 0 (SwiGLU: gate blocks 0 .. 3, then the up blocks at WN / 2)
 constexpr int hb_wrow(int s, bool swiglu, int WN) { return swiglu ? (s < 4 ? 16 * s : WN / 2 + 16 * (s - 4)) : 16 * s; }
 // ... of 32-row block S (F8HB)
 constexpr int hb_wrow32(int S, bool swiglu, int WN) { return swiglu ? (S < 2 ? 32 * S : WN / 2 + 32 * (S - 2)) : 32 * S; }
-// HB bit 7 (HBV & 128): k-step 0 of a slab in growing-square order — MFMA (s, t) as soon as fa[s] and fb[t] can
+// VAR 5: k-step 0 of a slab in growing-square order — MFMA (s, t) as soon as fa[s] and fb[t] can
 // have landed — with the set-0 reads alternating fa[0], fb[0], fb[1], fa[1], fb[2], fa[2], ...: the slab head's first
 // k MFMAs need ~2 sqrt(k) of the 16 reads issued at the end of the previous slab instead of k + 1, so fewer of them
 // wait on the tail of that read burst
@@ -120,29 +127,23 @@ constexpr int hb_sq_t(int ii) {
 // 2 n + 1 -> fa[n]
 constexpr bool hb_sq_isw(int r) { return r == 0 || (r >= 2 && (r & 1)); }
 constexpr int hb_sq_blk(int r) { return r < 2 ? 0 : r / 2; }
-// F8HB slab schedule (32 MFMA slots): x pieces spread over [B1, B2), W pieces over [B2, B3)
-constexpr int hb8_piece(int i, int B1, int B2, int B3, int NPW, int NPX) {
-    for (int p = 0; p < NPX; ++p)
-        if (B1 + p * (B2 - B1) / NPX == i) return NPW + p;
-    for (int p = 0; p < NPW; ++p)
-        if (B2 + p * (B3 - B2) / NPW == i) return p;
+// HB slab schedule: the DMA piece issued before MFMA slot i (-1: none): n pieces spread evenly over slots [rel, end)
+constexpr int hb_piece(int i, int rel, int end, int n) {
+    for (int p = 0; p < n; ++p)
+        if (rel + p * (end - rel) / n == i) return p;
     return -1;
 }
-
-// HB slab schedule: the DMA piece issued before MFMA i of the 128 (-1: none).  Pieces 0 .. NPW-1 are W, the rest x.
-constexpr int hb_piece(int i, int B1, int B2, int B3, int DX, int DW, int NPW, int NPX) {
-    return (i >= B1 && i < B2 && (i - B1) % DX == 0 && (i - B1) / DX < NPX) ? NPW + (i - B1) / DX
-           : (i >= B2 && i < B3 && (i - B2) % DW == 0 && (i - B2) / DW < NPW) ? (i - B2) / DW
-                                                                              : -1;
+// read r of a group of n reads spread evenly over slots [from, to): is it due at slot i?  (first one due at i, or -1; several may
+// share a slot when the group is denser than the slots: hb_due_n of them, consecutive)
+constexpr int hb_due(int i, int from, int to, int n) {
+    for (int r = 0; r < n; ++r)
+        if (from + r * (to - from) / n == i) return r;
+    return -1;
 }
-// hipBLASLt's distribution: x pieces 0-4 after B1 and 5-7 after B2 (every 2 MFMAs), W pieces 0-4 spread over
-// B2+8 .. B3 and 5-7 after B3
-constexpr int hb_piece_lib(int i, int B1, int B2, int B3, int NPW, int NPX) {
-    return (i >= B1 && i < B1 + 10 && (i - B1) % 2 == 0) ? NPW + (i - B1) / 2
-           : (i >= B2 && i < B2 + 6 && (i - B2) % 2 == 0) ? NPW + 5 + (i - B2) / 2
-           : (i >= B2 + 8 && i < B2 + 58 && (i - B2 - 8) % 10 == 0) ? (i - B2 - 8) / 10
-           : (i >= B3 + 4 && i < B3 + 16 && (i - B3 - 4) % 4 == 0) ? 5 + (i - B3 - 4) / 4
-                                                                    : -1;
+constexpr int hb_due_n(int i, int from, int to, int n) {
+    int c = 0;
+    for (int r = 0; r < n; ++r) c += from + r * (to - from) / n == i;
+    return c;
 }
 
 // W8A8 fp8 (F8): a fragment of v_mfma_scale_f32_16x16x128_f8f6f4 is 32 k-bytes per lane (two 16-B chunks)
@@ -183,31 +184,21 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
     // halves); the accumulators are copied into the 16x16 register order before split-K / the epilogue, which then
     // maps (block, register) -> (n, m) with the 32x32 output layout
     constexpr bool M32 = VAR == 3;
-    // VAR 4 (HB): one wave per SIMD (NWX = 2), 128 x 128 outputs per wave, and the slab loop of three barriers per
-    // 64-deep slab (profiles/r6_gemm_isa_diff.md): the wave reads ALL of slab j's fragments into registers early (k-step
-    // 0 at the end of slab j-1, k-step 1 in the first quarter of slab j), so the slab's LDS buffer is released per
-    // operand after a quarter (x) / half (W) of the slab and slab j+2's LDS-DMA gets ~1.5 slabs to land (vmcnt counted,
-    // never 0); every wave stages a share of both operands, so each release barrier is followed by DMA on all waves
-    // HB variants (timing study, VAR 5-11 = 4 + bits; every one computes the same result): bit 0 LDS-DMA pieces
-    // without the s_nop after the M0 write; bit 1 hipBLASLt's DMA distribution (x: 5 pieces after B1 + 3 after B2,
-    // W: 5 after B2 + 3 after B3, vmcnt(13)); bit 2 lgkmcnt(0) before the slab's last MFMA instead of hipcc's counted
-    // waits at the next slab's head; bit 3 precomputed addressing (below); bit 4 LDS-staged epilogue; bit 5 the next
-    // slab's reads from MFMA 94 (below)
-    constexpr bool HB = VAR >= 4 && VAR < 260;
-    constexpr int HBV = HB ? VAR - 4 : 0;
+    // VAR 4 - 6 (HB): one wave per SIMD (NWX = 2), 128 x 128 outputs per wave, a 64-deep slab in two k-steps whose fragments
+    // all live in registers, two barriers per slab (schedule at the loop), LDS-staged epilogue.  5: k-step 0 in
+    // growing-square order; 6: 32x32x16 MFMAs
+    constexpr bool HB = VAR >= 4;
     constexpr int ES = F8 ? 1 : 2;  // operand bytes per element
-    // F8 + HB (VAR with bits 8 and 16: precomputed addressing, staged epilogue): the HB slab loop on
-    // v_mfma_scale_f32_32x32x64_f8f6f4 (F8HB below)
+    // F8 + HB: the HB slab loop on v_mfma_scale_f32_32x32x64_f8f6f4 (F8HB below)
     static_assert(!F8 || (RB == 128 && MODE != kResid && !NORMP && ABL == 0 &&
-                          (ST >= 3 ? VAR == 0 : (HB && (HBV & 24) == 24 && !(HBV & 2) && !(HBV & 32)))),
+                          (ST >= 3 ? VAR == 0 : VAR == 4)),
                   "fp8: ring schedule or the HB slab loop, 128-B rows, plain / SwiGLU epilogue");
     constexpr bool F8HB = F8 && HB;
-    // bit 6 (HBV & 64, bf16): the F8HB loop on v_mfma_f32_32x32x16_bf16 — a slot is two 16-deep MFMAs (the lo / hi
+    // VAR 6 (bf16): the F8HB loop on v_mfma_f32_32x32x16_bf16 — a slot is two 16-deep MFMAs (the lo / hi
     // 16 B of a 32-B fragment), so a slab is 32 slots of 64 MFMA cycles as in F8HB, with half the MFMA issues of
     // the 16x16x32 loop
-    constexpr bool B32HB = HB && !F8 && (HBV & 64);
+    constexpr bool B32HB = VAR == 6 && !F8;
     constexpr bool XHB = F8HB || B32HB;  // the 32-slot slab loop
-    static_assert(!B32HB || ((HBV & 24) == 24 && !(HBV & 2) && !(HBV & 32)), "32x32 HB: precomputed + staged");
     constexpr bool L32 = M32 || XHB;  // 32x32 accumulator blocks
     using FT = std::conditional_t<F8, lg_i32x8, bf16x8>;  // MFMA operand fragment
     constexpr int NW = 2 * NWX;                       // waves: 2 along W x NWX along x (NWX = 4: two per SIMD)
@@ -507,7 +498,7 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
             for (int u = 0; u < MT / 2; ++u) gb0[u] = f8rd(0, 1, 0, 32 * RB * u);
 #pragma unroll
             for (int s = 1; s < NT / 2; ++s) ga0[s] = f8rd(0, 0, 0, hb_wrow32(s, MODE == kSwiglu, WN) * RB);
-        } else if constexpr (HB && (HBV & 128)) {  // (the loop's alternating set-0 read order, see hb_sq_isw)
+        } else if constexpr (VAR == 5) {  // (the loop's alternating set-0 read order, see hb_sq_isw)
 #pragma unroll
             for (int r = 0; r < NT + MT; ++r) {
                 const int b = hb_sq_blk(r);
@@ -564,25 +555,22 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
             }
         };
         if constexpr (HB) {
-            // slab j, MFMA i of 128 (k-step i / 64; W block s = (i % 64) / 8, x block t = i % 8), issue order pinned:
-            //   i = 1, 3, .. 15 : ds_read of slab j k-step 1 x fragments (set 1)
-            //   B1 (before 22)  : lgkmcnt(0) + barrier — every wave holds slab j's x fragments: x buffer released
-            //   22 .. 51        : the wave's NPX x pieces of slab j+2 (one per 3 MFMAs) + slab j k-step 1 W reads
-            //   B2 (before 52)  : lgkmcnt(0) + barrier — W buffer released
-            //   52 .. 111       : the wave's NPW W pieces of slab j+2 (one per 7 MFMAs)
-            //   B3 (before 112) : vmcnt(NPER) (this wave's slab j+1 pieces landed; slab j+2's stay in flight) + barrier
-            //   112 .. 127      : ds_read of slab j+1 k-step 0 (set 0): fa[0], fb[0..7], fa[1..7]
-            // hipcc inserts the counted lgkmcnt waits of the set-0 reads at the next slab's first MFMAs.
-            // bit 5 (HBV & 32): hipBLASLt's B3 placement — the next slab's fragment reads start at MFMA 94 and are
-            // spread one per two MFMAs (instead of one per MFMA from 112), the W pieces one per 5 MFMAs before it
-            constexpr int MFK = NT * MT, B1 = 22, B2 = 52, B3 = (HBV & 32) ? 94 : 2 * MFK - (NT + MT);
-            constexpr int RSP = (HBV & 32) ? 2 : 1;  // MFMAs per set-0 read after B3
-            constexpr int DX = 3, DW = (HBV & 32) ? 5 : 7;
+            // A slab keeps its LDS buffer only until its second k-step's fragments are in registers, so the two buffers hold
+            // nearly two slabs in flight.  Slab j, slot i of 128 MFMAs (k-step i / 64), issue order pinned:
+            //   [0, RD1)     : the 16 fragment reads of slab j, k-step 1 (set 1)
+            //   REL          : lgkmcnt(0) + barrier: every wave holds both k-steps of slab j, its buffer is free
+            //   [REL, PEND)  : the wave's 16 LDS-DMA pieces of slab j+2, evenly, x then W
+            //   LAND         : vmcnt(16) (this wave's pieces of slab j+1, issued one slab ago, have landed; those of slab j+2 stay
+            //                  in flight) + barrier: slab j+1 is readable
+            //   [LAND, RD0)  : the 16 fragment reads of slab j+1, k-step 0 (set 0)
+            // What was measured, us at 8192^3 / 5952 x 4096 x 14336 / 1024 x 128256 x 4096: the pieces want to be spread over all the
+            // slots that the dependences leave: over 32 slots 820 / 643 / 891, 48 788 / 617 / 856, 64 751 / 584 / 819, 88 729 / 559 / 797
+            // (with three more instructions a piece than now; REL from 20 to 56 and LAND from 96 to 112 matter little); a piece as
+            // two instructions on either side of an MFMA instead of three before it: 698 / 559 / 764.
+            constexpr int MFK = NT * MT;
+            constexpr int RD1 = 16, REL = 20, PEND = 108, LAND = 112, RD0 = 128;
             static_assert(NPW == 8 && NPX == 8, "HB: 8 W + 8 x pieces per wave and slab");
             const int pstride = RPI * K * ES;  // source bytes between a wave's consecutive pieces of one operand
-            static_assert(B1 >= 2 * MT + 2 && B1 + DX * NPX <= B2 && B1 + 1 + 3 * NT <= B2 && B2 + DW * NPW <= B3 &&
-                              B3 + RSP * (NT + MT) <= 2 * MFK,
-                          "HB schedule");
             // the accumulators live in AGPRs across the whole loop: pinned at both ends, so the epilogue's VGPR use
             // (resid / SwiGLU / norm-scale forms) cannot make the register allocator shuffle them inside the loop
             auto pin_acc = [&]() {
@@ -599,56 +587,52 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
                 }
             };
             pin_acc();
-            if constexpr (XHB) {
-                // W8A8 on the HB loop: a 128-B slab row is 128 e4m3 k = two 64-deep k-steps of 16
-                // v_mfma_scale_f32_32x32x64_f8f6f4 (4 W x 4 x blocks of 32, each MFMA 4x the issue time of a bf16
-                // 16x16x32), so a slab is 32 MFMA slots with the same per-slab bytes, fragment reads (2 ds_read_b128
-                // per fragment, 32 per slab) and DMA pieces as the bf16 loop's 128, and the same three barriers:
-                //   slots 0-3    : set-1 (k-step 1) x fragments of slab j
-                //   B1 (5)       : lgkmcnt(0) + barrier — x buffer released; x pieces of slab j+2 over [B1, B2)
-                //   6, 8, 10, 12 : set-1 W fragments
-                //   B2 (14)      : W buffer released; W pieces of slab j+2 over [B2, B3)
-                //   B3 (28)      : vmcnt(NPER) + barrier — slab j+1 landed
-                //   28-31        : set-0 fragments of slab j+1, two per slot (ga[0], gb[*], ga[1..])
-                constexpr int MK = (NT / 2) * (MT / 2), F1 = 5, F2 = 14, F3 = 28;
-                static_assert(MK == 16 && F1 >= MT / 2 + 1 && F1 + 1 + 2 * (NT / 2 - 1) < F2 - 1 && F3 + 4 == 2 * MK,
-                              "F8HB schedule");
-                uint32_t m0w[2], m0x[2];
+            // LDS destinations of a slab's pieces by buffer: piece q of an operand lands 1 KiB * q behind the wave's first
+            uint32_t dw[2], dx[2];
 #pragma unroll
-                for (int p = 0; p < 2; ++p) {
-                    m0w[p] = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uintptr_t)(smem + p * STAGE + dsto[0]));
-                    m0x[p] = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uintptr_t)(smem + p * STAGE + dsto[NPW]));
-                }
-                const uint32_t vw = voff[0], vx = voff[NPW];
+            for (int p = 0; p < 2; ++p) {
+                dw[p] = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uintptr_t)(smem + p * STAGE + dsto[0]));
+                dx[p] = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uintptr_t)(smem + p * STAGE + dsto[NPW]));
+            }
+            // source offsets of the wave's first piece of each operand, advanced by a slab each (past the end: the last slab again)
+            uint32_t vw = voff[0] + min(1, NS1) * RB, vx = voff[NPW] + min(1, NS1) * RB;
+            auto advance = [&](int j) {
+                const uint32_t d = j + 2 <= NS1 ? RB : 0;
+                vw += d;
+                vx += d;
+            };
+            // piece p of slab j+2 into buffer P: piece q of an operand is q * RPI rows behind its first
+            auto dst = [&](auto PC, auto IC) {
+                constexpr int P = decltype(PC)::value, p = decltype(IC)::value, q = p % 8;
+                lg_dma_dst<1024 * q>(p < NPX ? dx[P] : dw[P]);
+            };
+            auto go = [&](auto IC) {
+                constexpr int p = decltype(IC)::value, q = p % 8;
+                if constexpr (p < NPX) lg_dma_go(a.x, xbytes, vx, q * pstride);
+                else lg_dma_go(a.w, wbytes, vw, q * pstride);
+            };
+            if constexpr (XHB) {
+                // The same schedule on 32 slots of four times the MFMA cycles: W8A8, where a 128-B slab row is 128 e4m3 k = two
+                // 64-deep k-steps of 16 v_mfma_scale_f32_32x32x64_f8f6f4 (4 W x 4 x blocks of 32), and the 32x32x16 form.
+                // A fragment is two ds_read_b128: 8 per group here.
+                constexpr int MK = (NT / 2) * (MT / 2);
+                constexpr int RD1 = 4, REL = 6, PEND = 26, LAND = 28, RD0 = 32;
+                static_assert(MK == 16 && RD1 < REL && REL + 16 <= PEND && PEND <= LAND && RD0 <= 2 * MK, "HB schedule, 32 slots");
                 auto half = [&](auto PC, int j) {
                     constexpr int P = decltype(PC)::value;  // slab j in buffer P, slab j+1 in 1 - P
-                    const int kb = min(j + 2, NS1) * RB;
-                    const void* bw = (const unsigned char*)a.w + kb;
-                    const void* bx = (const unsigned char*)a.x + kb;
-                    const int nw = wbytes - kb, nx = xbytes - kb;
+                    advance(j);
                     auto slot = [&](auto IC) {
                         constexpr int i = decltype(IC)::value;
-                        if constexpr (i == F1 || i == F2) {
+                        if constexpr (i == REL) {
                             __builtin_amdgcn_s_waitcnt(0xC07F);
                             lg_bar();
                         }
-                        if constexpr (i == F3) {
+                        if constexpr (i == LAND) {
                             lg_vmcnt<NPER>();
                             lg_bar();
                         }
-                        constexpr int piece = hb8_piece(i, F1, F2, F3, NPW, NPX);
-                        if constexpr (piece >= 0) {
-                            constexpr bool isW = piece < NPW;
-                            constexpr int q = isW ? piece : piece - NPW;
-                            const uint64_t b = (uint64_t)(isW ? bw : bx);
-                            const lg_i32x4 r = {(int)(uint32_t)b, (int)(uint32_t)(b >> 32), isW ? nw : nx, 0x00020000};
-                            if constexpr (q == 0)
-                                asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
-                                             ::"v"(isW ? vw : vx), "s"(r), "s"(isW ? m0w[P] : m0x[P]) : "memory");
-                            else
-                                asm volatile("s_add_u32 m0, m0, 0x400\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-                                             ::"v"(isW ? vw : vx), "s"(r), "s"(q * pstride) : "memory");
-                        }
+                        constexpr int piece = hb_piece(i, REL, PEND, NPER);
+                        if constexpr (piece >= 0) dst(PC, std::integral_constant<int, piece>{});
                         constexpr int ii = i % MK, S = ii / (MT / 2), U = ii % (MT / 2);
                         const lg_i32x8& fa = i < MK ? ga0[S] : ga1[S];
                         const lg_i32x8& fb = i < MK ? gb0[U] : gb1[U];
@@ -666,23 +650,21 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
                                 __builtin_bit_cast(lg_bf16x8, __builtin_shufflevector(fb, fb, 4, 5, 6, 7)), acc32[S][U], 0, 0,
                                 0);
                         }
-                        if constexpr (i < MT / 2) gb1[i] = f8rd(P, 1, 1, 32 * RB * i);
-                        if constexpr (i > F1 && (i - F1 - 1) % 2 == 0 && (i - F1 - 1) / 2 < NT / 2) {
-                            constexpr int s = (i - F1 - 1) / 2;
-                            ga1[s] = f8rd(P, 0, 1, hb_wrow32(s, MODE == kSwiglu, WN) * RB);
-                        }
-                        if constexpr (i >= F3) {
-                            lg_static_for(
-                                [&](auto RC) {
-                                    constexpr int r = 2 * (i - F3) + decltype(RC)::value;  // ga[0], gb[0..3], ga[1..3]
-                                    if constexpr (r == 0) ga0[0] = f8rd(1 - P, 0, 0, 0);
-                                    else if constexpr (r <= MT / 2) gb0[r - 1] = f8rd(1 - P, 1, 0, 32 * RB * (r - 1));
-                                    else
-                                        ga0[r - MT / 2] =
-                                            f8rd(1 - P, 0, 0, hb_wrow32(r - MT / 2, MODE == kSwiglu, WN) * RB);
-                                },
-                                std::make_integer_sequence<int, 2>{});
-                        }
+                        if constexpr (piece >= 0) go(std::integral_constant<int, piece>{});
+                        // both groups in the order ga[0], gb[0..3], ga[1..3]
+                        auto read = [&](auto RC, int p, int kk, lg_i32x8 (&ga)[NT / 2], lg_i32x8 (&gb)[MT / 2]) {
+                            constexpr int r = decltype(RC)::value;
+                            if constexpr (r == 0) ga[0] = f8rd(p, 0, kk, 0);
+                            else if constexpr (r <= MT / 2) gb[r - 1] = f8rd(p, 1, kk, 32 * RB * (r - 1));
+                            else ga[r - MT / 2] = f8rd(p, 0, kk, hb_wrow32(r - MT / 2, MODE == kSwiglu, WN) * RB);
+                        };
+                        constexpr int r1 = hb_due(i, 0, RD1, NT), r0 = hb_due(i, LAND, RD0, NT);
+                        if constexpr (r1 >= 0)
+                            lg_static_for([&](auto K_) { read(std::integral_constant<int, r1 + decltype(K_)::value>{}, P, 1, ga1, gb1); },
+                                          std::make_integer_sequence<int, hb_due_n(i, 0, RD1, NT)>{});
+                        if constexpr (r0 >= 0)
+                            lg_static_for([&](auto K_) { read(std::integral_constant<int, r0 + decltype(K_)::value>{}, 1 - P, 0, ga0, gb0); },
+                                          std::make_integer_sequence<int, hb_due_n(i, LAND, RD0, NT)>{});
                         __builtin_amdgcn_sched_barrier(0);
                     };
                     lg_static_for(slot, std::make_integer_sequence<int, 2 * MK>{});
@@ -691,12 +673,10 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
                     half(std::integral_constant<int, 0>{}, j);
                     if (j + 1 < NS) half(std::integral_constant<int, 1>{}, j + 1);
                 }
-            } else if constexpr (HBV & 8) {
-                // precomputed addressing: the slab loop unrolled by two, so each half's LDS buffer is a compile-time
-                // parity; fragment reads from 8 per-lane base VGPRs (parity x operand x k-step) + immediate offsets;
-                // the LDS-DMA destination kept in M0 (one s_mov per operand and slab, then s_add 1 KiB per piece, as
-                // hipBLASLt's gfx950 code does: nothing else in the loop uses M0) and the source's k offset folded
-                // into the descriptor base once per slab, so a piece's scalar offset is a loop-invariant row stride
+            } else {
+                static_assert(RD1 < REL && REL + 16 <= PEND && PEND <= LAND && RD0 <= 2 * MFK, "HB schedule");
+                // unrolled by two slabs, so a half's LDS buffer is known at compile time: fragment reads are a per-lane base
+                // (buffer x operand x k-step) + an immediate
                 const unsigned char* rbw[2][2];
                 const unsigned char* rbx[2][2];
 #pragma unroll
@@ -706,72 +686,43 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
                         rbw[p][kk] = smem + p * STAGE + wrow0[0] * RB + loff[kk];
                         rbx[p][kk] = smem + p * STAGE + WIMG + xrow0 * RB + loff[kk];
                     }
-                uint32_t m0w[2], m0x[2];
-#pragma unroll
-                for (int p = 0; p < 2; ++p) {
-                    m0w[p] = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uintptr_t)(smem + p * STAGE + dsto[0]));
-                    m0x[p] = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uintptr_t)(smem + p * STAGE + dsto[NPW]));
-                }
-                const uint32_t vw = voff[0], vx = voff[NPW];
                 auto half = [&](auto PC, int j) {
                     constexpr int P = decltype(PC)::value;  // slab j lives in buffer P, slab j+1 in 1 - P
-                    const int kb = min(j + 2, NS1) * RB;
-                    const void* bw = (const unsigned char*)a.w + kb;
-                    const void* bx = (const unsigned char*)a.x + kb;
-                    const int nw = wbytes - kb, nx = xbytes - kb;
+                    advance(j);
                     auto slot = [&](auto IC) {
                         constexpr int i = decltype(IC)::value;
-                        if constexpr (i == B1 || i == B2) {
-                            __builtin_amdgcn_s_waitcnt(0xC07F);
+                        if constexpr (i == REL) {
+                            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), visible to hipcc's wait bookkeeping
                             lg_bar();
                         }
-                        if constexpr (i == B3) {
-                            lg_vmcnt<(HBV & 2) ? 13 : NPER>();
+                        if constexpr (i == LAND) {
+                            lg_vmcnt<NPER>();
                             lg_bar();
                         }
-                        if constexpr ((HBV & 4) && i == 2 * MFK - 1) __builtin_amdgcn_s_waitcnt(0xC07F);
-                        constexpr int piece = (HBV & 2) ? hb_piece_lib(i, B1, B2, B3, NPW, NPX)
-                                                        : hb_piece(i, B1, B2, B3, DX, DW, NPW, NPX);
-                        if constexpr (piece >= 0) {
-                            constexpr bool isW = piece < NPW;
-                            constexpr int q = isW ? piece : piece - NPW;
-                            const uint64_t b = (uint64_t)(isW ? bw : bx);
-                            const lg_i32x4 r = {(int)(uint32_t)b, (int)(uint32_t)(b >> 32), isW ? nw : nx, 0x00020000};
-                            if constexpr (q == 0)
-                                asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
-                                             ::"v"(isW ? vw : vx), "s"(r), "s"(isW ? m0w[P] : m0x[P]) : "memory");
-                            else
-                                asm volatile("s_add_u32 m0, m0, 0x400\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-                                             ::"v"(isW ? vw : vx), "s"(r), "s"(q * pstride) : "memory");
-                        }
+                        constexpr int piece = hb_piece(i, REL, PEND, NPER);
+                        if constexpr (piece >= 0) dst(PC, std::integral_constant<int, piece>{});
                         constexpr int ii = i % MFK;
-                        constexpr bool SQ = (HBV & 128) && i < MFK;  // (k-step 0 only: k-step 1's reads land early)
+                        constexpr bool SQ = VAR == 5 && i < MFK;  // (k-step 0 only: k-step 1's reads land early)
                         constexpr int s = SQ ? hb_sq_s(ii) : ii / MT, t = SQ ? hb_sq_t(ii) : ii % MT;
                         if constexpr (i < MFK)
                             acc[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa0[s], fb0[t], acc[s][t], 0, 0, 0);
                         else
                             acc[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa1[s], fb1[t], acc[s][t], 0, 0, 0);
-                        if constexpr (i < B1 && (i & 1) && i / 2 < MT)
-                            fb1[i / 2] = *reinterpret_cast<const bf16x8*>(rbx[P][1] + 16 * RB * (i / 2));
-                        if constexpr (i > B1 && i < B2 && (i - B1 - 1) % 3 == 0 && (i - B1 - 1) / 3 < NT) {
-                            constexpr int r = (i - B1 - 1) / 3;
-                            fa1[r] = *reinterpret_cast<const bf16x8*>(rbw[P][1] + hb_wrow(r, MODE == kSwiglu, WN) * RB);
-                        }
-                        if constexpr ((HBV & 128) && i >= B3 && (i - B3) % RSP == 0 && (i - B3) / RSP < NT + MT) {
-                            constexpr int r = (i - B3) / RSP, b = hb_sq_blk(r);  // fa0, fb0, fb1, fa1, fb2, fa2, ...
-                            if constexpr (hb_sq_isw(r))
-                                fa0[b] = *reinterpret_cast<const bf16x8*>(rbw[1 - P][0] + hb_wrow(b, MODE == kSwiglu, WN) * RB);
+                        if constexpr (piece >= 0) go(std::integral_constant<int, piece>{});
+                        auto read = [&](auto RC, int p, int kk, bf16x8 (&fa)[NT], bf16x8 (&fb)[MT]) {
+                            constexpr int r = decltype(RC)::value;
+                            // set 0 of VAR 5: fa0, fb0, fb1, fa1, fb2, fa2, ...; else fa[0], fb[0..MT-1], fa[1..NT-1]
+                            constexpr bool isw = VAR == 5 ? hb_sq_isw(r) : r == 0 || r > MT;
+                            constexpr int b = VAR == 5 ? hb_sq_blk(r) : r == 0 ? 0 : r <= MT ? r - 1 : r - MT;
+                            if constexpr (isw)
+                                fa[b] = *reinterpret_cast<const bf16x8*>(rbw[p][kk] + hb_wrow(b, MODE == kSwiglu, WN) * RB);
                             else
-                                fb0[b] = *reinterpret_cast<const bf16x8*>(rbx[1 - P][0] + 16 * RB * b);
-                        } else if constexpr (i >= B3 && (i - B3) % RSP == 0 && (i - B3) / RSP < NT + MT) {
-                            constexpr int r = (i - B3) / RSP;  // fa[0], fb[0..MT-1], fa[1..NT-1]
-                            if constexpr (r == 0) fa0[0] = *reinterpret_cast<const bf16x8*>(rbw[1 - P][0]);
-                            else if constexpr (r <= MT)
-                                fb0[r - 1] = *reinterpret_cast<const bf16x8*>(rbx[1 - P][0] + 16 * RB * (r - 1));
-                            else
-                                fa0[r - MT] = *reinterpret_cast<const bf16x8*>(
-                                    rbw[1 - P][0] + hb_wrow(r - MT, MODE == kSwiglu, WN) * RB);
-                        }
+                                fb[b] = *reinterpret_cast<const bf16x8*>(rbx[p][kk] + 16 * RB * b);
+                        };
+                        constexpr int r1 = hb_due(i, 0, RD1, NT + MT), r0 = hb_due(i, LAND, RD0, NT + MT);
+                        static_assert(hb_due_n(i, 0, RD1, NT + MT) <= 1 && hb_due_n(i, LAND, RD0, NT + MT) <= 1, "one read a slot");
+                        if constexpr (r1 >= 0) read(std::integral_constant<int, r1>{}, P, 1, fa1, fb1);
+                        if constexpr (r0 >= 0) read(std::integral_constant<int, r0>{}, 1 - P, 0, fa0, fb0);
                         __builtin_amdgcn_sched_barrier(0);
                     };
                     lg_static_for(slot, std::make_integer_sequence<int, 2 * MFK>{});
@@ -780,55 +731,6 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
                     half(std::integral_constant<int, 0>{}, j);
                     if (j + 1 < NS) half(std::integral_constant<int, 1>{}, j + 1);
                 }
-            } else
-            for (int j = 0; j < NS; ++j) {
-                const unsigned char* cwb = smem + (j & 1) * STAGE;        // slab j (W image, x image at + WIMG)
-                const unsigned char* nwb = smem + ((j + 1) & 1) * STAGE;  // slab j+1
-                const uint32_t dbase = (uint32_t)(uintptr_t)(smem + (j & 1) * STAGE);  // slab j+2 lands here
-                const int kb = min(j + 2, NS1) * RB;
-                // one MFMA slot of the slab, everything decided at compile time
-                auto slot = [&](auto IC) {
-                    constexpr int i = decltype(IC)::value;
-                    if constexpr (i == B1 || i == B2) {
-                        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), visible to hipcc's wait bookkeeping
-                        lg_bar();
-                    }
-                    if constexpr (i == B3) {
-                        lg_vmcnt<(HBV & 2) ? 13 : NPER>();  // (the pieces this wave issued since the last B3)
-                        lg_bar();
-                    }
-                    if constexpr ((HBV & 4) && i == 2 * MFK - 1) __builtin_amdgcn_s_waitcnt(0xC07F);
-                    constexpr int piece = (HBV & 2) ? hb_piece_lib(i, B1, B2, B3, NPW, NPX)
-                                                    : hb_piece(i, B1, B2, B3, DX, DW, NPW, NPX);
-                    // a wave's pieces of one operand are consecutive 8-row groups of the source (the chunk swizzle
-                    // depends on lane / 8 only): one VGPR offset per operand, the piece's rows in the scalar offset
-                    if constexpr (piece >= 0)
-                        lg_dma16_asm<!(HBV & 1)>(piece < NPW ? (const void*)a.w : (const void*)a.x, piece < NPW ? wbytes : xbytes,
-                                     (uint32_t)__builtin_amdgcn_readfirstlane((int)(dbase + dsto[piece])),
-                                     piece < NPW ? voff[0] : voff[NPW],
-                                     kb + (piece < NPW ? piece : piece - NPW) * pstride);
-                    constexpr int ii = i % MFK, s = ii / MT, t = ii % MT;
-                    if constexpr (i < MFK)
-                        acc[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa0[s], fb0[t], acc[s][t], 0, 0, 0);
-                    else
-                        acc[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa1[s], fb1[t], acc[s][t], 0, 0, 0);
-                    if constexpr (i < B1 && (i & 1) && i / 2 < MT)
-                        fb1[i / 2] = *reinterpret_cast<const bf16x8*>(cwb + WIMG + (xrow0 + 16 * (i / 2)) * RB + loff[1]);
-                    if constexpr (i > B1 && i < B2 && (i - B1 - 1) % 3 == 0 && (i - B1 - 1) / 3 < NT) {
-                        constexpr int r = (i - B1 - 1) / 3;
-                        fa1[r] = *reinterpret_cast<const bf16x8*>(cwb + wrow0[r] * RB + loff[1]);
-                    }
-                    if constexpr (i >= B3) {
-                        constexpr int r = i - B3;  // fa[0], fb[0..MT-1], fa[1..NT-1]
-                        if constexpr (r == 0) fa0[0] = *reinterpret_cast<const bf16x8*>(nwb + wrow0[0] * RB + loff[0]);
-                        else if constexpr (r <= MT)
-                            fb0[r - 1] =
-                                *reinterpret_cast<const bf16x8*>(nwb + WIMG + (xrow0 + 16 * (r - 1)) * RB + loff[0]);
-                        else fa0[r - MT] = *reinterpret_cast<const bf16x8*>(nwb + wrow0[r - MT] * RB + loff[0]);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                };
-                lg_static_for(slot, std::make_integer_sequence<int, 2 * MFK>{});
             }
             pin_acc();
         }
@@ -998,9 +900,9 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
     }  // ring schedule
     lg_vmcnt<0>();  // the past-the-end DMAs must land before the workgroup's LDS is released
 
-    if constexpr (HB && (HBV & 16)) {
+    if constexpr (HB) {
         if (S > 1) {
-            // ---- split-K for the staged HB configs (M <= 2048 shapes whose 256 x 256 tile grid under-fills the chip):
+            // ---- split-K for the HB configs (M <= 2048 shapes whose 256 x 256 tile grid under-fills the chip):
             // every slice stores its fp32 tile in register order (plain stores + agent release), the last arriver of
             // the ticket sums all slices' slabs in slice order (deterministic) into its accumulators, one W block at a
             // time (a compiler barrier per block keeps hipcc from hoisting all 64 slab loads at once), then runs the
@@ -1052,7 +954,7 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
                 asm volatile("" ::: "memory");
             }
         }
-        // ---- staged epilogue (HB bit 4): the wave's bf16 results go through its own 32 KiB of the (now free) LDS
+        // ---- staged epilogue: the wave's bf16 results go through its own 32 KiB of the (now free) LDS
         // ring, so every global store is a 16-B-per-lane piece of whole 128-B lines (32 dwordx4 stores per lane instead
         // of 64 dwordx2 ones covering 32-B segments); the residual form reads its residual the same way.  Register
         // phase: lane (row r = 16 u + lane % 16, columns 16 s + 4 (lane / 16) .. +3) writes 8 B into row r of the
@@ -1204,7 +1106,7 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
     }
 
     // ---- split-K: fp32 slab in register order, ticket, the last arriver sums every slab in slice order
-    if (!HB && S > 1) {  // (HB: no split-K; its fp32 slab code doubles the kernel's register pressure)
+    if (!HB && S > 1) {  // (HB has its own above)
         // slab hand-off: plain stores + agent release / acquire fences (each a write-back / invalidate of the XCD's
         // L2), or write-through stores + agent-scope loads with no fence (gemm_skinny.hip's form).  Write-through
         // wins on the 8-16 KB slabs of the 32/64-row tiles (O M = 128 cfg39 split-K 2: 17.5 vs 20.1 us) and loses
@@ -1442,24 +1344,18 @@ void lg_launch(const PPArgs& a, hipStream_t st) {
     X(78, 128, 32, 128, 7, 2)      \
     X(79, 64, 32, 128, 12, 2)      \
     X(80, 256, 256, 128, 2, 4, 3)  \
-    X(81, 256, 256, 128, 2, 2, 4)  \
-    X(82, 256, 256, 128, 2, 2, 5)  \
-    X(83, 256, 256, 128, 2, 2, 6)  \
-    X(84, 256, 256, 128, 2, 2, 8)  \
-    X(85, 256, 256, 128, 2, 2, 7)  \
-    X(86, 256, 256, 128, 2, 2, 13) \
-    X(87, 256, 256, 128, 2, 2, 15) \
-    X(88, 256, 256, 128, 2, 2, 29) \
-    X(89, 256, 256, 128, 2, 2, 31) \
-    X(90, 256, 256, 128, 2, 2, 60) \
-    X(91, 256, 256, 128, 2, 2, 93) \
-    X(92, 256, 256, 128, 2, 2, 157) \
-    X(93, 256, 256, 128, 2, 2, 159) \
-    X(94, 256, 256, 128, 2, 2, 189)
+    X(88, 256, 256, 128, 2, 2, 4)  \
+    X(91, 256, 256, 128, 2, 2, 6)  \
+    X(92, 256, 256, 128, 2, 2, 5)
+
+// Ids 81 .. 94 name the HB kernels: 88 (81 .. 87, 89, 90: the same kernel), 92 with the square order (93, 94), 91 on 32x32x16 MFMAs
+constexpr int lg_id(int cfg) {
+    return cfg < 81 || cfg > 94 || cfg == 91 ? cfg : cfg >= 92 ? 92 : 88;
+}
 
 template <int MODE, bool NORMP>
 bool lg_mode(int cfg, const PPArgs& a, hipStream_t st) {
-    switch (cfg) {
+    switch (lg_id(cfg)) {
 #define LG_CASE(ID, WN_, XM_, RB_, ST_, NWX_, ...) \
     case ID: lg_launch<WN_, XM_, RB_, ST_, MODE, NORMP, NWX_, 0, ##__VA_ARGS__>(a, st); return true;
         LG_CONFIGS(LG_CASE)
@@ -1512,7 +1408,7 @@ bool gemm_lg_ablations_built() {
 
 int gemm_lg_xm(int cfg) {
     if (gemm_lg_ablations_built() && cfg >= 40 && cfg < 72) return 256;  // ablation ids
-    switch (cfg) {
+    switch (lg_id(cfg)) {
 #define LG_XM(ID, WN_, XM_, RB_, ST_, NWX_, ...) case ID: return XM_;
         LG_CONFIGS(LG_XM)
 #undef LG_XM
@@ -1523,7 +1419,7 @@ bool gemm_lg_splitk_ok(int cfg) { return cfg < 81 || cfg > 94 || cfg >= 88; }
 
 int gemm_lg_wn(int cfg) {
     if (gemm_lg_ablations_built() && cfg >= 40 && cfg < 72) return 256;
-    switch (cfg) {
+    switch (lg_id(cfg)) {
 #define LG_WN(ID, WN_, XM_, RB_, ST_, NWX_, ...) case ID: return WN_;
         LG_CONFIGS(LG_WN)
 #undef LG_WN
@@ -1533,14 +1429,13 @@ int gemm_lg_wn(int cfg) {
 
 // W8A8 fp8 configs {id, WN, XM, RB, ST, NWX}: ring schedule, one 128-deep v_mfma_scale_f32_16x16x128_f8f6f4 k-step
 // per 128-B stage row (every staged byte carries twice the bf16 kernel's K)
-// 4 (F8HB): the HB slab loop (4 waves, 128 x 128 outputs per wave, three barriers per slab) on
-// v_mfma_scale_f32_32x32x64_f8f6f4, precomputed addressing + LDS-staged epilogue (VAR 29 = bf16 cfg 88's bits)
+// 4 (F8HB): the HB slab loop (4 waves, 128 x 128 outputs per wave) on v_mfma_scale_f32_32x32x64_f8f6f4
 #define LG_F8_CONFIGS(X)       \
     X(0, 256, 128, 128, 3, 4)  \
     X(1, 128, 256, 128, 3, 4)  \
     X(2, 128, 128, 128, 4, 2)  \
     X(3, 128, 128, 128, 3, 4)  \
-    X(4, 256, 256, 128, 2, 2, 29)
+    X(4, 256, 256, 128, 2, 2, 4)
 
 namespace {
 constexpr int lg_f8_var(int v = 0) { return v; }  // (the config's VAR, 0 when the row gives none)
