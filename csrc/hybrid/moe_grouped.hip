@@ -19,6 +19,7 @@
 // The tile loop is an LDS-DMA ring (16x16x32 bf16 MFMAs, XOR-swizzled images, one barrier per k-step with a counted vmcnt) at
 // three tile sizes, below.  Needs d % 128 == 0 and F % 128 == 0.
 #include "hybrid_common.h"
+#include "chronos_slab.h"
 #include "moe_tile.h"
 
 namespace chronos {
@@ -29,7 +30,7 @@ typedef __attribute__((address_space(1))) void* gbl_ptr_t;
 
 // A tile: TM rows (tokens) by TN weight rows, k taken 64 at a time (whole 128-byte lines: rows of half lines reach a CU at a
 // third of the rate) through a ring of ST stages; waves as 2 (weight rows) x WX (tokens).
-//   256 x 256, two stages (128 KB), 8 waves of 128 x 64 outputs (moe_gemm256_kernel): experts with many tokens; half the bytes
+//   256 x 256, two stages (128 KB), 4 waves of 128 x 128 outputs (moe_gemm256_kernel): experts with many tokens; half the bytes
 //    per product of
 //   128 x 128, two stages (64 KB: two workgroups per CU, one multiplies while the other waits), 4 waves of 64 x 64
 //    32 x 128, four stages (80 KB: two workgroups per CU, the weights of three k-steps in flight in each): few tokens
@@ -275,12 +276,61 @@ __global__ void __launch_bounds__(256, 2) moe_gemm_kernel(const uint16_t* __rest
     moe_store<ACT, C::NS, C::NM>(acc, y, row_item, m0 + 16 * C::NM * wm, tn * C::TN + C::TN / 2 * wn, N, lane, limit, slope, shift);
 }
 
-// The 256 x 256 tile (x and one expert's weights below 4 and 2 GiB; weight rows past the end repeat the last one).  Two sets of operands in registers: while
-// one half of a k-step (32 deep) is multiplied the other half's fragments are read from LDS, so that neither the LDS nor
-// the matrix cores wait for the other; one barrier per k-step, in its middle, behind which the buffer that everybody has read is
-// refilled for the step after next.
+// The wave's 128 x 128 outputs of the 256 x 256 tile, through its own 32 KiB of LDS, so that a store instruction writes whole lines: 16
+// lanes a row (8 for a gated unit's 64 columns).  Registers as in moe_store; row r's 16-byte piece c lies at c ^ (r % pieces).
+template <int ACT>
+__device__ __forceinline__ void moe_store_staged(const f32x4 (&acc)[8][8], unsigned char* stg, uint16_t* __restrict__ y,
+                                                 const int32_t* __restrict__ row_item, int m0, int n0, int N, int lane, float limit,
+                                                 float slope, float shift) {
+    constexpr bool GLU = ACT == kActGlu;
+    constexpr int NCH = GLU ? 8 : 16, RPI = 64 / NCH, NK = 128 / RPI;   // pieces per row, rows per store, stores
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        const int r = 16 * t + (lane & 15);
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            if (GLU && (s & 2)) continue;
+            const int col = GLU ? 32 * (s >> 2) + 16 * (s & 1) + 4 * (lane >> 4) : 16 * s + 4 * (lane >> 4);
+            u16x4 o;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float v = acc[s][t][i];
+                if constexpr (GLU) {
+                    // every 64 rows: blocks 0 and 1 are gate rows, 2 and 3 the up rows of the same outputs
+                    const float a = fminf(bf2f(f2bf(v)), limit);
+                    const float u = fminf(fmaxf(bf2f(f2bf(acc[s | 2][t][i])), -limit), limit);
+                    v = a * sigmoid_act<uint16_t>(slope * a) * (u + shift);
+                } else if constexpr (ACT >= 0) {
+                    v = act_apply(bf2f(f2bf(v)), ACT);
+                }
+                o[i] = f2bf(v);
+            }
+            *reinterpret_cast<u16x4*>(stg + r * (NCH * 16) + (((col >> 3) ^ (r % NCH)) << 4) + ((col >> 2) & 1) * 8) = o;
+        }
+    }
+    const int c = lane % NCH, ld = GLU ? N / 2 : N, n = (GLU ? n0 / 2 : n0) + 8 * c;
+    if (n >= ld) return;   // (the last tile may be half)
+#pragma unroll
+    for (int k0 = 0; k0 < NK; k0 += 8) {
+        u16x8 v[8];
+        int it[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int r = RPI * (k0 + k) + lane / NCH;
+            v[k] = *reinterpret_cast<const u16x8*>(stg + r * (NCH * 16) + ((c ^ (r % NCH)) << 4));
+            it[k] = row_item[m0 + r];
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (it[k] >= 0) *reinterpret_cast<u16x8*>(y + (int64_t)(m0 + RPI * (k0 + k) + lane / NCH) * ld + n) = v[k];
+    }
+}
+
+// The 256 x 256 tile (x and one expert's weights below 4 and 2 GiB; weight rows past the end repeat the last one) on the slab loop
+// of chronos_slab.h: 4 waves of 128 x 128 outputs, the accumulators in the AGPRs.  Bound by the matrix cores and by the last, partly
+// filled round of tiles.
 template <bool GATHER, int ACT>
-__global__ void __launch_bounds__(512, 1) moe_gemm256_kernel(const uint16_t* __restrict__ x, uint32_t xbytes,
+__global__ void __launch_bounds__(256, 1) moe_gemm256_kernel(const uint16_t* __restrict__ x, uint32_t xbytes,
                                                              const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
                                                              const int32_t* __restrict__ meta, int maxTiles, int top, int N,
                                                              int K, float limit, float slope, float shift) {
@@ -294,13 +344,13 @@ __global__ void __launch_bounds__(512, 1) moe_gemm256_kernel(const uint16_t* __r
     const int32_t* row_item = meta + 1 + maxTiles;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m0 = tile * 256;
-    // wave w stages image rows 32 w .. 32 w + 31 of both operands in four pieces of 8 rows
+    // wave w stages image rows 64 w .. 64 w + 63 of both operands in eight pieces of 8 rows
     const int pr = lane >> 3, pc = (lane & 7) ^ pr;
-    uint32_t wvoff[4], xvoff[4];
+    uint32_t wvoff[8], xvoff[8];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        wvoff[i] = moe_weight_offset(tn, wave, i, lane, N, K);
-        uint32_t xr = m0 + 32 * wave + 8 * i + pr;
+    for (int i = 0; i < 8; ++i) {
+        wvoff[i] = moe_weight_offset(tn, 2 * wave + (i >> 2), i & 3, lane, N, K);
+        uint32_t xr = m0 + 64 * wave + 8 * i + pr;
         if constexpr (GATHER) {
             const int it = row_item[xr];
             xr = it < 0 ? 0 : it / top;  // padding rows read token 0 and are never stored
@@ -308,67 +358,66 @@ __global__ void __launch_bounds__(512, 1) moe_gemm256_kernel(const uint16_t* __r
         xvoff[i] = (xr * (uint32_t)K + pc * 8) * 2;
     }
     const uint16_t* we = w + (int64_t)e * N * K;
-    const uint32_t lds0 = lds_offset(smem);
-    auto dma_w = [&](int kt, int i) {
-        dma_1k_buf(we, (uint32_t)N * K * 2, lds0 + (kt & 1) * STAGE + (4 * wave + i) * 1024, wvoff[i], kt * 128);
-    };
-    auto dma_x = [&](int kt, int i) {
-        dma_1k_buf(x, xbytes, lds0 + (kt & 1) * STAGE + IMG + (4 * wave + i) * 1024, xvoff[i], kt * 128);
-    };
-    const int wn = wave >> 2, wm = wave & 3;
-    const int ln = lane & 15, g = lane >> 4;
-    const unsigned char* const wimg = smem + (128 * wn + ln) * 128;   // (16-row blocks: the swizzle depends on ln only)
-    const unsigned char* const ximg = smem + IMG + (64 * wm + ln) * 128;
-    const int ch[2] = {(g ^ (ln & 7)) * 16, ((4 + g) ^ (ln & 7)) * 16};
-    bf16x8 a[2][8], b[2][4];
-    auto ldw = [&](int st, int h, int s) { a[h][s] = *reinterpret_cast<const bf16x8*>(wimg + st * STAGE + s * 2048 + ch[h]); };
-    auto ldx = [&](int st, int h, int t) { b[h][t] = *reinterpret_cast<const bf16x8*>(ximg + st * STAGE + t * 2048 + ch[h]); };
-    f32x4 acc[8][4];
-#pragma unroll
-    for (int s = 0; s < 8; ++s)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) acc[s][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const uint32_t lds0 = lds_offset(smem) + wave * 8192, wbytes = (uint32_t)N * K * 2;
     const int KT = K / 64;
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) { dma_w(kt, i); dma_x(kt, i); }
-    wait_vm<8>();
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-#pragma unroll
-    for (int t = 0; t < 4; ++t) ldx(0, 0, t);
-#pragma unroll
-    for (int s = 0; s < 8; ++s) ldw(0, 0, s);
-    for (int kt = 0; kt < KT; ++kt) {
-        const int st = kt & 1;
-        // first half of the step; the second half's fragments on their way
-#pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            if (s < 4) ldx(st, 1, s);
-            ldw(st, 1, s);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) acc[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0][s], b[0][t], acc[s][t], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
+        for (int i = 0; i < 8; ++i) {
+            const int off = min(kt, KT - 1) * 128;
+            dma_1k_buf(we, wbytes, lds0 + kt * STAGE + i * 1024, wvoff[i], off);
+            dma_1k_buf(x, xbytes, lds0 + kt * STAGE + IMG + i * 1024, xvoff[i], off);
         }
-        // this wave's pieces of the next step have landed and its reads of this one are done; behind the barrier: everybody's
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        const bool more = kt + 2 < KT;
+    const int wn = wave >> 1, wm = wave & 1;
+    const int ln = lane & 15, g = lane >> 4;
+    const unsigned char *rbw[2][2], *rbx[2][2];   // (16-row blocks: the swizzle depends on ln only)
 #pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            if (more && s < 4) { dma_w(kt + 2, s); dma_x(kt + 2, s); }
-            // (the last step reads the other buffer once more, for nothing)
-            if (s < 4) ldx(st ^ 1, 0, s);
-            ldw(st ^ 1, 0, s);
+    for (int p = 0; p < 2; ++p)
 #pragma unroll
-            for (int t = 0; t < 4; ++t) acc[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1][s], b[1][t], acc[s][t], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
+        for (int h = 0; h < 2; ++h) {
+            const int ch = ((4 * h + g) ^ (ln & 7)) * 16;
+            rbw[p][h] = smem + p * STAGE + (128 * wn + ln) * 128 + ch;
+            rbx[p][h] = smem + p * STAGE + IMG + (128 * wm + ln) * 128 + ch;
         }
+    f32x4 acc[8][8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+#pragma unroll
+        for (int t = 0; t < 8; ++t) acc[s][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 fa0[8], fb0[8], fa1[8], fb1[8];
+    lg_vmcnt<16>();
+    lg_bar();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {   // (the order of the loop's own reads)
+        const int b = hb_sq_blk(r);
+        if (hb_sq_isw(r)) fa0[b] = *reinterpret_cast<const bf16x8*>(rbw[0][0] + 2048 * b);
+        else fb0[b] = *reinterpret_cast<const bf16x8*>(rbx[0][0] + 2048 * b);
     }
-    moe_store<ACT, 8, 4>(acc, y, row_item, m0 + 64 * wm, tn * 256 + 128 * wn, N, lane, limit, slope, shift);
+    auto pin = [&]() {
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+#pragma unroll
+            for (int t = 0; t < 8; ++t) asm volatile("" : "+a"(acc[s][t]));
+    };
+    pin();
+    int off = 0;   // byte offset of the slab whose pieces are issued: every row has its own address, the slab's comes on top
+    auto advance = [&](int j) { off = min(j + 2, KT - 1) * 128; };
+    auto dst = [&](auto PC, auto IC) {
+        constexpr int P = decltype(PC)::value, p = decltype(IC)::value;
+        lg_dma_dst<P * STAGE + (p < 8 ? IMG : 0) + (p & 7) * 1024>(lds0);
+    };
+    auto go = [&](auto IC) {
+        constexpr int p = decltype(IC)::value;
+        if constexpr (p < 8) lg_dma_go(x, (int)xbytes, xvoff[p], off);
+        else lg_dma_go(we, (int)wbytes, wvoff[p - 8], off);
+    };
+    struct Row { constexpr int operator()(int b) const { return 2048 * b; } };
+    slab_loop<true>(acc, fa0, fb0, fa1, fb1, rbw, rbx, KT, dst, go, advance, Row{});
+    pin();
+    // the last pieces, which nobody reads, have landed everywhere before the images become the staging rows
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    lg_bar();
+    moe_store_staged<ACT>(acc, smem + wave * 32768, y, row_item, m0 + 128 * wm, tn * 256 + 128 * wn, N, lane, limit, slope, shift);
 }
 
 // An index of E and above is an identity expert (its output is the token itself) where the experts' layer has such
@@ -430,7 +479,7 @@ static void moe_gemm(const uint16_t* x, int64_t rows, const uint16_t* w, uint16_
         constexpr int lds = 4 * 256 * 128;
         static const hipError_t once = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         (void)once;
-        kern<<<maxTiles * ((N + 255) / 256), 512, lds, s>>>(x, (uint32_t)(rows * K * 2), w, y, meta, maxTiles, top, N, K, limit, slope, shift);
+        kern<<<maxTiles * ((N + 255) / 256), 256, lds, s>>>(x, (uint32_t)(rows * K * 2), w, y, meta, maxTiles, top, N, K, limit, slope, shift);
     } else {
         const auto kern = hy::moe_gemm_kernel<TM, GATHER, ACT>;
         constexpr int lds = hy::Tile<TM>::lds;

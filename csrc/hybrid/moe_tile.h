@@ -11,7 +11,7 @@
 namespace chronos {
 namespace hy {
 
-// Byte offset in one expert's matrix [N, K] (bfloat16, below 2 GiB) of what a lane loads for piece i (0 .. 3) of its wave (0 .. 7), k-step 0;
+// Byte offset in one expert's matrix [N, K] (bfloat16, below 2 GiB) of what a lane loads for piece i (0 .. 3) of 32 rows (group wave = 0 .. 7), k-step 0;
 // step kt lies 128 kt bytes further.  The piece holds 8 rows of 128 bytes, permuted by 16-byte pieces.  Rows past the end (a last tile may
 // hold 128) repeat the last one: a buffer descriptor's range check need not see the scalar part of an address, and nothing is read
 // past the matrix this way.  Their products are not stored.

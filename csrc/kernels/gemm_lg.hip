@@ -30,6 +30,7 @@
 // What bounds the large-M configs against hipBLASLt (ablations, PMC, microbenchmarks): profiles/r4_studies.md.
 #include "chronos_hip.h"
 #include "chronos_gemm.h"
+#include "chronos_slab.h"
 
 #include <type_traits>
 #include <utility>
@@ -41,21 +42,6 @@ typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef __attribute__((address_space(1))) void* gbl_ptr_t;
 
 enum : int { kPlain = kPPPlain, kSwiglu = kPPSwiglu, kResid = kPPResid };
-
-template <int N>
-__device__ __forceinline__ void lg_vmcnt() {
-    static_assert(N >= 0 && N < 64, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt((N & 0xF) | (0x7 << 4) | (0xF << 8) | ((N >> 4) << 14));
-}
-
-// raw workgroup barrier nothing is scheduled across
-__device__ __forceinline__ void lg_bar() {
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-}
 
 // compile-time interleave of one MFMA block (T19: sched_group_barrier masks MFMA 0x008, VMEM 0x010, DS read 0x100):
 // the NV DMA pieces one per MFMA at the head, then the NR ds_reads spread over the remaining MFMAs.  Every DMA goes
@@ -87,65 +73,17 @@ __device__ __forceinline__ void lg_dma16(const void* base, int bytes, unsigned c
 // The same piece as inline asm (VAR 2): M0 = the LDS destination, written in the same statement that reads it, with the one
 // wait state a scalar write of M0 needs before an LDS-DMA.  No VGPR destination; completion is counted by the kernel's own
 // vmcnt waits.
-typedef int lg_i32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ lg_i32x4 lg_rsrc(const void* base, int bytes) {
-    const uint64_t b = (uint64_t)base;
-    return lg_i32x4{(int)(uint32_t)b, (int)(uint32_t)(b >> 32), bytes, 0x00020000};
-}
 __device__ __forceinline__ void lg_dma16_asm(const void* base, int bytes, uint32_t lds, uint32_t voff, int soff) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %3 offen lds"
                  ::"v"(voff), "s"(lg_rsrc(base, bytes)), "s"(lds), "s"(soff) : "memory");
 }
-// HB: the two halves of a piece, with an MFMA between them for the wait state.  One wave per SIMD has issue slots for three
-// instructions beside a 16-cycle MFMA: a third one per piece measured 80 of a slab's 2300 cycles.
-template <int OFF>
-__device__ __forceinline__ void lg_dma_dst(uint32_t lds) {
-    asm volatile("s_add_u32 m0, %0, %1" ::"s"(lds), "n"(OFF) : "memory", "scc");
-}
-__device__ __forceinline__ void lg_dma_go(const void* base, int bytes, uint32_t voff, int soff) {
-    asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(lg_rsrc(base, bytes)), "s"(soff) : "memory");
-}
-
 // HB: image row of W fragment block s relative to block 0 (SwiGLU: gate blocks 0 .. 3, then the up blocks at WN / 2)
 constexpr int hb_wrow(int s, bool swiglu, int WN) { return swiglu ? (s < 4 ? 16 * s : WN / 2 + 16 * (s - 4)) : 16 * s; }
+template <bool SWIGLU, int WN, int RB> struct HbRow {
+    constexpr int operator()(int b) const { return hb_wrow(b, SWIGLU, WN) * RB; }
+};
 // ... of 32-row block S (F8HB)
 constexpr int hb_wrow32(int S, bool swiglu, int WN) { return swiglu ? (S < 2 ? 32 * S : WN / 2 + 32 * (S - 2)) : 32 * S; }
-// VAR 5: k-step 0 of a slab in growing-square order — MFMA (s, t) as soon as fa[s] and fb[t] can
-// have landed — with the set-0 reads alternating fa[0], fb[0], fb[1], fa[1], fb[2], fa[2], ...: the slab head's first
-// k MFMAs need ~2 sqrt(k) of the 16 reads issued at the end of the previous slab instead of k + 1, so fewer of them
-// wait on the tail of that read burst
-constexpr int hb_isqrt(int v) {
-    int n = 0;
-    while ((n + 1) * (n + 1) <= v) ++n;
-    return n;
-}
-constexpr int hb_sq_s(int ii) { return ii - hb_isqrt(ii) * hb_isqrt(ii) < hb_isqrt(ii) ? ii - hb_isqrt(ii) * hb_isqrt(ii) : hb_isqrt(ii); }
-constexpr int hb_sq_t(int ii) {
-    return ii - hb_isqrt(ii) * hb_isqrt(ii) < hb_isqrt(ii) ? hb_isqrt(ii) : ii - hb_isqrt(ii) * hb_isqrt(ii) - hb_isqrt(ii);
-}
-// set-0 read r of the alternating order: W (fa) or x (fb) block index; r = 0 -> fa[0], 1 -> fb[0], 2 n -> fb[n],
-// 2 n + 1 -> fa[n]
-constexpr bool hb_sq_isw(int r) { return r == 0 || (r >= 2 && (r & 1)); }
-constexpr int hb_sq_blk(int r) { return r < 2 ? 0 : r / 2; }
-// HB slab schedule: the DMA piece issued before MFMA slot i (-1: none): n pieces spread evenly over slots [rel, end)
-constexpr int hb_piece(int i, int rel, int end, int n) {
-    for (int p = 0; p < n; ++p)
-        if (rel + p * (end - rel) / n == i) return p;
-    return -1;
-}
-// read r of a group of n reads spread evenly over slots [from, to): is it due at slot i?  (first one due at i, or -1; several may
-// share a slot when the group is denser than the slots: hb_due_n of them, consecutive)
-constexpr int hb_due(int i, int from, int to, int n) {
-    for (int r = 0; r < n; ++r)
-        if (from + r * (to - from) / n == i) return r;
-    return -1;
-}
-constexpr int hb_due_n(int i, int from, int to, int n) {
-    int c = 0;
-    for (int r = 0; r < n; ++r) c += from + r * (to - from) / n == i;
-    return c;
-}
-
 // W8A8 fp8 (F8): a fragment of v_mfma_scale_f32_16x16x128_f8f6f4 is 32 k-bytes per lane (two 16-B chunks)
 typedef int lg_i32x8 __attribute__((ext_vector_type(8)));
 __device__ __forceinline__ f32x4 lg_mma(const bf16x8& a, const bf16x8& b, f32x4 c) {
@@ -154,12 +92,6 @@ __device__ __forceinline__ f32x4 lg_mma(const bf16x8& a, const bf16x8& b, f32x4 
 // block-scaled form fed the unit MX exponent (127 = 2^0): the per-token / per-channel scales go in the epilogue
 __device__ __forceinline__ f32x4 lg_mma(const lg_i32x8& a, const lg_i32x8& b, f32x4 c) {
     return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 127, 0, 127);
-}
-
-// f(std::integral_constant<int, I>{}) for every I of the sequence, in order (a compile-time unrolled loop)
-template <typename F, int... Is>
-__device__ __forceinline__ void lg_static_for(F&& f, std::integer_sequence<int, Is...>) {
-    (f(std::integral_constant<int, Is>{}), ...);
 }
 
 // 64-B-row chunk swizzle (the 16x16x32 fragment reads of a 16-row block land on 16 distinct 16-B slots)
@@ -555,20 +487,6 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
             }
         };
         if constexpr (HB) {
-            // A slab keeps its LDS buffer only until its second k-step's fragments are in registers, so the two buffers hold
-            // nearly two slabs in flight.  Slab j, slot i of 128 MFMAs (k-step i / 64), issue order pinned:
-            //   [0, RD1)     : the 16 fragment reads of slab j, k-step 1 (set 1)
-            //   REL          : lgkmcnt(0) + barrier: every wave holds both k-steps of slab j, its buffer is free
-            //   [REL, PEND)  : the wave's 16 LDS-DMA pieces of slab j+2, evenly, x then W
-            //   LAND         : vmcnt(16) (this wave's pieces of slab j+1, issued one slab ago, have landed; those of slab j+2 stay
-            //                  in flight) + barrier: slab j+1 is readable
-            //   [LAND, RD0)  : the 16 fragment reads of slab j+1, k-step 0 (set 0)
-            // What was measured, us at 8192^3 / 5952 x 4096 x 14336 / 1024 x 128256 x 4096: the pieces want to be spread over all the
-            // slots that the dependences leave: over 32 slots 820 / 643 / 891, 48 788 / 617 / 856, 64 751 / 584 / 819, 88 729 / 559 / 797
-            // (with three more instructions a piece than now; REL from 20 to 56 and LAND from 96 to 112 matter little); a piece as
-            // two instructions on either side of an MFMA instead of three before it: 698 / 559 / 764.
-            constexpr int MFK = NT * MT;
-            constexpr int RD1 = 16, REL = 20, PEND = 108, LAND = 112, RD0 = 128;
             static_assert(NPW == 8 && NPX == 8, "HB: 8 W + 8 x pieces per wave and slab");
             const int pstride = RPI * K * ES;  // source bytes between a wave's consecutive pieces of one operand
             // the accumulators live in AGPRs across the whole loop: pinned at both ends, so the epilogue's VGPR use
@@ -616,7 +534,7 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
                 // 64-deep k-steps of 16 v_mfma_scale_f32_32x32x64_f8f6f4 (4 W x 4 x blocks of 32), and the 32x32x16 form.
                 // A fragment is two ds_read_b128: 8 per group here.
                 constexpr int MK = (NT / 2) * (MT / 2);
-                constexpr int RD1 = 4, REL = 6, PEND = 26, LAND = 28, RD0 = 32;
+                constexpr int RD1 = 8, REL = 10, PEND = 27, LAND = 27, RD0 = 32;
                 static_assert(MK == 16 && RD1 < REL && REL + 16 <= PEND && PEND <= LAND && RD0 <= 2 * MK, "HB schedule, 32 slots");
                 auto half = [&](auto PC, int j) {
                     constexpr int P = decltype(PC)::value;  // slab j in buffer P, slab j+1 in 1 - P
@@ -674,7 +592,6 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
                     if (j + 1 < NS) half(std::integral_constant<int, 1>{}, j + 1);
                 }
             } else {
-                static_assert(RD1 < REL && REL + 16 <= PEND && PEND <= LAND && RD0 <= 2 * MFK, "HB schedule");
                 // unrolled by two slabs, so a half's LDS buffer is known at compile time: fragment reads are a per-lane base
                 // (buffer x operand x k-step) + an immediate
                 const unsigned char* rbw[2][2];
@@ -686,51 +603,8 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
                         rbw[p][kk] = smem + p * STAGE + wrow0[0] * RB + loff[kk];
                         rbx[p][kk] = smem + p * STAGE + WIMG + xrow0 * RB + loff[kk];
                     }
-                auto half = [&](auto PC, int j) {
-                    constexpr int P = decltype(PC)::value;  // slab j lives in buffer P, slab j+1 in 1 - P
-                    advance(j);
-                    auto slot = [&](auto IC) {
-                        constexpr int i = decltype(IC)::value;
-                        if constexpr (i == REL) {
-                            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), visible to hipcc's wait bookkeeping
-                            lg_bar();
-                        }
-                        if constexpr (i == LAND) {
-                            lg_vmcnt<NPER>();
-                            lg_bar();
-                        }
-                        constexpr int piece = hb_piece(i, REL, PEND, NPER);
-                        if constexpr (piece >= 0) dst(PC, std::integral_constant<int, piece>{});
-                        constexpr int ii = i % MFK;
-                        constexpr bool SQ = VAR == 5 && i < MFK;  // (k-step 0 only: k-step 1's reads land early)
-                        constexpr int s = SQ ? hb_sq_s(ii) : ii / MT, t = SQ ? hb_sq_t(ii) : ii % MT;
-                        if constexpr (i < MFK)
-                            acc[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa0[s], fb0[t], acc[s][t], 0, 0, 0);
-                        else
-                            acc[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa1[s], fb1[t], acc[s][t], 0, 0, 0);
-                        if constexpr (piece >= 0) go(std::integral_constant<int, piece>{});
-                        auto read = [&](auto RC, int p, int kk, bf16x8 (&fa)[NT], bf16x8 (&fb)[MT]) {
-                            constexpr int r = decltype(RC)::value;
-                            // set 0 of VAR 5: fa0, fb0, fb1, fa1, fb2, fa2, ...; else fa[0], fb[0..MT-1], fa[1..NT-1]
-                            constexpr bool isw = VAR == 5 ? hb_sq_isw(r) : r == 0 || r > MT;
-                            constexpr int b = VAR == 5 ? hb_sq_blk(r) : r == 0 ? 0 : r <= MT ? r - 1 : r - MT;
-                            if constexpr (isw)
-                                fa[b] = *reinterpret_cast<const bf16x8*>(rbw[p][kk] + hb_wrow(b, MODE == kSwiglu, WN) * RB);
-                            else
-                                fb[b] = *reinterpret_cast<const bf16x8*>(rbx[p][kk] + 16 * RB * b);
-                        };
-                        constexpr int r1 = hb_due(i, 0, RD1, NT + MT), r0 = hb_due(i, LAND, RD0, NT + MT);
-                        static_assert(hb_due_n(i, 0, RD1, NT + MT) <= 1 && hb_due_n(i, LAND, RD0, NT + MT) <= 1, "one read a slot");
-                        if constexpr (r1 >= 0) read(std::integral_constant<int, r1>{}, P, 1, fa1, fb1);
-                        if constexpr (r0 >= 0) read(std::integral_constant<int, r0>{}, 1 - P, 0, fa0, fb0);
-                        __builtin_amdgcn_sched_barrier(0);
-                    };
-                    lg_static_for(slot, std::make_integer_sequence<int, 2 * MFK>{});
-                };
-                for (int j = 0; j < NS; j += 2) {
-                    half(std::integral_constant<int, 0>{}, j);
-                    if (j + 1 < NS) half(std::integral_constant<int, 1>{}, j + 1);
-                }
+                slab_loop<VAR == 5>(acc, fa0, fb0, fa1, fb1, rbw, rbx, NS, dst, go, advance,
+                                    HbRow<MODE == kSwiglu, WN, RB>{});
             }
             pin_acc();
         }
