@@ -276,148 +276,85 @@ __global__ void __launch_bounds__(256, 2) moe_gemm_kernel(const uint16_t* __rest
     moe_store<ACT, C::NS, C::NM>(acc, y, row_item, m0 + 16 * C::NM * wm, tn * C::TN + C::TN / 2 * wn, N, lane, limit, slope, shift);
 }
 
-// The wave's 128 x 128 outputs of the 256 x 256 tile, through its own 32 KiB of LDS, so that a store instruction writes whole lines: 16
-// lanes a row (8 for a gated unit's 64 columns).  Registers as in moe_store; row r's 16-byte piece c lies at c ^ (r % pieces).
-template <int ACT>
-__device__ __forceinline__ void moe_store_staged(const f32x4 (&acc)[8][8], unsigned char* stg, uint16_t* __restrict__ y,
-                                                 const int32_t* __restrict__ row_item, int m0, int n0, int N, int lane, float limit,
-                                                 float slope, float shift) {
-    constexpr bool GLU = ACT == kActGlu;
-    constexpr int NCH = GLU ? 8 : 16, RPI = 64 / NCH, NK = 128 / RPI;   // pieces per row, rows per store, stores
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        const int r = 16 * t + (lane & 15);
-#pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            if (GLU && (s & 2)) continue;
-            const int col = GLU ? 32 * (s >> 2) + 16 * (s & 1) + 4 * (lane >> 4) : 16 * s + 4 * (lane >> 4);
-            u16x4 o;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float v = acc[s][t][i];
-                if constexpr (GLU) {
-                    // every 64 rows: blocks 0 and 1 are gate rows, 2 and 3 the up rows of the same outputs
-                    const float a = fminf(bf2f(f2bf(v)), limit);
-                    const float u = fminf(fmaxf(bf2f(f2bf(acc[s | 2][t][i])), -limit), limit);
-                    v = a * sigmoid_act<uint16_t>(slope * a) * (u + shift);
-                } else if constexpr (ACT >= 0) {
-                    v = act_apply(bf2f(f2bf(v)), ACT);
-                }
-                o[i] = f2bf(v);
-            }
-            *reinterpret_cast<u16x4*>(stg + r * (NCH * 16) + (((col >> 3) ^ (r % NCH)) << 4) + ((col >> 2) & 1) * 8) = o;
-        }
-    }
-    const int c = lane % NCH, ld = GLU ? N / 2 : N, n = (GLU ? n0 / 2 : n0) + 8 * c;
-    if (n >= ld) return;   // (the last tile may be half)
-#pragma unroll
-    for (int k0 = 0; k0 < NK; k0 += 8) {
-        u16x8 v[8];
-        int it[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int r = RPI * (k0 + k) + lane / NCH;
-            v[k] = *reinterpret_cast<const u16x8*>(stg + r * (NCH * 16) + ((c ^ (r % NCH)) << 4));
-            it[k] = row_item[m0 + r];
-        }
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-            if (it[k] >= 0) *reinterpret_cast<u16x8*>(y + (int64_t)(m0 + RPI * (k0 + k) + lane / NCH) * ld + n) = v[k];
-    }
-}
-
-// The 256 x 256 tile (x and one expert's weights below 4 and 2 GiB; weight rows past the end repeat the last one) on the slab loop
-// of chronos_slab.h: 4 waves of 128 x 128 outputs, the accumulators in the AGPRs.  Bound by the matrix cores and by the last, partly
-// filled round of tiles.
+// The 256 x 256 tile (x and one expert's weights below 4 and 2 GiB; weight rows past the end repeat the last one): a workgroup per CU walks
+// its tiles on the slab loop of chronos_slab.h.  Bound by the matrix cores and the padding of every expert's last tile.
+// Results through the wave's 4 KiB of LDS, 16 rows at a time, so that a store instruction writes whole lines: 16 lanes a row (8 for a
+// gated unit's 64 columns); registers as in moe_store, row r's 16-byte piece c at c ^ (r % pieces).
 template <bool GATHER, int ACT>
 __global__ void __launch_bounds__(256, 1) moe_gemm256_kernel(const uint16_t* __restrict__ x, uint32_t xbytes,
                                                              const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
                                                              const int32_t* __restrict__ meta, int maxTiles, int top, int N,
                                                              int K, float limit, float slope, float shift) {
-    constexpr int IMG = 256 * 128, STAGE = 2 * IMG;
+    constexpr bool GLU = ACT == kActGlu;
+    constexpr int RBY = GLU ? 128 : 256, NCH = RBY / 16, RPS = 64 / NCH, NK = 16 / RPS;   // bytes and pieces per row, rows per store
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-    const int nt = (N + 255) / 256, used = meta[0];
-    if ((int)blockIdx.x >= used * nt) return;
-    const int id = xcd_remap(blockIdx.x, used * nt);
-    const int tile = id / nt, tn = id - tile * nt;
-    const int e = meta[1 + tile];
+    const int nt = (N + 255) / 256;
     const int32_t* row_item = meta + 1 + maxTiles;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int m0 = tile * 256;
-    // wave w stages image rows 64 w .. 64 w + 63 of both operands in eight pieces of 8 rows
-    const int pr = lane >> 3, pc = (lane & 7) ^ pr;
-    uint32_t wvoff[8], xvoff[8];
+    const int wn = wave >> 1, wm = wave & 1, in = lane >> 3, pc = (lane & 7) ^ in;
+    auto off = [&](auto NMC, int id, int m, uint32_t (&wv)[8], auto& xv, const void*& wb) {
+        constexpr int NM = decltype(NMC)::value;
+        const int tile = id / nt, tn = id - tile * nt;
+        wb = w + (int64_t)__builtin_amdgcn_readfirstlane(meta[1 + tile]) * N * K;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        wvoff[i] = moe_weight_offset(tn, 2 * wave + (i >> 2), i & 3, lane, N, K);
-        uint32_t xr = m0 + 64 * wave + 8 * i + pr;
-        if constexpr (GATHER) {
-            const int it = row_item[xr];
-            xr = it < 0 ? 0 : it / top;  // padding rows read token 0 and are never stored
+        for (int i = 0; i < 8; ++i) wv[i] = moe_weight_offset(tn, 2 * wave + (i >> 2), i & 3, lane, N, K);
+#pragma unroll
+        for (int i = 0; i < NM; ++i) {
+            uint32_t xr = tile * 256 + m + 8 * (NM * wave + i) + in;
+            if constexpr (GATHER) {
+                const int it = row_item[xr];
+                xr = it < 0 ? 0 : it / top;  // padding rows read token 0 and are never stored
+            }
+            xv[i] = (xr * (uint32_t)K + pc * 8) * 2;
         }
-        xvoff[i] = (xr * (uint32_t)K + pc * 8) * 2;
-    }
-    const uint16_t* we = w + (int64_t)e * N * K;
-    const uint32_t lds0 = lds_offset(smem) + wave * 8192, wbytes = (uint32_t)N * K * 2;
-    const int KT = K / 64;
+    };
+    unsigned char* const stg = smem + kSlabRows + wave * 4096;
+    const int c = lane % NCH, rr = lane / NCH;
+    auto epi = [&](auto NMC, int id, int m, auto& acc) {
+        constexpr int NM = decltype(NMC)::value;
+        const int tile = id / nt, tn = id - tile * nt, m0 = tile * 256 + m + 16 * NM * wm;
+        const int ld = GLU ? N / 2 : N, n = (tn * 256 + 128 * wn) / (GLU ? 2 : 1) + 8 * c;
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+        for (int t = 0; t < NM; ++t) {
+            int it[NK];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int off = min(kt, KT - 1) * 128;
-            dma_1k_buf(we, wbytes, lds0 + kt * STAGE + i * 1024, wvoff[i], off);
-            dma_1k_buf(x, xbytes, lds0 + kt * STAGE + IMG + i * 1024, xvoff[i], off);
+            for (int k = 0; k < NK; ++k) it[k] = row_item[m0 + 16 * t + RPS * k + rr];
+            const int r = lane & 15;
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                if (GLU && (s & 2)) continue;
+                const int col = GLU ? 32 * (s >> 2) + 16 * (s & 1) + 4 * (lane >> 4) : 16 * s + 4 * (lane >> 4);
+                u16x4 o;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    float v = acc[s][t][i];
+                    if constexpr (GLU) {
+                        // every 64 rows: blocks 0 and 1 are gate rows, 2 and 3 the up rows of the same outputs
+                        const float a = fminf(bf2f(f2bf(v)), limit);
+                        const float u = fminf(fmaxf(bf2f(f2bf(acc[s | 2][t][i])), -limit), limit);
+                        v = a * sigmoid_act<uint16_t>(slope * a) * (u + shift);
+                    } else if constexpr (ACT >= 0) {
+                        v = act_apply(bf2f(f2bf(v)), ACT);
+                    }
+                    o[i] = f2bf(v);
+                }
+                *reinterpret_cast<u16x4*>(stg + r * RBY + (((col >> 3) ^ (r % NCH)) << 4) + ((col >> 2) & 1) * 8) = o;
+            }
+#pragma unroll
+            for (int s = 0; s < 8; ++s) acc[s][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            u16x8 v[NK];
+#pragma unroll
+            for (int k = 0; k < NK; ++k) {   // (a wave's LDS operations complete in order)
+                const int q = RPS * k + rr;
+                v[k] = *reinterpret_cast<const u16x8*>(stg + q * RBY + ((c ^ (q % NCH)) << 4));
+            }
+#pragma unroll
+            for (int k = 0; k < NK; ++k)
+                if (it[k] >= 0 && n < ld)   // (the last tile along N may be half)
+                    *reinterpret_cast<u16x8*>(y + (int64_t)(m0 + 16 * t + RPS * k + rr) * ld + n) = v[k];
         }
-    const int wn = wave >> 1, wm = wave & 1;
-    const int ln = lane & 15, g = lane >> 4;
-    const unsigned char *rbw[2][2], *rbx[2][2];   // (16-row blocks: the swizzle depends on ln only)
-#pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int ch = ((4 * h + g) ^ (ln & 7)) * 16;
-            rbw[p][h] = smem + p * STAGE + (128 * wn + ln) * 128 + ch;
-            rbx[p][h] = smem + p * STAGE + IMG + (128 * wm + ln) * 128 + ch;
-        }
-    f32x4 acc[8][8];
-#pragma unroll
-    for (int s = 0; s < 8; ++s)
-#pragma unroll
-        for (int t = 0; t < 8; ++t) acc[s][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    bf16x8 fa0[8], fb0[8], fa1[8], fb1[8];
-    lg_vmcnt<16>();
-    lg_bar();
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {   // (the order of the loop's own reads)
-        const int b = hb_sq_blk(r);
-        if (hb_sq_isw(r)) fa0[b] = *reinterpret_cast<const bf16x8*>(rbw[0][0] + 2048 * b);
-        else fb0[b] = *reinterpret_cast<const bf16x8*>(rbx[0][0] + 2048 * b);
-    }
-    auto pin = [&]() {
-#pragma unroll
-        for (int s = 0; s < 8; ++s)
-#pragma unroll
-            for (int t = 0; t < 8; ++t) asm volatile("" : "+a"(acc[s][t]));
     };
-    pin();
-    int off = 0;   // byte offset of the slab whose pieces are issued: every row has its own address, the slab's comes on top
-    auto advance = [&](int j) { off = min(j + 2, KT - 1) * 128; };
-    auto dst = [&](auto PC, auto IC) {
-        constexpr int P = decltype(PC)::value, p = decltype(IC)::value;
-        lg_dma_dst<P * STAGE + (p < 8 ? IMG : 0) + (p & 7) * 1024>(lds0);
-    };
-    auto go = [&](auto IC) {
-        constexpr int p = decltype(IC)::value;
-        if constexpr (p < 8) lg_dma_go(x, (int)xbytes, xvoff[p], off);
-        else lg_dma_go(we, (int)wbytes, wvoff[p - 8], off);
-    };
-    struct Row { constexpr int operator()(int b) const { return 2048 * b; } };
-    slab_loop<true>(acc, fa0, fb0, fa1, fb1, rbw, rbx, KT, dst, go, advance, Row{});
-    pin();
-    // the last pieces, which nobody reads, have landed everywhere before the images become the staging rows
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    lg_bar();
-    moe_store_staged<ACT>(acc, smem + wave * 32768, y, row_item, m0 + 128 * wm, tn * 256 + 128 * wn, N, lane, limit, slope, shift);
+    slab_run<false>(smem, meta[0] * nt, K / 64, x, (int)xbytes, (int)((uint32_t)N * K * 2), off, [](auto, int, int) {}, epi);
 }
 
 // An index of E and above is an identity expert (its output is the token itself) where the experts' layer has such
@@ -476,10 +413,10 @@ static void moe_gemm(const uint16_t* x, int64_t rows, const uint16_t* w, uint16_
                      float limit, float slope, float shift, hipStream_t s) {
     if constexpr (TM == 256) {
         const auto kern = hy::moe_gemm256_kernel<GATHER, ACT>;
-        constexpr int lds = 4 * 256 * 128;
+        constexpr int lds = kSlabLds;
         static const hipError_t once = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         (void)once;
-        kern<<<maxTiles * ((N + 255) / 256), 256, lds, s>>>(x, (uint32_t)(rows * K * 2), w, y, meta, maxTiles, top, N, K, limit, slope, shift);
+        kern<<<kSlabCUs, 256, lds, s>>>(x, (uint32_t)(rows * K * 2), w, y, meta, maxTiles, top, N, K, limit, slope, shift);
     } else {
         const auto kern = hy::moe_gemm_kernel<TM, GATHER, ACT>;
         constexpr int lds = hy::Tile<TM>::lds;

@@ -18,13 +18,14 @@ struct PPArgs {
     float eps;
     int gm;      // tile order: M-tiles per group (0 = every M-tile of a W panel consecutive); knob pp_gm
     int handoff;       // gemm_lg split-K slab hand-off (knob lg_handoff): -1 auto, 0 fences, 1 write-through
+    float limit, slope, shift;  // kPPGlu: min(g, limit) sigmoid(slope g) (clamp(u, -limit, limit) + shift)
     const float* xsc;  // gemm_lg F8 (W8A8 e4m3fn bytes in x / w): per-token scales [M]
     const float* wsc;  // ... and per-output-channel scales [N]
     int ablate;  // timing-only diagnostics (knob pp_ablate): 1 skip loop DMA, 2 skip LDS reads, 4 skip MFMA, 8 nt weights, 16/32 alias every W/x tile onto tile 0
 };
 
 // epilogue modes
-enum : int { kPPPlain = 0, kPPSwiglu = 1, kPPResid = 2 };
+enum : int { kPPPlain = 0, kPPSwiglu = 1, kPPResid = 2, kPPGlu = 3, kPPRelu2 = 4, kPPGelu = 5 };  // (3 on: gemm_slab only)
 constexpr int kPPConfigs = 12;
 int gemm_pp_bm(int cfg);  // x rows per tile
 int gemm_pp_bn(int cfg);  // W rows per tile
@@ -43,6 +44,8 @@ int gemm_lg_wn(int cfg);  // W rows per tile
 bool gemm_lg_splitk_ok(int cfg);  // false for the HB configs (VAR 4): no split-K path
 bool gemm_lg_ablations_built();  // the timing-only ablation ids 40-71 exist (CHRONOS_GEMM_ABLATIONS build)
 bool launch_gemm_lg(int cfg, int mode, bool normp, const PPArgs& a, hipStream_t st);
+// configs 88 / 92 without split-K, and the hybrid decoders' epilogues (csrc/kernels/gemm_slab.hip)
+bool launch_gemm_slab(int mode, bool normp, const PPArgs& a, hipStream_t st);
 // W8A8 fp8 configs of the same kernel (ring schedule, 128-deep stages; a.kts counts 128-deep units), own id space
 constexpr int kLGF8Configs = 5;
 int gemm_lg_f8_xm(int cfg);

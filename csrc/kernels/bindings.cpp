@@ -611,6 +611,36 @@ std::tuple<Tensor, Tensor> gemm_pp(const Tensor& x, const Tensor& w, int64_t mod
     return {y, part_out};
 }
 
+// The hybrid decoders' first feed-forward products with their activation in the epilogue (gemm_slab.hip), K % 64 == 0: mode 3 the gated
+// unit of w = [gate; up] [2F, K], F % 128 == 0, y [M, F]; 4 / 5 squared ReLU / GELU of x w^T, N % 4 == 0, y [M, N].
+Tensor gemm_act(const Tensor& x, const Tensor& w, int64_t mode, double limit, double slope, double shift) {
+    chk_bf16(x, "x");
+    chk_bf16(w, "w");
+    CHK(x.dim() == 2 && w.dim() == 2 && w.size(1) == x.size(1), "gemm_act: x [M, K], w [N, K]");
+    const int64_t K = x.size(1), M = x.size(0), N = w.size(0);
+    CHK(mode >= chronos::kPPGlu && mode <= chronos::kPPGelu, "gemm_act: mode");
+    CHK(M >= 1 && K >= 64 && K % 64 == 0 && K <= (1 << 20) && N >= 1 && (mode == chronos::kPPGlu ? N % 256 == 0 : N % 4 == 0), "gemm_act: sizes");
+    CHK((N + 256) * K * 2 < (1LL << 31) && (M + 256) * K * 2 < (1LL << 31), "gemm_act: operand > 2 GiB");
+    CHK(((reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr())) & 15) == 0, "gemm_act: alignment");
+    c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+    chronos::PPArgs a{};
+    a.x = bf(x);
+    a.w = bf(w);
+    a.M = (int)M;
+    a.N = (int)N;
+    a.K = (int)K;
+    a.F = (int)(N / 2);
+    a.splitk = 1;
+    a.gm = chronos::knob("pp_gm", 8);
+    a.limit = (float)limit;
+    a.slope = (float)slope;
+    a.shift = (float)shift;
+    Tensor y = at::empty({M, mode == chronos::kPPGlu ? N / 2 : N}, x.options());
+    a.y = bfm(y);
+    CHK(chronos::launch_gemm_slab((int)mode, false, a, cur_stream()), "gemm_act: launch");
+    return y;
+}
+
 // Skinny-M GEMM (gemm_skinny.hip), M <= 16 * MT of the config: same epilogues and tensors as gemm_pp; the kResid
 // partials are [M, N / (16 * RT)].
 std::tuple<Tensor, Tensor> gemm_skinny(const Tensor& x, const Tensor& w, int64_t mode, int64_t cfg, int64_t splitk,
@@ -832,6 +862,7 @@ TORCH_LIBRARY(chronos, m) {
     m.def("silu_mul(Tensor gate_up) -> Tensor");
     m.def("gemv(Tensor x, Tensor w, bool swiglu, Tensor? ws=None) -> Tensor");
     m.def("gemm(Tensor x, Tensor w, bool swiglu, int stages=3) -> Tensor");
+    m.def("gemm_act(Tensor x, Tensor w, int mode, float limit, float slope, float shift) -> Tensor");
     m.def("gemm_pp(Tensor x, Tensor w, int mode, int cfg, int splitk, Tensor? resid, Tensor? part_in, float eps, bool prio) -> (Tensor, Tensor)");
     m.def("gemm_skinny(Tensor x, Tensor w, int mode, int cfg, int splitk, Tensor? resid, Tensor? part_in, float eps) "
           "-> (Tensor, Tensor)");
@@ -874,6 +905,7 @@ TORCH_LIBRARY_IMPL(chronos, CUDA, m) {
     m.impl("silu_mul", &silu_mul);
     m.impl("gemv", &gemv);
     m.impl("gemm", &gemm);
+    m.impl("gemm_act", &gemm_act);
     m.impl("gemm_pp", &gemm_pp);
     m.impl("gemm_skinny", &gemm_skinny);
     m.impl("gemv_resid", &gemv_resid);

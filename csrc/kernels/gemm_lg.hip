@@ -77,12 +77,7 @@ __device__ __forceinline__ void lg_dma16_asm(const void* base, int bytes, uint32
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %3 offen lds"
                  ::"v"(voff), "s"(lg_rsrc(base, bytes)), "s"(lds), "s"(soff) : "memory");
 }
-// HB: image row of W fragment block s relative to block 0 (SwiGLU: gate blocks 0 .. 3, then the up blocks at WN / 2)
-constexpr int hb_wrow(int s, bool swiglu, int WN) { return swiglu ? (s < 4 ? 16 * s : WN / 2 + 16 * (s - 4)) : 16 * s; }
-template <bool SWIGLU, int WN, int RB> struct HbRow {
-    constexpr int operator()(int b) const { return hb_wrow(b, SWIGLU, WN) * RB; }
-};
-// ... of 32-row block S (F8HB)
+// HB: image row of W 32-row block S relative to block 0 (SwiGLU: gate blocks, then the up blocks at WN / 2)
 constexpr int hb_wrow32(int S, bool swiglu, int WN) { return swiglu ? (S < 2 ? 32 * S : WN / 2 + 32 * (S - 2)) : 32 * S; }
 // W8A8 fp8 (F8): a fragment of v_mfma_scale_f32_16x16x128_f8f6f4 is 32 k-bytes per lane (two 16-B chunks)
 typedef int lg_i32x8 __attribute__((ext_vector_type(8)));
@@ -603,8 +598,16 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
                         rbw[p][kk] = smem + p * STAGE + wrow0[0] * RB + loff[kk];
                         rbx[p][kk] = smem + p * STAGE + WIMG + xrow0 * RB + loff[kk];
                     }
-                slab_loop<VAR == 5>(acc, fa0, fb0, fa1, fb1, rbw, rbx, NS, dst, go, advance,
-                                    HbRow<MODE == kSwiglu, WN, RB>{});
+                auto half = [&](auto PC, int j) {
+                    constexpr int P = decltype(PC)::value;  // slab j lives in buffer P, slab j+1 in 1 - P
+                    advance(j);
+                    slab_step<8, true, SlabRow<MODE == kSwiglu>>(acc, fa0, fb0, fa1, fb1, rbw[P][1], rbx[P][1], rbw[1 - P][0],
+                                                                 rbx[1 - P][0], [&](auto IC) { dst(PC, IC); }, go);
+                };
+                for (int j = 0; j < NS; j += 2) {
+                    half(std::integral_constant<int, 0>{}, j);
+                    if (j + 1 < NS) half(std::integral_constant<int, 1>{}, j + 1);
+                }
             }
             pin_acc();
         }
@@ -1218,13 +1221,12 @@ void lg_launch(const PPArgs& a, hipStream_t st) {
     X(78, 128, 32, 128, 7, 2)      \
     X(79, 64, 32, 128, 12, 2)      \
     X(80, 256, 256, 128, 2, 4, 3)  \
-    X(88, 256, 256, 128, 2, 2, 4)  \
     X(91, 256, 256, 128, 2, 2, 6)  \
     X(92, 256, 256, 128, 2, 2, 5)
 
-// Ids 81 .. 94 name the HB kernels: 88 (81 .. 87, 89, 90: the same kernel), 92 with the square order (93, 94), 91 on 32x32x16 MFMAs
+// Ids 81 .. 94 but 91 (on 32x32x16 MFMAs) name one kernel, gemm_slab.hip and, with a split-K, 92 here
 constexpr int lg_id(int cfg) {
-    return cfg < 81 || cfg > 94 || cfg == 91 ? cfg : cfg >= 92 ? 92 : 88;
+    return cfg < 81 || cfg > 94 || cfg == 91 ? cfg : 92;
 }
 
 template <int MODE, bool NORMP>
@@ -1349,6 +1351,7 @@ bool launch_gemm_lg_f8(int cfg, bool swiglu, const PPArgs& a, hipStream_t st) {
 
 bool launch_gemm_lg(int cfg, int mode, bool normp, const PPArgs& a, hipStream_t st) {
     if (a.M == 0) return true;
+    if (lg_id(cfg) == 92 && a.splitk == 1) return launch_gemm_slab(mode, normp, a, st);
     if (mode == kResid) return normp ? false : lg_mode<kResid, false>(cfg, a, st);
     if (mode == kSwiglu) return normp ? lg_mode<kSwiglu, true>(cfg, a, st) : lg_mode<kSwiglu, false>(cfg, a, st);
     return normp ? lg_mode<kPlain, true>(cfg, a, st) : lg_mode<kPlain, false>(cfg, a, st);

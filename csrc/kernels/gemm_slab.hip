@@ -1,0 +1,202 @@
+// gemm_slab.hip — projections of many rows: y[M, N] = x[M, K] W[N, K]^T in bfloat16 with float32 sums, 256 x 256 tiles on the
+// slab loop of chronos_slab.h.  A workgroup per CU walks its tiles; the slab pipeline runs on from one tile into the next, and where the
+// last round would leave half of the CUs idle its tiles are halved.  Configs 88 and 92 of the projection family (gemm_lg.hip has their split-K form).
+//
+// Epilogues, through 4 KiB of LDS per wave so that every store is 16 bytes of a whole line: plain; activation (squared ReLU, GELU); gated
+// units over W = [gate; up], of Llama (SwiGLU, roundings of the unfused form kept) and of the hybrid decoders (clamped, any slope and shift);
+// the new residual stream with its RMSNorm partials.  NORMP: the folded input RMSNorm as a scale per row.
+//
+// Bound by the matrix cores (a slab is 2048 of their cycles and takes 2200) and by the last round of tiles.
+// One workgroup per tile -> this, us: 8192 x 3648 x 2048 95.8 -> 93.0; 8192 x 6144 x 2048 157 -> 146 (3 rounds); 8192 x 2560 x 1024 (1.25
+// rounds) 52 -> 43; 8192 x 4096 x 4096 190 -> 179; a Llama-3 8B prefill of 5952 tokens, four layers, whole 8604 -> 7986.
+#include "chronos_act.h"
+#include "chronos_gemm.h"
+#include "chronos_hip.h"
+#include "chronos_slab.h"
+
+namespace chronos {
+namespace {
+
+// sum over the 16 lanes of a DPP row, in every lane
+__device__ __forceinline__ float row_sum16(float v) {
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xf, 0xf, false));
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x124, 0xf, 0xf, false));
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x122, 0xf, 0xf, false));
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x121, 0xf, 0xf, false));
+    return v;
+}
+
+template <int MODE, bool NORMP>
+__global__ void __launch_bounds__(256, 1) gemm_slab_kernel(PPArgs a) {
+    constexpr bool PAIR = MODE == kPPSwiglu || MODE == kPPGlu;
+    constexpr int OC = PAIR ? 64 : 128, RBY = 2 * OC, NCH = RBY / 16, RPS = 64 / NCH, NK = 16 / RPS;   // a wave's columns, bytes and
+    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];                            // pieces per row; rows per store
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wn = wave >> 1, wm = wave & 1, in = lane >> 3, piece = ((lane & 7) ^ in) * 8;
+    const int mt = (a.M + 255) / 256, nt = PAIR ? a.F / 128 : (a.N + 255) / 256;
+    // tiles in groups of gm along x, so that what an XCD runs at a time shares rows of both operands in its L2
+    auto where = [&](int tile, int& tm, int& tn) {
+        if (a.gm > 0 && mt > a.gm) {
+            const int per = a.gm * nt, grp = tile / per, r = tile - grp * per, gsz = min(a.gm, mt - grp * a.gm);
+            tm = grp * a.gm + r % gsz;
+            tn = r / gsz;
+        } else {
+            tm = tile % mt;
+            tn = tile / mt;
+        }
+    };
+    auto off = [&](auto NMC, int tile, int m, uint32_t (&wv)[8], auto& xv, const void*& wb) {
+        constexpr int NM = decltype(NMC)::value;
+        int tm, tn;
+        where(tile, tm, tn);
+        wb = a.w;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int r = 64 * wave + 8 * i + in;
+            const int row = !PAIR ? tn * 256 + r : wave < 2 ? tn * 128 + r : a.F + tn * 128 + r - 128;
+            wv[i] = ((uint32_t)row * (uint32_t)a.K + piece) * 2;
+        }
+#pragma unroll
+        for (int i = 0; i < NM; ++i) xv[i] = ((uint32_t)(tm * 256 + m + 8 * (NM * wave + i) + in) * (uint32_t)a.K + piece) * 2;
+    };
+    // NORMP: a lane sums its row's partials; two buffers in turn (a tile's slabs, with their barriers, lie between a buffer's
+    // writers and its readers, and between those and the next writers)
+    float* inv = reinterpret_cast<float*>(smem + kSlabLds) + 256;
+    auto scales = [&](auto NMC, int tile, int m) {
+        if constexpr (NORMP) {
+            constexpr int RPW = 8 * decltype(NMC)::value;   // rows per wave
+            int tm, tn;
+            where(tile, tm, tn);
+            const int row = RPW * wave + (lane & (RPW - 1));
+            const float* p = a.part_in + (int64_t)min(tm * 256 + m + row, a.M - 1) * a.nparts_in;
+            f32x4 t = {0.f, 0.f, 0.f, 0.f};
+            int i = 0;
+            if ((a.nparts_in & 3) == 0) {
+#pragma unroll 1
+                for (; i + 32 <= a.nparts_in; i += 32) {
+                    f32x4 q[8];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) q[k] = *reinterpret_cast<const f32x4*>(p + i + 4 * k);
+                    t += ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7]));
+                }
+            }
+            float ss = (t[0] + t[1]) + (t[2] + t[3]);
+#pragma unroll 1
+            for (; i < a.nparts_in; ++i) ss += p[i];
+            inv = reinterpret_cast<float*>(smem + kSlabLds) + (inv == reinterpret_cast<float*>(smem + kSlabLds) ? 256 : 0);
+            inv[row] = rsqrtf(ss / (float)a.K + a.eps);
+        }
+    };
+    unsigned char* const stg = smem + kSlabRows + wave * 4096;
+    const int c = lane % NCH, rr = lane / NCH;   // store phase: the lane's piece, its row within the RPS of an instruction
+    auto epi = [&](auto NMC, int tile, int m, auto& acc) {
+        constexpr int NM = decltype(NMC)::value;
+        int tm, tn;
+        where(tile, tm, tn);
+        const int m0 = tm * 256 + m + 16 * NM * wm;                      // the wave's first row
+        const int ld = PAIR ? a.F : a.N, n = (PAIR ? tn * 128 : tn * 256) + OC * wn + 8 * c;
+        u16x8 rv[MODE == kPPResid ? NK : 1];
+        auto resid = [&](int t) {
+            if constexpr (MODE == kPPResid) {
+#pragma unroll
+                for (int k = 0; k < NK; ++k)
+                    rv[k] = *reinterpret_cast<const u16x8*>(a.resid + (int64_t)min(m0 + 16 * t + RPS * k + rr, a.M - 1) * ld + n);
+            }
+        };
+        resid(0);
+#pragma unroll
+        for (int t = 0; t < NM; ++t) {
+            // 16 rows at a time; accumulator (s, t): row 16 t + lane % 16, columns 16 s + 4 (lane / 16) .. + 3.  Row r's piece p lies at
+            // p ^ (r % NCH)
+            const int r = lane & 15;
+            float sc = 1.f;
+            if constexpr (NORMP) sc = inv[16 * NM * wm + 16 * t + r];
+#pragma unroll
+            for (int s = 0; s < (PAIR ? 4 : 8); ++s) {
+                const int col = 16 * s + 4 * (lane >> 4);
+                u16x4 o;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float v = acc[s][t][i] * sc;
+                    if constexpr (MODE == kPPSwiglu) {
+                        const float gv = bf2f(f2bf(v));
+                        const float sg = bf2f(f2bf(gv / (1.f + __expf(-gv))));
+                        o[i] = f2bf(sg * bf2f(f2bf(acc[s + 4][t][i] * sc)));
+                    } else if constexpr (MODE == kPPGlu) {
+                        const float gv = fminf(v, a.limit), u = fminf(fmaxf(acc[s + 4][t][i] * sc, -a.limit), a.limit);
+                        o[i] = f2bf(gv * hy::sigmoid_act<uint16_t>(a.slope * gv) * (u + a.shift));
+                    } else if constexpr (MODE == kPPRelu2 || MODE == kPPGelu) {
+                        o[i] = f2bf(hy::act_apply(v, MODE == kPPRelu2 ? hy::kActRelu2 : hy::kActGelu));
+                    } else {
+                        o[i] = f2bf(v);
+                    }
+                }
+                *reinterpret_cast<u16x4*>(stg + r * RBY + (((col >> 3) ^ (r % NCH)) << 4) + ((col >> 2) & 1) * 8) = o;
+            }
+#pragma unroll
+            for (int s = 0; s < 8; ++s) acc[s][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            u16x8 v[NK];
+#pragma unroll
+            for (int k = 0; k < NK; ++k) {   // (a wave's LDS operations complete in order)
+                const int q = RPS * k + rr;
+                v[k] = *reinterpret_cast<const u16x8*>(stg + q * RBY + ((c ^ (q % NCH)) << 4));
+            }
+            float ss[NK];
+            if constexpr (MODE == kPPResid) {
+#pragma unroll
+                for (int k = 0; k < NK; ++k) {
+                    u16x8 o;
+                    ss[k] = 0.f;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        const float y = bf2f(f2bf(bf2f(v[k][i]) + bf2f(rv[k][i])));
+                        o[i] = f2bf(y);
+                        ss[k] += y * y;
+                    }
+                    v[k] = o;
+                    ss[k] = row_sum16(ss[k]);
+                }
+                if (t + 1 < NM) resid(t + 1);
+            }
+#pragma unroll
+            for (int k = 0; k < NK; ++k) {
+                const int row = m0 + 16 * t + RPS * k + rr;
+                if (row >= a.M) continue;
+                uint16_t* y = a.y + (int64_t)row * ld + n;
+                if (PAIR || MODE == kPPResid || n + 8 <= a.N) *reinterpret_cast<u16x8*>(y) = v[k];
+                else if (n < a.N) *reinterpret_cast<u16x4*>(y) = u16x4{v[k][0], v[k][1], v[k][2], v[k][3]};   // (N % 4 == 0)
+                if constexpr (MODE == kPPResid)
+                    if (c == 0) a.part_out[(int64_t)row * (a.N / 128) + tn * 2 + wn] = ss[k];
+            }
+        }
+    };
+    slab_run<PAIR>(smem, mt * nt, a.K / 64, a.x, (int)((int64_t)a.M * a.K * 2), (int)((int64_t)a.N * a.K * 2), off, scales, epi);
+}
+
+template <int MODE, bool NORMP>
+void slab_launch(const PPArgs& a, hipStream_t st) {
+    constexpr int lds = kSlabLds + (NORMP ? 2048 : 0);
+    const auto kern = gemm_slab_kernel<MODE, NORMP>;
+    static const hipError_t once = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    (void)once;
+    const bool pair = MODE == kPPSwiglu || MODE == kPPGlu;
+    const int tiles = (a.M + 255) / 256 * (pair ? a.F / 128 : (a.N + 255) / 256);
+    hipLaunchKernelGGL(kern, dim3(slab_grid(tiles)), dim3(256), lds, st, a);
+}
+
+}  // namespace
+
+bool launch_gemm_slab(int mode, bool normp, const PPArgs& a, hipStream_t st) {
+    if (a.splitk != 1 || (normp && mode != kPPPlain && mode != kPPSwiglu)) return false;
+    switch (mode) {
+        case kPPPlain: normp ? slab_launch<kPPPlain, true>(a, st) : slab_launch<kPPPlain, false>(a, st); return true;
+        case kPPSwiglu: normp ? slab_launch<kPPSwiglu, true>(a, st) : slab_launch<kPPSwiglu, false>(a, st); return true;
+        case kPPResid: slab_launch<kPPResid, false>(a, st); return true;
+        case kPPGlu: slab_launch<kPPGlu, false>(a, st); return true;
+        case kPPRelu2: slab_launch<kPPRelu2, false>(a, st); return true;
+        case kPPGelu: slab_launch<kPPGelu, false>(a, st); return true;
+        default: return false;
+    }
+}
+
+}  // namespace chronos

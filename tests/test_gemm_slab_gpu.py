@@ -1,0 +1,56 @@
+"""gemm_slab.hip: a workgroup's walk over its tiles (whole rounds, halves in the last one, one slab per tile), partial tiles in both
+directions, and the epilogues of the hybrid decoders against float32."""
+import pytest
+import torch
+
+DEV = "cuda"
+pytestmark = pytest.mark.gpu
+
+
+def _operands(m, n, k, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    x = torch.randn(m, k, device=DEV, generator=g).to(torch.bfloat16)
+    return x, (torch.randn(n, k, device=DEV, generator=g) * k ** -0.5).to(torch.bfloat16)
+
+
+def _close(y, ref):
+    """One rounding to bfloat16 (2^-9 of the value) on top of float32 sums, whose order may move a value by 2^-20 of the operands."""
+    err = (y.float() - ref).abs() - ref.abs() * 2.0 ** -8
+    assert err.max().item() < 1e-4 * max(1.0, ref.abs().max().item())
+
+
+@pytest.mark.parametrize("tiles", [1, 127, 128, 129, 255, 256, 257, 384, 385, 513])
+@pytest.mark.parametrize("k", [64, 192])
+def test_every_tile_once(tiles, k):
+    from chronos import ops
+    from chronos.ops import gemm as G
+
+    ops.load()
+    m = 256 * tiles - 5     # one column of W tiles, the last x tile partial
+    x, w = _operands(m, 256, k, tiles + k)
+    y, _ = G.pp_gemm(x, w, G.PP_PLAIN, (88, 1))
+    _close(y, x.float() @ w.float().t())
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 256, 64), (300, 512, 128), (2446, 5632, 192), (4100, 20224, 64)])
+@pytest.mark.parametrize("limit,slope,shift", [(float("inf"), 1.0, 0.0), (0.75, 1.702, 1.0)])
+def test_gated_unit(m, n, k, limit, slope, shift):
+    from chronos import ops
+
+    ops.load()
+    x, w = _operands(m, n, k, m + n)
+    h = x.float() @ w.float().t()
+    g, u = h[:, : n // 2].clamp(max=limit), h[:, n // 2:].clamp(-limit, limit)
+    _close(torch.ops.chronos.gemm_act(x, w, 3, limit, slope, shift), g * torch.sigmoid(slope * g) * (u + shift))
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 4, 64), (257, 1032, 128), (4100, 8196, 64)])
+@pytest.mark.parametrize("mode", [4, 5])
+def test_activation(m, n, k, mode):
+    from chronos import ops
+
+    ops.load()
+    x, w = _operands(m, n, k, m + n + mode)
+    h = x.float() @ w.float().t()
+    ref = h.relu() ** 2 if mode == 4 else torch.nn.functional.gelu(h)
+    _close(torch.ops.chronos.gemm_act(x, w, mode, 0.0, 0.0, 0.0), ref)
