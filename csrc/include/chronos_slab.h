@@ -266,7 +266,7 @@ __device__ __forceinline__ void slab_run(unsigned char* smem, int T, int NS, con
             epi(NMC, tile_of(v), m_of(v), acc);
             if (u >= count) break;
             rows(NMC, tile_of(u), m_of(u));
-            after(u + G);
+            if (NS > 1) after(u + G);   // (with one slab a tile next() is a tile further already)
             v = u;
         }
         // the last pieces have landed and the last reads are done everywhere before the buffers are filled anew or given back

@@ -19,7 +19,7 @@ def _close(y, ref):
     assert err.max().item() < 1e-4 * max(1.0, ref.abs().max().item())
 
 
-@pytest.mark.parametrize("tiles", [1, 127, 128, 129, 255, 256, 257, 384, 385, 513])
+@pytest.mark.parametrize("tiles", [1, 127, 128, 129, 255, 256, 257, 384, 385, 513, 800, 1100])
 @pytest.mark.parametrize("k", [64, 192])
 def test_every_tile_once(tiles, k):
     from chronos import ops
