@@ -1039,8 +1039,7 @@ def mix_gla(model, li: int, spec: GLASpec, w: dict, h, meta: StepMeta, cache: Hy
 
 
 def ff_glu(model, spec: GluFFSpec, w: dict, h):
-    return hops.matmul(hops.glu(hops.matmul(h, w["w_gu"]), spec.limit, spec.slope, spec.shift, model.act_dtype),
-                       w["w_down"])
+    return hops.matmul(hops.matmul_glu(h, w["w_gu"], spec.limit, spec.slope, spec.shift, model.act_dtype), w["w_down"])
 
 
 def ff_moe_glu(model, spec: MoEGluSpec, w: dict, h):
@@ -1057,13 +1056,12 @@ def ff_moe_group_glu(model, spec: MoEGroupGluSpec, w: dict, h):
                          bool(w.get("gu_tiled", False)))
     if not spec.shared_ff:
         return y
-    ys = hops.matmul(hops.glu(hops.matmul(h, w["ws_gu"]), spec.limit, spec.slope, spec.shift, model.act_dtype),
-                     w["ws_down"])
+    ys = hops.matmul(hops.matmul_glu(h, w["ws_gu"], spec.limit, spec.slope, spec.shift, model.act_dtype), w["ws_down"])
     return y, ys, hops.rowdot(h, w["ws_gate"])
 
 
 def ff_dense(model, spec: DenseFFSpec, w: dict, h):
-    return hops.matmul(hops.act_inplace(hops.matmul(h, w["w_up"]), spec.act), w["w_down"])
+    return hops.matmul(hops.matmul_act(h, w["w_up"], spec.act), w["w_down"])
 
 
 def ff_poly(model, spec: PolyFFSpec, w: dict, h):
@@ -1078,7 +1076,7 @@ def ff_moe(model, spec: MoEFFSpec, w: dict, h):
     y = hops.moe_ffn(h, idx, wt, w["w_up"], w["w_down"], spec.act, model.act_dtype)
     if not spec.shared_ff:
         return y
-    return y, hops.matmul(hops.act_inplace(hops.matmul(h, w["ws_up"]), spec.act), w["ws_down"])
+    return y, hops.matmul(hops.matmul_act(h, w["ws_up"], spec.act), w["ws_down"])
 
 
 MIXERS = {"mlstm": (mix_mlstm, pack_mlstm), "latent_attention": (mix_latent_attention, pack_latent),

@@ -12,7 +12,8 @@ Routing is by measured shape:
   with the kernel, tile config and split-K of the measured plan (``gemm_plan.json``: per (N, K, epilogue) the best
   by M range, from ``scripts/tune_gemm_pp.py`` on one MI355X, random operands, cold weights; plan cfg >= 100 is
   skinny config cfg - 100);
-* shapes that the plan does not list: up to 64 rows ``few_rows_plan``, where its measured range says that it wins;
+* shapes that the plan does not list: up to 64 rows ``few_rows_plan``, from 128 on ``many_rows_plan``, where their measured ranges say that
+  they win;
 * hipBLASLt (torch.matmul) only where the plan records that the library wins by more than 3 % (the "plain library
   GEMM" rule), for unlisted shapes outside that range, or for shapes the kernel does not take (K % 64, N % 4).  CHRONOS_PP=lib|own|auto forces a side.
 """
@@ -241,6 +242,84 @@ def few_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     return out
 
 
+# Many rows, shapes that the plan does not list: what a launch takes in us, fitted on a grid of M = 65 .. 8192, N = 512 .. 16384, K = 512 ..
+# 8192 (rms error 10 %, 18 % for 88).  88 (gemm_slab.hip): constant, per half tile of the last round, per 64-deep step of a round of
+# 256 x 256 tiles and of the halves, per M of results, per M of weights; 19 and 32 (128 x rows by 128 and 64 W rows): constant, per round of
+# 256 tiles, per 256 tiles, per 64-deep step of these two, per M of weights.  Of all tile configs these three suffice: the pick is within
+# 1 % of the fastest of eight on average.
+_MANY_88 = (2.6, 1.9, 1.17, 0.55, 0.52, 0.29)
+_MANY_TILES = {19: (128, 2.9, 1.9, 1.2, 0.294, 0.15, 0.16), 32: (64, 2.7, 1.45, 0.46, 0.224, 0.083, 0.13)}
+# ... and with an activation in 88's epilogue, the gated unit and the others; the same activation as a pass of its own: constant, per M of
+# its inputs
+_MANY_ACT = {True: ((2.1, 4.7, 1.22, 0.57, 0.41, 0.16), 4.45, (2.9, 0.44)), False: ((3.3, 2.2, 1.22, 0.55, 0.51, 0.17), 0.0, (2.8, 0.39))}
+MANY_MIN = 128
+
+
+def _many_slab(c, per_round: float, m: int, n: int, k: int) -> float:
+    t = -(-m // 256) * -(-n // 256)
+    half = 0 < t % 256 <= 128
+    rounds = t // 256 if half else -(-t // 256)
+    return c[0] + per_round * rounds + (c[1] + c[3] * (k // 64)) * half + c[2] * rounds * (k // 64) + (c[4] * m + c[5] * k) * n * 1e-6
+
+
+def _many_best(m: int, n: int, k: int) -> tuple[float, int]:
+    best = (_many_slab(_MANY_88, 0.0, m, n, k), 88)
+    for cfg, (bn, c0, c1, c2, c3, c4, c5) in _MANY_TILES.items():
+        t = -(-m // 128) * -(-n // bn)
+        steps = k // 64
+        best = min(best, (c0 + -(-t // 256) * (c1 + c3 * steps) + t / 256 * (c2 + c4 * steps) + c5 * n * k * 1e-6, cfg))
+    return best
+
+
+def _many_fits(m: int, n: int, k: int) -> bool:
+    return k % 64 == 0 and 0 < k <= 1 << 20 and n > 0 and n % 4 == 0 and (max(m, n) + 384) * k < 1 << 30
+
+
+def many_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
+    """(config, 1) of the hand-written GEMM for at least 128 rows of a shape that no plan lists, or None (the library): from 64 tiles of 128 x rows
+    by 64 W rows on, and K / 16 of them (below, K would have to be split for enough workgroups).  There, on the grid of _MANY_88: 1.13 times as
+    fast as the library on average (340 shapes; 38 slower by more than 3 %, the worst by 14 %: one round that 256 x 256 tiles fill to
+    between one and two thirds), below the line 0.9 times.  A library call also costs the host 22 us, this 7.  Rows count in 128s, so that a server's
+    steps of any size find their plan again."""
+    if PP_MODE != "auto":
+        return None
+    m = -(-m // 128) * 128
+    key = (m, n, k, -2)
+    hit = _plan_cache.get(key, False)
+    if hit is not False:
+        return hit
+    tiles = m // 128 * -(-n // 64)
+    out = None
+    if _many_fits(m, n, k) and tiles >= max(64, k // 16) and (n, k, PP_PLAIN) not in _plan_file():
+        out = (_many_best(m, n, k)[1], 1)
+    _plan_cache[key] = out
+    return out
+
+
+def product_act(x: torch.Tensor, w: torch.Tensor, mode: int, limit: float = 0.0, slope: float = 0.0, shift: float = 0.0) -> Optional[torch.Tensor]:
+    """x @ w.T with an activation in the epilogue (mode as in torch.ops.chronos.gemm_act: 3 a gated unit of w = [gate; up], 4 squared ReLU, 5
+    GELU), or None where that does not pay: where the best product (many_rows_plan's or, below it, as if it were) and a pass of its own are
+    faster by their models.  On the grid of _MANY_88: gated units 1.13 times as fast (189 shapes; the worst 0.94), the others 1.16
+    (196; 0.95)."""
+    m, (n, k) = x.numel() // max(1, x.shape[-1]), w.shape
+    if m < MANY_MIN or PP_MODE != "auto" or x.dim() != 2 or not _plain_rows(x, w):
+        return None
+    glu = mode == 3
+    rows = -(-m // 128) * 128
+    key = (rows, n, k, -3 if glu else -4)
+    pays = _plan_cache.get(key)
+    if pays is None:
+        c, per_round, own = _MANY_ACT[glu]
+        pays = _many_fits(rows, n, k) and (not glu or n % 256 == 0)
+        pays = pays and _many_slab(c, per_round, rows, n, k) < _many_best(rows, n, k)[0] + own[0] + own[1] * rows * n * 1e-6
+        _plan_cache[key] = pays
+    if not pays:
+        return None
+    from . import _k
+
+    return _k().gemm_act(x, w, mode, limit, slope, shift)
+
+
 def _plain_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Operands that the kernels take as they lie, and nothing that has to see the product (gradients, transforms,
     autocast, subclasses)."""
@@ -456,7 +535,9 @@ def linear(x, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tens
     if x.is_cuda:
         m, k = x.numel() // x.shape[-1], x.shape[-1]
         n = w.shape[0]
-        few = few_rows_plan(m, n, k) if out is None and 0 < m <= 64 and _plain_rows(x, w) else None
+        few = None
+        if out is None and (0 < m <= 64 or m >= MANY_MIN) and _plain_rows(x, w):
+            few = few_rows_plan(m, n, k) if m <= 64 else many_rows_plan(m, n, k)
         if few is None and gemv_ok(m, n, k):
             return _gemv(x, w)
         for pred, fn in _custom:

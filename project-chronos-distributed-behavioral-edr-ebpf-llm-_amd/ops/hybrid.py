@@ -96,6 +96,28 @@ def act_inplace(x, kind: int):
     return ref.act_inplace(x, kind)
 
 
+def matmul_act(x, w, kind: int):
+    """act_inplace(x @ w.T, kind), in the product's epilogue where that is faster (the activation then reads the unrounded product)."""
+    if _gpu(x) and x.dtype == torch.bfloat16 and kind in (ACT_RELU2, ACT_GELU):
+        from .gemm import product_act
+
+        y = product_act(x, w, 4 if kind == ACT_RELU2 else 5)
+        if y is not None:
+            return y
+    return act_inplace(matmul(x, w), kind)
+
+
+def matmul_glu(x, w, limit: float, slope: float, shift: float, act_dtype):
+    """glu(x @ w.T, ...), w = [gate; up], in the product's epilogue where that is faster (the unit then reads the unrounded product)."""
+    if _gpu(x) and x.dtype == torch.bfloat16 and act_dtype == torch.bfloat16:
+        from .gemm import product_act
+
+        y = product_act(x, w, 3, limit, slope, shift)
+        if y is not None:
+            return y
+    return glu(matmul(x, w), limit, slope, shift, act_dtype)
+
+
 def mlstm_scan(proj, gate_pre, q_start, pos0, slots, S, n, m, H: int, D: int, Dv: int, cap: float, max_q: int = 0):
     """``max_q``: the most tokens any sequence brings in this step (picks the kernel, any value gives the same
     results up to rounding; 0 = unknown)."""
