@@ -14,7 +14,8 @@
 #include <tuple>
 
 namespace chronos {
-void launch_hy_embed(const int32_t*, const void*, float*, int, int, float, bool, hipStream_t);
+void launch_hy_embed(const int32_t*, const void*, float*, uint16_t*, int, int, float, bool, hipStream_t);
+void launch_hy_low_rank_decay(const float*, const float*, const float*, float*, int, int, int, float, hipStream_t);
 void launch_hy_cast_bf16(const float*, uint16_t*, int64_t, hipStream_t);
 void launch_hy_layer_norm(const void*, bool, float*, const float*, void*, bool, int, int, float, hipStream_t);
 void launch_hy_rowdot(const void*, const void*, const float*, float*, int, int, int, bool, hipStream_t);
@@ -83,7 +84,7 @@ void launch_hy_window_attention(const void*, int, const void*, const void*, cons
                                 const float*, int64_t, hipStream_t);
 int hy_window_nsplit(bool, int, int, int, int, int, int, int, int, int, int, int, int, int, bool);
 void launch_hy_short_conv(const void*, int, const float*, const float*, const int32_t*, const int32_t*, const int32_t*,
-                          const int32_t*, void*, void*, int, int, int, int, bool, bool, hipStream_t);
+                          const int32_t*, void*, void*, int, int, int, int, bool, bool, bool, hipStream_t);
 void launch_hy_delta_prep(const void*, int, const float*, const float*, float*, float*, float*, float*, int, int, int, int,
                           float, bool, hipStream_t);
 bool launch_hy_linear_scan(const void*, int, int, int, int, const float*, const float*, float, const float*, bool, bool,
@@ -130,9 +131,21 @@ Tensor hy_embed(const Tensor& ids, const Tensor& table, double scale) {
     i32(ids, "embed: ids must be contiguous int32");
     need(is_act(table) && table.dim() == 2 && table.is_contiguous(), "embed: table [V, d] bf16 or f32");
     auto x = at::empty({ids.numel(), table.size(1)}, table.options().dtype(at::kFloat));
-    chronos::launch_hy_embed(ids.data_ptr<int32_t>(), table.data_ptr(), x.data_ptr<float>(), (int)ids.numel(),
+    chronos::launch_hy_embed(ids.data_ptr<int32_t>(), table.data_ptr(), x.data_ptr<float>(), nullptr, (int)ids.numel(),
                              (int)table.size(1), (float)scale, f32(table), stream());
     return x;
+}
+
+// the float32 rows and the same in bfloat16
+std::tuple<Tensor, Tensor> hy_embed_both(const Tensor& ids, const Tensor& table, double scale) {
+    c10::hip::HIPGuardMasqueradingAsCUDA g(table.device());
+    i32(ids, "embed: ids must be contiguous int32");
+    need(is_act(table) && table.dim() == 2 && table.is_contiguous(), "embed: table [V, d] bf16 or f32");
+    auto x = at::empty({ids.numel(), table.size(1)}, table.options().dtype(at::kFloat));
+    auto h = at::empty_like(x, x.options().dtype(at::kBFloat16));
+    chronos::launch_hy_embed(ids.data_ptr<int32_t>(), table.data_ptr(), x.data_ptr<float>(), (uint16_t*)h.data_ptr(), (int)ids.numel(),
+                             (int)table.size(1), (float)scale, f32(table), stream());
+    return {x, h};
 }
 
 Tensor hy_cast_bf16(const Tensor& x) {
@@ -579,6 +592,18 @@ void hy_decay_pow(Tensor& z, double p) {
     chronos::launch_hy_decay_pow(z.data_ptr<float>(), z.numel(), (float)p, stream());
 }
 
+Tensor hy_low_rank_decay(const Tensor& a, const Tensor& w, const Tensor& b, double p) {
+    c10::hip::HIPGuardMasqueradingAsCUDA g(a.device());
+    flt(a, "low_rank_decay: float32 a"); flt(w, "low_rank_decay: float32 w"); flt(b, "low_rank_decay: float32 b");
+    need(a.dim() == 2 && w.dim() == 2 && a.size(1) == w.size(0) && b.numel() == w.size(1), "low_rank_decay: a [T, R], w [R, C], b [C]");
+    need(w.size(1) % 4 == 0 && ((reinterpret_cast<uintptr_t>(w.data_ptr()) | reinterpret_cast<uintptr_t>(b.data_ptr())) & 15) == 0,
+         "low_rank_decay: channels in fours");
+    auto z = at::empty({a.size(0), w.size(1)}, a.options());
+    chronos::launch_hy_low_rank_decay(a.data_ptr<float>(), w.data_ptr<float>(), b.data_ptr<float>(), z.data_ptr<float>(), (int)a.size(0),
+                                      (int)a.size(1), (int)w.size(1), (float)p, stream());
+    return z;
+}
+
 Tensor hy_head_norm_gate(const Tensor& o, const Tensor& src, int64_t g_off, const Tensor& w, double eps, bool silu_gate,
                          bool out_f32) {
     c10::hip::HIPGuardMasqueradingAsCUDA g(o.device());
@@ -731,7 +756,7 @@ Tensor hy_window_attention(const Tensor& qkv, const c10::optional<Tensor>& kc_in
 }
 
 Tensor hy_short_conv(const Tensor& x, const Tensor& w, const Tensor& tok_seq, const Tensor& q_start, const Tensor& pos0,
-                     const Tensor& slots, Tensor& hist, bool silu, const c10::optional<Tensor>& bias, int64_t x_off) {
+                     const Tensor& slots, Tensor& hist, bool silu, const c10::optional<Tensor>& bias, int64_t x_off, int64_t max_q) {
     c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
     same_act(x, hist, "short_conv: the history holds the activation dtype");
     flt(w, "short_conv: float32 taps");
@@ -746,7 +771,7 @@ Tensor hy_short_conv(const Tensor& x, const Tensor& w, const Tensor& tok_seq, co
     chronos::launch_hy_short_conv(xp, (int)x.size(1), w.data_ptr<float>(), bias ? bias->data_ptr<float>() : nullptr,
                                   tok_seq.data_ptr<int32_t>(),
                                   q_start.data_ptr<int32_t>(), pos0.data_ptr<int32_t>(), slots.data_ptr<int32_t>(),
-                                  hist.data_ptr(), y.data_ptr(), (int)T, (int)B, (int)C, (int)K, silu, f32(x), stream());
+                                  hist.data_ptr(), y.data_ptr(), (int)T, (int)B, (int)C, (int)K, silu, max_q == 1, f32(x), stream());
     return y;
 }
 
@@ -1081,6 +1106,7 @@ Tensor hy_unrotate_gate(const Tensor& o, const Tensor& pos, const c10::optional<
 
 TORCH_LIBRARY_FRAGMENT(chronos, m) {
     m.def("hy_embed(Tensor ids, Tensor table, float scale=1.0) -> Tensor");
+    m.def("hy_embed_both(Tensor ids, Tensor table, float scale) -> (Tensor, Tensor)");
     m.def("hy_cast_bf16(Tensor x) -> Tensor");
     m.def("hy_layer_norm(Tensor x, Tensor w, float eps, bool out_f32) -> Tensor");
     m.def("hy_add_layer_norm(Tensor y, Tensor(a!) x, Tensor w, float eps, bool out_f32) -> Tensor");
@@ -1123,6 +1149,7 @@ TORCH_LIBRARY_FRAGMENT(chronos, m) {
           "Tensor pos, Tensor block_table, int H, int G, int D, float eps, Tensor? q_temp, Tensor(b!) ks, Tensor(c!) vc, "
           "int g_off, int max_q) -> (Tensor, Tensor)");
     m.def("hy_decay_pow(Tensor(a!) z, float p) -> ()");
+    m.def("hy_low_rank_decay(Tensor a, Tensor w, Tensor b, float p) -> Tensor");
     m.def("hy_head_norm_gate(Tensor o, Tensor src, int g_off, Tensor w, float eps, bool silu_gate, bool out_f32) -> Tensor");
     m.def("hy_window_prep(Tensor(a!) qkv, int H, int G, int D, int Dv, Tensor? v_first, Tensor? lam, Tensor pos, "
           "Tensor tok_seq, Tensor block_table, Tensor? q_norm, Tensor? k_norm, float eps, Tensor? cos_sin, int dims, "
@@ -1140,7 +1167,7 @@ TORCH_LIBRARY_FRAGMENT(chronos, m) {
           "float q_mul, float k_mul) -> ()");
     m.def("hy_unrotate_gate(Tensor o, Tensor pos, Tensor? cos_sin, Tensor? gate_src, int g_off, int H, int Dv) -> Tensor");
     m.def("hy_short_conv(Tensor x, Tensor w, Tensor tok_seq, Tensor q_start, Tensor pos0, Tensor slots, Tensor(a!) hist, "
-          "bool silu, Tensor? bias, int x_off) -> Tensor");
+          "bool silu, Tensor? bias, int x_off, int max_q=0) -> Tensor");
     m.def("hy_delta_prep(Tensor y, Tensor ab, Tensor a_log, int HK, int H, int D, float q_mul) -> (Tensor, Tensor, Tensor, Tensor)");
     m.def("hy_linear_scan(Tensor proj, int q_off, int k_off, int v_off, Tensor? qscale, Tensor? kscale, float q_mul, "
           "Tensor decay, Tensor? beta, Tensor q_start, Tensor pos0, Tensor slots, Tensor(a!) S, int HK, int H, int D, "
@@ -1161,6 +1188,7 @@ TORCH_LIBRARY_FRAGMENT(chronos, m) {
 
 TORCH_LIBRARY_IMPL(chronos, CUDA, m) {
     m.impl("hy_embed", &hy_embed);
+    m.impl("hy_embed_both", &hy_embed_both);
     m.impl("hy_cast_bf16", &hy_cast_bf16);
     m.impl("hy_layer_norm", &hy_layer_norm);
     m.impl("hy_add_layer_norm", &hy_add_layer_norm);
@@ -1185,6 +1213,7 @@ TORCH_LIBRARY_IMPL(chronos, CUDA, m) {
     m.impl("hy_norm_cols", &hy_norm_cols);
     m.impl("hy_conv_prep", &hy_conv_prep);
     m.impl("hy_decay_pow", &hy_decay_pow);
+    m.impl("hy_low_rank_decay", &hy_low_rank_decay);
     m.impl("hy_head_norm_gate", &hy_head_norm_gate);
     m.impl("hy_window_prep", &hy_window_prep);
     m.impl("hy_window_attention", &hy_window_attention);

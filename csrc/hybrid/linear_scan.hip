@@ -59,8 +59,8 @@ __global__ void __launch_bounds__(256) short_conv_vec_kernel(const uint16_t* __r
                                                              const int32_t* __restrict__ q_start,
                                                              const int32_t* __restrict__ pos0,
                                                              const int32_t* __restrict__ slots,
-                                                             const uint16_t* __restrict__ hist, uint16_t* __restrict__ y, int T,
-                                                             int C, int TK, int silu, const float* __restrict__ bias) {
+                                                             uint16_t* __restrict__ hist, uint16_t* __restrict__ y, int T,
+                                                             int C, int TK, int silu, const float* __restrict__ bias, bool one_each) {
     const int gx = (C / 8 + 255) / 256, c = (blockIdx.x % gx * 256 + threadIdx.x) * 8;   // workgroups of the same tokens side by side
     if (c >= C) return;
     const int tb = blockIdx.x / gx * TK, te = min(tb + TK, T);
@@ -77,7 +77,7 @@ __global__ void __launch_bounds__(256) short_conv_vec_kernel(const uint16_t* __r
         if (b != seq) {   // the block's first token, or another sequence's: the inputs in front of it
             seq = b;
             const int t0 = q_start[b];
-            const uint16_t* hrow = pos0[b] > 0 ? hist + (int64_t)slots[b] * (K - 1) * C + c : nullptr;
+            const uint16_t* const hrow = pos0[b] > 0 ? hist + (int64_t)slots[b] * (K - 1) * C + c : nullptr;
 #pragma unroll
             for (int i = 1; i < K; ++i) {
                 const int s = t - K + i;   // lands in in[i - 1] below
@@ -103,6 +103,10 @@ __global__ void __launch_bounds__(256) short_conv_vec_kernel(const uint16_t* __r
             if (silu) acc[e] *= sigmoid_act<uint16_t>(acc[e]);
         }
         st8(y + (int64_t)t * C + c, acc);
+        if (one_each) {   // the sequence's only token of this step (TK is 1): these channels' history in the same pass
+#pragma unroll
+            for (int i = 0; i + 1 < K; ++i) st8(hist + ((int64_t)slots[b] * (K - 1) + i) * C + c, in[i + 1]);
+        }
     }
 }
 
@@ -438,19 +442,21 @@ void launch_hy_conv_hist(const void* x, int ldx, const int32_t* q_start, const i
     else hy::conv_hist_kernel<uint16_t><<<hg, 256, 0, s>>>((const uint16_t*)x, ldx, q_start, pos0, slots, (uint16_t*)hist, C, K);
 }
 
+// one_each: no sequence brings more than one token (the history is then rewritten in the same pass where 8 channels go together)
 void launch_hy_short_conv(const void* x, int ldx, const float* w, const float* bias, const int32_t* tok_seq,
                           const int32_t* q_start, const int32_t* pos0, const int32_t* slots, void* hist, void* y, int T,
-                          int B, int C, int K, bool silu, bool f32, hipStream_t s) {
+                          int B, int C, int K, bool silu, bool one_each, bool f32, hipStream_t s) {
     if (T == 0 || C == 0) return;
     if (!f32 && K >= 2 && K <= 4 && C % 8 == 0 && ldx % 8 == 0 && hy::aligned16(x, hist, y)) {
         // 8 tokens per thread where that leaves a workgroup per CU, else one
-        const int gx = (C / 8 + 255) / 256, tk = (int64_t)gx * ((T + 7) / 8) >= 256 ? 8 : 1;
+        const int gx = (C / 8 + 255) / 256, tk = !one_each && (int64_t)gx * ((T + 7) / 8) >= 256 ? 8 : 1;
         const unsigned grid = (unsigned)gx * ((T + tk - 1) / tk);   // (one axis: the second ends at 65535 blocks)
-#define HY_CONV(KK) hy::short_conv_vec_kernel<KK><<<grid, 256, 0, s>>>((const uint16_t*)x, ldx, w, tok_seq, q_start, pos0, slots, (const uint16_t*)hist, (uint16_t*)y, T, C, tk, silu, bias)
+#define HY_CONV(KK) hy::short_conv_vec_kernel<KK><<<grid, 256, 0, s>>>((const uint16_t*)x, ldx, w, tok_seq, q_start, pos0, slots, (uint16_t*)hist, (uint16_t*)y, T, C, tk, silu, bias, one_each)
         if (K == 2) HY_CONV(2);
         else if (K == 3) HY_CONV(3);
         else HY_CONV(4);
 #undef HY_CONV
+        if (one_each) return;
     } else if (f32) {
         hy::short_conv_kernel<float><<<T, 256, 0, s>>>((const float*)x, ldx, w, tok_seq, q_start, pos0, slots, (const float*)hist, (float*)y, C, K, silu, bias);
     } else {

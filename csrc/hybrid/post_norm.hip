@@ -137,17 +137,19 @@ __global__ void __launch_bounds__(256) glu_vec_kernel(const uint16_t* __restrict
 // units of the result's last place at p = 1/16, this and the library throughout: z in -100 .. -20 0.83, 0.300 both; -20 .. -6 1.14, 0.344 and
 // 1.08, 0.343; -0.1 .. 0.1 0.67, 0.292 and 0.64, 0.291 (at p = 1/8 0.90, 0.315 and 0.89, 0.308, hence the line).  Through exp2 to the end the
 // rounding of z p log2 e shows: 4.2, 1.33 at z < -40.  16 bytes per lane.  8192 x 2048 values: 67 us with the library, which bounds it, 20 so.
-__global__ void __launch_bounds__(256) decay_pow_vec_kernel(f32x4* __restrict__ z, int64_t n4, float p) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n4) return;
+__device__ __forceinline__ f32x4 decay_pow4(f32x4 v, float p) {
     constexpr float kLog2e = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
-    f32x4 v = z[i];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const float t = __builtin_amdgcn_exp2f(-fabsf(v[e]) * kLog2e);
         v[e] = expf(p * __builtin_fmaf(-kLn2, __builtin_amdgcn_logf(1.f + t), fminf(v[e], 0.f)));
     }
-    z[i] = v;
+    return v;
+}
+__global__ void __launch_bounds__(256) decay_pow_vec_kernel(f32x4* __restrict__ z, int64_t n4, float p) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n4) return;
+    z[i] = decay_pow4(z[i], p);
 }
 
 __global__ void __launch_bounds__(256) decay_pow_kernel(float* __restrict__ z, int64_t n, float p) {
@@ -155,7 +157,58 @@ __global__ void __launch_bounds__(256) decay_pow_kernel(float* __restrict__ z, i
     if (i < n) z[i] = expf(logsigmoidf_(z[i]) * p);
 }
 
+// Decays of a gated linear recurrence from their low-rank logits, in one pass: out[t, c] = sigmoid(b[c] + sum_r a[t, r] w[r, c])^p, float
+// throughout, the sum in the order of r.  A thread takes 4 channels of TT tokens, so that w is read once for them; the tokens' a is
+// the same in all lanes.  Bound by writing out (8192 x 4096
+// of rank 16: 28 us, 4.8 TB/s); a library product, the copy of its bias and decay_pow took 120 there, 15 for 2446 x 512 (8 so), 16 for a single
+// token (6).
+template <int TT, bool POW4>
+__global__ void __launch_bounds__(256) low_rank_decay_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                             const float* __restrict__ b, float* __restrict__ out, int T, int R, int C,
+                                                             float p) {
+    const int c = (blockIdx.x * 256 + threadIdx.x) * 4;
+    if (c >= C) return;
+    const int t0 = blockIdx.y * TT;
+    f32x4 z[TT];
+#pragma unroll
+    for (int u = 0; u < TT; ++u) z[u] = *reinterpret_cast<const f32x4*>(b + c);
+    for (int r = 0; r < R; ++r) {
+        const f32x4 wr = *reinterpret_cast<const f32x4*>(w + (int64_t)r * C + c);
+#pragma unroll
+        for (int u = 0; u < TT; ++u) {
+            const float av = a[(int64_t)min(t0 + u, T - 1) * R + r];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) z[u][e] = __builtin_fmaf(av, wr[e], z[u][e]);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < TT; ++u) {
+        if (t0 + u >= T) break;
+        f32x4 v = z[u];
+        if constexpr (POW4) v = decay_pow4(v, p);
+        else
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = expf(logsigmoidf_(v[e]) * p);
+        *reinterpret_cast<f32x4*>(out + (int64_t)(t0 + u) * C + c) = v;
+    }
+}
+
 }  // namespace hy
+
+// C % 4 == 0, w, b and out on 16 bytes
+void launch_hy_low_rank_decay(const float* a, const float* w, const float* b, float* out, int T, int R, int C, float p, hipStream_t s) {
+    if (T == 0 || C == 0) return;
+    const int gx = (C / 4 + 255) / 256;
+    const bool pow4 = p > 0.f && p <= 0.0625f;   // (as in launch_hy_decay_pow)
+#define HY_LRD(TT) do { \
+        const dim3 grid(gx, (T + TT - 1) / TT); \
+        if (pow4) hy::low_rank_decay_kernel<TT, true><<<grid, 256, 0, s>>>(a, w, b, out, T, R, C, p); \
+        else hy::low_rank_decay_kernel<TT, false><<<grid, 256, 0, s>>>(a, w, b, out, T, R, C, p); \
+    } while (0)
+    if ((int64_t)gx * T >= 4096) HY_LRD(4);   // (four tokens a thread once that leaves four workgroups per CU)
+    else HY_LRD(1);
+#undef HY_LRD
+}
 
 // y == nullptr: plain norm of x (h in float when out_f32, else bfloat16).  Otherwise the joined form; y is in the
 // activation type (float when out_f32), h may be nullptr (float activations read the stream itself).

@@ -19,13 +19,16 @@ struct PPArgs {
     int gm;      // tile order: M-tiles per group (0 = every M-tile of a W panel consecutive); knob pp_gm
     int handoff;       // gemm_lg split-K slab hand-off (knob lg_handoff): -1 auto, 0 fences, 1 write-through
     float limit, slope, shift;  // kPPGlu: min(g, limit) sigmoid(slope g) (clamp(u, -limit, limit) + shift)
+    float* yf;          // gemm_skinny, plain: outputs n0 .. n0 + nf go here, float32 [M, nf], plus bias; y is [M, n0] then
+    const float* bias;
+    int n0, nf;
     const float* xsc;  // gemm_lg F8 (W8A8 e4m3fn bytes in x / w): per-token scales [M]
     const float* wsc;  // ... and per-output-channel scales [N]
     int ablate;  // timing-only diagnostics (knob pp_ablate): 1 skip loop DMA, 2 skip LDS reads, 4 skip MFMA, 8 nt weights, 16/32 alias every W/x tile onto tile 0
 };
 
 // epilogue modes
-enum : int { kPPPlain = 0, kPPSwiglu = 1, kPPResid = 2, kPPGlu = 3, kPPRelu2 = 4, kPPGelu = 5 };  // (3 on: gemm_slab only)
+enum : int { kPPPlain = 0, kPPSwiglu = 1, kPPResid = 2, kPPGlu = 3, kPPRelu2 = 4, kPPGelu = 5 };  // (3 on: gemm_slab, gemm_skinny)
 constexpr int kPPConfigs = 12;
 int gemm_pp_bm(int cfg);  // x rows per tile
 int gemm_pp_bn(int cfg);  // W rows per tile
@@ -55,8 +58,8 @@ bool launch_gemm_lg_f8(int cfg, bool swiglu, const PPArgs& a, hipStream_t st);
 // skinny-M family (csrc/kernels/gemm_skinny.hip, M <= 16 * MT): same PPArgs / epilogues; the workgroup owns 16 * RT
 // W rows (swiglu: 8 * RT gate + 8 * RT up), ws holds [groups * splitk, 64 * RT * MT] f32x4 slabs, cnt one ticket per
 // group, kResid partials are [M, N / (16 * RT)]; K % (64 * NW * splitk) == 0
-constexpr int kSkinnyConfigs = 16;
-constexpr int kSkinnyUneven = 12;  // from this config on: plain epilogue only, K any multiple of 64 (the shares of slices
+constexpr int kSkinnyConfigs = 18;
+constexpr int kSkinnyUneven = 12;  // from this config on: plain epilogue and activations only, K any multiple of 64 (the shares of slices
                                   // and waves differ by a unit), the split's sums in a second launch instead of tickets
 int gemm_skinny_rt(int cfg);
 int gemm_skinny_mt(int cfg);

@@ -641,6 +641,52 @@ Tensor gemm_act(const Tensor& x, const Tensor& w, int64_t mode, double limit, do
     return y;
 }
 
+// Products of few rows for the hybrid decoders (gemm_skinny.hip from kSkinnyUneven on, no split of K): mode 0 plain with the last nf of w's
+// rows as float32 outputs [M, nf] (plus bias; w may have rows of padding behind them), else an activation as in gemm_act.
+std::tuple<Tensor, Tensor> gemm_few(const Tensor& x, const Tensor& w, int64_t cfg, int64_t mode, int64_t n0, int64_t nf,
+                                    const c10::optional<Tensor>& bias, double limit, double slope, double shift) {
+    chk_bf16(x, "x");
+    chk_bf16(w, "w");
+    CHK(x.dim() == 2 && w.dim() == 2 && w.size(1) == x.size(1), "gemm_few: x [M, K], w [N, K]");
+    const int64_t K = x.size(1), M = x.size(0), N = w.size(0);
+    CHK(cfg >= chronos::kSkinnyUneven && cfg < chronos::kSkinnyConfigs, "gemm_few: cfg");
+    CHK(mode == 0 || (mode >= chronos::kPPGlu && mode <= chronos::kPPGelu), "gemm_few: mode");
+    const int RT = chronos::gemm_skinny_rt((int)cfg), MT = chronos::gemm_skinny_mt((int)cfg);
+    CHK(M >= 1 && M <= 16 * MT, "gemm_few: M must be in [1, 16 * MT] of the config");
+    CHK(K >= 64 && K % 64 == 0 && K <= (1 << 20) && N * K < (1LL << 40), "gemm_few: K % 64 == 0");
+    CHK(mode == chronos::kPPGlu ? RT % 2 == 0 && N % (16 * RT) == 0 : N % (16 * RT) == 0, "gemm_few: N % (16 RT) (gated units: RT even)");
+    CHK(mode == 0 ? n0 >= 0 && nf >= 0 && n0 % 4 == 0 && n0 + nf <= N : nf == 0, "gemm_few: n0 % 4 == 0, n0 + nf <= N; with an activation no float32 outputs");
+    CHK(((reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr())) & 15) == 0, "gemm_few: alignment");
+    if (bias.has_value()) {
+        chk_gpu(*bias, "bias");
+        CHK(bias->scalar_type() == at::kFloat && bias->numel() == nf, "gemm_few: bias [nf] f32");
+    }
+    c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+    chronos::PPArgs a{};
+    a.x = bf(x);
+    a.w = bf(w);
+    a.M = (int)M;
+    a.N = (int)N;
+    a.K = (int)K;
+    a.F = (int)(N / 2);
+    a.splitk = 1;
+    a.limit = (float)limit;
+    a.slope = (float)slope;
+    a.shift = (float)shift;
+    Tensor y = at::empty({M, mode == chronos::kPPGlu ? N / 2 : mode == 0 ? n0 : N}, x.options()), yf;
+    a.y = bfm(y);
+    if (mode == 0) {
+        yf = at::empty({M, nf}, x.options().dtype(at::kFloat));
+        a.yf = yf.data_ptr<float>();
+        a.bias = bias.has_value() ? bias->data_ptr<float>() : nullptr;
+        a.n0 = (int)n0;
+        a.nf = (int)nf;
+        CHK(nf > 0, "gemm_few: nf");
+    }
+    CHK(chronos::launch_gemm_skinny((int)cfg, (int)mode, false, a, cur_stream()), "gemm_few: launch");
+    return {y, yf};
+}
+
 // Skinny-M GEMM (gemm_skinny.hip), M <= 16 * MT of the config: same epilogues and tensors as gemm_pp; the kResid
 // partials are [M, N / (16 * RT)].
 std::tuple<Tensor, Tensor> gemm_skinny(const Tensor& x, const Tensor& w, int64_t mode, int64_t cfg, int64_t splitk,
@@ -863,6 +909,7 @@ TORCH_LIBRARY(chronos, m) {
     m.def("gemv(Tensor x, Tensor w, bool swiglu, Tensor? ws=None) -> Tensor");
     m.def("gemm(Tensor x, Tensor w, bool swiglu, int stages=3) -> Tensor");
     m.def("gemm_act(Tensor x, Tensor w, int mode, float limit, float slope, float shift) -> Tensor");
+    m.def("gemm_few(Tensor x, Tensor w, int cfg, int mode, int n0, int nf, Tensor? bias, float limit, float slope, float shift) -> (Tensor, Tensor)");
     m.def("gemm_pp(Tensor x, Tensor w, int mode, int cfg, int splitk, Tensor? resid, Tensor? part_in, float eps, bool prio) -> (Tensor, Tensor)");
     m.def("gemm_skinny(Tensor x, Tensor w, int mode, int cfg, int splitk, Tensor? resid, Tensor? part_in, float eps) "
           "-> (Tensor, Tensor)");
@@ -906,6 +953,7 @@ TORCH_LIBRARY_IMPL(chronos, CUDA, m) {
     m.impl("gemv", &gemv);
     m.impl("gemm", &gemm);
     m.impl("gemm_act", &gemm_act);
+    m.impl("gemm_few", &gemm_few);
     m.impl("gemm_pp", &gemm_pp);
     m.impl("gemm_skinny", &gemm_skinny);
     m.impl("gemv_resid", &gemv_resid);

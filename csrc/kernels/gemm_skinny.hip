@@ -25,24 +25,26 @@
 //   * epilogue per (row m, 4 consecutive outputs): 8-byte stores, CPR consecutive lanes cover a row's 16 RT outputs.
 #include <algorithm>
 
+#include "chronos_act.h"
 #include "chronos_gemm.h"
 #include "chronos_hip.h"
 
 namespace chronos {
 namespace {
 
-enum : int { kPlain = kPPPlain, kSwiglu = kPPSwiglu, kResid = kPPResid };
+enum : int { kPlain = kPPPlain, kSwiglu = kPPSwiglu, kResid = kPPResid, kGlu = kPPGlu };
+constexpr bool sk_pair(int mode) { return mode == kSwiglu || mode == kGlu; }   // w = [gate; up]
 constexpr int XL_MIN_MT = 2;  // x staged through LDS from MT = 2 (x bytes >= the weight bytes per wave)
 
 template <int RT, int MT, int D, int NW, int MODE, bool NORMP>
 __global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a) {
-    static_assert(MODE != kSwiglu || RT % 2 == 0, "swiglu: RT/2 gate tiles + RT/2 up tiles");
+    static_assert(!sk_pair(MODE) || RT % 2 == 0, "swiglu: RT/2 gate tiles + RT/2 up tiles");
     constexpr int NT = 64 * NW;                        // threads
     constexpr int UNITS = RT * MT * 64;                // f32x4 accumulators per wave
-    constexpr int CPR = MODE == kSwiglu ? 2 * RT : 4 * RT;  // output units (4 columns each) per row
+    constexpr int CPR = sk_pair(MODE) ? 2 * RT : 4 * RT;  // output units (4 columns each) per row
     constexpr int NOUT = 16 * MT * CPR;                // output units per workgroup (a multiple of 64)
     constexpr int VP = NOUT >= NT ? NOUT / NT : 1;     // output units per thread
-    constexpr int PAIR = MODE == kSwiglu ? 2 : 1;       // swiglu: a gate unit and its up unit
+    constexpr int PAIR = sk_pair(MODE) ? 2 : 1;       // swiglu: a gate unit and its up unit
     constexpr int NP = NOUT + NOUT / 16;               // one padded half (pad: 1 slot per 16, see red_at)
     constexpr int SZ = PAIR * NP;                      // f32x4 slots per wave
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -52,7 +54,7 @@ __global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a) {
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int M = a.M, K = a.K, S = a.splitk;
-    const int G = MODE == kSwiglu ? a.F / (8 * RT) : a.N / (16 * RT);
+    const int G = sk_pair(MODE) ? a.F / (8 * RT) : a.N / (16 * RT);
     const int task = xcd_remap(blockIdx.x, G * S);
     const int g = task / S, s = task - g * S;
     const int unit0 = K / 64 * s / S;  // the slice's 64-k units (slices and waves differ by one where they do not divide; may be 0)
@@ -63,7 +65,7 @@ __global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a) {
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
         int row;
-        if constexpr (MODE == kSwiglu)
+        if constexpr (sk_pair(MODE))
             row = rt < RT / 2 ? g * 8 * RT + 16 * rt : a.F + g * 8 * RT + 16 * (rt - RT / 2);
         else
             row = g * 16 * RT + 16 * rt;
@@ -196,7 +198,7 @@ __global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a) {
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            constexpr int HALF = MODE == kSwiglu ? RT / 2 : RT;
+            constexpr int HALF = sk_pair(MODE) ? RT / 2 : RT;
             const int p = rt / HALF, c = 4 * (rt % HALF) + (lane >> 4);
             red[red_at(wave, p, (16 * mt + (lane & 15)) * CPR + c)] = acc[rt][mt];
         }
@@ -282,6 +284,16 @@ __global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a) {
                 }
                 *reinterpret_cast<u16x4*>(a.y + (int64_t)r * a.F + g * 8 * RT + 4 * c) = o;
             }
+        } else if constexpr (MODE == kGlu) {
+            if (live) {
+                u16x4 o;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float gv = fminf(val[j][0][i], a.limit), u = fminf(fmaxf(val[j][1][i], -a.limit), a.limit);
+                    o[i] = f2bf(gv * hy::sigmoid_act<uint16_t>(a.slope * gv) * (u + a.shift));
+                }
+                *reinterpret_cast<u16x4*>(a.y + (int64_t)r * a.F + g * 8 * RT + 4 * c) = o;
+            }
         } else if constexpr (MODE == kResid) {
             const int64_t at = (int64_t)r * a.N + g * 16 * RT + 4 * c;
             float ss = 0.f;
@@ -301,11 +313,21 @@ __global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a) {
             for (int off = 1; off < CPR; off <<= 1) ss += __shfl_xor(ss, off, 64);
             if (c == 0 && live) a.part_out[(int64_t)r * (a.N / (16 * RT)) + g] = ss;
         } else {
-            if (live) {
+            const int n = g * 16 * RT + 4 * c;
+            if (MODE == kPlain && !NORMP && a.yf != nullptr && n >= a.n0) {   // (n0 is a multiple of 4)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (live && n + i < a.n0 + a.nf)
+                        a.yf[(int64_t)r * a.nf + n + i - a.n0] = val[j][0][i] + (a.bias != nullptr ? a.bias[n + i - a.n0] : 0.f);
+            } else if (live) {
                 u16x4 o;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) o[i] = f2bf(val[j][0][i] * sc);
-                *reinterpret_cast<u16x4*>(a.y + (int64_t)r * a.N + g * 16 * RT + 4 * c) = o;
+                for (int i = 0; i < 4; ++i) {
+                    float v = val[j][0][i] * sc;
+                    if constexpr (MODE == kPPRelu2 || MODE == kPPGelu) v = hy::act_apply(v, MODE == kPPRelu2 ? hy::kActRelu2 : hy::kActGelu);
+                    o[i] = f2bf(v);
+                }
+                *reinterpret_cast<u16x4*>(a.y + (int64_t)r * (a.yf != nullptr ? a.n0 : a.N) + n) = o;
             }
         }
     }
@@ -334,7 +356,7 @@ void launch_cfg(const PPArgs& a, hipStream_t st) {
         hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         attr = true;
     }
-    const int G = MODE == kSwiglu ? a.F / (8 * RT) : a.N / (16 * RT);
+    const int G = sk_pair(MODE) ? a.F / (8 * RT) : a.N / (16 * RT);
     hipLaunchKernelGGL(kern, dim3(G * a.splitk), dim3(64 * NW), lds, st, a);
     if (a.splitk > 1 && a.cnt == nullptr) {
         const int64_t n = (int64_t)a.M * a.N;
@@ -345,7 +367,10 @@ void launch_cfg(const PPArgs& a, hipStream_t st) {
 // configs {RT (W tiles of 16 rows per workgroup), MT (x tiles: M <= 16 MT), D (ring depth in 64-k units), NW (waves
 // splitting K inside the workgroup; K % (64 NW splitk) == 0, from kSkinnyUneven on K % 64 == 0: the shares then differ by a unit.  At a few MB of weights what bounds a launch is latency, so these run 8 short waves: 2048 x 2048 with 16 rows 6.0 us (the
 // library 11.0), 1024 x 2816 with one row 5.7 (8.6).  Their split across workgroups writes [split, M, N] sums that a second launch adds
-// up: 2.0-2.3 us, as much as tickets cost, with nothing kept between calls)}
+// up: 2.0-2.3 us, as much as tickets cost, with nothing kept between calls.  16 and 17 are for the products with more to
+// do behind them (gemm_few): activations, which a launch of its own costs 2.8 to 3.5 us, and float32 outputs of a few rows behind the others',
+// 3.6 to 7.8 as a product of their own.  One row, us: 3072 x 1024 and 8 rows 4.7 + 3.8 -> 4.8; gated unit of 5632 x 1024 6.8 + 2.8 -> 6.1; 64 rows:
+// 6720 x 4096 and 32 rows 19.1 + 7.5 -> 23.4; GELU of 8192 x 2048 15.3 + 3.5 -> 15.5)}
 #define SK_CONFIGS(X)  \
     X(0, 1, 1, 4, 16)  \
     X(1, 2, 1, 4, 8)   \
@@ -362,15 +387,17 @@ void launch_cfg(const PPArgs& a, hipStream_t st) {
     X(12, 1, 2, 4, 8)  \
     X(13, 1, 4, 2, 8)  \
     X(14, 1, 1, 4, 8)  \
-    X(15, 2, 1, 4, 8)
+    X(15, 2, 1, 4, 8)  \
+    X(16, 2, 2, 4, 8)  \
+    X(17, 2, 4, 2, 8)
 
 template <int MODE, bool NORMP>
 bool launch_mode(int cfg, const PPArgs& a, hipStream_t st) {
     switch (cfg) {
 #define SK_CASE(ID, RT_, MT_, D_, NW_)                                     \
     case ID:                                                               \
-        if constexpr (MODE == kSwiglu && RT_ % 2) return false;            \
-        else if constexpr (ID >= kSkinnyUneven && (MODE != kPlain || NORMP)) return false; \
+        if constexpr (sk_pair(MODE) && RT_ % 2) return false;              \
+        else if constexpr (ID >= kSkinnyUneven ? MODE == kSwiglu || MODE == kResid || NORMP : MODE >= kGlu) return false; \
         else {                                                             \
             launch_cfg<RT_, MT_, D_, NW_, MODE, NORMP>(a, st);             \
             return true;                                                   \
@@ -411,6 +438,11 @@ int gemm_skinny_mt(int cfg) {
 bool launch_gemm_skinny(int cfg, int mode, bool normp, const PPArgs& a, hipStream_t st) {
     if (a.M == 0) return true;
     if (mode == kResid) return normp ? false : launch_mode<kResid, false>(cfg, a, st);
+    if (mode >= kGlu) {   // activations: one slice
+        if (normp || a.splitk != 1) return false;
+        return mode == kGlu ? launch_mode<kGlu, false>(cfg, a, st)
+               : mode == kPPRelu2 ? launch_mode<kPPRelu2, false>(cfg, a, st) : launch_mode<kPPGelu, false>(cfg, a, st);
+    }
     if (mode == kSwiglu) return normp ? launch_mode<kSwiglu, true>(cfg, a, st) : launch_mode<kSwiglu, false>(cfg, a, st);
     return normp ? launch_mode<kPlain, true>(cfg, a, st) : launch_mode<kPlain, false>(cfg, a, st);
 }

@@ -591,13 +591,25 @@ def ff_rides_along(mixer, ff) -> bool:
         ff.ff % 8 == 0 and mixer.heads * mixer.vdim % 8 == 0
 
 
+def _rows_behind(out: dict, key: str, few: str) -> dict:
+    """out[few], the rows of a float32-output projection, moved behind those of out[key], which reads the same input (both stay as
+    views): out["joined"] = (all rows and zeros up to a multiple of 32, rows of out[key], rows of out[few]) for hops.matmul_rowdot."""
+    a, b = out[key], out[few]
+    if a.is_cuda and a.dtype == b.dtype == torch.bfloat16 and a.shape[0] % 4 == 0 and a.shape[1] % 64 == 0:
+        n0, nf = a.shape[0], b.shape[0]
+        rows = torch.zeros(-(-(n0 + nf) // 32) * 32, a.shape[1], device=a.device, dtype=a.dtype)
+        rows[:n0], rows[n0:n0 + nf] = a, b
+        out[key], out[few], out["joined"] = rows[:n0], rows[n0:n0 + nf], (rows, n0, nf)
+    return out
+
+
 def pack_mlstm(spec: MLSTMSpec, t: dict, device, act_dtype) -> dict:
     """t: q, k, v, g, o, norm, i, i.b, f, f.b (checkpoint layout, [out, in]).  q | k | v | g become one projection,
     the two gate rows one few-row float32-output projection."""
     a = lambda x: x.to(device=device, dtype=act_dtype).contiguous()  # noqa: E731
     f = lambda x: x.to(device=device, dtype=torch.float32).contiguous()  # noqa: E731
-    return dict(w_proj=a(torch.cat([t["q"], t["k"], t["v"], t["g"]], 0)), w_if=a(torch.cat([t["i"], t["f"]], 0)),
-                b_if=f(torch.cat([t["i.b"], t["f.b"]], 0)), norm=f(t["norm"]), w_o=a(t["o"]))
+    return _rows_behind(dict(w_proj=a(torch.cat([t["q"], t["k"], t["v"], t["g"]], 0)), w_if=a(torch.cat([t["i"], t["f"]], 0)),
+                             b_if=f(torch.cat([t["i.b"], t["f.b"]], 0)), norm=f(t["norm"]), w_o=a(t["o"])), "w_proj", "w_if")
 
 
 def pack_latent(spec: LatentAttentionSpec, t: dict, device, act_dtype) -> dict:
@@ -627,6 +639,7 @@ def pack_latent(spec: LatentAttentionSpec, t: dict, device, act_dtype) -> dict:
         out["sink"] = f(t["sink"])
     if spec.gate and not spec.gate_wide:
         out["w_g"] = a(t["g"])
+        _rows_behind(out, "w_in", "w_g")
     return out
 
 
@@ -677,6 +690,8 @@ def pack_window_attention(spec: WindowAttentionSpec, t: dict, device, act_dtype)
         out["sink"] = f(t["sink"] if spec.sink_fixed is None else torch.full((spec.heads,), float(spec.sink_fixed)))
     if few and "g_off" not in out:
         out["w_g"] = a(t["g"])
+        if not spec.bias:
+            _rows_behind(out, "w_qkv", "w_g")
     if spec.bias:
         rest = out["w_qkv"].shape[0] - spec.heads * spec.dim - spec.kv_heads * (spec.dim + spec.vdim)  # gate rows: none
         out["b_qkv"] = a(torch.cat([t["q.b"], t["k.b"], t["v.b"], torch.zeros(rest, dtype=t["q.b"].dtype)], 0))
@@ -693,8 +708,9 @@ def pack_mamba2(spec: Mamba2Spec, t: dict, device, act_dtype) -> dict:
     a = lambda x: x.to(device=device, dtype=act_dtype).contiguous()  # noqa: E731
     f = lambda x: x.to(device=device, dtype=torch.float32).contiguous()  # noqa: E731
     n = 2 * spec.inner + 2 * spec.groups * spec.state
-    return dict(w_in=a(t["in"][:n]), w_dt=a(t["in"][n:]), b_dt=f(t["dt_bias"]), taps=f(t["conv"]),
-                b_conv=f(t["conv.b"]), a_log=f(t["A_log"]), skip=f(t["D"]), norm=f(t["norm"]), w_o=a(t["o"]))
+    out = dict(w_in=a(t["in"][:n]), w_dt=a(t["in"][n:]), b_dt=f(t["dt_bias"]), taps=f(t["conv"]),
+               b_conv=f(t["conv.b"]), a_log=f(t["A_log"]), skip=f(t["D"]), norm=f(t["norm"]), w_o=a(t["o"]))
+    return _rows_behind(out, "w_in", "w_dt")
 
 
 def pack_rglru(spec: RGLRUSpec, t: dict, device, act_dtype) -> dict:
@@ -716,11 +732,12 @@ def pack_delta_rule(spec: DeltaRuleSpec, t: dict, device, act_dtype) -> dict:
     float32-output projection (bias: dt_bias for the decay rows, zero for the others)."""
     a = lambda x: x.to(device=device, dtype=act_dtype).contiguous()  # noqa: E731
     f = lambda x: x.to(device=device, dtype=torch.float32).contiguous()  # noqa: E731
-    return dict(w_proj=a(torch.cat([t["q"], t["k"], t["v"], t["g"]], 0)),
-                taps=f(torch.cat([t["q.conv"], t["k.conv"], t["v.conv"]], 0)),
-                w_ab=a(torch.cat([t["a"], t["b"]], 0)),
-                b_ab=f(torch.cat([t["dt_bias"].float(), torch.zeros(spec.heads)], 0)), a_log=f(t["A_log"]),
-                norm=f(t["norm"].float().repeat(spec.heads)), w_o=a(t["o"]))
+    out = dict(w_proj=a(torch.cat([t["q"], t["k"], t["v"], t["g"]], 0)),
+               taps=f(torch.cat([t["q.conv"], t["k.conv"], t["v.conv"]], 0)),
+               w_ab=a(torch.cat([t["a"], t["b"]], 0)),
+               b_ab=f(torch.cat([t["dt_bias"].float(), torch.zeros(spec.heads)], 0)), a_log=f(t["A_log"]),
+               norm=f(t["norm"].float().repeat(spec.heads)), w_o=a(t["o"]))
+    return _rows_behind(out, "w_proj", "w_ab")
 
 
 def pack_gla(spec: GLASpec, t: dict, device, act_dtype) -> dict:
@@ -731,7 +748,7 @@ def pack_gla(spec: GLASpec, t: dict, device, act_dtype) -> dict:
     out = dict(w_a1=a(t["a1"]), w_a2t=f(t["a2"].float().t()), b_a2=f(t["a2.b"]),
                norm=f(t["norm"].float().repeat(spec.heads)), w_o=a(t["o"]))
     _in_proj([t["q"], t["k"], t["v"], t["g"]], t, out, "w_proj", a)
-    return out
+    return _rows_behind(out, "w_proj", "w_a1")
 
 
 def pack_retention(spec: RetentionSpec, t: dict, device, act_dtype) -> dict:
@@ -849,8 +866,7 @@ class StepMeta:
 
 def mix_mlstm(model, li: int, spec: MLSTMSpec, w: dict, h, meta: StepMeta, cache: HybridCache):
     H, D, Dv = spec.heads, spec.dim, spec.vdim
-    proj = hops.matmul(h, w["w_proj"])
-    gate_pre = hops.rowdot(h, w["w_if"], w["b_if"])
+    proj, gate_pre = hops.matmul_rowdot(h, w["w_proj"], w["w_if"], w["b_if"], w.get("joined"))
     o = hops.mlstm_scan(proj, gate_pre, meta.q_start, meta.pos0, meta.slots, cache.S[li], cache.n[li], cache.m[li],
                         H, D, Dv, spec.gate_cap, meta.max_q)
     y = hops.mlstm_out(o, proj, 2 * H * D + H * Dv, w["norm"], model.cfg.norm_eps, model.act_dtype)
@@ -896,12 +912,15 @@ def mix_latent_attention(model, li: int, spec: LatentAttentionSpec, w: dict, h, 
     H, D, R, rank = spec.heads, spec.dim, spec.rot_dim, spec.kv_rank
     eps = model.cfg.norm_eps
     nq, nkv = spec.q_rank or H * (D + R), rank + R
-    proj = hops.matmul(h, w["w_in"])    # q or its latent | dkv (| one gate per output column)
+    gate = None
+    if "w_g" in w:
+        proj, gate = hops.matmul_rowdot(h, w["w_in"], w["w_g"], None, w.get("joined"))
+    else:
+        proj = hops.matmul(h, w["w_in"])    # q or its latent | dkv (| one gate per output column)
     q = proj[:, :nq]
     if spec.q_rank:
         q = hops.matmul(hops.norm_cols(proj, 0, nq, w["dq_norm"], eps), w["w_uq"])
     q = q.view(T, H, D + R)
-    gate = hops.rowdot(h, w["w_g"]) if spec.gate and not spec.gate_wide else None
     own = spec.kv_from is None
     wide, ov = _wide_out(w, proj, H * spec.vdim)
     if meta.fresh and "w_kv" in w and T * H * meta.max_q >= EXPAND_MIN and q.stride(0) % 8 == 0 and (ov is None or ov.stride(0) % 4 == 0):
@@ -929,8 +948,12 @@ def mix_latent_attention(model, li: int, spec: LatentAttentionSpec, w: dict, h, 
 
 def mix_window_attention(model, li, spec: WindowAttentionSpec, w: dict, h, meta: StepMeta, cache: HybridCache):
     H, G, D, Dv = spec.heads, spec.kv_heads, spec.dim, spec.vdim
-    proj = qkv = hops.matmul(h, w["w_qkv"], w.get("b_qkv"))
-    gate = hops.rowdot(h, w["w_g"]) if "w_g" in w else None
+    if "joined" in w:
+        proj, gate = hops.matmul_rowdot(h, w["w_qkv"], w["w_g"], None, w["joined"])
+    else:
+        proj = hops.matmul(h, w["w_qkv"], w.get("b_qkv"))
+        gate = hops.rowdot(h, w["w_g"]) if "w_g" in w else None
+    qkv = proj
     temp = model.q_temp.get(li)
     if spec.conv and spec.unit_keys:
         # convolution, norms, temperature, cache write and the gate's float32 copy in one pass over the projection
@@ -940,7 +963,8 @@ def mix_window_attention(model, li, spec: WindowAttentionSpec, w: dict, h, meta:
         gate = gate if gate_cols is None else gate_cols
     else:
         if spec.conv:
-            qkv = hops.short_conv(proj, w["taps"], meta.tok_seq, meta.q_start, meta.pos0, meta.slots, cache.hist[li], False)
+            qkv = hops.short_conv(proj, w["taps"], meta.tok_seq, meta.q_start, meta.pos0, meta.slots, cache.hist[li], False,
+                                  max_q=meta.max_q)
         if "g_off" in w:
             gate = proj[:, w["g_off"]:w["g_off"] + H].float()
         mixes = spec.v_mix and not spec.v_mix_first
@@ -991,10 +1015,10 @@ def mix_parallel(model, li, spec: ParallelSpec, w: dict, h, meta: StepMeta, cach
 def mix_mamba2(model, li: int, spec: Mamba2Spec, w: dict, h, meta: StepMeta, cache: HybridCache):
     H, P, N, G = spec.heads, spec.vdim, spec.state, spec.groups
     inner, GN = spec.inner, spec.groups * spec.state
-    proj = hops.matmul(h, w["w_in"])                 # z | x | B | C
-    dt_pre = hops.rowdot(h, w["w_dt"], w["b_dt"])    # float32 step pre-activations, bias included
+    # z | x | B | C; float32 step pre-activations, bias included
+    proj, dt_pre = hops.matmul_rowdot(h, w["w_in"], w["w_dt"], w["b_dt"], w.get("joined"))
     xbc = hops.short_conv(proj, w["taps"], meta.tok_seq, meta.q_start, meta.pos0, meta.slots, cache.hist[li], True,
-                          w["b_conv"], inner)        # x | B | C after convolution and SiLU
+                          w["b_conv"], inner, meta.max_q)   # x | B | C after convolution and SiLU
     decay, dt = hops.ssm_prep(dt_pre, w["a_log"])
     # state rows = B, read by C, written with dt x: S <- decay S + B (dt x)^T, o = S^T C
     o = hops.linear_scan(xbc, inner + GN, inner, 0, None, None, 1.0, decay, None, meta.q_start, meta.pos0, meta.slots,
@@ -1008,7 +1032,7 @@ def mix_rglru(model, li: int, spec: RGLRUSpec, w: dict, h, meta: StepMeta, cache
     W = spec.width
     proj = hops.matmul(h, w["w_yx"], w["b_yx"])      # y branch | x branch
     u = hops.short_conv(proj, w["taps"], meta.tok_seq, meta.q_start, meta.pos0, meta.slots, cache.hist[li], False,
-                        w["b_conv"], W)
+                        w["b_conv"], W, meta.max_q)
     gates = hops.block_gates(u, w["w_gates"], w["b_gates"])   # float32 [blocks, T, 2 W / blocks]
     o = hops.rglru_scan(u, gates, w["sp"], spec.c, proj, 0, meta.q_start, meta.pos0, meta.slots, cache.S[li],
                         model.act_dtype, meta.max_q)
@@ -1018,9 +1042,9 @@ def mix_rglru(model, li: int, spec: RGLRUSpec, w: dict, h, meta: StepMeta, cache
 def mix_delta_rule(model, li: int, spec: DeltaRuleSpec, w: dict, h, meta: StepMeta, cache: HybridCache):
     H, HK, D, Dv = spec.heads, spec.kv_heads, spec.dim, spec.vdim
     C = 2 * HK * D + H * Dv
-    proj = hops.matmul(h, w["w_proj"])          # q | k | v | g
-    ab = hops.rowdot(h, w["w_ab"], w["b_ab"])   # decay and write-strength pre-activations, float32
-    y = hops.short_conv(proj, w["taps"], meta.tok_seq, meta.q_start, meta.pos0, meta.slots, cache.hist[li], True)
+    # q | k | v | g; decay and write-strength pre-activations, float32
+    proj, ab = hops.matmul_rowdot(h, w["w_proj"], w["w_ab"], w["b_ab"], w.get("joined"))
+    y = hops.short_conv(proj, w["taps"], meta.tok_seq, meta.q_start, meta.pos0, meta.slots, cache.hist[li], True, max_q=meta.max_q)
     qscale, kscale, decay, beta = hops.delta_prep(y, ab, w["a_log"], HK, H, D, D ** -0.5)
     o = hops.linear_scan(y, 0, HK * D, 2 * HK * D, qscale, kscale, 1.0, decay, beta, meta.q_start, meta.pos0,
                          meta.slots, cache.S[li], HK, H, D, Dv, max_q=meta.max_q)
@@ -1029,9 +1053,8 @@ def mix_delta_rule(model, li: int, spec: DeltaRuleSpec, w: dict, h, meta: StepMe
 
 def mix_gla(model, li: int, spec: GLASpec, w: dict, h, meta: StepMeta, cache: HybridCache):
     H, D, Dv = spec.heads, spec.dim, spec.vdim
-    proj = hops.matmul(h, w["w_proj"])          # q | k | v | g
-    z = torch.addmm(w["b_a2"], hops.rowdot(h, w["w_a1"]), w["w_a2t"])  # float32 decay logits [T, H D]
-    decay = hops.decay_pow(z, 1.0 / spec.tau)
+    proj, low = hops.matmul_rowdot(h, w["w_proj"], w["w_a1"], None, w.get("joined"))   # q | k | v | g; the decay's latent
+    decay = hops.low_rank_decay(low, w["w_a2t"], w["b_a2"], 1.0 / spec.tau)           # float32 [T, H D]
     o = hops.linear_scan(proj, 0, H * D, 2 * H * D, None, None, D ** -0.5, decay, None, meta.q_start, meta.pos0,
                          meta.slots, cache.S[li], H, H, D, Dv, max_q=meta.max_q)
     o = hops.head_norm_gate(o, proj, 2 * H * D + H * Dv, w["norm"], model.cfg.norm_eps, True, model.act_dtype)

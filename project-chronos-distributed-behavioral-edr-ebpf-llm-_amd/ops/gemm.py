@@ -298,12 +298,17 @@ def many_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
 
 def product_act(x: torch.Tensor, w: torch.Tensor, mode: int, limit: float = 0.0, slope: float = 0.0, shift: float = 0.0) -> Optional[torch.Tensor]:
     """x @ w.T with an activation in the epilogue (mode as in torch.ops.chronos.gemm_act: 3 a gated unit of w = [gate; up], 4 squared ReLU, 5
-    GELU), or None where that does not pay: where the best product (many_rows_plan's or, below it, as if it were) and a pass of its own are
+    GELU), or None where that does not pay: with up to 64 rows by _FEW_MORE, from 128 on where the best product (many_rows_plan's or, below it, as if it were) and a pass of its own are
     faster by their models.  On the grid of _MANY_88: gated units 1.13 times as fast (189 shapes; the worst 0.94), the others 1.16
     (196; 0.95)."""
     m, (n, k) = x.numel() // max(1, x.shape[-1]), w.shape
-    if m < MANY_MIN or PP_MODE != "auto" or x.dim() != 2 or not _plain_rows(x, w):
+    if 64 < m < MANY_MIN or PP_MODE != "auto" or x.dim() != 2 or not _plain_rows(x, w):
         return None
+    if m <= 64:
+        from . import _k
+
+        cfg = _few_more(m, n, k, 2 if mode == 3 else 1)
+        return _k().gemm_few(x, w, cfg, mode, 0, 0, None, limit, slope, shift)[0] if cfg else None
     glu = mode == 3
     rows = -(-m // 128) * 128
     key = (rows, n, k, -3 if glu else -4)
@@ -318,6 +323,38 @@ def product_act(x: torch.Tensor, w: torch.Tensor, mode: int, limit: float = 0.0,
     from . import _k
 
     return _k().gemm_act(x, w, mode, limit, slope, shift)
+
+
+# Few rows with more to do behind the product (gemm_few): by the most rows (config up to 8 M elements of weights, beyond; the most of them
+# where it wins with float32 outputs behind, with an activation, with a gated unit).  Measured at M = 1 .. 64 on six shapes of the first, three of the
+# others (K = 1024, 2048 and 4096), us, two launches -> one: 16 rows of 6144 x 2048 and 16 behind 15.8 -> 11.6, 12288 x 4096 and 64 36.8 -> 31.8; 32 rows
+# of that 32.8 -> 34.6; 16 rows of 8192 x 2048 with GELU 18.0 -> 12.3, 14336 x 4096 33.7 -> 33.2; gated units of 11264 x 2048 19.7 -> 18.0 (16 rows),
+# 19.6 -> 20.3 (32), of 5632 x 1024 9.1 -> 7.9 (32), 9.3 -> 9.0 (64).
+_FEW_MORE = ((16, 114, 115, 60e6, 24e6, 24e6), (32, 112, 116, 30e6, 24e6, 8e6), (64, 113, 117, 30e6, 24e6, 0))
+
+
+def _few_more(m: int, n: int, k: int, kind: int) -> int:
+    """Config of gemm_few, or 0: kind 0 float32 outputs behind, 1 an activation, 2 a gated unit."""
+    if not 0 < m <= 64 or PP_MODE != "auto" or 1 < m <= GEMV_MAX_M or n % 32 or n <= 0 or k % 64 or not 0 < k <= 1 << 20:
+        return 0
+    for most, small, large, *limits in _FEW_MORE:
+        if m <= most:
+            if n * k > limits[kind]:
+                return 0
+            return (large if kind == 2 or n * k > 8e6 else small) - SK_BASE
+    return 0
+
+
+def product_rows(x: torch.Tensor, w: torch.Tensor, n0: int, nf: int, bias: Optional[torch.Tensor]):
+    """(x @ w[:n0].T, float32 x @ w[n0 : n0 + nf].T + bias) in one launch, or None where two are faster."""
+    if x.dim() != 2 or not 0 < x.shape[0] <= 64 or not _plain_rows(x, w):
+        return None
+    cfg = _few_more(x.shape[0], *w.shape, 0)
+    if not cfg:
+        return None
+    from . import _k
+
+    return _k().gemm_few(x, w, cfg, 0, n0, nf, bias, 0.0, 0.0, 0.0)
 
 
 def _plain_rows(x: torch.Tensor, w: torch.Tensor) -> bool:

@@ -63,8 +63,10 @@ def matmul(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None) -
 def embed_rows(ids, table, act_dtype, scale: float = 1.0, emit: bool = True):
     """(float32 residual rows times ``scale``, the same rows in the activation dtype or None when ``emit`` is off)."""
     if _gpu(table):
+        if emit and not _f32(act_dtype):
+            return _k().hy_embed_both(ids, table, scale)
         x = _k().hy_embed(ids, table, scale)
-        return x, ((x if _f32(act_dtype) else _k().hy_cast_bf16(x)) if emit else None)
+        return x, (x if emit else None)
     return ref.embed_rows(ids, table, act_dtype, scale, emit)
 
 
@@ -87,6 +89,18 @@ def rowdot(h, w, bias=None):
     if _gpu(h):
         return _k().hy_rowdot(h, w, bias)
     return ref.rowdot(h, w, bias)
+
+
+def matmul_rowdot(h, w, w_few, bias=None, joined=None):
+    """(h @ w.T, rowdot(h, w_few, bias)); ``joined`` (whole, n0, nf): both matrices' rows one behind the other, which few rows of h take in
+    one launch."""
+    if joined is not None and _gpu(h) and h.dtype == torch.bfloat16:
+        from .gemm import product_rows
+
+        y = product_rows(h, *joined, bias)
+        if y is not None:
+            return y
+    return matmul(h, w), rowdot(h, w_few, bias)
 
 
 def act_inplace(x, kind: int):
@@ -269,9 +283,11 @@ def window_attention(qkv, kc, vc, block_table, q_start, pos, sink, gate, scale: 
     return o
 
 
-def short_conv(x, w, tok_seq, q_start, pos0, slots, hist, silu: bool = True, bias=None, x_off: int = 0):
+def short_conv(x, w, tok_seq, q_start, pos0, slots, hist, silu: bool = True, bias=None, x_off: int = 0, max_q: int = 0):
+    """``max_q``: the most tokens any sequence brings in this step (with 1 the history is rewritten in the same pass; 0 =
+    unknown)."""
     if _gpu(x):
-        return _k().hy_short_conv(x, w, tok_seq, q_start, pos0, slots, hist, silu, bias, x_off)
+        return _k().hy_short_conv(x, w, tok_seq, q_start, pos0, slots, hist, silu, bias, x_off, max_q)
     return ref.short_conv(x, w, q_start, pos0, slots, hist, silu, bias, x_off)
 
 
@@ -286,6 +302,13 @@ def decay_pow(z, inv_tau: float):
         _k().hy_decay_pow(z, inv_tau)
         return z
     return ref.decay_pow(z, inv_tau)
+
+
+def low_rank_decay(a, w, b, inv_tau: float):
+    """sigmoid(b + a @ w) ** inv_tau, float32: a [T, rank], w [rank, C], b [C]."""
+    if _gpu(a) and w.shape[1] % 4 == 0:
+        return _k().hy_low_rank_decay(a, w, b, inv_tau)
+    return decay_pow(torch.addmm(b, a, w), inv_tau)
 
 
 def linear_scan(proj, q_off: int, k_off: int, v_off: int, qscale, kscale, q_mul: float, decay, beta, q_start, pos0,

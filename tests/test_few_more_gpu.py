@@ -1,0 +1,113 @@
+"""Launches that took over a neighbour's work: few-row products with float32 rows or an activation behind (gemm_few), the low-rank decays in
+one kernel, the embedding's two copies, the convolution that rewrites its history, the plain layer norm of float rows."""
+import pytest
+import torch
+
+DEV = "cuda"
+BF = torch.bfloat16
+pytestmark = pytest.mark.gpu
+
+
+def _g(seed):
+    return torch.Generator(device=DEV).manual_seed(seed)
+
+
+def _check(y, want):
+    """float32 sums and one rounding to bfloat16: 2^-8 |y| + 1e-4 rms(y)."""
+    assert ((y.double() - want).abs() <= want.abs() * 2 ** -8 + 1e-4 * want.square().mean().sqrt()).all()
+
+
+@pytest.mark.parametrize("m", [1, 2, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("n0,nf,k", [(512, 8, 64), (1040, 13, 576), (3072, 1, 1024), (4, 60, 192)])
+@pytest.mark.parametrize("with_bias", [False, True])
+def test_rows_behind(m, n0, nf, k, with_bias):
+    from chronos.models.hybrid import _rows_behind
+    from chronos.ops import gemm as G, hybrid as H
+
+    g = _g(m + n0 + nf)
+    x, a, b = (torch.randn(s, device=DEV, generator=g).to(BF) for s in ((m, k), (n0, k), (nf, k)))
+    bias = torch.randn(nf, device=DEV, generator=g) if with_bias else None
+    out = _rows_behind(dict(a=a, b=b), "a", "b")
+    rows, m0, mf = out["joined"]
+    assert rows.shape[0] % 32 == 0 and (m0, mf) == (n0, nf) and torch.equal(out["a"], a) and torch.equal(out["b"], b)
+    y, yf = G.product_rows(x, *out["joined"], bias)
+    _check(y, x.double() @ a.double().t())
+    want = x.double() @ b.double().t() + (0 if bias is None else bias.double())
+    assert yf.dtype == torch.float32 and yf.shape == (m, nf)
+    assert (yf.double() - want).abs().max() <= 2e-6 * k ** 0.5 * want.abs().max()      # float32 sums of exact products
+    y2, yf2 = H.matmul_rowdot(x, out["a"], out["b"], bias, out["joined"])
+    assert torch.equal(y, y2) and torch.equal(yf, yf2)
+
+
+@pytest.mark.parametrize("m", [1, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("n,k", [(64, 64), (1056, 576), (5632, 1024), (8192, 2048)])
+def test_activations(m, n, k):
+    from chronos.ops import hybrid as H
+
+    g = _g(m + n + k)
+    x, w = torch.randn(m, k, device=DEV, generator=g).to(BF), (torch.randn(n, k, device=DEV, generator=g) * k ** -0.5).to(BF)
+    h = x.double() @ w.double().t()
+    F = n // 2
+    for limit, slope, shift in ((float("inf"), 1.0, 0.0), (0.75, 1.702, 1.0)):
+        a, u = h[:, :F].clamp(max=limit), h[:, F:].clamp(-limit, limit)
+        want = a * torch.sigmoid(slope * a) * (u + shift)
+        y = H.matmul_glu(x, w, limit, slope, shift, BF)
+        assert ((y.double() - want).norm() / want.norm()).item() < 2 ** -7
+    for kind, want in ((H.ACT_RELU2, h.relu() ** 2), (H.ACT_GELU, torch.nn.functional.gelu(h))):
+        y = H.matmul_act(x, w, kind)
+        assert ((y.double() - want).norm() / want.norm()).item() < 2 ** -7
+
+
+@pytest.mark.parametrize("T,R,C", [(1, 16, 512), (3, 1, 4), (21, 16, 2048), (700, 16, 4096), (2500, 7, 1028)])
+@pytest.mark.parametrize("p", [1.0 / 16, 0.25])
+def test_low_rank_decay(T, R, C, p):
+    from chronos.ops import hybrid as H
+
+    g = _g(T + R + C)
+    a, w, b = (torch.randn(s, device=DEV, generator=g) for s in ((T, R), (R, C), (C,)))
+    a[0, 0] = 40.0
+    want = torch.sigmoid(b.double() + a.double() @ w.double()) ** p
+    ours = H.low_rank_decay(a, w, b, p)
+    theirs = H.decay_pow(torch.addmm(b, a, w), p)     # the two launches it replaces
+    assert (ours.double() - want).norm() <= 1.05 * (theirs.double() - want).norm() + 1e-7 * want.norm()
+
+
+@pytest.mark.parametrize("d", [64, 1000, 2052])
+@pytest.mark.parametrize("dt", [BF, torch.float32])
+def test_embed_both(d, dt):
+    from chronos.ops import hybrid as H
+
+    table = torch.randn(50, d, device=DEV, generator=_g(d)).to(dt)
+    ids = torch.tensor([3, 49, 0, 3], dtype=torch.int32, device=DEV)
+    x, h = H.embed_rows(ids, table, BF, 1.5)
+    assert torch.equal(x, table[ids.long()].float() * 1.5) and h.dtype == BF and torch.equal(h, x.to(BF))
+
+
+@pytest.mark.parametrize("C,K", [(512, 4), (1032, 2), (100, 3), (64, 6)])
+def test_one_token_each_convolution(C, K):
+    """max_q = 1 gives the bits of the two launches, outputs and history: a first token, one in the middle, a sequence without a token."""
+    from chronos.ops import hybrid as H
+
+    g = _g(C + K)
+    x, w = torch.randn(3, C, device=DEV, generator=g).to(BF), torch.randn(C, K, device=DEV, generator=g)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    hist = torch.randn(6, K - 1, C, device=DEV, generator=g).to(BF)
+    args = (x, w, i32([0, 1, 3]), i32([0, 1, 2, 2, 3]), i32([0, 5, 9, 1]), i32([4, 1, 3, 0]))
+    h1, h2 = hist.clone(), hist.clone()
+    y1, y2 = H.short_conv(*args, h1, True), H.short_conv(*args, h2, True, max_q=1)
+    assert torch.equal(y1, y2) and torch.equal(h1, h2)
+    assert torch.equal(h2[3], hist[3]) and torch.equal(h2[4, -1], x[0])
+
+
+@pytest.mark.parametrize("rows,d", [(1, 4), (64, 4096), (7, 1000), (3, 2052), (2, 5000)])
+@pytest.mark.parametrize("dt", [BF, torch.float32])
+def test_plain_layer_norm(rows, d, dt):
+    from chronos.ops import hybrid as H
+
+    x = torch.randn(rows, d, device=DEV, generator=_g(rows + d)) * 3 + 1
+    w = torch.randn(d, device=DEV, generator=_g(d))
+    want = torch.nn.functional.layer_norm(x.double(), (d,), w.double(), None, 1e-5)
+    y = H.layer_norm(x, w, 1e-5, dt)
+    assert y.dtype == dt
+    tol = 2 ** -8 if dt == BF else 2e-6
+    assert ((y.double() - want).abs() <= want.abs() * tol + 2e-6 * want.abs().max()).all()
