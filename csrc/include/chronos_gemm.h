@@ -64,6 +64,8 @@ constexpr int kSkinnyUneven = 12;  // from this config on: plain epilogue and ac
 int gemm_skinny_rt(int cfg);
 int gemm_skinny_mt(int cfg);
 int gemm_skinny_nw(int cfg);  // waves per workgroup
+// y [n] = the sum of S float32 slices [S, n], in their order
+void launch_gemm_slices(const float* ws, uint16_t* y, int64_t n, int S, hipStream_t st);
 bool launch_gemm_skinny(int cfg, int mode, bool normp, const PPArgs& a, hipStream_t st);
 
 }  // namespace chronos

@@ -687,6 +687,37 @@ std::tuple<Tensor, Tensor> gemm_few(const Tensor& x, const Tensor& w, int64_t cf
     return {y, yf};
 }
 
+// A plain product of few rows whose K is split over workgroups, nothing kept between calls (gemm_lg.hip's 64-row tiles and smaller).
+Tensor gemm_split(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk) {
+    chk_bf16(x, "x");
+    chk_bf16(w, "w");
+    const int64_t K = x.size(-1), M = x.numel() / K, N = w.size(0);
+    CHK(w.dim() == 2 && w.size(1) == K, "gemm_split: w must be [N, K]");
+    CHK(cfg == 33 || cfg == 36 || (cfg >= 38 && cfg <= 39) || (cfg >= 72 && cfg <= 75) || cfg == 78 || cfg == 79, "gemm_split: cfg");
+    const int BM = chronos::gemm_lg_xm((int)cfg), BN = chronos::gemm_lg_wn((int)cfg);
+    CHK((N + BN) * K * 2 < (1LL << 31) && (M + BM) * K * 2 < (1LL << 31), "gemm_split: operand > 2 GiB");
+    CHK(M >= 1 && K % 64 == 0 && K <= (1 << 20) && N >= 4 && N % 4 == 0, "gemm_split: size");
+    CHK(splitk > 1 && splitk <= 64 && (K / 64) % splitk == 0, "gemm_split: splitk must divide K / 64");
+    CHK(((reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr())) & 15) == 0, "gemm_split: alignment");
+    c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+    chronos::PPArgs a{};
+    a.x = bf(x);
+    a.w = bf(w);
+    a.M = (int)M;
+    a.N = (int)N;
+    a.K = (int)K;
+    a.F = (int)(N / 2);
+    a.splitk = (int)splitk;
+    a.kts = (int)(K / 64 / splitk);
+    a.gm = chronos::knob("pp_gm", 8);
+    Tensor y = at::empty({M, N}, x.options()), ws = at::empty({splitk * M * N}, x.options().dtype(at::kFloat));
+    a.y = bfm(y);
+    a.ws = ws.data_ptr<float>();
+    CHK(chronos::launch_gemm_lg((int)cfg, 0, false, a, cur_stream()), "gemm_split: launch");
+    chronos::launch_gemm_slices(a.ws, a.y, M * N, (int)splitk, cur_stream());
+    return y;
+}
+
 // Skinny-M GEMM (gemm_skinny.hip), M <= 16 * MT of the config: same epilogues and tensors as gemm_pp; the kResid
 // partials are [M, N / (16 * RT)].
 std::tuple<Tensor, Tensor> gemm_skinny(const Tensor& x, const Tensor& w, int64_t mode, int64_t cfg, int64_t splitk,
@@ -910,6 +941,7 @@ TORCH_LIBRARY(chronos, m) {
     m.def("gemm(Tensor x, Tensor w, bool swiglu, int stages=3) -> Tensor");
     m.def("gemm_act(Tensor x, Tensor w, int mode, float limit, float slope, float shift) -> Tensor");
     m.def("gemm_few(Tensor x, Tensor w, int cfg, int mode, int n0, int nf, Tensor? bias, float limit, float slope, float shift) -> (Tensor, Tensor)");
+    m.def("gemm_split(Tensor x, Tensor w, int cfg, int splitk) -> Tensor");
     m.def("gemm_pp(Tensor x, Tensor w, int mode, int cfg, int splitk, Tensor? resid, Tensor? part_in, float eps, bool prio) -> (Tensor, Tensor)");
     m.def("gemm_skinny(Tensor x, Tensor w, int mode, int cfg, int splitk, Tensor? resid, Tensor? part_in, float eps) "
           "-> (Tensor, Tensor)");
@@ -954,6 +986,7 @@ TORCH_LIBRARY_IMPL(chronos, CUDA, m) {
     m.impl("gemm", &gemm);
     m.impl("gemm_act", &gemm_act);
     m.impl("gemm_few", &gemm_few);
+    m.impl("gemm_split", &gemm_split);
     m.impl("gemm_pp", &gemm_pp);
     m.impl("gemm_skinny", &gemm_skinny);
     m.impl("gemv_resid", &gemv_resid);

@@ -982,6 +982,23 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
         return;
     }
 
+    // ---- split-K without state (plain, no tickets): the slice's sums [S, M, N], which a second launch adds up
+    if constexpr (MODE == kPlain && !NORMP && !HB && !F8 && !M32 && ABL == 0) {
+        if (S > 1 && a.cnt == nullptr) {
+#pragma unroll
+            for (int u = 0; u < MT; ++u) {
+                const int m = m0 + xrow0 + 16 * u + (lane & 15);
+                if (m >= M) continue;
+#pragma unroll
+                for (int s = 0; s < NT; ++s) {
+                    const int n = tn * WN + wrow0[s] + 4 * (lane >> 4);
+                    if (n < a.N) *reinterpret_cast<f32x4*>(a.ws + ((int64_t)ks * M + m) * a.N + n) = acc[s][u];   // N % 4 == 0
+                }
+            }
+            return;
+        }
+    }
+
     // ---- split-K: fp32 slab in register order, ticket, the last arriver sums every slab in slice order
     if (!HB && S > 1) {  // (HB has its own above)
         // slab hand-off: plain stores + agent release / acquire fences (each a write-back / invalidate of the XCD's

@@ -345,6 +345,14 @@ __global__ void __launch_bounds__(256) skinny_sum_kernel(const float* __restrict
     *reinterpret_cast<u16x4*>(y + i) = o;
 }
 
+}  // namespace
+
+void launch_gemm_slices(const float* ws, uint16_t* y, int64_t n, int S, hipStream_t st) {   // n % 4 == 0
+    skinny_sum_kernel<<<(unsigned)((n / 4 + 255) / 256), 256, 0, st>>>(ws, y, n, S);
+}
+
+namespace {
+
 template <int RT, int MT, int D, int NW, int MODE, bool NORMP>
 void launch_cfg(const PPArgs& a, hipStream_t st) {
     constexpr int UNITS = RT * MT * 64;
@@ -358,10 +366,7 @@ void launch_cfg(const PPArgs& a, hipStream_t st) {
     }
     const int G = sk_pair(MODE) ? a.F / (8 * RT) : a.N / (16 * RT);
     hipLaunchKernelGGL(kern, dim3(G * a.splitk), dim3(64 * NW), lds, st, a);
-    if (a.splitk > 1 && a.cnt == nullptr) {
-        const int64_t n = (int64_t)a.M * a.N;
-        skinny_sum_kernel<<<(unsigned)((n / 4 + 255) / 256), 256, 0, st>>>(a.ws, a.y, n, a.splitk);
-    }
+    if (a.splitk > 1 && a.cnt == nullptr) launch_gemm_slices(a.ws, a.y, (int64_t)a.M * a.N, a.splitk, st);
 }
 
 // configs {RT (W tiles of 16 rows per workgroup), MT (x tiles: M <= 16 MT), D (ring depth in 64-k units), NW (waves

@@ -545,12 +545,12 @@ class HybridWeights:
         return n
 
 
-def _in_proj(rows: list, t: dict, out: dict, key: str, cast, gate: bool = False) -> None:
+def _in_proj(rows: list, t: dict, out: dict, key: str, cast, gate: bool = False, behind=None) -> None:
     """out[key] = the sublayer's first projection: ``rows`` stacked and behind them what else reads the same input, each
     from a column of its own on: with t["rg"] a residual gate's rows (out["rg_off"]); with t["ff"] = (spec, gate and up
     rows, down) the first projection of a gated feed-forward that runs beside the mixer (out["ff"] = its column and
     its spec) and, with ``gate``, the per-head gate's rows t["g"] (out["g_off"]).  The latter start on multiples of 8
-    columns and end on one of 16 (rows of zeros between)."""
+    columns and end on one of 16 (rows of zeros between).  ``behind`` = (name, rows): see _stacked."""
     if "rg" in t:
         out["rg_off"] = sum(r.shape[0] for r in rows)
         rows = rows + [t["rg"]]
@@ -575,6 +575,9 @@ def _in_proj(rows: list, t: dict, out: dict, key: str, cast, gate: bool = False)
             out["g_off"] = n
             put(t["g"], 16)
         rows = stack
+    if behind is not None:
+        _stacked(rows, behind[1], cast, out, key, behind[0])
+        return
     out[key] = cast(rows[0] if len(rows) == 1 else torch.cat(rows, 0))
 
 
@@ -591,15 +594,14 @@ def ff_rides_along(mixer, ff) -> bool:
         ff.ff % 8 == 0 and mixer.heads * mixer.vdim % 8 == 0
 
 
-def _rows_behind(out: dict, key: str, few: str) -> dict:
-    """out[few], the rows of a float32-output projection, moved behind those of out[key], which reads the same input (both stay as
-    views): out["joined"] = (all rows and zeros up to a multiple of 32, rows of out[key], rows of out[few]) for hops.matmul_rowdot."""
-    a, b = out[key], out[few]
-    if a.is_cuda and a.dtype == b.dtype == torch.bfloat16 and a.shape[0] % 4 == 0 and a.shape[1] % 64 == 0:
-        n0, nf = a.shape[0], b.shape[0]
-        rows = torch.zeros(-(-(n0 + nf) // 32) * 32, a.shape[1], device=a.device, dtype=a.dtype)
-        rows[:n0], rows[n0:n0 + nf] = a, b
-        out[key], out[few], out["joined"] = rows[:n0], rows[n0:n0 + nf], (rows, n0, nf)
+def _stacked(rows: list, behind, cast, out: dict, key: str, few: str) -> dict:
+    """out[key] = ``rows`` stacked, out[few] = ``behind``, the rows of a float32-output projection that reads the same input: views of one
+    matrix, out["joined"] = (it, with zeros up to a multiple of 32 rows, rows of out[key], rows of out[few]) for hops.matmul_rowdot."""
+    n0, nf = sum(r.shape[0] for r in rows), behind.shape[0]
+    whole = cast(torch.cat([*rows, behind, behind.new_zeros(-(n0 + nf) % 32, behind.shape[1])], 0))
+    out[key], out[few] = whole[:n0], whole[n0:n0 + nf]
+    if whole.is_cuda and whole.dtype == torch.bfloat16 and n0 % 4 == 0 and whole.shape[1] % 64 == 0:
+        out["joined"] = (whole, n0, nf)
     return out
 
 
@@ -608,8 +610,8 @@ def pack_mlstm(spec: MLSTMSpec, t: dict, device, act_dtype) -> dict:
     the two gate rows one few-row float32-output projection."""
     a = lambda x: x.to(device=device, dtype=act_dtype).contiguous()  # noqa: E731
     f = lambda x: x.to(device=device, dtype=torch.float32).contiguous()  # noqa: E731
-    return _rows_behind(dict(w_proj=a(torch.cat([t["q"], t["k"], t["v"], t["g"]], 0)), w_if=a(torch.cat([t["i"], t["f"]], 0)),
-                             b_if=f(torch.cat([t["i.b"], t["f.b"]], 0)), norm=f(t["norm"]), w_o=a(t["o"])), "w_proj", "w_if")
+    out = dict(b_if=f(torch.cat([t["i.b"], t["f.b"]], 0)), norm=f(t["norm"]), w_o=a(t["o"]))
+    return _stacked([t["q"], t["k"], t["v"], t["g"]], torch.cat([t["i"], t["f"]], 0), a, out, "w_proj", "w_if")
 
 
 def pack_latent(spec: LatentAttentionSpec, t: dict, device, act_dtype) -> dict:
@@ -633,13 +635,11 @@ def pack_latent(spec: LatentAttentionSpec, t: dict, device, act_dtype) -> dict:
     if spec.kv_from is None:
         out["dkv_norm"] = f(t["dkv.norm"])
         rows.append(t["dkv"])
-    _in_proj(rows + ([t["g"]] if spec.gate and spec.gate_wide else []), t, out, "w_in", a)
+    _in_proj(rows + ([t["g"]] if spec.gate and spec.gate_wide else []), t, out, "w_in", a,
+             behind=("w_g", t["g"]) if spec.gate and not spec.gate_wide else None)
     _out_proj(t, out, a)
     if spec.sink:
         out["sink"] = f(t["sink"])
-    if spec.gate and not spec.gate_wide:
-        out["w_g"] = a(t["g"])
-        _rows_behind(out, "w_in", "w_g")
     return out
 
 
@@ -679,7 +679,7 @@ def pack_window_attention(spec: WindowAttentionSpec, t: dict, device, act_dtype)
     rows = [t["q"], t["k"]] + ([] if spec.v_from_k else [t["v"]]) + ([t["g"]] if spec.gate and spec.gate_wide else [])
     out = {}
     few = spec.gate and not spec.gate_wide
-    _in_proj(rows, t, out, "w_qkv", a, few)
+    _in_proj(rows, t, out, "w_qkv", a, few, behind=("w_g", t["g"]) if few and "ff" not in t and not spec.bias else None)
     _out_proj(t, out, a)
     if spec.conv:
         out["taps"] = f(torch.cat([t["q.conv"], t["k.conv"]] + ([] if spec.v_from_k else [t["v.conv"]]), 0))
@@ -688,10 +688,8 @@ def pack_window_attention(spec: WindowAttentionSpec, t: dict, device, act_dtype)
         out.update(q_norm=f(t["q.norm"] if spec.qk_norm_weight else one), k_norm=f(t["k.norm"] if spec.qk_norm_weight else one))
     if spec.sink:
         out["sink"] = f(t["sink"] if spec.sink_fixed is None else torch.full((spec.heads,), float(spec.sink_fixed)))
-    if few and "g_off" not in out:
+    if few and "g_off" not in out and "w_g" not in out:
         out["w_g"] = a(t["g"])
-        if not spec.bias:
-            _rows_behind(out, "w_qkv", "w_g")
     if spec.bias:
         rest = out["w_qkv"].shape[0] - spec.heads * spec.dim - spec.kv_heads * (spec.dim + spec.vdim)  # gate rows: none
         out["b_qkv"] = a(torch.cat([t["q.b"], t["k.b"], t["v.b"], torch.zeros(rest, dtype=t["q.b"].dtype)], 0))
@@ -708,9 +706,9 @@ def pack_mamba2(spec: Mamba2Spec, t: dict, device, act_dtype) -> dict:
     a = lambda x: x.to(device=device, dtype=act_dtype).contiguous()  # noqa: E731
     f = lambda x: x.to(device=device, dtype=torch.float32).contiguous()  # noqa: E731
     n = 2 * spec.inner + 2 * spec.groups * spec.state
-    out = dict(w_in=a(t["in"][:n]), w_dt=a(t["in"][n:]), b_dt=f(t["dt_bias"]), taps=f(t["conv"]),
-               b_conv=f(t["conv.b"]), a_log=f(t["A_log"]), skip=f(t["D"]), norm=f(t["norm"]), w_o=a(t["o"]))
-    return _rows_behind(out, "w_in", "w_dt")
+    out = dict(b_dt=f(t["dt_bias"]), taps=f(t["conv"]), b_conv=f(t["conv.b"]), a_log=f(t["A_log"]), skip=f(t["D"]), norm=f(t["norm"]),
+               w_o=a(t["o"]))
+    return _stacked([t["in"][:n]], t["in"][n:], a, out, "w_in", "w_dt")
 
 
 def pack_rglru(spec: RGLRUSpec, t: dict, device, act_dtype) -> dict:
@@ -732,12 +730,10 @@ def pack_delta_rule(spec: DeltaRuleSpec, t: dict, device, act_dtype) -> dict:
     float32-output projection (bias: dt_bias for the decay rows, zero for the others)."""
     a = lambda x: x.to(device=device, dtype=act_dtype).contiguous()  # noqa: E731
     f = lambda x: x.to(device=device, dtype=torch.float32).contiguous()  # noqa: E731
-    out = dict(w_proj=a(torch.cat([t["q"], t["k"], t["v"], t["g"]], 0)),
-               taps=f(torch.cat([t["q.conv"], t["k.conv"], t["v.conv"]], 0)),
-               w_ab=a(torch.cat([t["a"], t["b"]], 0)),
+    out = dict(taps=f(torch.cat([t["q.conv"], t["k.conv"], t["v.conv"]], 0)),
                b_ab=f(torch.cat([t["dt_bias"].float(), torch.zeros(spec.heads)], 0)), a_log=f(t["A_log"]),
                norm=f(t["norm"].float().repeat(spec.heads)), w_o=a(t["o"]))
-    return _rows_behind(out, "w_proj", "w_ab")
+    return _stacked([t["q"], t["k"], t["v"], t["g"]], torch.cat([t["a"], t["b"]], 0), a, out, "w_proj", "w_ab")
 
 
 def pack_gla(spec: GLASpec, t: dict, device, act_dtype) -> dict:
@@ -745,10 +741,10 @@ def pack_gla(spec: GLASpec, t: dict, device, act_dtype) -> dict:
     float32 outputs (a1 through the few-row projection, a2 as a float32 matrix)."""
     a = lambda x: x.to(device=device, dtype=act_dtype).contiguous()  # noqa: E731
     f = lambda x: x.to(device=device, dtype=torch.float32).contiguous()  # noqa: E731
-    out = dict(w_a1=a(t["a1"]), w_a2t=f(t["a2"].float().t()), b_a2=f(t["a2.b"]),
+    out = dict(w_a2t=f(t["a2"].float().t()), b_a2=f(t["a2.b"]),
                norm=f(t["norm"].float().repeat(spec.heads)), w_o=a(t["o"]))
-    _in_proj([t["q"], t["k"], t["v"], t["g"]], t, out, "w_proj", a)
-    return _rows_behind(out, "w_proj", "w_a1")
+    _in_proj([t["q"], t["k"], t["v"], t["g"]], t, out, "w_proj", a, behind=("w_a1", t["a1"]))
+    return out
 
 
 def pack_retention(spec: RetentionSpec, t: dict, device, act_dtype) -> dict:

@@ -77,6 +77,11 @@ _FEW = ((16, {114: (2.4, 2.0, 0.77, 0.016, 0.23, 0.69, 3.4), 115: (2.2, 2.1, 1.4
               75: (1.8, 0.0, 0.29, 0.085, 1.7, 0.0, 12.0)}),
         (64, {113: (2.4, 2.3, 1.5, 0.0, 0.9, 1.0, 0.75), 72: (2.2, 0.0, 0.16, 0.0, 1.3, 0.19, 5.1),
               38: (3.0, 0.0, 0.31, 0.0, 0.54, 0.0, 35.0), 39: (2.4, 0.0, 0.21, 0.0, 1.2, 0.22, 14.0)}))
+# Few rows, more weights than that: gemm_lg.hip's small tiles, K split over workgroups without tickets (gemm_split).  The same terms, and per M
+# of partial sums (rms error 7 %), fitted at 19 shapes of 4 to 134 M elements by 2 .. 64 rows.
+_FEW_LARGE = ((32, {72: (2.1, 1.8, 0.13, 0.122, 1.54, 0.121, 0.17, 1.5), 74: (1.1, 2.35, 0.189, 0.118, 0.8, 0.099, 0.12, 1.7),
+                    79: (2.6, 1.9, 0.139, 0.101, 1.8, 0.17, 0.26, 1.4)}),
+              (64, {39: (1.1, 2.7, 0.223, 0.0915, 0.94, 0.229, 0.0, 1.9), 38: (1.4, 2.7, 0.35, 0.105, 1.65, 0.259, 0.0, 1.7)}))
 _plan_cache: dict = {}
 _plan_table: Optional[dict] = None
 _qplan_table: Optional[dict] = None
@@ -211,8 +216,11 @@ def few_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     two are level), and K % 512, which the GEMV does not take (1024 x 2816: 8.6 -> 5.7): no slower at any of 41 shapes;
     2 .. 64 rows: weights up to 12.5 M elements, from 33 rows on up to 7 M or K <= 2048 (2048 x 2048, 16 rows: 11.0 -> 6.0; 64 rows:
     11.7 -> 8.1): 1.3 .. 1.6 times as fast on average, 4 of 590 slower by more than 3 %, the worst by 6 %; 48 shapes off the grid: 1.7
-    times, none slower.  More weights than that stream from memory at the library's rate too (8192 x 8192, 16 rows: 30.5, 31.1 here),
-    except that it keeps half the chip idle for wide outputs of up to 48 rows (22016 x 2048, 16 rows: 44 -> 21)."""
+    times, none slower.  Where the library keeps half the
+    chip idle, wide outputs of up to 48 rows, more weights too (22016 x 2048, 16 rows: 44 -> 21).
+    Beyond, 2 .. 64 rows: _FEW_LARGE, from 33 rows on for less than 12288 outputs: library -> this, 16 rows of 4096 x 4096 16.1 -> 11.6, 4096 x
+    11008 36.6 -> 21.8, 12288 x 4096 29.3 -> 23.8; 64 rows of 4096 x 14336 40.4 -> 28.7, 2048 x 8192 23.1 -> 13.9: 1.15 times on average over 96; 8
+    slower by 3 % or more, the worst 4096 x 8192 with 8 rows 16.8 -> 20.2; 64 rows of 14336 x 4096 would be 28.3 -> 30.2."""
     if 1 < m <= GEMV_MAX_M or PP_MODE != "auto":   # (programs set both while they run: nothing of them in the cache)
         return None
     key = (m, n, k, -1)
@@ -236,6 +244,18 @@ def few_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
                 steps = k / (64 * sk * nw)
                 t = (c[0] + c[1] * (sk > 1) + c[2] * steps + c[3] * nk * 2e-6 + c[4] * groups / 256
                      + c[5] * (-(-groups // 256) - 1) * steps + c[6] * m * k * groups * 2e-8)
+                if best is None or t < best:
+                    best, out = t, (cfg, sk)
+    elif 1 < m <= 64 and n > 0 and n % 16 == 0 and 4_000_000 <= nk and (n + 128) * k < 1 << 30 and k % 64 == 0 and 0 < k <= 1 << 20 and (
+            m <= 32 or n < 12288) and (n, k, PP_PLAIN) not in _plan_file():
+        best = None
+        for cfg, c in next(models for most, models in _FEW_LARGE if m <= most).items():
+            for sk in (1, 2, 4, 8):
+                groups, steps = -(-n // _PP_BN[cfg]) * sk, k / (64 * sk)
+                if k // 64 % sk or (sk > 1 and groups > 2048):
+                    continue
+                t = (c[0] + c[1] * (sk > 1) + c[2] * steps + c[3] * nk * 2e-6 + c[4] * groups / 256
+                     + c[5] * (-(-groups // 256) - 1) * steps + c[6] * m * k * groups * 2e-8 + c[7] * sk * m * n * 1e-6)
                 if best is None or t < best:
                     best, out = t, (cfg, sk)
     _plan_cache[key] = out
@@ -580,6 +600,10 @@ def linear(x, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tens
         for pred, fn in _custom:
             if pred(m, n, k):
                 return fn(x, w)
+        if few is not None and few[1] > 1 and few[0] < SK_BASE:   # a split without tickets
+            from . import _k
+
+            return _k().gemm_split(x.reshape(-1, k), w, *few).view(*x.shape[:-1], n)
         plan = (few or pp_plan(m, n, k, PP_PLAIN)) if out is None else None
         if plan is not None:
             y, _ = pp_gemm(x, w, PP_PLAIN, plan)

@@ -21,13 +21,13 @@ def _check(y, want):
 @pytest.mark.parametrize("n0,nf,k", [(512, 8, 64), (1040, 13, 576), (3072, 1, 1024), (4, 60, 192)])
 @pytest.mark.parametrize("with_bias", [False, True])
 def test_rows_behind(m, n0, nf, k, with_bias):
-    from chronos.models.hybrid import _rows_behind
+    from chronos.models.hybrid import _stacked
     from chronos.ops import gemm as G, hybrid as H
 
     g = _g(m + n0 + nf)
     x, a, b = (torch.randn(s, device=DEV, generator=g).to(BF) for s in ((m, k), (n0, k), (nf, k)))
     bias = torch.randn(nf, device=DEV, generator=g) if with_bias else None
-    out = _rows_behind(dict(a=a, b=b), "a", "b")
+    out = _stacked([a[:n0 // 2], a[n0 // 2:]], b, lambda t: t.contiguous(), {}, "a", "b")
     rows, m0, mf = out["joined"]
     assert rows.shape[0] % 32 == 0 and (m0, mf) == (n0, nf) and torch.equal(out["a"], a) and torch.equal(out["b"], b)
     y, yf = G.product_rows(x, *out["joined"], bias)
@@ -111,3 +111,22 @@ def test_plain_layer_norm(rows, d, dt):
     assert y.dtype == dt
     tol = 2 ** -8 if dt == BF else 2e-6
     assert ((y.double() - want).abs() <= want.abs() * tol + 2e-6 * want.abs().max()).all()
+
+
+@pytest.mark.parametrize("m", [2, 16, 31, 32, 33, 64])
+@pytest.mark.parametrize("n,k", [(2064, 2048), (4096, 4096), (1040, 14336), (12304, 1024), (4112, 11008)])
+def test_large_weights_split(m, n, k):
+    """ops.linear where few_rows_plan splits K over workgroups without tickets: twice the same bits, float64 within the roundings."""
+    from chronos import ops
+    from chronos.ops import gemm as G
+
+    g = _g(m + n + k)
+    x, w = torch.randn(m, k, device=DEV, generator=g).to(BF), torch.randn(n, k, device=DEV, generator=g).to(BF)
+    want = x.double() @ w.double().t()
+    y = ops.linear(x, w)
+    _check(y, want)
+    assert torch.equal(y, ops.linear(x, w))
+    for cfg in (72, 74, 79) if m <= 32 else (38, 39):
+        for sk in (2, 4, 8):
+            if k // 64 % sk == 0:
+                _check(torch.ops.chronos.gemm_split(x, w, cfg, sk), want)
