@@ -81,6 +81,20 @@ __device__ __forceinline__ void dma_1k_buf(const void* base, uint32_t bytes, uin
                  ::"v"(voff), "s"(r), "s"(lds), "s"(soff) : "memory");
 }
 __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// All but the PW pieces of each of the AHEAD newest tiles, or of the `left` that are still to come, have landed
+template <int PW, int AHEAD> __device__ __forceinline__ void dma_wait_for(int left) {
+    static_assert(PW * AHEAD < 64, "counted waits");
+    if constexpr (AHEAD > 0) {
+        if (left >= AHEAD) {
+            __builtin_amdgcn_s_waitcnt(((PW * AHEAD) & 0xF) | (0x7 << 4) | (0xF << 8) | (((PW * AHEAD) >> 4) << 14));
+            asm volatile("" ::: "memory");
+        } else {
+            dma_wait_for<PW, AHEAD - 1>(left);
+        }
+    } else {
+        dma_wait();
+    }
+}
 __device__ __forceinline__ uint32_t lds_offset(const void* p) {
     typedef __attribute__((address_space(3))) const void* lds_ptr;
     return (uint32_t)(uintptr_t)(lds_ptr)p;
@@ -88,9 +102,10 @@ __device__ __forceinline__ uint32_t lds_offset(const void* p) {
 // Piece j of a tile of rows: an LDS image of row-major rows, each CPR chunks of 16 bytes of which the last is padding
 // (it spreads the rows over the banks; like the chunks past the row's n real ones it receives a copy of the last real
 // one).  rows: element offset factor of each row of the tile; width: elements per row in memory.
-template <int CPR> __device__ __forceinline__ void dma_rows(const uint16_t* src, const int* rows, int width, int n, int j,
+// KT > 0: the tile has KT rows; chunks past them (a tile's last piece may hold some) repeat its last row.
+template <int CPR, int KT = 0> __device__ __forceinline__ void dma_rows(const uint16_t* src, const int* rows, int width, int n, int j,
                                                             uint32_t lds, int lane) {
-    const int i = j * 64 + lane, row = i / CPR, ch = i - row * CPR;
+    const int i = j * 64 + lane, at = i / CPR, ch = i - at * CPR, row = KT > 0 ? min(at, KT - 1) : at;
     dma_1k(src + (int64_t)rows[row] * width + min(ch, n - 1) * 8, __builtin_amdgcn_readfirstlane(lds + j * 1024));
 }
 

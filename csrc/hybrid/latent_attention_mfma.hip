@@ -3,8 +3,8 @@
 //
 // One workgroup takes up to 128 (token, head) rows of one sequence — 16 per wave, rows are (token * H + head), so any
 // head count tiles the same way — and walks the sequence's keys 64 at a time:
-//   * the key tile goes from memory straight into LDS (no staging registers), row-major [64][DK], two tiles deep: the
-//     next tile is on its way while the current one is computed, one barrier per tile.  Both MFMA operands want 8
+//   * the key tile goes from memory straight into LDS (no staging registers), row-major [KT][DK], NB tiles deep: the
+//     next ones are on their way while one is computed, one barrier per tile.  Both MFMA operands want 8
 //     k-values per lane — dims for the scores, KEYS for the weighted sum: the scores read rows as they lie, the sum
 //     reads the same image through gfx950's transposing LDS reads (4 keys of 16 columns each).
 //   * scores  S^T = K Q^T : 16x16x32 MFMAs with the key rows as A operand and the wave's 16 query rows (held in
@@ -25,7 +25,8 @@
 namespace chronos {
 namespace hy {
 
-constexpr int MKT = 64;  // keys per tile
+constexpr int MKT = 64;  // keys per tile (decode of wide rows: 32)
+constexpr int kRowsAhead = 1024;   // keys whose cache rows are looked up at a time
 constexpr float kLog2e = 1.4426950408889634f;
 
 // NS: k-steps of the scores (DK / 32) at most; NCT: 16-column tiles of the output (rank / 16) at most.  All of them are
@@ -34,9 +35,18 @@ constexpr float kLog2e = 1.4426950408889634f;
 // NW: waves per workgroup, 4 or 8 (16 query rows each): with 8 a staged key tile serves 128 rows and every SIMD holds two
 // waves, so one wave's softmax and staging run beside the other's MFMAs.
 // TT: weights as two bfloat16 terms.
+// KT, NB: keys per tile and tiles in LDS; CS: waves that share the output columns.  A decode launch (up to 32 rows per
+// sequence) has one workgroup per CU and is a chain of latencies: with an operand read behind every product, a row look-up
+// behind every 1 KiB piece and one tile on its way, a tile of 64 keys of 576 columns took 8 us.  There (NB > 2) the operands
+// of a tile are read together, the row numbers too, two (rows over 320 columns: three, of 32 keys) tiles are on their way,
+// and in rows over 320 columns 8 waves take 16 keys and half of the output columns each (the scores twice; half of the
+// accumulators, so two waves fit a SIMD).  With its combine, 64 sequences of 1230 - 2870 keys, mean 2048: 576 columns, 32
+// heads 67.7 -> 59.5 us, 16 heads 60.6 -> 46.9, 320 columns, 16 heads 37.7 -> 32.7, 32 heads 41.4 -> 36.4; one sequence of
+// 700, 576 columns, 16 heads 26.1 -> 21.3.  All of equal length 51.8 (2.9 TB/s; the longest sequence's splits are the rest).
+// Four waves with three tiles ahead, operands read one by one: 68.  Rows up to 192 columns: several workgroups per CU, as before.
 // KS: waves that share 16 query rows.  With few rows (decode) a tile's keys are dealt to 2 or 4 waves, each with a softmax
 // of its own over its keys (16 keys per wave: 16x16x16 products in the sum), and merged through LDS at the end.
-template <int NS, int NCT, int NW, int KS, bool TT>
+template <int NS, int NCT, int NW, int KS, int CS, int KT, int NB, bool TT>
 __global__ void __launch_bounds__(64 * NW) latent_attention_mfma_kernel(
         const uint16_t* __restrict__ qa, const uint16_t* __restrict__ cache, const int32_t* __restrict__ block_table,
         int max_blocks, const int32_t* __restrict__ q_start, const int32_t* __restrict__ pos,
@@ -47,16 +57,20 @@ __global__ void __launch_bounds__(64 * NW) latent_attention_mfma_kernel(
     const int b = blockIdx.x;
     const int t0 = q_start[b], t1 = q_start[b + 1];
     const int rows_total = (t1 - t0) * H;
-    constexpr int KT = MKT, RPB = 16 * NW / KS;  // query rows per workgroup
+    constexpr int RPB = 16 * NW / (KS * CS);  // query rows per workgroup
+    constexpr int NCW = NCT / CS;             // column tiles per wave
+    constexpr bool AHEAD = NB > 2;            // decode: operands read in front of the products, deeper staging
     const int rb0 = blockIdx.y * RPB;
     if (rb0 >= rows_total) return;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, g = lane >> 4, qi = lane & 15;
     const int nct = rank / 16;
     constexpr int CPR = NS * 4 + 1, krs = CPR * 16;   // key row in LDS: 16-byte chunks, bytes
-    __shared__ int krow[2][KT];  // cache row (page * page size + slot) of each key of a tile
+    constexpr int PT = (KT * CPR + 63) / 64, PW = (PT + NW - 1) / NW, TB = PT * 1024;   // 1 KiB pieces per tile and per wave; a tile's bytes
+    __shared__ int krow[kRowsAhead];  // cache row (page * page size + slot) of the keys of the next tiles
     // this lane's query row (for the B operand and for the softmax): row r of the sequence, token t0 + r / H
     const int kpart = wv % KS;   // which part of a tile's keys this wave takes
-    const int r = rb0 + wv / KS * 16 + qi;
+    const int c0 = CS > 1 ? wv / KS % CS * NCW : 0, wr = wv / (KS * CS) * 16;   // its first column tile, its first row
+    const int r = rb0 + wr + qi;
     const bool rok = r < rows_total;
     const int rc = rok ? r : rows_total - 1;
     const int64_t grow = (int64_t)t0 * H + rc;              // row of qa / out / gate
@@ -72,9 +86,9 @@ __global__ void __launch_bounds__(64 * NW) latent_attention_mfma_kernel(
         qf[s] = 32 * s + 8 * g < DK ? *reinterpret_cast<const bf16x8*>(qa + grow * DK + 32 * s + 8 * g)
                                     : __builtin_bit_cast(bf16x8, z);
     }
-    f32x4 O[NCT];
+    f32x4 O[NCW];
 #pragma unroll
-    for (int c = 0; c < NCT; ++c) O[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < NCW; ++c) O[c] = f32x4{0.f, 0.f, 0.f, 0.f};
     float mrow = -INFINITY, lrow = 0.f;
     const float scale2 = scale * kLog2e;   // scores, maxima and sums live in the base-2 domain
     const int32_t* bt = block_table + (int64_t)b * max_blocks;
@@ -83,33 +97,95 @@ __global__ void __launch_bounds__(64 * NW) latent_attention_mfma_kernel(
     // key tiles are dealt round-robin to the nsplit workgroups of this row block (blockIdx.z): the context length is
     // only known on the device, and a split that gets no tile contributes an empty partial
     const int kfirst = k_lo + blockIdx.z * KT, kstep = KT * nsplit;
-    auto row_of = [&](int k0) {
-        const int key = min(k0 + (int)threadIdx.x, pmax);  // past the end: a real row, masked below
-        return bs_shift >= 0 ? ((bt[key >> bs_shift] << bs_shift) + (key & (BS - 1))) : (bt[key / BS] * BS + key % BS);
+    const int n = __builtin_amdgcn_readfirstlane(kfirst <= pmax ? (pmax - kfirst) / kstep + 1 : 0);   // tiles of this workgroup
+    constexpr int RA = kRowsAhead / KT;
+    auto look_up = [&](int t0) {   // cache rows of tiles t0 .. t0 + RA - 1
+        for (int i = threadIdx.x; i < min(RA, n - t0) * KT; i += 64 * NW) {
+            const int key = min(kfirst + (t0 + i / KT) * kstep + i % KT, pmax);  // past the end: a real row, masked below
+            krow[i] = bs_shift >= 0 ? ((bt[key >> bs_shift] << bs_shift) + (key & (BS - 1))) : (bt[key / BS] * BS + key % BS);
+        }
     };
-    auto stage = [&](int buf) {
+    const int wu = __builtin_amdgcn_readfirstlane(wv);
+    int prow_of[AHEAD ? PW : 1], pcol[AHEAD ? PW : 1];   // row of the tile and column of this lane's chunk of each piece
+    if constexpr (AHEAD) {
 #pragma unroll
-        for (int j = wv; j < CPR; j += NW) dma_rows<CPR>(cache, krow[buf], DK, chunks, j, lds0 + buf * KT * krs, lane);
+        for (int j = 0; j < PW; ++j) {
+            const int i = min(wu + j * NW, PT - 1) * 64 + lane, at = i / CPR;
+            prow_of[j] = min(at, KT - 1);
+            pcol[j] = min(i - at * CPR, chunks - 1) * 8;
+        }
+    }
+    auto stage = [&](int t) {
+        if constexpr (AHEAD) {   // counted waits: every wave as many pieces (the last ones of some twice)
+            int kr[PW];
+#pragma unroll
+            for (int j = 0; j < PW; ++j) kr[j] = krow[t % RA * KT + prow_of[j]];
+#pragma unroll
+            for (int j = 0; j < PW; ++j)
+                dma_1k(cache + ((int64_t)kr[j] * DK + pcol[j]), lds0 + t % NB * TB + min(wu + j * NW, PT - 1) * 1024);
+        } else {
+#pragma unroll
+            for (int j = wv; j < PT; j += NW)
+                dma_rows<CPR, KT>(cache, krow + t % RA * KT, DK, chunks, j, lds0 + t % NB * TB, lane);
+        }
     };
-    if (threadIdx.x < KT) krow[0][threadIdx.x] = row_of(kfirst);
+    look_up(0);
     __syncthreads();
-    if (kfirst <= pmax) stage(0);
-    if (threadIdx.x < KT) krow[1][threadIdx.x] = row_of(kfirst + kstep);
-    const bool wave_on = rb0 + wv / KS * 16 < rows_total;   // (a wave without rows only helps to stage)
-    int buf = 0;
-    for (int k0 = kfirst; k0 <= pmax; k0 += kstep, buf ^= 1) {
-        dma_wait();        // this wave's pieces of the tile have landed
-        __syncthreads();   // ... everyone's; the other buffer's tile has been read by all; its next rows are known
-        if (k0 + kstep <= pmax) stage(buf ^ 1);
-        const int nrow = threadIdx.x < KT ? row_of(k0 + 2 * kstep) : 0;
-        const unsigned char* kimg = smem + buf * KT * krs;
+#pragma unroll
+    for (int t = 0; t + 1 < NB; ++t)
+        if (t < n) stage(t);
+    const bool wave_on = rb0 + wr < rows_total;   // (a wave without rows only helps to stage)
+    for (int t = 0; t < n; ++t) {
+        const int k0 = kfirst + t * kstep;
+        // this wave's pieces of the tile have landed; behind the barrier: everyone's, and the tile before it has been read by all
+        dma_wait_for<PW, NB - 2>(n - 1 - t);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (t + NB - 1 < n) {
+            if ((t + NB - 1) % RA == 0) {   // (every kRowsAhead keys)
+                look_up(t + NB - 1);
+                __syncthreads();
+            }
+            stage(t + NB - 1);
+        }
+        const unsigned char* kimg = smem + t % NB * TB;
         if (wave_on) {
         // ---- scores: KT / 16 key tiles of 16; lane gets keys 16 kt + 4 g + i of query row qi
         constexpr int NKT = KT / 16 / KS;
         const int key0 = kpart * (KT / KS);
         f32x4 S[NKT];
+        const unsigned char* vt = kimg + (key0 + 4 * g + (qi >> 2)) * krs + (qi & 3) * 8 + c0 * 32;
+        bf16x4 vr[AHEAD ? NKT : 1][AHEAD ? NCW : 1];
+        if constexpr (AHEAD) {
+            // The compiler would read each operand into the registers of the one before it, behind its product: all of the
+            // scores' are read first, then, behind their products and under the softmax, all of the sum's.
+            bf16x8 kf[NKT][NS];
+            f32x4 odd[NKT];
 #pragma unroll
-        for (int kt = 0; kt < NKT; ++kt) {
+            for (int kt = 0; kt < NKT; ++kt) {
+#pragma unroll
+                for (int s = 0; s < NS; ++s)
+                    kf[kt][s] = *reinterpret_cast<const bf16x8*>(kimg + (key0 + 16 * kt + qi) * krs + g * 16 + s * 64);
+                S[kt] = odd[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+#pragma unroll
+                for (int kt = 0; kt < NKT; ++kt)
+                    (s & 1 ? odd[kt] : S[kt]) = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[kt][s], qf[s], s & 1 ? odd[kt] : S[kt], 0, 0, 0);
+#pragma unroll
+            for (int kt = 0; kt < NKT; ++kt) S[kt] += odd[kt];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int kt = 0; kt < NKT; ++kt)
+#pragma unroll
+                for (int c = 0; c < NCW; ++c) vr[kt][c] = lds_read_tr4(vt + 16 * kt * krs + c * 32);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int kt = 0; kt < NKT && !AHEAD; ++kt) {
             S[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
             const unsigned char* arow = kimg + (key0 + 16 * kt + qi) * krs + g * 16;
 #pragma unroll
@@ -150,9 +226,8 @@ __global__ void __launch_bounds__(64 * NW) latent_attention_mfma_kernel(
         constexpr int NU = NKT / 2;
         if (__builtin_amdgcn_ballot_w64(corr != 1.f) != 0) {   // (rarely, once the maxima have settled)
 #pragma unroll
-            for (int c = 0; c < NCT; ++c) O[c] *= corr;
+            for (int c = 0; c < NCW; ++c) O[c] *= corr;
         }
-        const unsigned char* vt = kimg + (key0 + 4 * g + (qi >> 2)) * krs + (qi & 3) * 8;
         if constexpr (NKT == 1) {
             bf16x4 pf, pl;
 #pragma unroll
@@ -161,8 +236,8 @@ __global__ void __launch_bounds__(64 * NW) latent_attention_mfma_kernel(
                 if constexpr (TT) pl[e] = (__bf16)(S[0][e] - (float)pf[e]);
             }
 #pragma unroll
-            for (int c = 0; c < NCT; ++c) {
-                const bf16x4 vf = lds_read_tr4(vt + c * 32);
+            for (int c = 0; c < NCW; ++c) {
+                const bf16x4 vf = AHEAD ? vr[0][AHEAD ? c : 0] : lds_read_tr4(vt + c * 32);
                 O[c] = mfma_16x16x16(vf, pf, O[c]);
                 if constexpr (TT) O[c] = mfma_16x16x16(vf, pl, O[c]);
             }
@@ -177,25 +252,24 @@ __global__ void __launch_bounds__(64 * NW) latent_attention_mfma_kernel(
                 if constexpr (TT) pl[e] = (__bf16)(w - (float)pf[e]);
             }
 #pragma unroll
-            for (int c = 0; c < NCT; ++c) {
-                const bf16x4 lo = lds_read_tr4(vt + 32 * u * krs + c * 32);
-                const bf16x4 hi = lds_read_tr4(vt + (32 * u + 16) * krs + c * 32);
+            for (int c = 0; c < NCW; ++c) {
+                const bf16x4 lo = AHEAD ? vr[AHEAD ? 2 * u : 0][AHEAD ? c : 0] : lds_read_tr4(vt + 32 * u * krs + c * 32);
+                const bf16x4 hi = AHEAD ? vr[AHEAD ? 2 * u + 1 : 0][AHEAD ? c : 0] : lds_read_tr4(vt + (32 * u + 16) * krs + c * 32);
                 const bf16x8 vf = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
                 O[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, O[c], 0, 0, 0);
                 if constexpr (TT) O[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl, O[c], 0, 0, 0);
             }
         }
         }
-        if (threadIdx.x < KT) krow[buf][threadIdx.x] = nrow;
     }
     if constexpr (KS > 1) {   // the waves that share these rows merge their partial results; the first one goes on
-        constexpr int MS = NCT * 16 + 4;    // floats per row (padded)
+        constexpr int MS = NCW * 16 + 4;    // floats per row (padded)
         float* mb = reinterpret_cast<float*>(smem);
-        static_assert(NW * 16 * MS * 4 <= 2 * KT * krs, "the partial rows fit the key tiles' LDS");
+        static_assert(NW * 16 * MS * 4 <= NB * TB, "the partial rows fit the key tiles' LDS");
         __shared__ float ml[NW][16][2];
         __syncthreads();                    // everyone is done with the key tiles
 #pragma unroll
-        for (int c = 0; c < NCT; ++c) *reinterpret_cast<f32x4*>(mb + (wv * 16 + qi) * MS + 16 * c + 4 * g) = O[c];
+        for (int c = 0; c < NCW; ++c) *reinterpret_cast<f32x4*>(mb + (wv * 16 + qi) * MS + 16 * c + 4 * g) = O[c];
         if (g == 0) {
             ml[wv][qi][0] = mrow;
             ml[wv][qi][1] = lrow;
@@ -215,7 +289,7 @@ __global__ void __launch_bounds__(64 * NW) latent_attention_mfma_kernel(
         }
         mrow = mn;
 #pragma unroll
-        for (int c = 0; c < NCT; ++c) {
+        for (int c = 0; c < NCW; ++c) {
             O[c] *= e[0];
 #pragma unroll
             for (int k = 1; k < KS; ++k)
@@ -225,13 +299,13 @@ __global__ void __launch_bounds__(64 * NW) latent_attention_mfma_kernel(
     if (!rok) return;
     if (nsplit > 1) {  // unnormalised partial: the combine kernel merges the splits
         const int64_t pr = grow * nsplit + blockIdx.z;
-        if (g == 0) {
+        if (g == 0 && c0 == 0) {
             part_ml[pr * 2] = mrow;
             part_ml[pr * 2 + 1] = lrow;
         }
 #pragma unroll
-        for (int c = 0; c < NCT; ++c)
-            if (c < nct) *reinterpret_cast<f32x4*>(part_o + pr * rank + 16 * c + 4 * g) = O[c];
+        for (int c = 0; c < NCW; ++c)
+            if (c0 + c < nct) *reinterpret_cast<f32x4*>(part_o + pr * rank + 16 * (c0 + c) + 4 * g) = O[c];
         return;
     }
     float f = 1.f / lrow;
@@ -242,10 +316,10 @@ __global__ void __launch_bounds__(64 * NW) latent_attention_mfma_kernel(
     if (gate != nullptr) f *= sigmoidf_(gate[grow]);
     // lane holds O^T[col = 16 c + 4 g + i][query row qi]
 #pragma unroll
-    for (int c = 0; c < NCT; ++c)
-        if (c < nct) {
+    for (int c = 0; c < NCW; ++c)
+        if (c0 + c < nct) {
             const u16x4 o = u16x4{f2bf(O[c][0] * f), f2bf(O[c][1] * f), f2bf(O[c][2] * f), f2bf(O[c][3] * f)};
-            *reinterpret_cast<u16x4*>(out + grow * rank + 16 * c + 4 * g) = o;
+            *reinterpret_cast<u16x4*>(out + grow * rank + 16 * (c0 + c) + 4 * g) = o;
         }
 }
 
@@ -280,19 +354,21 @@ __global__ void __launch_bounds__(256) latent_combine_kernel(const float* __rest
 
 }  // namespace hy
 
-template <int NS, int NCT, int NW, int KS, bool TT>
+template <int NS, int NCT, int NW, int KS, int CS, int KT, int NB, bool TT>
 static void la_mfma_launch(const uint16_t* qa, const uint16_t* cache, const int32_t* bt, int max_blocks,
                            const int32_t* q_start, const int32_t* pos, const float* gate, uint16_t* out, int B, int H,
                            int DK, int rank, int BS, int max_q, float scale, int window, int nsplit, float* part_o,
                            float* part_ml, const float* sink, hipStream_t s) {
-    auto kern = hy::latent_attention_mfma_kernel<NS, NCT, NW, KS, TT>;
-    constexpr int bytes = 2 * hy::MKT * (NS * 64 + 16);
+    auto kern = hy::latent_attention_mfma_kernel<NS, NCT, NW, KS, CS, KT, NB, TT>;
+    constexpr int bytes = NB * ((KT * (NS * 4 + 1) + 63) / 64) * 1024;
+    static_assert(bytes <= 152 * 1024, "LDS");
     static int set_bytes = 0;
     if (bytes > set_bytes) {
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
         set_bytes = bytes;
     }
-    const dim3 grid(B, (max_q * H + 16 * NW / KS - 1) / (16 * NW / KS), nsplit);
+    constexpr int rpb = 16 * NW / (KS * CS);
+    const dim3 grid(B, (max_q * H + rpb - 1) / rpb, nsplit);
     const int bs_shift = (BS & (BS - 1)) == 0 ? __builtin_ctz(BS) : -1;
     kern<<<grid, 64 * NW, bytes, s>>>(qa, cache, bt, max_blocks, q_start, pos, gate, out, H, DK, rank, BS, scale, window,
                                   nsplit, part_o, part_ml, bs_shift, sink);
@@ -320,15 +396,16 @@ bool launch_hy_latent_attention_mfma(const uint16_t* qa, const uint16_t* cache, 
                                      hipStream_t s) {
     if (!hy_latent_mfma_ok(DK, rank)) return false;
     if (B == 0 || max_q == 0) return true;
-#define HY_LAM(NS, NCT, NW, KS, TT) la_mfma_launch<NS, NCT, NW, KS, TT>(qa, cache, bt, max_blocks, q_start, pos, gate, out, B, H, DK, rank, BS, max_q, scale, window, nsplit, part_o, part_ml, sink, s)
-    // 8 waves per workgroup when a sequence brings more than 64 rows; up to 32 or 16 rows 2 or 4 waves share them
+#define HY_LAM(NS, NCT, NW, KS, CS, KT, NB, TT) la_mfma_launch<NS, NCT, NW, KS, CS, KT, NB, TT>(qa, cache, bt, max_blocks, q_start, pos, gate, out, B, H, DK, rank, BS, max_q, scale, window, nsplit, part_o, part_ml, sink, s)
+    // 8 waves per workgroup when a sequence brings more than 64 rows; up to 32 or 16 rows 2 or 4 waves share them (each
+    // instance's figures stand at the kernel)
     const int rows = max_q * H;
 #define HY_LAM_R(NS, NCT, TT)                             \
     do {                                                  \
-        if (rows > 64) HY_LAM(NS, NCT, 8, 1, TT);         \
-        else if (rows > 32) HY_LAM(NS, NCT, 4, 1, TT);    \
-        else if (rows > 16) HY_LAM(NS, NCT, 4, 2, TT);    \
-        else HY_LAM(NS, NCT, 4, 4, TT);                   \
+        if (rows > 64) HY_LAM(NS, NCT, 8, 1, 1, 64, 2, TT);      \
+        else if (rows > 32) HY_LAM(NS, NCT, 4, 1, 1, 64, 2, TT); \
+        else if (NS > 10 || rows > 16) HY_LAM(NS, NCT, (NS > 10 ? 8 : 4), 2, (NS > 10 ? 2 : 1), (NS > 10 ? 32 : 64), (NS > 10 ? 4 : NS > 6 ? 3 : 2), TT); \
+        else HY_LAM(NS, NCT, (NS > 10 ? 8 : 4), (NS > 10 ? 2 : 4), (NS > 10 ? 2 : 1), (NS > 10 ? 32 : 64), (NS > 10 ? 4 : NS > 6 ? 3 : 2), TT); \
     } while (0)
 #define HY_LAM_T(NS, NCT)                                                                       \
     do {                                                                                        \
