@@ -354,7 +354,7 @@ __global__ void __launch_bounds__(256, 1) moe_gemm256_kernel(const uint16_t* __r
                     *reinterpret_cast<u16x8*>(y + (int64_t)(m0 + 16 * t + RPS * k + rr) * ld + n) = v[k];
         }
     };
-    slab_run<false>(smem, meta[0] * nt, K / 64, x, (int)xbytes, (int)((uint32_t)N * K * 2), off, [](auto, int, int) {}, epi);
+    slab_run<false>(smem, meta[0] * nt, 0, K / 64, x, (int)xbytes, (int)((uint32_t)N * K * 2), off, [](auto, int, int) {}, epi);
 }
 
 // An index of E and above is an identity expert (its output is the token itself) where the experts' layer has such

@@ -154,15 +154,22 @@ constexpr int kSlabLds = kSlabRows + 4 * 4096;   // two buffers and the epilogue
 
 // T tiles of 256 x 256 on 256 CUs: whole rounds of them and, where at most half of the CUs would have a tile in the last round, that
 // round's tiles as two halves of 128 x rows each, so that all CUs share it (a half takes 0.59 of a tile's time: it reads the W rows for
-// half as many products).
-__host__ __device__ inline void slab_split(int T, int& full, int& half) {
+// half as many products).  tail: that many further tiles, numbered from T on, are one half each (slab_tail).
+__host__ __device__ inline void slab_split(int T, int tail, int& full, int& half) {
     const int r = T % kSlabCUs;
-    half = r <= kSlabCUs / 2 ? 2 * r : 0;
+    half = tail > 0 || r <= kSlabCUs / 2 ? 2 * r + tail : 0;
     full = half ? T - r : T;
 }
-__host__ __device__ inline int slab_grid(int T) {
+// A launch of nt tiles along the W rows whose last x tile has at most 128 rows: nt if all that whole rounds of the full tiles leave fits one
+// round of halves when these last tiles count as one each, else 0 (they are tiles like the others).  585 x 11264 x 2048, 220 halves
+// instead of 132 tiles: 41.7 -> 31.4 us; 1100 x 7168 x 2048 39.9 -> 30.0; 350 x 20480 x 2048 (240 halves) 36.9.
+__host__ __device__ inline int slab_tail(int M, int nt) {
+    const int r = M % 256;
+    return r > 0 && r <= 128 && 2 * (int)((int64_t)(M / 256) * nt % kSlabCUs) + nt <= kSlabCUs ? nt : 0;
+}
+__host__ __device__ inline int slab_grid(int T, int tail) {
     int full, half;
-    slab_split(T, full, half);
+    slab_split(T, tail, full, half);
     return full >= kSlabCUs ? kSlabCUs : full > half ? full : half;
 }
 
@@ -172,12 +179,12 @@ template <bool PAIR> struct SlabRow {   // byte offset of the wave's W block b; 
 
 // The tiles of one workgroup, one after the other without a pause of the slab pipeline: the pieces that a tile's last two slabs issue are
 // those of the next tile's first two, which land while this tile's results are stored.  Tile v of the launch goes to workgroup
-// v % gridDim.x (gridDim.x = slab_grid(T)); xcd_remap gives neighbouring tiles to the same XCD.
+// v % gridDim.x (gridDim.x = slab_grid(T, tail)); xcd_remap gives neighbouring tiles to the same XCD.
 //   off(NM, tile, m, wv, xv, wb): byte offsets of the lane's rows of slab 0 (x rows from row m of the tile on) and the W matrix
 //   rows(NM, tile, m): called before a tile's first slab, for what its epilogue needs of its rows
 //   epi(NM, tile, m, acc): store the results (rows: the wave's 4 KiB of LDS)
 template <bool PAIR, class Off, class Rows, class Epi>
-__device__ __forceinline__ void slab_run(unsigned char* smem, int T, int NS, const void* x, int xbytes, int wbytes, const Off& off,
+__device__ __forceinline__ void slab_run(unsigned char* smem, int T, int tail, int NS, const void* x, int xbytes, int wbytes, const Off& off,
                                          const Rows& rows, const Epi& epi) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wn = wave >> 1, wm = wave & 1, ln = lane & 15, g = lane >> 4, G = gridDim.x;
@@ -186,7 +193,7 @@ __device__ __forceinline__ void slab_run(unsigned char* smem, int T, int NS, con
     const uint32_t lds = (uint32_t)(uintptr_t)(lg_lds_cptr)smem;
     using Row = SlabRow<PAIR>;
     int full, half;
-    slab_split(T, full, half);
+    slab_split(T, tail, full, half);
     uint32_t wv[8];
     const void* wb;
     auto walk = [&](auto NMC, int first, int count, auto tile_of, auto m_of) {
@@ -276,9 +283,17 @@ __device__ __forceinline__ void slab_run(unsigned char* smem, int T, int NS, con
     const int b = blockIdx.x;
     if (b < full)
         walk(std::integral_constant<int, 8>{}, b, full, [&](int v) { return xcd_remap(v, full); }, [](int) { return 0; });
+    const int pairs = half - tail;   // halves that are two of a tile
     if (b < half)
-        walk(std::integral_constant<int, 4>{}, b, half, [&](int v) { return full + xcd_remap(v, half) / 2; },
-             [&](int v) { return (xcd_remap(v, half) & 1) * 128; });
+        walk(std::integral_constant<int, 4>{}, b, half,
+             [&](int v) {
+                 const int h = xcd_remap(v, half);
+                 return h < pairs ? full + h / 2 : T + h - pairs;
+             },
+             [&](int v) {
+                 const int h = xcd_remap(v, half);
+                 return h < pairs ? (h & 1) * 128 : 0;
+             });
 }
 
 }  // namespace chronos

@@ -33,10 +33,13 @@ __global__ void __launch_bounds__(256, 1) gemm_slab_kernel(PPArgs a) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];                            // pieces per row; rows per store
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wn = wave >> 1, wm = wave & 1, in = lane >> 3, piece = ((lane & 7) ^ in) * 8;
-    const int mt = (a.M + 255) / 256, nt = PAIR ? a.F / 128 : (a.N + 255) / 256;
+    const int nt = PAIR ? a.F / 128 : (a.N + 255) / 256, tail = slab_tail(a.M, nt), mt = tail > 0 ? a.M / 256 : (a.M + 255) / 256;
     // tiles in groups of gm along x, so that what an XCD runs at a time shares rows of both operands in its L2
     auto where = [&](int tile, int& tm, int& tn) {
-        if (a.gm > 0 && mt > a.gm) {
+        if (tail > 0 && tile >= mt * nt) {
+            tm = mt;
+            tn = tile - mt * nt;
+        } else if (a.gm > 0 && mt > a.gm) {
             const int per = a.gm * nt, grp = tile / per, r = tile - grp * per, gsz = min(a.gm, mt - grp * a.gm);
             tm = grp * a.gm + r % gsz;
             tn = r / gsz;
@@ -170,7 +173,7 @@ __global__ void __launch_bounds__(256, 1) gemm_slab_kernel(PPArgs a) {
             }
         }
     };
-    slab_run<PAIR>(smem, mt * nt, a.K / 64, a.x, (int)((int64_t)a.M * a.K * 2), (int)((int64_t)a.N * a.K * 2), off, scales, epi);
+    slab_run<PAIR>(smem, mt * nt, tail, a.K / 64, a.x, (int)((int64_t)a.M * a.K * 2), (int)((int64_t)a.N * a.K * 2), off, scales, epi);
 }
 
 template <int MODE, bool NORMP>
@@ -180,8 +183,9 @@ void slab_launch(const PPArgs& a, hipStream_t st) {
     static const hipError_t once = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     (void)once;
     const bool pair = MODE == kPPSwiglu || MODE == kPPGlu;
-    const int tiles = (a.M + 255) / 256 * (pair ? a.F / 128 : (a.N + 255) / 256);
-    hipLaunchKernelGGL(kern, dim3(slab_grid(tiles)), dim3(256), lds, st, a);
+    const int nt = pair ? a.F / 128 : (a.N + 255) / 256, tail = slab_tail(a.M, nt);
+    const int tiles = (tail > 0 ? a.M / 256 : (a.M + 255) / 256) * nt;
+    hipLaunchKernelGGL(kern, dim3(slab_grid(tiles, tail)), dim3(256), lds, st, a);
 }
 
 }  // namespace

@@ -276,8 +276,11 @@ MANY_MIN = 128
 
 
 def _many_slab(c, per_round: float, m: int, n: int, k: int) -> float:
-    t = -(-m // 256) * -(-n // 256)
+    nt = -(-n // 256)
+    t = -(-m // 256) * nt
     half = 0 < t % 256 <= 128
+    if 0 < m % 256 <= 128 and 2 * (m // 256 * nt % 256) + nt <= 256:   # (chronos_slab.h slab_tail)
+        t, half = m // 256 * nt, True
     rounds = t // 256 if half else -(-t // 256)
     return c[0] + per_round * rounds + (c[1] + c[3] * (k // 64)) * half + c[2] * rounds * (k // 64) + (c[4] * m + c[5] * k) * n * 1e-6
 

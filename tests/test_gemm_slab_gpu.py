@@ -32,6 +32,25 @@ def test_every_tile_once(tiles, k):
     _close(y, x.float() @ w.float().t())
 
 
+@pytest.mark.parametrize("m,n", [(585, 11264), (641, 11264), (128, 65536), (100, 65540), (300, 21760), (300, 22016), (256 * 256 + 5, 256),
+                                 (256 * 300 + 77, 512), (256 * 300 + 129, 512), (1025, 8192), (2400, 7168)])
+@pytest.mark.parametrize("k", [64, 128, 320])
+def test_last_rows_as_halves(m, n, k):
+    """x tiles of at most 128 rows at the end are one half each where one round of halves holds them and what whole rounds leave, at
+    and past that line."""
+    from chronos import ops
+    from chronos.ops import gemm as G
+
+    ops.load()
+    x, w = _operands(m, n, k, m + n + k)
+    ref = x.float() @ w.float().t()
+    y, _ = G.pp_gemm(x, w, G.PP_PLAIN, (88, 1))
+    _close(y, ref)
+    g, u = ref[:, : n // 2], ref[:, n // 2:]
+    if n % 256 == 0:
+        _close(torch.ops.chronos.gemm_act(x, w, 3, float("inf"), 1.0, 1.0), g * torch.sigmoid(g) * (u + 1))
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 256, 64), (300, 512, 128), (2446, 5632, 192), (4100, 20224, 64)])
 @pytest.mark.parametrize("limit,slope,shift", [(float("inf"), 1.0, 0.0), (0.75, 1.702, 1.0)])
 def test_gated_unit(m, n, k, limit, slope, shift):
