@@ -28,7 +28,7 @@ struct PPArgs {
 };
 
 // epilogue modes
-enum : int { kPPPlain = 0, kPPSwiglu = 1, kPPResid = 2, kPPGlu = 3, kPPRelu2 = 4, kPPGelu = 5 };  // (3 on: gemm_slab, gemm_skinny)
+enum : int { kPPPlain = 0, kPPSwiglu = 1, kPPResid = 2, kPPGlu = 3, kPPRelu2 = 4, kPPGelu = 5, kPPPart = 6 };  // (3 on: gemm_slab, gemm_skinny; 6 its own)
 constexpr int kPPConfigs = 12;
 int gemm_pp_bm(int cfg);  // x rows per tile
 int gemm_pp_bn(int cfg);  // W rows per tile
@@ -45,9 +45,10 @@ constexpr int kLGTinyFirst = 72, kLGTinyConfigs = 23;
 int gemm_lg_xm(int cfg);  // x rows per tile
 int gemm_lg_wn(int cfg);  // W rows per tile
 bool gemm_lg_splitk_ok(int cfg);  // false for the HB configs (VAR 4): no split-K path
+bool gemm_lg_sliced(int cfg, int mode);  // its split-K writes float32 slices [splitk, M, N] and needs no tickets (gemm_slab.hip)
 bool gemm_lg_ablations_built();  // the timing-only ablation ids 40-71 exist (CHRONOS_GEMM_ABLATIONS build)
 bool launch_gemm_lg(int cfg, int mode, bool normp, const PPArgs& a, hipStream_t st);
-// configs 88 / 92 without split-K, and the hybrid decoders' epilogues (csrc/kernels/gemm_slab.hip)
+// configs 88 / 92 without split-K or (plain, resid) with it, and the hybrid decoders' epilogues (csrc/kernels/gemm_slab.hip)
 bool launch_gemm_slab(int mode, bool normp, const PPArgs& a, hipStream_t st);
 // W8A8 fp8 configs of the same kernel (ring schedule, 128-deep stages; a.kts counts 128-deep units), own id space
 constexpr int kLGF8Configs = 5;

@@ -163,9 +163,11 @@ __host__ __device__ inline void slab_split(int T, int tail, int& full, int& half
 // A launch of nt tiles along the W rows whose last x tile has at most 128 rows: nt if all that whole rounds of the full tiles leave fits one
 // round of halves when these last tiles count as one each, else 0 (they are tiles like the others).  585 x 11264 x 2048, 220 halves
 // instead of 132 tiles: 41.7 -> 31.4 us; 1100 x 7168 x 2048 39.9 -> 30.0; 350 x 20480 x 2048 (240 halves) 36.9.
-__host__ __device__ inline int slab_tail(int M, int nt) {
+// (S: times that the tiles are walked, over slices of K)
+__host__ __device__ inline int slab_tail(int M, int nt, int S) {
     const int r = M % 256;
-    return r > 0 && r <= 128 && 2 * (int)((int64_t)(M / 256) * nt % kSlabCUs) + nt <= kSlabCUs ? nt : 0;
+    return r > 0 && r <= 128 && (int64_t)nt * S <= kSlabCUs &&
+                   2 * (int)((int64_t)(M / 256) * nt * S % kSlabCUs) + nt * S <= kSlabCUs ? nt * S : 0;
 }
 __host__ __device__ inline int slab_grid(int T, int tail) {
     int full, half;

@@ -601,7 +601,7 @@ std::tuple<Tensor, Tensor> gemm_pp(const Tensor& x, const Tensor& w, int64_t mod
     if (splitk > 1) {
         ws = at::empty({tiles * splitk * BM * BN}, x.options().dtype(at::kFloat));
         a.ws = ws.data_ptr<float>();
-        a.cnt = split_tickets(x, tiles);
+        if (!chronos::gemm_lg_sliced((int)cfg, (int)mode)) a.cnt = split_tickets(x, tiles);
     }
     if (lg) {
         CHK(!prio && chronos::launch_gemm_lg((int)cfg, (int)mode, part_in.has_value(), a, cur_stream()), "gemm_lg: launch");

@@ -1,12 +1,17 @@
 // gemm_slab.hip — projections of many rows: y[M, N] = x[M, K] W[N, K]^T in bfloat16 with float32 sums, 256 x 256 tiles on the
 // slab loop of chronos_slab.h.  A workgroup per CU walks its tiles; the slab pipeline runs on from one tile into the next, and where the
-// last round would leave half of the CUs idle its tiles are halved.  Configs 88 and 92 of the projection family (gemm_lg.hip has their split-K form).
+// last round would leave half of the CUs idle its tiles are halved.  Configs 88 and 92 of the projection family (gemm_lg.hip has SwiGLU's split-K).
 //
 // Epilogues, through 4 KiB of LDS per wave so that every store is 16 bytes of a whole line: plain; activation (squared ReLU, GELU); gated
 // units over W = [gate; up], of Llama (SwiGLU, roundings of the unfused form kept) and of the hybrid decoders (clamped, any slope and shift);
 // the new residual stream with its RMSNorm partials.  NORMP: the folded input RMSNorm as a scale per row.
 //
 // Bound by the matrix cores (a slab is 2048 of their cycles and takes 2200) and by the last round of tiles.
+// Split-K (plain, resid): the tiles are walked once per slice of K and leave float32 slices [S, M, N], whose stores run beside the next
+// tile's first slabs where there is one; a second launch sums them in slice order, with the residual and its partials.  For products whose
+// tiles are too few for the chip: the tiles of a launch have to fit one round.  us, the residual form's best tiles before -> this: 4096 x
+// 14336 at 128 rows 42 -> 36 (16 slices), 256 56 -> 45 (8), 512 76 -> 65 (4), 768 110 -> 86, 1024 119 -> 101 (88 and 13: the slices are 67 MB,
+// written and read), 1536 185 -> 147 (2), 2048 198 -> 182; 2560 249 -> 274, not taken.
 // One workgroup per tile -> this, us: 8192 x 3648 x 2048 95.8 -> 93.0; 8192 x 6144 x 2048 157 -> 146 (3 rounds); 8192 x 2560 x 1024 (1.25
 // rounds) 52 -> 43; 8192 x 4096 x 4096 190 -> 179; a Llama-3 8B prefill of 5952 tokens, four layers, whole 8604 -> 7986.
 #include "chronos_act.h"
@@ -33,13 +38,26 @@ __global__ void __launch_bounds__(256, 1) gemm_slab_kernel(PPArgs a) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];                            // pieces per row; rows per store
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wn = wave >> 1, wm = wave & 1, in = lane >> 3, piece = ((lane & 7) ^ in) * 8;
-    const int nt = PAIR ? a.F / 128 : (a.N + 255) / 256, tail = slab_tail(a.M, nt), mt = tail > 0 ? a.M / 256 : (a.M + 255) / 256;
+    const int nt = PAIR ? a.F / 128 : (a.N + 255) / 256, S = MODE == kPPPart ? a.splitk : 1;
+    const int tail = slab_tail(a.M, nt, S), mt = tail > 0 ? a.M / 256 : (a.M + 255) / 256;
     // tiles in groups of gm along x, so that what an XCD runs at a time shares rows of both operands in its L2
-    auto where = [&](int tile, int& tm, int& tn) {
-        if (tail > 0 && tile >= mt * nt) {
+    // (kPPPart: slice by slice; the short last rows of all slices behind)
+    auto where = [&](int tile, int& tm, int& tn, int& sl) {
+        sl = 0;
+        if (tail > 0 && tile >= mt * nt * S) {
             tm = mt;
-            tn = tile - mt * nt;
-        } else if (a.gm > 0 && mt > a.gm) {
+            tn = tile - mt * nt * S;
+            if constexpr (MODE == kPPPart) {
+                sl = tn / nt;
+                tn -= sl * nt;
+            }
+            return;
+        }
+        if constexpr (MODE == kPPPart) {
+            sl = tile / (mt * nt);
+            tile -= sl * mt * nt;
+        }
+        if (a.gm > 0 && mt > a.gm) {
             const int per = a.gm * nt, grp = tile / per, r = tile - grp * per, gsz = min(a.gm, mt - grp * a.gm);
             tm = grp * a.gm + r % gsz;
             tn = r / gsz;
@@ -50,17 +68,18 @@ __global__ void __launch_bounds__(256, 1) gemm_slab_kernel(PPArgs a) {
     };
     auto off = [&](auto NMC, int tile, int m, uint32_t (&wv)[8], auto& xv, const void*& wb) {
         constexpr int NM = decltype(NMC)::value;
-        int tm, tn;
-        where(tile, tm, tn);
+        int tm, tn, sl;
+        where(tile, tm, tn, sl);
+        const int at = MODE == kPPPart ? sl * a.kts * 64 + piece : piece;
         wb = a.w;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int r = 64 * wave + 8 * i + in;
             const int row = !PAIR ? tn * 256 + r : wave < 2 ? tn * 128 + r : a.F + tn * 128 + r - 128;
-            wv[i] = ((uint32_t)row * (uint32_t)a.K + piece) * 2;
+            wv[i] = ((uint32_t)row * (uint32_t)a.K + at) * 2;
         }
 #pragma unroll
-        for (int i = 0; i < NM; ++i) xv[i] = ((uint32_t)(tm * 256 + m + 8 * (NM * wave + i) + in) * (uint32_t)a.K + piece) * 2;
+        for (int i = 0; i < NM; ++i) xv[i] = ((uint32_t)(tm * 256 + m + 8 * (NM * wave + i) + in) * (uint32_t)a.K + at) * 2;
     };
     // NORMP: a lane sums its row's partials; two buffers in turn (a tile's slabs, with their barriers, lie between a buffer's
     // writers and its readers, and between those and the next writers)
@@ -68,8 +87,8 @@ __global__ void __launch_bounds__(256, 1) gemm_slab_kernel(PPArgs a) {
     auto scales = [&](auto NMC, int tile, int m) {
         if constexpr (NORMP) {
             constexpr int RPW = 8 * decltype(NMC)::value;   // rows per wave
-            int tm, tn;
-            where(tile, tm, tn);
+            int tm, tn, sl;
+            where(tile, tm, tn, sl);
             const int row = RPW * wave + (lane & (RPW - 1));
             const float* p = a.part_in + (int64_t)min(tm * 256 + m + row, a.M - 1) * a.nparts_in;
             f32x4 t = {0.f, 0.f, 0.f, 0.f};
@@ -94,8 +113,8 @@ __global__ void __launch_bounds__(256, 1) gemm_slab_kernel(PPArgs a) {
     const int c = lane % NCH, rr = lane / NCH;   // store phase: the lane's piece, its row within the RPS of an instruction
     auto epi = [&](auto NMC, int tile, int m, auto& acc) {
         constexpr int NM = decltype(NMC)::value;
-        int tm, tn;
-        where(tile, tm, tn);
+        int tm, tn, sl;
+        where(tile, tm, tn, sl);
         const int m0 = tm * 256 + m + 16 * NM * wm;                      // the wave's first row
         const int ld = PAIR ? a.F : a.N, n = (PAIR ? tn * 128 : tn * 256) + OC * wn + 8 * c;
         u16x8 rv[MODE == kPPResid ? NK : 1];
@@ -114,6 +133,16 @@ __global__ void __launch_bounds__(256, 1) gemm_slab_kernel(PPArgs a) {
             const int r = lane & 15;
             float sc = 1.f;
             if constexpr (NORMP) sc = inv[16 * NM * wm + 16 * t + r];
+            if constexpr (MODE == kPPPart) {   // (two blocks of columns make a line)
+                const int row = m0 + 16 * t + r;
+#pragma unroll
+                for (int s = 0; s < 8; ++s) {
+                    const int col = tn * 256 + OC * wn + 16 * s + 4 * (lane >> 4);
+                    if (row < a.M && col < a.N) *reinterpret_cast<f32x4*>(a.ws + ((int64_t)sl * a.M + row) * a.N + col) = acc[s][t] * sc;
+                    acc[s][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+                continue;
+            }
 #pragma unroll
             for (int s = 0; s < (PAIR ? 4 : 8); ++s) {
                 const int col = 16 * s + 4 * (lane >> 4);
@@ -173,7 +202,32 @@ __global__ void __launch_bounds__(256, 1) gemm_slab_kernel(PPArgs a) {
             }
         }
     };
-    slab_run<PAIR>(smem, mt * nt, tail, a.K / 64, a.x, (int)((int64_t)a.M * a.K * 2), (int)((int64_t)a.N * a.K * 2), off, scales, epi);
+    slab_run<PAIR>(smem, mt * nt * S, tail, MODE == kPPPart ? a.kts : a.K / 64, a.x, (int)((int64_t)a.M * a.K * 2), (int)((int64_t)a.N * a.K * 2), off, scales, epi);
+}
+
+// y = the new residual stream: the S slices of 8 columns per thread in their order, the residual, RMSNorm partials per 128 columns
+__global__ void __launch_bounds__(256) slab_sum_resid_kernel(const float* __restrict__ ws, const uint16_t* __restrict__ resid,
+                                                             uint16_t* __restrict__ y, float* __restrict__ part, int64_t n, int S) {
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;   // (n % 256 == 0: 16 lanes leave or stay together)
+    if (i >= n) return;
+    const u16x8 rv = *reinterpret_cast<const u16x8*>(resid + i);
+    f32x4 v0 = *reinterpret_cast<const f32x4*>(ws + i), v1 = *reinterpret_cast<const f32x4*>(ws + i + 4);
+#pragma unroll 4
+    for (int s = 1; s < S; ++s) {
+        v0 += *reinterpret_cast<const f32x4*>(ws + s * n + i);
+        v1 += *reinterpret_cast<const f32x4*>(ws + s * n + i + 4);
+    }
+    u16x8 o;
+    float ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const float t = bf2f(f2bf(bf2f(f2bf(k < 4 ? v0[k & 3] : v1[k & 3])) + bf2f(rv[k])));
+        o[k] = f2bf(t);
+        ss += t * t;
+    }
+    *reinterpret_cast<u16x8*>(y + i) = o;
+    ss = row_sum16(ss);
+    if ((threadIdx.x & 15) == 0) part[i / 128] = ss;
 }
 
 template <int MODE, bool NORMP>
@@ -183,15 +237,23 @@ void slab_launch(const PPArgs& a, hipStream_t st) {
     static const hipError_t once = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     (void)once;
     const bool pair = MODE == kPPSwiglu || MODE == kPPGlu;
-    const int nt = pair ? a.F / 128 : (a.N + 255) / 256, tail = slab_tail(a.M, nt);
-    const int tiles = (tail > 0 ? a.M / 256 : (a.M + 255) / 256) * nt;
+    const int nt = pair ? a.F / 128 : (a.N + 255) / 256, S = MODE == kPPPart ? a.splitk : 1;
+    const int tail = slab_tail(a.M, nt, S), tiles = (tail > 0 ? a.M / 256 : (a.M + 255) / 256) * nt * S;
     hipLaunchKernelGGL(kern, dim3(slab_grid(tiles, tail)), dim3(256), lds, st, a);
 }
 
 }  // namespace
 
 bool launch_gemm_slab(int mode, bool normp, const PPArgs& a, hipStream_t st) {
-    if (a.splitk != 1 || (normp && mode != kPPPlain && mode != kPPSwiglu)) return false;
+    if (normp && mode != kPPPlain && mode != kPPSwiglu) return false;
+    if (a.splitk > 1) {
+        if (mode != kPPPlain && mode != kPPResid) return false;
+        normp ? slab_launch<kPPPart, true>(a, st) : slab_launch<kPPPart, false>(a, st);
+        const int64_t n = (int64_t)a.M * a.N;
+        if (mode == kPPPlain) launch_gemm_slices(a.ws, a.y, n, a.splitk, st);
+        else slab_sum_resid_kernel<<<(unsigned)((n / 8 + 255) / 256), 256, 0, st>>>(a.ws, a.resid, a.y, a.part_out, n, a.splitk);
+        return true;
+    }
     switch (mode) {
         case kPPPlain: normp ? slab_launch<kPPPlain, true>(a, st) : slab_launch<kPPPlain, false>(a, st); return true;
         case kPPSwiglu: normp ? slab_launch<kPPSwiglu, true>(a, st) : slab_launch<kPPSwiglu, false>(a, st); return true;

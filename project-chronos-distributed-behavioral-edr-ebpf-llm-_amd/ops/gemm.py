@@ -273,6 +273,10 @@ _MANY_TILES = {19: (128, 2.9, 1.9, 1.2, 0.294, 0.15, 0.16), 32: (64, 2.7, 1.45, 
 # its inputs
 _MANY_ACT = {True: ((2.1, 4.7, 1.22, 0.57, 0.41, 0.16), 4.45, (2.9, 0.44)), False: ((3.3, 2.2, 1.22, 0.55, 0.51, 0.17), 0.0, (2.8, 0.39))}
 MANY_MIN = 128
+# 88 with K split over workgroups (float32 slices and a launch that sums them), one round of tiles or of halves: constant, per slab of halves, of
+# them as all CUs have one, of tiles, of them as all CUs have one, per M of all slices' results, per M of weights.  Fitted on 708 launches, M = 128 ..
+# 3072, N = 1024 .. 6144, K = 1024 .. 14336 (rms error 8 %; the split picked takes 1 % longer than the best on average).
+_MANY_SPLIT = (11.3, 0.51, 0.13, 0.80, 0.31, 1.09, 0.088)
 
 
 def _many_slab(c, per_round: float, m: int, n: int, k: int) -> float:
@@ -283,6 +287,19 @@ def _many_slab(c, per_round: float, m: int, n: int, k: int) -> float:
         t, half = m // 256 * nt, True
     rounds = t // 256 if half else -(-t // 256)
     return c[0] + per_round * rounds + (c[1] + c[3] * (k // 64)) * half + c[2] * rounds * (k // 64) + (c[4] * m + c[5] * k) * n * 1e-6
+
+
+def _many_split(m: int, n: int, k: int) -> tuple[float, int]:
+    nt, last, best = -(-n // 256), 0 < m % 256 <= 128, (float("inf"), 1)
+    c = _MANY_SPLIT
+    for s in range(2, 17):
+        tiles, whole, slabs = -(-m // 256) * nt * s, m // 256 * nt * s, k // 64 // s
+        if k // 64 % s or slabs < 2 or tiles > 256:
+            continue
+        half = 2 * whole + nt * s if last and 2 * whole + nt * s <= 256 else 2 * tiles if tiles <= 128 else 0
+        t = slabs * (c[1] + c[2] * half / 256 if half else c[3] + c[4] * tiles / 256)
+        best = min(best, (c[0] + t + (c[5] * s * m + c[6] * k) * n * 1e-6, s))
+    return best
 
 
 def _many_best(m: int, n: int, k: int) -> tuple[float, int]:
@@ -299,8 +316,10 @@ def _many_fits(m: int, n: int, k: int) -> bool:
 
 
 def many_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
-    """(config, 1) of the hand-written GEMM for at least 128 rows of a shape that no plan lists, or None (the library): from 64 tiles of 128 x rows
-    by 64 W rows on, and K / 16 of them (below, K would have to be split for enough workgroups).  There, on the grid of _MANY_88: 1.13 times as
+    """(config, split-K) of the hand-written GEMM for at least 128 rows of a shape that no plan lists, or None (the library): from 64 tiles of 128 x rows
+    by 64 W rows on, and K / 16 of them; (88, split-K) where at least 12 tiles of 256 x 256 are too few for the chip and the split's model is a
+    tenth below the others' (53 shapes of _MANY_SPLIT's grid, 1.23 times as fast as the library or the others, one 9 % slower; 768 x 4096 x 11008
+    83 -> 71 us, 1024 x 4096 x 11008 102 -> 83; fewer tiles: the library's own splits are faster).  There, on the grid of _MANY_88: 1.13 times as
     fast as the library on average (340 shapes; 38 slower by more than 3 %, the worst by 14 %: one round that 256 x 256 tiles fill to
     between one and two thirds), below the line 0.9 times.  A library call also costs the host 22 us, this 7.  Rows count in 128s, so that a server's
     steps of any size find their plan again."""
@@ -315,6 +334,10 @@ def many_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     out = None
     if _many_fits(m, n, k) and tiles >= max(64, k // 16) and (n, k, PP_PLAIN) not in _plan_file():
         out = (_many_best(m, n, k)[1], 1)
+    if _many_fits(m, n, k) and -(-m // 256) * -(-n // 256) >= 12 and (n, k, PP_PLAIN) not in _plan_file():
+        t, s = _many_split(m, n, k)
+        if t < 0.9 * _many_best(m, n, k)[0]:
+            out = (88, s)
     _plan_cache[key] = out
     return out
 

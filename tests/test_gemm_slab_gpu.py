@@ -73,3 +73,31 @@ def test_activation(m, n, k, mode):
     h = x.float() @ w.float().t()
     ref = h.relu() ** 2 if mode == 4 else torch.nn.functional.gelu(h)
     _close(torch.ops.chronos.gemm_act(x, w, mode, 0.0, 0.0, 0.0), ref)
+
+
+@pytest.mark.parametrize("m,n,k,s", [(1, 4, 128, 2), (129, 260, 192, 3), (585, 2048, 5632, 4), (384, 4096, 1024, 8), (300, 1032, 704, 11),
+                                     (1100, 1024, 1024, 16), (2047, 2048, 256, 4), (70, 4096, 14336, 16)])
+def test_slices_of_k(m, n, k, s):
+    """Tiles and halves over slices of K, plain, with the residual's epilogue, and the same bits again in a graph's replays."""
+    from chronos import ops
+    from chronos.ops import gemm as G
+
+    ops.load()
+    x, w = _operands(m, n, k, m + n + k)
+    ref = x.float() @ w.float().t()
+    y, _ = G.pp_gemm(x, w, G.PP_PLAIN, (88, s))
+    _close(y, ref)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y2, _ = G.pp_gemm(x, w, G.PP_PLAIN, (88, s))
+    for _ in range(3):
+        y2.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y2, y)
+    if n % 256 == 0:
+        res = torch.randn(m, n, device=DEV).to(torch.bfloat16)
+        z, part = G.pp_gemm(x, w, G.PP_RESID, (88, s), resid=res)
+        assert torch.equal(z, y + res)
+        want = z.double().square().view(m, n // 128, 128).sum(-1)
+        assert ((part.double() - want).abs() <= want * 128 * 2.0 ** -24).all()

@@ -16,8 +16,11 @@ def test_rule_returns_what_the_kernels_take():
         if plan is not None:
             assert plan[0] in (19, 32, 88) and G._pp_valid(plan[0], n, k, G.PP_PLAIN, 1, m)
             assert (max(m, n) + 256) * k * 2 < 1 << 31
+            assert k // 64 % plan[1] == 0 and (plan[1] == 1 or (plan[0] == 88 and G._pp_valid(88, n, k, G.PP_PLAIN, plan[1], m)
+                                                                and -(-m // 256) * -(-n // 256) * plan[1] <= 256))
     assert G.many_rows_plan(8192, 2048, 96) is None and G.many_rows_plan(8192, 2050, 128) is None
     assert G.many_rows_plan(128, 64, 4096) is None         # too few tiles without a split of K
+    assert G.many_rows_plan(1000, 4096, 11008)[1] > 1      # ... with one
     assert G.many_rows_plan(2446, 1536, 1024) == G.many_rows_plan(2550, 1536, 1024)   # rows count in 128s
     assert G.many_rows_plan(4096, 6144, 4096) is None      # the measured plan's own
 
