@@ -626,7 +626,7 @@ def linear(x, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tens
         for pred, fn in _custom:
             if pred(m, n, k):
                 return fn(x, w)
-        if few is not None and few[1] > 1 and few[0] < SK_BASE:   # a split without tickets
+        if few is not None and m <= 64 and few[1] > 1 and few[0] < SK_BASE:   # a split without tickets
             from . import _k
 
             return _k().gemm_split(x.reshape(-1, k), w, *few).view(*x.shape[:-1], n)

@@ -44,7 +44,8 @@ def _check(y, want):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,n,k", [(128, 4096, 64), (129, 4100, 192), (2446, 1536, 1024), (2446, 5632, 1024), (1000, 8196, 64), (8192, 260, 512)])
+@pytest.mark.parametrize("m,n,k", [(128, 4096, 64), (129, 4100, 192), (2446, 1536, 1024), (2446, 5632, 1024), (1000, 8196, 64), (8192, 260, 512),
+                                   (1000, 4096, 11008), (600, 4096, 14336), (300, 2048, 8192)])
 def test_linear(m, n, k):
     from chronos import ops
 
