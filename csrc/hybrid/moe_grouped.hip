@@ -17,7 +17,7 @@
 // positions of the same lane; the epilogue combines them and writes 64 columns of Z [rows, F] per tile.
 //
 // The tile loop is an LDS-DMA ring (16x16x32 bf16 MFMAs, XOR-swizzled images, one barrier per k-step with a counted vmcnt) at
-// three tile sizes, below.  Needs d % 128 == 0 and F % 128 == 0.
+// two tile sizes, below, and for experts with many tokens the projections' slab walk (chronos_slab.h).  Needs d % 128 == 0 and F % 128 == 0.
 #include "hybrid_common.h"
 #include "chronos_slab.h"
 #include "moe_tile.h"
