@@ -18,6 +18,8 @@ void launch_hy_embed(const int32_t*, const void*, float*, uint16_t*, int, int, f
 void launch_hy_low_rank_decay(const float*, const float*, const float*, float*, int, int, int, float, hipStream_t);
 void launch_hy_cast_bf16(const float*, uint16_t*, int64_t, hipStream_t);
 void launch_hy_layer_norm(const void*, bool, float*, const float*, void*, bool, int, int, float, hipStream_t);
+void launch_hy_layer_norm_slices(const float*, int, float*, const float*, uint16_t*, int, int, float, hipStream_t);
+void launch_hy_rms_norm_slices(const float*, int, float*, const float*, uint16_t*, int, int, float, float, hipStream_t);
 void launch_hy_rowdot(const void*, const void*, const float*, float*, int, int, int, bool, hipStream_t);
 void launch_hy_act(void*, int64_t, int, bool, hipStream_t);
 void launch_hy_mlstm_scan(const void*, int, const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*,
@@ -167,10 +169,27 @@ Tensor hy_layer_norm(const Tensor& x, const Tensor& w, double eps, bool out_f32)
     return h;
 }
 
+// y as float32 slices [S, T, D] of a bfloat16 product: the output of a join, checked
+static Tensor join_slices(const Tensor& y, const Tensor& x, const Tensor& w, bool out_f32) {
+    flt(y, "join: float32 slices");
+    need(!out_f32 && y.is_contiguous() && x.is_contiguous() && x.dim() == 2 && y.size(1) == x.size(0) && y.size(2) == x.size(1) && y.size(0) >= 1 && y.size(0) <= 64,
+         "join: slices [S, T, D], 1 <= S <= 64, of a bfloat16 stream");
+    need(x.size(1) % 8 == 0 && x.size(1) <= 8192 && w.numel() == x.size(1), "join: slices of rows of up to 8192 columns, a multiple of 8");
+    need(((reinterpret_cast<uintptr_t>(y.data_ptr()) | reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr())) & 15) == 0,
+         "join: slices need 16-byte aligned operands");
+    return at::empty_like(x, x.options().dtype(at::kBFloat16));
+}
+
 Tensor hy_add_layer_norm(const Tensor& y, Tensor& x, const Tensor& w, double eps, bool out_f32) {
     c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
     flt(x, "add_layer_norm: float32 residual");
     flt(w, "add_layer_norm: float32 weight");
+    if (y.dim() == 3) {
+        Tensor h = join_slices(y, x, w, out_f32);
+        chronos::launch_hy_layer_norm_slices(y.data_ptr<float>(), (int)y.size(0), x.data_ptr<float>(), w.data_ptr<float>(),
+                                             reinterpret_cast<uint16_t*>(h.data_ptr()), (int)x.size(0), (int)x.size(1), (float)eps, stream());
+        return h;
+    }
     need(is_act(y) && y.is_contiguous() && y.dim() == 2 && y.sizes() == x.sizes(), "add_layer_norm: y shape");
     need(f32(y) == out_f32, "add_layer_norm: y must be in the activation dtype");
     need(w.numel() == x.size(1), "add_layer_norm: weight size");
@@ -496,6 +515,12 @@ Tensor hy_scale_add_rms_norm(const Tensor& y, Tensor& x, const Tensor& w, double
     c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
     flt(x, "scale_add_rms_norm: float32 residual");
     flt(w, "scale_add_rms_norm: float32 weight");
+    if (y.dim() == 3) {
+        Tensor h = join_slices(y, x, w, out_f32);
+        chronos::launch_hy_rms_norm_slices(y.data_ptr<float>(), (int)y.size(0), x.data_ptr<float>(), w.data_ptr<float>(),
+                                           reinterpret_cast<uint16_t*>(h.data_ptr()), (int)x.size(0), (int)x.size(1), (float)alpha, (float)eps, stream());
+        return h;
+    }
     need(is_act(y) && y.is_contiguous() && y.dim() == 2 && y.sizes() == x.sizes(), "scale_add_rms_norm: y shape");
     need(f32(y) == out_f32, "scale_add_rms_norm: y must be in the activation dtype");
     need(w.numel() == x.size(1), "scale_add_rms_norm: weight size");

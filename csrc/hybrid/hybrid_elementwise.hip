@@ -113,10 +113,12 @@ __global__ void __launch_bounds__(256) layer_norm_plain_kernel(const float* __re
 // in registers between the statistics and the write, 8 columns per lane and step.  W waves share a row (1: four rows per
 // workgroup, no barrier; 4: one row).  Bound by the bytes of y, x in and out and h: 8192 x 2048 takes 35 us (5.8 TB/s) where
 // three strided passes took 68; 64 rows of 4096 take 5 us, not 14.
-template <int W, int NV>
-__global__ void __launch_bounds__(256) layer_norm_vec_kernel(const uint16_t* __restrict__ y, float* __restrict__ x,
-                                                             const float* __restrict__ w, uint16_t* __restrict__ h, int rows,
-                                                             int d, float eps) {
+// SL: y is S float32 slices [rows, d] of a product, summed in order and rounded here (a launch of 3 - 5 us
+// less; decode steps of 64 rows at width 4096 968 -> 958 us, of 3 rows at width 1024 213 -> 206).
+template <int W, int NV, bool SL>
+__global__ void __launch_bounds__(256) layer_norm_vec_kernel(const uint16_t* __restrict__ y, const float* __restrict__ ys, int S,
+                                                             float* __restrict__ x, const float* __restrict__ w,
+                                                             uint16_t* __restrict__ h, int rows, int d, float eps) {
     __shared__ float red[2][4];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int64_t row = W == 1 ? (int64_t)blockIdx.x * 4 + wv : blockIdx.x;
@@ -129,7 +131,21 @@ __global__ void __launch_bounds__(256) layer_norm_vec_kernel(const uint16_t* __r
     for (int j = 0; j < NV; ++j) {
         const int c = c0 + j * STEP;
         if (c < d) {
-            ld8(y + row * d + c, v[j]);
+            if constexpr (SL) {
+                const float* p = ys + row * d + c;
+                ld8f(p, v[j]);
+#pragma unroll 4
+                for (int k = 1; k < S; ++k) {
+                    float t[8];
+                    ld8f(p + (int64_t)k * rows * d, t);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[j][e] += t[e];
+                }
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[j][e] = bf2f(f2bf(v[j][e]));
+            } else {
+                ld8(y + row * d + c, v[j]);
+            }
             ld8f(x + row * d + c, xs[j]);
 #pragma unroll
             for (int e = 0; e < 8; ++e) s += v[j][e];
@@ -356,10 +372,10 @@ void launch_hy_layer_norm(const void* y, bool y_f32, float* x, const float* w, v
     if (x != nullptr && !y_f32 && d % 8 == 0 && d <= 8192 && hy::aligned16(y, x, w, h)) {
         const uint16_t* yb = (const uint16_t*)y;
         uint16_t* hb = (uint16_t*)h;
-        if (d <= 1024) hy::layer_norm_vec_kernel<1, 2><<<(rows + 3) / 4, 256, 0, s>>>(yb, x, w, hb, rows, d, eps);
-        else if (d <= 2048) hy::layer_norm_vec_kernel<4, 1><<<rows, 256, 0, s>>>(yb, x, w, hb, rows, d, eps);
-        else if (d <= 4096) hy::layer_norm_vec_kernel<4, 2><<<rows, 256, 0, s>>>(yb, x, w, hb, rows, d, eps);
-        else hy::layer_norm_vec_kernel<4, 4><<<rows, 256, 0, s>>>(yb, x, w, hb, rows, d, eps);
+        if (d <= 1024) hy::layer_norm_vec_kernel<1, 2, false><<<(rows + 3) / 4, 256, 0, s>>>(yb, nullptr, 0, x, w, hb, rows, d, eps);
+        else if (d <= 2048) hy::layer_norm_vec_kernel<4, 1, false><<<rows, 256, 0, s>>>(yb, nullptr, 0, x, w, hb, rows, d, eps);
+        else if (d <= 4096) hy::layer_norm_vec_kernel<4, 2, false><<<rows, 256, 0, s>>>(yb, nullptr, 0, x, w, hb, rows, d, eps);
+        else hy::layer_norm_vec_kernel<4, 4, false><<<rows, 256, 0, s>>>(yb, nullptr, 0, x, w, hb, rows, d, eps);
     } else if (x != nullptr) {
         if (y_f32) hy::layer_norm_kernel<float, float, true><<<rows, 256, 0, s>>>((const float*)y, x, w, (float*)h, d, eps);
         else hy::layer_norm_kernel<uint16_t, uint16_t, true><<<rows, 256, 0, s>>>((const uint16_t*)y, x, w, (uint16_t*)h, d, eps);
@@ -370,6 +386,13 @@ void launch_hy_layer_norm(const void* y, bool y_f32, float* x, const float* w, v
         if (out_f32) hy::layer_norm_kernel<float, float, false><<<rows, 256, 0, s>>>((const float*)y, nullptr, w, (float*)h, d, eps);
         else hy::layer_norm_kernel<float, uint16_t, false><<<rows, 256, 0, s>>>((const float*)y, nullptr, w, (uint16_t*)h, d, eps);
     }
+}
+// d % 8 == 0, d <= 8192, everything on 16 bytes
+void launch_hy_layer_norm_slices(const float* ys, int S, float* x, const float* w, uint16_t* h, int rows, int d, float eps, hipStream_t s) {
+    if (rows == 0) return;
+    if (d <= 2048) hy::layer_norm_vec_kernel<4, 1, true><<<rows, 256, 0, s>>>(nullptr, ys, S, x, w, h, rows, d, eps);
+    else if (d <= 4096) hy::layer_norm_vec_kernel<4, 2, true><<<rows, 256, 0, s>>>(nullptr, ys, S, x, w, h, rows, d, eps);
+    else hy::layer_norm_vec_kernel<4, 4, true><<<rows, 256, 0, s>>>(nullptr, ys, S, x, w, h, rows, d, eps);
 }
 template <typename T>
 static void rowdot_t(const T* h, const T* w, const float* bias, float* out, int rows, int d, int n, hipStream_t s) {

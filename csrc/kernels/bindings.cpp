@@ -687,17 +687,20 @@ std::tuple<Tensor, Tensor> gemm_few(const Tensor& x, const Tensor& w, int64_t cf
     return {y, yf};
 }
 
-// A plain product of few rows whose K is split over workgroups, nothing kept between calls (gemm_lg.hip's 64-row tiles and smaller).
-Tensor gemm_split(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk) {
+// The float32 slices [splitk, M, N] of a plain product of few rows whose K is split over workgroups, nothing kept between calls: gemm_lg.hip's
+// 64-row tiles and smaller, or (skinny) gemm_skinny.hip's uneven configs.  Their sum in order, rounded, is the product.
+Tensor gemm_slices(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk, bool skinny) {
     chk_bf16(x, "x");
     chk_bf16(w, "w");
     const int64_t K = x.size(-1), M = x.numel() / K, N = w.size(0);
     CHK(w.dim() == 2 && w.size(1) == K, "gemm_split: w must be [N, K]");
-    CHK(cfg == 33 || cfg == 36 || (cfg >= 38 && cfg <= 39) || (cfg >= 72 && cfg <= 75) || cfg == 78 || cfg == 79, "gemm_split: cfg");
-    const int BM = chronos::gemm_lg_xm((int)cfg), BN = chronos::gemm_lg_wn((int)cfg);
+    CHK(skinny ? cfg >= chronos::kSkinnyUneven && cfg < chronos::kSkinnyConfigs : cfg == 33 || cfg == 36 || (cfg >= 38 && cfg <= 39) || (cfg >= 72 && cfg <= 75) || cfg == 78 || cfg == 79, "gemm_split: cfg");
+    const int BM = skinny ? 16 * chronos::gemm_skinny_mt((int)cfg) : chronos::gemm_lg_xm((int)cfg);
+    const int BN = skinny ? 16 * chronos::gemm_skinny_rt((int)cfg) : chronos::gemm_lg_wn((int)cfg);
     CHK((N + BN) * K * 2 < (1LL << 31) && (M + BM) * K * 2 < (1LL << 31), "gemm_split: operand > 2 GiB");
+    CHK(!skinny || (M <= BM && N % BN == 0), "gemm_split: M, N of the config");
     CHK(M >= 1 && K % 64 == 0 && K <= (1 << 20) && N >= 4 && N % 4 == 0, "gemm_split: size");
-    CHK(splitk > 1 && splitk <= 64 && (K / 64) % splitk == 0, "gemm_split: splitk must divide K / 64");
+    CHK(splitk > 1 && splitk <= 64 && (skinny || (K / 64) % splitk == 0), "gemm_split: splitk must divide K / 64");
     CHK(((reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr())) & 15) == 0, "gemm_split: alignment");
     c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
     chronos::PPArgs a{};
@@ -710,11 +713,18 @@ Tensor gemm_split(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk)
     a.splitk = (int)splitk;
     a.kts = (int)(K / 64 / splitk);
     a.gm = chronos::knob("pp_gm", 8);
-    Tensor y = at::empty({M, N}, x.options()), ws = at::empty({splitk * M * N}, x.options().dtype(at::kFloat));
-    a.y = bfm(y);
+    Tensor ws = at::empty({splitk, M, N}, x.options().dtype(at::kFloat));
     a.ws = ws.data_ptr<float>();
-    CHK(chronos::launch_gemm_lg((int)cfg, 0, false, a, cur_stream()), "gemm_split: launch");
-    chronos::launch_gemm_slices(a.ws, a.y, M * N, (int)splitk, cur_stream());
+    CHK(skinny ? chronos::launch_gemm_skinny((int)cfg, 0, false, a, cur_stream()) : chronos::launch_gemm_lg((int)cfg, 0, false, a, cur_stream()),
+        "gemm_split: launch");
+    return ws;
+}
+
+Tensor gemm_split(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk) {
+    const Tensor ws = gemm_slices(x, w, cfg, splitk, false);
+    c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+    Tensor y = at::empty({ws.size(1), ws.size(2)}, x.options());
+    chronos::launch_gemm_slices(ws.data_ptr<float>(), bfm(y), y.numel(), (int)splitk, cur_stream());
     return y;
 }
 
@@ -942,6 +952,7 @@ TORCH_LIBRARY(chronos, m) {
     m.def("gemm_act(Tensor x, Tensor w, int mode, float limit, float slope, float shift) -> Tensor");
     m.def("gemm_few(Tensor x, Tensor w, int cfg, int mode, int n0, int nf, Tensor? bias, float limit, float slope, float shift) -> (Tensor, Tensor)");
     m.def("gemm_split(Tensor x, Tensor w, int cfg, int splitk) -> Tensor");
+    m.def("gemm_slices(Tensor x, Tensor w, int cfg, int splitk, bool skinny) -> Tensor");
     m.def("gemm_pp(Tensor x, Tensor w, int mode, int cfg, int splitk, Tensor? resid, Tensor? part_in, float eps, bool prio) -> (Tensor, Tensor)");
     m.def("gemm_skinny(Tensor x, Tensor w, int mode, int cfg, int splitk, Tensor? resid, Tensor? part_in, float eps) "
           "-> (Tensor, Tensor)");
@@ -987,6 +998,7 @@ TORCH_LIBRARY_IMPL(chronos, CUDA, m) {
     m.impl("gemm_act", &gemm_act);
     m.impl("gemm_few", &gemm_few);
     m.impl("gemm_split", &gemm_split);
+    m.impl("gemm_slices", &gemm_slices);
     m.impl("gemm_pp", &gemm_pp);
     m.impl("gemm_skinny", &gemm_skinny);
     m.impl("gemv_resid", &gemv_resid);

@@ -366,7 +366,7 @@ void launch_cfg(const PPArgs& a, hipStream_t st) {
     }
     const int G = sk_pair(MODE) ? a.F / (8 * RT) : a.N / (16 * RT);
     hipLaunchKernelGGL(kern, dim3(G * a.splitk), dim3(64 * NW), lds, st, a);
-    if (a.splitk > 1 && a.cnt == nullptr) launch_gemm_slices(a.ws, a.y, (int64_t)a.M * a.N, a.splitk, st);
+    if (a.splitk > 1 && a.cnt == nullptr && a.y != nullptr) launch_gemm_slices(a.ws, a.y, (int64_t)a.M * a.N, a.splitk, st);
 }
 
 // configs {RT (W tiles of 16 rows per workgroup), MT (x tiles: M <= 16 MT), D (ring depth in 64-k units), NW (waves

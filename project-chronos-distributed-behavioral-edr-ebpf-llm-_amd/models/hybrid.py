@@ -866,7 +866,7 @@ def mix_mlstm(model, li: int, spec: MLSTMSpec, w: dict, h, meta: StepMeta, cache
     o = hops.mlstm_scan(proj, gate_pre, meta.q_start, meta.pos0, meta.slots, cache.S[li], cache.n[li], cache.m[li],
                         H, D, Dv, spec.gate_cap, meta.max_q)
     y = hops.mlstm_out(o, proj, 2 * H * D + H * Dv, w["norm"], model.cfg.norm_eps, model.act_dtype)
-    return hops.matmul(y, w["w_o"])
+    return model.last_product(y, w["w_o"])
 
 
 @dataclass
@@ -928,7 +928,7 @@ def mix_latent_attention(model, li: int, spec: LatentAttentionSpec, w: dict, h, 
         kv = hops.matmul(lat, w["w_kv"]).view(T, H, D + spec.vdim)
         ov = hops.latent_expanded(q, kv, kr, meta.q_start, gate, proj if spec.gate and spec.gate_wide else None, nq + nkv,
                                   w.get("sink"), spec.scale, meta.max_q, spec.window, None if ov is None else ov.view(T, H, spec.vdim))
-        return _with_gate(hops.matmul(ov.view(T, H * spec.vdim) if wide is None else wide, w["w_o"]), proj, w)
+        return _with_gate(model.last_product(ov.view(T, H * spec.vdim) if wide is None else wide, w["w_o"]), proj, w)
     # the query goes into the latent space (q_u W_uk per head), so a key is the cached row itself; the output
     # comes back through W_uv per head
     qa = torch.empty(T, H, rank + R, device=h.device, dtype=h.dtype)
@@ -939,7 +939,7 @@ def mix_latent_attention(model, li: int, spec: LatentAttentionSpec, w: dict, h, 
                                model.act_dtype, meta.max_q, spec.window, spec.two_term, w.get("sink"))
     ov = hops.head_matmul(oa, w["w_uv"], None if ov is None else ov.view(T, H, spec.vdim),
                           proj if spec.gate and spec.gate_wide else None, nq + nkv if own else nq)
-    return _with_gate(hops.matmul(ov.view(T, H * spec.vdim) if wide is None else wide, w["w_o"]), proj, w)
+    return _with_gate(model.last_product(ov.view(T, H * spec.vdim) if wide is None else wide, w["w_o"]), proj, w)
 
 
 def mix_window_attention(model, li, spec: WindowAttentionSpec, w: dict, h, meta: StepMeta, cache: HybridCache):
@@ -980,7 +980,7 @@ def mix_window_attention(model, li, spec: WindowAttentionSpec, w: dict, h, meta:
                               spec.chunk, spec.pool if pooled else 0, cache.kp.get(li), cache.vp.get(li),
                               model.rope_v.get(li), (H + G) * D + G * Dv if spec.gate and spec.gate_wide else -1,
                               cache.ks.get(li), out)
-    return _with_gate(hops.matmul(o if wide is None else wide, w["w_o"], w.get("b_o")), proj, w)
+    return _with_gate(model.last_product(o if wide is None else wide, w["w_o"], w.get("b_o")), proj, w)
 
 
 def mix_retention(model, li, spec: RetentionSpec, w: dict, h, meta: StepMeta, cache: HybridCache):
@@ -1044,7 +1044,7 @@ def mix_delta_rule(model, li: int, spec: DeltaRuleSpec, w: dict, h, meta: StepMe
     qscale, kscale, decay, beta = hops.delta_prep(y, ab, w["a_log"], HK, H, D, D ** -0.5)
     o = hops.linear_scan(y, 0, HK * D, 2 * HK * D, qscale, kscale, 1.0, decay, beta, meta.q_start, meta.pos0,
                          meta.slots, cache.S[li], HK, H, D, Dv, max_q=meta.max_q)
-    return hops.matmul(hops.head_norm_gate(o, proj, C, w["norm"], model.cfg.norm_eps, True, model.act_dtype), w["w_o"])
+    return model.last_product(hops.head_norm_gate(o, proj, C, w["norm"], model.cfg.norm_eps, True, model.act_dtype), w["w_o"])
 
 
 def mix_gla(model, li: int, spec: GLASpec, w: dict, h, meta: StepMeta, cache: HybridCache):
@@ -1054,11 +1054,11 @@ def mix_gla(model, li: int, spec: GLASpec, w: dict, h, meta: StepMeta, cache: Hy
     o = hops.linear_scan(proj, 0, H * D, 2 * H * D, None, None, D ** -0.5, decay, None, meta.q_start, meta.pos0,
                          meta.slots, cache.S[li], H, H, D, Dv, max_q=meta.max_q)
     o = hops.head_norm_gate(o, proj, 2 * H * D + H * Dv, w["norm"], model.cfg.norm_eps, True, model.act_dtype)
-    return _with_gate(hops.matmul(o, w["w_o"]), proj, w)
+    return _with_gate(model.last_product(o, w["w_o"]), proj, w)
 
 
 def ff_glu(model, spec: GluFFSpec, w: dict, h):
-    return hops.matmul(hops.matmul_glu(h, w["w_gu"], spec.limit, spec.slope, spec.shift, model.act_dtype), w["w_down"])
+    return model.last_product(hops.matmul_glu(h, w["w_gu"], spec.limit, spec.slope, spec.shift, model.act_dtype), w["w_down"])
 
 
 def ff_moe_glu(model, spec: MoEGluSpec, w: dict, h):
@@ -1080,7 +1080,7 @@ def ff_moe_group_glu(model, spec: MoEGroupGluSpec, w: dict, h):
 
 
 def ff_dense(model, spec: DenseFFSpec, w: dict, h):
-    return hops.matmul(hops.matmul_act(h, w["w_up"], spec.act), w["w_down"])
+    return model.last_product(hops.matmul_act(h, w["w_up"], spec.act), w["w_down"])
 
 
 def ff_poly(model, spec: PolyFFSpec, w: dict, h):
@@ -1404,6 +1404,12 @@ class HybridDecoder:
             h = hops.layer_norm_join(y, x, None if last else w.layers[runs[ri + 1]].norm1, eps, at, y2, emit=not last)
             if self.layer_tap is not None:
                 self.layer_tap(ri, x)
+
+    def last_product(self, x, w, bias=None):
+        """A sublayer's last product, in the form that its stream's join takes (see _join and matmul_slices)."""
+        if bias is None and self.cfg.residual in ("out_norm", "post_norm"):
+            return hops.matmul_slices(x, w)
+        return hops.matmul(x, w, bias)
 
     def _join(self, y, x, w):
         """The residual rule: folds the sublayer output y into the float32 stream x (in place) and returns the

@@ -262,6 +262,20 @@ def few_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     return out
 
 
+def product_slices(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
+    """The float32 slices [S, M, N] of x @ w.T where few_rows_plan splits K, or None: for kernels that take them in the product's place."""
+    (m, k), n = x.shape if x.dim() == 2 else (0, 0), w.shape[0]
+    if not 0 < m <= 64 or n % 8 or n > 8192 or not _plain_rows(x, w):
+        return None
+    plan = few_rows_plan(m, n, k)
+    if plan is None or plan[1] == 1 or (plan[0] >= SK_BASE and plan[0] not in _UNEVEN):
+        return None
+    from . import _k
+
+    skinny = plan[0] >= SK_BASE
+    return _k().gemm_slices(x, w, plan[0] - SK_BASE * skinny, plan[1], skinny)
+
+
 # Many rows, shapes that the plan does not list: what a launch takes in us, fitted on a grid of M = 65 .. 8192, N = 512 .. 16384, K = 512 ..
 # 8192 (rms error 10 %, 18 % for 88).  88 (gemm_slab.hip): constant, per half tile of the last round, per 64-deep step of a round of
 # 256 x 256 tiles and of the halves, per M of results, per M of weights; 19 and 32 (128 x rows by 128 and 64 W rows): constant, per round of

@@ -60,6 +60,18 @@ def matmul(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None) -
     return torch.matmul(x, w.t())
 
 
+def matmul_slices(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x @ w.T for add_layer_norm or scale_add_rms_norm, which also take a product of few rows as the float32 slices [S, T, n] of its split and
+    sum and round them themselves, a launch less."""
+    if _gpu(x) and x.dtype == torch.bfloat16:
+        from .gemm import product_slices
+
+        y = product_slices(x, w)
+        if y is not None:
+            return y
+    return matmul(x, w)
+
+
 def embed_rows(ids, table, act_dtype, scale: float = 1.0, emit: bool = True):
     """(float32 residual rows times ``scale``, the same rows in the activation dtype or None when ``emit`` is off)."""
     if _gpu(table):
@@ -78,7 +90,7 @@ def layer_norm(x, w, eps: float, act_dtype):
 
 def add_layer_norm(y, x, w, eps: float, act_dtype):
     """x (float32 residual, in place) <- x + layer_norm(y) * w; returns the updated rows in the activation dtype
-    (x itself when that is float32)."""
+    (x itself when that is float32).  y: rows, or on the GPU a product's slices (matmul_slices)."""
     if _gpu(x):
         h = _k().hy_add_layer_norm(y, x, w, eps, _f32(act_dtype))
         return x if _f32(act_dtype) else h
