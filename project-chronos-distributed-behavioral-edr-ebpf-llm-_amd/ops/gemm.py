@@ -280,7 +280,7 @@ def product_slices(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
 # 8192 (rms error 10 %, 18 % for 88).  88 (gemm_slab.hip): constant, per half tile of the last round, per 64-deep step of a round of
 # 256 x 256 tiles and of the halves, per M of results, per M of weights; 19 and 32 (128 x rows by 128 and 64 W rows): constant, per round of
 # 256 tiles, per 256 tiles, per 64-deep step of these two, per M of weights.  Of all tile configs these three suffice: the pick is within
-# 1 % of the fastest of eight on average.
+# 1 % of the fastest of eight on average.  Both grids, here and at _MANY_SPLIT: profiles/many_rows_gemm.json.
 _MANY_88 = (2.6, 1.9, 1.17, 0.55, 0.52, 0.29)
 _MANY_TILES = {19: (128, 2.9, 1.9, 1.2, 0.294, 0.15, 0.16), 32: (64, 2.7, 1.45, 0.46, 0.224, 0.083, 0.13)}
 # ... and with an activation in 88's epilogue, the gated unit and the others; the same activation as a pass of its own: constant, per M of
