@@ -63,7 +63,17 @@ __global__ void __launch_bounds__(256) short_conv_vec_kernel(const uint16_t* __r
                                                              int C, int TK, int silu, const float* __restrict__ bias, bool one_each) {
     const int gx = (C / 8 + 255) / 256, c = (blockIdx.x % gx * 256 + threadIdx.x) * 8;   // workgroups of the same tokens side by side
     if (c >= C) return;
-    const int tb = blockIdx.x / gx * TK, te = min(tb + TK, T);
+    const int tb = blockIdx.x / gx * TK;
+    int te = min(tb + TK, T);
+    uint16_t* last = nullptr;   // one_each: where the history behind the sequence's last token goes
+    if (one_each) {   // (TK is 1)  a sequence that does bring more tokens is walked by its first one's thread: history that is read and
+        const int b = tok_seq[tb], t0 = q_start[b], t1 = min(q_start[b + 1], T);   // written in one pass stays with one thread
+        if (tb > t0 && tb < t1) return;
+        if (tb == t0 && t1 > t0) {
+            te = t1;
+            last = hist + (int64_t)slots[b] * (K - 1) * C + c;
+        }
+    }
     float wf[8][K], bv[8], in[K][8];   // in[i]: the input K - 1 - i tokens back
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -103,10 +113,10 @@ __global__ void __launch_bounds__(256) short_conv_vec_kernel(const uint16_t* __r
             if (silu) acc[e] *= sigmoid_act<uint16_t>(acc[e]);
         }
         st8(y + (int64_t)t * C + c, acc);
-        if (one_each) {   // the sequence's only token of this step (TK is 1): these channels' history in the same pass
+    }
+    if (last != nullptr) {
 #pragma unroll
-            for (int i = 0; i + 1 < K; ++i) st8(hist + ((int64_t)slots[b] * (K - 1) + i) * C + c, in[i + 1]);
-        }
+        for (int i = 0; i + 1 < K; ++i) st8(last + (int64_t)i * C, in[i + 1]);
     }
 }
 
@@ -442,7 +452,8 @@ void launch_hy_conv_hist(const void* x, int ldx, const int32_t* q_start, const i
     else hy::conv_hist_kernel<uint16_t><<<hg, 256, 0, s>>>((const uint16_t*)x, ldx, q_start, pos0, slots, (uint16_t*)hist, C, K);
 }
 
-// one_each: no sequence brings more than one token (the history is then rewritten in the same pass where 8 channels go together)
+// one_each: sequences bring one token, as a rule (the history is then rewritten in the same pass where 8 channels go together; one of more
+// tokens is right too, only slower)
 void launch_hy_short_conv(const void* x, int ldx, const float* w, const float* bias, const int32_t* tok_seq,
                           const int32_t* q_start, const int32_t* pos0, const int32_t* slots, void* hist, void* y, int T,
                           int B, int C, int K, bool silu, bool one_each, bool f32, hipStream_t s) {

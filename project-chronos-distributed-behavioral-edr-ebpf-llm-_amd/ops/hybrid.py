@@ -296,8 +296,8 @@ def window_attention(qkv, kc, vc, block_table, q_start, pos, sink, gate, scale: 
 
 
 def short_conv(x, w, tok_seq, q_start, pos0, slots, hist, silu: bool = True, bias=None, x_off: int = 0, max_q: int = 0):
-    """``max_q``: the most tokens any sequence brings in this step (with 1 the history is rewritten in the same pass; 0 =
-    unknown)."""
+    """``max_q``: the most tokens any sequence brings in this step (with 1 the history is rewritten in the same pass; any value gives the
+    same results; 0 = unknown)."""
     if _gpu(x):
         return _k().hy_short_conv(x, w, tok_seq, q_start, pos0, slots, hist, silu, bias, x_off, max_q)
     return ref.short_conv(x, w, q_start, pos0, slots, hist, silu, bias, x_off)

@@ -99,6 +99,23 @@ def test_one_token_each_convolution(C, K):
     assert torch.equal(h2[3], hist[3]) and torch.equal(h2[4, -1], x[0])
 
 
+@pytest.mark.parametrize("C,K", [(512, 4), (4104, 3), (8, 2)])
+def test_convolution_whatever_max_q_says(C, K):
+    """max_q = 1 beside sequences of 0, 1, 2 and 9 tokens: the bits of the two launches, outputs and history."""
+    from chronos.ops import hybrid as H
+
+    g = _g(C + K)
+    lens = [2, 1, 0, 9, 1]
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    q = [sum(lens[:i]) for i in range(len(lens) + 1)]
+    x, w = torch.randn(q[-1], C, device=DEV, generator=g).to(BF), torch.randn(C, K, device=DEV, generator=g)
+    hist = torch.randn(7, K - 1, C, device=DEV, generator=g).to(BF)
+    args = (x, w, i32([b for b, n in enumerate(lens) for _ in range(n)]), i32(q), i32([6, 0, 4, 1, 8]), i32([5, 1, 2, 0, 6]))
+    h1, h2 = hist.clone(), hist.clone()
+    y1, y2 = H.short_conv(*args, h1, True), H.short_conv(*args, h2, True, max_q=1)
+    assert torch.equal(y1, y2) and torch.equal(h1, h2) and torch.equal(h2[2:5], hist[2:5])
+
+
 @pytest.mark.parametrize("rows,d", [(1, 4), (64, 4096), (7, 1000), (3, 2052), (2, 5000)])
 @pytest.mark.parametrize("dt", [BF, torch.float32])
 def test_plain_layer_norm(rows, d, dt):
