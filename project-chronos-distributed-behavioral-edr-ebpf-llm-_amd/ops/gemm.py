@@ -265,7 +265,7 @@ def few_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
 def product_slices(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
     """The float32 slices [S, M, N] of x @ w.T where few_rows_plan splits K, or None: for kernels that take them in the product's place."""
     (m, k), n = x.shape if x.dim() == 2 else (0, 0), w.shape[0]
-    if not 0 < m <= 64 or n % 8 or n > 8192 or not _plain_rows(x, w):
+    if not 0 < m <= 64 or n % 8 or n > 8192 or not _plain_rows(x, w) or _registered(m, n, k):
         return None
     plan = few_rows_plan(m, n, k)
     if plan is None or plan[1] == 1 or (plan[0] >= SK_BASE and plan[0] not in _UNEVEN):
@@ -362,7 +362,7 @@ def product_act(x: torch.Tensor, w: torch.Tensor, mode: int, limit: float = 0.0,
     faster by their models.  On the grid of _MANY_88: gated units 1.13 times as fast (189 shapes; the worst 0.94), the others 1.16
     (196; 0.95)."""
     m, (n, k) = x.numel() // max(1, x.shape[-1]), w.shape
-    if 64 < m < MANY_MIN or PP_MODE != "auto" or x.dim() != 2 or not _plain_rows(x, w):
+    if 64 < m < MANY_MIN or PP_MODE != "auto" or x.dim() != 2 or not _plain_rows(x, w) or _registered(m, n, k):
         return None
     if m <= 64:
         from . import _k
@@ -407,7 +407,7 @@ def _few_more(m: int, n: int, k: int, kind: int) -> int:
 
 def product_rows(x: torch.Tensor, w: torch.Tensor, n0: int, nf: int, bias: Optional[torch.Tensor]):
     """(x @ w[:n0].T, float32 x @ w[n0 : n0 + nf].T + bias) in one launch, or None where two are faster."""
-    if x.dim() != 2 or not 0 < x.shape[0] <= 64 or not _plain_rows(x, w):
+    if x.dim() != 2 or not 0 < x.shape[0] <= 64 or not _plain_rows(x, w) or _registered(x.shape[0], n0, w.shape[1]):
         return None
     cfg = _few_more(x.shape[0], *w.shape, 0)
     if not cfg:
@@ -445,6 +445,11 @@ _custom: list[tuple[Callable[[int, int, int], bool], Callable[[torch.Tensor, tor
 
 def register(pred: Callable[[int, int, int], bool], fn: Callable[[torch.Tensor, torch.Tensor], torch.Tensor]) -> None:
     _custom.append((pred, fn))
+
+
+def _registered(m: int, n: int, k: int) -> bool:
+    """Is a kernel registered for this product?  Then linear() calls it, and no launch that takes the product along with something else."""
+    return any(pred(m, n, k) for pred, _ in _custom)
 
 
 @dataclass

@@ -32,6 +32,33 @@ def test_measured_plan_and_modes_come_first(monkeypatch):
         assert G.many_rows_plan(8192, 2048, 2048) is None
 
 
+def test_registered_kernels_get_their_products(monkeypatch):
+    """A product that a kernel is registered for is linear()'s: no launch that takes it along with a sum, rows behind or an activation."""
+    import chronos.ops as ops
+
+    calls = []
+
+    class Kernels:
+        def __getattr__(self, name):
+            return lambda *args: calls.append(name) or ("y", "f")
+
+    monkeypatch.setattr(ops, "_k", Kernels)
+    x, w = torch.zeros(8, 1024, dtype=torch.bfloat16), torch.zeros(4096, 1024, dtype=torch.bfloat16)
+    x2 = torch.zeros(4, 4096, dtype=torch.bfloat16)
+    w2 = torch.zeros(4096, 4096, dtype=torch.bfloat16)
+    xm = torch.zeros(4096, 1024, dtype=torch.bfloat16)
+    monkeypatch.setattr(G, "_custom", [])
+
+    def every():
+        return (G.product_slices(x2, w2), G.product_rows(x, w, 4064, 32, None), G.product_act(x, w, 3), G.product_act(xm, w, 5))
+
+    assert None not in every() and calls == ["gemm_slices", "gemm_few", "gemm_few", "gemm_act"]
+    G.register(lambda m, n, k: (m, n, k) in ((4, 4096, 4096), (8, 4064, 1024), (8, 4096, 1024), (4096, 4096, 1024)), lambda x, w: None)
+    assert every() == (None, None, None, None) and len(calls) == 4
+    G._custom[:] = [(lambda m, n, k: (m, n, k) == (8, 4064, 1025), None)]
+    assert None not in every()
+
+
 def _operands(m, n, k):
     g = torch.Generator(device=DEV).manual_seed(m + n + k)
     return torch.randn(m, k, device=DEV, generator=g).bfloat16(), (torch.randn(n, k, device=DEV, generator=g) * k ** -0.5).bfloat16()
