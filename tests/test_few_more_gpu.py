@@ -72,6 +72,17 @@ def test_low_rank_decay(T, R, C, p):
     assert (ours.double() - want).norm() <= 1.05 * (theirs.double() - want).norm() + 1e-7 * want.norm()
 
 
+@pytest.mark.parametrize("T", [4 * 65535, 4 * 65535 + 1, 300001])
+def test_low_rank_decay_of_many_tokens(T):
+    """More tokens than a grid's second axis has blocks for."""
+    from chronos.ops import hybrid as H
+
+    g = _g(T)
+    a, w, b = (torch.randn(s, device=DEV, generator=g) for s in ((T, 2), (2, 4), (4,)))
+    want = torch.sigmoid(b.double() + a.double() @ w.double()) ** 0.25
+    assert ((H.low_rank_decay(a, w, b, 0.25).double() - want).abs() <= 1e-6).all()   # (values below 1, a few units of the last place)
+
+
 @pytest.mark.parametrize("d", [64, 1000, 2052])
 @pytest.mark.parametrize("dt", [BF, torch.float32])
 def test_embed_both(d, dt):
