@@ -69,8 +69,8 @@ _UNEVEN = {112: (16, 32, 8), 113: (16, 64, 8), 114: (16, 16, 8), 115: (32, 16, 8
 # Few rows, plain epilogue, shapes that the plan does not list: per largest M the configs that won somewhere on a grid of
 # N = 512 .. 32768 by K = 512 .. 14336, and what a launch of each takes in us, fitted on that grid (cold weights; rms error 5 %):
 # constant, split-K's second launch, per 64-deep step of a wave, per MB of weights, per 256 workgroups, per such step of each
-# further round of 256 workgroups, per 100 MB of x that all workgroups read together.  The pick is within 1 % of the best config on average.
-# profiles/few_rows_gemm.json: 68 of the shapes, every one measured with the library, the best config and the pick.
+# further round of 256 workgroups, per 100 MB of x that all workgroups read together.  The pick of the rule takes 3 % longer than the best config on average.
+# profiles/few_rows_gemm.json: 86 shapes by 12 numbers of rows, every one measured with the library, the best config and the pick.
 _FEW = ((16, {114: (2.4, 2.0, 0.77, 0.016, 0.23, 0.69, 3.4), 115: (2.2, 2.1, 1.4, 0.0082, 0.57, 1.3, 5.1),
               72: (2.2, 0.0, 0.16, 0.07, 1.2, 0.24, 8.3), 75: (1.7, 0.0, 0.28, 0.1, 1.4, 0.0, 10.0)}),
         (32, {112: (2.3, 2.1, 1.1, 0.0, 0.67, 0.9, 1.0), 72: (2.1, 0.0, 0.18, 0.052, 1.5, 0.22, 8.7),
@@ -78,9 +78,10 @@ _FEW = ((16, {114: (2.4, 2.0, 0.77, 0.016, 0.23, 0.69, 3.4), 115: (2.2, 2.1, 1.4
         (64, {113: (2.4, 2.3, 1.5, 0.0, 0.9, 1.0, 0.75), 72: (2.2, 0.0, 0.16, 0.0, 1.3, 0.19, 5.1),
               38: (3.0, 0.0, 0.31, 0.0, 0.54, 0.0, 35.0), 39: (2.4, 0.0, 0.21, 0.0, 1.2, 0.22, 14.0)}))
 # Few rows, more weights than that: gemm_lg.hip's small tiles, K split over workgroups without tickets (gemm_split).  The same terms, and per M
-# of partial sums (rms error 7 %), fitted at 19 shapes of 4 to 134 M elements by 2 .. 64 rows.
-_FEW_LARGE = ((32, {72: (2.1, 1.8, 0.13, 0.122, 1.54, 0.121, 0.17, 1.5), 74: (1.1, 2.35, 0.189, 0.118, 0.8, 0.099, 0.12, 1.7),
-                    79: (2.6, 1.9, 0.139, 0.101, 1.8, 0.17, 0.26, 1.4)}),
+# of partial sums, fitted on the "large" table of profiles/few_rows_gemm.json: 2 .. 32 rows at 65 shapes of 4 to 134 M elements (rms error 7 %;
+# 33 .. 64 rows at 19 shapes of them, 10 % over all 65).
+_FEW_LARGE = ((32, {72: (2.2, 2.32, 0.17, 0.0623, 1.53, 0.206, 1.66, 0.92), 74: (2.19, 2.32, 0.238, 0.049, 0.744, 0.186, 1.55, 1.02),
+                    79: (2.6, 2.3, 0.172, 0.0595, 1.78, 0.225, 1.72, 0.917)}),
               (64, {39: (1.1, 2.7, 0.223, 0.0915, 0.94, 0.229, 0.0, 1.9), 38: (1.4, 2.7, 0.35, 0.105, 1.65, 0.259, 0.0, 1.7)}))
 _plan_cache: dict = {}
 _plan_table: Optional[dict] = None
@@ -208,19 +209,26 @@ def pp_plan(m: int, n: int, k: int, mode: int = PP_PLAIN) -> Optional[tuple[int,
     return out
 
 
+def _library_streams(m: int, n: int, k: int) -> bool:
+    """Shapes beyond _FEW's where the library reads the weights at 4 TB/s and these kernels do not.  us, library and the pick without this line:
+    16 rows of 4096 x 8192 16.4 and 19.2, 8192 x 4096 16.1 and 18.5, 5120 x 5120 15.8 and 16.7, 8192 x 8192 29.5 and 31.2; 64 rows of 8192 x 4096 19.1
+    and 20.6.  Not at other K, nor with more rows for fewer outputs: 16 rows of 4096 x 6400 23.6 and 14.5, 24 rows of 3584 x 7168 20.3 and 14.6, 64
+    of 5632 x 5632 23.4 and 22.1.  Of 437 shapes 53 would be slower than the library by more than 3 % without this line, 7 are with it."""
+    return n * k >= 25_000_000 and 2560 <= n <= 8192 and k <= 8192 and k % 1024 == 0 and (m <= 16 or n >= 4096 and m <= 32 or n > 7168)
+
+
 def few_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     """(config, split-K) of the hand-written GEMM for few rows of a shape that no plan lists, or None (the GEMV or the
     library): of shapes that the kernels take (rows of w in 16s, at least one; K in 64s up to 2^20).  Where it wins, measured on the
     grid of _FEW, us, GEMV or library -> this:
     one row: K < 2048, where the GEMV's waves have one step each (5632 x 1024: 7.3 -> 5.7; 32768 x 512: 22 -> 9.7; at K = 2048 the
     two are level), and K % 512, which the GEMV does not take (1024 x 2816: 8.6 -> 5.7): no slower at any of 41 shapes;
-    2 .. 64 rows: weights up to 12.5 M elements, from 33 rows on up to 7 M or K <= 2048 (2048 x 2048, 16 rows: 11.0 -> 6.0; 64 rows:
-    11.7 -> 8.1): 1.3 .. 1.6 times as fast on average, 4 of 590 slower by more than 3 %, the worst by 6 %; 48 shapes off the grid: 1.7
-    times, none slower.  Where the library keeps half the
-    chip idle, wide outputs of up to 48 rows, more weights too (22016 x 2048, 16 rows: 44 -> 21).
-    Beyond, 2 .. 64 rows: _FEW_LARGE, from 33 rows on for less than 12288 outputs: library -> this, 16 rows of 4096 x 4096 16.1 -> 11.6, 4096 x
-    11008 36.6 -> 21.8, 12288 x 4096 29.3 -> 23.8; 64 rows of 4096 x 14336 40.4 -> 28.7, 2048 x 8192 23.1 -> 13.9: 1.15 times on average over 96; 8
-    slower by 3 % or more, the worst 4096 x 8192 with 8 rows 16.8 -> 20.2; 64 rows of 14336 x 4096 would be 28.3 -> 30.2."""
+    2 .. 64 rows: weights up to 12.5 M elements, from 33 rows on up to 7 M or K <= 2048 (2048 x 2048, 16 rows: 11.0 -> 6.4; 64 rows:
+    11.6 -> 9.8), and where the library keeps half the chip idle, wide outputs of up to 48 rows, more weights too (22016 x 2048, 16 rows:
+    41 -> 21): 1.54 times as fast on average over 622, one slower by more than 3 % (24 rows of 1536 x 5632, 10.3 -> 11.0);
+    Beyond, 2 .. 64 rows: _FEW_LARGE, from 33 rows on for less than 12288 outputs, but for _library_streams: library -> this, 16 rows of 4096 x
+    4096 15.7 -> 10.6, 4096 x 11008 37.6 -> 21.5, 12288 x 4096 27.7 -> 22.8; 64 rows of 4096 x 14336 39.9 -> 28.5, 2048 x 8192 22.3 -> 13.8;
+    64 rows of 14336 x 4096 would be 27.4 -> 28.8.  Tables: profiles/few_rows_gemm.json, which tests/test_measured_rules.py replays."""
     if 1 < m <= GEMV_MAX_M or PP_MODE != "auto":   # (programs set both while they run: nothing of them in the cache)
         return None
     key = (m, n, k, -1)
@@ -247,7 +255,7 @@ def few_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
                 if best is None or t < best:
                     best, out = t, (cfg, sk)
     elif 1 < m <= 64 and n > 0 and n % 16 == 0 and 4_000_000 <= nk and (n + 128) * k < 1 << 30 and k % 64 == 0 and 0 < k <= 1 << 20 and (
-            m <= 32 or n < 12288) and (n, k, PP_PLAIN) not in _plan_file():
+            m <= 32 or n < 12288) and (n, k, PP_PLAIN) not in _plan_file() and not _library_streams(m, n, k):
         best = None
         for cfg, c in next(models for most, models in _FEW_LARGE if m <= most).items():
             for sk in (1, 2, 4, 8):
