@@ -393,12 +393,13 @@ def product_act(x: torch.Tensor, w: torch.Tensor, mode: int, limit: float = 0.0,
     return _k().gemm_act(x, w, mode, limit, slope, shift)
 
 
-# Few rows with more to do behind the product (gemm_few): by the most rows (config up to 8 M elements of weights, beyond; the most of them
-# where it wins with float32 outputs behind, with an activation, with a gated unit).  Measured at M = 1 .. 64 on six shapes of the first, three of the
-# others (K = 1024, 2048 and 4096), us, two launches -> one: 16 rows of 6144 x 2048 and 16 behind 15.8 -> 11.6, 12288 x 4096 and 64 36.8 -> 31.8; 32 rows
-# of that 32.8 -> 34.6; 16 rows of 8192 x 2048 with GELU 18.0 -> 12.3, 14336 x 4096 33.7 -> 33.2; gated units of 11264 x 2048 19.7 -> 18.0 (16 rows),
-# 19.6 -> 20.3 (32), of 5632 x 1024 9.1 -> 7.9 (32), 9.3 -> 9.0 (64).
-_FEW_MORE = ((16, 114, 115, 60e6, 24e6, 24e6), (32, 112, 116, 30e6, 24e6, 8e6), (64, 113, 117, 30e6, 24e6, 0))
+# Few rows with more to do behind the product (gemm_few): by the most rows (config up to 8 M elements of weights and for one row, beyond; the most of
+# them where it wins with float32 outputs behind, with an activation, with a gated unit, whose config is always the second).  Measured at nine M = 1 .. 64
+# on 25 shapes ("more behind" in profiles/few_rows_gemm.json), us, two launches -> one: 16 rows of 6144 x 2048 and 16 behind 16.2 -> 9.7, 12288 x 4096
+# and 64 33.8 -> 30.1; 32 rows of that 34.6 -> 34.1; 16 rows of 8192 x 2048 with GELU 13.5 -> 10.6, 14336 x 4096 29.7 -> 30.7; gated units of 11264 x
+# 2048 15.2 -> 16.7 (16 rows), 15.8 -> 20.0 (32), of 5632 x 1024 9.5 -> 6.9 (32).  On average 1.53, 1.40 and 1.25 times as fast
+# where they are taken, the worst 0.95: a gated unit of 4096 x 2048 8.3 -> 8.7.
+_FEW_MORE = ((16, 114, 115, 60e6, 24e6, 20e6), (32, 112, 116, 30e6, 24e6, 8e6), (64, 113, 117, 30e6, 24e6, 0))
 
 
 def _few_more(m: int, n: int, k: int, kind: int) -> int:
@@ -409,7 +410,7 @@ def _few_more(m: int, n: int, k: int, kind: int) -> int:
         if m <= most:
             if n * k > limits[kind]:
                 return 0
-            return (large if kind == 2 or n * k > 8e6 else small) - SK_BASE
+            return (large if kind == 2 or m > 1 and n * k > 8e6 else small) - SK_BASE
     return 0
 
 

@@ -32,3 +32,15 @@ def test_few_rows():
             if us is not None:
                 ratios.append(min(library, gemv or library) / us)
         assert len(ratios) == count and _mean(ratios) >= mean and _slower(ratios) <= slower and min(ratios) >= worst
+
+
+def test_few_rows_with_more_behind():
+    table = _table("few_rows_gemm.json")["more behind"]
+    taken = {"rows": [], "act": [], "glu": []}
+    for kind, m, n, k, nf, plain, two, picked, *us in table["rows"]:
+        rows = -(-(n + nf) // 32) * 32
+        assert G._few_more(m, rows, k, {"rows": 0, "act": 1, "glu": 2}[kind]) == picked, (kind, m, n, k)
+        if picked:
+            taken[kind].append(two / us[picked - 12])
+    for kind, count, mean in (("rows", 91, 1.53), ("act", 45, 1.39), ("glu", 24, 1.20)):
+        assert len(taken[kind]) == count and _mean(taken[kind]) >= mean and min(taken[kind]) >= 0.94, kind
