@@ -285,10 +285,10 @@ def product_slices(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
 
 
 # Many rows, shapes that the plan does not list: what a launch takes in us, fitted on a grid of M = 65 .. 8192, N = 512 .. 16384, K = 512 ..
-# 8192 (rms error 10 %, 18 % for 88).  88 (gemm_slab.hip): constant, per half tile of the last round, per 64-deep step of a round of
+# 8192 (rms error 8 %).  88 (gemm_slab.hip): constant, per half tile of the last round, per 64-deep step of a round of
 # 256 x 256 tiles and of the halves, per M of results, per M of weights; 19 and 32 (128 x rows by 128 and 64 W rows): constant, per round of
-# 256 tiles, per 256 tiles, per 64-deep step of these two, per M of weights.  Of all tile configs these three suffice: the pick is within
-# 1 % of the fastest of eight on average.  Both grids, here and at _MANY_SPLIT: profiles/many_rows_gemm.json.
+# 256 tiles (there is one), per 256 tiles, per 64-deep step of these two, per M of weights.  Of all tile configs these three suffice, and the pick
+# is the fastest of them.  Both grids, here and at _MANY_SPLIT: profiles/many_rows_gemm.json.
 _MANY_88 = (2.6, 1.9, 1.17, 0.55, 0.52, 0.29)
 _MANY_TILES = {19: (128, 2.9, 1.9, 1.2, 0.294, 0.15, 0.16), 32: (64, 2.7, 1.45, 0.46, 0.224, 0.083, 0.13)}
 # ... and with an activation in 88's epilogue, the gated unit and the others; the same activation as a pass of its own: constant, per M of
@@ -296,18 +296,30 @@ _MANY_TILES = {19: (128, 2.9, 1.9, 1.2, 0.294, 0.15, 0.16), 32: (64, 2.7, 1.45, 
 _MANY_ACT = {True: ((2.1, 4.7, 1.22, 0.57, 0.41, 0.16), 4.45, (2.9, 0.44)), False: ((3.3, 2.2, 1.22, 0.55, 0.51, 0.17), 0.0, (2.8, 0.39))}
 MANY_MIN = 128
 # 88 with K split over workgroups (float32 slices and a launch that sums them), one round of tiles or of halves: constant, per slab of halves, of
-# them as all CUs have one, of tiles, of them as all CUs have one, per M of all slices' results, per M of weights.  Fitted on 708 launches, M = 128 ..
+# them as all CUs have one, of tiles, of them as all CUs have one, per M of all slices' results, per M of weights.  Fitted on 696 launches, M = 128 ..
 # 3072, N = 1024 .. 6144, K = 1024 .. 14336 (rms error 8 %; the split picked takes 1 % longer than the best on average).
 _MANY_SPLIT = (11.3, 0.51, 0.13, 0.80, 0.31, 1.09, 0.088)
 
 
-def _many_slab(c, per_round: float, m: int, n: int, k: int) -> float:
+def _many_tiles(m: int, n: int) -> tuple[int, int, bool]:
+    """(whole rounds of 256 x 256 tiles, what is left for the last one, as halves?) of a launch on 256 CUs (chronos_slab.h slab_split, slab_tail)."""
     nt = -(-n // 256)
     t = -(-m // 256) * nt
-    half = 0 < t % 256 <= 128
-    if 0 < m % 256 <= 128 and 2 * (m // 256 * nt % 256) + nt <= 256:   # (chronos_slab.h slab_tail)
-        t, half = m // 256 * nt, True
-    rounds = t // 256 if half else -(-t // 256)
+    if 0 < m % 256 <= 128 and 2 * (m // 256 * nt % 256) + nt <= 256:
+        return m // 256 * nt // 256, 2 * (m // 256 * nt % 256) + nt, True
+    return (t // 256, 2 * (t % 256), True) if 0 < t % 256 <= 128 else (t // 256, t % 256, False)
+
+
+def _third_idle(m: int, n: int) -> bool:
+    """One round of tiles, or of halves, that leaves a third of the CUs idle, where the library's other tile sizes need not (of whole tiles with
+    outputs in 256s only: ragged ones cost the library as much)."""
+    rounds, last, halves = _many_tiles(m, n)
+    return rounds == 0 and last <= 170 and (halves or n % 256 == 0)
+
+
+def _many_slab(c, per_round: float, m: int, n: int, k: int) -> float:
+    rounds, last, half = _many_tiles(m, n)
+    rounds += last > 0 and not half
     return c[0] + per_round * rounds + (c[1] + c[3] * (k // 64)) * half + c[2] * rounds * (k // 64) + (c[4] * m + c[5] * k) * n * 1e-6
 
 
@@ -328,8 +340,10 @@ def _many_best(m: int, n: int, k: int) -> tuple[float, int]:
     best = (_many_slab(_MANY_88, 0.0, m, n, k), 88)
     for cfg, (bn, c0, c1, c2, c3, c4, c5) in _MANY_TILES.items():
         t = -(-m // 128) * -(-n // bn)
+        if t > 256:   # (of no shape in either table are these tiles the faster ones beyond a round)
+            continue
         steps = k // 64
-        best = min(best, (c0 + -(-t // 256) * (c1 + c3 * steps) + t / 256 * (c2 + c4 * steps) + c5 * n * k * 1e-6, cfg))
+        best = min(best, (c0 + c1 + c3 * steps + t / 256 * (c2 + c4 * steps) + c5 * n * k * 1e-6, cfg))
     return best
 
 
@@ -339,12 +353,14 @@ def _many_fits(m: int, n: int, k: int) -> bool:
 
 def many_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     """(config, split-K) of the hand-written GEMM for at least 128 rows of a shape that no plan lists, or None (the library): from 64 tiles of 128 x rows
-    by 64 W rows on, and K / 16 of them; (88, split-K) where at least 12 tiles of 256 x 256 are too few for the chip and the split's model is a
-    tenth below the others' (53 shapes of _MANY_SPLIT's grid, 1.23 times as fast as the library or the others, one 9 % slower; 768 x 4096 x 11008
-    83 -> 71 us, 1024 x 4096 x 11008 102 -> 83; fewer tiles: the library's own splits are faster).  There, on the grid of _MANY_88: 1.13 times as
-    fast as the library on average (340 shapes; 38 slower by more than 3 %, the worst by 14 %: one round that 256 x 256 tiles fill to
-    between one and two thirds), below the line 0.9 times.  A library call also costs the host 22 us, this 7.  Rows count in 128s, so that a server's
-    steps of any size find their plan again."""
+    by 64 W rows on, and K / 16 of them, but for _third_idle from K = 1024 on (768 x 5632 x 8192 84 us, here 97; 2446 x 4096 x 2048 39.5, 45.1; at K =
+    512 768 x 5632 is 15.8, here 11.3); (88, split-K) where at least 12 tiles of 256 x 256 are too few for the chip and the split's model is a
+    tenth below the others' (51 shapes of _MANY_SPLIT's grid, 1.23 times as fast as the library, one 9 % slower; 768 x 4096 x 11008
+    83 -> 71 us, 1024 x 4096 x 11008 102 -> 83; fewer tiles: the library's own splits are faster).  There, on the grid of _MANY_88: 1.15 times as
+    fast as the library on average (289 shapes; 21 slower by more than 3 %, the worst by 13 %: whole rounds at K up to 2048, where the library's
+    first loads and stores cost less, and rounds that are nearly full); at 260 shapes drawn off the grid 1.17 times (158; 14 slower, the worst 13 %);
+    below the line 0.84 times.  A library call also costs the host 22 us, this 7.  Rows count in 128s, so that a server's
+    steps of any size find their plan again.  Tables: profiles/many_rows_gemm.json, which tests/test_measured_rules.py replays."""
     if PP_MODE != "auto":
         return None
     m = -(-m // 128) * 128
@@ -356,6 +372,8 @@ def many_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     out = None
     if _many_fits(m, n, k) and tiles >= max(64, k // 16) and (n, k, PP_PLAIN) not in _plan_file():
         out = (_many_best(m, n, k)[1], 1)
+        if out[0] == 88 and k >= 1024 and _third_idle(m, n):
+            out = None
     if _many_fits(m, n, k) and -(-m // 256) * -(-n // 256) >= 12 and (n, k, PP_PLAIN) not in _plan_file():
         t, s = _many_split(m, n, k)
         if t < 0.9 * _many_best(m, n, k)[0]:
@@ -364,11 +382,18 @@ def many_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     return out
 
 
+def _many_act_pays(m: int, n: int, k: int, glu: bool) -> bool:
+    if not _many_fits(m, n, k) or glu and n % 256 or k >= 4096 and _third_idle(m, n):
+        return False
+    c, per_round, apart = _MANY_ACT[glu]
+    return _many_slab(c, per_round, m, n, k) < _many_best(m, n, k)[0] + apart[0] + apart[1] * m * n * 1e-6
+
+
 def product_act(x: torch.Tensor, w: torch.Tensor, mode: int, limit: float = 0.0, slope: float = 0.0, shift: float = 0.0) -> Optional[torch.Tensor]:
     """x @ w.T with an activation in the epilogue (mode as in torch.ops.chronos.gemm_act: 3 a gated unit of w = [gate; up], 4 squared ReLU, 5
     GELU), or None where that does not pay: with up to 64 rows by _FEW_MORE, from 128 on where the best product (many_rows_plan's or, below it, as if it were) and a pass of its own are
-    faster by their models.  On the grid of _MANY_88: gated units 1.13 times as fast (189 shapes; the worst 0.94), the others 1.16
-    (196; 0.95)."""
+    faster by their models, and not _third_idle from K = 4096 on.  On the grid of _MANY_88: gated units 1.13 times as fast (175 shapes; the worst
+    0.94), the others 1.16 (182; 0.95)."""
     m, (n, k) = x.numel() // max(1, x.shape[-1]), w.shape
     if 64 < m < MANY_MIN or PP_MODE != "auto" or x.dim() != 2 or not _plain_rows(x, w) or _registered(m, n, k):
         return None
@@ -382,10 +407,7 @@ def product_act(x: torch.Tensor, w: torch.Tensor, mode: int, limit: float = 0.0,
     key = (rows, n, k, -3 if glu else -4)
     pays = _plan_cache.get(key)
     if pays is None:
-        c, per_round, own = _MANY_ACT[glu]
-        pays = _many_fits(rows, n, k) and (not glu or n % 256 == 0)
-        pays = pays and _many_slab(c, per_round, rows, n, k) < _many_best(rows, n, k)[0] + own[0] + own[1] * rows * n * 1e-6
-        _plan_cache[key] = pays
+        pays = _plan_cache[key] = _many_act_pays(rows, n, k, glu)
     if not pays:
         return None
     from . import _k

@@ -44,3 +44,34 @@ def test_few_rows_with_more_behind():
             taken[kind].append(two / us[picked - 12])
     for kind, count, mean in (("rows", 91, 1.53), ("act", 45, 1.39), ("glu", 24, 1.20)):
         assert len(taken[kind]) == count and _mean(taken[kind]) >= mean and min(taken[kind]) >= 0.94, kind
+
+
+def _rows(table):
+    for row in table["rows"]:
+        yield dict(zip(table["columns"], row))
+
+
+def test_many_rows():
+    table = _table("many_rows_gemm.json")
+    for key, count, mean, slower, worst in (("unsplit", 289, 1.15, 21, 0.87), ("off the grid", 162, 1.16, 14, 0.86), ("split", 51, 1.23, 1, 0.91)):
+        ratios = []
+        for r in _rows(table[key]):
+            plan = G.many_rows_plan(r["m"], r["n"], r["k"]) if r["m"] >= G.MANY_MIN else None
+            if plan is None or (key == "split") != (plan[1] > 1) and key != "off the grid":
+                continue
+            us = r.get("%d,%d" % plan) if key != "off the grid" or plan[1] == 1 else r["88,split"] if r["split"] == plan[1] else None
+            if us is not None:
+                ratios.append(r["lib"] / us)
+        assert len(ratios) == count and _mean(ratios) >= mean and _slower(ratios) <= slower and min(ratios) >= worst, key
+
+
+def test_many_rows_with_an_activation():
+    taken = {True: [], False: []}
+    for r in _rows(_table("many_rows_gemm.json")["unsplit"]):
+        m, n, k = r["m"], r["n"], r["k"]
+        for glu, own, apart in ((True, "glu", "sepglu"), (False, "act", "sepact")):
+            if m >= G.MANY_MIN and r[own] and G._many_act_pays(-(-m // 128) * 128, n, k, glu):
+                plan = G.many_rows_plan(m, n, k)
+                taken[glu].append(((r["%d,1" % plan[0]] if plan and plan[1] == 1 else r["lib"]) + r[apart]) / r[own])
+    for glu, count, mean, worst in ((True, 175, 1.13, 0.94), (False, 182, 1.16, 0.95)):
+        assert len(taken[glu]) == count and _mean(taken[glu]) >= mean and min(taken[glu]) >= worst
