@@ -389,19 +389,21 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(const uint16_t* __rest
 
 // Rows per tile.  32 where experts see at most 16 tokens on average, so that a tile's padding rows cost little and the launch
 // streams weights with more of them in flight; 256, whose loop is the fastest per product, where most tiles fill (192 tokens per
-// expert) and the smaller product has a tile for a quarter of the CUs; else 128.  up: rows of an expert's first matrix.  Measured on gated
+// expert, 384 of narrow ones) and the smaller product has a tile for a quarter of the CUs; else 128.  up: rows of an expert's first matrix.  Measured on gated
 // experts, us at 32 / 128 / 256 rows: 16 experts of 2048 by 1024 with 64 tokens (4 experts each) 46 / 54 / 57, 200 tokens 51 / 57 / 58, 512
 // tokens 81 / 66 / 62, 2048 tokens 248 / 154 / 150, 8192 tokens 870 / 516 / 407; 32 experts of 4096 by 1536 with 512 tokens 329 / 282 / 323,
 // 1536 tokens 606 / 424 / 352, 8192 tokens 2640 / 1610 / 1180; 8 experts of 1024 by 512 with 1024 tokens (2 each) 39 / 35 / 39, 8192 tokens
 // 140 / 98 / 100.  (At 200 tokens of 2048, 50 items per expert, 32 rows still win by a tenth; at 128 per expert they lose by a fifth: the
 // line lies lower because a skewed choice fills more tiles.  So does 128 rows against 256: at 128 tokens per expert of 16 256 rows win by 6 %,
-// but with expert e chosen in proportion to 1 / e they lose 27 %, 84 for 66 us; from 192 on they win there too, but for 64 experts of 1024 by
-// 512, 103 for 88 where an even choice gives 77 for 84.)  All three at 55 sizes, and at 40 skewed: profiles/prompt_form_rules.json.
+// but with expert e chosen in proportion to 1 / e they lose 27 %, 84 for 66 us; from 192 on they win there too, but for experts of at most four
+// tiles across: 64 of 1024 by 512 at 192 tokens each 84 / 77, skewed 88 / 103, at 256 113 / 118, skewed 117 / 118, at 384 153 / 130, skewed 160 / 131:
+// those take 256 rows from 384 on.)  All three at 55 sizes, and at 40 skewed: profiles/prompt_form_rules.json.
 int hy_moe_tile(int items, int E, int d, int F, int up) {
     const int64_t G4 = (int64_t)1 << 32, rows = (int64_t)items + 256 * E;
     const bool fits = rows * (d > F ? d : F) * 2 < G4 && (int64_t)up * d * 2 < G4 / 2;   // 32-bit offsets
-    const int64_t big = (int64_t)(items / 256) * (up < d ? up : d) / 256;
-    return items <= 16 * E ? 32 : items < 192 * E || big < 64 || !fits ? 128 : 256;
+    const int least = up < d ? up : d;
+    const int64_t big = (int64_t)(items / 256) * least / 256;
+    return items <= 16 * E ? 32 : items < (least <= 1024 ? 384 : 192) * E || big < 64 || !fits ? 128 : 256;
 }
 int hy_moe_max_tiles(int items, int E, int tm) {
     const int n = items / tm + E;   // an expert's last tile may hold a single item

@@ -51,11 +51,11 @@ def test_experts(T, d, F, E, top, kind):
     _close(hops.moe_glu_ffn(h, idx, wt, tiled, wd, 2.0, 1.702, 1.0, BF, True), ref.moe_glu_ffn(h, idx, wt, wgu, wd, 2.0, 1.702, 1.0, BF))
 
 
-@pytest.mark.parametrize("T,d,F,E,top", [(768, 2048, 2048, 12, 3), (2051, 2176, 2048, 5, 1), (1300, 1024, 512, 32, 8),
+@pytest.mark.parametrize("T,d,F,E,top", [(768, 2048, 2048, 12, 3), (2051, 2176, 2048, 5, 1), (1300, 1024, 512, 32, 8), (1540, 1024, 512, 32, 8),
                                          (8200, 640, 512, 20, 1)])
 @pytest.mark.parametrize("kind", ["even", "skew", "empty", "nobody"])
 def test_experts_with_less_than_a_round_of_large_tiles(T, d, F, E, top, kind):
-    """From 192 items per expert on the 256-row tile takes launches that have fewer tiles than the chip has CUs."""
+    """From 192 items per expert on, 384 of narrow ones, the 256-row tile takes launches that have fewer tiles than the chip has CUs."""
     test_experts(T, d, F, E, top, kind)
 
 
