@@ -40,15 +40,16 @@ constexpr int kLGConfigs = 28;
 // gemm_lg 72-75 (32-row x tiles, after the 40-71 timing-ablation ids), 76-77 (192 W x 128 x rows: 256 tiles at
 // N = 6144, M = 1024 — one round on 256 CUs) and 78-79 (32-row x tiles with 7 / 12-stage rings: mid-M weight streams
 // are bound by the W bytes in flight per CU, so nearly all of the 160 KiB LDS holds W stages) and 80 (cfg 20's slab
-// schedule on 32x32x16 MFMAs) and 81-94 (4 waves, 128 x 128 per wave: gemm_slab.hip, or here, SwiGLU with a split-K and 91)
+// schedule on 32x32x16 MFMAs), 88 (4 waves, 128 x 128 per wave: gemm_slab.hip, or here, SwiGLU with a split-K; any other id of 81-94 but 91 names it too)
+// and 91 (its loop on 32x32x16 MFMAs)
 constexpr int kLGTinyFirst = 72, kLGTinyConfigs = 23;
 int gemm_lg_xm(int cfg);  // x rows per tile
 int gemm_lg_wn(int cfg);  // W rows per tile
-bool gemm_lg_splitk_ok(int cfg);  // false for 81-87
+bool gemm_lg_splitk_ok(int cfg);  // false for 81-87, names of 88 that never took a split
 bool gemm_lg_sliced(int cfg, int mode);  // its split-K writes float32 slices [splitk, M, N] and needs no tickets (gemm_slab.hip)
 bool gemm_lg_ablations_built();  // the timing-only ablation ids 40-71 exist (CHRONOS_GEMM_ABLATIONS build)
 bool launch_gemm_lg(int cfg, int mode, bool normp, const PPArgs& a, hipStream_t st);
-// configs 88 / 92 without split-K or (plain, resid) with it, and the hybrid decoders' epilogues (csrc/kernels/gemm_slab.hip)
+// config 88 without split-K or (plain, resid) with it, and the hybrid decoders' epilogues (csrc/kernels/gemm_slab.hip)
 bool launch_gemm_slab(int mode, bool normp, const PPArgs& a, hipStream_t st);
 // W8A8 fp8 configs of the same kernel (ring schedule, 128-deep stages; a.kts counts 128-deep units), own id space
 constexpr int kLGF8Configs = 5;

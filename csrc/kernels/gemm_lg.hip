@@ -1239,11 +1239,12 @@ void lg_launch(const PPArgs& a, hipStream_t st) {
     X(79, 64, 32, 128, 12, 2)      \
     X(80, 256, 256, 128, 2, 4, 3)  \
     X(91, 256, 256, 128, 2, 2, 6)  \
-    X(92, 256, 256, 128, 2, 2, 5)
+    X(88, 256, 256, 128, 2, 2, 5)
 
-// Ids 81 .. 94 but 91 (on 32x32x16 MFMAs) name one kernel, gemm_slab.hip and, for SwiGLU with a split-K, 92 here
+// Ids 81 .. 94 but 91 (on 32x32x16 MFMAs) name one kernel, gemm_slab.hip and, for SwiGLU with a split-K, 88 here (no plan in the tree
+// has one; gemm_pp takes it, and a tuned plan may)
 constexpr int lg_id(int cfg) {
-    return cfg < 81 || cfg > 94 || cfg == 91 ? cfg : 92;
+    return cfg < 81 || cfg > 94 || cfg == 91 ? cfg : 88;
 }
 
 template <int MODE, bool NORMP>
@@ -1251,7 +1252,7 @@ bool lg_mode(int cfg, const PPArgs& a, hipStream_t st) {
     switch (lg_id(cfg)) {
 #define LG_CASE(ID, WN_, XM_, RB_, ST_, NWX_, ...) \
     case ID:                                           \
-        if constexpr (ID == 92 && MODE != kSwiglu) return false; /* gemm_slab.hip's */ \
+        if constexpr (ID == 88 && MODE != kSwiglu) return false; /* gemm_slab.hip's */ \
         else lg_launch<WN_, XM_, RB_, ST_, MODE, NORMP, NWX_, 0, ##__VA_ARGS__>(a, st); \
         return true;
         LG_CONFIGS(LG_CASE)
@@ -1311,7 +1312,7 @@ int gemm_lg_xm(int cfg) {
         default: return 0;
     }
 }
-bool gemm_lg_sliced(int cfg, int mode) { return lg_id(cfg) == 92 && (mode == kPlain || mode == kResid); }
+bool gemm_lg_sliced(int cfg, int mode) { return lg_id(cfg) == 88 && (mode == kPlain || mode == kResid); }
 bool gemm_lg_splitk_ok(int cfg) { return cfg < 81 || cfg > 94 || cfg >= 88; }
 
 int gemm_lg_wn(int cfg) {
@@ -1372,7 +1373,7 @@ bool launch_gemm_lg_f8(int cfg, bool swiglu, const PPArgs& a, hipStream_t st) {
 
 bool launch_gemm_lg(int cfg, int mode, bool normp, const PPArgs& a, hipStream_t st) {
     if (a.M == 0) return true;
-    if (lg_id(cfg) == 92 && (a.splitk == 1 || gemm_lg_sliced(cfg, mode))) return launch_gemm_slab(mode, normp, a, st);
+    if (lg_id(cfg) == 88 && (a.splitk == 1 || gemm_lg_sliced(cfg, mode))) return launch_gemm_slab(mode, normp, a, st);
     if (mode == kResid) return normp ? false : lg_mode<kResid, false>(cfg, a, st);
     if (mode == kSwiglu) return normp ? lg_mode<kSwiglu, true>(cfg, a, st) : lg_mode<kSwiglu, false>(cfg, a, st);
     return normp ? lg_mode<kPlain, true>(cfg, a, st) : lg_mode<kPlain, false>(cfg, a, st);

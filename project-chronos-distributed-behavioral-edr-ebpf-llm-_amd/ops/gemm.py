@@ -36,8 +36,8 @@ PP_PLAIN, PP_SWIGLU, PP_RESID = 0, 1, 2
 # x rows (BM) / W rows (BN) per tile.  0-11: gemm_pp.hip (ping-pong); 12-35: gemm_lg.hip (software-pipelined: 12-19 and
 # 29-31 the ring schedule, 20-28 the 64-deep slab schedule, 32-39 mid-M weight streaming with 64 W rows, 72-75 the
 # same for M <= 32 with 32-row x tiles; 76-77 192 W rows x 128 x rows; 78-79 32-row x tiles with 7 / 12-stage rings;
-# 80 = 20 on 32x32x16 MFMAs; 81-94 the 4-wave HB slab loop, 256 x 256 tiles, LDS-staged epilogue: 88 (81-87, 89, 90 name it too),
-# 91 on 32x32x16 MFMAs, 92 (93, 94) with the first k-step in square order
+# 80 = 20 on 32x32x16 MFMAs; 88 the 4-wave slab walk, 256 x 256 tiles, LDS-staged epilogue (gemm_slab.hip), 91 its loop on 32x32x16 MFMAs.
+# Plans and programs from before may name 88 by any other id of 81-94: one kernel, but that 81-87 never took a split of K and do not now
 _PP_BM = {0: 256, 1: 128, 2: 256, 3: 128, 4: 256, 5: 128, 6: 256, 7: 128, 8: 256, 9: 128, 10: 256, 11: 128,
           12: 256, 13: 128, 14: 256, 15: 128, 16: 256, 17: 128, 18: 256, 19: 128, 20: 256, 21: 256, 22: 128, 23: 128,
           24: 256, 25: 128, 26: 256, 27: 128, 28: 128, 29: 128, 30: 256, 31: 128, 32: 128, 33: 64, 34: 128, 35: 256,
@@ -47,7 +47,7 @@ _PP_BN = {0: 256, 1: 256, 2: 128, 3: 128, 4: 256, 5: 256, 6: 128, 7: 128, 8: 256
           12: 256, 13: 256, 14: 128, 15: 128, 16: 256, 17: 256, 18: 128, 19: 128, 20: 256, 21: 256, 22: 256, 23: 128,
           24: 256, 25: 256, 26: 256, 27: 256, 28: 128, 29: 256, 30: 128, 31: 128, 32: 64, 33: 64, 34: 64, 35: 64, 36: 64, 37: 64, 38: 128, 39: 64, 72: 64, 73: 128, 74: 64, 75: 128, 76: 192, 77: 192, 78: 128, 79: 64, 80: 256,
           **{c: 256 for c in range(81, 95)}}
-HB_FIRST, HB_LAST = 81, 94  # gemm_lg.hip HB configs
+HB_FIRST, HB_LAST = 81, 94  # 88, its former ids, and 91
 HB_SPLITK = (88, 89, 90, 91, 92, 93, 94)  # ... the ids that take a split-K
 LG_FIRST = 12  # first gemm_lg.hip config: kResid partials every BN/2 columns (gemm_pp: BN/4)
 # relative per-CU MAC rate of each tile config at full occupancy (gate_up M = 1024 / 16384 sweeps, profiles/r3_gemm_pp_*,

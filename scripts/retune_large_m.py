@@ -1,9 +1,8 @@
-"""Re-measure the large-M rows of ops/gemm_plan.json with the HB configs of gemm_lg.hip (cfg 88 / 92: the 4-wave
-slab loop + LDS-staged epilogue) among the candidates, and write the
-updated plan.
+"""Re-measure the large-M rows of ops/gemm_plan.json with config 88 (gemm_slab.hip: the 4-wave slab walk + LDS-staged
+epilogue) among the candidates, and write the updated plan.
 
 For every plan key (N, K, epilogue) and every M row >= --min-m (plus --add-ms rows for keys whose table stops early):
-the row's current hand-written config (if any), cfg 88, cfg 92 and the library path of the same epilogue (hipBLASLt +
+the row's current hand-written config (if any), cfg 88 and the library path of the same epilogue (hipBLASLt +
 silu_mul for SwiGLU, + the residual add for the residual epilogue), timed interleaved in one process on random data
 with cold weights (copies rotated over >= 1 GiB).  The fastest hand-written config wins the row unless the library is
 more than --lib-margin faster (the plan's rule since round 2).  JSON lines per row go to --out-table.
@@ -20,7 +19,7 @@ import torch
 
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 
-HB_CFGS = (88, 92)  # 92: 88 with the first k-step in square order
+HB_CFGS = (88,)
 
 
 def t_us(fn, iters=8, rounds=5):
@@ -142,7 +141,7 @@ def main():
         torch.cuda.empty_cache()
     if a.out_plan:
         meta = plan.setdefault("meta", {})
-        meta["r6_hb"] = ("large-M rows re-measured with the HB configs 88 / 92 (4-wave slab loop + "
+        meta["r6_hb"] = ("large-M rows re-measured with config 88 (4-wave slab walk + "
                          "LDS-staged epilogue) among the candidates: scripts/retune_large_m.py "
                          "(profiles/r6/retune_large_m.jsonl)")
         with open(a.out_plan, "w") as fo:

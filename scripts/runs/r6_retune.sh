@@ -1,5 +1,5 @@
 #!/bin/bash
-# r6: large-M plan rows re-measured with the HB configs (88 / 89) among the candidates
+# large-M plan rows re-measured with config 88 among the candidates
 cd "${GRAFT_REPO_ROOT:-/root/repo}"
 export TMPDIR=/tmp
 O=gpurun_out/r6plan

@@ -88,13 +88,12 @@ def candidates(m, n, k, mode, keep=6):
     # tile grid under-fills the chip
     # (from M = 128: the wide-W-row tiles over the whole x panel, split-K to fill the chip — at mid-M the L2 -> LDS
     # feed, not HBM, bounds the stream, and x bytes per workgroup scale with x rows / W rows)
-    # the HB configs (88 / 92: 4-wave slab loop + staged epilogue; split-K only when the grid is small)
+    # the 4-wave slab walk (split-K only when the grid is small)
     if m >= 512:
-        for cfg in (88, 92):
-            tiles = -(-m // 256) * -(-n // 256)
-            for sk in (1, 2):
-                if G._pp_valid(cfg, n, k, mode, sk) and (sk == 1 or tiles < 128) and (cfg, sk) not in out:
-                    out.append((cfg, sk))
+        tiles = -(-m // 256) * -(-n // 256)
+        for sk in (1, 2):
+            if G._pp_valid(88, n, k, mode, sk) and (sk == 1 or tiles < 128) and (88, sk) not in out:
+                out.append((88, sk))
     if m >= 128:
         for cfg in (20, 80, 29, 30, 19, 31, 23, 76, 77, 22):
             bm, bn = G._PP_BM[cfg], G._PP_BN[cfg]
