@@ -16,7 +16,6 @@
 namespace chronos {
 void launch_hy_embed(const int32_t*, const void*, float*, uint16_t*, int, int, float, bool, hipStream_t);
 void launch_hy_low_rank_decay(const float*, const float*, const float*, float*, int, int, int, float, hipStream_t);
-void launch_hy_cast_bf16(const float*, uint16_t*, int64_t, hipStream_t);
 void launch_hy_layer_norm(const void*, bool, float*, const float*, void*, bool, int, int, float, hipStream_t);
 void launch_hy_layer_norm_slices(const float*, int, float*, const float*, uint16_t*, int, int, float, hipStream_t);
 void launch_hy_rms_norm_slices(const float*, int, float*, const float*, uint16_t*, int, int, float, float, hipStream_t);
@@ -148,14 +147,6 @@ std::tuple<Tensor, Tensor> hy_embed_both(const Tensor& ids, const Tensor& table,
     chronos::launch_hy_embed(ids.data_ptr<int32_t>(), table.data_ptr(), x.data_ptr<float>(), (uint16_t*)h.data_ptr(), (int)ids.numel(),
                              (int)table.size(1), (float)scale, f32(table), stream());
     return {x, h};
-}
-
-Tensor hy_cast_bf16(const Tensor& x) {
-    c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
-    flt(x, "cast: float32 contiguous input");
-    auto y = at::empty_like(x, x.options().dtype(at::kBFloat16));
-    chronos::launch_hy_cast_bf16(x.data_ptr<float>(), (uint16_t*)y.data_ptr(), x.numel(), stream());
-    return y;
 }
 
 Tensor hy_layer_norm(const Tensor& x, const Tensor& w, double eps, bool out_f32) {
@@ -1132,7 +1123,6 @@ Tensor hy_unrotate_gate(const Tensor& o, const Tensor& pos, const c10::optional<
 TORCH_LIBRARY_FRAGMENT(chronos, m) {
     m.def("hy_embed(Tensor ids, Tensor table, float scale=1.0) -> Tensor");
     m.def("hy_embed_both(Tensor ids, Tensor table, float scale) -> (Tensor, Tensor)");
-    m.def("hy_cast_bf16(Tensor x) -> Tensor");
     m.def("hy_layer_norm(Tensor x, Tensor w, float eps, bool out_f32) -> Tensor");
     m.def("hy_add_layer_norm(Tensor y, Tensor(a!) x, Tensor w, float eps, bool out_f32) -> Tensor");
     m.def("hy_rowdot(Tensor h, Tensor w, Tensor? bias) -> Tensor");
@@ -1214,7 +1204,6 @@ TORCH_LIBRARY_FRAGMENT(chronos, m) {
 TORCH_LIBRARY_IMPL(chronos, CUDA, m) {
     m.impl("hy_embed", &hy_embed);
     m.impl("hy_embed_both", &hy_embed_both);
-    m.impl("hy_cast_bf16", &hy_cast_bf16);
     m.impl("hy_layer_norm", &hy_layer_norm);
     m.impl("hy_add_layer_norm", &hy_add_layer_norm);
     m.impl("hy_rowdot", &hy_rowdot);

@@ -71,15 +71,6 @@ __device__ __forceinline__ f32x4 mfma_16x16x16(bf16x4 a, bf16x4 b, f32x4 c) {
 __device__ __forceinline__ void dma_1k(const void* src, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds) : "memory");
 }
-// The same through a buffer descriptor: byte voff + soff of a buffer of `bytes` bytes, which must lie inside (the range check may leave
-// out soff)
-__device__ __forceinline__ void dma_1k_buf(const void* base, uint32_t bytes, uint32_t lds, uint32_t voff, int soff) {
-    typedef int i32x4 __attribute__((ext_vector_type(4)));
-    const uint64_t b = (uint64_t)base;
-    const i32x4 r = {(int)(uint32_t)b, (int)(uint32_t)(b >> 32), (int)bytes, 0x00020000};
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %3 offen lds"
-                 ::"v"(voff), "s"(r), "s"(lds), "s"(soff) : "memory");
-}
 __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 // All but the PW pieces of each of the AHEAD newest tiles, or of the `left` that are still to come, have landed
 template <int PW, int AHEAD> __device__ __forceinline__ void dma_wait_for(int left) {

@@ -35,16 +35,6 @@ __global__ void __launch_bounds__(256) embed_kernel(const int32_t* __restrict__ 
     }
 }
 
-__global__ void __launch_bounds__(256) cast_bf16_kernel(const float* __restrict__ x, uint16_t* __restrict__ y, int64_t n) {
-    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-    if (i + 3 < n) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(x + i);
-        *reinterpret_cast<u16x4*>(y + i) = u16x4{f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
-    } else {
-        for (int64_t j = i; j < n; ++j) y[j] = f2bf(x[j]);
-    }
-}
-
 // y [rows, d] (activation type, or float for the plain norm of the stream itself) -> float statistics in two passes
 // (mean, then the mean of squared deviations), then
 //   ADD:   x[row] += (y - mean) * rstd * w;   h[row] = T(x[row])   (h == nullptr: not written)
@@ -359,11 +349,6 @@ void launch_hy_embed(const int32_t* ids, const void* table, float* x, uint16_t* 
     if (T == 0) return;
     if (f32) hy::embed_kernel<float><<<T, 256, 0, s>>>(ids, (const float*)table, x, h, d, scale);
     else hy::embed_kernel<uint16_t><<<T, 256, 0, s>>>(ids, (const uint16_t*)table, x, h, d, scale);
-}
-void launch_hy_cast_bf16(const float* x, uint16_t* y, int64_t n, hipStream_t s) {
-    if (n == 0) return;
-    const int64_t blocks = (n + 1023) / 1024;
-    hy::cast_bf16_kernel<<<(unsigned)blocks, 256, 0, s>>>(x, y, n);
 }
 // y_f32: the input is float (the plain norm of the stream); out_f32: h is float.  x == nullptr: plain norm.
 void launch_hy_layer_norm(const void* y, bool y_f32, float* x, const float* w, void* h, bool out_f32, int rows, int d,

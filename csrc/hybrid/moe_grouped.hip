@@ -171,7 +171,6 @@ __device__ __forceinline__ void moe_store(const f32x4 (&acc)[NS][NM], uint16_t* 
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             const int row = n0 + 16 * s;   // first weight row of the block
-            if (row >= N) break;           // (the last tile of a 256-row launch may be half)
             u16x4 o;
             if constexpr (ACT == kActGlu) {
                 // every 64 rows: blocks 0 and 1 are gate rows, 2 and 3 the up rows of the same outputs
