@@ -39,15 +39,45 @@ def test_rows_behind(m, n0, nf, k, with_bias):
     assert torch.equal(y, y2) and torch.equal(yf, yf2)
 
 
+_CONFIGS = ((12, (1, 17, 31, 32)), (13, (1, 33, 63, 64)), (14, (1, 15, 16)), (15, (1, 15, 16)), (16, (1, 17, 31, 32)), (17, (1, 33, 63, 64)))
+
+
+# (gated units take configs of 32 weight rows: a pair of gate and up rows in a workgroup)
+@pytest.mark.parametrize("cfg,ms,mode", [(cfg, ms, mode) for cfg, ms in _CONFIGS for mode in (3, 4, 5) if mode > 3 or cfg >= 15])
+@pytest.mark.parametrize("n,k", [(32, 64), (96, 192), (2080, 576), (4096, 1024)])
+def test_every_activation_of_every_config(cfg, ms, mode, n, k):
+    """gemm_few's epilogues element by element.  float32 sums move a value by less than 2e-5 (sums of products of variance 1 / K, activations of
+    slope below 3 there, the square's up to 2 |h|), and there is one rounding to bfloat16: 2^-8 |y| + 2e-5 max(1, |h|)."""
+    from chronos import ops
+
+    ops.load()
+    g = _g(cfg + mode + n + k)
+    w = (torch.randn(n, k, device=DEV, generator=g) * k ** -0.5).to(BF)
+    F = n // 2
+    for m in ms:
+        x = torch.randn(m, k, device=DEV, generator=g).to(BF)
+        h = x.double() @ w.double().t()
+        for limit, slope, shift in ((float("inf"), 1.0, 0.0), (0.75, 1.702, 1.0)) if mode == 3 else ((0.0, 0.0, 0.0),):
+            y, rows = torch.ops.chronos.gemm_few(x, w, cfg, mode, 0, 0, None, limit, slope, shift)
+            a, u = h[:, :F].clamp(max=limit), h[:, F:].clamp(-limit, limit)
+            want = a * torch.sigmoid(slope * a) * (u + shift) if mode == 3 else h.relu() ** 2 if mode == 4 else torch.nn.functional.gelu(h)
+            size = torch.maximum(h[:, :F].abs(), h[:, F:].abs()) if mode == 3 else h.abs()
+            assert y.dtype == BF and y.shape == want.shape
+            assert ((y.double() - want).abs() <= want.abs() * 2 ** -8 + 2e-5 * size.clamp(min=1)).all(), (m, limit)
+
+
 @pytest.mark.parametrize("m", [1, 16, 17, 32, 33, 64])
 @pytest.mark.parametrize("n,k", [(64, 64), (1056, 576), (5632, 1024), (8192, 2048)])
 def test_activations(m, n, k):
-    from chronos.ops import hybrid as H
+    from chronos.ops import gemm as G, hybrid as H
 
     g = _g(m + n + k)
     x, w = torch.randn(m, k, device=DEV, generator=g).to(BF), (torch.randn(n, k, device=DEV, generator=g) * k ** -0.5).to(BF)
     h = x.double() @ w.double().t()
     F = n // 2
+    # in the product's epilogue, but for gated units of many rows or weights, which stay a launch of their own
+    assert G.product_act(x, w, 4) is not None and G.product_act(x, w, 5) is not None
+    assert (G.product_act(x, w, 3) is not None) == (m <= 16 or m <= 32 and n * k < 8e6)
     for limit, slope, shift in ((float("inf"), 1.0, 0.0), (0.75, 1.702, 1.0)):
         a, u = h[:, :F].clamp(max=limit), h[:, F:].clamp(-limit, limit)
         want = a * torch.sigmoid(slope * a) * (u + shift)

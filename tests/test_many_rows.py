@@ -101,12 +101,16 @@ def test_other_forms_keep_their_way():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,n,k", [(100, 512, 128), (300, 512, 4096), (2446, 5632, 1024), (4100, 8192, 64), (1000, 768, 320)])
-def test_activations(m, n, k):
-    """Either way of the rule: in the product's epilogue, or a pass of its own on the rounded product."""
+@pytest.mark.parametrize("m,n,k,unit,other", [(100, 512, 128, False, False), (300, 512, 4096, False, False), (2446, 5632, 1024, True, True),
+                                              (4100, 8192, 64, True, True), (1000, 768, 320, False, True)])
+def test_activations(m, n, k, unit, other):
+    """Either way of the rule: in the product's epilogue (unit: the gated unit's, other: the others'), or a pass of its own on the rounded
+    product.  The epilogue's elements one by one: test_gemm_slab_gpu.py."""
     from chronos.ops import hybrid as H
 
     x, w = _operands(m, n, k)
+    assert (G.product_act(x, w, 3) is not None) == unit
+    assert (G.product_act(x, w, 4) is not None) == other and (G.product_act(x, w, 5) is not None) == other
     h = x.double() @ w.double().t()
     F = n // 2
     for limit, slope, shift in ((float("inf"), 1.0, 0.0), (0.75, 1.702, 1.0)):
