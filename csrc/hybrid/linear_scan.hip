@@ -65,15 +65,6 @@ __global__ void __launch_bounds__(256) short_conv_vec_kernel(const uint16_t* __r
     if (c >= C) return;
     const int tb = blockIdx.x / gx * TK;
     int te = min(tb + TK, T);
-    uint16_t* last = nullptr;   // one_each: where the history behind the sequence's last token goes
-    if (one_each) {   // (TK is 1)  a sequence that does bring more tokens is walked by its first one's thread: history that is read and
-        const int b = tok_seq[tb], t0 = q_start[b], t1 = min(q_start[b + 1], T);   // written in one pass stays with one thread
-        if (tb > t0 && tb < t1) return;
-        if (tb == t0 && t1 > t0) {
-            te = t1;
-            last = hist + (int64_t)slots[b] * (K - 1) * C + c;
-        }
-    }
     float wf[8][K], bv[8], in[K][8];   // in[i]: the input K - 1 - i tokens back
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -81,13 +72,22 @@ __global__ void __launch_bounds__(256) short_conv_vec_kernel(const uint16_t* __r
 #pragma unroll
         for (int i = 0; i < K; ++i) wf[e][i] = w[(c + e) * K + i];
     }
+    uint16_t* last = nullptr;   // one_each: where the history behind the sequence's last token goes
     int seq = -1;
     for (int t = tb; t < te; ++t) {
         const int b = tok_seq[t];
         if (b != seq) {   // the block's first token, or another sequence's: the inputs in front of it
             seq = b;
-            const int t0 = q_start[b];
-            const uint16_t* const hrow = pos0[b] > 0 ? hist + (int64_t)slots[b] * (K - 1) * C + c : nullptr;
+            const int t0 = q_start[b], t1 = q_start[b + 1], p0 = pos0[b], slot = slots[b];
+            uint16_t* const row = hist + (int64_t)slot * (K - 1) * C + c;
+            const uint16_t* const hrow = p0 > 0 ? row : nullptr;
+            if (one_each) {   // (TK is 1)  a sequence that does bring more tokens is walked by its first one's thread: history that is
+                if (t > t0 && t < t1) return;   // read and written in one pass stays with one thread
+                if (t == t0 && t < t1) {
+                    te = min(t1, T);
+                    last = row;
+                }
+            }
 #pragma unroll
             for (int i = 1; i < K; ++i) {
                 const int s = t - K + i;   // lands in in[i - 1] below
