@@ -311,10 +311,11 @@ def _many_tiles(m: int, n: int) -> tuple[int, int, bool]:
 
 
 def _third_idle(m: int, n: int) -> bool:
-    """One round of tiles, or of halves, that leaves a third of the CUs idle, where the library's other tile sizes need not (of whole tiles with
-    outputs in 256s only: ragged ones cost the library as much)."""
+    """One round of tiles, or of halves, that leaves a third of the CUs idle, where the library's other tile sizes need not.  Of whole tiles only
+    where there are more outputs than rows, in 256s: ragged outputs cost the library as much, and tall products are no faster there (8192 x
+    1280 x 1024, 160 tiles: 28.5 us, here 27.8)."""
     rounds, last, halves = _many_tiles(m, n)
-    return rounds == 0 and last <= 170 and (halves or n % 256 == 0)
+    return rounds == 0 and last <= 170 and (halves or n % 256 == 0 and n > m)
 
 
 def _many_slab(c, per_round: float, m: int, n: int, k: int) -> float:
@@ -357,7 +358,7 @@ def many_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     512 768 x 5632 is 15.8, here 11.3); (88, split-K) where at least 12 tiles of 256 x 256 are too few for the chip and the split's model is a
     tenth below the others' (51 shapes of _MANY_SPLIT's grid, 1.23 times as fast as the library, one 9 % slower; 768 x 4096 x 11008
     83 -> 71 us, 1024 x 4096 x 11008 102 -> 83; fewer tiles: the library's own splits are faster).  There, on the grid of _MANY_88: 1.15 times as
-    fast as the library on average (289 shapes; 21 slower by more than 3 %, the worst by 13 %: whole rounds at K up to 2048, where the library's
+    fast as the library on average (292 shapes; 22 slower by more than 3 %, the worst by 13 %: whole rounds at K up to 2048, where the library's
     first loads and stores cost less, and rounds that are nearly full); at 260 shapes drawn off the grid 1.17 times (158; 14 slower, the worst 13 %);
     below the line 0.84 times.  A library call also costs the host 22 us, this 7.  Rows count in 128s, so that a server's
     steps of any size find their plan again.  Tables: profiles/many_rows_gemm.json, which tests/test_measured_rules.py replays."""
@@ -392,8 +393,8 @@ def _many_act_pays(m: int, n: int, k: int, glu: bool) -> bool:
 def product_act(x: torch.Tensor, w: torch.Tensor, mode: int, limit: float = 0.0, slope: float = 0.0, shift: float = 0.0) -> Optional[torch.Tensor]:
     """x @ w.T with an activation in the epilogue (mode as in torch.ops.chronos.gemm_act: 3 a gated unit of w = [gate; up], 4 squared ReLU, 5
     GELU), or None where that does not pay: with up to 64 rows by _FEW_MORE, from 128 on where the best product (many_rows_plan's or, below it, as if it were) and a pass of its own are
-    faster by their models, and not _third_idle from K = 4096 on.  On the grid of _MANY_88: gated units 1.13 times as fast (175 shapes; the worst
-    0.94), the others 1.16 (182; 0.95)."""
+    faster by their models, and not _third_idle from K = 4096 on.  On the grid of _MANY_88: gated units 1.13 times as fast (176 shapes; the worst
+    0.94), the others 1.16 (184; 0.95)."""
     m, (n, k) = x.numel() // max(1, x.shape[-1]), w.shape
     if 64 < m < MANY_MIN or PP_MODE != "auto" or x.dim() != 2 or not _plain_rows(x, w) or _registered(m, n, k):
         return None

@@ -53,7 +53,7 @@ def _rows(table):
 
 def test_many_rows():
     table = _table("many_rows_gemm.json")
-    for key, count, mean, slower, worst in (("unsplit", 289, 1.15, 21, 0.87), ("off the grid", 162, 1.16, 14, 0.86), ("split", 51, 1.23, 1, 0.91)):
+    for key, count, mean, slower, worst in (("unsplit", 292, 1.14, 22, 0.87), ("off the grid", 162, 1.16, 14, 0.86), ("split", 51, 1.23, 1, 0.91)):
         ratios = []
         for r in _rows(table[key]):
             plan = G.many_rows_plan(r["m"], r["n"], r["k"]) if r["m"] >= G.MANY_MIN else None
@@ -73,5 +73,5 @@ def test_many_rows_with_an_activation():
             if m >= G.MANY_MIN and r[own] and G._many_act_pays(-(-m // 128) * 128, n, k, glu):
                 plan = G.many_rows_plan(m, n, k)
                 taken[glu].append(((r["%d,1" % plan[0]] if plan and plan[1] == 1 else r["lib"]) + r[apart]) / r[own])
-    for glu, count, mean, worst in ((True, 175, 1.13, 0.94), (False, 182, 1.16, 0.95)):
+    for glu, count, mean, worst in ((True, 176, 1.13, 0.94), (False, 184, 1.16, 0.95)):
         assert len(taken[glu]) == count and _mean(taken[glu]) >= mean and min(taken[glu]) >= worst
