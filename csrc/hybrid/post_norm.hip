@@ -204,7 +204,7 @@ __global__ void __launch_bounds__(256) decay_pow_kernel(float* __restrict__ z, i
 // Decays of a gated linear recurrence from their low-rank logits, in one pass: out[t, c] = sigmoid(b[c] + sum_r a[t, r] w[r, c])^p, float
 // throughout, the sum in the order of r.  A thread takes 4 channels of TT tokens, so that w is read once for them; the tokens' a is
 // the same in all lanes.  Bound by writing out (8192 x 4096
-// of rank 16: 28 us, 4.8 TB/s); a library product, the copy of its bias and decay_pow took 120 there, 15 for 2446 x 512 (8 so), 16 for a single
+// of rank 16: 28 us, 4.8 TB/s, 38 where launches follow each other); a library product, the copy of its bias and decay_pow took 120 there, 15 for 2446 x 512 (8 so), 16 for a single
 // token (6).
 template <int TT, bool POW4>
 __global__ void __launch_bounds__(256) low_rank_decay_kernel(const float* __restrict__ a, const float* __restrict__ w,

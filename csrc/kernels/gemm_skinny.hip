@@ -370,12 +370,12 @@ void launch_cfg(const PPArgs& a, hipStream_t st) {
 }
 
 // configs {RT (W tiles of 16 rows per workgroup), MT (x tiles: M <= 16 MT), D (ring depth in 64-k units), NW (waves
-// splitting K inside the workgroup; K % (64 NW splitk) == 0, from kSkinnyUneven on K % 64 == 0: the shares then differ by a unit.  At a few MB of weights what bounds a launch is latency, so these run 8 short waves: 2048 x 2048 with 16 rows 6.0 us (the
-// library 11.0), 1024 x 2816 with one row 5.7 (8.6).  Their split across workgroups writes [split, M, N] sums that a second launch adds
+// splitting K inside the workgroup; K % (64 NW splitk) == 0, from kSkinnyUneven on K % 64 == 0: the shares then differ by a unit.  At a few MB of weights what bounds a launch is latency, so these run 8 short waves: 2048 x 2048 with 16 rows 6.4 us (the
+// library 11.0), 1024 x 2816 with one row 5.5 (11.1).  Their split across workgroups writes [split, M, N] sums that a second launch adds
 // up: 2.0-2.3 us, as much as tickets cost, with nothing kept between calls.  16 and 17 are for the products with more to
 // do behind them (gemm_few): activations, which a launch of its own costs 2.8 to 3.5 us, and float32 outputs of a few rows behind the others',
-// 3.6 to 7.8 as a product of their own.  One row, us: 3072 x 1024 and 8 rows 4.7 + 3.8 -> 4.8; gated unit of 5632 x 1024 6.8 + 2.8 -> 6.1; 64 rows:
-// 6720 x 4096 and 32 rows 19.1 + 7.5 -> 23.4; GELU of 8192 x 2048 15.3 + 3.5 -> 15.5)}
+// 3.6 to 7.8 as a product of their own.  Two launches -> one, us, one row: 3072 x 1024 and 8 rows 6.3 -> 4.0; gated unit of 5632 x 1024 7.9 -> 6.2; 64
+// rows: 6720 x 4096 and 32 rows 28.7 -> 22.7; GELU of 8192 x 2048 16.7 -> 13.8)}
 #define SK_CONFIGS(X)  \
     X(0, 1, 1, 4, 16)  \
     X(1, 2, 1, 4, 8)   \
