@@ -310,12 +310,13 @@ def _many_tiles(m: int, n: int) -> tuple[int, int, bool]:
     return (t // 256, 2 * (t % 256), True) if 0 < t % 256 <= 128 else (t // 256, t % 256, False)
 
 
-def _third_idle(m: int, n: int) -> bool:
-    """One round of tiles, or of halves, that leaves a third of the CUs idle, where the library's other tile sizes need not.  Of whole tiles only
-    where there are more outputs than rows, in 256s: ragged outputs cost the library as much, and tall products are no faster there (8192 x
-    1280 x 1024, 160 tiles: 28.5 us, here 27.8)."""
+def _third_idle(m: int, n: int, k: int) -> bool:
+    """One long round of tiles, or of halves, that leaves a third of the CUs idle, where the library's other tile sizes need not: halves beyond
+    K = 2048 (768 x 5632 x 8192 84 us, here 97; at K = 1024 and 2048 the two are level, and a library call costs the host more), whole tiles from 2048 on
+    where there are more outputs than rows, in 256s (2446 x 4096 x 2048 39.5, here 45.1; ragged outputs cost the library as much, and tall products
+    are hardly faster there: 8192 x 1280 x 2048 44.0 and 45.3)."""
     rounds, last, halves = _many_tiles(m, n)
-    return rounds == 0 and last <= 170 and (halves or n % 256 == 0 and n > m)
+    return rounds == 0 and last <= 170 and (halves and k > 2048 or not halves and n % 256 == 0 and n > m and k >= 2048)
 
 
 def _many_slab(c, per_round: float, m: int, n: int, k: int) -> float:
@@ -354,12 +355,11 @@ def _many_fits(m: int, n: int, k: int) -> bool:
 
 def many_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     """(config, split-K) of the hand-written GEMM for at least 128 rows of a shape that no plan lists, or None (the library): from 64 tiles of 128 x rows
-    by 64 W rows on, and K / 16 of them, but for _third_idle from K = 1024 on (768 x 5632 x 8192 84 us, here 97; 2446 x 4096 x 2048 39.5, 45.1; at K =
-    512 768 x 5632 is 15.8, here 11.3); (88, split-K) where at least 12 tiles of 256 x 256 are too few for the chip and the split's model is a
+    by 64 W rows on, and K / 16 of them, but for _third_idle; (88, split-K) where at least 12 tiles of 256 x 256 are too few for the chip and the split's model is a
     tenth below the others' (51 shapes of _MANY_SPLIT's grid, 1.23 times as fast as the library, one 9 % slower; 768 x 4096 x 11008
-    83 -> 71 us, 1024 x 4096 x 11008 102 -> 83; fewer tiles: the library's own splits are faster).  There, on the grid of _MANY_88: 1.15 times as
-    fast as the library on average (292 shapes; 22 slower by more than 3 %, the worst by 13 %: whole rounds at K up to 2048, where the library's
-    first loads and stores cost less, and rounds that are nearly full); at 260 shapes drawn off the grid 1.17 times (158; 14 slower, the worst 13 %);
+    83 -> 71 us, 1024 x 4096 x 11008 102 -> 83; fewer tiles: the library's own splits are faster).  There, on the grid of _MANY_88: 1.14 times as
+    fast as the library on average (302 shapes; 25 slower by more than 3 %, the worst by 14 %: whole or part rounds at K up to 2048, where the library's
+    first loads and stores cost less, and rounds that are nearly full); at 260 shapes drawn off the grid 1.16 times (162; 16 slower, the worst 13 %);
     below the line 0.84 times.  A library call also costs the host 22 us, this 7.  Rows count in 128s, so that a server's
     steps of any size find their plan again.  Tables: profiles/many_rows_gemm.json, which tests/test_measured_rules.py replays."""
     if PP_MODE != "auto":
@@ -373,7 +373,7 @@ def many_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     out = None
     if _many_fits(m, n, k) and tiles >= max(64, k // 16) and (n, k, PP_PLAIN) not in _plan_file():
         out = (_many_best(m, n, k)[1], 1)
-        if out[0] == 88 and k >= 1024 and _third_idle(m, n):
+        if out[0] == 88 and _third_idle(m, n, k):
             out = None
     if _many_fits(m, n, k) and -(-m // 256) * -(-n // 256) >= 12 and (n, k, PP_PLAIN) not in _plan_file():
         t, s = _many_split(m, n, k)
@@ -384,7 +384,7 @@ def many_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
 
 
 def _many_act_pays(m: int, n: int, k: int, glu: bool) -> bool:
-    if not _many_fits(m, n, k) or glu and n % 256 or k >= 4096 and _third_idle(m, n):
+    if not _many_fits(m, n, k) or glu and n % 256:
         return False
     c, per_round, apart = _MANY_ACT[glu]
     return _many_slab(c, per_round, m, n, k) < _many_best(m, n, k)[0] + apart[0] + apart[1] * m * n * 1e-6
@@ -392,9 +392,10 @@ def _many_act_pays(m: int, n: int, k: int, glu: bool) -> bool:
 
 def product_act(x: torch.Tensor, w: torch.Tensor, mode: int, limit: float = 0.0, slope: float = 0.0, shift: float = 0.0) -> Optional[torch.Tensor]:
     """x @ w.T with an activation in the epilogue (mode as in torch.ops.chronos.gemm_act: 3 a gated unit of w = [gate; up], 4 squared ReLU, 5
-    GELU), or None where that does not pay: with up to 64 rows by _FEW_MORE, from 128 on where the best product (many_rows_plan's or, below it, as if it were) and a pass of its own are
-    faster by their models, and not _third_idle from K = 4096 on.  On the grid of _MANY_88: gated units 1.13 times as fast (176 shapes; the worst
-    0.94), the others 1.16 (184; 0.95)."""
+    GELU), or None where that does not pay: with up to 64 rows by _FEW_MORE, from 128 on where the best product (many_rows_plan's or, below it,
+    as if it were) and a pass of its own are faster by their models.  On the grid of _MANY_88, against the faster of the library and this product with
+    its pass: gated units 1.12 times as fast (188 shapes; the worst 0.92), the others 1.15 (196; 0.90).  Both worst are long rounds that leave a
+    third of the CUs idle (_third_idle); they stay, because the pass reads a rounded product: a step with it is further from float64 (0.0076 for 0.0067)."""
     m, (n, k) = x.numel() // max(1, x.shape[-1]), w.shape
     if 64 < m < MANY_MIN or PP_MODE != "auto" or x.dim() != 2 or not _plain_rows(x, w) or _registered(m, n, k):
         return None
@@ -416,13 +417,14 @@ def product_act(x: torch.Tensor, w: torch.Tensor, mode: int, limit: float = 0.0,
     return _k().gemm_act(x, w, mode, limit, slope, shift)
 
 
-# Few rows with more to do behind the product (gemm_few): by the most rows (config up to 8 M elements of weights and for one row, beyond; the most of
+# Few rows with more to do behind the product (gemm_few): by the most rows (config up to 8 M elements of weights and for one row from 30 M on, beyond; the most of
 # them where it wins with float32 outputs behind, with an activation, with a gated unit, whose config is always the second).  Measured at nine M = 1 .. 64
 # on 25 shapes ("more behind" in profiles/few_rows_gemm.json), us, two launches -> one: 16 rows of 6144 x 2048 and 16 behind 16.2 -> 9.7, 12288 x 4096
 # and 64 33.8 -> 30.1; 32 rows of that 34.6 -> 34.1; 16 rows of 8192 x 2048 with GELU 13.5 -> 10.6, 14336 x 4096 29.7 -> 30.7; gated units of 11264 x
-# 2048 15.2 -> 16.7 (16 rows), 15.8 -> 20.0 (32), of 5632 x 1024 9.5 -> 6.9 (32).  On average 1.53, 1.40 and 1.25 times as fast
-# where they are taken, the worst 0.95: a gated unit of 4096 x 2048 8.3 -> 8.7.
-_FEW_MORE = ((16, 114, 115, 60e6, 24e6, 20e6), (32, 112, 116, 30e6, 24e6, 8e6), (64, 113, 117, 30e6, 24e6, 0))
+# 2048 15.2 -> 16.7 (16 rows), 15.8 -> 20.0 (32), of 5632 x 1024 9.5 -> 6.9 (32).  On average 1.53, 1.40 and 1.20 times as fast
+# where they are taken, the worst 0.91, those 16 rows: they stay, because the pass of its own reads a rounded product (a step's error against float64
+# 0.0042, 0.0046 with it).
+_FEW_MORE = ((16, 114, 115, 60e6, 24e6, 24e6), (32, 112, 116, 30e6, 24e6, 8e6), (64, 113, 117, 30e6, 24e6, 0))
 
 
 def _few_more(m: int, n: int, k: int, kind: int) -> int:
@@ -433,7 +435,7 @@ def _few_more(m: int, n: int, k: int, kind: int) -> int:
         if m <= most:
             if n * k > limits[kind]:
                 return 0
-            return (large if kind == 2 or m > 1 and n * k > 8e6 else small) - SK_BASE
+            return (large if kind == 2 or 8e6 < n * k and (m > 1 or n * k < 30e6) else small) - SK_BASE
     return 0
 
 

