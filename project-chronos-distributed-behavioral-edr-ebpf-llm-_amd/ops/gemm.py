@@ -483,7 +483,7 @@ def register(pred: Callable[[int, int, int], bool], fn: Callable[[torch.Tensor, 
 
 def _registered(m: int, n: int, k: int) -> bool:
     """Is a kernel registered for this product?  Then linear() calls it, and no launch that takes the product along with something else."""
-    return any(pred(m, n, k) for pred, _ in _custom)
+    return bool(_custom) and any(pred(m, n, k) for pred, _ in _custom)
 
 
 @dataclass
