@@ -188,3 +188,26 @@ def test_large_weights_split(m, n, k):
         for sk in (2, 4, 8):
             if k // 64 % sk == 0:
                 _check(torch.ops.chronos.gemm_split(x, w, cfg, sk), want)
+
+
+@pytest.mark.parametrize("m", [2, 16, 32])
+@pytest.mark.parametrize("n,k", [(4096, 8192), (8192, 4096), (5120, 5120), (8192, 8192)])
+def test_library_products_replay(m, n, k):
+    """Shapes that few_rows_plan leaves to the library (_library_streams): a captured one gives the eager bits at every replay, with other work between."""
+    from chronos import ops
+    from chronos.ops import gemm as G
+
+    assert G.few_rows_plan(m, n, k) is None
+    g = _g(m + n + k)
+    x, w = torch.randn(m, k, device=DEV, generator=g).to(BF), (torch.randn(n, k, device=DEV, generator=g) * k ** -0.5).to(BF)
+    want = ops.linear(x, w)
+    _check(want, x.double() @ w.double().t())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = ops.linear(x, w)
+    for _ in range(4):
+        y.fill_(float("nan"))
+        torch.randn(1 << 20, device=DEV).sum().item()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
