@@ -14,7 +14,11 @@
 #include <tuple>
 
 namespace chronos {
-void launch_hy_embed(const int32_t*, const void*, float*, uint16_t*, int, int, float, bool, hipStream_t);
+void launch_hy_embed(const int32_t*, const void*, float*, uint16_t*, int, int, float, bool, const int32_t*, const int32_t*, int32_t*, int,
+                     hipStream_t);
+bool hy_rows_norm_ok(int);
+void launch_hy_layer_norm_rows(const float*, const int64_t*, int, const float*, void*, bool, int, int, float, hipStream_t);
+void launch_hy_rms_norm_rows(const float*, const int64_t*, int, const float*, void*, bool, int, int, float, hipStream_t);
 void launch_hy_low_rank_decay(const float*, const float*, const float*, float*, int, int, int, float, hipStream_t);
 void launch_hy_layer_norm(const void*, bool, float*, const float*, void*, bool, int, int, float, hipStream_t);
 void launch_hy_layer_norm_slices(const float*, int, float*, const float*, uint16_t*, int, int, float, hipStream_t);
@@ -72,8 +76,9 @@ void launch_hy_window_prep(void*, int, int, int, int, int, const void*, const fl
 void launch_hy_pool_blocks(const void*, const void*, void*, void*, const int32_t*, int, const int32_t*, const int32_t*, int,
                            int, int, int, int, int, int, bool, hipStream_t);
 void launch_hy_sandwich_join(const void*, const void*, float*, const float*, const float*, const float*, const float*,
-                             void*, int, int, int, float, bool, bool, hipStream_t);
+                             void*, int, int, int, float, bool, bool, const int64_t*, int, hipStream_t);
 bool hy_sandwich_groups_ok(int, int);
+bool hy_sandwich_rows_ok(int, int);
 void launch_hy_rotate_qk(void*, int, int, int, int, int, int, int, const float*, const int32_t*, float, float, int, bool,
                          hipStream_t);
 void launch_hy_unrotate_gate(const void*, const int32_t*, const float*, const void*, int, int, void*, int, int, int, bool,
@@ -133,7 +138,7 @@ Tensor hy_embed(const Tensor& ids, const Tensor& table, double scale) {
     need(is_act(table) && table.dim() == 2 && table.is_contiguous(), "embed: table [V, d] bf16 or f32");
     auto x = at::empty({ids.numel(), table.size(1)}, table.options().dtype(at::kFloat));
     chronos::launch_hy_embed(ids.data_ptr<int32_t>(), table.data_ptr(), x.data_ptr<float>(), nullptr, (int)ids.numel(),
-                             (int)table.size(1), (float)scale, f32(table), stream());
+                             (int)table.size(1), (float)scale, f32(table), nullptr, nullptr, nullptr, 0, stream());
     return x;
 }
 
@@ -145,15 +150,49 @@ std::tuple<Tensor, Tensor> hy_embed_both(const Tensor& ids, const Tensor& table,
     auto x = at::empty({ids.numel(), table.size(1)}, table.options().dtype(at::kFloat));
     auto h = at::empty_like(x, x.options().dtype(at::kBFloat16));
     chronos::launch_hy_embed(ids.data_ptr<int32_t>(), table.data_ptr(), x.data_ptr<float>(), (uint16_t*)h.data_ptr(), (int)ids.numel(),
-                             (int)table.size(1), (float)scale, f32(table), stream());
+                             (int)table.size(1), (float)scale, f32(table), nullptr, nullptr, nullptr, 0, stream());
     return {x, h};
 }
 
-Tensor hy_layer_norm(const Tensor& x, const Tensor& w, double eps, bool out_f32) {
+// The same (the bfloat16 rows with `both`) with pos0 [B] = pos at every sequence's first token; at least one token.
+std::tuple<Tensor, Tensor, Tensor> hy_embed_start(const Tensor& ids, const Tensor& table, double scale, bool both, const Tensor& pos,
+                                                  const Tensor& q_start) {
+    c10::hip::HIPGuardMasqueradingAsCUDA g(table.device());
+    i32(ids, "embed: ids must be contiguous int32");
+    i32(pos, "embed: pos must be contiguous int32");
+    i32(q_start, "embed: q_start must be contiguous int32");
+    need(is_act(table) && table.dim() == 2 && table.is_contiguous(), "embed: table [V, d] bf16 or f32");
+    need(ids.numel() >= 1 && pos.numel() == ids.numel() && q_start.numel() >= 1, "embed: a position per token, at least one token, q_start [B + 1]");
+    auto x = at::empty({ids.numel(), table.size(1)}, table.options().dtype(at::kFloat));
+    Tensor h = both ? at::empty_like(x, x.options().dtype(at::kBFloat16)) : at::empty({0}, x.options().dtype(at::kBFloat16));
+    auto pos0 = at::empty({q_start.numel() - 1}, pos.options());
+    chronos::launch_hy_embed(ids.data_ptr<int32_t>(), table.data_ptr(), x.data_ptr<float>(), both ? (uint16_t*)h.data_ptr() : nullptr, (int)ids.numel(),
+                             (int)table.size(1), (float)scale, f32(table), pos.data_ptr<int32_t>(), q_start.data_ptr<int32_t>(),
+                             pos0.data_ptr<int32_t>(), (int)pos0.numel(), stream());
+    return {x, h, pos0};
+}
+
+// rows to norm: indices into x's rows, as the kernels take them
+static Tensor pick_rows(const Tensor& rows, const Tensor& x) {
+    need((rows.scalar_type() == at::kLong || rows.scalar_type() == at::kInt) && rows.dim() <= 1 && rows.device() == x.device(), "norm: rows are indices on x's device");
+    need(x.size(0) > 0 || rows.numel() == 0, "norm: rows of a stream without tokens");
+    return rows.reshape({-1}).to(at::kLong).contiguous();
+}
+
+Tensor hy_layer_norm(const Tensor& x, const Tensor& w, double eps, bool out_f32, const c10::optional<Tensor>& rows) {
     c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
     flt(x, "layer_norm: float32 rows");
     flt(w, "layer_norm: float32 weight");
     need(x.dim() == 2 && w.numel() == x.size(1), "layer_norm: weight size");
+    if (rows) {
+        const Tensor r = pick_rows(*rows, x);
+        Tensor h = at::empty({r.numel(), x.size(1)}, x.options().dtype(out_f32 ? at::kFloat : at::kBFloat16));
+        if (!chronos::hy_rows_norm_ok((int)x.size(1)) || ((reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr())) & 15) != 0)
+            return hy_layer_norm(x.index_select(0, r), w, eps, out_f32, c10::nullopt);
+        chronos::launch_hy_layer_norm_rows(x.data_ptr<float>(), r.data_ptr<int64_t>(), (int)x.size(0), w.data_ptr<float>(), h.data_ptr(), out_f32,
+                                           (int)r.numel(), (int)x.size(1), (float)eps, stream());
+        return h;
+    }
     auto h = at::empty_like(x, x.options().dtype(out_f32 ? at::kFloat : at::kBFloat16));
     chronos::launch_hy_layer_norm(x.data_ptr(), true, nullptr, w.data_ptr<float>(), h.data_ptr(), out_f32,
                                   (int)x.size(0), (int)x.size(1), (float)eps, stream());
@@ -491,11 +530,19 @@ Tensor hy_moe_ffn(const Tensor& h, const Tensor& idx, const Tensor& wt, const Te
     return out;
 }
 
-Tensor hy_rms_norm(const Tensor& x, const Tensor& w, double eps, bool out_f32) {
+Tensor hy_rms_norm(const Tensor& x, const Tensor& w, double eps, bool out_f32, const c10::optional<Tensor>& rows) {
     c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
     flt(x, "rms_norm: float32 rows");
     flt(w, "rms_norm: float32 weight");
     need(x.dim() == 2 && w.numel() == x.size(1), "rms_norm: weight size");
+    if (rows) {
+        const Tensor r = pick_rows(*rows, x);
+        if (x.size(1) % 4 != 0) return hy_rms_norm(x.index_select(0, r), w, eps, out_f32, c10::nullopt);
+        auto h = at::empty({r.numel(), x.size(1)}, x.options().dtype(out_f32 ? at::kFloat : at::kBFloat16));
+        chronos::launch_hy_rms_norm_rows(x.data_ptr<float>(), r.data_ptr<int64_t>(), (int)x.size(0), w.data_ptr<float>(), h.data_ptr(), out_f32,
+                                         (int)r.numel(), (int)x.size(1), (float)eps, stream());
+        return h;
+    }
     auto h = at::empty_like(x, x.options().dtype(out_f32 ? at::kFloat : at::kBFloat16));
     chronos::launch_hy_rms_norm(nullptr, const_cast<float*>(x.data_ptr<float>()), w.data_ptr<float>(), h.data_ptr(),
                                 out_f32, (int)x.size(0), (int)x.size(1), 1.f, (float)eps, stream());
@@ -1036,12 +1083,22 @@ void hy_pool_blocks(const Tensor& kc, const Tensor& vc, Tensor& kp, Tensor& vp, 
 Tensor hy_sandwich_join(const c10::optional<Tensor>& y, const c10::optional<Tensor>& y2, Tensor& x,
                         const c10::optional<Tensor>& w_y, const c10::optional<Tensor>& w_out,
                         const c10::optional<Tensor>& w_a, const c10::optional<Tensor>& w_b, int64_t groups, double eps,
-                        bool out_f32, bool add, bool emit) {
+                        bool out_f32, bool add, bool emit, const c10::optional<Tensor>& rows) {
     c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
     flt(x, "sandwich_join: the stream is contiguous float32");
     need(x.dim() == 2, "sandwich_join: x [T, d]");
-    const int64_t T = x.size(0), d = x.size(1);
+    const int64_t d = x.size(1);
     need(chronos::hy_sandwich_groups_ok((int)d, (int)groups), "sandwich_join: groups >= 1 and d % groups == 0");
+    Tensor r;
+    if (rows) {
+        r = pick_rows(*rows, x);
+        need(!add && emit, "sandwich_join: rows are picked for the plain norm only");
+        if (!chronos::hy_sandwich_rows_ok((int)d, (int)groups)) {
+            Tensor xs = x.index_select(0, r);
+            return hy_sandwich_join(y, y2, xs, w_y, w_out, w_a, w_b, groups, eps, out_f32, add, emit, c10::nullopt);
+        }
+    }
+    const int64_t T = rows ? r.numel() : x.size(0);
     need(add == y.has_value() && (add || emit), "sandwich_join: an addend when adding, something to do otherwise");
     if (add) {
         need(is_act(*y) && y->is_contiguous() && y->dim() == 2 && y->size(0) == T && y->size(1) == d, "sandwich_join: y [T, d]");
@@ -1071,7 +1128,8 @@ Tensor hy_sandwich_join(const c10::optional<Tensor>& y, const c10::optional<Tens
                                      add ? w_y->data_ptr<float>() : nullptr, emit ? w_out->data_ptr<float>() : nullptr,
                                      (add && w_a) ? w_a->data_ptr<float>() : nullptr,
                                      (add && w_b) ? w_b->data_ptr<float>() : nullptr, emit ? h.data_ptr() : nullptr, (int)T,
-                                     (int)d, (int)groups, (float)eps, add ? f32(*y) : true, out_f32, stream());
+                                     (int)d, (int)groups, (float)eps, add ? f32(*y) : true, out_f32, rows ? r.data_ptr<int64_t>() : nullptr,
+                                     (int)x.size(0), stream());
     return h;
 }
 
@@ -1123,7 +1181,8 @@ Tensor hy_unrotate_gate(const Tensor& o, const Tensor& pos, const c10::optional<
 TORCH_LIBRARY_FRAGMENT(chronos, m) {
     m.def("hy_embed(Tensor ids, Tensor table, float scale=1.0) -> Tensor");
     m.def("hy_embed_both(Tensor ids, Tensor table, float scale) -> (Tensor, Tensor)");
-    m.def("hy_layer_norm(Tensor x, Tensor w, float eps, bool out_f32) -> Tensor");
+    m.def("hy_embed_start(Tensor ids, Tensor table, float scale, bool both, Tensor pos, Tensor q_start) -> (Tensor, Tensor, Tensor)");
+    m.def("hy_layer_norm(Tensor x, Tensor w, float eps, bool out_f32, Tensor? rows=None) -> Tensor");
     m.def("hy_add_layer_norm(Tensor y, Tensor(a!) x, Tensor w, float eps, bool out_f32) -> Tensor");
     m.def("hy_rowdot(Tensor h, Tensor w, Tensor? bias) -> Tensor");
     m.def("hy_act(Tensor(a!) x, int kind) -> ()");
@@ -1154,7 +1213,7 @@ TORCH_LIBRARY_FRAGMENT(chronos, m) {
           "float scale, int rank, int max_q, int window=0, bool two_term=False, Tensor? sink=None) -> Tensor");
     m.def("hy_moe_route(Tensor h, Tensor w, Tensor corr, int top) -> (Tensor, Tensor)");
     m.def("hy_moe_ffn(Tensor h, Tensor idx, Tensor wt, Tensor w_up, Tensor w_down, int act) -> Tensor");
-    m.def("hy_rms_norm(Tensor x, Tensor w, float eps, bool out_f32) -> Tensor");
+    m.def("hy_rms_norm(Tensor x, Tensor w, float eps, bool out_f32, Tensor? rows=None) -> Tensor");
     m.def("hy_scale_add_rms_norm(Tensor y, Tensor(a!) x, Tensor w, float alpha, float eps, bool out_f32) -> Tensor");
     m.def("hy_glu(Tensor gu, float limit, float slope, float shift) -> Tensor");
     m.def("hy_glu_cols(Tensor src, int off, int F, float limit, float slope, float shift, Tensor(a!) out) -> ()");
@@ -1177,7 +1236,7 @@ TORCH_LIBRARY_FRAGMENT(chronos, m) {
     m.def("hy_pool_blocks(Tensor kc, Tensor vc, Tensor(a!) kp, Tensor(b!) vp, Tensor block_table, Tensor q_start, "
           "Tensor pos0, int pool, int max_q) -> ()");
     m.def("hy_sandwich_join(Tensor? y, Tensor? y2, Tensor(a!) x, Tensor? w_y, Tensor? w_out, Tensor? w_a, Tensor? w_b, "
-          "int groups, float eps, bool out_f32, bool add, bool emit) -> Tensor");
+          "int groups, float eps, bool out_f32, bool add, bool emit, Tensor? rows=None) -> Tensor");
     m.def("hy_rotate_qk(Tensor(a!) proj, int q_off, int k_off, int HQ, int HK, int D, int dims, Tensor? cos_sin, Tensor pos, "
           "float q_mul, float k_mul) -> ()");
     m.def("hy_unrotate_gate(Tensor o, Tensor pos, Tensor? cos_sin, Tensor? gate_src, int g_off, int H, int Dv) -> Tensor");
@@ -1204,6 +1263,7 @@ TORCH_LIBRARY_FRAGMENT(chronos, m) {
 TORCH_LIBRARY_IMPL(chronos, CUDA, m) {
     m.impl("hy_embed", &hy_embed);
     m.impl("hy_embed_both", &hy_embed_both);
+    m.impl("hy_embed_start", &hy_embed_start);
     m.impl("hy_layer_norm", &hy_layer_norm);
     m.impl("hy_add_layer_norm", &hy_add_layer_norm);
     m.impl("hy_rowdot", &hy_rowdot);

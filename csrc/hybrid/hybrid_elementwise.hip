@@ -9,11 +9,17 @@
 namespace chronos {
 namespace hy {
 
-// h (or nullptr): the rows in bfloat16 as well
+// h (or nullptr): the rows in bfloat16 as well.  pos0 (or nullptr) [B]: pos at every sequence's first token, which a prompt step's recurrences
+// ask for; sequences without tokens read the last one's.  Here it costs nothing (three launches of torch's, 4.7 us each and 10 us of the host's
+// time, which is what bounds prompts of a few hundred tokens).
 template <typename T>
 __global__ void __launch_bounds__(256) embed_kernel(const int32_t* __restrict__ ids, const T* __restrict__ table,
-                                                    float* __restrict__ x, uint16_t* __restrict__ h, int d, float scale) {
+                                                    float* __restrict__ x, uint16_t* __restrict__ h, int d, float scale,
+                                                    const int32_t* __restrict__ pos, const int32_t* __restrict__ q_start,
+                                                    int32_t* __restrict__ pos0, int B) {
     const int64_t t = blockIdx.x;
+    if (pos0 != nullptr && t == 0)
+        for (int b = threadIdx.x; b < B; b += 256) pos0[b] = pos[min(max(q_start[b], 0), (int)gridDim.x - 1)];
     const T* src = table + (int64_t)ids[t] * d;
     if constexpr (sizeof(T) == 2) {
         if (d % 8 == 0 && ((reinterpret_cast<uintptr_t>(table) | reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(h)) & 15) == 0) {   // 8 columns a thread
@@ -69,15 +75,16 @@ __global__ void __launch_bounds__(256) layer_norm_kernel(const TY* __restrict__ 
 // three strided passes, 5.0 so).
 template <typename TH>
 __global__ void __launch_bounds__(256) layer_norm_plain_kernel(const float* __restrict__ y, const float* __restrict__ w, TH* __restrict__ h,
-                                                               int d, float eps) {
+                                                               int d, float eps, const int64_t* __restrict__ rows, int total) {
     __shared__ float red[16];
-    const int64_t row = blockIdx.x;
+    const int64_t row = blockIdx.x, src = rows != nullptr ? rows[row] : row;
+    const bool there = src >= 0 && src < total;
     f32x4 v[4];
     float s = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int i = (threadIdx.x + 256 * j) * 4;
-        v[j] = i < d ? *reinterpret_cast<const f32x4*>(y + row * d + i) : f32x4{0.f, 0.f, 0.f, 0.f};
+        v[j] = i < d ? there ? *reinterpret_cast<const f32x4*>(y + src * d + i) : f32x4{NAN, NAN, NAN, NAN} : f32x4{0.f, 0.f, 0.f, 0.f};
         s += (v[j][0] + v[j][1]) + (v[j][2] + v[j][3]);
     }
     const float mean = block_sum(s, red) / (float)d;
@@ -345,10 +352,19 @@ __global__ void __launch_bounds__(256) act_vec_kernel(uint16_t* __restrict__ x, 
 
 }  // namespace hy
 
-void launch_hy_embed(const int32_t* ids, const void* table, float* x, uint16_t* h, int T, int d, float scale, bool f32, hipStream_t s) {
+void launch_hy_embed(const int32_t* ids, const void* table, float* x, uint16_t* h, int T, int d, float scale, bool f32, const int32_t* pos,
+                     const int32_t* q_start, int32_t* pos0, int B, hipStream_t s) {
     if (T == 0) return;
-    if (f32) hy::embed_kernel<float><<<T, 256, 0, s>>>(ids, (const float*)table, x, h, d, scale);
-    else hy::embed_kernel<uint16_t><<<T, 256, 0, s>>>(ids, (const uint16_t*)table, x, h, d, scale);
+    if (f32) hy::embed_kernel<float><<<T, 256, 0, s>>>(ids, (const float*)table, x, h, d, scale, pos, q_start, pos0, B);
+    else hy::embed_kernel<uint16_t><<<T, 256, 0, s>>>(ids, (const uint16_t*)table, x, h, d, scale, pos, q_start, pos0, B);
+}
+// Row r of a norm over chosen rows: row rows[r] of the `total` there are (none of them: NaN, as memory past the stream is not its)
+bool hy_rows_norm_ok(int d) { return d % 4 == 0 && d <= 4096; }
+void launch_hy_layer_norm_rows(const float* x, const int64_t* rows, int total, const float* w, void* h, bool out_f32, int n, int d, float eps,
+                               hipStream_t s) {
+    if (n == 0) return;
+    if (out_f32) hy::layer_norm_plain_kernel<float><<<n, 256, 0, s>>>(x, w, (float*)h, d, eps, rows, total);
+    else hy::layer_norm_plain_kernel<uint16_t><<<n, 256, 0, s>>>(x, w, (uint16_t*)h, d, eps, rows, total);
 }
 // y_f32: the input is float (the plain norm of the stream); out_f32: h is float.  x == nullptr: plain norm.
 void launch_hy_layer_norm(const void* y, bool y_f32, float* x, const float* w, void* h, bool out_f32, int rows, int d,
@@ -365,8 +381,8 @@ void launch_hy_layer_norm(const void* y, bool y_f32, float* x, const float* w, v
         if (y_f32) hy::layer_norm_kernel<float, float, true><<<rows, 256, 0, s>>>((const float*)y, x, w, (float*)h, d, eps);
         else hy::layer_norm_kernel<uint16_t, uint16_t, true><<<rows, 256, 0, s>>>((const uint16_t*)y, x, w, (uint16_t*)h, d, eps);
     } else if (y_f32 && d % 4 == 0 && d <= 4096 && hy::aligned16(y, w, h)) {
-        if (out_f32) hy::layer_norm_plain_kernel<float><<<rows, 256, 0, s>>>((const float*)y, w, (float*)h, d, eps);
-        else hy::layer_norm_plain_kernel<uint16_t><<<rows, 256, 0, s>>>((const float*)y, w, (uint16_t*)h, d, eps);
+        if (out_f32) hy::layer_norm_plain_kernel<float><<<rows, 256, 0, s>>>((const float*)y, w, (float*)h, d, eps, nullptr, rows);
+        else hy::layer_norm_plain_kernel<uint16_t><<<rows, 256, 0, s>>>((const float*)y, w, (uint16_t*)h, d, eps, nullptr, rows);
     } else {
         if (out_f32) hy::layer_norm_kernel<float, float, false><<<rows, 256, 0, s>>>((const float*)y, nullptr, w, (float*)h, d, eps);
         else hy::layer_norm_kernel<float, uint16_t, false><<<rows, 256, 0, s>>>((const float*)y, nullptr, w, (uint16_t*)h, d, eps);

@@ -72,14 +72,16 @@ __global__ void __launch_bounds__(256) rms_norm_slices_kernel(Slices y, float* _
     }
 }
 
-// JOIN: v = alpha * x + y (y in TY), x <- norm(v) * w, h <- TH(x).   plain: v = x (float), h <- TH(norm(v) * w).
+// JOIN: v = alpha * x + y (y in TY), x <- norm(v) * w, h <- TH(x).   plain: v = x (float), h <- TH(norm(v) * w); with `rows` (VEC only) v = x's
+// row rows[r] of `total`, NaN where there is none.
 template <typename TY, typename TH, bool JOIN, bool VEC>
 __global__ void __launch_bounds__(256) rms_norm_kernel(const TY* __restrict__ y, float* __restrict__ x,
                                                        const float* __restrict__ w, TH* __restrict__ h, int d,
-                                                       float alpha, float eps) {
+                                                       float alpha, float eps, const int64_t* __restrict__ rows, int total) {
     __shared__ float red[16];
-    const int64_t row = blockIdx.x;
-    float* xr = x + row * d;
+    const int64_t row = blockIdx.x, src = !JOIN && VEC && rows != nullptr ? rows[row] : row;
+    const bool there = JOIN || !VEC || (src >= 0 && src < total);
+    float* xr = x + (there ? src : 0) * d;
     const TY* yr = JOIN ? y + row * d : nullptr;
     TH* hr = h != nullptr ? h + row * d : nullptr;
     float ss = 0.f;
@@ -92,6 +94,7 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(const TY* __restrict__ y,
             if (i < d) {
                 f32x4 v = *reinterpret_cast<const f32x4*>(xr + i);
                 if constexpr (JOIN) v = v * alpha + ld4<TY>(yr + i);
+                if (!there) v *= NAN;
                 c[j] = v;
                 ss += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
             }
@@ -114,7 +117,7 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(const TY* __restrict__ y,
         for (int i = (threadIdx.x + 1024) * 4; i < d; i += 1024) {
             f32x4 v = *reinterpret_cast<const f32x4*>(xr + i);
             if constexpr (JOIN) v = v * alpha + ld4<TY>(yr + i);
-            v = v * rstd * *reinterpret_cast<const f32x4*>(w + i);
+            v = v * rstd * *reinterpret_cast<const f32x4*>(w + i);   // (of no row there is: rstd is NaN)
             if constexpr (JOIN) *reinterpret_cast<f32x4*>(xr + i) = v;
             if (hr != nullptr) st4<TH>(hr + i, v);
         }
@@ -266,8 +269,8 @@ void launch_hy_rms_norm(const void* y, float* x, const float* w, void* h, bool o
     const bool vec = d % 4 == 0;
 #define HY_RN(TY, TH, JOIN)                                                                                           \
     do {                                                                                                              \
-        if (vec) hy::rms_norm_kernel<TY, TH, JOIN, true><<<rows, 256, 0, s>>>((const TY*)y, x, w, (TH*)h, d, alpha, eps); \
-        else hy::rms_norm_kernel<TY, TH, JOIN, false><<<rows, 256, 0, s>>>((const TY*)y, x, w, (TH*)h, d, alpha, eps);    \
+        if (vec) hy::rms_norm_kernel<TY, TH, JOIN, true><<<rows, 256, 0, s>>>((const TY*)y, x, w, (TH*)h, d, alpha, eps, nullptr, rows); \
+        else hy::rms_norm_kernel<TY, TH, JOIN, false><<<rows, 256, 0, s>>>((const TY*)y, x, w, (TH*)h, d, alpha, eps, nullptr, rows);    \
     } while (0)
     if (y != nullptr) {
         if (out_f32) HY_RN(float, float, true);
@@ -277,6 +280,15 @@ void launch_hy_rms_norm(const void* y, float* x, const float* w, void* h, bool o
         else HY_RN(float, uint16_t, false);
     }
 #undef HY_RN
+}
+
+// the plain norm of rows[0 .. n) of x's `total` rows, d % 4 == 0
+void launch_hy_rms_norm_rows(const float* x, const int64_t* rows, int total, const float* w, void* h, bool out_f32, int n, int d, float eps,
+                             hipStream_t s) {
+    if (n == 0) return;
+    float* const xs = const_cast<float*>(x);
+    if (out_f32) hy::rms_norm_kernel<float, float, false, true><<<n, 256, 0, s>>>(nullptr, xs, w, (float*)h, d, 1.f, eps, rows, total);
+    else hy::rms_norm_kernel<float, uint16_t, false, true><<<n, 256, 0, s>>>(nullptr, xs, w, (uint16_t*)h, d, 1.f, eps, rows, total);
 }
 
 void launch_hy_rms_norm_slices(const float* ys, int S, float* x, const float* w, uint16_t* h, int rows, int d, float alpha, float eps,

@@ -58,18 +58,21 @@ __device__ __forceinline__ float sw_total(const float* red, int g) {
     return (red[g] + red[kSwMaxGroups + g]) + (red[2 * kSwMaxGroups + g] + red[3 * kSwMaxGroups + g]);
 }
 
-// VEC: d <= 4096, d / groups % 4 == 0: every thread owns up to 4 chunks of 4 columns, read once.
+// VEC: d <= 4096, d / groups % 4 == 0: every thread owns up to 4 chunks of 4 columns, read once.  pick (or nullptr; only without y): row r is
+// x's row pick[r] of `total`, NaN where there is none.
 // TY: the sublayer outputs' type; TH: the emitted type.
 template <typename TY, typename TH>
 __global__ void __launch_bounds__(256) sandwich_join_vec_kernel(const TY* __restrict__ y, const TY* __restrict__ y2,
                                                                 float* __restrict__ x, const float* __restrict__ w_y,
                                                                 const float* __restrict__ w_out,
                                                                 const float* __restrict__ w_a, const float* __restrict__ w_b,
-                                                                TH* __restrict__ h, int d, int groups, float eps) {
+                                                                TH* __restrict__ h, int d, int groups, float eps,
+                                                                const int64_t* __restrict__ pick, int total) {
     __shared__ float red3[3][4 * kSwMaxGroups];   // one scratch area per reduction of the kernel
-    const int64_t row = blockIdx.x;
+    const int64_t row = blockIdx.x, src = pick != nullptr ? pick[row] : row;
+    const bool there = src >= 0 && src < total;
     const int gsz = d / groups;
-    float* xr = x + row * d;
+    float* xr = x + (there ? src : 0) * d;
     int gidx[4];
     f32x4 v[4];
     float ss[4];
@@ -135,7 +138,7 @@ __global__ void __launch_bounds__(256) sandwich_join_vec_kernel(const TY* __rest
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int i = (threadIdx.x + 256 * j) * 4;
-            if (i < d) v[j] = *reinterpret_cast<const f32x4*>(xr + i);
+            if (i < d) v[j] = *reinterpret_cast<const f32x4*>(xr + i) * (there ? 1.f : NAN);
         }
     }
     if (h == nullptr) return;
@@ -160,13 +163,16 @@ __global__ void __launch_bounds__(256) sandwich_join_wave_kernel(const TY* __res
                                                                  float* __restrict__ x, const float* __restrict__ w_y,
                                                                  const float* __restrict__ w_out,
                                                                  const float* __restrict__ w_a, const float* __restrict__ w_b,
-                                                                 TH* __restrict__ h, int rows, int d, int groups, float eps) {
+                                                                 TH* __restrict__ h, int rows, int d, int groups, float eps,
+                                                                 const int64_t* __restrict__ pick, int total) {
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
+    const int64_t src = pick != nullptr ? pick[row] : row;
+    const bool there = src >= 0 && src < total;
     const int gsz = d / groups;
     const float inv_g = 1.f / (float)gsz;
-    float* xr = x + row * d;
+    float* xr = x + (there ? src : 0) * d;
     int gidx[NJ];
     f32x4 v[NJ];
 #pragma unroll
@@ -239,7 +245,7 @@ __global__ void __launch_bounds__(256) sandwich_join_wave_kernel(const TY* __res
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             const int i = (lane + 64 * j) * 4;
-            if (i < d) v[j] = *reinterpret_cast<const f32x4*>(xr + i);
+            if (i < d) v[j] = *reinterpret_cast<const f32x4*>(xr + i) * (there ? 1.f : NAN);
         }
     }
     if (h == nullptr) return;
@@ -360,19 +366,22 @@ __global__ void __launch_bounds__(256) unrotate_gate_kernel(const T* o, const in
 }  // namespace hy
 
 bool hy_sandwich_groups_ok(int d, int groups) { return groups >= 1 && d % groups == 0; }
+// may launch_hy_sandwich_join be told which rows to take?
+bool hy_sandwich_rows_ok(int d, int groups) { return d <= 4096 && (d / groups) % 4 == 0 && groups <= hy::kSwMaxGroups; }
 
 // y == nullptr: the plain grouped norm of x (x untouched).  h == nullptr: nothing is emitted.  y_f32: y and y2 are
-// float (else bfloat16); out_f32: h is float (else bfloat16).  w_a != nullptr: the pair form (y2 and w_b given).
+// float (else bfloat16); out_f32: h is float (else bfloat16).  w_a != nullptr: the pair form (y2 and w_b given).  pick != nullptr (y == nullptr,
+// hy_sandwich_rows_ok): the norm of x's rows pick[0 .. rows) of `total`.
 void launch_hy_sandwich_join(const void* y, const void* y2, float* x, const float* w_y, const float* w_out,
                              const float* w_a, const float* w_b, void* h, int rows, int d, int groups, float eps,
-                             bool y_f32, bool out_f32, hipStream_t s) {
+                             bool y_f32, bool out_f32, const int64_t* pick, int total, hipStream_t s) {
     if (rows == 0) return;
-    const bool vec = d <= 4096 && (d / groups) % 4 == 0 && groups <= hy::kSwMaxGroups;
+    const bool vec = hy_sandwich_rows_ok(d, groups);
     const int wg4 = (rows + 3) / 4;
 #define HY_SW(TY, TH)                                                                                                      \
     do {                                                                                                                   \
-        if (vec && d <= 1024) hy::sandwich_join_wave_kernel<TY, TH, 4><<<wg4, 256, 0, s>>>((const TY*)y, (const TY*)y2, x, w_y, w_out, w_a, w_b, (TH*)h, rows, d, groups, eps); \
-        else if (vec) hy::sandwich_join_vec_kernel<TY, TH><<<rows, 256, 0, s>>>((const TY*)y, (const TY*)y2, x, w_y, w_out, w_a, w_b, (TH*)h, d, groups, eps); \
+        if (vec && d <= 1024) hy::sandwich_join_wave_kernel<TY, TH, 4><<<wg4, 256, 0, s>>>((const TY*)y, (const TY*)y2, x, w_y, w_out, w_a, w_b, (TH*)h, rows, d, groups, eps, pick, total); \
+        else if (vec) hy::sandwich_join_vec_kernel<TY, TH><<<rows, 256, 0, s>>>((const TY*)y, (const TY*)y2, x, w_y, w_out, w_a, w_b, (TH*)h, d, groups, eps, pick, total); \
         else hy::sandwich_join_any_kernel<TY, TH><<<rows, 256, 0, s>>>((const TY*)y, (const TY*)y2, x, w_y, w_out, w_a, w_b, (TH*)h, d, groups, eps); \
     } while (0)
     if (y_f32 && out_f32) HY_SW(float, float);

@@ -68,6 +68,7 @@ int gemm_skinny_mt(int cfg);
 int gemm_skinny_nw(int cfg);  // waves per workgroup
 // y [n] = the sum of S float32 slices [S, n], in their order
 void launch_gemm_slices(const float* ws, uint16_t* y, int64_t n, int S, hipStream_t st);
+void launch_gemm_slices_f32(const float* ws, float* y, int64_t n, int S, hipStream_t st);
 bool launch_gemm_skinny(int cfg, int mode, bool normp, const PPArgs& a, hipStream_t st);
 
 }  // namespace chronos

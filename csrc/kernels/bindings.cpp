@@ -688,7 +688,7 @@ std::tuple<Tensor, Tensor> gemm_few(const Tensor& x, const Tensor& w, int64_t cf
 }
 
 // The float32 slices [splitk, M, N] of a plain product of few rows whose K is split over workgroups, nothing kept between calls: gemm_lg.hip's
-// 64-row tiles and smaller, or (skinny) gemm_skinny.hip's uneven configs.  Their sum in order, rounded, is the product.
+// 64-row tiles and smaller, or (skinny) gemm_skinny.hip's uneven configs.  Their sum in order, rounded, is the product; one slice is the product unrounded.
 Tensor gemm_slices(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk, bool skinny) {
     chk_bf16(x, "x");
     chk_bf16(w, "w");
@@ -700,7 +700,7 @@ Tensor gemm_slices(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk
     CHK((N + BN) * K * 2 < (1LL << 31) && (M + BM) * K * 2 < (1LL << 31), "gemm_split: operand > 2 GiB");
     CHK(!skinny || (M <= BM && N % BN == 0), "gemm_split: M, N of the config");
     CHK(M >= 1 && K % 64 == 0 && K <= (1 << 20) && N >= 4 && N % 4 == 0, "gemm_split: size");
-    CHK(splitk > 1 && splitk <= 64 && (skinny || (K / 64) % splitk == 0), "gemm_split: splitk must divide K / 64");
+    CHK(splitk >= 1 && splitk <= 64 && (skinny || (K / 64) % splitk == 0), "gemm_split: splitk must divide K / 64");
     CHK(((reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr())) & 15) == 0, "gemm_split: alignment");
     c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
     chronos::PPArgs a{};
@@ -721,10 +721,21 @@ Tensor gemm_slices(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk
 }
 
 Tensor gemm_split(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk) {
+    CHK(splitk > 1, "gemm_split: splitk");
     const Tensor ws = gemm_slices(x, w, cfg, splitk, false);
     c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
     Tensor y = at::empty({ws.size(1), ws.size(2)}, x.options());
     chronos::launch_gemm_slices(ws.data_ptr<float>(), bfm(y), y.numel(), (int)splitk, cur_stream());
+    return y;
+}
+
+// The same product as float32 [M, N]: its sums without the rounding
+Tensor gemm_f32(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk, bool skinny) {
+    const Tensor ws = gemm_slices(x, w, cfg, splitk, skinny);
+    if (splitk == 1) return ws[0];
+    c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+    Tensor y = at::empty({ws.size(1), ws.size(2)}, ws.options());
+    chronos::launch_gemm_slices_f32(ws.data_ptr<float>(), y.data_ptr<float>(), y.numel(), (int)splitk, cur_stream());
     return y;
 }
 
@@ -953,6 +964,7 @@ TORCH_LIBRARY(chronos, m) {
     m.def("gemm_few(Tensor x, Tensor w, int cfg, int mode, int n0, int nf, Tensor? bias, float limit, float slope, float shift) -> (Tensor, Tensor)");
     m.def("gemm_split(Tensor x, Tensor w, int cfg, int splitk) -> Tensor");
     m.def("gemm_slices(Tensor x, Tensor w, int cfg, int splitk, bool skinny) -> Tensor");
+    m.def("gemm_f32(Tensor x, Tensor w, int cfg, int splitk, bool skinny) -> Tensor");
     m.def("gemm_pp(Tensor x, Tensor w, int mode, int cfg, int splitk, Tensor? resid, Tensor? part_in, float eps, bool prio) -> (Tensor, Tensor)");
     m.def("gemm_skinny(Tensor x, Tensor w, int mode, int cfg, int splitk, Tensor? resid, Tensor? part_in, float eps) "
           "-> (Tensor, Tensor)");
@@ -999,6 +1011,7 @@ TORCH_LIBRARY_IMPL(chronos, CUDA, m) {
     m.impl("gemm_few", &gemm_few);
     m.impl("gemm_split", &gemm_split);
     m.impl("gemm_slices", &gemm_slices);
+    m.impl("gemm_f32", &gemm_f32);
     m.impl("gemm_pp", &gemm_pp);
     m.impl("gemm_skinny", &gemm_skinny);
     m.impl("gemv_resid", &gemv_resid);

@@ -982,9 +982,9 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
         return;
     }
 
-    // ---- split-K without state (plain, no tickets): the slice's sums [S, M, N], which a second launch adds up
+    // ---- split-K without state (plain, no tickets): the slice's sums [S, M, N], which a second launch adds up; one slice: float32 outputs
     if constexpr (MODE == kPlain && !NORMP && !HB && !F8 && !M32 && ABL == 0) {
-        if (S > 1 && a.cnt == nullptr) {
+        if (a.ws != nullptr && a.cnt == nullptr) {
 #pragma unroll
             for (int u = 0; u < MT; ++u) {
                 const int m = m0 + xrow0 + 16 * u + (lane & 15);

@@ -219,7 +219,7 @@ __global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a) {
             }
     }
 
-    if (MODE == kPlain && !NORMP && S > 1 && a.cnt == nullptr) {  // the slice's sums [S, M, N]: skinny_sum_kernel adds them
+    if (MODE == kPlain && !NORMP && a.ws != nullptr && a.cnt == nullptr) {  // the slice's sums [S, M, N]: skinny_sum_kernel adds them
         if (active) {
 #pragma unroll
             for (int j = 0; j < VP; ++j) {
@@ -333,22 +333,30 @@ __global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a) {
     }
 }
 
-// y = the sum over S slices of 4 outputs per thread, in slice order
-__global__ void __launch_bounds__(256) skinny_sum_kernel(const float* __restrict__ ws, uint16_t* __restrict__ y, int64_t n, int S) {
+// y = the sum over S slices of 4 outputs per thread, in slice order; F: y stays float
+template <bool F>
+__global__ void __launch_bounds__(256) skinny_sum_kernel(const float* __restrict__ ws, void* __restrict__ y, int64_t n, int S) {
     const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= n) return;
     f32x4 v = *reinterpret_cast<const f32x4*>(ws + i);
     for (int s = 1; s < S; ++s) v += *reinterpret_cast<const f32x4*>(ws + s * n + i);
-    u16x4 o;
+    if constexpr (F) {
+        *reinterpret_cast<f32x4*>(static_cast<float*>(y) + i) = v;
+    } else {
+        u16x4 o;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) o[k] = f2bf(v[k]);
-    *reinterpret_cast<u16x4*>(y + i) = o;
+        for (int k = 0; k < 4; ++k) o[k] = f2bf(v[k]);
+        *reinterpret_cast<u16x4*>(static_cast<uint16_t*>(y) + i) = o;
+    }
 }
 
 }  // namespace
 
 void launch_gemm_slices(const float* ws, uint16_t* y, int64_t n, int S, hipStream_t st) {   // n % 4 == 0
-    skinny_sum_kernel<<<(unsigned)((n / 4 + 255) / 256), 256, 0, st>>>(ws, y, n, S);
+    skinny_sum_kernel<false><<<(unsigned)((n / 4 + 255) / 256), 256, 0, st>>>(ws, y, n, S);
+}
+void launch_gemm_slices_f32(const float* ws, float* y, int64_t n, int S, hipStream_t st) {
+    skinny_sum_kernel<true><<<(unsigned)((n / 4 + 255) / 256), 256, 0, st>>>(ws, y, n, S);
 }
 
 namespace {

@@ -1232,13 +1232,14 @@ class HybridDecoder:
             sb.fresh = (sb.pos, sb.pos._version, sb.q_start, sb.q_start._version)
         return sb
 
-    def _meta(self, sb: StepBatch) -> StepMeta:
+    def _meta(self, sb: StepBatch, first=None) -> StepMeta:
+        """``first``: the sequences' first positions, where the caller has them."""
         def one(p: StepBatch) -> StepMeta:
             if p.slots is None:
                 raise ValueError("a hybrid decoder's step batch needs the sequences' state slots")
             if p.tiles is None:  # decode rows: token i is sequence i
                 return StepMeta(p.ids, p.pos, p.tok_seq, p.block_table, p.q_start, p.pos, p.slots, p.last_idx, 1)
-            pos0 = p.pos.index_select(0, p.q_start[:-1].long().clamp(max=max(0, p.pos.numel() - 1)))
+            pos0 = p.pos.index_select(0, p.q_start[:-1].long().clamp(max=max(0, p.pos.numel() - 1))) if first is None else first
             f = p.fresh
             fresh = f is not None and f[0] is p.pos and f[2] is p.q_start and f[1] == p.pos._version and f[3] == p.q_start._version
             # a graph's replays read whatever positions its tensors hold then
@@ -1259,8 +1260,13 @@ class HybridDecoder:
         """Logits [len(sb.last_idx), V] of the tokens at sb.last_idx (with ``sb.dec``: indices into prefill tokens
         followed by decode rows)."""
         cfg, w, at = self.cfg, self.w, self.act_dtype
-        meta = self._meta(sb)
-        x, h = hops.embed_rows(meta.ids, w.embed, at, cfg.embed_scale, cfg.residual not in ("pre_norm", "sandwich", "parallel"))
+        emit = cfg.residual not in ("pre_norm", "sandwich", "parallel")
+        if sb.dec is None and sb.tiles is not None and sb.slots is not None:   # one range per sequence: its first position comes along
+            x, h, first = hops.embed_start(sb.ids, w.embed, at, cfg.embed_scale, emit, sb.pos, sb.q_start)
+            meta = self._meta(sb, first)
+        else:
+            meta = self._meta(sb)
+            x, h = hops.embed_rows(meta.ids, w.embed, at, cfg.embed_scale, emit)
         if self.gated_stream:
             self._forward_gated(x, meta, cache)
         elif cfg.residual == "pre_norm":
@@ -1279,16 +1285,15 @@ class HybridDecoder:
                     h = self._join(y, x, lw.norm2)
                 if self.layer_tap is not None:
                     self.layer_tap(ri, x)
-        xs = x.index_select(0, meta.last_idx)
         if cfg.residual == "out_norm":
-            xn = hops.layer_norm(xs, w.final_norm, cfg.norm_eps, at)
+            xn = hops.layer_norm(x, w.final_norm, cfg.norm_eps, at, meta.last_idx)
         elif cfg.norm == "tanh":
-            xn = hops.dyn_tanh(xs, w.final_norm, at)
+            xn = hops.dyn_tanh(x.index_select(0, meta.last_idx), w.final_norm, at)
         elif cfg.norm == "layer":
-            xn = hops.layer_norm_join(None, xs, w.final_norm, cfg.norm_eps, at)
+            xn = hops.layer_norm_join(None, x.index_select(0, meta.last_idx), w.final_norm, cfg.norm_eps, at)
         else:
-            xn = hops.rms_norm(xs, w.final_norm, cfg.norm_eps, at, cfg.norm_groups if cfg.residual == "sandwich" else 1)
-        logits = hops.matmul(xn, w.head).float()
+            xn = hops.rms_norm(x, w.final_norm, cfg.norm_eps, at, cfg.norm_groups if cfg.residual == "sandwich" else 1, meta.last_idx)
+        logits = hops.matmul_f32(xn, w.head)
         if cfg.logit_scale != 1.0:
             logits = logits * cfg.logit_scale
         return logits if logits.dtype == logits_dtype else logits.to(logits_dtype)

@@ -270,6 +270,25 @@ def few_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     return out
 
 
+# Configs of gemm_slices (csrc/kernels/bindings.cpp)
+_SLICED = (33, 36, 38, 39, 72, 73, 74, 75, 78, 79, *_UNEVEN)
+
+
+def product_f32(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
+    """x @ w.T as float32 [M, N], the product's sums before their rounding, where few_rows_plan takes it, or None.  A vocabulary's logits: 8 rows of
+    32768 x 1024 16 us as a rounded product and a conversion, 12 so."""
+    (m, k), n = x.shape if x.dim() == 2 else (0, 0), w.shape[0]
+    if not 0 < m <= 64 or n % 4 or not _plain_rows(x, w) or _registered(m, n, k) or (n + 128) * k >= 1 << 30:
+        return None
+    plan = few_rows_plan(m, n, k)
+    if plan is None or plan[0] not in _SLICED:
+        return None
+    from . import _k
+
+    skinny = plan[0] >= SK_BASE
+    return _k().gemm_f32(x, w, plan[0] - SK_BASE * skinny, plan[1], skinny)
+
+
 def product_slices(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
     """The float32 slices [S, M, N] of x @ w.T where few_rows_plan splits K, or None: for kernels that take them in the product's place."""
     (m, k), n = x.shape if x.dim() == 2 else (0, 0), w.shape[0]

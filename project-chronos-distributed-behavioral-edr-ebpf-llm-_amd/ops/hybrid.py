@@ -60,6 +60,17 @@ def matmul(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None) -
     return torch.matmul(x, w.t())
 
 
+def matmul_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x @ w.T as float32: the product's sums themselves where the framework's kernels take it, else the rounded product's values."""
+    if _gpu(x) and x.dtype == torch.bfloat16:
+        from .gemm import product_f32
+
+        y = product_f32(x, w)
+        if y is not None:
+            return y
+    return matmul(x, w).float()
+
+
 def matmul_slices(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x @ w.T for add_layer_norm or scale_add_rms_norm, which also take a product of few rows as the float32 slices [S, T, n] of its split and
     sum and round them themselves, a launch less."""
@@ -82,10 +93,21 @@ def embed_rows(ids, table, act_dtype, scale: float = 1.0, emit: bool = True):
     return ref.embed_rows(ids, table, act_dtype, scale, emit)
 
 
-def layer_norm(x, w, eps: float, act_dtype):
+def embed_start(ids, table, act_dtype, scale: float, emit: bool, pos, q_start):
+    """embed_rows and, behind them, pos at every sequence's first token (int32 [B]; sequences without tokens: at the next one's, or the last)."""
+    if _gpu(table) and ids.numel() and pos.numel() == ids.numel():
+        both = emit and not _f32(act_dtype)
+        x, h, pos0 = _k().hy_embed_start(ids, table, scale, both, pos, q_start)
+        return x, (h if both else x if emit else None), pos0
+    pos0 = pos.index_select(0, q_start[:-1].long().clamp(max=max(0, pos.numel() - 1)))
+    return (*embed_rows(ids, table, act_dtype, scale, emit), pos0)
+
+
+def layer_norm(x, w, eps: float, act_dtype, rows=None):
+    """``rows`` (int64): of these rows of x only."""
     if _gpu(x):
-        return _k().hy_layer_norm(x, w, eps, _f32(act_dtype))
-    return ref.layer_norm(x, w, eps, act_dtype)
+        return _k().hy_layer_norm(x, w, eps, _f32(act_dtype), rows)
+    return ref.layer_norm(x if rows is None else x.index_select(0, rows), w, eps, act_dtype)
 
 
 def add_layer_norm(y, x, w, eps: float, act_dtype):
@@ -224,13 +246,14 @@ def moe_ffn(h, idx, wt, w_up, w_down, act: int, act_dtype):
 # ---- post-norm residual stream, clamped GLU, windowed attention with sinks, linear-state recurrences ---------------
 
 
-def rms_norm(x, w, eps: float, act_dtype, groups: int = 1):
-    """``groups`` > 1: every one of that many equal parts of a row is divided by its own root mean square."""
+def rms_norm(x, w, eps: float, act_dtype, groups: int = 1, rows=None):
+    """``groups`` > 1: every one of that many equal parts of a row is divided by its own root mean square.  ``rows`` (int64): of these
+    rows of x only."""
     if _gpu(x):
         if groups > 1:
-            return _k().hy_sandwich_join(None, None, x, None, w, None, None, groups, eps, _f32(act_dtype), False, True)
-        return _k().hy_rms_norm(x, w, eps, _f32(act_dtype))
-    return ref.rms_norm(x, w, eps, act_dtype, groups)
+            return _k().hy_sandwich_join(None, None, x, None, w, None, None, groups, eps, _f32(act_dtype), False, True, rows)
+        return _k().hy_rms_norm(x, w, eps, _f32(act_dtype), rows)
+    return ref.rms_norm(x if rows is None else x.index_select(0, rows), w, eps, act_dtype, groups)
 
 
 def scale_add_rms_norm(y, x, w, alpha: float, eps: float, act_dtype):
