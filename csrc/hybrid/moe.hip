@@ -14,23 +14,32 @@
 // No step of either kernel depends on the host knowing the routing: both capture into a graph.
 #include "hybrid_common.h"
 
+#include <type_traits>
+
 namespace chronos {
 namespace hy {
 
-// router outputs N <= 256 (4 per lane)
-// One wave per token: z [T, N] float router logits -> the chosen outputs and their weights.
-__global__ void __launch_bounds__(256) moe_select_kernel(const float* __restrict__ z, const float* __restrict__ corr,
-                                                         int32_t* __restrict__ idx, float* __restrict__ wt, int rows,
-                                                         int N, int top) {
+__device__ __forceinline__ void unpack8(const uint4& r, float (&v)[8]) {
+    const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        v[2 * i] = __uint_as_float(w[i] << 16);
+        v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    }
+}
+
+
+// The choice of one token by one wave: zr its N <= 256 logits (4 per lane; LDS or memory) -> idx[top], wt[top].  Softmax over all N, the largest of
+// score + correction chosen, plain scores as weights.
+__device__ __forceinline__ void select_softmax(const float* zr, const float* __restrict__ corr, int32_t* __restrict__ idx, float* __restrict__ wt,
+                                               int N, int top) {
     const int lane = threadIdx.x & 63;
-    const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= rows) return;
     float s[4], c[4];
     float mx = -INFINITY;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int e = lane + 64 * j;
-        s[j] = e < N ? z[t * N + e] : -INFINITY;
+        s[j] = e < N ? zr[e] : -INFINITY;
         mx = fmaxf(mx, s[j]);
     }
     mx = wave_max(mx);
@@ -67,8 +76,8 @@ __global__ void __launch_bounds__(256) moe_select_kernel(const float* __restrict
             }
         }
         if (lane == 0) {
-            idx[t * top + k] = be;
-            wt[t * top + k] = bs;
+            idx[k] = be;
+            wt[k] = bs;
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
@@ -123,18 +132,14 @@ __global__ void __launch_bounds__(256) moe_ffn_token_kernel(const T* __restrict_
     for (int i = threadIdx.x; i < d; i += 256) st<T>(out + t * d + i, os[i]);
 }
 
-// One wave per token: the `top` largest of z [T, N] (ties: the lower index), weighted by the softmax over the chosen
-// logits only.  top <= 64 (lane k keeps the k-th choice).
-__global__ void __launch_bounds__(256) moe_select_topk_kernel(const float* __restrict__ z, int32_t* __restrict__ idx,
-                                                              float* __restrict__ wt, int rows, int N, int top) {
+// ... the `top` largest logits (ties: the lower index), weighted by the softmax over the chosen only.  top <= 64 (lane k keeps the k-th choice).
+__device__ __forceinline__ void select_topk(const float* zr, int32_t* __restrict__ idx, float* __restrict__ wt, int N, int top) {
     const int lane = threadIdx.x & 63;
-    const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= rows) return;
     float c[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int e = lane + 64 * j;
-        c[j] = e < N ? z[t * N + e] : -INFINITY;
+        c[j] = e < N ? zr[e] : -INFINITY;
     }
     float first = 0.f, sum = 0.f, mine = 0.f;  // lane k keeps the k-th chosen logit's exponential
     for (int k = 0; k < top; ++k) {
@@ -160,34 +165,28 @@ __global__ void __launch_bounds__(256) moe_select_topk_kernel(const float* __res
         sum += ex;
         if (k == lane) {
             mine = ex;
-            idx[t * top + k] = be;
+            idx[k] = be;
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             if (lane + 64 * j == be) c[j] = -INFINITY;
     }
-    if (lane < top) wt[t * top + lane] = mine / sum;
+    if (lane < top) wt[lane] = mine / sum;
 }
 
-// One wave per token: sigmoid scores of z [T, N], the choice limited to the best groups (ng groups of N / ng
-// neighbouring outputs, a group's score = its top two scores added up, the `keep` best stay; ties: the lower
-// index), then the `top` largest eligible scores (ties: the lower index), weights = score / (their sum + 1e-20) * scale.
-// ng <= 64 (lane g ranks group g), top <= 64 (lane k keeps the k-th choice).  LDS per wave: N scores, ng flags.
-__global__ void __launch_bounds__(256) moe_select_group_kernel(const float* __restrict__ z, int32_t* __restrict__ idx,
-                                                               float* __restrict__ wt, int rows, int N, int top, int ng,
-                                                               int keep, float scale) {
-    __shared__ float sc[4][256];
-    __shared__ int okg[4][64];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int64_t t = (int64_t)blockIdx.x * 4 + wv;
-    if (t >= rows) return;   // (a whole wave leaves; the waves of a block share no barrier)
+// ... sigmoid scores, the choice limited to the best groups (ng groups of N / ng neighbouring outputs, a group's score = its top two scores added up,
+// the `keep` best stay; ties: the lower index), then the `top` largest eligible scores (ties: the lower index), weights = score / (their sum +
+// 1e-20) * scale.  ng <= 64 (lane g ranks group g), top <= 64.  sc, okg: LDS of the wave's own, N scores and ng flags.
+__device__ __forceinline__ void select_group(const float* zr, int32_t* __restrict__ idx, float* __restrict__ wt, int N, int top, int ng, int keep,
+                                             float scale, float* sc, int* okg) {
+    const int lane = threadIdx.x & 63;
     const int per = N / ng;
     float s[4], c[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int e = lane + 64 * j;
-        s[j] = e < N ? sigmoidf_(z[t * N + e]) : 0.f;
-        if (e < N) sc[wv][e] = s[j];
+        s[j] = e < N ? sigmoidf_(zr[e]) : 0.f;
+        if (e < N) sc[e] = s[j];
     }
     // (wave-private LDS rows: a wave's own writes are visible to its later reads)
     if (keep < ng) {
@@ -195,7 +194,7 @@ __global__ void __launch_bounds__(256) moe_select_group_kernel(const float* __re
         if (lane < ng) {
             float a = -INFINITY, b = -INFINITY;   // the group's two largest
             for (int i = 0; i < per; ++i) {
-                const float v = sc[wv][lane * per + i];
+                const float v = sc[lane * per + i];
                 if (v > a) { b = a; a = v; }
                 else if (v > b) b = v;
             }
@@ -206,12 +205,12 @@ __global__ void __launch_bounds__(256) moe_select_group_kernel(const float* __re
             const float o = __shfl(gsc, g, 64);
             rank += (o > gsc || (o == gsc && g < lane)) ? 1 : 0;
         }
-        if (lane < ng) okg[wv][lane] = rank < keep ? 1 : 0;
+        if (lane < ng) okg[lane] = rank < keep ? 1 : 0;
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int e = lane + 64 * j;
-        c[j] = (e < N && (keep >= ng || okg[wv][e / per])) ? s[j] : -INFINITY;
+        c[j] = (e < N && (keep >= ng || okg[e / per])) ? s[j] : -INFINITY;
     }
     float sum = 0.f, mine = 0.f;
     for (int k = 0; k < top; ++k) {
@@ -235,13 +234,99 @@ __global__ void __launch_bounds__(256) moe_select_group_kernel(const float* __re
         sum += bv;
         if (k == lane) {
             mine = bv;
-            idx[t * top + k] = be;
+            idx[k] = be;
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             if (lane + 64 * j == be) c[j] = -INFINITY;
     }
-    if (lane < top) wt[t * top + lane] = mine / (sum + 1e-20f) * scale;
+    if (lane < top) wt[lane] = mine / (sum + 1e-20f) * scale;
+}
+
+struct Choice {   // which of the three, and its parameters
+    const float* corr;   // softmax form
+    int N, top, ng, keep;
+    float scale;
+};
+enum { kSoftmax = 0, kTopk = 1, kGroups = 2 };
+template <int FORM>
+__device__ __forceinline__ void select_any(const float* zr, int32_t* idx, float* wt, const Choice& c, float* sc, int* okg) {
+    if constexpr (FORM == kSoftmax) select_softmax(zr, c.corr, idx, wt, c.N, c.top);
+    else if constexpr (FORM == kTopk) select_topk(zr, idx, wt, c.N, c.top);
+    else select_group(zr, idx, wt, c.N, c.top, c.ng, c.keep, c.scale, sc, okg);
+}
+
+// One wave per token of logits z [T, N].
+template <int FORM>
+__global__ void __launch_bounds__(256) moe_select_kernel(const float* __restrict__ z, int32_t* __restrict__ idx, float* __restrict__ wt, int rows, Choice c) {
+    __shared__ float sc[FORM == kGroups ? 4 : 1][256];
+    __shared__ int okg[FORM == kGroups ? 4 : 1][64];
+    const int wv = FORM == kGroups ? threadIdx.x >> 6 : 0;
+    const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (t >= rows) return;   // (a whole wave leaves; the waves of a block share no barrier)
+    select_any<FORM>(z + t * c.N, idx + t * c.top, wt + t * c.top, c, sc[wv], okg[wv]);
+}
+
+// Projection and choice of one token by one workgroup: 16 waves share the N rows of w (N <= 64), the first wave chooses.  For up to 256 tokens, which
+// as a projection and a choice were two launches and two chains of latencies.  What bounds it is latency: a wave has up to 16 loads of 16
+// bytes a lane on their way.  us, two launches -> this: 1 token of 1024 by 10 rows 6.0 -> 5.2, 64 of 2048 by 18 11.4 -> 7.5, of 4096 by 34 12.6 -> 9.8, 256 of
+// 4096 by 64 13.9 -> 12.2; 300 tokens, more than there are CUs, 8.0 -> 9.5, 11.5 -> 13.5 and 14.9 -> 21.8.
+constexpr int kRouteN = 64, kRouteWaves = 16;
+template <int FORM>
+__global__ void __launch_bounds__(64 * kRouteWaves) moe_route_token_kernel(const uint16_t* __restrict__ h, const uint16_t* __restrict__ w,
+                                                                           const float* __restrict__ bias, int32_t* __restrict__ idx,
+                                                                           float* __restrict__ wt, int d, Choice c) {
+    __shared__ float z[kRouteN], sc[FORM == kGroups ? kRouteN : 1];
+    __shared__ int okg[FORM == kGroups ? kRouteN : 1];
+    constexpr int R = kRouteN / kRouteWaves;   // rows of a wave: wave, wave + 16, ..
+    const int64_t t = blockIdx.x;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = (c.N - wave + kRouteWaves - 1) / kRouteWaves;
+    const uint16_t *hr = h + t * d, *wr = w + (int64_t)wave * d;
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = 0.f;
+    auto part = [&](auto MC, auto UC, int k) {   // M rows by U runs of 512 columns
+        constexpr int M = decltype(MC)::value, U = decltype(UC)::value;
+        uint4 hq[U], q[M][U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) hq[u] = *reinterpret_cast<const uint4*>(hr + k + 512 * u);
+#pragma unroll
+        for (int r = 0; r < M; ++r)
+#pragma unroll
+            for (int u = 0; u < U; ++u) q[r][u] = *reinterpret_cast<const uint4*>(wr + (int64_t)r * kRouteWaves * d + k + 512 * u);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            float hv[8], wv[8];
+            unpack8(hq[u], hv);
+#pragma unroll
+            for (int r = 0; r < M; ++r) {
+                unpack8(q[r][u], wv);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) acc[r] += hv[e] * wv[e];
+            }
+        }
+    };
+    auto rows = [&](auto MC) {
+        constexpr int M = decltype(MC)::value, U = M == 1 ? 8 : M <= 3 ? 4 : 2;
+        int k = 0;
+        for (; k + 512 * U <= d; k += 512 * U) part(MC, std::integral_constant<int, U>{}, k + lane * 8);
+        if constexpr (U > 4)
+            for (; k + 2048 <= d; k += 2048) part(MC, std::integral_constant<int, 4>{}, k + lane * 8);
+        if constexpr (U > 2)
+            for (; k + 1024 <= d; k += 1024) part(MC, std::integral_constant<int, 2>{}, k + lane * 8);
+        for (k += lane * 8; k < d; k += 512) part(MC, std::integral_constant<int, 1>{}, k);
+    };
+    if (n == 1) rows(std::integral_constant<int, 1>{});
+    else if (n == 2) rows(std::integral_constant<int, 2>{});
+    else if (n == 3) rows(std::integral_constant<int, 3>{});
+    else if (n == 4) rows(std::integral_constant<int, 4>{});
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const float v = wave_sum(acc[r]);
+        if (lane == 0 && r < n) z[wave + kRouteWaves * r] = v + (bias != nullptr ? bias[wave + kRouteWaves * r] : 0.f);
+    }
+    __syncthreads();
+    if (wave == 0) select_any<FORM>(z, idx + t * c.top, wt + t * c.top, c, sc, okg);
 }
 
 // Gated experts: per token sum_k weight_k * W_down,e ( g sigmoid(slope g) (u + shift) ), g = min(W_gate,e h, limit),
@@ -304,12 +389,22 @@ __global__ void __launch_bounds__(256) moe_glu_token_kernel(const T* __restrict_
 
 void launch_hy_rowdot(const void*, const void*, const float*, float*, int, int, int, bool, hipStream_t);
 
-// z: float [T, N] scratch for the router logits (the few-row float32-output projection, then the selection)
+// z: float [T, N] scratch for the router logits (the few-row float32-output projection, then the selection); not touched where one launch does both
+template <int FORM>
+static void moe_route(const void* h, const void* w, const float* bias, float* z, int32_t* idx, float* wt, int T, int d, const hy::Choice& c, bool f32,
+                      hipStream_t s) {
+    if (T == 0) return;
+    if (!f32 && T <= 256 && c.N <= hy::kRouteN && d % 8 == 0 && hy::aligned16(h, w)) {
+        hy::moe_route_token_kernel<FORM><<<T, 64 * hy::kRouteWaves, 0, s>>>((const uint16_t*)h, (const uint16_t*)w, bias, idx, wt, d, c);
+        return;
+    }
+    launch_hy_rowdot(h, w, bias, z, T, d, c.N, f32, s);
+    hy::moe_select_kernel<FORM><<<(T + 3) / 4, 256, 0, s>>>(z, idx, wt, T, c);
+}
+
 void launch_hy_moe_route(const void* h, const void* w, const float* corr, float* z, int32_t* idx, float* wt, int T, int d,
                          int N, int top, bool f32, hipStream_t s) {
-    if (T == 0) return;
-    launch_hy_rowdot(h, w, nullptr, z, T, d, N, f32, s);
-    hy::moe_select_kernel<<<(T + 3) / 4, 256, 0, s>>>(z, corr, idx, wt, T, N, top);
+    moe_route<hy::kSoftmax>(h, w, nullptr, z, idx, wt, T, d, {corr, N, top, 0, 0, 0.f}, f32, s);
 }
 
 void launch_hy_moe_ffn_token(const void* h, const int32_t* idx, const float* wt, const void* w_up, const void* w_down,
@@ -330,17 +425,13 @@ void launch_hy_moe_ffn_token(const void* h, const int32_t* idx, const float* wt,
 // z: float [T, N] scratch for the router logits (bias added by the projection), N <= 256
 void launch_hy_moe_route_topk(const void* h, const void* w, const float* bias, float* z, int32_t* idx, float* wt, int T,
                               int d, int N, int top, bool f32, hipStream_t s) {
-    if (T == 0) return;
-    launch_hy_rowdot(h, w, bias, z, T, d, N, f32, s);
-    hy::moe_select_topk_kernel<<<(T + 3) / 4, 256, 0, s>>>(z, idx, wt, T, N, top);
+    moe_route<hy::kTopk>(h, w, bias, z, idx, wt, T, d, {nullptr, N, top, 0, 0, 0.f}, f32, s);
 }
 
 // z: float [T, N] scratch for the router logits, N <= 256, groups <= 64, top <= 64
 void launch_hy_moe_route_group(const void* h, const void* w, float* z, int32_t* idx, float* wt, int T, int d, int N,
                                int top, int ng, int keep, float scale, bool f32, hipStream_t s) {
-    if (T == 0) return;
-    launch_hy_rowdot(h, w, nullptr, z, T, d, N, f32, s);
-    hy::moe_select_group_kernel<<<(T + 3) / 4, 256, 0, s>>>(z, idx, wt, T, N, top, ng, keep, scale);
+    moe_route<hy::kGroups>(h, w, nullptr, z, idx, wt, T, d, {nullptr, N, top, ng, keep, scale}, f32, s);
 }
 
 void launch_hy_moe_glu_token(const void* h, const int32_t* idx, const float* wt, const void* w_gu, const void* w_down,

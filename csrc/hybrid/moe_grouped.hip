@@ -1,7 +1,7 @@
 // moe_grouped.hip — the experts of a mixture-of-experts layer as two grouped MFMA GEMMs (bfloat16), for any number of
 // tokens: every expert's weights are streamed once per tile of its tokens, never once per token.
 //
-//   align     (count and place kernels) counts the (token, choice) items of every expert with weights, gives each expert a
+//   align     (count and place kernels, or for few items the up GEMM itself) counts the (token, choice) items of every expert with weights, gives each expert a
 //             run of whole tiles in a sorted row space, and writes row -> item (or -1 for padding), item -> row
 //             and the tile -> expert table.  Everything stays on the device: the GEMM grids are sized for the worst
 //             case (items / tile + experts tiles) and surplus workgroups leave at once, so the host never learns the
@@ -159,15 +159,97 @@ __global__ void __launch_bounds__(1024) moe_place_kernel(const int32_t* __restri
     }
 }
 
-// The wave's outputs: NS x NM accumulator tiles of 16 weight rows by 16 tokens, from weight row n0 and token row m0 on.  Lane l
+// Placing inside the first product of few items: every workgroup of 256 threads finds its tile's expert and items for itself (one that
+// takes the first rows of a tile's expert leaves them in meta for the launches behind it), so there is no launch in front of it.  Items keep their order
+// within an expert, so all workgroups agree.  Returns whether there is such a tile; rows: its TM items (-1: padding).
+// With the combining's loads in one go (below), us for the whole feed-forward: 8 experts of 1024 by 512, 1 to 64 tokens 20 -> 17.5; 16 of 2048 by
+// 1024 (gated), 1 and 64 tokens 28.0 -> 24.8, 42.7 -> 39.3; 32 of 4096 by 2048, 1 and 64 tokens 47.4 -> 42.2, 237 -> 230.
+constexpr int kPlaceItems = 512, kPlaceE = 64;
+struct PlaceLds {
+    int cnt[kPlaceItems / 64][kPlaceE];   // items of every run of 64 by expert
+    int start[kPlaceE + 1], expert;
+};
+template <int TM>
+__device__ __forceinline__ bool moe_place_tile(const int32_t* __restrict__ idx, int items, int E, int tile, bool writes, bool first, int maxTiles,
+                                               int32_t* __restrict__ meta, PlaceLds& p, int* rows) {
+    constexpr int RUNS = kPlaceItems / 64;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (int i = tid; i < RUNS * kPlaceE; i += 256) (&p.cnt[0][0])[i] = 0;
+    if (tid < TM) rows[tid] = -1;
+    int e[RUNS / 4], k[RUNS / 4];   // of the thread's items: expert, and rank within the run
+#pragma unroll
+    for (int j = 0; j < RUNS / 4; ++j) {
+        const int i = (wave + 4 * j) * 64 + lane;
+        const int v = i < items ? idx[i] : -1;
+        e[j] = v >= 0 && v < E ? v : -1;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < RUNS / 4; ++j) {
+        unsigned long long same = __ballot(e[j] >= 0);
+#pragma unroll
+        for (int b = 0; b < 6; ++b) {
+            const unsigned long long one = __ballot((e[j] >> b) & 1);
+            same &= ((e[j] >> b) & 1) ? one : ~one;
+        }
+        k[j] = __popcll(same & ((1ull << lane) - 1));
+        if (e[j] >= 0 && k[j] == 0) p.cnt[wave + 4 * j][e[j]] = __popcll(same);
+    }
+    __syncthreads();
+    if (wave == 0) {   // running sums: over the runs, then over the experts' tiles
+        int sum = 0;
+#pragma unroll
+        for (int r = 0; r < RUNS; ++r) {
+            const int n = p.cnt[r][lane];
+            p.cnt[r][lane] = sum;
+            sum += n;
+        }
+        const int n = (sum + TM - 1) / TM;
+        int to = n;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int v = __shfl_up(to, o, 64);
+            if (lane >= o) to += v;
+        }
+        p.start[lane] = to - n;
+        if (lane == 63) p.start[kPlaceE] = to;
+        if (tile >= to - n && tile < to) p.expert = lane;
+        if (lane == 63 && first) meta[0] = to;
+    }
+    __syncthreads();
+    const bool there = tile < p.start[kPlaceE];
+    const int mine = there ? p.expert : -1, lo = there ? (tile - p.start[mine]) * TM : 0;
+    int32_t* const row_item = meta + 1 + maxTiles;
+    int32_t* const item_row = row_item + maxTiles * TM;
+#pragma unroll
+    for (int j = 0; j < RUNS / 4; ++j) {
+        const int i = (wave + 4 * j) * 64 + lane;
+        if (i >= items) continue;
+        const int r = e[j] >= 0 ? p.cnt[wave + 4 * j][e[j]] + k[j] - lo : -1;
+        if (there && e[j] == mine && r >= 0 && r < TM) {
+            rows[r] = i;
+            if (writes) item_row[i] = tile * TM + r;
+        }
+        if (first && e[j] < 0) item_row[i] = -1;
+    }
+    __syncthreads();
+    if (there && writes) {
+        if (tid == 0) meta[1 + tile] = mine;
+        if (tid < TM) row_item[tile * TM + tid] = rows[tid];
+    }
+    return there;
+}
+
+// The wave's outputs: NS x NM accumulator tiles of 16 weight rows by 16 tokens, from weight row n0 and token row m0 on (item: the items of the lane's
+// tokens, -1: padding, not stored).  Lane l
 // holds D[n = 4 (l >> 4) + i][m = l & 15] of each = y[m][n .. n + 3].
 template <int ACT, int NS, int NM>
-__device__ __forceinline__ void moe_store(const f32x4 (&acc)[NS][NM], uint16_t* __restrict__ y, const int32_t* __restrict__ row_item,
+__device__ __forceinline__ void moe_store(const f32x4 (&acc)[NS][NM], uint16_t* __restrict__ y, const int (&item)[NM],
                                           int m0, int n0, int N, int lane, float limit, float slope, float shift) {
 #pragma unroll
     for (int t = 0; t < NM; ++t) {
         const int m = m0 + 16 * t + (lane & 15);
-        if (row_item[m] < 0) continue;
+        if (item[t] < 0) continue;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             const int row = n0 + 16 * s;   // first weight row of the block
@@ -198,20 +280,34 @@ __device__ __forceinline__ void moe_store(const f32x4 (&acc)[NS][NM], uint16_t* 
 
 // The tiles there are go to the XCDs in contiguous runs (their L2s then share rows of x and w); a launch of small tiles is
 // bound by the weights' bytes and spreads them over all.
-template <int TM, bool GATHER, int ACT>
+template <int TM, bool GATHER, int ACT, bool PLACE>
 __global__ void __launch_bounds__(256, 2) moe_gemm_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
-                                                          uint16_t* __restrict__ y, const int32_t* __restrict__ meta,
+                                                          uint16_t* __restrict__ y, int32_t* __restrict__ meta,
                                                           int maxTiles, int top, int N, int K, float limit, float slope,
-                                                          float shift) {
+                                                          float shift, const int32_t* __restrict__ idx, int items, int E) {
     using C = Tile<TM>;
     constexpr int ST = C::ST, BK = 64;
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-    const int nt = N / C::TN, used = meta[0];
-    if ((int)blockIdx.x >= used * nt) return;
-    const int id = TM == 128 ? xcd_remap(blockIdx.x, used * nt) : (int)blockIdx.x;
-    const int tile = id / nt, tn = id - tile * nt;
-    const int e = meta[1 + tile];
-    const int32_t* row_item = meta + 1 + maxTiles;
+    const int nt = N / C::TN;
+    int tile, tn, e;
+    const int32_t* row_item;
+    if constexpr (PLACE) {   // (TM == 32)
+        tile = blockIdx.x / nt;
+        tn = blockIdx.x - tile * nt;
+        PlaceLds& place = *reinterpret_cast<PlaceLds*>(smem);   // (in the ring's memory: two workgroups' rings fill the CU's)
+        int* const own = reinterpret_cast<int*>(smem + sizeof(PlaceLds));
+        if (!moe_place_tile<TM>(idx, items, E, tile, tn == 0, blockIdx.x == 0, maxTiles, meta, place, own)) return;
+        e = place.expert;
+        row_item = own - tile * TM;
+    } else {
+        const int used = meta[0];
+        if ((int)blockIdx.x >= used * nt) return;
+        const int id = TM == 128 ? xcd_remap(blockIdx.x, used * nt) : (int)blockIdx.x;
+        tile = id / nt;
+        tn = id - tile * nt;
+        e = meta[1 + tile];
+        row_item = meta + 1 + maxTiles;
+    }
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int m0 = tile * TM;
     const uint16_t* we = w + (int64_t)e * N * K;
@@ -232,6 +328,16 @@ __global__ void __launch_bounds__(256, 2) moe_gemm_kernel(const uint16_t* __rest
         }
         xsrc[i] = x + xr * K + c * 8;
     }
+    const int wn = wave / C::WX, wm = wave % C::WX;
+    int item[C::NM];   // of the lane's outputs
+    auto items_of = [&]() {
+#pragma unroll
+        for (int t = 0; t < C::NM; ++t) item[t] = row_item[m0 + 16 * (C::NM * wm + t) + (lane & 15)];
+    };
+    if constexpr (PLACE) {
+        items_of();
+        __syncthreads();   // the ring's memory is read
+    }
     auto issue = [&](int kt) {
         unsigned char* st = smem + (kt % ST) * (C::W + C::X);
 #pragma unroll
@@ -241,7 +347,6 @@ __global__ void __launch_bounds__(256, 2) moe_gemm_kernel(const uint16_t* __rest
         for (int i = 0; i < C::XP; ++i)
             __builtin_amdgcn_global_load_lds((gbl_ptr_t)(xsrc[i] + kt * BK), (lds_ptr_t)(st + C::W + (C::XP * wave + i) * 1024), 16, 0, 0);
     };
-    const int wn = wave / C::WX, wm = wave % C::WX;
     f32x4 acc[C::NS][C::NM];
 #pragma unroll
     for (int s = 0; s < C::NS; ++s)
@@ -275,7 +380,8 @@ __global__ void __launch_bounds__(256, 2) moe_gemm_kernel(const uint16_t* __rest
                     acc[s][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], b[t], acc[s][t], 0, 0, 0);
         }
     }
-    moe_store<ACT, C::NS, C::NM>(acc, y, row_item, m0 + 16 * C::NM * wm, tn * C::TN + C::TN / 2 * wn, N, lane, limit, slope, shift);
+    if constexpr (!PLACE) items_of();
+    moe_store<ACT, C::NS, C::NM>(acc, y, item, m0 + 16 * C::NM * wm, tn * C::TN + C::TN / 2 * wn, N, lane, limit, slope, shift);
 }
 
 // The 256 x 256 tile (x and one expert's weights below 4 and 2 GiB; weight rows past the end repeat the last one): a workgroup per CU walks
@@ -366,22 +472,35 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(const uint16_t* __rest
                                                           const int32_t* __restrict__ item_row, uint16_t* __restrict__ out,
                                                           int d, int top, int E, int identity) {
     const int64_t t = blockIdx.x;
-    for (int c = threadIdx.x * 8; c < d; c += 256 * 8) {
-        float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        for (int k = 0; k < top; ++k) {
-            const int e = idx[t * top + k], r = item_row[t * top + k];
-            const float g = wt[t * top + k];
-            if (r < 0 && !(identity && e >= E)) continue;
-            const uint16_t* src = r < 0 ? h + t * d + c : yrows + (int64_t)r * d + c;
-            const u16x8 v = *reinterpret_cast<const u16x8*>(src);
+    const int c = (blockIdx.y * 256 + threadIdx.x) * 8;
+    if (c >= d) return;
+    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    constexpr int U = 4;   // choices whose numbers, then rows, are under way together (one after the other: 6.7 us for 64 tokens of 4096)
+    for (int k0 = 0; k0 < top; k0 += U) {
+        int e[U], r[U];
+        float g[U];
+        u16x8 v[U];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) acc[j] += g * bf2f(v[j]);
+        for (int u = 0; u < U; ++u) {
+            const int64_t i = t * top + min(k0 + u, top - 1);
+            e[u] = idx[i];
+            r[u] = item_row[i];
+            g[u] = wt[i];
         }
-        u16x8 o;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) o[j] = f2bf(acc[j]);
-        *reinterpret_cast<u16x8*>(out + t * d + c) = o;
+        for (int u = 0; u < U; ++u)   // (a choice that is nobody's reads the token's own row and adds nothing)
+            v[u] = *reinterpret_cast<const u16x8*>(r[u] < 0 ? h + t * d + c : yrows + (int64_t)r[u] * d + c);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (k0 + u >= top || (r[u] < 0 && !(identity && e[u] >= E))) continue;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[j] += g[u] * bf2f(v[u][j]);
+        }
     }
+    u16x8 o;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = f2bf(acc[j]);
+    *reinterpret_cast<u16x8*>(out + t * d + c) = o;
 }
 
 }  // namespace hy
@@ -414,9 +533,9 @@ int64_t hy_moe_meta_ints(int items, int E, int tm) {
     return 1 + n + n * tm + items + (int64_t)moe_align_wgs(items) * E;
 }
 
-template <int TM, bool GATHER, int ACT>
-static void moe_gemm(const uint16_t* x, int64_t rows, const uint16_t* w, uint16_t* y, const int32_t* meta, int maxTiles, int top, int N, int K,
-                     float limit, float slope, float shift, hipStream_t s) {
+template <int TM, bool GATHER, int ACT, bool PLACE = false>
+static void moe_gemm(const uint16_t* x, int64_t rows, const uint16_t* w, uint16_t* y, int32_t* meta, int maxTiles, int top, int N, int K,
+                     float limit, float slope, float shift, hipStream_t s, const int32_t* idx = nullptr, int items = 0, int E = 0) {
     if constexpr (TM == 256) {
         const auto kern = hy::moe_gemm256_kernel<GATHER, ACT>;
         constexpr int lds = kSlabLds;
@@ -424,11 +543,11 @@ static void moe_gemm(const uint16_t* x, int64_t rows, const uint16_t* w, uint16_
         (void)once;
         kern<<<kSlabCUs, 256, lds, s>>>(x, (uint32_t)(rows * K * 2), w, y, meta, maxTiles, top, N, K, limit, slope, shift);
     } else {
-        const auto kern = hy::moe_gemm_kernel<TM, GATHER, ACT>;
+        const auto kern = hy::moe_gemm_kernel<TM, GATHER, ACT, PLACE>;
         constexpr int lds = hy::Tile<TM>::lds;
         static const hipError_t once = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         (void)once;
-        kern<<<maxTiles * (N / hy::Tile<TM>::TN), 256, lds, s>>>(x, w, y, meta, maxTiles, top, N, K, limit, slope, shift);
+        kern<<<maxTiles * (N / hy::Tile<TM>::TN), 256, lds, s>>>(x, w, y, meta, maxTiles, top, N, K, limit, slope, shift, idx, items, E);
     }
 }
 
@@ -441,16 +560,25 @@ static void moe_grouped(const uint16_t* h, const int32_t* idx, const float* wt, 
     const int items = T * top, maxTiles = hy_moe_max_tiles(items, E, TM);
     const int nwg = moe_align_wgs(items);
     int32_t* item_row = meta + 1 + maxTiles + maxTiles * TM;
-    if (nwg > 1) hy::moe_count_kernel<<<nwg, 1024, 0, s>>>(idx, items, E, item_row + items, item_row);
-    hy::moe_place_kernel<<<nwg, 1024, 0, s>>>(idx, items, E, TM, maxTiles, meta);
-    moe_gemm<TM, true, ACT>(h, T, w_up, z, meta, maxTiles, top, ACT == hy::kActGlu ? 2 * F : F, d, limit, slope, shift, s);
+    const int up = ACT == hy::kActGlu ? 2 * F : F;
+    bool placed = false;
+    if constexpr (TM == 32)
+        if (items <= hy::kPlaceItems && E <= hy::kPlaceE) {
+            moe_gemm<TM, true, ACT, true>(h, T, w_up, z, meta, maxTiles, top, up, d, limit, slope, shift, s, idx, items, E);
+            placed = true;
+        }
+    if (!placed) {
+        if (nwg > 1) hy::moe_count_kernel<<<nwg, 1024, 0, s>>>(idx, items, E, item_row + items, item_row);
+        hy::moe_place_kernel<<<nwg, 1024, 0, s>>>(idx, items, E, TM, maxTiles, meta);
+        moe_gemm<TM, true, ACT>(h, T, w_up, z, meta, maxTiles, top, up, d, limit, slope, shift, s);
+    }
     moe_gemm<TM, false, -1>(z, (int64_t)maxTiles * TM, w_down, yrows, meta, maxTiles, top, d, F, 0.f, 0.f, 0.f, s);
-    hy::moe_combine_kernel<<<T, 256, 0, s>>>(h, yrows, idx, wt, item_row, out, d, top, E, ACT != hy::kActGlu);
+    hy::moe_combine_kernel<<<dim3(T, (d + 2047) / 2048), 256, 0, s>>>(h, yrows, idx, wt, item_row, out, d, top, E, ACT != hy::kActGlu);
 }
 
 // no expert chosen: the sum of nothing
 static void moe_no_choice(const uint16_t* h, uint16_t* out, int T, int d, hipStream_t s) {
-    hy::moe_combine_kernel<<<T, 256, 0, s>>>(h, nullptr, nullptr, nullptr, nullptr, out, d, 0, 0, 0);
+    hy::moe_combine_kernel<<<dim3(T, (d + 2047) / 2048), 256, 0, s>>>(h, nullptr, nullptr, nullptr, nullptr, out, d, 0, 0, 0);
 }
 
 void launch_hy_moe_grouped(const uint16_t* h, const int32_t* idx, const float* wt, const uint16_t* w_up,
