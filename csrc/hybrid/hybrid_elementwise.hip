@@ -110,11 +110,8 @@ __global__ void __launch_bounds__(256) layer_norm_plain_kernel(const float* __re
 // in registers between the statistics and the write, 8 columns per lane and step.  W waves share a row (1: four rows per
 // workgroup, no barrier; 4: one row).  Bound by the bytes of y, x in and out and h: 8192 x 2048 takes 35 us (5.8 TB/s) where
 // three strided passes took 68; 64 rows of 4096 take 5 us, not 14.
-// SL: y is S float32 slices [rows, d] of a product, summed in order and rounded here (a launch of 3 - 5 us
-// less; decode steps of 64 rows at width 4096 968 -> 958 us, of 3 rows at width 1024 213 -> 206).
-template <int W, int NV, bool SL>
-__global__ void __launch_bounds__(256) layer_norm_vec_kernel(const uint16_t* __restrict__ y, const float* __restrict__ ys, int S,
-                                                             float* __restrict__ x, const float* __restrict__ w,
+template <int W, int NV>
+__global__ void __launch_bounds__(256) layer_norm_vec_kernel(const uint16_t* __restrict__ y, float* __restrict__ x, const float* __restrict__ w,
                                                              uint16_t* __restrict__ h, int rows, int d, float eps) {
     __shared__ float red[2][4];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -128,21 +125,7 @@ __global__ void __launch_bounds__(256) layer_norm_vec_kernel(const uint16_t* __r
     for (int j = 0; j < NV; ++j) {
         const int c = c0 + j * STEP;
         if (c < d) {
-            if constexpr (SL) {
-                const float* p = ys + row * d + c;
-                ld8f(p, v[j]);
-#pragma unroll 4
-                for (int k = 1; k < S; ++k) {
-                    float t[8];
-                    ld8f(p + (int64_t)k * rows * d, t);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) v[j][e] += t[e];
-                }
-#pragma unroll
-                for (int e = 0; e < 8; ++e) v[j][e] = bf2f(f2bf(v[j][e]));
-            } else {
-                ld8(y + row * d + c, v[j]);
-            }
+            ld8(y + row * d + c, v[j]);
             ld8f(x + row * d + c, xs[j]);
 #pragma unroll
             for (int e = 0; e < 8; ++e) s += v[j][e];
@@ -180,6 +163,58 @@ __global__ void __launch_bounds__(256) layer_norm_vec_kernel(const uint16_t* __r
             if (h != nullptr) st8(h + row * d + c, xs[j]);
         }
     }
+}
+
+// The same with y as S float32 slices [rows, d] of a product of few rows, summed in order and rounded here, d % 4 == 0 (a launch of 3 - 5 us less).  NT threads
+// take a row, 4 columns each NJ times, everything that they read on its way before the first sum, as in post_norm.hip's.  64 rows of 4096 in 8
+// slices 5.0 us with 256 threads, 4.3 so; of 8192 7.6 and 6.3.
+template <int NT, int NJ>
+__global__ void __launch_bounds__(NT) layer_norm_slices_kernel(const float* __restrict__ ys, int S, int64_t stride, float* __restrict__ x,
+                                                               const float* __restrict__ w, uint16_t* __restrict__ h, int d, float eps) {
+    __shared__ float red[2][NT / 64];
+    const int64_t at = blockIdx.x * (int64_t)d;
+    f32x4 v[NJ], xs[NJ], wv[NJ];
+    bool in[NJ];
+    auto total = [&](float a, int k) {
+        a = wave_sum(a);
+        if ((threadIdx.x & 63) == 0) red[k][threadIdx.x >> 6] = a;
+        __syncthreads();
+        a = 0.f;
+#pragma unroll
+        for (int i = 0; i < NT / 64; ++i) a += red[k][i];
+        return a;
+    };
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        in[j] = (int)(threadIdx.x + NT * j) * 4 < d;
+        const int i = min((int)(threadIdx.x + NT * j) * 4, d - 4);   // (past the row: its last columns again, not counted)
+        const float* const p = ys + at + i;
+        v[j] = *reinterpret_cast<const f32x4*>(p);
+        xs[j] = *reinterpret_cast<const f32x4*>(x + at + i);
+        wv[j] = *reinterpret_cast<const f32x4*>(w + i);
+#pragma unroll 4
+        for (int k = 1; k < S; ++k) v[j] += *reinterpret_cast<const f32x4*>(p + k * stride);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[j][e] = bf2f(f2bf(v[j][e]));
+        if (in[j]) s += (v[j][0] + v[j][1]) + (v[j][2] + v[j][3]);
+    }
+    const float mean = total(s, 0) / (float)d;
+    float q = 0.f;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+        if (in[j])
+#pragma unroll
+            for (int e = 0; e < 4; ++e) q += (v[j][e] - mean) * (v[j][e] - mean);
+    const float rstd = 1.f / sqrtf(total(q, 1) / (float)d + eps);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+        if (in[j]) {
+            const int64_t i = at + (threadIdx.x + NT * j) * 4;
+            const f32x4 o = xs[j] + (v[j] - mean) * rstd * wv[j];
+            *reinterpret_cast<f32x4*>(x + i) = o;
+            *reinterpret_cast<u16x4*>(h + i) = u16x4{f2bf(o[0]), f2bf(o[1]), f2bf(o[2]), f2bf(o[3])};
+        }
 }
 
 // out[t, n] = sum_k h[t, k] * w[n, k] (+ bias[n]) in float.  A workgroup takes TB tokens (their rows sit in LDS) and
@@ -373,10 +408,10 @@ void launch_hy_layer_norm(const void* y, bool y_f32, float* x, const float* w, v
     if (x != nullptr && !y_f32 && d % 8 == 0 && d <= 8192 && hy::aligned16(y, x, w, h)) {
         const uint16_t* yb = (const uint16_t*)y;
         uint16_t* hb = (uint16_t*)h;
-        if (d <= 1024) hy::layer_norm_vec_kernel<1, 2, false><<<(rows + 3) / 4, 256, 0, s>>>(yb, nullptr, 0, x, w, hb, rows, d, eps);
-        else if (d <= 2048) hy::layer_norm_vec_kernel<4, 1, false><<<rows, 256, 0, s>>>(yb, nullptr, 0, x, w, hb, rows, d, eps);
-        else if (d <= 4096) hy::layer_norm_vec_kernel<4, 2, false><<<rows, 256, 0, s>>>(yb, nullptr, 0, x, w, hb, rows, d, eps);
-        else hy::layer_norm_vec_kernel<4, 4, false><<<rows, 256, 0, s>>>(yb, nullptr, 0, x, w, hb, rows, d, eps);
+        if (d <= 1024) hy::layer_norm_vec_kernel<1, 2><<<(rows + 3) / 4, 256, 0, s>>>(yb, x, w, hb, rows, d, eps);
+        else if (d <= 2048) hy::layer_norm_vec_kernel<4, 1><<<rows, 256, 0, s>>>(yb, x, w, hb, rows, d, eps);
+        else if (d <= 4096) hy::layer_norm_vec_kernel<4, 2><<<rows, 256, 0, s>>>(yb, x, w, hb, rows, d, eps);
+        else hy::layer_norm_vec_kernel<4, 4><<<rows, 256, 0, s>>>(yb, x, w, hb, rows, d, eps);
     } else if (x != nullptr) {
         if (y_f32) hy::layer_norm_kernel<float, float, true><<<rows, 256, 0, s>>>((const float*)y, x, w, (float*)h, d, eps);
         else hy::layer_norm_kernel<uint16_t, uint16_t, true><<<rows, 256, 0, s>>>((const uint16_t*)y, x, w, (uint16_t*)h, d, eps);
@@ -391,9 +426,11 @@ void launch_hy_layer_norm(const void* y, bool y_f32, float* x, const float* w, v
 // d % 8 == 0, d <= 8192, everything on 16 bytes
 void launch_hy_layer_norm_slices(const float* ys, int S, float* x, const float* w, uint16_t* h, int rows, int d, float eps, hipStream_t s) {
     if (rows == 0) return;
-    if (d <= 2048) hy::layer_norm_vec_kernel<4, 1, true><<<rows, 256, 0, s>>>(nullptr, ys, S, x, w, h, rows, d, eps);
-    else if (d <= 4096) hy::layer_norm_vec_kernel<4, 2, true><<<rows, 256, 0, s>>>(nullptr, ys, S, x, w, h, rows, d, eps);
-    else hy::layer_norm_vec_kernel<4, 4, true><<<rows, 256, 0, s>>>(nullptr, ys, S, x, w, h, rows, d, eps);
+    const int64_t n = (int64_t)rows * d;
+    if (d <= 1024) hy::layer_norm_slices_kernel<256, 1><<<rows, 256, 0, s>>>(ys, S, n, x, w, h, d, eps);
+    else if (d <= 2048) hy::layer_norm_slices_kernel<512, 1><<<rows, 512, 0, s>>>(ys, S, n, x, w, h, d, eps);
+    else if (d <= 4096) hy::layer_norm_slices_kernel<1024, 1><<<rows, 1024, 0, s>>>(ys, S, n, x, w, h, d, eps);
+    else hy::layer_norm_slices_kernel<1024, 2><<<rows, 1024, 0, s>>>(ys, S, n, x, w, h, d, eps);
 }
 template <typename T>
 static void rowdot_t(const T* h, const T* w, const float* bias, float* out, int rows, int d, int n, hipStream_t s) {

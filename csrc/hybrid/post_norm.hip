@@ -34,38 +34,44 @@ struct Slices {
     int S;
     int64_t stride;
 };
-__device__ __forceinline__ f32x4 ld4s(const Slices& y, int64_t i) {
-    f32x4 v = *reinterpret_cast<const f32x4*>(y.p + i);
-#pragma unroll 4
-    for (int k = 1; k < y.S; ++k) v += *reinterpret_cast<const f32x4*>(y.p + k * y.stride + i);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = bf2f(f2bf(v[e]));
-    return v;
-}
-// x <- norm(alpha * x + y) * w, h <- x in bfloat16, as below with y in slices, d % 4 == 0, d <= 8192: a launch less than a sum before it (a
-// decode step of one row at width 1024 189 -> 185 us, of 8 rows 207 -> 204)
-__global__ void __launch_bounds__(256) rms_norm_slices_kernel(Slices y, float* __restrict__ x, const float* __restrict__ w,
-                                                              uint16_t* __restrict__ h, int d, float alpha, float eps) {
-    __shared__ float red[16];
+// x <- norm(alpha * x + y) * w, h <- x in bfloat16, as below with y in slices, d % 4 == 0: a launch less than a sum before it (a
+// decode step of one row at width 1024 189 -> 185 us, of 8 rows 207 -> 204).  NT threads take a row, 4 columns each NJ times, and everything that
+// they read is on its way before the first sum: a few rows are a chain of latencies (256 threads that took one piece after the other: 26 rows of
+// 4096 in 4 slices 5.8 us, now 3.3; 64 rows of 8192 in 8 10.2, now 5.8; one row of 1024 in 4 3.2, now 2.5).
+template <int NT, int NJ>
+__global__ void __launch_bounds__(NT) rms_norm_slices_kernel(Slices y, float* __restrict__ x, const float* __restrict__ w,
+                                                             uint16_t* __restrict__ h, int d, float alpha, float eps) {
+    __shared__ float red[NT / 64];
     const int64_t at = blockIdx.x * (int64_t)d;
-    f32x4 c[8];
+    f32x4 c[NJ], wv[NJ];
     float ss = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const int i = (threadIdx.x + 256 * j) * 4;
-        c[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (i < d) {
-            const f32x4 v = *reinterpret_cast<const f32x4*>(x + at + i) * alpha + ld4s(y, at + i);
-            c[j] = v;
-            ss += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
-        }
-    }
-    const float rstd = 1.f / sqrtf(block_sum(ss, red) / (float)d + eps);
+    for (int j = 0; j < NJ; ++j) {
+        const int i = min((int)(threadIdx.x + NT * j) * 4, d - 4);   // (past the row: its last columns again, not counted)
+        const float* const p = y.p + at + i;
+        f32x4 v = *reinterpret_cast<const f32x4*>(p);
+        c[j] = *reinterpret_cast<const f32x4*>(x + at + i);
+        wv[j] = *reinterpret_cast<const f32x4*>(w + i);
+#pragma unroll 4
+        for (int k = 1; k < y.S; ++k) v += *reinterpret_cast<const f32x4*>(p + k * y.stride);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const int i = (threadIdx.x + 256 * j) * 4;
+        for (int e = 0; e < 4; ++e) v[e] = bf2f(f2bf(v[e]));
+        v = c[j] * alpha + v;
+        c[j] = v;
+        if ((int)(threadIdx.x + NT * j) * 4 < d) ss += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
+    }
+    ss = wave_sum(ss);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    float sum = 0.f;
+#pragma unroll
+    for (int k = 0; k < NT / 64; ++k) sum += red[k];
+    const float rstd = 1.f / sqrtf(sum / (float)d + eps);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const int i = (threadIdx.x + NT * j) * 4;
         if (i < d) {
-            const f32x4 v = c[j] * rstd * *reinterpret_cast<const f32x4*>(w + i);
+            const f32x4 v = c[j] * rstd * wv[j];
             *reinterpret_cast<f32x4*>(x + at + i) = v;
             st4<uint16_t>(h + at + i, v);
         }
@@ -294,7 +300,11 @@ void launch_hy_rms_norm_rows(const float* x, const int64_t* rows, int total, con
 void launch_hy_rms_norm_slices(const float* ys, int S, float* x, const float* w, uint16_t* h, int rows, int d, float alpha, float eps,
                                hipStream_t s) {
     if (rows == 0) return;
-    hy::rms_norm_slices_kernel<<<rows, 256, 0, s>>>(hy::Slices{ys, S, (int64_t)rows * d}, x, w, h, d, alpha, eps);
+    const hy::Slices y{ys, S, (int64_t)rows * d};   // (d <= 8192)
+    if (d <= 1024) hy::rms_norm_slices_kernel<256, 1><<<rows, 256, 0, s>>>(y, x, w, h, d, alpha, eps);
+    else if (d <= 2048) hy::rms_norm_slices_kernel<512, 1><<<rows, 512, 0, s>>>(y, x, w, h, d, alpha, eps);
+    else if (d <= 4096) hy::rms_norm_slices_kernel<1024, 1><<<rows, 1024, 0, s>>>(y, x, w, h, d, alpha, eps);
+    else hy::rms_norm_slices_kernel<1024, 2><<<rows, 1024, 0, s>>>(y, x, w, h, d, alpha, eps);
 }
 
 // ldg, ldy: row strides of gu and y
