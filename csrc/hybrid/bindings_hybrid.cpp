@@ -112,6 +112,13 @@ int hy_rglru_chunks(int);
 void launch_hy_rglru_scan(const void*, const float*, const float*, float, const void*, int, int, const int32_t*,
                           const int32_t*, const int32_t*, float*, float*, float*, void*, int, int, int, int, int, bool,
                           hipStream_t);
+bool hy_state_mix_ok(int, int, int);
+void launch_hy_delta_step(const uint16_t*, int, int, int, int, int, const float*, const float*, const float*, const int32_t*, const int32_t*,
+                          const int32_t*, uint16_t*, int, float*, const float*, uint16_t*, int, int, int, int, int, float, float, hipStream_t);
+void launch_hy_rows_step(const uint16_t*, int, int, int, int, int, const float*, const float*, const float*, int, float, const int32_t*, const int32_t*,
+                         const int32_t*, float*, const float*, uint16_t*, int, int, int, int, float, float, hipStream_t);
+void launch_hy_mlstm_step(const uint16_t*, int, int, const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*, float*, const float*,
+                          uint16_t*, int, int, int, int, float, float, hipStream_t);
 void launch_hy_moe_route_group(const void*, const void*, float*, int32_t*, float*, int, int, int, int, int, int, float, bool,
                                hipStream_t);
 }  // namespace chronos
@@ -655,6 +662,74 @@ void hy_decay_pow(Tensor& z, double p) {
     chronos::launch_hy_decay_pow(z.data_ptr<float>(), z.numel(), (float)p, stream());
 }
 
+// ---- recurrent mixers of decode rows in one launch (state_mix.hip) ----
+static bool on16(const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
+bool hy_state_mix_ok(int64_t D, int64_t Dv, int64_t heads_per_key, int64_t cols) {
+    return cols % 4 == 0 && chronos::hy_state_mix_ok((int)std::min<int64_t>(D, 1 << 20), (int)std::min<int64_t>(Dv, 1 << 20), (int)std::min<int64_t>(heads_per_key, 1 << 20));
+}
+// what the three have in common; returns y [T, H Dv]
+static Tensor mix_check(const Tensor& proj, const Tensor& q_start, const Tensor& pos0, const Tensor& slots, const Tensor& S, int64_t HK, int64_t H,
+                        int64_t D, int64_t Dv, int64_t g_off, const Tensor& w) {
+    need(proj.scalar_type() == at::kBFloat16 && proj.dim() == 2 && proj.is_contiguous() && proj.is_cuda(), "state step: proj [T, C] bf16");
+    need(HK >= 1 && H >= 1 && H % HK == 0 && hy_state_mix_ok(D, Dv, H / HK, proj.size(1)), "state step: sizes");
+    need(2 * HK * D + H * Dv <= proj.size(1) && g_off >= 0 && g_off % 4 == 0 && g_off + H * Dv <= proj.size(1) && proj.size(1) < (1LL << 31), "state step: column ranges");
+    i32(q_start, "state step: q_start"); i32(pos0, "state step: pos0"); i32(slots, "state step: slots");
+    need(q_start.numel() == slots.numel() + 1 && pos0.numel() == slots.numel(), "state step: q_start [B+1], pos0 [B], slots [B]");
+    flt(S, "state step: S"); flt(w, "state step: w");
+    need(S.dim() == 4 && S.size(1) == H && S.size(2) == D && S.size(3) == Dv && w.numel() == H * Dv, "state step: S [NS, H, D, Dv], w [H Dv]");
+    need((reinterpret_cast<uintptr_t>(proj.data_ptr()) & 7) == 0 && on16(S) && on16(w), "state step: alignment");
+    return at::empty({proj.size(0), H * Dv}, proj.options());
+}
+static const uint16_t* mix_bf(const Tensor& t) { return reinterpret_cast<const uint16_t*>(t.data_ptr()); }
+
+Tensor hy_delta_step(const Tensor& proj, const Tensor& taps, const Tensor& ab, const Tensor& a_log, const Tensor& q_start, const Tensor& pos0,
+                     const Tensor& slots, Tensor& hist, Tensor& S, int64_t HK, int64_t H, int64_t D, int64_t Dv, double q_mul, int64_t g_off,
+                     const Tensor& w, double eps) {
+    c10::hip::HIPGuardMasqueradingAsCUDA g(proj.device());
+    Tensor y = mix_check(proj, q_start, pos0, slots, S, HK, H, D, Dv, g_off, w);
+    const int64_t T = proj.size(0), C = 2 * HK * D + H * Dv;
+    flt(taps, "delta_step: taps"); flt(ab, "delta_step: ab"); flt(a_log, "delta_step: A_log");
+    need(taps.dim() == 2 && taps.size(0) == C && taps.size(1) == 4 && on16(taps) && ab.numel() == T * 2 * H && a_log.numel() == H, "delta_step: taps [C, 4], ab [T, 2H], A_log [H]");
+    need(hist.scalar_type() == at::kBFloat16 && hist.is_contiguous() && hist.dim() == 3 && hist.size(0) == S.size(0) && hist.size(1) == 3 && hist.size(2) == C &&
+         (reinterpret_cast<uintptr_t>(hist.data_ptr()) & 7) == 0, "delta_step: history [NS, 3, C] bf16");
+    if (T > 0)
+        chronos::launch_hy_delta_step(mix_bf(proj), (int)proj.size(1), 0, (int)(HK * D), (int)(2 * HK * D), (int)g_off, taps.data_ptr<float>(), ab.data_ptr<float>(),
+                                      a_log.data_ptr<float>(), q_start.data_ptr<int32_t>(), pos0.data_ptr<int32_t>(), slots.data_ptr<int32_t>(),
+                                      reinterpret_cast<uint16_t*>(hist.data_ptr()), (int)C, S.data_ptr<float>(), w.data_ptr<float>(),
+                                      reinterpret_cast<uint16_t*>(y.data_ptr()), (int)slots.numel(), (int)HK, (int)H, (int)D, (int)Dv, (float)q_mul, (float)eps, stream());
+    return y;
+}
+
+Tensor hy_rows_step(const Tensor& proj, const Tensor& low, const Tensor& w2, const Tensor& b2, double p, const Tensor& q_start, const Tensor& pos0,
+                    const Tensor& slots, Tensor& S, int64_t H, int64_t D, int64_t Dv, double q_mul, int64_t g_off, const Tensor& w, double eps) {
+    c10::hip::HIPGuardMasqueradingAsCUDA g(proj.device());
+    Tensor y = mix_check(proj, q_start, pos0, slots, S, H, H, D, Dv, g_off, w);
+    const int64_t T = proj.size(0);
+    flt(low, "rows_step: low"); flt(w2, "rows_step: w2"); flt(b2, "rows_step: b2");
+    need(low.dim() == 2 && low.size(0) == T && w2.dim() == 2 && w2.size(0) == low.size(1) && w2.size(1) == H * D && b2.numel() == H * D, "rows_step: low [T, R], w2 [R, H D], b2 [H D]");
+    if (T > 0)
+        chronos::launch_hy_rows_step(mix_bf(proj), (int)proj.size(1), 0, (int)(H * D), (int)(2 * H * D), (int)g_off, low.data_ptr<float>(), w2.data_ptr<float>(),
+                                     b2.data_ptr<float>(), (int)low.size(1), (float)p, q_start.data_ptr<int32_t>(), pos0.data_ptr<int32_t>(),
+                                     slots.data_ptr<int32_t>(), S.data_ptr<float>(), w.data_ptr<float>(), reinterpret_cast<uint16_t*>(y.data_ptr()),
+                                     (int)slots.numel(), (int)H, (int)D, (int)Dv, (float)q_mul, (float)eps, stream());
+    return y;
+}
+
+Tensor hy_mlstm_step(const Tensor& proj, const Tensor& gate_pre, const Tensor& q_start, const Tensor& pos0, const Tensor& slots, Tensor& S, Tensor& n,
+                     Tensor& m, int64_t H, int64_t D, int64_t Dv, double cap, int64_t g_off, const Tensor& w, double eps) {
+    c10::hip::HIPGuardMasqueradingAsCUDA g(proj.device());
+    Tensor y = mix_check(proj, q_start, pos0, slots, S, H, H, D, Dv, g_off, w);
+    const int64_t T = proj.size(0);
+    flt(gate_pre, "mlstm_step: gate_pre"); flt(n, "mlstm_step: n"); flt(m, "mlstm_step: m");
+    need(gate_pre.dim() == 2 && gate_pre.size(0) == T && gate_pre.size(1) == 2 * H, "mlstm_step: gate_pre [T, 2H]");
+    need(n.numel() == S.size(0) * H * D && m.numel() == S.size(0) * H, "mlstm_step: n [NS, H, D], m [NS, H]");
+    if (T > 0)
+        chronos::launch_hy_mlstm_step(mix_bf(proj), (int)proj.size(1), (int)g_off, gate_pre.data_ptr<float>(), q_start.data_ptr<int32_t>(), pos0.data_ptr<int32_t>(),
+                                      slots.data_ptr<int32_t>(), S.data_ptr<float>(), n.data_ptr<float>(), m.data_ptr<float>(), w.data_ptr<float>(),
+                                      reinterpret_cast<uint16_t*>(y.data_ptr()), (int)slots.numel(), (int)H, (int)D, (int)Dv, (float)cap, (float)eps, stream());
+    return y;
+}
+
 Tensor hy_low_rank_decay(const Tensor& a, const Tensor& w, const Tensor& b, double p) {
     c10::hip::HIPGuardMasqueradingAsCUDA g(a.device());
     flt(a, "low_rank_decay: float32 a"); flt(w, "low_rank_decay: float32 w"); flt(b, "low_rank_decay: float32 b");
@@ -1180,6 +1255,13 @@ Tensor hy_unrotate_gate(const Tensor& o, const Tensor& pos, const c10::optional<
 
 TORCH_LIBRARY_FRAGMENT(chronos, m) {
     m.def("hy_embed(Tensor ids, Tensor table, float scale=1.0) -> Tensor");
+    m.def("hy_state_mix_ok(int D, int Dv, int heads_per_key, int cols) -> bool", &hy_state_mix_ok);
+    m.def("hy_delta_step(Tensor proj, Tensor taps, Tensor ab, Tensor a_log, Tensor q_start, Tensor pos0, Tensor slots, Tensor(a!) hist, Tensor(b!) S, "
+          "int HK, int H, int D, int Dv, float q_mul, int g_off, Tensor w, float eps) -> Tensor");
+    m.def("hy_rows_step(Tensor proj, Tensor low, Tensor w2, Tensor b2, float p, Tensor q_start, Tensor pos0, Tensor slots, Tensor(a!) S, int H, int D, "
+          "int Dv, float q_mul, int g_off, Tensor w, float eps) -> Tensor");
+    m.def("hy_mlstm_step(Tensor proj, Tensor gate_pre, Tensor q_start, Tensor pos0, Tensor slots, Tensor(a!) S, Tensor(b!) n, Tensor(c!) m, int H, "
+          "int D, int Dv, float cap, int g_off, Tensor w, float eps) -> Tensor");
     m.def("hy_embed_both(Tensor ids, Tensor table, float scale) -> (Tensor, Tensor)");
     m.def("hy_embed_start(Tensor ids, Tensor table, float scale, bool both, Tensor pos, Tensor q_start) -> (Tensor, Tensor, Tensor)");
     m.def("hy_layer_norm(Tensor x, Tensor w, float eps, bool out_f32, Tensor? rows=None) -> Tensor");
@@ -1263,6 +1345,9 @@ TORCH_LIBRARY_FRAGMENT(chronos, m) {
 TORCH_LIBRARY_IMPL(chronos, CUDA, m) {
     m.impl("hy_embed", &hy_embed);
     m.impl("hy_embed_both", &hy_embed_both);
+    m.impl("hy_delta_step", &hy_delta_step);
+    m.impl("hy_rows_step", &hy_rows_step);
+    m.impl("hy_mlstm_step", &hy_mlstm_step);
     m.impl("hy_embed_start", &hy_embed_start);
     m.impl("hy_layer_norm", &hy_layer_norm);
     m.impl("hy_add_layer_norm", &hy_add_layer_norm);

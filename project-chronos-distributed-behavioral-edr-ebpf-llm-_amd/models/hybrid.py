@@ -863,6 +863,10 @@ class StepMeta:
 def mix_mlstm(model, li: int, spec: MLSTMSpec, w: dict, h, meta: StepMeta, cache: HybridCache):
     H, D, Dv = spec.heads, spec.dim, spec.vdim
     proj, gate_pre = hops.matmul_rowdot(h, w["w_proj"], w["w_if"], w["b_if"], w.get("joined"))
+    if hops.one_step_ok(proj, meta.max_q, D, Dv, 1, cache.S[li], w["norm"]):
+        y = hops.mlstm_step(proj, gate_pre, meta.q_start, meta.pos0, meta.slots, cache.S[li], cache.n[li], cache.m[li], H, D, Dv, spec.gate_cap,
+                            2 * H * D + H * Dv, w["norm"], model.cfg.norm_eps)
+        return model.last_product(y, w["w_o"])
     o = hops.mlstm_scan(proj, gate_pre, meta.q_start, meta.pos0, meta.slots, cache.S[li], cache.n[li], cache.m[li],
                         H, D, Dv, spec.gate_cap, meta.max_q)
     y = hops.mlstm_out(o, proj, 2 * H * D + H * Dv, w["norm"], model.cfg.norm_eps, model.act_dtype)
@@ -1040,6 +1044,10 @@ def mix_delta_rule(model, li: int, spec: DeltaRuleSpec, w: dict, h, meta: StepMe
     C = 2 * HK * D + H * Dv
     # q | k | v | g; decay and write-strength pre-activations, float32
     proj, ab = hops.matmul_rowdot(h, w["w_proj"], w["w_ab"], w["b_ab"], w.get("joined"))
+    if spec.conv == 4 and hops.one_step_ok(proj, meta.max_q, D, Dv, H // HK, cache.S[li], cache.hist[li], w["taps"], w["norm"]):
+        y = hops.delta_step(proj, w["taps"], ab, w["a_log"], meta.q_start, meta.pos0, meta.slots, cache.hist[li], cache.S[li], HK, H, D, Dv, D ** -0.5, C,
+                            w["norm"], model.cfg.norm_eps)
+        return model.last_product(y, w["w_o"])
     y = hops.short_conv(proj, w["taps"], meta.tok_seq, meta.q_start, meta.pos0, meta.slots, cache.hist[li], True, max_q=meta.max_q)
     qscale, kscale, decay, beta = hops.delta_prep(y, ab, w["a_log"], HK, H, D, D ** -0.5)
     o = hops.linear_scan(y, 0, HK * D, 2 * HK * D, qscale, kscale, 1.0, decay, beta, meta.q_start, meta.pos0,
@@ -1050,6 +1058,10 @@ def mix_delta_rule(model, li: int, spec: DeltaRuleSpec, w: dict, h, meta: StepMe
 def mix_gla(model, li: int, spec: GLASpec, w: dict, h, meta: StepMeta, cache: HybridCache):
     H, D, Dv = spec.heads, spec.dim, spec.vdim
     proj, low = hops.matmul_rowdot(h, w["w_proj"], w["w_a1"], None, w.get("joined"))   # q | k | v | g; the decay's latent
+    if hops.one_step_ok(proj, meta.max_q, D, Dv, 1, cache.S[li], w["norm"]):
+        o = hops.rows_step(proj, low, w["w_a2t"], w["b_a2"], 1.0 / spec.tau, meta.q_start, meta.pos0, meta.slots, cache.S[li], H, D, Dv, D ** -0.5,
+                           2 * H * D + H * Dv, w["norm"], model.cfg.norm_eps)
+        return _with_gate(model.last_product(o, w["w_o"]), proj, w)
     decay = hops.low_rank_decay(low, w["w_a2t"], w["b_a2"], 1.0 / spec.tau)           # float32 [T, H D]
     o = hops.linear_scan(proj, 0, H * D, 2 * H * D, None, None, D ** -0.5, decay, None, meta.q_start, meta.pos0,
                          meta.slots, cache.S[li], H, H, D, Dv, max_q=meta.max_q)

@@ -357,6 +357,29 @@ def linear_scan(proj, q_off: int, k_off: int, v_off: int, qscale, kscale, q_mul:
                            H, D, Dv, vscale)
 
 
+def one_step_ok(proj, max_q: int, D: int, Dv: int, heads_per_key: int, *operands) -> bool:
+    """May a recurrent mixer's part between its projections run as one launch (delta_step, rows_step, mlstm_step)?  For decode rows, max_q 1; ``operands``:
+    what it reads 16 bytes at a time."""
+    if max_q != 1 or not _gpu(proj) or proj.dtype != torch.bfloat16 or not proj.is_contiguous() or any(t.data_ptr() % 16 for t in (proj, *operands)):
+        return False
+    return _k().hy_state_mix_ok(D, Dv, heads_per_key, proj.shape[1])
+
+
+def delta_step(proj, taps, ab, a_log, q_start, pos0, slots, hist, S, HK: int, H: int, D: int, Dv: int, q_mul: float, g_off: int, w, eps: float):
+    """short_conv, delta_prep, linear_scan and head_norm_gate (SiLU gate) of q | k | v columns at 0 and a gate at g_off, 4 taps, where one_step_ok."""
+    return _k().hy_delta_step(proj, taps, ab, a_log, q_start, pos0, slots, hist, S, HK, H, D, Dv, q_mul, g_off, w, eps)
+
+
+def rows_step(proj, low, w2, b2, inv_tau: float, q_start, pos0, slots, S, H: int, D: int, Dv: int, q_mul: float, g_off: int, w, eps: float):
+    """low_rank_decay, linear_scan and head_norm_gate (SiLU gate) of q | k | v columns at 0 and a gate at g_off, where one_step_ok."""
+    return _k().hy_rows_step(proj, low, w2, b2, inv_tau, q_start, pos0, slots, S, H, D, Dv, q_mul, g_off, w, eps)
+
+
+def mlstm_step(proj, gate_pre, q_start, pos0, slots, S, n, m, H: int, D: int, Dv: int, cap: float, g_off: int, w, eps: float):
+    """mlstm_scan and mlstm_out, where one_step_ok."""
+    return _k().hy_mlstm_step(proj, gate_pre, q_start, pos0, slots, S, n, m, H, D, Dv, cap, g_off, w, eps)
+
+
 def head_norm_gate(o, src, g_off: int, w, eps: float, silu_gate: bool, act_dtype):
     if _gpu(o):
         return _k().hy_head_norm_gate(o, src, g_off, w, eps, silu_gate, _f32(act_dtype))
