@@ -11,6 +11,7 @@
 //                      memory straight into registers as B operands; both for the next step while the current one
 //                      multiplies.  C^T = W A^T in 16x16x32 MFMAs: a lane ends up with 4 neighbouring output columns
 //                      of one token (8-byte stores), which the gate multiplies in float.
+//   head_matmul_few    the same for up to 64 tokens.
 //   head_matmul        any sizes and types: 64 x 64 tiles on the vector ALUs, float accumulation.
 #include "hybrid_common.h"
 
@@ -108,6 +109,78 @@ __global__ void __launch_bounds__(256) head_matmul_mfma_kernel(
     }
 }
 
+// The same for few tokens: a workgroup of 8 waves takes 16 MT tokens and 16 NTL output columns of one head; the waves share K, 32 at a time, straight
+// from memory into operands, and meet in LDS.  Bound by one memory latency; above, K steps of 64 follow each other.  us, above and this, 32 heads: 128 columns of
+// K = 512, 6 tokens 6.4 and 3.5, 64 tokens 6.7 and 4.5, 128 6.9 and 6.9; 512 columns of K = 128, 6 tokens 3.5 and 3.1, 32 tokens 3.6 and 3.7, 64 4.0 and
+// 5.3: up to 16 tokens, and 64 where K is 256 and more.
+template <int MT, int NTL>
+__global__ void __launch_bounds__(512) head_matmul_few_kernel(
+        const uint16_t* __restrict__ a, int64_t lda, int64_t ha, const uint16_t* __restrict__ w,
+        uint16_t* __restrict__ out, int64_t ldo, int64_t ho, const uint16_t* __restrict__ gsrc, int64_t ldg, int T, int N,
+        int K, int vst) {
+    constexpr int P = MT * NTL, PW = (P + 7) / 8;
+    __shared__ __attribute__((aligned(16))) f32x4 red[8][P][64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, g = lane >> 4, r = lane & 15;
+    const int h = blockIdx.z, n0 = blockIdx.y * NTL * 16, t0 = blockIdx.x * 16 * MT;
+    const uint16_t *ar[MT], *wr[NTL];   // rows past the end repeat the last one and are not stored
+#pragma unroll
+    for (int m = 0; m < MT; ++m) ar[m] = a + (int64_t)min(t0 + 16 * m + r, T - 1) * lda + h * ha + 8 * g;
+#pragma unroll
+    for (int n = 0; n < NTL; ++n) wr[n] = w + ((int64_t)h * N + min(n0 + 16 * n + r, N - 1)) * K + 8 * g;
+    f32x4 acc[MT][NTL];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NTL; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = wv * 32; k0 < K; k0 += 512) {   // (two steps of a wave under way together)
+        bf16x8 af[2][MT], wf[2][NTL];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const bool ok = k0 + 256 * u + 8 * g < K;   // (K is a multiple of 8)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) af[u][m] = ok ? *reinterpret_cast<const bf16x8*>(ar[m] + k0 + 256 * u) : bf16x8{};
+#pragma unroll
+            for (int n = 0; n < NTL; ++n) wf[u][n] = ok ? *reinterpret_cast<const bf16x8*>(wr[n] + k0 + 256 * u) : bf16x8{};
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int n = 0; n < NTL; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][n], af[u][m], acc[m][n], 0, 0, 0);
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NTL; ++n) red[wv][m * NTL + n][lane] = acc[m][n];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PW; ++q) {
+        const int p = wv + 8 * q;
+        if (p >= P) return;
+        f32x4 v = red[0][p][lane];
+#pragma unroll
+        for (int u = 1; u < 8; ++u) v += red[u][p][lane];
+        // lane holds out[token r of tile p / NTL][column 16 (p % NTL) + 4 g + i]
+        const int t = t0 + 16 * (p / NTL) + r, c = n0 + 16 * (p % NTL) + 4 * g;
+        if (t >= T || c >= N) continue;
+        uint16_t* orow = out + (int64_t)t * ldo + h * ho;
+        const uint16_t* grow = gsrc != nullptr ? gsrc + (int64_t)t * ldg + (int64_t)h * N : nullptr;
+        if (vst && c + 3 < N) {
+            if (grow != nullptr) {
+                const u16x4 z = *reinterpret_cast<const u16x4*>(grow + c);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] *= sigmoidf_(bf2f(z[i]));
+            }
+            *reinterpret_cast<u16x4*>(orow + c) = u16x4{f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (c + i < N) orow[c + i] = f2bf(grow != nullptr ? v[i] * sigmoidf_(bf2f(grow[c + i])) : v[i]);
+        }
+    }
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256) head_matmul_kernel(const T* __restrict__ a, int64_t lda, int64_t ha,
                                                           const T* __restrict__ w, T* __restrict__ out, int64_t ldo,
@@ -158,7 +231,10 @@ void launch_hy_head_matmul(const void* a, int64_t lda, int64_t ha, const void* w
     if (!f32 && K % 8 == 0 && lda % 8 == 0 && ha % 8 == 0 && al(a, 16) && al(w, 16)) {
         const bool vst = ldo % 4 == 0 && ho % 4 == 0 && al(out, 8) && (gsrc == nullptr || (ldg % 4 == 0 && N % 4 == 0 && al(gsrc, 8)));
 #define HY_HM(MT, NTL) hy::head_matmul_mfma_kernel<MT, NTL><<<dim3((T + 64 * MT - 1) / (64 * MT), (N + 16 * NTL - 1) / (16 * NTL), H), 256, 0, s>>>((const uint16_t*)a, lda, ha, (const uint16_t*)w, (uint16_t*)out, ldo, ho, (const uint16_t*)gsrc, ldg, T, N, K, vst)
-        if (T <= 256) HY_HM(1, 4);
+#define HY_HF(MT, NTL) hy::head_matmul_few_kernel<MT, NTL><<<dim3((T + 16 * MT - 1) / (16 * MT), (N + 16 * NTL - 1) / (16 * NTL), H), 512, 0, s>>>((const uint16_t*)a, lda, ha, (const uint16_t*)w, (uint16_t*)out, ldo, ho, (const uint16_t*)gsrc, ldg, T, N, K, vst)
+        if (T <= 16) HY_HF(1, 2);
+        else if (T <= 64 && K >= 256) HY_HF(2, 2);
+        else if (T <= 256) HY_HM(1, 4);
         else if (N <= 64) HY_HM(2, 4);
         else HY_HM(2, 8);
 #undef HY_HM

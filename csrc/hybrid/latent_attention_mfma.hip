@@ -323,17 +323,25 @@ __global__ void __launch_bounds__(64 * NW) latent_attention_mfma_kernel(
         }
 }
 
-// one wave per (token, head) row: out = sum_z 2^(m_z - m) O_z / (sum_z 2^(m_z - m) l_z + 2^(sink log2 e - m)) * sigmoid(gate)
+// one wave per (token, head) row and 256 columns: out = sum_z 2^(m_z - m) O_z / (sum_z 2^(m_z - m) l_z + 2^(sink log2 e - m)) * sigmoid(gate)
 // (the partial maxima are in the base-2 domain: score * scale * log2 e).  Lane z holds
-// split z's maximum and sum (nsplit <= 16); a lane then sums 4 neighbouring columns over the splits, whose loads do not
-// depend on each other.
+// split z's maximum and sum (nsplit <= 64); a lane then sums 4 neighbouring columns over the splits.  16 splits' columns are on their way before
+// the maxima are looked at: a few rows are one memory latency, not one per four splits behind another: 6 rows of 8 heads in 13 splits 6.7 -> 3.6 us.
 __global__ void __launch_bounds__(256) latent_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                                              const float* __restrict__ gate, uint16_t* __restrict__ out,
                                                              int64_t rows, int rank, int nsplit,
                                                              const float* __restrict__ sink, int H) {
     const int lane = threadIdx.x & 63;
-    const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int nc = (rank + 255) / 256;
+    const int64_t it = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), r = it / nc;
     if (r >= rows) return;
+    const int c = (int)(it - r * nc) * 256 + lane * 4;    // (rank is a multiple of 16; lanes past it read its last columns)
+    const float* const po = part_o + r * nsplit * rank + min(c, rank - 4);
+    constexpr int U = 16;
+    f32x4 v[U];
+#pragma unroll
+    for (int z = 0; z < U; ++z)
+        if (z < nsplit) v[z] = *reinterpret_cast<const f32x4*>(po + (int64_t)z * rank);
     const float mz = lane < nsplit ? part_ml[(r * nsplit + lane) * 2] : -INFINITY;
     const float lz = lane < nsplit ? part_ml[(r * nsplit + lane) * 2 + 1] : 0.f;
     const float sk = sink != nullptr ? sink[r % H] * kLog2e : -INFINITY;
@@ -341,15 +349,13 @@ __global__ void __launch_bounds__(256) latent_combine_kernel(const float* __rest
     float e = mz == -INFINITY ? 0.f : exp2f(mz - m);   // (a split without a visible key adds nothing)
     const float l = wave_sum(e * lz) + (sink != nullptr ? exp2f(sk - m) : 0.f);
     e *= (gate != nullptr ? sigmoidf_(gate[r]) : 1.f) / l;
-    for (int c = lane * 4; c < rank; c += 256) {      // (rank is a multiple of 16)
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-        for (int z = 0; z < nsplit; ++z) {
-            const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(e), z));
-            acc += w * *reinterpret_cast<const f32x4*>(part_o + (r * nsplit + z) * rank + c);
-        }
-        *reinterpret_cast<u16x4*>(out + r * rank + c) = u16x4{f2bf(acc[0]), f2bf(acc[1]), f2bf(acc[2]), f2bf(acc[3])};
-    }
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int z = 0; z < U; ++z)
+        if (z < nsplit) acc += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(e), z)) * v[z];
+    for (int z = U; z < nsplit; ++z)
+        acc += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(e), z)) * *reinterpret_cast<const f32x4*>(po + (int64_t)z * rank);
+    if (c < rank) *reinterpret_cast<u16x4*>(out + r * rank + c) = u16x4{f2bf(acc[0]), f2bf(acc[1]), f2bf(acc[2]), f2bf(acc[3])};
 }
 
 }  // namespace hy
@@ -377,11 +383,14 @@ static void la_mfma_launch(const uint16_t* qa, const uint16_t* cache, const int3
 bool hy_latent_mfma_ok(int DK, int rank) { return !(DK % 8 || rank % 16 || DK > 576 || rank > 512 || rank > DK); }
 
 // Splits of the key range (flash-decoding) for a launch of `wgs` workgroups over contexts of at most max_ctx keys:
-// enough workgroups to cover the chip, at least 4 key tiles per split (2 behind a window, whose few tiles are all of the
-// walk), at most 16.
+// enough workgroups to cover the chip, at least one key tile per split (2 behind a window, whose few tiles are all of the
+// walk), at most 16.  A tile of a few rows is a chain of latencies, dearer than its partials: at least 4 tiles, 2 tiles and one, us with the combining,
+// 1 sequence of 700 keys, 8 heads of 288 columns 15.1, 12.1, 11.1, 32 heads of 576 30.8, 21.0, 17.8; 6 of about 200 12.2, 12.2, 11.0, 23.5, 20.5,
+// 17.7; 16 of about 700 15.3, 12.5, 11.2.  Not two splits: 1 of 120 keys 8.2, 9.4.  32 splits: 6 of about 2000, 32 heads 24.1 -> 26.2.
 int hy_latent_nsplit(int wgs, int max_ctx, bool windowed) {
     if (wgs >= 128) return 1;
-    int want = (256 + wgs - 1) / wgs, cap = max_ctx / ((windowed ? 2 : 4) * hy::MKT);
+    int want = (256 + wgs - 1) / wgs, cap = max_ctx / ((windowed ? 2 : 1) * hy::MKT);
+    if (!windowed && cap < 3) cap = 1;
     if (want > 16) want = 16;
     if (want > cap) want = cap;
     return want < 1 ? 1 : want;
@@ -419,7 +428,7 @@ bool launch_hy_latent_attention_mfma(const uint16_t* qa, const uint16_t* cache, 
 #undef HY_LAM_R
 #undef HY_LAM
     if (nsplit > 1)
-        hy::latent_combine_kernel<<<(unsigned)((total_rows + 3) / 4), 256, 0, s>>>(part_o, part_ml, gate, out, total_rows, rank, nsplit, sink, H);
+        hy::latent_combine_kernel<<<(unsigned)((total_rows * ((rank + 255) / 256) + 3) / 4), 256, 0, s>>>(part_o, part_ml, gate, out, total_rows, rank, nsplit, sink, H);
     return true;
 }
 
