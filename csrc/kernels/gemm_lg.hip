@@ -313,7 +313,18 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
 #pragma unroll
         for (int i = 4; i < 16; i += 4) t4 += (pv4[i] + pv4[i + 1]) + (pv4[i + 2] + pv4[i + 3]);
         float ss = (t4[0] + t4[1]) + (t4[2] + t4[3]);
-        for (int i = pv_vec ? 64 : 0; i < a.nparts_in; ++i) ss += pp[i];
+        int i = pv_vec ? 64 : 0;
+        if (pv_vec) {   // the rest in order, 64 on their way together (one behind the other, 256 partials: gate and up of 28672 x 4096, 2 - 32 rows 61 us, now 49; qkv and head likewise)
+            for (; i < a.nparts_in; i += 64) {
+#pragma unroll
+                for (int q = 0; q < 16; ++q)
+                    pv4[q] = i + 4 * q < a.nparts_in ? *reinterpret_cast<const f32x4*>(pp + i + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int q = 0; q < 16; ++q)
+                    if (i + 4 * q < a.nparts_in) ss = (((ss + pv4[q][0]) + pv4[q][1]) + pv4[q][2]) + pv4[q][3];
+            }
+        }
+        for (; i < a.nparts_in; ++i) ss += pp[i];
         if (lane < RPW) inv[prow] = rsqrtf(ss / (float)K + a.eps);
     }
 
