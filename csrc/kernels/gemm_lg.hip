@@ -64,10 +64,11 @@ __device__ __forceinline__ void lg_sched() {
 // One 1 KiB LDS-DMA piece through a buffer descriptor (base / size wave-uniform: kernel arguments): lane l's 16 bytes
 // from byte voff + soff of the buffer to LDS dst + 16 l; bytes past `bytes` read as zeros.  (A descriptor held in
 // a kernel-body variable made hipcc's host pass drop the kernel stubs; built here it is hoisted all the same.)
+template <int AUX = 0>
 __device__ __forceinline__ void lg_dma16(const void* base, int bytes, unsigned char* dst, uint32_t voff, int soff) {
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, bytes,
                                                                        0x00020000);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)dst, 16, voff, soff, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)dst, 16, voff, soff, 0, AUX);
 }
 
 // The same piece as inline asm (VAR 2): M0 = the LDS destination, written in the same statement that reads it, with the one
@@ -103,7 +104,11 @@ __device__ __forceinline__ int lg_swz64(int row) { return (4 - ((row >> 2) & 3))
 // lgkmcnt wait in front of it; the ring buffers it writes are disjoint from the ones being read by construction)
 // F8 (ring schedule only): W8A8 e4m3fn operands (PPArgs x / w hold the bytes), one 128-deep MFMA k-step per 128-B
 // stage row, y = (x W^T) * xsc[m] * wsc[n] in the epilogue (plain / SwiGLU)
-template <int WN, int XM, int RB, int ST, int MODE, bool NORMP, int NWX, int ABL = 0, int VAR = 0, bool F8 = false>
+// ONCE: every weight row is read by one workgroup alone (few rows: one x tile), and its DMA says so (nt: no room in the caches for what nobody reads again).
+// Memory gives such reads 12 % more: 1 GB 181 -> 162 us, 180 MB 37.5 -> 34.8, 117 MB 22.7 -> 21.0 by themselves; products of 2 / 16 rows, us: 128256 x
+// 4096 183 -> 167 / 188 -> 170, 32768 x 4096 56.3 -> 51.0 / 58.4 -> 52.7, 22016 x 4096 41.5 -> 37.5 / 42.4 -> 38.6, 4096 x 14336 in 4 slices 27.1 -> 24.7 /
+// 26.9 -> 25.0.  Read by two workgroups they are slower for it: 128256 x 4096 by 64 rows on 32-row tiles 267 -> 320.
+template <int WN, int XM, int RB, int ST, int MODE, bool NORMP, int NWX, int ABL = 0, int VAR = 0, bool F8 = false, bool ONCE = false>
 __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
     constexpr bool STG = VAR == 1, MAN = VAR == 2;
     // VAR 3 (M32): the slab schedule on v_mfma_f32_32x32x16_bf16 — 32 x 32 blocks, half the MFMA issues per k-step
@@ -186,11 +191,12 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
     uint32_t voff[NPER];
     int dsto[NPER];
     bool isw[NPER];
-    // HB: wave w stages W image pieces [w NPW, +NPW) (pieces 0 .. NPW-1 of its list) and x pieces [w NPX, +NPX)
+    // HB, ONCE: wave w stages W image pieces [w NPW, +NPW) (pieces 0 .. NPW-1 of its list) and x pieces [w NPX, +NPX)
     constexpr int NPW = WN / RPI / NW, NPX = XM / RPI / NW;
+    static_assert(!ONCE || (!SLAB && !F8 && NPW * NW * RPI == WN && NPX * NW * RPI == XM), "whole pieces of W and of x per wave");
 #pragma unroll
     for (int i = 0; i < NPER; ++i) {
-        const int q = HB ? (i < NPW ? wave * NPW + i : WN / RPI + wave * NPX + (i - NPW)) : wave * NPER + i;
+        const int q = HB || ONCE ? (i < NPW ? wave * NPW + i : WN / RPI + wave * NPX + (i - NPW)) : wave * NPER + i;
         const int r = q * RPI + lane / (RB / 16);
         const int pc = lane % (RB / 16);
         dsto[i] = q * 1024;
@@ -217,8 +223,14 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
         unsigned char* st = smem + (j % ST) * STAGE;
         const int kb = min(j, NS1) * RB;  // byte offset of stage j in the row
 #pragma unroll
-        for (int i = 0; i < NPER; ++i)
-            lg_dma16(isw[i] ? (const void*)a.w : (const void*)a.x, isw[i] ? wbytes : xbytes, st + dsto[i], voff[i], kb);
+        for (int i = 0; i < NPER; ++i) {
+            if constexpr (ONCE) {
+                if (i < NPW) lg_dma16<2>(a.w, wbytes, st + dsto[i], voff[i], kb);
+                else lg_dma16(a.x, xbytes, st + dsto[i], voff[i], kb);
+            } else {
+                lg_dma16(isw[i] ? (const void*)a.w : (const void*)a.x, isw[i] ? wbytes : xbytes, st + dsto[i], voff[i], kb);
+            }
+        }
     };
 
     // ---- fragment addressing: W rows (MFMA A) and x rows (MFMA B); the swizzle term is lane-constant
@@ -1195,15 +1207,24 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
 template <int WN, int XM, int RB, int ST, int MODE, bool NORMP, int NWX, int ABL = 0, int VAR = 0, bool F8 = false>
 void lg_launch(const PPArgs& a, hipStream_t st) {
     const int lds = ST * (WN + XM) * RB + 16 + XM * 4 + (F8 && ST == 2 ? (WN + XM) * 4 : 0);
-    auto kern = gemm_lg_kernel<WN, XM, RB, ST, MODE, NORMP, NWX, ABL, VAR, F8>;
-    static bool attr = false;
-    if (!attr) {
-        hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        attr = true;
-    }
     const int mt = (a.M + XM - 1) / XM;
     const int ntl = MODE == kSwiglu ? a.F / (WN / 2) : (a.N + WN - 1) / WN;
-    hipLaunchKernelGGL(kern, dim3(mt * ntl * a.splitk), dim3(128 * NWX), lds, st, a);
+    auto go = [&](auto kern, bool& attr) {
+        if (!attr) {
+            hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+            attr = true;
+        }
+        hipLaunchKernelGGL(kern, dim3(mt * ntl * a.splitk), dim3(128 * NWX), lds, st, a);
+    };
+    if constexpr (XM <= 64 && NWX == 2 && ST > 2 && !F8 && ABL == 0) {
+        if (mt == 1) {
+            static bool attr = false;
+            go(gemm_lg_kernel<WN, XM, RB, ST, MODE, NORMP, NWX, ABL, VAR, F8, true>, attr);
+            return;
+        }
+    }
+    static bool attr = false;
+    go(gemm_lg_kernel<WN, XM, RB, ST, MODE, NORMP, NWX, ABL, VAR, F8>, attr);
 }
 
 // tile configs (ids continue gemm_pp's): {WN = W rows, XM = x rows, RB = LDS row bytes (BK = RB/2), ST = ring depth,
