@@ -280,7 +280,8 @@ __device__ __forceinline__ void moe_store(const f32x4 (&acc)[NS][NM], uint16_t* 
 
 // The tiles there are go to the XCDs in contiguous runs (their L2s then share rows of x and w); a launch of small tiles is
 // bound by the weights' bytes and spreads them over all.
-template <int TM, bool GATHER, int ACT, bool PLACE>
+// ONCE: the weights' DMA is marked as read once (nt), which memory itself gives faster and which leaves nothing behind for a next call.
+template <int TM, bool GATHER, int ACT, bool PLACE, bool ONCE>
 __global__ void __launch_bounds__(256, 2) moe_gemm_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
                                                           uint16_t* __restrict__ y, int32_t* __restrict__ meta,
                                                           int maxTiles, int top, int N, int K, float limit, float slope,
@@ -342,7 +343,7 @@ __global__ void __launch_bounds__(256, 2) moe_gemm_kernel(const uint16_t* __rest
         unsigned char* st = smem + (kt % ST) * (C::W + C::X);
 #pragma unroll
         for (int i = 0; i < C::WP; ++i)
-            __builtin_amdgcn_global_load_lds((gbl_ptr_t)(wsrc[i] + kt * BK), (lds_ptr_t)(st + (C::WP * wave + i) * 1024), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gbl_ptr_t)(wsrc[i] + kt * BK), (lds_ptr_t)(st + (C::WP * wave + i) * 1024), 16, 0, ONCE ? 2 : 0);
 #pragma unroll
         for (int i = 0; i < C::XP; ++i)
             __builtin_amdgcn_global_load_lds((gbl_ptr_t)(xsrc[i] + kt * BK), (lds_ptr_t)(st + C::W + (C::XP * wave + i) * 1024), 16, 0, 0);
@@ -533,6 +534,16 @@ int64_t hy_moe_meta_ints(int items, int E, int tm) {
     return 1 + n + n * tm + items + (int64_t)moe_align_wgs(items) * E;
 }
 
+template <typename F> static hipError_t moe_lds(F kern, int lds) {
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+}
+
+// Weights of the experts chosen (one product's, at most) from which their reads are marked as read once: what the memory-side cache holds.  Below
+// it a decoder of few layers finds them there again.  The whole feed-forward, us, plain -> marked: GELU 4096 wide, 32 experts of 2048, top 4:
+// 4 tokens (268 MB each product) 101 -> 89, 16 204 -> 181, 64 (512 MB) 238 -> 210, 128 239 -> 212, but 2 tokens 54 -> 62; 2048 wide, 16 gated experts of
+// 1024 (134 MB), 64 tokens 42 -> 48.
+constexpr int64_t kOnceBytes = 256 << 20;
+
 template <int TM, bool GATHER, int ACT, bool PLACE = false>
 static void moe_gemm(const uint16_t* x, int64_t rows, const uint16_t* w, uint16_t* y, int32_t* meta, int maxTiles, int top, int N, int K,
                      float limit, float slope, float shift, hipStream_t s, const int32_t* idx = nullptr, int items = 0, int E = 0) {
@@ -543,11 +554,19 @@ static void moe_gemm(const uint16_t* x, int64_t rows, const uint16_t* w, uint16_
         (void)once;
         kern<<<kSlabCUs, 256, lds, s>>>(x, (uint32_t)(rows * K * 2), w, y, meta, maxTiles, top, N, K, limit, slope, shift);
     } else {
-        const auto kern = hy::moe_gemm_kernel<TM, GATHER, ACT, PLACE>;
         constexpr int lds = hy::Tile<TM>::lds;
-        static const hipError_t once = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        auto go = [&](auto kern) {
+            kern<<<maxTiles * (N / hy::Tile<TM>::TN), 256, lds, s>>>(x, w, y, meta, maxTiles, top, N, K, limit, slope, shift, idx, items, E);
+        };
+        if constexpr (TM == 32)
+            if (std::min<int64_t>(items, E) * N * K * 2 >= kOnceBytes) {
+                static const hipError_t once = moe_lds(hy::moe_gemm_kernel<TM, GATHER, ACT, PLACE, true>, lds);
+                (void)once;
+                return go(hy::moe_gemm_kernel<TM, GATHER, ACT, PLACE, true>);
+            }
+        static const hipError_t once = moe_lds(hy::moe_gemm_kernel<TM, GATHER, ACT, PLACE, false>, lds);
         (void)once;
-        kern<<<maxTiles * (N / hy::Tile<TM>::TN), 256, lds, s>>>(x, w, y, meta, maxTiles, top, N, K, limit, slope, shift, idx, items, E);
+        go(hy::moe_gemm_kernel<TM, GATHER, ACT, PLACE, false>);
     }
 }
 
@@ -570,9 +589,9 @@ static void moe_grouped(const uint16_t* h, const int32_t* idx, const float* wt, 
     if (!placed) {
         if (nwg > 1) hy::moe_count_kernel<<<nwg, 1024, 0, s>>>(idx, items, E, item_row + items, item_row);
         hy::moe_place_kernel<<<nwg, 1024, 0, s>>>(idx, items, E, TM, maxTiles, meta);
-        moe_gemm<TM, true, ACT>(h, T, w_up, z, meta, maxTiles, top, up, d, limit, slope, shift, s);
+        moe_gemm<TM, true, ACT>(h, T, w_up, z, meta, maxTiles, top, up, d, limit, slope, shift, s, nullptr, items, E);
     }
-    moe_gemm<TM, false, -1>(z, (int64_t)maxTiles * TM, w_down, yrows, meta, maxTiles, top, d, F, 0.f, 0.f, 0.f, s);
+    moe_gemm<TM, false, -1>(z, (int64_t)maxTiles * TM, w_down, yrows, meta, maxTiles, top, d, F, 0.f, 0.f, 0.f, s, nullptr, items, E);
     hy::moe_combine_kernel<<<dim3(T, (d + 2047) / 2048), 256, 0, s>>>(h, yrows, idx, wt, item_row, out, d, top, E, ACT != hy::kActGlu);
 }
 

@@ -28,12 +28,7 @@ def test_route(n, d, t):
         assert ((got[1] - want[1]).abs() * same).max() < 2e-5
 
 
-# items around a run of 64 and the most that place themselves (512), up to 64 experts; skewed: all items one expert's, several tiles
-@pytest.mark.parametrize("t,top,e", [(1, 1, 1), (1, 4, 64), (31, 2, 8), (33, 2, 8), (16, 4, 64), (127, 4, 32), (128, 4, 64), (129, 4, 64), (64, 2, 65)])
-@pytest.mark.parametrize("skew", ["even", "one", "holes"])
-@pytest.mark.parametrize("form", ["gelu", "glu"])
-def test_ffn(t, top, e, skew, form):
-    d, f = 128, 128
+def _ffn(t, top, e, skew, form, d, f):
     g = torch.Generator().manual_seed(t)
     idx = torch.stack([torch.randperm(e + 2, generator=g)[:top] for _ in range(t)]) if e + 2 >= top else torch.zeros(t, top)
     if skew == "one":
@@ -69,3 +64,17 @@ def test_ffn(t, top, e, skew, form):
             want[rows] += v * wt[rows, k].double()[:, None]
     # three roundings to bfloat16 on the way (products, activation, rows) and one of the sum: 2^-9 each
     assert (y.double() - want).norm() <= 2 ** -7 * want.norm() + 1e-12
+
+
+# items around a run of 64 and the most that place themselves (512), up to 64 experts; skewed: all items one expert's, several tiles
+@pytest.mark.parametrize("t,top,e", [(1, 1, 1), (1, 4, 64), (31, 2, 8), (33, 2, 8), (16, 4, 64), (127, 4, 32), (128, 4, 64), (129, 4, 64), (64, 2, 65)])
+@pytest.mark.parametrize("skew", ["even", "one", "holes"])
+@pytest.mark.parametrize("form", ["gelu", "glu"])
+def test_ffn(t, top, e, skew, form):
+    _ffn(t, top, e, skew, form, 128, 128)
+
+
+# weights around what one product marks as read once (256 MB of the experts that can be chosen), with and without placing in the launch
+@pytest.mark.parametrize("t,top,e,d,f", [(3, 2, 8, 4096, 4096), (4, 2, 8, 4096, 4096), (4, 2, 8, 4096, 3968), (300, 2, 40, 2048, 2048)])
+def test_ffn_read_once(t, top, e, d, f):
+    _ffn(t, top, e, "even", "gelu", d, f)
