@@ -390,9 +390,11 @@ constexpr int sd_smem() {
 
 // One 1 KiB LDS-DMA piece as inline asm (lane l's 16 bytes from its own source address to LDS dst + 16 l).  hipcc
 // cannot see it write LDS, so it does not drain the whole ring (vmcnt(0)) before every ds_read of the step being
-// computed; its completion is counted by the kernel's own sd_vmcnt waits (cdna_hip_programming.md §5.7).
+// computed; its completion is counted by the kernel's own sd_vmcnt waits (cdna_hip_programming.md §5.7).  nt: one
+// workgroup alone reads a page's head, once, and memory gives such reads more (a decode step of four layers: two rows
+// of 131 k tokens, fp8, 1000 -> 978 us, six of 8 k 697 -> 685).
 __device__ __forceinline__ void sd_dma(const void* gsrc, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gsrc), "s"(lds) : "memory");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(gsrc), "s"(lds) : "memory");
 }
 
 template <int N>
@@ -724,7 +726,8 @@ constexpr int kPdKlds = 4 * 8192 + 4 * 256;
 // 4 whole 256-B rows each, into the wave's private 8 KiB, XOR-swizzled on the source address) and are read back in
 // the MFMA layout with conflict-free ds_read_b128.  Loaded straight into the MFMA layout each instruction touches 16
 // rows x 64 B, which the L2 -> CU path serves at ~18 B/clk per CU against ~60 for lane-linear LDS-DMA pieces
-// (csrc/microbench/l2_feed.hip, profiles/r3s2_decode_attn.md).
+// (csrc/microbench/l2_feed.hip, profiles/r3s2_decode_attn.md).  K and V of bf16 pages are read as data used once (nt),
+// which memory serves faster: four layers of 1024 rows, 120 tokens each, 2816 -> 2777 us a step.
 template <bool FP8, bool PF, bool LEAN, int OCC, bool RP = false, bool KL = true>
 __global__ void __launch_bounds__(256, OCC) paged_decode_kernel(
     const uint16_t* __restrict__ q, const void* __restrict__ kcv, const void* __restrict__ vcv,
@@ -864,7 +867,7 @@ __global__ void __launch_bounds__(256, OCC) paged_decode_kernel(
                     const int t = 4 * i + (lane >> 4);
                     const int64_t pg = t < 16 ? blkA : blkB;
                     const uint16_t* src = kc + (((pg * hkv + h) * block_size) + (t & 15)) * kD + 8 * ((lane & 15) ^ kswz(t));
-                    __builtin_amdgcn_global_load_lds((pd_gbl_ptr_t)src, (pd_lds_ptr_t)(kl + i * 1024), 16, 0, 0);
+                    __builtin_amdgcn_global_load_lds((pd_gbl_ptr_t)src, (pd_lds_ptr_t)(kl + i * 1024), 16, 0, 2);
                 }
             }
             const int64_t kblk = r < 8 ? blkA : blkB;
@@ -894,7 +897,7 @@ __global__ void __launch_bounds__(256, OCC) paged_decode_kernel(
             } else {
 #pragma unroll
                 for (int dt = 0; dt < 8; ++dt)
-                    vf[dt] = *reinterpret_cast<const bf16x8*>(vc + voff + (int64_t)(dt * 16 + r) * block_size);
+                    vf[dt] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(vc + voff + (int64_t)(dt * 16 + r) * block_size));
             }
         } else {
 #pragma unroll
