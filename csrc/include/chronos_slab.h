@@ -101,8 +101,8 @@ template <int NM, bool SQ, class RowW, class Dst, class Go>
 __device__ __forceinline__ void slab_step(f32x4 (&acc)[8][NM], bf16x8 (&fa0)[8], bf16x8 (&fb0)[NM], bf16x8 (&fa1)[8], bf16x8 (&fb1)[NM],
                                           const unsigned char* cw, const unsigned char* cx, const unsigned char* nw,
                                           const unsigned char* nx, const Dst& dst, const Go& go) {
-    static_assert(NM == 8 || (NM == 4 && !SQ), "tile");
-    constexpr int NF = 8 + NM, END = 16 * NM, RD1 = NF, REL = NM == 8 ? 20 : 14, LAND = END - NF, PEND = NM == 8 ? 108 : LAND;
+    static_assert(NM >= 4 && NM <= 8 && (NM == 8 || !SQ), "tile");
+    constexpr int NF = 8 + NM, END = 16 * NM, RD1 = NF, REL = NM == 8 ? 20 : NM + 10, LAND = END - NF, PEND = NM == 8 ? 108 : LAND;
     static_assert(RD1 < REL && REL + NF <= PEND && PEND <= LAND, "slab schedule");
     auto read = [&](auto RC, const unsigned char* w, const unsigned char* x, bf16x8 (&fa)[8], bf16x8 (&fb)[NM]) {
         constexpr int r = decltype(RC)::value;
@@ -182,10 +182,11 @@ template <bool PAIR> struct SlabRow {   // byte offset of the wave's W block b; 
 // The tiles of one workgroup, one after the other without a pause of the slab pipeline: the pieces that a tile's last two slabs issue are
 // those of the next tile's first two, which land while this tile's results are stored.  Tile v of the launch goes to workgroup
 // v % gridDim.x (gridDim.x = slab_grid(T, tail)); xcd_remap gives neighbouring tiles to the same XCD.
+// NMX < 8: tiles of 256 W rows by 32 NMX x rows, all alike (T of them, no tail).
 //   off(NM, tile, m, wv, xv, wb): byte offsets of the lane's rows of slab 0 (x rows from row m of the tile on) and the W matrix
 //   rows(NM, tile, m): called before a tile's first slab, for what its epilogue needs of its rows
 //   epi(NM, tile, m, acc): store the results (rows: the wave's 4 KiB of LDS)
-template <bool PAIR, class Off, class Rows, class Epi>
+template <bool PAIR, int NMX = 8, class Off, class Rows, class Epi>
 __device__ __forceinline__ void slab_run(unsigned char* smem, int T, int tail, int NS, const void* x, int xbytes, int wbytes, const Off& off,
                                          const Rows& rows, const Epi& epi) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -194,8 +195,6 @@ __device__ __forceinline__ void slab_run(unsigned char* smem, int T, int tail, i
     const unsigned char* const iw = smem + ((PAIR ? 64 : 128) * wn + ln) * 128;
     const uint32_t lds = (uint32_t)(uintptr_t)(lg_lds_cptr)smem;
     using Row = SlabRow<PAIR>;
-    int full, half;
-    slab_split(T, tail, full, half);
     uint32_t wv[8];
     const void* wb;
     auto walk = [&](auto NMC, int first, int count, auto tile_of, auto m_of) {
@@ -283,6 +282,12 @@ __device__ __forceinline__ void slab_run(unsigned char* smem, int T, int tail, i
         lg_bar();
     };
     const int b = blockIdx.x;
+    if constexpr (NMX < 8) {
+        walk(std::integral_constant<int, NMX>{}, b, T, [&](int v) { return xcd_remap(v, T); }, [](int) { return 0; });
+        return;
+    }
+    int full, half;
+    slab_split(T, tail, full, half);
     if (b < full)
         walk(std::integral_constant<int, 8>{}, b, full, [&](int v) { return xcd_remap(v, full); }, [](int) { return 0; });
     const int pairs = half - tail;   // halves that are two of a tile

@@ -31,15 +31,16 @@ __device__ __forceinline__ float row_sum16(float v) {
     return v;
 }
 
-template <int MODE, bool NORMP>
+template <int MODE, bool NORMP, int NMX>
 __global__ void __launch_bounds__(256, 1) gemm_slab_kernel(PPArgs a) {
+    constexpr int TR = 32 * NMX;   // x rows of a tile
     constexpr bool PAIR = MODE == kPPSwiglu || MODE == kPPGlu;
     constexpr int OC = PAIR ? 64 : 128, RBY = 2 * OC, NCH = RBY / 16, RPS = 64 / NCH, NK = 16 / RPS;   // a wave's columns, bytes and
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];                            // pieces per row; rows per store
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wn = wave >> 1, wm = wave & 1, in = lane >> 3, piece = ((lane & 7) ^ in) * 8;
     const int nt = PAIR ? a.F / 128 : (a.N + 255) / 256, S = MODE == kPPPart ? a.splitk : 1;
-    const int tail = slab_tail(a.M, nt, S), mt = tail > 0 ? a.M / 256 : (a.M + 255) / 256;
+    const int tail = NMX == 8 ? slab_tail(a.M, nt, S) : 0, mt = tail > 0 ? a.M / TR : (a.M + TR - 1) / TR;
     // tiles in groups of gm along x, so that what an XCD runs at a time shares rows of both operands in its L2
     // (kPPPart: slice by slice; the short last rows of all slices behind)
     auto where = [&](int tile, int& tm, int& tn, int& sl) {
@@ -79,7 +80,7 @@ __global__ void __launch_bounds__(256, 1) gemm_slab_kernel(PPArgs a) {
             wv[i] = ((uint32_t)row * (uint32_t)a.K + at) * 2;
         }
 #pragma unroll
-        for (int i = 0; i < NM; ++i) xv[i] = ((uint32_t)(tm * 256 + m + 8 * (NM * wave + i) + in) * (uint32_t)a.K + at) * 2;
+        for (int i = 0; i < NM; ++i) xv[i] = ((uint32_t)(tm * TR + m + 8 * (NM * wave + i) + in) * (uint32_t)a.K + at) * 2;
     };
     // NORMP: a lane sums its row's partials; two buffers in turn (a tile's slabs, with their barriers, lie between a buffer's
     // writers and its readers, and between those and the next writers)
@@ -89,8 +90,8 @@ __global__ void __launch_bounds__(256, 1) gemm_slab_kernel(PPArgs a) {
             constexpr int RPW = 8 * decltype(NMC)::value;   // rows per wave
             int tm, tn, sl;
             where(tile, tm, tn, sl);
-            const int row = RPW * wave + (lane & (RPW - 1));
-            const float* p = a.part_in + (int64_t)min(tm * 256 + m + row, a.M - 1) * a.nparts_in;
+            const int row = RPW * wave + lane % RPW;
+            const float* p = a.part_in + (int64_t)min(tm * TR + m + row, a.M - 1) * a.nparts_in;
             f32x4 t = {0.f, 0.f, 0.f, 0.f};
             int i = 0;
             if ((a.nparts_in & 3) == 0) {
@@ -115,7 +116,7 @@ __global__ void __launch_bounds__(256, 1) gemm_slab_kernel(PPArgs a) {
         constexpr int NM = decltype(NMC)::value;
         int tm, tn, sl;
         where(tile, tm, tn, sl);
-        const int m0 = tm * 256 + m + 16 * NM * wm;                      // the wave's first row
+        const int m0 = tm * TR + m + 16 * NM * wm;                      // the wave's first row
         const int ld = PAIR ? a.F : a.N, n = (PAIR ? tn * 128 : tn * 256) + OC * wn + 8 * c;
         u16x8 rv[MODE == kPPResid ? NK : 1];
         auto resid = [&](int t) {
@@ -202,7 +203,7 @@ __global__ void __launch_bounds__(256, 1) gemm_slab_kernel(PPArgs a) {
             }
         }
     };
-    slab_run<PAIR>(smem, mt * nt * S, tail, MODE == kPPPart ? a.kts : a.K / 64, a.x, (int)((int64_t)a.M * a.K * 2), (int)((int64_t)a.N * a.K * 2), off, scales, epi);
+    slab_run<PAIR, NMX>(smem, mt * nt * S, tail, MODE == kPPPart ? a.kts : a.K / 64, a.x, (int)((int64_t)a.M * a.K * 2), (int)((int64_t)a.N * a.K * 2), off, scales, epi);
 }
 
 // y = the new residual stream: the S slices of 8 columns per thread in their order, the residual, RMSNorm partials per 128 columns
@@ -230,16 +231,49 @@ __global__ void __launch_bounds__(256) slab_sum_resid_kernel(const float* __rest
     if ((threadIdx.x & 15) == 0) part[i / 128] = ss;
 }
 
-template <int MODE, bool NORMP>
-void slab_launch(const PPArgs& a, hipStream_t st) {
+// x rows of a tile, in 32s, for M rows and nt tiles of W rows (walked S times): 8, whose last round may be of halves, or 4 to 7 where the
+// rounds of such tiles take less.  A round's time, in those of 256 x 256 tiles, is from 1 to 4 rounds of 28672 x 4096 (4 rows-in-32s: 69, 115, 167, 245
+// us; 5: 74, 127, 186, 247; 6: 77, 140, 213; 7: 84, 155, 235; 8: 95, 185, 267, its halves behind a round 50).  us, 256-row tiles -> the rows picked:
+// that shape at 272 rows 84.9 -> 72.7, 384 89.9 -> 79.1, 528 143 -> 124, 896 184 -> 169, 1152 244 -> 222; 4096 x 14336 in 4 slices at 528 81.8 ->
+// 69.0, 640 85.6 -> 73.1, in 8 at 272 55.9 -> 46.8, in 2 at 1152 137 -> 116; 6144 x 4096 at 1600 79.0 -> 65.7.
+// In one round all tiles alike are as good as halves or better, because the short last rows of slab_tail come behind all others, where no
+// XCD has their W rows any more (4096 x 14336 in 4 slices at 384 rows 66.8, 63.3 as three tiles of 128 rows).
+int slab_rows(int M, int nt, int S) {
+    constexpr float cost[] = {0.61f, 0.67f, 0.76f, 0.86f};
+    const int tail = slab_tail(M, nt, S);
+    int full, half;
+    slab_split((tail > 0 ? M / 256 : (M + 255) / 256) * nt * S, tail, full, half);
+    float best = (float)((full + kSlabCUs - 1) / kSlabCUs) + (full ? 0.57f : 0.63f) * ((half + kSlabCUs - 1) / kSlabCUs);
+    int nm = 8;
+    for (int n = 4; n < 8; ++n) {
+        const int64_t tiles = (int64_t)((M + 32 * n - 1) / (32 * n)) * nt * S;
+        const float t = cost[n - 4] * ((tiles + kSlabCUs - 1) / kSlabCUs);
+        if (t < best * 0.97f) best = t, nm = n;
+    }
+    return nm;
+}
+
+template <int MODE, bool NORMP, int NMX>
+void slab_launch_rows(const PPArgs& a, int nt, int S, hipStream_t st) {
     constexpr int lds = kSlabLds + (NORMP ? 2048 : 0);
-    const auto kern = gemm_slab_kernel<MODE, NORMP>;
+    const auto kern = gemm_slab_kernel<MODE, NORMP, NMX>;
     static const hipError_t once = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     (void)once;
+    const int tail = NMX == 8 ? slab_tail(a.M, nt, S) : 0, tiles = (tail > 0 ? a.M / 256 : (a.M + 32 * NMX - 1) / (32 * NMX)) * nt * S;
+    hipLaunchKernelGGL(kern, dim3(NMX == 8 ? slab_grid(tiles, tail) : tiles < kSlabCUs ? tiles : kSlabCUs), dim3(256), lds, st, a);
+}
+
+template <int MODE, bool NORMP>
+void slab_launch(const PPArgs& a, hipStream_t st) {
     const bool pair = MODE == kPPSwiglu || MODE == kPPGlu;
     const int nt = pair ? a.F / 128 : (a.N + 255) / 256, S = MODE == kPPPart ? a.splitk : 1;
-    const int tail = slab_tail(a.M, nt, S), tiles = (tail > 0 ? a.M / 256 : (a.M + 255) / 256) * nt * S;
-    hipLaunchKernelGGL(kern, dim3(slab_grid(tiles, tail)), dim3(256), lds, st, a);
+    switch (slab_rows(a.M, nt, S)) {
+        case 4: slab_launch_rows<MODE, NORMP, 4>(a, nt, S, st); break;
+        case 5: slab_launch_rows<MODE, NORMP, 5>(a, nt, S, st); break;
+        case 6: slab_launch_rows<MODE, NORMP, 6>(a, nt, S, st); break;
+        case 7: slab_launch_rows<MODE, NORMP, 7>(a, nt, S, st); break;
+        default: slab_launch_rows<MODE, NORMP, 8>(a, nt, S, st);
+    }
 }
 
 }  // namespace

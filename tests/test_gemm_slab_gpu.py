@@ -101,3 +101,33 @@ def test_slices_of_k(m, n, k, s):
         assert torch.equal(z, y + res)
         want = z.double().square().view(m, n // 128, 128).sum(-1)
         assert ((part.double() - want).abs() <= want * 128 * 2.0 ** -24).all()
+
+
+# x tiles of 128, 160, 192, 224 and 256 rows (80 tiles of W rows; their first and last row counts), two rounds of 160, whole rounds with halves
+# behind, and the same with two slices of K
+@pytest.mark.parametrize("m", [5, 384, 385, 480, 481, 576, 577, 672, 673, 768, 769, 960, 1300])
+@pytest.mark.parametrize("k,s", [(64, 1), (192, 1), (384, 2)])
+def test_rows_of_a_tile(m, k, s):
+    """Every epilogue against float32, and every row the same bits as among other rows, where tiles have another height."""
+    from chronos import ops
+    from chronos.ops import gemm as G
+
+    ops.load()
+    n = 20480 // s
+    x, w = _operands(m, n, k, m + k)
+    ref = x.float() @ w.float().t()
+    y, _ = G.pp_gemm(x, w, G.PP_PLAIN, (88, s))
+    _close(y, ref)
+    cut = m // 3 + 1
+    assert torch.equal(torch.cat([G.pp_gemm(v.contiguous(), w, G.PP_PLAIN, (88, s))[0] for v in (x[:cut], x[cut:])]), y)
+    res = torch.randn(m, n, device=DEV).to(torch.bfloat16)
+    z, part = G.pp_gemm(x, w, G.PP_RESID, (88, s), resid=res)
+    assert torch.equal(z, y + res)
+    want = z.double().square().view(m, n // 128, 128).sum(-1)
+    assert ((part.double() - want).abs() <= want * 128 * 2.0 ** -24).all()
+    if s == 1:
+        g, u = ref[:, : n // 2], ref[:, n // 2:]
+        _close(torch.ops.chronos.gemm_act(x, w, 3, 1.5, 1.7, 1.0), g.clamp(max=1.5) * torch.sigmoid(1.7 * g.clamp(max=1.5)) * (u.clamp(-1.5, 1.5) + 1))
+        sums = x.float().square().view(m, 32, -1).sum(-1).contiguous()
+        scale = torch.rsqrt(x.float().square().mean(-1, keepdim=True) + 1e-5)
+        _close(torch.ops.chronos.gemm_pp(x, w, 0, 88, 1, None, sums, 1e-5, False)[0], ref * scale)
