@@ -107,7 +107,8 @@ __device__ __forceinline__ int lg_swz64(int row) { return (4 - ((row >> 2) & 3))
 // ONCE: every weight row is read by one workgroup alone (few rows: one x tile), and its DMA says so (nt: no room in the caches for what nobody reads again).
 // Memory gives such reads 12 % more: 1 GB 181 -> 162 us, 180 MB 37.5 -> 34.8, 117 MB 22.7 -> 21.0 by themselves; products of 2 / 16 rows, us: 128256 x
 // 4096 183 -> 167 / 188 -> 170, 32768 x 4096 56.3 -> 51.0 / 58.4 -> 52.7, 22016 x 4096 41.5 -> 37.5 / 42.4 -> 38.6, 4096 x 14336 in 4 slices 27.1 -> 24.7 /
-// 26.9 -> 25.0.  Read by two workgroups they are slower for it: 128256 x 4096 by 64 rows on 32-row tiles 267 -> 320.
+// 26.9 -> 25.0; of 128 rows 28672 x 4096 59.6 -> 57.3, 4096 x 4096 31.7 -> 29.5, of 96 rows 4096 x 14336 in 4 slices 47.2 -> 44.8; tiles of 256 rows
+// gain nothing.  Read by two workgroups they are slower for it: 128256 x 4096 by 64 rows on 32-row tiles 267 -> 320.
 template <int WN, int XM, int RB, int ST, int MODE, bool NORMP, int NWX, int ABL = 0, int VAR = 0, bool F8 = false, bool ONCE = false>
 __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
     constexpr bool STG = VAR == 1, MAN = VAR == 2;
@@ -1216,7 +1217,7 @@ void lg_launch(const PPArgs& a, hipStream_t st) {
         }
         hipLaunchKernelGGL(kern, dim3(mt * ntl * a.splitk), dim3(128 * NWX), lds, st, a);
     };
-    if constexpr (XM <= 64 && NWX == 2 && ST > 2 && !F8 && ABL == 0) {
+    if constexpr (XM <= 128 && ST > 2 && !F8 && ABL == 0 && WN / (1024 / RB) % (2 * NWX) == 0 && XM / (1024 / RB) % (2 * NWX) == 0) {
         if (mt == 1) {
             static bool attr = false;
             go(gemm_lg_kernel<WN, XM, RB, ST, MODE, NORMP, NWX, ABL, VAR, F8, true>, attr);
