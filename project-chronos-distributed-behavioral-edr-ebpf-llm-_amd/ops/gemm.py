@@ -12,7 +12,7 @@ Routing is by measured shape:
   with the kernel, tile config and split-K of the measured plan (``gemm_plan.json``: per (N, K, epilogue) the best
   by M range, from ``scripts/tune_gemm_pp.py`` on one MI355X, random operands, cold weights; plan cfg >= 100 is
   skinny config cfg - 100);
-* shapes that the plan does not list: up to 64 rows ``few_rows_plan``, from 128 on ``many_rows_plan``, where their measured ranges say that
+* shapes that the plan does not list: up to 64 rows ``few_rows_plan``, from 128 on ``many_rows_plan``, between them ``mid_rows_plan``, where their measured ranges say that
   they win;
 * hipBLASLt (torch.matmul) only where the plan records that the library wins by more than 3 % (the "plain library
   GEMM" rule), for unlisted shapes outside that range, or for shapes the kernel does not take (K % 64, N % 4).  CHRONOS_PP=lib|own|auto forces a side.
@@ -270,17 +270,53 @@ def few_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     return out
 
 
+# 65 .. 128 rows, and 33 .. 64 of 12288 outputs and more that few_rows_plan leaves: gemm_lg.hip's tiles of 64 W by 64 x rows (39, K split without
+# tickets), 64 by 128 (32) and 128 by 128 (19).  The terms of _FEW_LARGE, fitted on profiles/mid_rows_gemm.json (rms error 7 %).
+_MID = ((64, {39: (0.247, 3.535, 0.273, 0.037, 1.296, 0.257, 0.392, 2.906), 19: (3.26, 2.0, 0.378, 0.067, 0.0, 0.1, 1.6, 0.605)}),
+        (128, {39: (2.318, 2.234, 0.227, 0.0, 1.264, 0.249, 0.892, 0.74), 32: (2.957, 2.0, 0.329, 0.0, 0.144, 0.377, 2.98, 1.176),
+               19: (3.861, 2.0, 0.482, 0.0, 0.006, 0.1, 7.939, 0.496)}))
+
+
+def mid_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
+    """(config, split-K) of the hand-written GEMM for the rows between few_rows_plan's and many_rows_plan's ranges, or None (the library), of shapes that no
+    plan lists: 65 .. 128 rows by at least 512 outputs and K >= 512, and 33 .. 64 rows by 12288 outputs and more.  Where every weight row is read
+    once, memory gives these tiles more than the library gets; us, library -> this: 80 rows of 1024 x 1024 10.9 -> 6.6, 4096 x 4096 17.1 -> 13.9, 2048 x
+    5632 16.4 -> 12.2, 12288 x 4096 33.4 -> 28.0, 32768 x 1024 22.9 -> 17.0; 64 rows of 14336 x 4096 28.6 -> 26.8, 32768 x 4096 62.2 -> 55.4.  On
+    average 1.29 and 1.21 times as fast (460 and 105 shapes; 11 and 0 slower by more than 3 %, the worst 96 rows of 2560 x 2816, 10.4 -> 11.4), 1 % behind
+    the best config.  Table: profiles/mid_rows_gemm.json, which tests/test_measured_rules.py replays."""
+    if PP_MODE != "auto":
+        return None
+    key = (m, n, k, -5)
+    hit = _plan_cache.get(key, False)
+    if hit is not False:
+        return hit
+    out = best = None
+    if (n >= (512 if m > 64 else 12288) and 32 < m <= 128 and k >= 512 and n % 16 == 0 and k % 64 == 0 and k <= 1 << 20 and (n + 128) * k < 1 << 30
+            and (n, k, PP_PLAIN) not in _plan_file()):
+        for cfg, c in next(models for most, models in _MID if m <= most).items():
+            for sk in (1, 2, 4, 8) if cfg == 39 else (1,):
+                groups, steps = -(-n // _PP_BN[cfg]) * -(-m // _PP_BM[cfg]) * sk, k / (64 * sk)
+                if k // 64 % sk or (sk > 1 and (groups > 1024 or k // 64 // sk < 2)):
+                    continue
+                t = (c[0] + c[1] * (sk > 1) + c[2] * steps + c[3] * n * k * 2e-6 + c[4] * groups / 256
+                     + c[5] * (-(-groups // 256) - 1) * steps + c[6] * m * k * groups * 2e-8 + c[7] * sk * m * n * 1e-6)
+                if best is None or t < best:
+                    best, out = t, (cfg, sk)
+    _plan_cache[key] = out
+    return out
+
+
 # Configs of gemm_slices (csrc/kernels/bindings.cpp)
 _SLICED = (33, 36, 38, 39, 72, 73, 74, 75, 78, 79, *_UNEVEN)
 
 
 def product_f32(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
-    """x @ w.T as float32 [M, N], the product's sums before their rounding, where few_rows_plan takes it, or None.  A vocabulary's logits: 8 rows of
+    """x @ w.T as float32 [M, N], the product's sums before their rounding, where few_rows_plan or mid_rows_plan takes it, or None.  A vocabulary's logits: 8 rows of
     32768 x 1024 16 us as a rounded product and a conversion, 12 so."""
     (m, k), n = x.shape if x.dim() == 2 else (0, 0), w.shape[0]
     if not 0 < m <= 64 or n % 4 or not _plain_rows(x, w) or _registered(m, n, k) or (n + 128) * k >= 1 << 30:
         return None
-    plan = few_rows_plan(m, n, k)
+    plan = few_rows_plan(m, n, k) or mid_rows_plan(m, n, k)
     if plan is None or plan[0] not in _SLICED:
         return None
     from . import _k
@@ -691,14 +727,14 @@ def linear(x, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tens
         m, k = x.numel() // x.shape[-1], x.shape[-1]
         n = w.shape[0]
         few = None
-        if out is None and (0 < m <= 64 or m >= MANY_MIN) and _plain_rows(x, w):
-            few = few_rows_plan(m, n, k) if m <= 64 else many_rows_plan(m, n, k)
+        if out is None and m > 0 and _plain_rows(x, w):
+            few = (few_rows_plan(m, n, k) if m <= 64 else many_rows_plan(m, n, k) if m >= MANY_MIN else None) or (mid_rows_plan(m, n, k) if 32 < m <= 128 else None)
         if few is None and gemv_ok(m, n, k):
             return _gemv(x, w)
         for pred, fn in _custom:
             if pred(m, n, k):
                 return fn(x, w)
-        if few is not None and m <= 64 and few[1] > 1 and few[0] < SK_BASE:   # a split without tickets
+        if few is not None and few[1] > 1 and few[0] < SK_BASE and few[0] != 88:   # a split without tickets
             from . import _k
 
             return _k().gemm_split(x.reshape(-1, k), w, *few).view(*x.shape[:-1], n)
