@@ -270,28 +270,33 @@ def few_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     return out
 
 
-# 65 .. 128 rows, and 33 .. 64 of 12288 outputs and more that few_rows_plan leaves: gemm_lg.hip's tiles of 64 W by 64 x rows (39, K split without
+# 65 .. 512 rows, and 33 .. 64 of 12288 outputs and more that few_rows_plan leaves: gemm_lg.hip's tiles of 64 W by 64 x rows (39, K split without
 # tickets), 64 by 128 (32) and 128 by 128 (19).  The terms of _FEW_LARGE, fitted on profiles/mid_rows_gemm.json (rms error 7 %).
 _MID = ((64, {39: (0.247, 3.535, 0.273, 0.037, 1.296, 0.257, 0.392, 2.906), 19: (3.26, 2.0, 0.378, 0.067, 0.0, 0.1, 1.6, 0.605)}),
         (128, {39: (2.318, 2.234, 0.227, 0.0, 1.264, 0.249, 0.892, 0.74), 32: (2.957, 2.0, 0.329, 0.0, 0.144, 0.377, 2.98, 1.176),
-               19: (3.861, 2.0, 0.482, 0.0, 0.006, 0.1, 7.939, 0.496)}))
+               19: (3.861, 2.0, 0.482, 0.0, 0.006, 0.1, 7.939, 0.496)}),
+        (256, {39: (2.545, 2.395, 0.242, 0.0, 1.391, 0.232, 0.196, 0.936)}), (512, {39: (2.187, 2.426, 0.258, 0.0, 2.095, 0.234, 0.059, 0.607)}))
 
 
 def mid_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
-    """(config, split-K) of the hand-written GEMM for the rows between few_rows_plan's and many_rows_plan's ranges, or None (the library), of shapes that no
-    plan lists: 65 .. 128 rows by at least 512 outputs and K >= 512, and 33 .. 64 rows by 12288 outputs and more.  Where every weight row is read
-    once, memory gives these tiles more than the library gets; us, library -> this: 80 rows of 1024 x 1024 10.9 -> 6.6, 4096 x 4096 17.1 -> 13.9, 2048 x
-    5632 16.4 -> 12.2, 12288 x 4096 33.4 -> 28.0, 32768 x 1024 22.9 -> 17.0; 64 rows of 14336 x 4096 28.6 -> 26.8, 32768 x 4096 62.2 -> 55.4.  On
-    average 1.29 and 1.21 times as fast (460 and 105 shapes; 11 and 0 slower by more than 3 %, the worst 96 rows of 2560 x 2816, 10.4 -> 11.4), 1 % behind
-    the best config.  Table: profiles/mid_rows_gemm.json, which tests/test_measured_rules.py replays."""
+    """(config, split-K) of the hand-written GEMM for rows and shapes that few_rows_plan, many_rows_plan and the measured plan leave, or None (the library):
+    65 .. 128 rows, 33 .. 64 rows by 12288 outputs and more, 129 .. 256 rows by up to 4096 outputs, 257 .. 512 by up to 2048 with K <= 8192; outputs and K
+    from 512 on.  Rows beyond 64 count in 32s, so that a server's steps find their plan again.  us, library -> this: 80 rows of 1024 x 1024 10.9 ->
+    6.6, 4096 x 4096 17.1 -> 13.9, 2048 x 5632 16.4 -> 12.2, 12288 x 4096 33.4 -> 28.0, 32768 x 1024 22.9 -> 17.0; 64 rows of 14336 x 4096 28.6 ->
+    26.8, 32768 x 4096 62.2 -> 55.4; 192 rows of 1024 x 1024 10.7 -> 7.5, 2048 x 5632 21.2 -> 19.1; 512 rows of 1024 x 4096 15.8 -> 14.7.  On average 1.29
+    (460 shapes of 65 .. 128 rows), 1.21 (105 of 33 .. 64), 1.21 (123 of 129 .. 256) and 1.10 times (86) as fast, of 774 shapes 35 slower by more than 3 %,
+    the worst by 9 % (512 x 1408, 8.4 -> 9.2); and a library call costs the host 22 us, this 7.  Beyond these ranges the two are level or the
+    library ahead.  Table: profiles/mid_rows_gemm.json, which tests/test_measured_rules.py replays."""
     if PP_MODE != "auto":
         return None
+    m = m if m <= 64 else -(-m // 32) * 32
     key = (m, n, k, -5)
     hit = _plan_cache.get(key, False)
     if hit is not False:
         return hit
     out = best = None
-    if (n >= (512 if m > 64 else 12288) and 32 < m <= 128 and k >= 512 and n % 16 == 0 and k % 64 == 0 and k <= 1 << 20 and (n + 128) * k < 1 << 30
+    if ((m > 32 and n >= 12288 if m <= 64 else n >= 512 if m <= 128 else 512 <= n <= 4096 if m <= 256 else m <= 512 and 512 <= n <= 2048 and k <= 8192)
+            and k >= 512 and n % 16 == 0 and k % 64 == 0 and k <= 1 << 20 and (n + 128) * k < 1 << 30
             and (n, k, PP_PLAIN) not in _plan_file()):
         for cfg, c in next(models for most, models in _MID if m <= most).items():
             for sk in (1, 2, 4, 8) if cfg == 39 else (1,):
@@ -728,7 +733,7 @@ def linear(x, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tens
         n = w.shape[0]
         few = None
         if out is None and m > 0 and _plain_rows(x, w):
-            few = (few_rows_plan(m, n, k) if m <= 64 else many_rows_plan(m, n, k) if m >= MANY_MIN else None) or (mid_rows_plan(m, n, k) if 32 < m <= 128 else None)
+            few = (few_rows_plan(m, n, k) if m <= 64 else many_rows_plan(m, n, k) if m >= MANY_MIN else None) or (mid_rows_plan(m, n, k) if 32 < m <= 512 else None)
         if few is None and gemv_ok(m, n, k):
             return _gemv(x, w)
         for pred, fn in _custom:

@@ -19,7 +19,7 @@ def _check(y, x, w, tol=2 ** -8):
 
 
 # rows at the edges of the rule and of the tiles, outputs that end inside a tile, K of one, two and odd numbers of steps per slice
-@pytest.mark.parametrize("m", [33, 63, 64, 65, 96, 127, 128])
+@pytest.mark.parametrize("m", [33, 63, 64, 65, 96, 127, 128, 129, 255, 257, 511, 512])
 @pytest.mark.parametrize("n,k", [(512, 512), (528, 11264), (1040, 576), (1024, 2816), (4112, 4096), (12288, 1024), (12304, 2048), (32768, 512), (16400, 4096)])
 def test_linear(m, n, k):
     from chronos import ops
