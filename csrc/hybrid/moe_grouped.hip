@@ -33,9 +33,11 @@ typedef __attribute__((address_space(1))) void* gbl_ptr_t;
 //   256 x 256, two stages (128 KB), 4 waves of 128 x 128 outputs (moe_gemm256_kernel): experts with many tokens; half the bytes
 //    per product of
 //   128 x 128, two stages (64 KB: two workgroups per CU, one multiplies while the other waits), 4 waves of 64 x 64
+//    64 x 128, three stages (72 KB: two workgroups per CU): experts with some tokens, whose time is the weights' (320 tokens of 4096, 32 experts of 2048,
+//    top 4: 265 -> 230 us against two stages of 128 rows)
 //    32 x 128, four stages (80 KB: two workgroups per CU, the weights of three k-steps in flight in each): few tokens
 template <int TM> struct Tile {
-    static constexpr int TN = 128, ST = TM == 32 ? 4 : 2, WX = 2, WAVES = 4;
+    static constexpr int TN = 128, ST = TM == 32 ? 4 : TM == 64 ? 3 : 2, WX = 2, WAVES = 4;
     static constexpr int W = TN * 128, X = TM * 128;                                     // bytes of the two images of a stage
     static constexpr int WP = W / 1024 / WAVES, XP = X / 1024 / WAVES;                   // 1 KiB pieces per wave and stage
     static constexpr int NS = TN / 32, NM = TM / 16 / WX;                                // 16-row blocks per wave
@@ -506,23 +508,30 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(const uint16_t* __rest
 
 }  // namespace hy
 
-// Rows per tile.  32 where experts see at most 16 tokens on average, so that a tile's padding rows cost little and the launch
-// streams weights with more of them in flight; 256, whose loop is the fastest per product, where most tiles fill (192 tokens per
-// expert, 384 of narrow ones) and the smaller product has a tile for a quarter of the CUs; else 128.  up: rows of an expert's first matrix.  Measured on gated
-// experts, us at 32 / 128 / 256 rows: 16 experts of 2048 by 1024 with 64 tokens (4 experts each) 46 / 54 / 57, 200 tokens 51 / 57 / 58, 512
+// Rows per tile.  32 where experts see few tokens on average, so that a tile's padding rows cost little and the launch streams weights with more of
+// them in flight; 64 above; 256, whose loop is the fastest per product, where most tiles fill (192 tokens per expert, 384 of narrow ones) and the smaller
+// product has a tile for a quarter of the CUs; else 128.  up: rows of an expert's first matrix.  The fewer workgroups a tile per expert and 128 of
+// the smaller product's columns makes (wide), the further the smaller tiles go, whose number fills the CUs.  us at 32 / 64 / 128 rows, GELU:
+// 8 experts of 1024 by 512 (wide 32), top 2, 128 tokens (32 items per expert) 20 / 28 / 33, 320 24 / 28 / 35, 1000 - / 32 / 39, 1400 - / 36 / 42; 16 of
+// 2048 by 1408 (176), top 4, 96 tokens 39 / 48 / 58, 160 60 / 49 / 61, 256 68 / 56 / 66, 400 - / 72 / 67; 32 of 4096 by 2048 (512), top 4, 160 218 / 230 /
+// 266, 200 248 / 231 / 269, 400 259 / 231 / 279, 600 310 / 286 / 288, 800 - / 299 / 291; with expert e chosen in proportion to 1 / e 200 tokens 230 / 233 / 339,
+// 400 274 / 253 / 348, 600 324 / 299 / 348, 1400 - / 438 / 405.  128 against 256, on gated
+// experts, us at 32 / 128 / 256 rows: 16 experts of 2048 by 1024, 512
 // tokens 81 / 66 / 62, 2048 tokens 248 / 154 / 150, 8192 tokens 870 / 516 / 407; 32 experts of 4096 by 1536 with 512 tokens 329 / 282 / 323,
 // 1536 tokens 606 / 424 / 352, 8192 tokens 2640 / 1610 / 1180; 8 experts of 1024 by 512 with 1024 tokens (2 each) 39 / 35 / 39, 8192 tokens
-// 140 / 98 / 100.  (At 200 tokens of 2048, 50 items per expert, 32 rows still win by a tenth; at 128 per expert they lose by a fifth: the
-// line lies lower because a skewed choice fills more tiles.  So does 128 rows against 256: at 128 tokens per expert of 16 256 rows win by 6 %,
+// 140 / 98 / 100.  (A skewed choice fills more tiles: at 128 tokens per expert of 16 256 rows win by 6 %,
 // but with expert e chosen in proportion to 1 / e they lose 27 %, 84 for 66 us; from 192 on they win there too, but for experts of at most four
 // tiles across: 64 of 1024 by 512 at 192 tokens each 84 / 77, skewed 88 / 103, at 256 113 / 118, skewed 117 / 118, at 384 153 / 130, skewed 160 / 131:
-// those take 256 rows from 384 on.)  All three at 55 sizes, and at 40 skewed: profiles/prompt_form_rules.json.
+// those take 256 rows from 384 on.)  32, 128 and 256 rows at 55 sizes, and at 40 skewed: profiles/prompt_form_rules.json.
 int hy_moe_tile(int items, int E, int d, int F, int up) {
     const int64_t G4 = (int64_t)1 << 32, rows = (int64_t)items + 256 * E;
     const bool fits = rows * (d > F ? d : F) * 2 < G4 && (int64_t)up * d * 2 < G4 / 2;   // 32-bit offsets
     const int least = up < d ? up : d;
     const int64_t big = (int64_t)(items / 256) * least / 256;
-    return items <= 16 * E ? 32 : items < (least <= 1024 ? 384 : 192) * E || big < 64 || !fits ? 128 : 256;
+    const int64_t wide = (int64_t)E * (least / 128);
+    if (items <= (wide <= 64 ? 72 : wide < 384 ? 32 : 20) * E) return 32;
+    if (items <= (wide <= 64 ? 320 : wide < 384 ? 88 : 72) * E) return 64;
+    return items < (least <= 1024 ? 384 : 192) * E || big < 64 || !fits ? 128 : 256;
 }
 int hy_moe_max_tiles(int items, int E, int tm) {
     const int n = items / tm + E;   // an expert's last tile may hold a single item
@@ -540,8 +549,9 @@ template <typename F> static hipError_t moe_lds(F kern, int lds) {
 
 // Weights of the experts chosen (one product's, at most) from which their reads are marked as read once: what the memory-side cache holds.  Below
 // it a decoder of few layers finds them there again.  The whole feed-forward, us, plain -> marked: GELU 4096 wide, 32 experts of 2048, top 4:
-// 4 tokens (268 MB each product) 101 -> 89, 16 204 -> 181, 64 (512 MB) 238 -> 210, 128 239 -> 212, but 2 tokens 54 -> 62; 2048 wide, 16 gated experts of
-// 1024 (134 MB), 64 tokens 42 -> 48.
+// 4 tokens (268 MB each product) 101 -> 89, 16 204 -> 181, 64 (512 MB) 238 -> 210, 128 239 -> 212, 400 253 -> 231, but 2 tokens 54 -> 62; 2048 wide, 16
+// gated experts of 1024 (134 MB), 64 tokens 42 -> 48.  And only while nearly every expert has one tile: with more the next tile reads them again from
+// memory (32 rows of a tile, 320 tokens: 249 -> 304; 64 rows, 600 tokens: 286 -> 326; tiles of 128 rows gain 3 % at best and lose 25 % at 1400 tokens).
 constexpr int64_t kOnceBytes = 256 << 20;
 
 template <int TM, bool GATHER, int ACT, bool PLACE = false>
@@ -558,8 +568,8 @@ static void moe_gemm(const uint16_t* x, int64_t rows, const uint16_t* w, uint16_
         auto go = [&](auto kern) {
             kern<<<maxTiles * (N / hy::Tile<TM>::TN), 256, lds, s>>>(x, w, y, meta, maxTiles, top, N, K, limit, slope, shift, idx, items, E);
         };
-        if constexpr (TM == 32)
-            if (std::min<int64_t>(items, E) * N * K * 2 >= kOnceBytes) {
+        if constexpr (TM <= 64)
+            if (std::min<int64_t>(items, E) * N * K * 2 >= kOnceBytes && items <= (TM == 32 ? 20 : 52) * E) {
                 static const hipError_t once = moe_lds(hy::moe_gemm_kernel<TM, GATHER, ACT, PLACE, true>, lds);
                 (void)once;
                 return go(hy::moe_gemm_kernel<TM, GATHER, ACT, PLACE, true>);
@@ -607,8 +617,8 @@ void launch_hy_moe_grouped(const uint16_t* h, const int32_t* idx, const float* w
     if (top == 0) return moe_no_choice(h, out, T, d, s);
     const int tm = hy_moe_tile(T * top, E, d, F, F);
 #define HY_MOE(TM, ACT) moe_grouped<TM, ACT>(h, idx, wt, w_up, w_down, out, meta, z, yrows, T, d, F, E, top, 0.f, 0.f, 0.f, s)
-    if (act == 0) { if (tm == 32) HY_MOE(32, 0); else if (tm == 128) HY_MOE(128, 0); else HY_MOE(256, 0); }
-    else { if (tm == 32) HY_MOE(32, 1); else if (tm == 128) HY_MOE(128, 1); else HY_MOE(256, 1); }
+    if (act == 0) { if (tm == 32) HY_MOE(32, 0); else if (tm == 64) HY_MOE(64, 0); else if (tm == 128) HY_MOE(128, 0); else HY_MOE(256, 0); }
+    else { if (tm == 32) HY_MOE(32, 1); else if (tm == 64) HY_MOE(64, 1); else if (tm == 128) HY_MOE(128, 1); else HY_MOE(256, 1); }
 #undef HY_MOE
 }
 
@@ -622,6 +632,7 @@ void launch_hy_moe_glu_grouped(const uint16_t* h, const int32_t* idx, const floa
     const int tm = hy_moe_tile(T * top, E, d, F, 2 * F);
 #define HY_MOE(TM) moe_grouped<TM, hy::kActGlu>(h, idx, wt, w_gu, w_down, out, meta, z, yrows, T, d, F, E, top, limit, slope, shift, s)
     if (tm == 32) HY_MOE(32);
+    else if (tm == 64) HY_MOE(64);
     else if (tm == 128) HY_MOE(128);
     else HY_MOE(256);
 #undef HY_MOE

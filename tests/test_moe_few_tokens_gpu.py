@@ -78,3 +78,12 @@ def test_ffn(t, top, e, skew, form):
 @pytest.mark.parametrize("t,top,e,d,f", [(3, 2, 8, 4096, 4096), (4, 2, 8, 4096, 4096), (4, 2, 8, 4096, 3968), (300, 2, 40, 2048, 2048)])
 def test_ffn_read_once(t, top, e, d, f):
     _ffn(t, top, e, "even", "gelu", d, f)
+
+
+# tokens per expert at the lines between tiles of 32, 64 and 128 rows, for experts that make few workgroups and more
+@pytest.mark.parametrize("t,top,e,d", [(288, 2, 8, 128), (289, 2, 8, 128), (1280, 2, 8, 128), (1281, 2, 8, 128), (512, 4, 64, 256), (513, 4, 64, 256), (1408, 4, 64, 256), (1409, 4, 64, 256),
+                                       (480, 4, 96, 512), (481, 4, 96, 512), (1728, 4, 96, 512), (1729, 4, 96, 512)])
+@pytest.mark.parametrize("skew", ["even", "one", "holes"])
+@pytest.mark.parametrize("form", ["gelu", "glu"])
+def test_ffn_tiles(t, top, e, d, skew, form):
+    _ffn(t, top, e, skew, form, d, d)
