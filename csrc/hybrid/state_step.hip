@@ -9,7 +9,7 @@
 // instruction.  A workgroup of 4 waves (8 for 256 rows) holds all rows of its columns in registers, every load in flight at once.
 //  q and k are handed to the lanes through LDS, sums over rows go over the lanes of a column, then over the waves.
 // Measured, 64 sequences, 8 heads of 256 x 512 float32 (537 MB): a lane per column took 157 us (3.4 TB/s),
-// this 92 (5.8 TB/s); one sequence: 16.9 and 10.5 us with the gate kernel; delta rule, 16 sequences, 32 heads of 128 x 128: 13.7 and 10.8.
+// this 92 (5.8 TB/s), 71 with the state read and written as data used once (nt: nothing else is pushed out of the caches for it); one sequence: 16.9 and 10.5 us with the gate kernel; delta rule, 16 sequences, 32 heads of 128 x 128: 13.7 and 10.8.
 #include "hybrid_common.h"
 
 namespace chronos {
@@ -45,7 +45,7 @@ __global__ void __launch_bounds__(D >= 128 ? 2 * D : 256) state_step_kernel(cons
     f32x4 S[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i)
-        S[i] = live && !fresh ? *reinterpret_cast<const f32x4*>(Sp + (int64_t)(RI * i) * a.Dv) : f32x4{0.f, 0.f, 0.f, 0.f};
+        S[i] = live && !fresh ? __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(Sp + (int64_t)(RI * i) * a.Dv)) : f32x4{0.f, 0.f, 0.f, 0.f};
     auto total = [&](f32x4 x) {   // the sum over all rows of this lane's columns, in every lane
 #pragma unroll
         for (int o = CL; o < 64; o <<= 1)
@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(D >= 128 ? 2 * D : 256) state_step_kernel(cons
         }
         if (live && t + 1 == t1)
 #pragma unroll
-            for (int i = 0; i < NI; ++i) *reinterpret_cast<f32x4*>(Sp + (int64_t)(RI * i) * a.Dv) = S[i];
+            for (int i = 0; i < NI; ++i) __builtin_nontemporal_store(S[i], reinterpret_cast<f32x4*>(Sp + (int64_t)(RI * i) * a.Dv));
         const f32x4 y = total(x[0] + x[1]) * r;
         if (wv == 0 && rl == 0 && live) *reinterpret_cast<f32x4*>(a.o + ((int64_t)t * a.H + hd) * a.Dv + col) = y;
     };
