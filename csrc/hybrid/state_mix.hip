@@ -15,6 +15,8 @@
 // 128 by 256 8.6 -> 6.8, 18.4 -> 12.8, 16 heads 9.2 -> 6.9, 57.1 -> 56.6; gates, 4 heads of 128 by 256 10.7 -> 6.9, 18.6 -> 12.1.
 #include "hybrid_common.h"
 
+#include <type_traits>
+
 namespace chronos {
 namespace hy {
 
@@ -41,7 +43,8 @@ struct StateMix {
 
 constexpr int mix_threads(int D) { return D >= 128 ? 2 * D : 256; }
 
-template <int D, int CL, int HPW, int FORM>
+// ONCE: the states are read and written as data used once (nt).  (A template: of two branches the compiler makes one again and drops the mark.)
+template <int D, int CL, int HPW, int FORM, bool ONCE>
 __global__ void __launch_bounds__(HPW * mix_threads(D)) state_mix_kernel(const StateMix a) {
     constexpr int NT = mix_threads(D), NW = NT / 64, RI = 64 / CL, NI = D / (NW * RI);
     constexpr bool ROWS = FORM == kMixRows, DELTA = FORM == kMixDelta, GATES = FORM == kMixGates;
@@ -57,8 +60,10 @@ __global__ void __launch_bounds__(HPW * mix_threads(D)) state_mix_kernel(const S
     float* const Sp = a.S + (((int64_t)slot * a.H + hd) * D + row0) * a.Dv + col;
     f32x4 S[NI];
 #pragma unroll
-    for (int i = 0; i < NI; ++i)
-        S[i] = live && !fresh ? *reinterpret_cast<const f32x4*>(Sp + (int64_t)(RI * i) * a.Dv) : f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < NI; ++i) {
+        const f32x4* const p = reinterpret_cast<const f32x4*>(Sp + (int64_t)(RI * i) * a.Dv);
+        S[i] = !live || fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : ONCE ? __builtin_nontemporal_load(p) : *p;
+    }
     f32x4 wn = {0.f, 0.f, 0.f, 0.f};
     if (live) wn = *reinterpret_cast<const f32x4*>(a.w + (int64_t)hd * a.Dv + col);
     // this thread's row of q or k (delta: q rows, then k rows), and what it keeps between tokens
@@ -192,7 +197,11 @@ __global__ void __launch_bounds__(HPW * mix_threads(D)) state_mix_kernel(const S
         }
         if (live && t + 1 == t1)
 #pragma unroll
-            for (int i = 0; i < NI; ++i) *reinterpret_cast<f32x4*>(Sp + (int64_t)(RI * i) * a.Dv) = S[i];
+            for (int i = 0; i < NI; ++i) {
+                f32x4* const p = reinterpret_cast<f32x4*>(Sp + (int64_t)(RI * i) * a.Dv);
+                if constexpr (ONCE) __builtin_nontemporal_store(S[i], p);
+                else *p = S[i];
+            }
         const f32x4 o = total(x[0] + x[1]) * rd;
         // the head's norm and gate: a row's columns lie over CL lanes (dead ones hold 0)
         float ss = o[0] * o[0] + o[1] * o[1] + o[2] * o[2] + o[3] * o[3];
@@ -237,20 +246,26 @@ bool hy_state_mix_ok(int D, int Dv, int heads_per_key) {
     return (D == 64 || D == 128 || D == 256) && Dv % 4 == 0 && Dv >= 4 && Dv <= 256 && (heads_per_key == 1 || (heads_per_key == 2 && D <= 128));
 }
 
-template <int D, int HPW, int FORM>
+template <int D, int HPW, int FORM, bool ONCE>
 static void state_mix_cols(const hy::StateMix& a, int B, hipStream_t s) {
     const dim3 grid(B, a.HK);
     constexpr int nt = HPW * hy::mix_threads(D);
-    if (a.Dv <= 64) hy::state_mix_kernel<D, 16, HPW, FORM><<<grid, nt, 0, s>>>(a);
-    else if (a.Dv <= 128) hy::state_mix_kernel<D, 32, HPW, FORM><<<grid, nt, 0, s>>>(a);
-    else hy::state_mix_kernel<D, 64, HPW, FORM><<<grid, nt, 0, s>>>(a);
+    if (a.Dv <= 64) hy::state_mix_kernel<D, 16, HPW, FORM, ONCE><<<grid, nt, 0, s>>>(a);
+    else if (a.Dv <= 128) hy::state_mix_kernel<D, 32, HPW, FORM, ONCE><<<grid, nt, 0, s>>>(a);
+    else hy::state_mix_kernel<D, 64, HPW, FORM, ONCE><<<grid, nt, 0, s>>>(a);
 }
 template <int HPW, int FORM>
 static void state_mix(const hy::StateMix& a, int B, int D, hipStream_t s) {
     if (B == 0) return;
-    if (D == 64) state_mix_cols<64, HPW, FORM>(a, B, s);
-    else if (D == 128) state_mix_cols<128, HPW, FORM>(a, B, s);
-    else if constexpr (HPW == 1) state_mix_cols<256, HPW, FORM>(a, B, s);
+    // states beyond an L2; smaller ones are found there again at the next step: a decode step of four layers, us, 64 rows of 16 heads (134 MB in two
+    // layers) 758 -> 714, 11 rows (6 MB) 175 -> 171; but 6 rows (3 MB) 169 -> 171, one row 154.6 -> 157.5
+    const bool once = (int64_t)B * a.H * D * a.Dv * 4 >= 4 << 20;
+    auto cols = [&](auto DC) {
+        once ? state_mix_cols<decltype(DC)::value, HPW, FORM, true>(a, B, s) : state_mix_cols<decltype(DC)::value, HPW, FORM, false>(a, B, s);
+    };
+    if (D == 64) cols(std::integral_constant<int, 64>{});
+    else if (D == 128) cols(std::integral_constant<int, 128>{});
+    else if constexpr (HPW == 1) cols(std::integral_constant<int, 256>{});
 }
 
 void launch_hy_delta_step(const uint16_t* proj, int ldp, int q_off, int k_off, int v_off, int g_off, const float* taps, const float* ab, const float* a_log,

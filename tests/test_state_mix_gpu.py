@@ -29,7 +29,8 @@ def _close(a, b, tol):
 # bfloat16 results: the launches round q, k and v between convolution and state (2^-9 each, relative; up to 4 of them reach an output) and
 # the result once more; float32 states see the first of these, or (rows, gates: no rounding between) float32 sums in another order
 @pytest.mark.parametrize("count", [[1, 0, 1, 1, 1], [3, 0, 2, 1, 6]])
-@pytest.mark.parametrize("HK,H,D,Dv", [(2, 4, 64, 40), (2, 2, 64, 64), (1, 2, 128, 128), (3, 3, 128, 72), (2, 4, 128, 256), (2, 2, 256, 132)])
+@pytest.mark.parametrize("HK,H,D,Dv", [(2, 4, 64, 40), (2, 2, 64, 64), (1, 2, 128, 128), (3, 3, 128, 72), (2, 4, 128, 256), (2, 2, 256, 132),
+                                      (8, 16, 128, 128), (13, 13, 128, 128), (12, 12, 128, 128)])   # (states from 4 MB on: read as data used once)
 def test_delta(count, HK, H, D, Dv):
     from chronos.ops import hybrid as hops
 
@@ -50,7 +51,7 @@ def test_delta(count, HK, H, D, Dv):
 
 
 @pytest.mark.parametrize("count", [[1, 0, 1, 1, 1], [3, 0, 2, 1, 6]])
-@pytest.mark.parametrize("H,D,Dv,R", [(2, 64, 40, 16), (4, 128, 256, 16), (3, 128, 72, 7), (2, 256, 132, 1)])
+@pytest.mark.parametrize("H,D,Dv,R", [(2, 64, 40, 16), (4, 128, 256, 16), (3, 128, 72, 7), (2, 256, 132, 1), (7, 128, 256, 16)])
 def test_rows(count, H, D, Dv, R):
     from chronos.ops import hybrid as hops
 
@@ -66,7 +67,7 @@ def test_rows(count, H, D, Dv, R):
 
 
 @pytest.mark.parametrize("count", [[1, 0, 1, 1, 1], [3, 0, 2, 1, 6]])
-@pytest.mark.parametrize("H,D,Dv", [(2, 64, 40), (4, 128, 256), (3, 128, 72), (2, 256, 132)])
+@pytest.mark.parametrize("H,D,Dv", [(2, 64, 40), (4, 128, 256), (3, 128, 72), (2, 256, 132), (5, 256, 192)])
 def test_gates(count, H, D, Dv):
     from chronos.ops import hybrid as hops
 
