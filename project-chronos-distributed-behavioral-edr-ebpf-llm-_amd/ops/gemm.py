@@ -12,7 +12,7 @@ Routing is by measured shape:
   with the kernel, tile config and split-K of the measured plan (``gemm_plan.json``: per (N, K, epilogue) the best
   by M range, from ``scripts/tune_gemm_pp.py`` on one MI355X, random operands, cold weights; plan cfg >= 100 is
   skinny config cfg - 100);
-* shapes that the plan does not list: up to 64 rows ``few_rows_plan``, from 128 on ``many_rows_plan``, between them ``mid_rows_plan``, where their measured ranges say that
+* shapes that the plan does not list: up to 64 rows ``few_rows_plan``, from 128 on ``slab_rows_plan`` (``many_rows_plan``), between them ``mid_rows_plan``, where their measured ranges say that
   they win;
 * hipBLASLt (torch.matmul) only where the plan records that the library wins by more than 3 % (the "plain library
   GEMM" rule), for unlisted shapes outside that range, or for shapes the kernel does not take (K % 64, N % 4).  CHRONOS_PP=lib|own|auto forces a side.
@@ -443,6 +443,55 @@ def many_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     return out
 
 
+# 88 with the x tiles that gemm_slab.hip's slab_rows picks, K split or not: constant, the split's second launch, per 64-deep step of a round of 256 x 256
+# tiles, per MB of weights, per round, per M of all slices' results, per M of results.  Fitted on profiles/slab_rows_gemm.json (rms error 8 %).
+_SLAB_ROWS = (2.0, 2.11, 1.09, 0.118, 1.035, 1.238, 0.829)
+
+
+def _slab_rounds(m: int, nt: int, s: int) -> float:
+    """What slab_rows takes the launch for, in rounds of 256 x 256 tiles."""
+    last = m % 256
+    tail = nt * s if 0 < last <= 128 and nt * s <= 256 and 2 * (m // 256 * nt * s % 256) + nt * s <= 256 else 0
+    tiles = (m // 256 if tail else -(-m // 256)) * nt * s
+    rest = tiles % 256
+    half = 2 * rest + tail if tail or rest <= 128 else 0
+    full = tiles - rest if half else tiles
+    best = -(-full // 256) + (0.57 if full else 0.63) * -(-half // 256)
+    for rows, cost in ((128, 0.61), (160, 0.67), (192, 0.76), (224, 0.86)):
+        t = cost * -(-(-(-m // rows) * nt * s) // 256)
+        if t < best * 0.97:
+            best = t
+    return best
+
+
+def slab_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
+    """many_rows_plan, or (88, split-K) in its place from 257 rows on, by 1024 to 8192 outputs, where the x tiles of 128 to 256 rows make that the faster one: in
+    place of another split by 5 % by the model, of the library where it would have to reach 950 TFLOP/s, which at these sizes it does not.  us, before ->
+    this: 1088 rows of 4096 x 14336 154 -> 119, of 11008 122 -> 98, 1500 153 -> 115, 1088 of 3648 x 8192 84 -> 70, 2100 of 4096 x 4096 82 -> 63.  Of 576 shapes 122 change, 1.18
+    times as fast, one slower by more than 3 % (2446 x 2048 x 4096, 0.90).  Table: profiles/slab_rows_gemm.json, which tests/test_measured_rules.py replays."""
+    out = many_rows_plan(m, n, k)
+    if PP_MODE != "auto" or not 256 < m <= 4096 or out is not None and out[0] != 88:
+        return out
+    m = -(-m // 32) * 32
+    key = (m, n, k, -6)
+    hit = _plan_cache.get(key, False)
+    if hit is not False:
+        return hit
+    if (1024 <= n <= 8192 and k >= 1024 and n * k <= 64_000_000 and _many_fits(m, n, k) and (n, k, PP_PLAIN) not in _plan_file()
+            and (out is not None or mid_rows_plan(m, n, k) is None)):
+        c, times = _SLAB_ROWS, {}
+        for sk in (1, 2, 4, 8, out[1] if out else 1):
+            if k // 64 % sk or k // 64 // sk < 2 or sk > 1 and -(-m // 256) * -(-n // 256) * sk > 768:
+                continue
+            r = _slab_rounds(m, -(-n // 256), sk)
+            times[sk] = c[0] + c[2] * r * (k // 64 // sk) + c[3] * n * k * 2e-6 + c[4] * r + c[6] * m * n * 1e-6 + (sk > 1) * (c[1] + c[5] * sk * m * n * 1e-6)
+        sk = min(times, key=times.get)
+        if times[sk] < 0.95 * (times[out[1]] if out else 5 + 2 * m * n * k / 900e6):
+            out = (88, sk)
+    _plan_cache[key] = out
+    return out
+
+
 def _many_act_pays(m: int, n: int, k: int, glu: bool) -> bool:
     if not _many_fits(m, n, k) or glu and n % 256:
         return False
@@ -733,7 +782,7 @@ def linear(x, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tens
         n = w.shape[0]
         few = None
         if out is None and m > 0 and _plain_rows(x, w):
-            few = (few_rows_plan(m, n, k) if m <= 64 else many_rows_plan(m, n, k) if m >= MANY_MIN else None) or (mid_rows_plan(m, n, k) if 32 < m <= 512 else None)
+            few = (few_rows_plan(m, n, k) if m <= 64 else slab_rows_plan(m, n, k) if m >= MANY_MIN else None) or (mid_rows_plan(m, n, k) if 32 < m <= 512 else None)
         if few is None and gemv_ok(m, n, k):
             return _gemv(x, w)
         for pred, fn in _custom:

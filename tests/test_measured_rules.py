@@ -62,6 +62,21 @@ def test_mid_rows():
         assert G.mid_rows_plan(m, n, k) is None   # (the last: a shape that the measured plan lists)
 
 
+def test_slab_rows():
+    table = _table("slab_rows_gemm.json")
+    ratios = []
+    for row in table["rows"]:
+        m, n, k, library, before, picked = *row[:4], *row[-2:]
+        name = lambda p: None if p is None else "%d/%d" % p  # noqa: E731
+        assert name(G.many_rows_plan(m, n, k)) == before and name(G.slab_rows_plan(m, n, k)) == picked, (m, n, k)
+        if before != picked:
+            of = lambda c: library if c is None else row[table["columns"].index(c)]  # noqa: E731
+            ratios.append(of(before) / of(picked))
+    assert len(ratios) == 122 and _mean(ratios) >= 1.18 and _slower(ratios) <= 1 and min(ratios) >= 0.89
+    for m, n, k in ((256, 4096, 8192), (4128, 4096, 11008), (1100, 1008, 8192), (1100, 8208, 4096), (1100, 5120, 14336)):
+        assert G.slab_rows_plan(m, n, k) == G.many_rows_plan(m, n, k)
+
+
 def _rows(table):
     for row in table["rows"]:
         yield dict(zip(table["columns"], row))

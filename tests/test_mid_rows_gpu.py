@@ -59,3 +59,17 @@ def test_other_operands():
     ops.linear(xg, w).float().sum().backward()
     want = w.float().sum(0)
     assert ((xg.grad.float() - want).abs() <= 2 ** -7 * want.abs() + 0.05 * want.abs().mean()).all()
+
+
+# what slab_rows_plan takes from the library or from whole K: two to eight slices, ragged rows and outputs
+@pytest.mark.parametrize("m,n,k", [(300, 4096, 8192), (1100, 4096, 11008), (1500, 4096, 11008), (2100, 2048, 5632), (2446, 4096, 4096), (1089, 3656, 8192), (1100, 4096, 14336)])
+def test_slab_rows(m, n, k):
+    from chronos import ops
+    from chronos.ops import gemm as G
+
+    plan = G.slab_rows_plan(m, n, k)
+    assert plan is not None and plan[0] == 88 and plan != G.many_rows_plan(m, n, k)
+    x, w = _operands(m, n, k)
+    y = ops.linear(x, w)
+    _check(y, x, w)
+    assert torch.equal(y, G.pp_gemm(x, w, G.PP_PLAIN, plan)[0])
