@@ -523,16 +523,47 @@ Tensor gemm(const Tensor& x, const Tensor& w, bool swiglu, int64_t stages) {
 
 
 // Split-K tickets: one zeroed int buffer per (device, stream), at least n long; every call leaves it zeroed (each
-// group's last arriver resets its own counter), so calls on one stream — and graph replays — share it.
+// group's last arriver resets its own counter), so calls on one stream — and graph replays — share it.  The buffers of a device's first
+// kTicketStreams streams are zeroed before anything runs (tickets_init, with attn_init): one made while a graph is captured
+// would be zeroed by that graph's replays only, and stay as it was found for every later graph of the stream if the first
+// is never replayed.
+constexpr int kTicketStreams = 32;
+constexpr int64_t kTicketInts = 1 << 16;
+static std::mutex g_ticket_mu;
+static int32_t* g_ticket_pool[64] = {nullptr};
+static int g_ticket_used[64] = {0};
+
+static void tickets_init() {
+    std::lock_guard<std::mutex> lk(g_ticket_mu);
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64 || g_ticket_pool[dev]) return;
+    int32_t* p = nullptr;
+    const size_t bytes = kTicketStreams * kTicketInts * sizeof(int32_t);
+    if (hipMalloc(&p, bytes) != hipSuccess) return;
+    if (hipMemset(p, 0, bytes) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
+        (void)hipFree(p);
+        return;
+    }
+    g_ticket_pool[dev] = p;
+}
+
 static int32_t* split_tickets(const Tensor& x, int64_t n) {
-    static std::mutex mu;
-    static std::unordered_map<int64_t, Tensor> cnts;
-    std::lock_guard<std::mutex> lk(mu);
-    const int64_t key = ((int64_t)x.get_device() << 48) ^ (int64_t)(intptr_t)cur_stream();
+    static std::unordered_map<int64_t, std::pair<int32_t*, int64_t>> cnts;
+    static std::vector<Tensor> more;   // beyond the pool
+    std::lock_guard<std::mutex> lk(g_ticket_mu);
+    const int dev = x.get_device();
+    const int64_t key = ((int64_t)dev << 48) ^ (int64_t)(intptr_t)cur_stream();
     auto it = cnts.find(key);
-    if (it == cnts.end() || it->second.numel() < n)
-        it = cnts.insert_or_assign(key, at::zeros({std::max<int64_t>(n, 1 << 16)}, x.options().dtype(at::kInt))).first;
-    return it->second.data_ptr<int32_t>();
+    if (it != cnts.end() && it->second.second >= n) return it->second.first;
+    std::pair<int32_t*, int64_t> b;
+    if (n <= kTicketInts && dev < 64 && g_ticket_pool[dev] && g_ticket_used[dev] < kTicketStreams) {
+        b = {g_ticket_pool[dev] + kTicketInts * g_ticket_used[dev]++, kTicketInts};
+    } else {
+        more.push_back(at::zeros({std::max(n, kTicketInts)}, x.options().dtype(at::kInt)));
+        b = {more.back().data_ptr<int32_t>(), more.back().numel()};
+    }
+    cnts[key] = b;
+    return b.first;
 }
 
 // Batched projection GEMM family (gemm_pp.hip): y = x @ w.T with a fused epilogue, M >= 3.
@@ -974,7 +1005,10 @@ TORCH_LIBRARY(chronos, m) {
           "Tensor block_table, Tensor cos_sin, Tensor(a!) q_out, Tensor(b!) k_cache, Tensor(c!) v_cache, int hq, "
           "int hkv, float k_scale=1.0, float v_scale=1.0, Tensor? ws=None) -> ()");
     m.def("set_decode_gate(Tensor? state, int n) -> ()", &set_decode_gate);
-    m.def("attn_init() -> ()", [] { chronos::attn_init(); });
+    m.def("attn_init() -> ()", [] {
+        chronos::attn_init();
+        tickets_init();
+    });
     m.def("quant_rows(Tensor x, Tensor(a!)? resid, Tensor? w, float eps, int mode) -> (Tensor, Tensor)");
     m.def("qlinear(Tensor xq, Tensor xs, Tensor wq, Tensor ws, bool swiglu) -> Tensor");
     m.def("qgemm_lg(Tensor xq, Tensor xs, Tensor wq, Tensor ws, bool swiglu, int cfg, int splitk) -> Tensor");
