@@ -19,7 +19,7 @@ def test_first_graph_never_replayed():
     stream, pool = torch.cuda.Stream(), torch.cuda.graph_pool_handle()
     dirty = torch.cuda.CUDAGraph()
     with torch.cuda.graph(dirty, pool=pool, stream=stream):   # what lies in the pool's memory
-        junk = [torch.full((1 << 16,), 3, device="cuda", dtype=torch.int32) for _ in range(24)]
+        junk = [torch.full((1 << 16,), 1 << 20, device="cuda", dtype=torch.int32) for _ in range(24)]
     dirty.replay()
     torch.cuda.synchronize()
     del junk
