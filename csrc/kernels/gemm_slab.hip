@@ -238,6 +238,7 @@ __global__ void __launch_bounds__(256) slab_sum_resid_kernel(const float* __rest
 // 69.0, 640 85.6 -> 73.1, in 8 at 272 55.9 -> 46.8, in 2 at 1152 137 -> 116; 6144 x 4096 at 1600 79.0 -> 65.7.
 // In one round all tiles alike are as good as halves or better, because the short last rows of slab_tail come behind all others, where no
 // XCD has their W rows any more (4096 x 14336 in 4 slices at 384 rows 66.8, 63.3 as three tiles of 128 rows).
+// (Beyond two rounds the chip's power decides, which rows that are not there cost too: 28672 x 4096 at 5130 rows 937, as 27 tiles of 192 946.)
 int slab_rows(int M, int nt, int S) {
     constexpr float cost[] = {0.61f, 0.67f, 0.76f, 0.86f};
     const int tail = slab_tail(M, nt, S);
@@ -248,7 +249,7 @@ int slab_rows(int M, int nt, int S) {
     for (int n = 4; n < 8; ++n) {
         const int64_t tiles = (int64_t)((M + 32 * n - 1) / (32 * n)) * nt * S;
         const float t = cost[n - 4] * ((tiles + kSlabCUs - 1) / kSlabCUs);
-        if (t < best * 0.97f) best = t, nm = n;
+        if (t < best * (best > 2.5f ? 0.94f : 0.97f)) best = t, nm = n;
     }
     return nm;
 }

@@ -459,7 +459,7 @@ def _slab_rounds(m: int, nt: int, s: int) -> float:
     best = -(-full // 256) + (0.57 if full else 0.63) * -(-half // 256)
     for rows, cost in ((128, 0.61), (160, 0.67), (192, 0.76), (224, 0.86)):
         t = cost * -(-(-(-m // rows) * nt * s) // 256)
-        if t < best * 0.97:
+        if t < best * (0.94 if best > 2.5 else 0.97):
             best = t
     return best
 
