@@ -1,5 +1,5 @@
-// gemm_slab.hip — projections of many rows: y[M, N] = x[M, K] W[N, K]^T in bfloat16 with float32 sums, 256 x 256 tiles on the
-// slab loop of chronos_slab.h.  A workgroup per CU walks its tiles; the slab pipeline runs on from one tile into the next, and where the
+// gemm_slab.hip — projections of many rows: y[M, N] = x[M, K] W[N, K]^T in bfloat16 with float32 sums, tiles of 256 W rows by 128 to 256 x rows
+// (slab_rows) on the slab loop of chronos_slab.h.  A workgroup per CU walks its tiles; the slab pipeline runs on from one tile into the next, and where the
 // last round would leave half of the CUs idle its tiles are halved.  Config 88 of the projection family (gemm_lg.hip has SwiGLU's split-K).
 //
 // Epilogues, through 4 KiB of LDS per wave so that every store is 16 bytes of a whole line: plain; activation (squared ReLU, GELU); gated

@@ -228,7 +228,8 @@ def few_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     41 -> 21): 1.54 times as fast on average over 622, one slower by more than 3 % (24 rows of 1536 x 5632, 10.3 -> 11.0);
     Beyond, 2 .. 64 rows: _FEW_LARGE, from 33 rows on for less than 12288 outputs, but for _library_streams: library -> this, 16 rows of 4096 x
     4096 15.7 -> 10.6, 4096 x 11008 37.6 -> 21.5, 12288 x 4096 27.7 -> 22.8; 64 rows of 4096 x 14336 39.9 -> 28.5, 2048 x 8192 22.3 -> 13.8;
-    64 rows of 14336 x 4096 would be 27.4 -> 28.8.  Tables: profiles/few_rows_gemm.json, which tests/test_measured_rules.py replays."""
+    the wider ones are mid_rows_plan's.  (Both tables from before the ring tiles' weights were marked as read once, which takes 5 to 12 % off 72, 74,
+    75, 79, 38 and 39; picks are still within 3 % of the best on average.)  Tables: profiles/few_rows_gemm.json, which tests/test_measured_rules.py replays."""
     if 1 < m <= GEMV_MAX_M or PP_MODE != "auto":   # (programs set both while they run: nothing of them in the cache)
         return None
     key = (m, n, k, -1)
