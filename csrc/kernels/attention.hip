@@ -21,6 +21,8 @@
 // of keys past the split end are zeroed so stale cache bytes can never reach the accumulator (p = 0 * NaN guard).
 #include "chronos_hip.h"
 
+#include <type_traits>
+
 namespace chronos {
 
 constexpr int kD = 128;
@@ -388,13 +390,26 @@ constexpr int sd_smem() {
     return ring > merge ? ring : merge;
 }
 
+// Pages that a decode step reads for one sequence alone are marked as read once (nt): memory gives such reads more, and they leave the
+// caches to others.  Pages that sequences share (a prompt's template, a common history) must stay for the next reader, so every
+// sequence compares its table with a neighbour's and marks what is not the neighbour's too.  A decode step of four layers, us, nothing marked, all
+// marked and this:
+//   pages of their own  1024 rows of 120 tokens 2731, 2730, 2672; 1024 of 300 3287, 3181, 3180; 8 of 16000 987, 955, 955; 2 of 131000 (fp8) 1028, 1004, 1006
+//   shared in front     1024 of 120 (6 pages) 2521, 2555, 2524; 1024 of 300 (12 pages) 2813, 2870, 2792; halves: 16 of 2000 694, 726, 708; 16 of 8000
+//                       907, 944, 898; 8 of 30000 (fp8) 919, 928, 891
+// The neighbour's row of the table, or nullptr: there is no other.
+__device__ __forceinline__ const int32_t* neighbour_pages(const int32_t* block_table, int bt_stride, int seq, int rows) {
+    return rows == 1 ? nullptr : block_table + (int64_t)(seq + 1 < rows ? seq + 1 : seq - 1) * bt_stride;
+}
+
 // One 1 KiB LDS-DMA piece as inline asm (lane l's 16 bytes from its own source address to LDS dst + 16 l).  hipcc
 // cannot see it write LDS, so it does not drain the whole ring (vmcnt(0)) before every ds_read of the step being
-// computed; its completion is counted by the kernel's own sd_vmcnt waits (cdna_hip_programming.md §5.7).  nt: one
-// workgroup alone reads a page's head, once, and memory gives such reads more (a decode step of four layers: two rows
-// of 131 k tokens, fp8, 1000 -> 978 us, six of 8 k 697 -> 685).
+// computed; its completion is counted by the kernel's own sd_vmcnt waits.  ONCE: marked as read once
+// (nt), see neighbour_pages.
+template <bool ONCE>
 __device__ __forceinline__ void sd_dma(const void* gsrc, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(gsrc), "s"(lds) : "memory");
+    if constexpr (ONCE) asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(gsrc), "s"(lds) : "memory");
+    else asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gsrc), "s"(lds) : "memory");
 }
 
 template <int N>
@@ -448,13 +463,15 @@ __global__ void __launch_bounds__(256, 1) split_decode_kernel(
     const int ke = min(ctx, ks + chunk);
     const int kl = min(ke, kcap);  // this lane's column: keys past it are masked
     const int32_t* bt = block_table + (int64_t)seq * bt_stride;
+    const int32_t* bn = neighbour_pages(block_table, bt_stride, seq, gridDim.x);
     const float sl2 = FP8 ? scale_log2 * k_scale : scale_log2;  // fp8: K's cache scale folded into the score scale
 
     // stage step t0 (wave-uniform) into ring slot j: pages A = t0 / 16, B = A + 1 (past the range: A again, masked)
-    auto stage = [&](int t0, int j) {
+    auto page_a = [&](int t0) { return bt[t0 / block_size]; };
+    auto page_b = [&](int t0, int a) { return t0 + block_size < ke ? bt[t0 / block_size + 1] : a; };
+    auto stage = [&](auto OC, int64_t pa, int64_t pb, int j) {
+        constexpr bool ONCE = decltype(OC)::value;
         const uint32_t dl = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(ring + j * SB));
-        const int64_t pa = bt[t0 / block_size];
-        const int64_t pb = t0 + block_size < ke ? bt[t0 / block_size + 1] : pa;
         if constexpr (!FP8) {
             // K page: 16 rows x 256 B; piece i of page g = rows 4 i .. +3, lane -> row 4 i + (l >> 4), slot l & 15,
             // holding the row's chunk slot ^ row (the fragment reads then hit 16 distinct slots)
@@ -464,7 +481,7 @@ __global__ void __launch_bounds__(256, 1) split_decode_kernel(
                 const int64_t pg = g ? pb : pa;
                 const uint16_t* src = reinterpret_cast<const uint16_t*>(kcv) +
                                       ((pg * hkv + h) * block_size + row) * kD + 8 * ((lane & 15) ^ row);
-                sd_dma(src, dl + i * 1024);
+                sd_dma<ONCE>(src, dl + i * 1024);
             }
             // V^T page: 128 dims x 32 B contiguous in the cache; piece i of page g = dims 32 (i & 3) .. +31
 #pragma unroll
@@ -473,7 +490,7 @@ __global__ void __launch_bounds__(256, 1) split_decode_kernel(
                 const int64_t pg = g ? pb : pa;
                 const uint16_t* src = reinterpret_cast<const uint16_t*>(vcv) + (pg * hkv + h) * kD * block_size +
                                       (i & 3) * 512 + 8 * lane;
-                sd_dma(src, dl + KB + i * 1024);
+                sd_dma<ONCE>(src, dl + KB + i * 1024);
             }
         } else {
             // fp8 K page: 16 rows x 128 B = 2 pieces (rows 8 i .. +7, lane -> row 8 i + (l >> 3), slot l & 7 holding
@@ -484,7 +501,7 @@ __global__ void __launch_bounds__(256, 1) split_decode_kernel(
                 const int64_t pg = g ? pb : pa;
                 const uint8_t* src = reinterpret_cast<const uint8_t*>(kcv) + ((pg * hkv + h) * block_size + row) * kD +
                                      16 * ((lane & 7) ^ (row & 7));
-                sd_dma(src, dl + i * 1024);
+                sd_dma<ONCE>(src, dl + i * 1024);
             }
 #pragma unroll
             for (int i = 0; i < PV; ++i) {
@@ -492,7 +509,7 @@ __global__ void __launch_bounds__(256, 1) split_decode_kernel(
                 const int64_t pg = g ? pb : pa;
                 const uint8_t* src = reinterpret_cast<const uint8_t*>(vcv) + (pg * hkv + h) * kD * block_size +
                                      (i & 1) * 1024 + 16 * lane;
-                sd_dma(src, dl + KB + i * 1024);
+                sd_dma<ONCE>(src, dl + KB + i * 1024);
             }
         }
     };
@@ -587,20 +604,41 @@ __global__ void __launch_bounds__(256, 1) split_decode_kernel(
     // the wave's steps: t0 = ks + 32 w + 128 i; NB of them in flight (ring slot i % NB)
     const int t_first = ks + 32 * w;
     const int nsteps = t_first < ke ? (ke - t_first + 127) / 128 : 0;
+    auto walk = [&](auto OC, int a0, int b0) {
+        if (NB > 1 && nsteps > 0) stage(OC, a0, b0, 0);
 #pragma unroll
-    for (int i = 0; i < NB - 1; ++i)
-        if (i < nsteps) stage(t_first + 128 * i, i);
-    for (int i = 0; i < nsteps; ++i) {
-        const int ahead = i + NB - 1;
-        const bool more = ahead < nsteps;  // wave-uniform
-        if (more) stage(t_first + 128 * ahead, ahead % NB);
-        // step i landed: the pieces issued after it (up to NB - 1 steps) may stay in flight
-        const int newer = min(nsteps - 1 - i, NB - 1);
-        if (newer >= 2) sd_vmcnt<2 * NP>();
-        else if (newer == 1) sd_vmcnt<NP>();
-        else sd_vmcnt<0>();
-        compute(t_first + 128 * i, i % NB);
+        for (int i = 1; i < NB - 1; ++i)
+            if (i < nsteps) {
+                const int a = page_a(t_first + 128 * i);
+                stage(OC, a, page_b(t_first + 128 * i, a), i);
+            }
+        for (int i = 0; i < nsteps; ++i) {
+            const int ahead = i + NB - 1;
+            const bool more = ahead < nsteps;  // wave-uniform
+            if (more) {
+                const int a = page_a(t_first + 128 * ahead);
+                stage(OC, a, page_b(t_first + 128 * ahead, a), ahead % NB);
+            }
+            // step i landed: the pieces issued after it (up to NB - 1 steps) may stay in flight
+            const int newer = min(nsteps - 1 - i, NB - 1);
+            if (newer >= 2) sd_vmcnt<2 * NP>();
+            else if (newer == 1) sd_vmcnt<NP>();
+            else sd_vmcnt<0>();
+            compute(t_first + 128 * i, i % NB);
+        }
+    };
+    // one look at the middle of the range (rows share the front of their histories; a look at every step costs 4 to 10 %), on its way with the
+    // first step's pages
+    int a0 = 0, b0 = 0;
+    bool own = true;
+    if (nsteps > 0) {
+        a0 = page_a(t_first);
+        b0 = page_b(t_first, a0);
+        const int pm = (ks + ke) / 2 / block_size;
+        own = bn == nullptr || bt[pm] != bn[pm];
     }
+    if (own) walk(std::true_type{}, a0, b0);
+    else walk(std::false_type{}, a0, b0);
     sd_vmcnt<0>();
     __syncthreads();  // the ring is reused as the merge buffer below
 
@@ -726,8 +764,8 @@ constexpr int kPdKlds = 4 * 8192 + 4 * 256;
 // 4 whole 256-B rows each, into the wave's private 8 KiB, XOR-swizzled on the source address) and are read back in
 // the MFMA layout with conflict-free ds_read_b128.  Loaded straight into the MFMA layout each instruction touches 16
 // rows x 64 B, which the L2 -> CU path serves at ~18 B/clk per CU against ~60 for lane-linear LDS-DMA pieces
-// (csrc/microbench/l2_feed.hip, profiles/r3s2_decode_attn.md).  K and V of bf16 pages are read as data used once (nt),
-// which memory serves faster: four layers of 1024 rows, 120 tokens each, 2816 -> 2777 us a step.
+// (csrc/microbench/l2_feed.hip, profiles/r3s2_decode_attn.md).  bf16 pages of one sequence alone are read as data used once
+// (neighbour_pages).
 template <bool FP8, bool PF, bool LEAN, int OCC, bool RP = false, bool KL = true>
 __global__ void __launch_bounds__(256, OCC) paged_decode_kernel(
     const uint16_t* __restrict__ q, const void* __restrict__ kcv, const void* __restrict__ vcv,
@@ -763,6 +801,8 @@ __global__ void __launch_bounds__(256, OCC) paged_decode_kernel(
     // the first 64 block-table entries without waiting for ctx (entries past the context are never shuffled out):
     // the table load, ctx and pos all issue together instead of as a ctx -> table dependent pair
     int btv = lane < bt_stride ? bt[lane] : 0;
+    const int32_t* bn = FP8 ? nullptr : neighbour_pages(block_table, bt_stride, seq, nitems / hkv);
+    const int btn = bn != nullptr && lane < bt_stride ? bn[lane] : -1;
 
     // cascade (shared prefix): a sequence whose first P blocks are the cascade prefix (casc[1..P]) and that has
     // tokens past it starts its walk at token 16 P; casc_prefix_kernel already attended its rows over the prefix and
@@ -850,26 +890,18 @@ __global__ void __launch_bounds__(256, OCC) paged_decode_kernel(
     // accumulator i of S^T[g] is token 8 h4 + 4 g + i and its PV operand element j is token 8 h4 + j — one 16-B V^T
     // load per (lane, 16 dims) instead of two 8-B ones (8 V loads per step instead of 16; the texture addresser was
     // 70-75 % busy on the wave's decode shape, profiles/r3s2_decode_attn_pmc.txt).
+    uint64_t both = __ballot(lane < nblk && btv == btn);   // bit i: the neighbour's entry win + i is the same page
     auto load = [&](int t0, bf16x8 (&kf)[2][4], bf16x8 (&vf)[8]) {
         if (t0 < ctx) {
             const int bi = t0 / block_size;  // page A (B = bi + 1): both must sit in the 64-entry window
             if (bi + 1 >= win + 64) {  // wave-uniform: the window of 64 block-table entries from page A on
                 win = bi;
                 btv = win + lane < nblk ? bt[win + lane] : 0;
+                both = bn == nullptr ? 0 : __ballot(win + lane < nblk && btv == bn[win + lane]);
             }
             const int64_t blkA = __shfl(btv, bi - win, 64);
             // past the context the B lanes re-read page A (valid memory); those tokens are masked in step()
             const int64_t blkB = t0 + block_size < ctx ? (int64_t)__shfl(btv, bi + 1 - win, 64) : blkA;
-            if constexpr (KLDS) {
-                // piece i = step rows 4 i .. 4 i + 3, lane l -> row 4 i + (l >> 4), slot l & 15 <- chunk slot ^ kswz
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const int t = 4 * i + (lane >> 4);
-                    const int64_t pg = t < 16 ? blkA : blkB;
-                    const uint16_t* src = kc + (((pg * hkv + h) * block_size) + (t & 15)) * kD + 8 * ((lane & 15) ^ kswz(t));
-                    __builtin_amdgcn_global_load_lds((pd_gbl_ptr_t)src, (pd_lds_ptr_t)(kl + i * 1024), 16, 0, 2);
-                }
-            }
             const int64_t kblk = r < 8 ? blkA : blkB;
 #pragma unroll
             for (int g = 0; KLDS ? false : g < 2; ++g) {
@@ -895,9 +927,35 @@ __global__ void __launch_bounds__(256, OCC) paged_decode_kernel(
                     vf[dt] = fp8x8_to_bf16x8(v.x, v.y, v_scale);
                 }
             } else {
+                auto bytes = [&](auto OC) {   // K's pieces to LDS, V
+                    constexpr bool ONCE = decltype(OC)::value;
+                    if constexpr (KLDS) {
+                        // piece i = step rows 4 i .. 4 i + 3, lane l -> row 4 i + (l >> 4), slot l & 15 <- chunk slot ^ kswz
 #pragma unroll
-                for (int dt = 0; dt < 8; ++dt)
-                    vf[dt] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(vc + voff + (int64_t)(dt * 16 + r) * block_size));
+                        for (int i = 0; i < 8; ++i) {
+                            const int t = 4 * i + (lane >> 4);
+                            const int64_t pg = t < 16 ? blkA : blkB;
+                            const uint16_t* src = kc + (((pg * hkv + h) * block_size) + (t & 15)) * kD + 8 * ((lane & 15) ^ kswz(t));
+                            __builtin_amdgcn_global_load_lds((pd_gbl_ptr_t)src, (pd_lds_ptr_t)(kl + i * 1024), 16, 0, ONCE ? 2 : 0);
+                        }
+                    }
+#pragma unroll
+                    for (int dt = 0; dt < 8; ++dt) {
+                        const bf16x8* src = reinterpret_cast<const bf16x8*>(vc + voff + (int64_t)(dt * 16 + r) * block_size);
+                        if constexpr (ONCE) vf[dt] = __builtin_nontemporal_load(src);
+                        else vf[dt] = *src;
+                    }
+                };
+                // (the empty statements differ: of two branches of like loads the compiler makes one and drops the mark)
+                if ((both >> (bi - win) & 3) == 0) {
+                    asm volatile("; own pages" ::: "memory");
+                    bytes(std::true_type{});
+                    asm volatile("; own pages read" ::: "memory");
+                } else {
+                    asm volatile("; shared pages" ::: "memory");
+                    bytes(std::false_type{});
+                    asm volatile("; shared pages read" ::: "memory");
+                }
             }
         } else {
 #pragma unroll
