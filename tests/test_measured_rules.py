@@ -107,3 +107,11 @@ def test_many_rows_with_an_activation():
                 taken[glu].append((product + r[apart]) / r[own])
     for glu, count, mean, worst in ((True, 188, 1.11, 0.91), (False, 196, 1.14, 0.89)):
         assert len(taken[glu]) == count and _mean(taken[glu]) >= mean and min(taken[glu]) >= worst
+
+
+def test_vocabulary_rows():
+    table = _table("vocabulary_rows_steps.json")["decode"]
+    for row in table["rows"]:
+        us = dict(zip(table["columns"][1:], row[1:]))
+        cfg, split = G.pp_plan(row[0], 128256, 4096, G.PP_PLAIN)
+        assert split == 1 and us[str(cfg)] <= 1.015 * min(v for v in us.values() if v), row   # (captures of one config differ by 0.7 %)
