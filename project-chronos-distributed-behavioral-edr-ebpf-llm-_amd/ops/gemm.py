@@ -313,7 +313,7 @@ def mid_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
 
 
 # Configs of gemm_slices (csrc/kernels/bindings.cpp)
-_SLICED = (33, 36, 38, 39, 72, 73, 74, 75, 78, 79, *_UNEVEN)
+_SLICED = (19, 32, 33, 36, 38, 39, 72, 73, 74, 75, 78, 79, *_UNEVEN)
 
 
 def product_f32(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:

@@ -63,3 +63,17 @@ def test_float32_products(m, n, k):
     off = (y.double() - want).norm() / want.norm()
     assert off < (k ** 0.5 * 2 ** -23 if own else 2 ** -8)
     assert own or m in (1, 33, 64, 96)
+
+
+# a vocabulary's rows: whichever tiles the rules pick for up to 64 of them, the sums come unrounded
+@pytest.mark.parametrize("m", [2, 32, 33, 48, 64])
+@pytest.mark.parametrize("n,k", [(32768, 1024), (32768, 4096), (12288, 2048), (22016, 2816), (16388, 512)])
+def test_float32_logits_of_any_rows(m, n, k):
+    x, w = _rand(m, k).bfloat16(), (_rand(n, k, seed=1) * k ** -0.5).bfloat16()
+    y = gemm.product_f32(x, w)
+    if n % 16:   # (no rule takes it)
+        assert y is None
+        assert torch.equal(hops.matmul_f32(x, w), hops.matmul(x, w).float())
+    else:
+        want = x.double() @ w.double().t()
+        assert (y.double() - want).norm() / want.norm() < k ** 0.5 * 2 ** -23
