@@ -110,8 +110,9 @@ def test_many_rows_with_an_activation():
 
 
 def test_vocabulary_rows():
-    table = _table("vocabulary_rows_steps.json")["decode"]
-    for row in table["rows"]:
-        us = dict(zip(table["columns"][1:], row[1:]))
-        cfg, split = G.pp_plan(row[0], 128256, 4096, G.PP_PLAIN)
-        assert split == 1 and us[str(cfg)] <= 1.015 * min(v for v in us.values() if v), row   # (captures of one config differ by 0.7 %)
+    tables = _table("vocabulary_rows_steps.json")
+    for key, first in (("decode", 1), ("other contexts", 2)):
+        for row in tables[key]["rows"]:
+            us = dict(zip(tables[key]["columns"][first:], row[first:]))
+            cfg, split = G.pp_plan(row[0], 128256, 4096, G.PP_PLAIN)
+            assert split == 1 and us[str(cfg)] <= 1.015 * min(v for v in us.values() if v), row   # (captures of one config differ by 0.7 %)
