@@ -524,10 +524,11 @@ Tensor gemm(const Tensor& x, const Tensor& w, bool swiglu, int64_t stages) {
 
 // Split-K tickets: one zeroed int buffer per (device, stream), at least n long; every call leaves it zeroed (each
 // group's last arriver resets its own counter), so calls on one stream — and graph replays — share it.  The buffers of a device's first
-// kTicketStreams streams are zeroed before anything runs (tickets_init, with attn_init): one made while a graph is captured
-// would be zeroed by that graph's replays only, and stay as it was found for every later graph of the stream if the first
-// is never replayed.
-constexpr int kTicketStreams = 32;
+// kTicketStreams streams (torch's pools hold 64, and there is the default one) are zeroed before anything runs (tickets_init, with attn_init): one
+// made while a graph is captured would be zeroed by that graph's replays only, and stay as it was found for every later graph of the stream if the
+// first is never replayed.  So what is made in a capture (streams beyond those, larger counts) is that call's alone, held by `own` until its launch is in
+// the graph, and zeroed by every replay.
+constexpr int kTicketStreams = 80;
 constexpr int64_t kTicketInts = 1 << 16;
 static std::mutex g_ticket_mu;
 static int32_t* g_ticket_pool[64] = {nullptr};
@@ -547,7 +548,7 @@ static void tickets_init() {
     g_ticket_pool[dev] = p;
 }
 
-static int32_t* split_tickets(const Tensor& x, int64_t n) {
+static int32_t* split_tickets(const Tensor& x, int64_t n, Tensor& own) {
     static std::unordered_map<int64_t, std::pair<int32_t*, int64_t>> cnts;
     static std::vector<Tensor> more;   // beyond the pool
     std::lock_guard<std::mutex> lk(g_ticket_mu);
@@ -559,7 +560,17 @@ static int32_t* split_tickets(const Tensor& x, int64_t n) {
     if (n <= kTicketInts && dev < 64 && g_ticket_pool[dev] && g_ticket_used[dev] < kTicketStreams) {
         b = {g_ticket_pool[dev] + kTicketInts * g_ticket_used[dev]++, kTicketInts};
     } else {
-        more.push_back(at::zeros({std::max(n, kTicketInts)}, x.options().dtype(at::kInt)));
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(cur_stream(), &st) != hipSuccess) {
+            (void)hipGetLastError();
+            st = hipStreamCaptureStatusActive;   // (a capture elsewhere is in the way of the question)
+        }
+        Tensor z = at::zeros({std::max(n, kTicketInts)}, x.options().dtype(at::kInt));
+        if (st != hipStreamCaptureStatusNone) {
+            own = z;
+            return own.data_ptr<int32_t>();
+        }
+        more.push_back(z);
         b = {more.back().data_ptr<int32_t>(), more.back().numel()};
     }
     cnts[key] = b;
@@ -628,11 +639,11 @@ std::tuple<Tensor, Tensor> gemm_pp(const Tensor& x, const Tensor& w, int64_t mod
         a.nparts_in = (int)part_in->size(1);
     }
     const int64_t tiles = ((M + BM - 1) / BM) * (mode == 1 ? (N / 2) / (BN / 2) : (N + BN - 1) / BN);
-    Tensor ws;
+    Tensor ws, tk;
     if (splitk > 1) {
         ws = at::empty({tiles * splitk * BM * BN}, x.options().dtype(at::kFloat));
         a.ws = ws.data_ptr<float>();
-        if (!chronos::gemm_lg_sliced((int)cfg, (int)mode)) a.cnt = split_tickets(x, tiles);
+        if (!chronos::gemm_lg_sliced((int)cfg, (int)mode)) a.cnt = split_tickets(x, tiles, tk);
     }
     if (lg) {
         CHK(!prio && chronos::launch_gemm_lg((int)cfg, (int)mode, part_in.has_value(), a, cur_stream()), "gemm_lg: launch");
@@ -818,11 +829,11 @@ std::tuple<Tensor, Tensor> gemm_skinny(const Tensor& x, const Tensor& w, int64_t
         a.nparts_in = (int)part_in->size(1);
     }
     const int64_t groups = mode == 1 ? (N / 2) / (8 * RT) : N / (16 * RT);
-    Tensor ws;
+    Tensor ws, tk;
     if (splitk > 1) {
         ws = at::empty({uneven ? splitk * M * N : groups * splitk * 64 * RT * MT * 4}, x.options().dtype(at::kFloat));
         a.ws = ws.data_ptr<float>();
-        if (!uneven) a.cnt = split_tickets(x, groups);
+        if (!uneven) a.cnt = split_tickets(x, groups, tk);
     }
     CHK(chronos::launch_gemm_skinny((int)cfg, (int)mode, part_in.has_value(), a, cur_stream()), "gemm_skinny: launch");
     return {y, part_out};
@@ -914,11 +925,11 @@ Tensor qgemm_lg(const Tensor& xq, const Tensor& xs, const Tensor& wq, const Tens
     Tensor y = at::empty({M, swiglu ? N / 2 : N}, xq.options().dtype(at::kBFloat16));
     a.y = bfm(y);
     const int64_t tiles = ((M + BM - 1) / BM) * (swiglu ? (N / 2) / (BN / 2) : (N + BN - 1) / BN);
-    Tensor wsl;
+    Tensor wsl, tk;
     if (splitk > 1) {
         wsl = at::empty({tiles * splitk * BM * BN}, xs.options());
         a.ws = wsl.data_ptr<float>();
-        a.cnt = split_tickets(xq, tiles);
+        a.cnt = split_tickets(xq, tiles, tk);
     }
     CHK(chronos::launch_gemm_lg_f8((int)cfg, swiglu, a, cur_stream()), "qgemm_lg: launch");
     return y;
