@@ -282,11 +282,12 @@ _MID = ((64, {39: (0.247, 3.535, 0.273, 0.037, 1.296, 0.257, 0.392, 2.906), 19: 
 def mid_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     """(config, split-K) of the hand-written GEMM for rows and shapes that few_rows_plan, many_rows_plan and the measured plan leave, or None (the library):
     65 .. 128 rows, 33 .. 64 rows by 12288 outputs and more, 129 .. 256 rows by up to 4096 outputs, 257 .. 512 by up to 2048 with K <= 8192; outputs and K
-    from 512 on.  Rows beyond 64 count in 32s, so that a server's steps find their plan again.  us, library -> this: 80 rows of 1024 x 1024 10.9 ->
+    from 512 on, outputs to 153600, K to 32768 (28672 from 129 rows on) and 640 M weights, which is what was measured.  Rows beyond 64 count in 32s, so that a server's steps find their plan again.  us, library -> this: 80 rows of 1024 x 1024 10.9 ->
     6.6, 4096 x 4096 17.1 -> 13.9, 2048 x 5632 16.4 -> 12.2, 12288 x 4096 33.4 -> 28.0, 32768 x 1024 22.9 -> 17.0; 64 rows of 14336 x 4096 28.6 ->
-    26.8, 32768 x 4096 62.2 -> 55.4; 192 rows of 1024 x 1024 10.7 -> 7.5, 2048 x 5632 21.2 -> 19.1; 512 rows of 1024 x 4096 15.8 -> 14.7.  On average 1.29
+    26.8, 32768 x 4096 62.2 -> 58.3 (39 would be 55.4: the model is off there); 192 rows of 1024 x 1024 10.7 -> 7.5, 2048 x 5632 21.2 -> 19.1; 512 rows of 1024 x 4096 15.8 -> 14.7.  On average 1.29
     (460 shapes of 65 .. 128 rows), 1.21 (105 of 33 .. 64), 1.21 (123 of 129 .. 256) and 1.10 times (86) as fast, of 774 shapes 35 slower by more than 3 %,
-    the worst by 9 % (512 x 1408, 8.4 -> 9.2); and a library call costs the host 22 us, this 7.  Beyond these ranges the two are level or the
+    the worst by 9 % (512 x 1408, 8.4 -> 9.2); 58 shapes beyond the fit's, up to 622 M weights and K = 32768: 1.29
+    times, 5 slower, the worst by 7 %; and a library call costs the host 22 us, this 7.  Beyond these ranges the two are level or the
     library ahead.  Table: profiles/mid_rows_gemm.json, which tests/test_measured_rules.py replays."""
     if PP_MODE != "auto":
         return None
@@ -297,7 +298,7 @@ def mid_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
         return hit
     out = best = None
     if ((m > 32 and n >= 12288 if m <= 64 else n >= 512 if m <= 128 else 512 <= n <= 4096 if m <= 256 else m <= 512 and 512 <= n <= 2048 and k <= 8192)
-            and k >= 512 and n % 16 == 0 and k % 64 == 0 and k <= 1 << 20 and (n + 128) * k < 1 << 30
+            and 512 <= k <= (32768 if m <= 128 else 28672) and n % 16 == 0 and k % 64 == 0 and n <= 153600 and n * k <= 640_000_000
             and (n, k, PP_PLAIN) not in _plan_file()):
         for cfg, c in next(models for most, models in _MID if m <= most).items():
             for sk in (1, 2, 4, 8) if cfg == 39 else (1,):

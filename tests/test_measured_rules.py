@@ -58,7 +58,10 @@ def test_mid_rows():
                 assert "%d/%d" % plan == row[-1], (m, n, k)
                 ratios.append(library / row[table["columns"].index(row[-1])])
         assert len(ratios) == count and _mean(ratios) >= mean and _slower(ratios) <= slower and min(ratios) >= worst
-    for m, n, k in ((32, 16384, 1024), (129, 4112, 1024), (257, 2064, 1024), (512, 2048, 8256), (513, 1024, 1024), (100, 496, 1024), (100, 1024, 448), (64, 8192, 1024), (100, 1032, 1024), (100, 1024, 1056), (100, 6144, 4096)):
+    assert all("%d/%d" % G.mid_rows_plan(*row[:3]) == row[-1] for row in table["beyond"])
+    ratios = [row[3] / row[table["columns"].index(row[-1])] for row in table["beyond"]]
+    assert len(ratios) == 58 and _mean(ratios) >= 1.28 and _slower(ratios) <= 5 and min(ratios) >= 0.92
+    for m, n, k in ((32, 16384, 1024), (64, 153616, 1024), (100, 153616, 1024), (100, 1024, 32832), (256, 1024, 28736), (100, 151936, 4288), (129, 4112, 1024), (257, 2064, 1024), (512, 2048, 8256), (513, 1024, 1024), (100, 496, 1024), (100, 1024, 448), (64, 8192, 1024), (100, 1032, 1024), (100, 1024, 1056), (100, 6144, 4096)):
         assert G.mid_rows_plan(m, n, k) is None   # (the last: a shape that the measured plan lists)
 
 
