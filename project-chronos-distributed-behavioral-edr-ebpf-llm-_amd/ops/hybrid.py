@@ -95,7 +95,7 @@ def embed_rows(ids, table, act_dtype, scale: float = 1.0, emit: bool = True):
 
 def embed_start(ids, table, act_dtype, scale: float, emit: bool, pos, q_start):
     """embed_rows and, behind them, pos at every sequence's first token (int32 [B]; sequences without tokens: at the next one's, or the last)."""
-    if _gpu(table) and ids.numel() and pos.numel() == ids.numel():
+    if _gpu(table) and ids.numel() and pos.numel() == ids.numel() and all(t.dtype == torch.int32 and t.is_contiguous() for t in (pos, q_start)):
         both = emit and not _f32(act_dtype)
         x, h, pos0 = _k().hy_embed_start(ids, table, scale, both, pos, q_start)
         return x, (h if both else x if emit else None), pos0

@@ -27,6 +27,17 @@ def test_first_positions(lens, dt, d):
         assert torch.equal(p0, pos[qs[:-1].long().clamp(max=T - 1)])
 
 
+def test_first_positions_of_other_layouts():
+    """Positions that only the first of a sequence are taken of may lie in any stride and type, as the sequences' starts may."""
+    qs = torch.tensor([0, 3, 7], device=DEV)
+    pos = torch.arange(100, 114, dtype=torch.int32, device=DEV)[::2]
+    ids, table = torch.arange(7, dtype=torch.int32, device=DEV), _rand(50, 64).bfloat16()
+    for p, q in ((pos, qs.int()), (pos.long(), qs.int()), (pos.contiguous(), qs), (pos, qs)):
+        x, h, p0 = hops.embed_start(ids, table, torch.bfloat16, 1.0, True, p, q)
+        wx, wh = ref.embed_rows(ids, table, torch.bfloat16, 1.0, True)
+        assert torch.equal(x, wx) and torch.equal(h, wh) and p0.dtype == p.dtype and p0.tolist() == [100, 106]
+
+
 @pytest.mark.parametrize("d", [64, 1024, 1028, 4096, 4100, 30])
 @pytest.mark.parametrize("idx", [[3], [0, 8, 8, 2, 5], []])
 def test_chosen_rows(d, idx):
