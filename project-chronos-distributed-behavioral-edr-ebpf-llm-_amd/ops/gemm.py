@@ -228,8 +228,10 @@ def few_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     41 -> 21): 1.54 times as fast on average over 622, one slower by more than 3 % (24 rows of 1536 x 5632, 10.3 -> 11.0);
     Beyond, 2 .. 64 rows: _FEW_LARGE, from 33 rows on for less than 12288 outputs, but for _library_streams: library -> this, 16 rows of 4096 x
     4096 15.7 -> 10.6, 4096 x 11008 37.6 -> 21.5, 12288 x 4096 27.7 -> 22.8; 64 rows of 4096 x 14336 39.9 -> 28.5, 2048 x 8192 22.3 -> 13.8;
-    the wider ones are mid_rows_plan's.  (Both tables from before the ring tiles' weights were marked as read once, which takes 5 to 12 % off 72, 74,
-    75, 79, 38 and 39; picks are still within 3 % of the best on average.)  Tables: profiles/few_rows_gemm.json, which tests/test_measured_rules.py replays."""
+    the wider ones are mid_rows_plan's.  (Both tables and the figures here are from before the ring tiles' weights were marked as read once, which takes 5 to
+    12 % off 72, 74, 75, 79, 38 and 39.  Measured again with it, mid_rows_plan's among them: 1072 shapes 1.43 times as fast as the library, 8 slower by more than 3 %, the
+    worst by 11 % (64 rows of 12288 x 5632, 34.2 -> 38.1); picks take 2 % longer than the best on average, 4 % from 33 rows on; of 84 shapes that are left to the library 61
+    would be faster here by more than 3 %, up to 1.24 times, 8192 x 6144 by 2 to 40 rows.)  Tables: profiles/few_rows_gemm.json, which tests/test_measured_rules.py replays."""
     if 1 < m <= GEMV_MAX_M or PP_MODE != "auto":   # (programs set both while they run: nothing of them in the cache)
         return None
     key = (m, n, k, -1)
@@ -423,7 +425,9 @@ def many_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     fast as the library on average (302 shapes; 25 slower by more than 3 %, the worst by 14 %: whole or part rounds at K up to 2048, where the library's
     first loads and stores cost less, and rounds that are nearly full); at 260 shapes drawn off the grid 1.16 times (162; 16 slower, the worst 13 %);
     below the line 0.84 times.  A library call also costs the host 22 us, this 7.  Rows count in 128s, so that a server's
-    steps of any size find their plan again.  Tables: profiles/many_rows_gemm.json, which tests/test_measured_rules.py replays."""
+    steps of any size find their plan again.  (Measured with 256 x 256 tiles and halves only, on one card.  With 88's x tiles by rows, slab_rows_plan's
+    and mid_rows_plan's picks among them, on another: 781 shapes 1.15 times as fast, 100 slower by more than 3 %, the worst by 23 %, most of them one round of 19 or 32,
+    which were no faster there before: 256 x 4096 x 2048 13.4 and 16.4, 1536 x 2048 x 5632 44.4 and 54.0.)  Tables: profiles/many_rows_gemm.json, which tests/test_measured_rules.py replays."""
     if PP_MODE != "auto":
         return None
     m = -(-m // 128) * 128

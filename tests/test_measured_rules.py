@@ -119,3 +119,20 @@ def test_vocabulary_rows():
             us = dict(zip(tables[key]["columns"][first:], row[first:]))
             cfg, split = G.pp_plan(row[0], 128256, 4096, G.PP_PLAIN)
             assert split == 1 and us[str(cfg)] <= 1.015 * min(v for v in us.values() if v), row   # (captures of one config differ by 0.7 %)
+
+
+def _linear(m, n, k):
+    """The plan that linear() takes a plain product by."""
+    return (G.few_rows_plan(m, n, k) if m <= 64 else G.slab_rows_plan(m, n, k) if m >= G.MANY_MIN else None) or (G.mid_rows_plan(m, n, k) if 32 < m <= 512 else None)
+
+
+def test_the_tables_measured_again():
+    for name, key, count, mean, slower, worst in (("few_rows_gemm.json", "weights read once", 1072, 1.43, 8, 0.89), ("many_rows_gemm.json", "by rows", 781, 1.15, 100, 0.81)):
+        ratios, behind = [], []
+        for r in _rows(_table(name)[key]):
+            plan = _linear(r["m"], r["n"], r["k"])
+            assert (None if plan is None else "%d/%d" % plan) == r["picked"], r
+            if plan is not None:
+                ratios.append(min(r.get("library", r.get("lib")), r.get("gemv") or math.inf) / r["us"])
+                behind.append(r["us"] / r.get("best_us", r["us"]))
+        assert len(ratios) == count and _mean(ratios) >= mean and _slower(ratios) <= slower and min(ratios) >= worst and _mean(behind) <= 1.021, name
