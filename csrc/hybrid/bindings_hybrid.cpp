@@ -1255,6 +1255,10 @@ Tensor hy_unrotate_gate(const Tensor& o, const Tensor& pos, const c10::optional<
 
 TORCH_LIBRARY_FRAGMENT(chronos, m) {
     m.def("hy_embed(Tensor ids, Tensor table, float scale=1.0) -> Tensor");
+    m.def("hy_moe_tile(int items, int E, int d, int F, int up) -> int", [](int64_t items, int64_t E, int64_t d, int64_t F, int64_t up) {
+        need(items >= 0 && E >= 1 && d >= 1 && F >= 1 && up >= 1 && std::max({items, E, d, F, up}) < (1LL << 31), "moe_tile: sizes");
+        return (int64_t)chronos::hy_moe_tile((int)items, (int)E, (int)d, (int)F, (int)up);
+    });
     m.def("hy_state_mix_ok(int D, int Dv, int heads_per_key, int cols) -> bool", &hy_state_mix_ok);
     m.def("hy_delta_step(Tensor proj, Tensor taps, Tensor ab, Tensor a_log, Tensor q_start, Tensor pos0, Tensor slots, Tensor(a!) hist, Tensor(b!) S, "
           "int HK, int H, int D, int Dv, float q_mul, int g_off, Tensor w, float eps) -> Tensor");

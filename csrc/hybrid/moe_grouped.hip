@@ -515,7 +515,12 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(const uint16_t* __rest
 // 8 experts of 1024 by 512 (wide 32), top 2, 128 tokens (32 items per expert) 20 / 28 / 33, 320 24 / 28 / 35, 1000 - / 32 / 39, 1400 - / 36 / 42; 16 of
 // 2048 by 1408 (176), top 4, 96 tokens 39 / 48 / 58, 160 60 / 49 / 61, 256 68 / 56 / 66, 400 - / 72 / 67; 32 of 4096 by 2048 (512), top 4, 160 218 / 230 /
 // 266, 200 248 / 231 / 269, 400 259 / 231 / 279, 600 310 / 286 / 288, 800 - / 299 / 291; with expert e chosen in proportion to 1 / e 200 tokens 230 / 233 / 339,
-// 400 274 / 253 / 348, 600 324 / 299 / 348, 1400 - / 438 / 405.  128 against 256, on gated
+// 400 274 / 253 / 348, 600 324 / 299 / 348, 1400 - / 438 / 405.  Beyond 56 items an expert takes two tiles of 64, and where the two products'
+// tile columns (cols) then make more than two rounds of 512 workgroups 128 rows are faster, evenly chosen: 16 gated of 2048 by 1408, 64 and 80 items 75 for
+// 90, 78 for 97; 64 of 1024 by 512, 80 items 57 for 70; 32 gated of 4096 by 2048, 64 items 340 for 364; unevenly chosen ones lose by it there (64 gated of 2048 by
+// 1024, choice as 1 / e, 64 items 243 for 217).  Over 17 shapes of experts, gated and not, 21 numbers of items, even and as 1 / e: 2.5 % behind the best of the three on
+// average, 1.09 times as fast as 32 rows to 16 items and 128 beyond, 27 of 1428 slower than that by more than 3 %, the worst by 22 % (64 gated of 1024 by 512, 52 items).
+// profiles/moe_tiles.json, which tests/test_measured_rules.py replays.  128 against 256, on gated
 // experts, us at 32 / 128 / 256 rows: 16 experts of 2048 by 1024, 512
 // tokens 81 / 66 / 62, 2048 tokens 248 / 154 / 150, 8192 tokens 870 / 516 / 407; 32 experts of 4096 by 1536 with 512 tokens 329 / 282 / 323,
 // 1536 tokens 606 / 424 / 352, 8192 tokens 2640 / 1610 / 1180; 8 experts of 1024 by 512 with 1024 tokens (2 each) 39 / 35 / 39, 8192 tokens
@@ -530,7 +535,8 @@ int hy_moe_tile(int items, int E, int d, int F, int up) {
     const int64_t big = (int64_t)(items / 256) * least / 256;
     const int64_t wide = (int64_t)E * (least / 128);
     if (items <= (wide <= 64 ? 72 : wide < 384 ? 32 : 20) * E) return 32;
-    if (items <= (wide <= 64 ? 320 : wide < 384 ? 88 : 72) * E) return 64;
+    const int64_t cols = wide + (int64_t)E * ((up < d ? d : up) / 128);
+    if (items <= (wide <= 64 ? 320 : cols > 512 ? 56 : wide < 384 ? 88 : 72) * E) return 64;
     return items < (least <= 1024 ? 384 : 192) * E || big < 64 || !fits ? 128 : 256;
 }
 int hy_moe_max_tiles(int items, int E, int tm) {

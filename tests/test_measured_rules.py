@@ -136,3 +136,20 @@ def test_the_tables_measured_again():
                 ratios.append(min(r.get("library", r.get("lib")), r.get("gemv") or math.inf) / r["us"])
                 behind.append(r["us"] / r.get("best_us", r["us"]))
         assert len(ratios) == count and _mean(ratios) >= mean and _slower(ratios) <= slower and min(ratios) >= worst and _mean(behind) <= 1.021, name
+
+
+def test_tiles_of_experts():
+    import torch
+
+    from chronos.ops import hybrid as hops
+
+    hops.load()
+    behind, before = [], []
+    for r in _rows(_table("moe_tiles.json")):
+        items, up = r["T"] * r["top"], r["F"] * (2 if r["form"] == "glu" else 1)
+        tile = torch.ops.chronos.hy_moe_tile(items, r["E"], r["d"], r["F"], up)
+        us = r[str(min(tile, 128))]   # (256 rows are another rule's, over 128)
+        behind.append(min(r["32"], r["64"], r["128"]) / us)
+        before.append(r["32" if items <= 16 * r["E"] else "128"] / us)
+    assert len(behind) == 1428 and _mean(behind) >= 1 / 1.026 and min(behind) >= 1 / 1.42
+    assert _mean(before) >= 1.08 and _slower(before) <= 27 and min(before) >= 1 / 1.23
