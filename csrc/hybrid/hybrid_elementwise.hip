@@ -10,7 +10,7 @@ namespace chronos {
 namespace hy {
 
 // h (or nullptr): the rows in bfloat16 as well.  pos0 (or nullptr) [B]: pos at every sequence's first token, which a prompt step's recurrences
-// ask for; sequences without tokens read the last one's.  Here it costs nothing (three launches of torch's, 4.7 us each and 10 us of the host's
+// ask for; sequences without tokens read the next one's, or the last.  Here it costs nothing (three launches of torch's, 4.7 us each and 10 us of the host's
 // time, which is what bounds prompts of a few hundred tokens).
 template <typename T>
 __global__ void __launch_bounds__(256) embed_kernel(const int32_t* __restrict__ ids, const T* __restrict__ table,

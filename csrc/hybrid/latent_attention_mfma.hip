@@ -325,8 +325,9 @@ __global__ void __launch_bounds__(64 * NW) latent_attention_mfma_kernel(
 
 // one wave per (token, head) row and 256 columns: out = sum_z 2^(m_z - m) O_z / (sum_z 2^(m_z - m) l_z + 2^(sink log2 e - m)) * sigmoid(gate)
 // (the partial maxima are in the base-2 domain: score * scale * log2 e).  Lane z holds
-// split z's maximum and sum (nsplit <= 64); a lane then sums 4 neighbouring columns over the splits.  16 splits' columns are on their way before
+// split z's maximum and sum; a lane then sums 4 neighbouring columns over the splits, all on their way before
 // the maxima are looked at: a few rows are one memory latency, not one per four splits behind another: 6 rows of 8 heads in 13 splits 6.7 -> 3.6 us.
+constexpr int kLatentSplits = 16;   // at most (hy_latent_nsplit)
 __global__ void __launch_bounds__(256) latent_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                                              const float* __restrict__ gate, uint16_t* __restrict__ out,
                                                              int64_t rows, int rank, int nsplit,
@@ -337,10 +338,9 @@ __global__ void __launch_bounds__(256) latent_combine_kernel(const float* __rest
     if (r >= rows) return;
     const int c = (int)(it - r * nc) * 256 + lane * 4;    // (rank is a multiple of 16; lanes past it read its last columns)
     const float* const po = part_o + r * nsplit * rank + min(c, rank - 4);
-    constexpr int U = 16;
-    f32x4 v[U];
+    f32x4 v[kLatentSplits];
 #pragma unroll
-    for (int z = 0; z < U; ++z)
+    for (int z = 0; z < kLatentSplits; ++z)
         if (z < nsplit) v[z] = *reinterpret_cast<const f32x4*>(po + (int64_t)z * rank);
     const float mz = lane < nsplit ? part_ml[(r * nsplit + lane) * 2] : -INFINITY;
     const float lz = lane < nsplit ? part_ml[(r * nsplit + lane) * 2 + 1] : 0.f;
@@ -351,10 +351,8 @@ __global__ void __launch_bounds__(256) latent_combine_kernel(const float* __rest
     e *= (gate != nullptr ? sigmoidf_(gate[r]) : 1.f) / l;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int z = 0; z < U; ++z)
+    for (int z = 0; z < kLatentSplits; ++z)
         if (z < nsplit) acc += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(e), z)) * v[z];
-    for (int z = U; z < nsplit; ++z)
-        acc += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(e), z)) * *reinterpret_cast<const f32x4*>(po + (int64_t)z * rank);
     if (c < rank) *reinterpret_cast<u16x4*>(out + r * rank + c) = u16x4{f2bf(acc[0]), f2bf(acc[1]), f2bf(acc[2]), f2bf(acc[3])};
 }
 
@@ -391,7 +389,7 @@ int hy_latent_nsplit(int wgs, int max_ctx, bool windowed) {
     if (wgs >= 128) return 1;
     int want = (256 + wgs - 1) / wgs, cap = max_ctx / ((windowed ? 2 : 1) * hy::MKT);
     if (!windowed && cap < 3) cap = 1;
-    if (want > 16) want = 16;
+    if (want > hy::kLatentSplits) want = hy::kLatentSplits;
     if (want > cap) want = cap;
     return want < 1 ? 1 : want;
 }

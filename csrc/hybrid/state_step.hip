@@ -8,8 +8,13 @@
 // What bounds it is the state's traffic, so a lane takes 16 bytes of a row: CL lanes a row's 4 CL columns, 64 / CL rows per
 // instruction.  A workgroup of 4 waves (8 for 256 rows) holds all rows of its columns in registers, every load in flight at once.
 //  q and k are handed to the lanes through LDS, sums over rows go over the lanes of a column, then over the waves.
-// Measured, 64 sequences, 8 heads of 256 x 512 float32 (537 MB): a lane per column took 157 us (3.4 TB/s),
-// this 92 (5.8 TB/s), 71 with the state read and written as data used once (nt: nothing else is pushed out of the caches for it); one sequence: 16.9 and 10.5 us with the gate kernel; delta rule, 16 sequences, 32 heads of 128 x 128: 13.7 and 10.8.
+// Measured, 64 sequences, 8 heads of 256 x 512 float32 (537 MB read and written): a lane per column took 157 us, this 92; one sequence: 16.9 and
+// 10.5 us with the gate kernel; delta rule, 16 sequences, 32 heads of 128 x 128: 13.7 and 10.8.
+// The state is read and written as data used once (nt).  Eight layers' states in turn, us, plain, reads alone marked, writes alone, both: 64 sequences
+// 116, 112, 120, 107 (5.0 TB/s); 16 28.9, 24.2, 29.9, 22.9; 4 9.8, 9.4, 9.8, 7.9; one 5.7, 5.8, 5.6, 5.4; heads of 32 x 64 and 64 x 64 level.  (One
+// state stepped over and over, which no decoder does, finds half of itself in the memory-side cache unmarked: 84, marked 106.)  More is gained by
+// what stays cached beside it: in a decode step of 64 rows, two of four layers so, the kernel takes 106 us for 100 and the latent attention behind it
+// 52 for 71; the step 878 for 913 (reads alone 901, writes alone 907), 32 rows 650 for 683, 16 rows and fewer level.
 #include "hybrid_common.h"
 
 namespace chronos {

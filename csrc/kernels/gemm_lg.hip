@@ -108,7 +108,10 @@ __device__ __forceinline__ int lg_swz64(int row) { return (4 - ((row >> 2) & 3))
 // Memory gives such reads 12 % more: 1 GB 181 -> 162 us, 180 MB 37.5 -> 34.8, 117 MB 22.7 -> 21.0 by themselves; products of 2 / 16 rows, us: 128256 x
 // 4096 183 -> 167 / 188 -> 170, 32768 x 4096 56.3 -> 51.0 / 58.4 -> 52.7, 22016 x 4096 41.5 -> 37.5 / 42.4 -> 38.6, 4096 x 14336 in 4 slices 27.1 -> 24.7 /
 // 26.9 -> 25.0; of 128 rows 28672 x 4096 59.6 -> 57.3, 4096 x 4096 31.7 -> 29.5, of 96 rows 4096 x 14336 in 4 slices 47.2 -> 44.8; tiles of 256 rows
-// gain nothing.  Read by two workgroups they are slower for it: 128256 x 4096 by 64 rows on 32-row tiles 267 -> 320.
+// gain nothing.  Read by two workgroups they are slower for it: 128256 x 4096 by 64 rows on 32-row tiles 267 -> 320.  No line by size: products by themselves
+// gain at every one (8 rows, us, in turn over 1.2 GB, 300 MB, 150 MB of weights: 2048 x 1024 5.8 -> 5.6, 5.6 -> 5.0, 5.7 -> 5.1; 8192 x 2048 10.0 -> 9.5, 10.2 -> 8.5, 11.3 ->
+// 9.8; 32768 x 4096 59.6 -> 51.2, 64.3 -> 47.1, 65.1 -> 47.0).  Of 44 decode steps of hybrid decoders (2 - 64 rows, widths 1024 - 4096) the mark makes all up to 7 % faster or level but for
+// 6 to 16 rows of width 2048, up to 3 % slower (12 rows 280 -> 290): four such layers and the head together just about fill the memory-side cache.
 template <int WN, int XM, int RB, int ST, int MODE, bool NORMP, int NWX, int ABL = 0, int VAR = 0, bool F8 = false, bool ONCE = false>
 __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
     constexpr bool STG = VAR == 1, MAN = VAR == 2;
