@@ -1058,7 +1058,7 @@ def mix_delta_rule(model, li: int, spec: DeltaRuleSpec, w: dict, h, meta: StepMe
 def mix_gla(model, li: int, spec: GLASpec, w: dict, h, meta: StepMeta, cache: HybridCache):
     H, D, Dv = spec.heads, spec.dim, spec.vdim
     proj, low = hops.matmul_rowdot(h, w["w_proj"], w["w_a1"], None, w.get("joined"))   # q | k | v | g; the decay's latent
-    if hops.one_step_ok(proj, meta.max_q, D, Dv, 1, cache.S[li], w["norm"]):
+    if hops.rows_step_pays(proj.shape[0], H, D, Dv, low.shape[1]) and hops.one_step_ok(proj, meta.max_q, D, Dv, 1, cache.S[li], w["norm"]):
         o = hops.rows_step(proj, low, w["w_a2t"], w["b_a2"], 1.0 / spec.tau, meta.q_start, meta.pos0, meta.slots, cache.S[li], H, D, Dv, D ** -0.5,
                            2 * H * D + H * Dv, w["norm"], model.cfg.norm_eps)
         return _with_gate(model.last_product(o, w["w_o"]), proj, w)

@@ -357,6 +357,17 @@ def linear_scan(proj, q_off: int, k_off: int, v_off: int, qscale, kscale, q_mul:
                            H, D, Dv, vscale)
 
 
+def rows_step_pays(B: int, H: int, D: int, Dv: int, rank: int) -> bool:
+    """rows_step or the launches that it stands for?  Every workgroup, one of a row and head, multiplies its head's decays out itself: few of them wait less for
+    it than a launch takes, many pay for it from 100 MB of its weights between them on; and a lane of 256 x 256 states does not have the registers.  us, launches and one: 128 x 128, 32 heads, 1, 64
+    and 128 rows: rank 16 10.0 and 6.6, 57 and 53, 97 and 94; 128 22 and 10, 72 and 68, 111 and 137; 256 36 and 13, 90 and 112, 132 and 216.  256 x 256, rank 16, 1 row of 4
+    heads 10.1 and 13.5, 64 of 16 105 and 118; rank 128 22 and 17, 120 and 153.  Table: profiles/decode_forms.json, which tests/test_measured_rules.py
+    replays."""
+    if D == 256 and Dv > 128:
+        return 64 <= rank <= 256 and B * H <= 400
+    return rank <= 32 or rank <= 256 and B * H * rank * D <= (34_000_000 if B * H <= 2048 else 27_000_000)
+
+
 def one_step_ok(proj, max_q: int, D: int, Dv: int, heads_per_key: int, *operands) -> bool:
     """May a recurrent mixer's part between its projections run as one launch (delta_step, rows_step, mlstm_step)?  For decode rows, max_q 1; ``operands``:
     what it reads 16 bytes at a time."""

@@ -153,3 +153,17 @@ def test_tiles_of_experts():
         before.append(r["32" if items <= 16 * r["E"] else "128"] / us)
     assert len(behind) == 1428 and _mean(behind) >= 1 / 1.026 and min(behind) >= 1 / 1.42
     assert _mean(before) >= 1.08 and _slower(before) <= 27 and min(before) >= 1 / 1.23
+
+
+def _lines(key, pick, least):
+    """Every measured pair of forms: what the rule picks is not slower than the other form by more than `least`."""
+    for r in _rows(_table("decode_forms.json")[key]):
+        a, b = list(r)[-2:]
+        first = r[a] if pick(r) else r[b]
+        assert first <= least * min(r[a], r[b]) or first - min(r[a], r[b]) <= 0.25, (key, r)   # (launches of 5 us scatter by a quarter)
+
+
+def test_rows_of_decays_in_one_launch():
+    from chronos.ops import hybrid as hops
+
+    _lines("rows", lambda r: not hops.rows_step_pays(r["B"], r["H"], r["D"], r["Dv"], r["R"]), 1.18)
