@@ -270,7 +270,8 @@ __global__ void __launch_bounds__(256) moe_select_kernel(const float* __restrict
 // Projection and choice of one token by one workgroup: 16 waves share the N rows of w (N <= 64), the first wave chooses.  For up to 256 tokens, which
 // as a projection and a choice were two launches and two chains of latencies.  What bounds it is latency: a wave has up to 16 loads of 16
 // bytes a lane on their way.  us, two launches -> this: 1 token of 1024 by 10 rows 6.0 -> 5.2, 64 of 2048 by 18 11.4 -> 7.5, of 4096 by 34 12.6 -> 9.8, 256 of
-// 4096 by 64 13.9 -> 12.2; 300 tokens, more than there are CUs, 8.0 -> 9.5, 11.5 -> 13.5 and 14.9 -> 21.8.
+// 4096 by 64 13.9 -> 12.2; 300 tokens, more than there are CUs, 8.0 -> 9.5, 11.5 -> 13.5 and 14.9 -> 21.8.  Up to 2^18 weights, which every token's workgroup reads: 7168 by 34 (238 K) 12.8 -> 12.1 at 64
+// tokens, by 48 (336 K) 13.0 -> 13.6, by 64 (448 K) 12.8 -> 14.9; one token 14.8 -> 14.3, 200 18.6 -> 15.7.
 constexpr int kRouteN = 64, kRouteWaves = 16;
 template <int FORM>
 __global__ void __launch_bounds__(64 * kRouteWaves) moe_route_token_kernel(const uint16_t* __restrict__ h, const uint16_t* __restrict__ w,
@@ -389,12 +390,16 @@ __global__ void __launch_bounds__(256) moe_glu_token_kernel(const T* __restrict_
 
 void launch_hy_rowdot(const void*, const void*, const float*, float*, int, int, int, bool, hipStream_t);
 
+bool hy_moe_route_one(int T, int N, int d) {
+    const int64_t nd = (int64_t)N * d;
+    return T <= 256 && N <= hy::kRouteN && d % 8 == 0 && (nd <= 1 << 18 || (nd <= 1 << 19 && (T == 1 || T > 160)));
+}
 // z: float [T, N] scratch for the router logits (the few-row float32-output projection, then the selection); not touched where one launch does both
 template <int FORM>
 static void moe_route(const void* h, const void* w, const float* bias, float* z, int32_t* idx, float* wt, int T, int d, const hy::Choice& c, bool f32,
                       hipStream_t s) {
     if (T == 0) return;
-    if (!f32 && T <= 256 && c.N <= hy::kRouteN && d % 8 == 0 && hy::aligned16(h, w)) {
+    if (!f32 && hy_moe_route_one(T, c.N, d) && hy::aligned16(h, w)) {
         hy::moe_route_token_kernel<FORM><<<T, 64 * hy::kRouteWaves, 0, s>>>((const uint16_t*)h, (const uint16_t*)w, bias, idx, wt, d, c);
         return;
     }

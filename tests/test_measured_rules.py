@@ -167,3 +167,12 @@ def test_rows_of_decays_in_one_launch():
     from chronos.ops import hybrid as hops
 
     _lines("rows", lambda r: not hops.rows_step_pays(r["B"], r["H"], r["D"], r["Dv"], r["R"]), 1.18)
+
+
+def test_router_in_one_launch():
+    import torch
+
+    from chronos.ops import hybrid as hops
+
+    hops.load()
+    _lines("router", lambda r: not torch.ops.chronos.hy_moe_route_one(r["T"], r["N"], r["d"]), 1.04)
