@@ -51,6 +51,7 @@ bool launch_hy_latent_attention(const void*, const void*, const int32_t*, int, c
                                 float*, int64_t, const float*, hipStream_t);
 bool hy_latent_use_mfma(bool, int, int);
 int hy_latent_nsplit(int, int, bool);
+int hy_head_few_rows(int, int, int, int);
 bool hy_moe_route_one(int, int, int);
 void launch_hy_moe_route(const void*, const void*, const float*, float*, int32_t*, float*, int, int, int, int, bool,
                          hipStream_t);
@@ -1257,6 +1258,7 @@ Tensor hy_unrotate_gate(const Tensor& o, const Tensor& pos, const c10::optional<
 TORCH_LIBRARY_FRAGMENT(chronos, m) {
     m.def("hy_embed(Tensor ids, Tensor table, float scale=1.0) -> Tensor");
     // which form a launch of these sizes takes, without one
+    m.def("hy_head_few_rows(int T, int N, int H, int K) -> int", [](int64_t T, int64_t N, int64_t H, int64_t K) { return (int64_t)chronos::hy_head_few_rows((int)T, (int)N, (int)H, (int)K); });
     m.def("hy_moe_route_one(int T, int N, int d) -> bool", [](int64_t T, int64_t N, int64_t d) { return chronos::hy_moe_route_one((int)T, (int)N, (int)d); });
     m.def("hy_moe_tile(int items, int E, int d, int F, int up) -> int", [](int64_t items, int64_t E, int64_t d, int64_t F, int64_t up) {
         need(items >= 0 && E >= 1 && d >= 1 && F >= 1 && up >= 1 && std::max({items, E, d, F, up}) < (1LL << 31), "moe_tile: sizes");

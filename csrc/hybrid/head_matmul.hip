@@ -112,7 +112,9 @@ __global__ void __launch_bounds__(256) head_matmul_mfma_kernel(
 // The same for few tokens: a workgroup of 8 waves takes 16 MT tokens and 16 NTL output columns of one head; the waves share K, 32 at a time, straight
 // from memory into operands, and meet in LDS.  Bound by one memory latency; above, K steps of 64 follow each other.  us, above and this, 32 heads: 128 columns of
 // K = 512, 6 tokens 6.4 and 3.5, 64 tokens 6.7 and 4.5, 128 6.9 and 6.9; 512 columns of K = 128, 6 tokens 3.5 and 3.1, 32 tokens 3.6 and 3.7, 64 4.0 and
-// 5.3: up to 16 tokens, and 64 where K is 256 and more.
+// 5.3: up to 16 tokens, and 64 where K is 256 and more.  And while its workgroups, of half the columns and twice the waves, are few: with more of them than the
+// chip takes at once nothing is waited for any more: 128 heads, 48 tokens, 128 columns of K = 512 (1024 workgroups) 10.1 and 13.3, 256 of 256 (2048) 6.8 and 13.3; 64 heads, 48
+// tokens, 64 of 512 (512) 7.7 and 7.8; up to 16 tokens 1024 columns of K = 128, 32 heads (1024) 5.0 and 5.0, 64 heads (2048) 6.0 and 6.8.
 template <int MT, int NTL>
 __global__ void __launch_bounds__(512) head_matmul_few_kernel(
         const uint16_t* __restrict__ a, int64_t lda, int64_t ha, const uint16_t* __restrict__ w,
@@ -224,6 +226,12 @@ __global__ void __launch_bounds__(256) head_matmul_kernel(const T* __restrict__ 
 
 // a: row t, head h at a + t lda + h ha (K columns); out likewise with ldo / ho (N columns); w [H, N, K] contiguous; gsrc
 // (first gate column of row 0, row stride ldg) or nullptr.
+// tokens of a workgroup of head_matmul_few_kernel, or 0: the tiles above it
+int hy_head_few_rows(int T, int N, int H, int K) {
+    const int64_t cols = (int64_t)((N + 31) / 32) * H;
+    if (T <= 16) return cols <= 1024 ? 16 : 0;
+    return T <= 64 && K >= 256 && (T + 31) / 32 * cols <= 512 ? 32 : 0;
+}
 void launch_hy_head_matmul(const void* a, int64_t lda, int64_t ha, const void* w, void* out, int64_t ldo, int64_t ho,
                            const void* gsrc, int64_t ldg, int T, int H, int N, int K, bool f32, hipStream_t s) {
     if (T == 0 || H == 0 || N == 0) return;
@@ -232,8 +240,9 @@ void launch_hy_head_matmul(const void* a, int64_t lda, int64_t ha, const void* w
         const bool vst = ldo % 4 == 0 && ho % 4 == 0 && al(out, 8) && (gsrc == nullptr || (ldg % 4 == 0 && N % 4 == 0 && al(gsrc, 8)));
 #define HY_HM(MT, NTL) hy::head_matmul_mfma_kernel<MT, NTL><<<dim3((T + 64 * MT - 1) / (64 * MT), (N + 16 * NTL - 1) / (16 * NTL), H), 256, 0, s>>>((const uint16_t*)a, lda, ha, (const uint16_t*)w, (uint16_t*)out, ldo, ho, (const uint16_t*)gsrc, ldg, T, N, K, vst)
 #define HY_HF(MT, NTL) hy::head_matmul_few_kernel<MT, NTL><<<dim3((T + 16 * MT - 1) / (16 * MT), (N + 16 * NTL - 1) / (16 * NTL), H), 512, 0, s>>>((const uint16_t*)a, lda, ha, (const uint16_t*)w, (uint16_t*)out, ldo, ho, (const uint16_t*)gsrc, ldg, T, N, K, vst)
-        if (T <= 16) HY_HF(1, 2);
-        else if (T <= 64 && K >= 256) HY_HF(2, 2);
+        const int rows = hy_head_few_rows(T, N, H, K);
+        if (rows == 16) HY_HF(1, 2);
+        else if (rows == 32) HY_HF(2, 2);
         else if (T <= 256) HY_HM(1, 4);
         else if (N <= 64) HY_HM(2, 4);
         else HY_HM(2, 8);

@@ -176,3 +176,12 @@ def test_router_in_one_launch():
 
     hops.load()
     _lines("router", lambda r: not torch.ops.chronos.hy_moe_route_one(r["T"], r["N"], r["d"]), 1.04)
+
+
+def test_products_per_head():
+    import torch
+
+    from chronos.ops import hybrid as hops
+
+    hops.load()
+    _lines("head", lambda r: torch.ops.chronos.hy_head_few_rows(r["T"], r["N"], r["H"], r["K"]) == 0, 1.06)
