@@ -50,7 +50,7 @@ bool launch_hy_latent_attention(const void*, const void*, const int32_t*, int, c
                                 const float*, void*, int, int, int, int, int, int, float, int, bool, bool, int, float*,
                                 float*, int64_t, const float*, hipStream_t);
 bool hy_latent_use_mfma(bool, int, int);
-int hy_latent_nsplit(int, int, bool);
+int hy_latent_nsplit(int, int, bool, int);
 int hy_head_few_rows(int, int, int, int);
 bool hy_moe_route_one(int, int, int);
 void launch_hy_moe_route(const void*, const void*, const float*, float*, int32_t*, float*, int, int, int, int, bool,
@@ -441,7 +441,7 @@ Tensor hy_latent_attention(const Tensor& qa, const Tensor& cache, const Tensor& 
     if (chronos::hy_latent_use_mfma(f32(qa), (int)DK, (int)rank)) {
         int64_t span = block_table.size(1) * cache.size(1);   // keys a row block walks at most
         if (window > 0) span = std::min<int64_t>(span, window + mq);
-        nsplit = chronos::hy_latent_nsplit((int)(B * ((mq * H + 63) / 64)), (int)span, window > 0);
+        nsplit = chronos::hy_latent_nsplit((int)(B * ((mq * H + 63) / 64)), (int)span, window > 0, (int)rank);
         if (nsplit > 1) {
             part_o = at::empty({T * H * nsplit, rank}, qa.options().dtype(at::kFloat));
             part_ml = at::empty({T * H * nsplit, 2}, qa.options().dtype(at::kFloat));
@@ -1260,6 +1260,7 @@ TORCH_LIBRARY_FRAGMENT(chronos, m) {
     // which form a launch of these sizes takes, without one
     m.def("hy_head_few_rows(int T, int N, int H, int K) -> int", [](int64_t T, int64_t N, int64_t H, int64_t K) { return (int64_t)chronos::hy_head_few_rows((int)T, (int)N, (int)H, (int)K); });
     m.def("hy_moe_route_one(int T, int N, int d) -> bool", [](int64_t T, int64_t N, int64_t d) { return chronos::hy_moe_route_one((int)T, (int)N, (int)d); });
+    m.def("hy_latent_nsplit(int wgs, int max_ctx, bool windowed, int rank) -> int", [](int64_t w, int64_t c, bool win, int64_t r) { return (int64_t)chronos::hy_latent_nsplit((int)w, (int)c, win, (int)r); });
     m.def("hy_moe_tile(int items, int E, int d, int F, int up) -> int", [](int64_t items, int64_t E, int64_t d, int64_t F, int64_t up) {
         need(items >= 0 && E >= 1 && d >= 1 && F >= 1 && up >= 1 && std::max({items, E, d, F, up}) < (1LL << 31), "moe_tile: sizes");
         return (int64_t)chronos::hy_moe_tile((int)items, (int)E, (int)d, (int)F, (int)up);

@@ -385,10 +385,12 @@ bool hy_latent_mfma_ok(int DK, int rank) { return !(DK % 8 || rank % 16 || DK > 
 // walk), at most 16.  A tile of a few rows is a chain of latencies, dearer than its partials: at least 4 tiles, 2 tiles and one, us with the combining,
 // 1 sequence of 700 keys, 8 heads of 288 columns 15.1, 12.1, 11.1, 32 heads of 576 30.8, 21.0, 17.8; 6 of about 200 12.2, 12.2, 11.0, 23.5, 20.5,
 // 17.7; 16 of about 700 15.3, 12.5, 11.2.  Not two splits: 1 of 120 keys 8.2, 9.4.  32 splits: 6 of about 2000, 32 heads 24.1 -> 26.2.
-int hy_latent_nsplit(int wgs, int max_ctx, bool windowed) {
+// Three only where the rank is large and workgroups few: 200 keys, us, whole and in three: 16 heads of rank 128, 1 and 64 sequences 9.1, 9.8 and 9.4, 11.1; 8 of rank 256
+// 11.7, 11.6 and 12.3, 12.9; 32 of rank 512 21.3, 18.6 and 22.1, 24.8 (16 sequences 21.6, 20.0; 32 level).
+int hy_latent_nsplit(int wgs, int max_ctx, bool windowed, int rank) {
     if (wgs >= 128) return 1;
     int want = (256 + wgs - 1) / wgs, cap = max_ctx / ((windowed ? 2 : 1) * hy::MKT);
-    if (!windowed && cap < 3) cap = 1;
+    if (!windowed && cap < (rank > 256 && wgs <= 32 ? 3 : 4)) cap = 1;
     if (want > hy::kLatentSplits) want = hy::kLatentSplits;
     if (want > cap) want = cap;
     return want < 1 ? 1 : want;

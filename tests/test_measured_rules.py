@@ -185,3 +185,12 @@ def test_products_per_head():
 
     hops.load()
     _lines("head", lambda r: torch.ops.chronos.hy_head_few_rows(r["T"], r["N"], r["H"], r["K"]) == 0, 1.06)
+
+
+def test_splits_of_latent_attention():
+    import torch
+
+    from chronos.ops import hybrid as hops
+
+    hops.load()
+    _lines("latent", lambda r: torch.ops.chronos.hy_latent_nsplit(r["B"] * -(-r["H"] // 64), 200, False, r["rank"]) == 1, 1.05)
