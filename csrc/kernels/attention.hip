@@ -604,41 +604,36 @@ __global__ void __launch_bounds__(256, 1) split_decode_kernel(
     // the wave's steps: t0 = ks + 32 w + 128 i; NB of them in flight (ring slot i % NB)
     const int t_first = ks + 32 * w;
     const int nsteps = t_first < ke ? (ke - t_first + 127) / 128 : 0;
-    auto walk = [&](auto OC, int a0, int b0) {
-        if (NB > 1 && nsteps > 0) stage(OC, a0, b0, 0);
-#pragma unroll
-        for (int i = 1; i < NB - 1; ++i)
-            if (i < nsteps) {
-                const int a = page_a(t_first + 128 * i);
-                stage(OC, a, page_b(t_first + 128 * i, a), i);
-            }
-        for (int i = 0; i < nsteps; ++i) {
-            const int ahead = i + NB - 1;
-            const bool more = ahead < nsteps;  // wave-uniform
-            if (more) {
-                const int a = page_a(t_first + 128 * ahead);
-                stage(OC, a, page_b(t_first + 128 * ahead, a), ahead % NB);
-            }
-            // step i landed: the pieces issued after it (up to NB - 1 steps) may stay in flight
-            const int newer = min(nsteps - 1 - i, NB - 1);
-            if (newer >= 2) sd_vmcnt<2 * NP>();
-            else if (newer == 1) sd_vmcnt<NP>();
-            else sd_vmcnt<0>();
-            compute(t_first + 128 * i, i % NB);
-        }
-    };
     // one look at the middle of the range (rows share the front of their histories; a look at every step costs 4 to 10 %), on its way with the
     // first step's pages
-    int a0 = 0, b0 = 0;
     bool own = true;
     if (nsteps > 0) {
-        a0 = page_a(t_first);
-        b0 = page_b(t_first, a0);
-        const int pm = (ks + ke) / 2 / block_size;
+        const int a0 = page_a(t_first), b0 = page_b(t_first, a0), pm = (ks + ke) / 2 / block_size;
         own = bn == nullptr || bt[pm] != bn[pm];
+        if (NB > 1) {
+            if (own) stage(std::true_type{}, a0, b0, 0);
+            else stage(std::false_type{}, a0, b0, 0);
+        }
     }
-    if (own) walk(std::true_type{}, a0, b0);
-    else walk(std::false_type{}, a0, b0);
+    auto next = [&](int t0, int j) {
+        const int a = page_a(t0), b = page_b(t0, a);
+        if (own) stage(std::true_type{}, a, b, j);
+        else stage(std::false_type{}, a, b, j);
+    };
+#pragma unroll
+    for (int i = 1; i < NB - 1; ++i)
+        if (i < nsteps) next(t_first + 128 * i, i);
+    for (int i = 0; i < nsteps; ++i) {
+        const int ahead = i + NB - 1;
+        const bool more = ahead < nsteps;  // wave-uniform
+        if (more) next(t_first + 128 * ahead, ahead % NB);
+        // step i landed: the pieces issued after it (up to NB - 1 steps) may stay in flight
+        const int newer = min(nsteps - 1 - i, NB - 1);
+        if (newer >= 2) sd_vmcnt<2 * NP>();
+        else if (newer == 1) sd_vmcnt<NP>();
+        else sd_vmcnt<0>();
+        compute(t_first + 128 * i, i % NB);
+    }
     sd_vmcnt<0>();
     __syncthreads();  // the ring is reused as the merge buffer below
 
