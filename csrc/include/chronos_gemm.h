@@ -24,6 +24,7 @@ struct PPArgs {
     int n0, nf;
     const float* xsc;  // gemm_lg F8 (W8A8 e4m3fn bytes in x / w): per-token scales [M]
     const float* wsc;  // ... and per-output-channel scales [N]
+    int turn;          // gemm_lg, ring tiles, one x tile: workgroups start their K at different stages (sums in another order)
     int ablate;  // timing-only diagnostics (knob pp_ablate): 1 skip loop DMA, 2 skip LDS reads, 4 skip MFMA, 8 nt weights, 16/32 alias every W/x tile onto tile 0
 };
 

@@ -621,6 +621,9 @@ std::tuple<Tensor, Tensor> gemm_pp(const Tensor& x, const Tensor& w, int64_t mod
     a.ablate = chronos::gemm_lg_ablations_built() ? chronos::knob("pp_ablate", 0) : 0;
     a.gm = chronos::knob("pp_gm", 8);  // +7-9 % at M = 16384 (profiles/r3_gemm_tile_order_m16384.jsonl)
     a.handoff = chronos::knob("lg_handoff", -1);
+    // up to 8 rows a layer's sums keep their order: steps of so few rows are the ones over long fp8 caches, whose bytes would follow a last bit of
+    // the stream; the vocabulary's logits are cached nowhere
+    a.turn = M > 8 || N > 65536;
     Tensor y = at::empty({M, mode == 1 ? N / 2 : N}, x.options());
     a.y = bfm(y);
     Tensor part_out;
@@ -755,6 +758,7 @@ Tensor gemm_slices(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk
     a.splitk = (int)splitk;
     a.kts = (int)(K / 64 / splitk);
     a.gm = chronos::knob("pp_gm", 8);
+    a.turn = 1;
     Tensor ws = at::empty({splitk, M, N}, x.options().dtype(at::kFloat));
     a.ws = ws.data_ptr<float>();
     CHK(skinny ? chronos::launch_gemm_skinny((int)cfg, 0, false, a, cur_stream()) : chronos::launch_gemm_lg((int)cfg, 0, false, a, cur_stream()),

@@ -223,9 +223,22 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
     // interleaved with (and every stage leaves the same vmcnt count): a stage past the end re-reads the last stage's
     // source into a buffer no later stage reads
     const int NS1 = NS - 1;
+    // TURN: every workgroup takes its stages round from one of its own, an XCD's neighbours one stage apart and the XCDs eight.  All from
+    // the first, they read the same columns of rows that lie a power of two apart, lines that share few of the memory's and the
+    // L2s' channels.  One x tile, weights cold, us, from the first stage / turned: 28672 x 4096, 64 rows 49.4 / 40.2 (128-row tiles) and 53.1 / 50.0, 16
+    // rows 41.3 / 37.8, 128 rows 55.6 / 49.1, 256 rows 72.6 / 66.3; 32768 x 4096, 64 rows 60.6 / 44.2, 32 rows 48.3 / 42.1; 14336 x 4096, 64 rows 29.0 /
+    // 26.7; 128256 x 4096, 64 rows 191 / 177, 32 rows 186 / 184; 6144 x 4096 in two slices, 32 rows 13.1 / 12.0; level at 4096 x 14336 in four slices.
+    // From K = 4096 on: level at 2048 (64 rows of 8192: 13.8 / 13.9), at 1024 slower (a decode step of one row, its weights in the memory-side cache: 156 / 161).  With more x tiles neighbours share their W rows and lose them from the L2 (1024 rows of 6144 x 4096: 52.1 / 54.1).
+    constexpr bool TURN = !SLAB && !F8 && (ONCE || XM > 128);
+    const int turn0 = TURN && a.turn ? ((int)(blockIdx.x >> 3) + 8 * (int)(blockIdx.x & 7)) % NS : 0;
     auto issue = [&](int j) {
         unsigned char* st = smem + (j % ST) * STAGE;
-        const int kb = min(j, NS1) * RB;  // byte offset of stage j in the row
+        int stage = min(j, NS1);
+        if constexpr (TURN) {
+            stage += turn0;
+            stage -= stage >= NS ? NS : 0;
+        }
+        const int kb = stage * RB;  // byte offset of the stage in the row
 #pragma unroll
         for (int i = 0; i < NPER; ++i) {
             if constexpr (ONCE) {
@@ -1213,12 +1226,14 @@ void lg_launch(const PPArgs& a, hipStream_t st) {
     const int lds = ST * (WN + XM) * RB + 16 + XM * 4 + (F8 && ST == 2 ? (WN + XM) * 4 : 0);
     const int mt = (a.M + XM - 1) / XM;
     const int ntl = MODE == kSwiglu ? a.F / (WN / 2) : (a.N + WN - 1) / WN;
+    PPArgs b = a;
+    b.turn = a.turn && mt == 1 && a.K >= 4096;
     auto go = [&](auto kern, bool& attr) {
         if (!attr) {
             hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
             attr = true;
         }
-        hipLaunchKernelGGL(kern, dim3(mt * ntl * a.splitk), dim3(128 * NWX), lds, st, a);
+        hipLaunchKernelGGL(kern, dim3(mt * ntl * a.splitk), dim3(128 * NWX), lds, st, b);
     };
     if constexpr (XM <= 128 && ST > 2 && !F8 && ABL == 0 && WN / (1024 / RB) % (2 * NWX) == 0 && XM / (1024 / RB) % (2 * NWX) == 0) {
         if (mt == 1) {
