@@ -42,3 +42,26 @@ def test_sums_of_up_to_eight_rows_keep_their_order(cfg, rows):
     for m in rows:
         y, _ = torch.ops.chronos.gemm_pp(x[:m].contiguous(), w, 0, cfg, 1, None, None, 1e-5, False)
         assert torch.equal(y, all_rows[:m])
+
+
+# k-steps of the two products: 2 and 256 (fewer and more than the ring holds), 30 and 32; tiles of 32, 64 and 128 rows
+@pytest.mark.parametrize("d,F", [(128, 16384), (1920, 2048)])
+@pytest.mark.parametrize("T", [5, 60, 300, 900])
+def test_turned_experts(d, F, T):
+    """moe_grouped.hip's tiles over experts' weights of 256 MB and more, against the PyTorch reference (tolerance of the other expert tests), and a
+    token's result whatever else is in the batch."""
+    from chronos.ops import hybrid as hops, hybrid_ref as ref
+
+    E, top, bf = 80, 8, torch.bfloat16
+    assert E * F * d * 2 >= 1 << 28
+    g = torch.Generator(device=DEV).manual_seed(T + d)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
+    h, wt = rnd(T + 11, d).to(bf), torch.rand(T + 11, top, device=DEV, generator=g)
+    idx = torch.rand(T + 11, E, device=DEV, generator=g).topk(top, -1).indices.int()
+    idx[:10] = torch.arange(E, device=DEV).view(10, top)      # (every expert has an item, so both batches below take the same tiles)
+    wu, wd = (rnd(E, F, d) * d ** -0.5).to(bf), (rnd(E, d, F) * F ** -0.5).to(bf)
+    more = hops.moe_ffn(h, idx, wt, wu, wd, 1, bf)
+    want = ref.moe_ffn(h, idx, wt, wu, wd, 1, bf).float()
+    assert (more.float() - want).abs().max() <= 1.5e-2 * want.abs().max()
+    n = max(T, 10)
+    assert torch.equal(hops.moe_ffn(h[:n].contiguous(), idx[:n].contiguous(), wt[:n].contiguous(), wu, wd, 1, bf), more[:n])
