@@ -29,10 +29,12 @@
 // 64 x 64 weights (ten 16 x 16 tiles on and below the diagonal) through LDS; the delta rule's tiles lie beside.
 //
 // What bounds it: the chain of a sequence's chunks, one wave per SIMD: vector instructions (the cutting into terms, the
-// exponentials) and 114 matrix instructions (delta: 162) per chunk and wave at D = 128, and two barriers, 5 us a chunk (delta: 10).
+// exponentials) and 114 matrix instructions (delta: 162) per chunk and wave at D = 128, and two barriers, 5 us a chunk (delta: 10, 4.8 with
+// its tiles made ahead).
 // Measured, 4 sequences of 2048 tokens, token by token -> this: retention, 8 heads of 128 x 128: 797 -> 177 us, in four
 // segments 73; 32 heads: 857 -> 182; state-space form, 128 heads of 128 x 64: 1058 -> 442; mlstm, 4 heads of 128 x 256: 1987
-// -> 220, in four segments 95, 4 heads of 256 x 512: 3050 -> 299, in two 213; delta rule, 32 heads of 128 x 128: 959 -> 352.
+// -> 220, in four segments 95, 4 heads of 256 x 512: 3050 -> 299, in two 213; delta rule, 32 heads of 128 x 128: 959 -> 352,
+// with the tiles ahead 270.
 // One and two waves per workgroup: 436 and 302 us where four took 233 (of 171, before addresses, weights and stores lost
 // their branches).
 #include "chunk_common.h"
@@ -92,27 +94,215 @@ struct ChunkScan {
     const int32_t *q_start, *pos0, *slots;
     const float* n0;   // [B, H, D]: the normaliser before the step (workgroups of one (sequence, head) start at any time)
     float *S, *n, *o;
-    int B, HK, H, Dv;
+    int B, HK, H, Dv, T;
     // more than one segment per sequence: states before it [B, H, D, Dv], then of each segment but the last; mlstm: normalisers and all:
     // products of decays of each segment but the last, [segs - 1, B, H, ..]
     int segs;
     float *seg_s, *seg_n, *seg_d;
+    unsigned char* tiles;   // delta: [slots, H, kDeltaTiles] of delta_tiles_kernel, or nullptr
 };
+
+// What the delta rule's chunks need of their q, k and decays alone, per chunk and head, written by delta_tiles_kernel (bytes): tiles as three terms, 512
+// bytes a term: the weights [10], the solve's below the diagonal [6], the inverses of its diagonal ones less the identity [4] | floats: beta,
+// beta k-scale e^L, c, e^L, r [64] each, e^L_C
+constexpr int kDtTile = 1536, kDtA = 10 * kDtTile, kDtT = 16 * kDtTile, kDtSc = 20 * kDtTile, kDtEnd = kDtSc + 5 * kCH * 4, kDeltaTiles = 32 * 1024;
+static_assert(kDtEnd + 4 <= kDeltaTiles, "tiles of a chunk");
+// Chunk c of sequence b, tokens from s0 on, is chunk s0 / 64 + b + c of the launch: no two alike, T / 64 + B + 1 of them at most.
+__host__ __device__ constexpr int64_t delta_slots(int T, int B) { return (int64_t)T / kCH + B + 1; }
+__device__ __forceinline__ Terms4 load_terms(const unsigned char* tile, int lane) {
+    const bf16x4* const at = reinterpret_cast<const bf16x4*>(tile) + lane;
+    return {at[0], at[64], at[128]};
+}
 
 // LDS (bytes): two buffers of q | k | v | weight tiles [10][64 lanes] x 16 (delta: and the solve's tiles [10], the inverses of
 // the diagonal ones [4]) | every wave's own copy of the scalars (L in float64, w, c; delta: beta, beta k-scale, and that times
-// e^L) | mlstm: the weight tiles' sums over s [10][16] and the waves' parts of n . q [NW][64]
-template <int D, int MODE> struct ChunkLds {
-    static constexpr int Q = kCH * D * 2, V = kCH * kCW * 32, BUF = 2 * Q + V;
-    static constexpr int PT = 2 * BUF, AT = PT + 10 * 1024, TT = AT + (MODE == kScanDelta ? 10 * 1024 : 0);
-    static constexpr int OWN = TT + (MODE == kScanDelta ? 4 * 1024 : 0), OWN_SIZE = kCH * (MODE == kScanDelta ? 28 : 16);
+// e^L) | mlstm: the weight tiles' sums over s [10][16] and the waves' parts of n . q [NW][64].  PRE: two buffers of q | k | v | delta_tiles_kernel's.
+template <int D, int MODE, bool PRE> struct ChunkLds {
+    static constexpr int Q = kCH * D * 2, V = kCH * kCW * 32, BUF = 2 * Q + V + (PRE ? kDeltaTiles : 0);
+    static constexpr int PT = 2 * BUF, AT = PT + (PRE ? 0 : 10 * 1024), TT = AT + (MODE == kScanDelta && !PRE ? 10 * 1024 : 0);
+    static constexpr int OWN = TT + (MODE == kScanDelta && !PRE ? 4 * 1024 : 0), OWN_SIZE = PRE ? 0 : kCH * (MODE == kScanDelta ? 28 : 16);
     static constexpr int SUM = OWN + kCW * OWN_SIZE, SIZE = SUM + (MODE == kScanMlstm ? 640 + kCW * 256 : 0);
 };
 
+// A chunk's scalars, lane t token t of nt: its sum of log decays, the factors on what it writes (w) and reads (rd), the sign gC of the product of the
+// chunk's decays, and their sum LC
+template <bool MLSTM>
+__device__ __forceinline__ double chunk_logs(bool valid, float sd, float sw, int lane, float& w, float& rd, float& gC, double& LC) {
+    double L = 0.0;
+    w = 0.f;
+    gC = 1.f;
+    if (valid) {
+        if constexpr (MLSTM) {
+            L = sd;
+            w = expf(sw);
+        } else {
+            const float lg = logf(fabsf(sd));
+            L = lg < -110.f ? -110.f : lg;   // e^-110 is 0 in float32, as a decay of 0 is
+            w = sw;
+        }
+    }
+    if constexpr (!MLSTM) {   // the sign of a product of decays up to t goes with what t writes and reads
+        const uint64_t neg = __ballot(valid && sd < 0.f);
+        if (__popcll(neg & (~0ull >> (63 - lane))) & 1) {
+            w = -w;
+            rd = -rd;
+        }
+        if (__popcll(neg) & 1) gC = -1.f;
+    }
+    L = lanes_running_sum(L);
+    LC = __builtin_bit_cast(double, (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(__builtin_bit_cast(uint64_t, L) >> 32), 63) << 32 |
+                                        (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)__builtin_bit_cast(uint64_t, L), 63));
+    return L;
+}
+
+// Rows 16 i + ln of a chunk's q or k, columns 32 kk + 8 g ..: either operand of a product over columns
+template <int D> __device__ __forceinline__ bf16x8 chunk_row8(const unsigned char* base, int i, int kk, int ln, int g) {
+    return *reinterpret_cast<const bf16x8*>(base + (16 * i + ln) * (D * 2) + (((kk * 4 + g) ^ spread<D / 8>(ln)) * 16));
+}
+// Weights: tile (i, j) holds rows s = 16 j.. (4 g + r) and columns t = 16 i.. (ln): k_s . tbase_t times e^(L_t - L_s) w_s, for s <= t
+template <int D>
+__device__ __forceinline__ f32x4 chunk_weights(const unsigned char* kb, const unsigned char* tbase, int i, int j, const double* Ls, const float* ws, int ln, int g) {
+    constexpr int KK = D / 32;
+    bf16x8 x[KK], y[KK];
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) { x[kk] = chunk_row8<D>(kb, j, kk, ln, g); y[kk] = chunk_row8<D>(tbase, i, kk, ln, g); }
+    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) acc[kk & 1] = mfma_16x16x32(x[kk], y[kk], acc[kk & 1]);
+    f32x4 v = acc[0];
+    if (KK > 1) v += acc[1];
+    const int t = 16 * i + ln;
+    const double Lt = Ls[t];
+    const f32x4 wsv = *reinterpret_cast<const f32x4*>(ws + 16 * j + 4 * g);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int s = 16 * j + 4 * g + r;
+        v[r] = s <= t ? v[r] * (wsv[r] * exp_d(Lt - Ls[s])) : 0.f;
+    }
+    return v;
+}
+// Delta: tile (i, j) of -A, A[t, s] = beta_t k-scale_t k-scale_s e^(L_t - L_s) (k_t . k_s) for s < t (bk: beta k-scale)
+template <int D>
+__device__ __forceinline__ f32x4 chunk_minus_a(const unsigned char* kb, int i, int j, const double* Ls, const float* ws, const float* bk, int ln, int g) {
+    const int t = 16 * i + ln;
+    f32x4 v = chunk_weights<D>(kb, kb, i, j, Ls, ws, ln, g);
+    const float f = -bk[t];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = 16 * j + 4 * g + r < t ? v[r] * f : 0.f;
+    return v;
+}
+// (I + A)^-1 - I of a diagonal tile whose -A is at `a`, by forward substitution, lane n column n, to `out` in operand layout: lane (t, g) holds
+// columns 4 g ..  A wave by itself.
+__device__ __forceinline__ void chunk_inverse(const f32x4* a, float* out, int ln, int g) {
+    __builtin_amdgcn_wave_barrier();   // the wave's own writes
+    float x[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        float acc[4] = {r == ln ? 1.f : 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < (r + 3) / 4; ++q) {
+            const f32x4 row = a[q * 16 + r];   // -A[r][4 q ..]
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (4 * q + e < r) acc[e] += row[e] * x[4 * q + e];
+        }
+        x[r] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    }
+    if (g == 0) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) out[((ln >> 2) * 16 + r) * 4 + (ln & 3)] = r == ln ? 0.f : x[r];
+    }
+}
+
+// The delta rule's tiles and scalars of every chunk and head, all chunks side by side: what the walk over a sequence's chunks had done between its steps, half
+// of a chunk's time there, and once for every 64 value columns.  Same arithmetic, same bits.  Both launches, us, heads of 128 x 128, before -> this: 8
+// heads, one sequence of 4000 tokens 670 -> 306 (14 of them this launch), 113 29 -> 23, 21 of about 100 52 -> 40; 32 heads, one of 1351 240 -> 124, 4 of 2048 383 -> 292
+// (74: 32 KB written per chunk and head, three workgroups per CU; the walk then reads 3.9 TB/s).  A workgroup per chunk and head; in small
+// launches bound by one chunk's latencies.
+template <int D>
+__global__ void __launch_bounds__(256) delta_tiles_kernel(const ChunkScan a) {
+    constexpr int CPR = D / 8, NW = 4, Q = kCH * D * 2;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char cs_smem[];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = lane & 15, g = lane >> 4;
+    const int hd = blockIdx.x % a.H, slot = blockIdx.x / a.H, hk = hd / (a.H / a.HK);
+    int upto = 0;   // sequences whose first chunk is this one or an earlier one
+    for (int j = 0; j < a.B; j += 64) {
+        const int q = j + lane;
+        upto += __popcll(__ballot(q < a.B && (a.q_start[min(q, a.B - 1)] >> 6) + q <= slot));
+    }
+    if (upto == 0) return;
+    const int b = upto - 1, s0 = a.q_start[b], t1 = a.q_start[b + 1], tb = s0 + (slot - (s0 >> 6) - b) * kCH;
+    if (tb >= t1) return;
+    const int nt = min(kCH, t1 - tb), last = nt - 1, nrow = (nt + 15) / 16;
+    unsigned char* const qb = cs_smem;
+    unsigned char* const kb = cs_smem + Q;
+    f32x4* const diag = reinterpret_cast<f32x4*>(cs_smem + 2 * Q) + wv * 64;
+    float* const inv = reinterpret_cast<float*>(cs_smem + 2 * Q + 4096) + wv * 256;
+    double* const Ls = reinterpret_cast<double*>(cs_smem + 2 * Q + 8192 + wv * 1024);
+    float *const ws = reinterpret_cast<float*>(Ls + kCH), *const bk = ws + kCH;
+    const uint32_t lds0 = lds_offset(cs_smem);
+    const uint16_t* const q = a.proj + a.q_off + (int64_t)hk * D + (int64_t)tb * a.ldp;
+    const uint16_t* const k = a.proj + a.k_off + (int64_t)hk * D + (int64_t)tb * a.ldp;
+#pragma unroll
+    for (int u = 0; u < (CPR + NW - 1) / NW; ++u) {
+        const int j = wv + NW * u, i = j * 64 + lane, row = i / CPR, c = (i % CPR) ^ spread<CPR>(row);
+        if (CPR % NW == 0 || j < CPR) {
+            const int64_t at = (int64_t)min(row, last) * a.ldp + c * 8;
+            dma_1k(q + at, __builtin_amdgcn_readfirstlane(lds0 + j * 1024));
+            dma_1k(k + at, __builtin_amdgcn_readfirstlane(lds0 + Q + j * 1024));
+        }
+    }
+    const int64_t t = min(tb + lane, t1 - 1);
+    const bool valid = lane < nt;
+    const float sd = a.dts != 0 ? a.decay[t * a.dts + hd] : a.decay[hd];
+    float rd = a.qscale != nullptr ? a.qscale[t * a.HK + hk] : a.q_mul, w, gC;
+    const float sb = a.beta[t * a.H + hd];
+    double LC;
+    const double L = chunk_logs<false>(valid, sd, a.kscale != nullptr ? a.kscale[t * a.HK + hk] : 1.f, lane, w, rd, gC, LC);
+    const float eL = exp_d(L), bt = valid ? sb : 0.f;
+    Ls[lane] = L;
+    ws[lane] = w;
+    bk[lane] = bt * w;
+    unsigned char* const out = a.tiles + ((int64_t)slot * a.H + hd) * kDeltaTiles;
+    if (wv == 0) {
+        float* const sc = reinterpret_cast<float*>(out + kDtSc);
+        sc[lane] = bt;
+        sc[kCH + lane] = bt * w * eL;
+        sc[2 * kCH + lane] = gC * exp_d(LC - L) * w;
+        sc[3 * kCH + lane] = eL;
+        sc[4 * kCH + lane] = rd;
+        if (lane == 0) sc[5 * kCH] = gC * exp_d(LC);
+    }
+    auto put = [&](int at, const Terms4& v) {
+        bf16x4* const to = reinterpret_cast<bf16x4*>(out + at) + lane;
+        to[0] = v.h;
+        to[64] = v.m;
+        to[128] = v.l;
+    };
+    dma_wait();
+    __syncthreads();
+    for (int p = wv; p < 10; p += NW) {
+        const int i = p < 1 ? 0 : p < 3 ? 1 : p < 6 ? 2 : 3, j = p - i * (i + 1) / 2;
+        if (i < nrow) put(p * kDtTile, split3(chunk_weights<D>(kb, qb, i, j, Ls, ws, ln, g)));
+    }
+    for (int p = NW - 1 - wv; p < 6; p += NW) {   // (the last waves had a tile less)
+        const int i = p < 1 ? 1 : p < 3 ? 2 : 3, j = p - i * (i - 1) / 2;
+        if (i < nrow) put(kDtA + p * kDtTile, split3(chunk_minus_a<D>(kb, i, j, Ls, ws, bk, ln, g)));
+    }
+    if (wv < nrow) {
+        diag[lane] = chunk_minus_a<D>(kb, wv, wv, Ls, ws, bk, ln, g);
+        chunk_inverse(diag, inv, ln, g);
+        __builtin_amdgcn_wave_barrier();
+        put(kDtT + wv * kDtTile, split3(reinterpret_cast<const f32x4*>(inv)[lane]));
+    }
+}
+
 // STATE: the first pass over segments, which only carries the state on (each from 0, the first from the sequence's state)
-template <int D, int MODE, bool STATE>
+// PRE (delta): the tiles and scalars of the chunks come from delta_tiles_kernel
+template <int D, int MODE, bool STATE, bool PRE = false>
 __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) chunk_scan_kernel(const ChunkScan a) {
-    using M = ChunkLds<D, MODE>;
+    using M = ChunkLds<D, MODE, PRE>;
+    static_assert(!PRE || (MODE == kScanDelta && !STATE), "tiles ahead: the delta rule");
     constexpr bool DELTA = MODE == kScanDelta, MLSTM = MODE == kScanMlstm;
     constexpr int NW = kCW, CPR = D / 8, VC = 2 * NW, KK = D / 32;   // 16-byte pieces per row of q and k, of v; 32-row steps of the state
     extern __shared__ __attribute__((aligned(1024))) unsigned char cs_smem[];
@@ -222,6 +412,12 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
             const int j = wv + NW * u, i = j * 64 + lane, row = i / VC, c = (i % VC) ^ spread<VC>(row);
             dma_1k(v + (int64_t)min(row, last) * a.ldp + min(c, vn - 1) * 8, __builtin_amdgcn_readfirstlane(dst + 2 * M::Q + j * 1024));
         }
+        if constexpr (PRE) {
+            const unsigned char* const from = a.tiles + ((int64_t)((s0 >> 6) + b + (tb - s0) / kCH) * a.H + hd) * kDeltaTiles + lane * 16;
+#pragma unroll
+            for (int u = 0; u < kDeltaTiles / 1024 / NW; ++u)
+                dma_1k(from + (wv + NW * u) * 1024, __builtin_amdgcn_readfirstlane(dst + 2 * M::Q + M::V + (wv + NW * u) * 1024));
+        }
     };
     // the scalars of token tb + lane, as loaded; past the range: nothing decays, nothing is written
     float sd = 1.f, sw = 0.f, sr = 0.f, sb = 0.f;
@@ -244,42 +440,24 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
     const uint32_t orow = (uint32_t)a.H * a.Dv * 4, ocol = live ? (uint32_t)col * 4 : 0x80000000u;
     if (t0 < te) {
         fetch(t0, 0);
-        scalars(t0);
+        if constexpr (!PRE) scalars(t0);
     }
     for (int tb = t0, buf = 0; tb < te; tb += kCH, buf ^= 1) {
         const int nt = min(kCH, te - tb);
-        dma_wait();
+        // (PRE: the chunk before, a whole one, issued 16 stores after this one's pieces; they need not be done)
+        if (PRE && tb != t0) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+        else dma_wait();
         // ---- the chunk's scalars (before the next chunk's DMA is issued: what waits for them would wait for that, too)
         const bool valid = lane < nt;
-        double L = 0.0;
-        float w = 0.f;
-        float rd = sr, gC = 1.f;   // gC: the sign of the product of the chunk's decays
-        if (valid) {
-            if constexpr (MLSTM) {
-                L = sd;
-                w = expf(sw);
-            } else {
-                const float lg = logf(fabsf(sd));
-                L = lg < -110.f ? -110.f : lg;   // e^-110 is 0 in float32, as a decay of 0 is
-                w = sw;
-            }
-        }
-        if constexpr (!MLSTM) {   // the sign of a product of decays up to t goes with what t writes and reads
-            const uint64_t neg = __ballot(valid && sd < 0.f);
-            if (__popcll(neg & (~0ull >> (63 - lane))) & 1) {
-                w = -w;
-                rd = -rd;
-            }
-            if (__popcll(neg) & 1) gC = -1.f;
-        }
-        L = lanes_running_sum(L);
-        const double LC = __builtin_bit_cast(double, (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(__builtin_bit_cast(uint64_t, L) >> 32), 63) << 32 |
-                                                         (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)__builtin_bit_cast(uint64_t, L), 63));
+        double LC = 0.0;
+        float w, rd = sr, gC = 1.f, eL = 0.f;
+        if constexpr (!PRE) {
+        const double L = chunk_logs<MLSTM>(valid, sd, sw, lane, w, rd, gC, LC);
         if constexpr (STATE) {
             Lseg += LC;
             gseg *= gC;
         }
-        const float eL = exp_d(L);
+        eL = exp_d(L);
         Ls[lane] = L;
         ws[lane] = w;
         cs[lane] = gC * exp_d(LC - L) * w;
@@ -289,51 +467,29 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
             bk[lane] = bt * w;
             be[lane] = bt * w * eL;
         }
+        }
         __syncthreads();   // this chunk's rows are in LDS; nobody reads the other buffer or the last chunk's weights any more
         if (tb + kCH < te) {
             fetch(tb + kCH, buf ^ 1);
-            scalars(tb + kCH);
+            if constexpr (!PRE) scalars(tb + kCH);
         }
         const unsigned char* const qb = cs_smem + buf * M::BUF;
         const unsigned char* const kb = qb + M::Q;
         const unsigned char* const vb = kb + M::Q;
-        // rows 16 i + ln of q or k, columns 32 kk + 8 g ..: either operand of a product over columns
-        const int sp = spread<CPR>(ln);
-        auto row8 = [&](const unsigned char* base, int i, int kk) {
-            return *reinterpret_cast<const bf16x8*>(base + (16 * i + ln) * (D * 2) + (((kk * 4 + g) ^ sp) * 16));
-        };
+        const unsigned char* const pre = vb + M::V;   // PRE
+        const float* const psc = reinterpret_cast<const float*>(pre + kDtSc);
+        auto row8 = [&](const unsigned char* base, int i, int kk) { return chunk_row8<D>(base, i, kk, ln, g); };
         // k rows 32 p + 4 g + (0..3), 32 p + 16 + 4 g + (0..3), column 32 kk + 8 (ln / 4) + 4 h + ln % 4: the update's left operand
         const int r4 = 4 * g + (ln >> 2), sp4 = spread<CPR>(r4);
         auto kcol8 = [&](int p, int kk, int h) {
             const unsigned char* at = kb + (32 * p + r4) * (D * 2) + ((kk * 4 + (ln & 3)) ^ sp4) * 16 + h * 8;
             return join8(lds_read_tr4(at), lds_read_tr4(at + 16 * (D * 2)));
         };
-        // ---- weights: tile (i, j) holds rows s = 16 j.. (4 g + r) and columns t = 16 i.. (ln)
-        auto product = [&](const unsigned char* tbase, int i, int j) {
-            bf16x8 x[KK], y[KK];
-#pragma unroll
-            for (int kk = 0; kk < KK; ++kk) { x[kk] = row8(kb, j, kk); y[kk] = row8(tbase, i, kk); }
-            f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-            for (int kk = 0; kk < KK; ++kk) acc[kk & 1] = mfma_16x16x32(x[kk], y[kk], acc[kk & 1]);
-            f32x4 v = acc[0];
-            if (KK > 1) v += acc[1];
-            // times e^(L_t - L_s) w_s, for s <= t
-            const int t = 16 * i + ln;
-            const double Lt = Ls[t];
-            const f32x4 wsv = *reinterpret_cast<const f32x4*>(ws + 16 * j + 4 * g);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int s = 16 * j + 4 * g + r;
-                v[r] = s <= t ? v[r] * (wsv[r] * exp_d(Lt - Ls[s])) : 0.f;
-            }
-            return v;
-        };
         const int nrow = (nt + 15) / 16;   // 16-token rows of tiles that hold tokens
-        for (int p = STATE ? 10 : wv; p < 10; p += NW) {
+        for (int p = STATE || PRE ? 10 : wv; p < 10; p += NW) {
             const int i = p < 1 ? 0 : p < 3 ? 1 : p < 6 ? 2 : 3, j = p - i * (i + 1) / 2;
             if (i >= nrow) continue;
-            const f32x4 v = product(qb, i, j);
+            const f32x4 v = chunk_weights<D>(kb, qb, i, j, Ls, ws, ln, g);
             pt[p * 64 + lane] = v;
             if constexpr (MLSTM) {
                 float sum = (v[0] + v[1]) + (v[2] + v[3]);
@@ -342,37 +498,11 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
                 if (g == 0) psum[p * 16 + ln] = sum;
             }
         }
-        if constexpr (DELTA) {
-            // -A, A[t, s] = beta_t k-scale_t k-scale_s e^(L_t - L_s) (k_t . k_s) for s < t: wave w the tiles of column w below the
-            // diagonal, and the diagonal one's (I + A)^-1 by forward substitution, lane n column n
+        if constexpr (DELTA && !PRE) {   // wave w the tiles of column w of -A, and the diagonal one's inverse
             for (int i = wv; i < nrow; ++i) {
-                const int p = i * (i + 1) / 2 + wv, t = 16 * i + ln;
-                f32x4 v = product(kb, i, wv);
-                const float f = -bk[t];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] = 16 * wv + 4 * g + r < t ? v[r] * f : 0.f;
-                at[p * 64 + lane] = v;
-                if (i == wv) {
-                    __builtin_amdgcn_wave_barrier();   // the wave's own writes
-                    float x[16];
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        float acc[4] = {r == ln ? 1.f : 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                        for (int q = 0; q < (r + 3) / 4; ++q) {
-                            const f32x4 row = at[p * 64 + q * 16 + r];   // -A[r][4 q ..]
-#pragma unroll
-                            for (int e = 0; e < 4; ++e)
-                                if (4 * q + e < r) acc[e] += row[e] * x[4 * q + e];
-                        }
-                        x[r] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-                    }
-                    float* out = reinterpret_cast<float*>(tt + wv * 64);   // operand layout: lane (t, g) holds columns 4 g ..
-                    if (g == 0) {
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) out[((ln >> 2) * 16 + r) * 4 + (ln & 3)] = r == ln ? 0.f : x[r];   // less the identity
-                    }
-                }
+                const int p = i * (i + 1) / 2 + wv;
+                at[p * 64 + lane] = chunk_minus_a<D>(kb, i, wv, Ls, ws, bk, ln, g);
+                if (i == wv) chunk_inverse(at + p * 64, reinterpret_cast<float*>(tt + wv * 64), ln, g);
             }
         }
         if constexpr (MLSTM && !STATE) {   // n . q of the state before the chunk, this wave's rows
@@ -400,7 +530,7 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
                 for (int i = 0; i < 4; ++i) *reinterpret_cast<f32x4*>(nq + wv * kCH + 16 * i + 4 * g) = acc[i];
             }
         }
-        if constexpr (!STATE) __syncthreads();   // the weights are there
+        if constexpr (!STATE && !PRE) __syncthreads();   // the weights are there
         float fr = rd;
         if constexpr (MLSTM && !STATE) {
             const int i = lane >> 4, p0 = i * (i + 1) / 2;
@@ -411,7 +541,7 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
             odd = __builtin_fmaf(inter, 0.f, odd);
             fr = a.q_mul / (fmaxf(fabsf((intra + eL * inter) * a.q_mul), rd) + 1e-6f);
         }
-        const float eC = gC * exp_d(LC);
+        const float eC = PRE ? psc[5 * kCH] : gC * exp_d(LC);
         // ---- read-out and the state after the chunk, NI rows of tiles
         auto rest = [&](auto ni) {
             constexpr int NI = decltype(ni)::value;
@@ -453,16 +583,29 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
             for (int i = 0; i < NI; ++i)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    el[i][r] = __shfl(eL, 16 * i + 4 * g + r, 64);
-                    fo[i][r] = __shfl(fr, 16 * i + 4 * g + r, 64);
+                    el[i][r] = PRE ? psc[3 * kCH + 16 * i + 4 * g + r] : __shfl(eL, 16 * i + 4 * g + r, 64);
+                    fo[i][r] = PRE ? psc[4 * kCH + 16 * i + 4 * g + r] : __shfl(fr, 16 * i + 4 * g + r, 64);
                     oq[i][r] *= el[i][r];
                 }
             if constexpr (DELTA) {
+                const float *const bsp = PRE ? psc : bs, *const bep = PRE ? psc + kCH : be;
+                auto tile_a = [&](int i, int j) {
+                    if constexpr (PRE) return load_terms(pre + kDtA + (i * (i - 1) / 2 + j) * kDtTile, lane);
+                    else return split3(at[(i * (i + 1) / 2 + j) * 64 + lane]);
+                };
+                auto tile_t = [&](int i) {
+                    if constexpr (PRE) return load_terms(pre + kDtT + i * kDtTile, lane);
+                    else return split3(tt[i * 64 + lane]);
+                };
+                auto tile_p = [&](int i, int j) {
+                    if constexpr (PRE) return load_terms(pre + (i * (i + 1) / 2 + j) * kDtTile, lane);
+                    else return split3(pt[(i * (i + 1) / 2 + j) * 64 + lane]);
+                };
                 // (I + A) U = beta (v - e^L k-scale S^T k), 16 rows at a time
                 Terms4 ut[NI];
 #pragma unroll
                 for (int i = 0; i < NI; ++i) {
-                    const f32x4 b0 = *reinterpret_cast<const f32x4*>(bs + 16 * i + 4 * g), b1 = *reinterpret_cast<const f32x4*>(be + 16 * i + 4 * g);
+                    const f32x4 b0 = *reinterpret_cast<const f32x4*>(bsp + 16 * i + 4 * g), b1 = *reinterpret_cast<const f32x4*>(bep + 16 * i + 4 * g);
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const float p = b1[r] * ok[i][r];
@@ -481,14 +624,14 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
                         Terms4 w[NI];
                         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                        for (int j = 0; j < i; ++j) acc = mul_low(w[j] = split3(at[(i * (i + 1) / 2 + j) * 64 + lane]), ut[j], acc);
+                        for (int j = 0; j < i; ++j) acc = mul_low(w[j] = tile_a(i, j), ut[j], acc);
 #pragma unroll
                         for (int j = 0; j < i; ++j) acc = mul_high(w[j], ut[j], acc);
                         const f32x4 sum = U[i] + acc, part = sum - U[i];
                         ok[i] += (U[i] - (sum - part)) + (acc - part);
                         U[i] = sum;
                     }
-                    const Terms4 w = split3(tt[i * 64 + lane]), u = split3(U[i]);
+                    const Terms4 w = tile_t(i), u = split3(U[i]);
                     U[i] += mul_high(w, u, mul_low(w, u, ok[i]));
                     ut[i] = split3(U[i]);
                 }
@@ -498,7 +641,7 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
                     Terms4 w[NI];
                     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int j = 0; j <= i; ++j) acc = mul_low(w[j] = split3(pt[(i * (i + 1) / 2 + j) * 64 + lane]), ut[j], acc);
+                    for (int j = 0; j <= i; ++j) acc = mul_low(w[j] = tile_p(i, j), ut[j], acc);
 #pragma unroll
                     for (int j = 0; j <= i; ++j) acc = mul_high(w[j], ut[j], acc);
                     oq[i] += acc;
@@ -536,8 +679,9 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
             }
 #pragma unroll
             for (int p = 0; p < NI / 2; ++p) {
-                const f32x4 f0 = *reinterpret_cast<const f32x4*>(cs + 32 * p + 4 * g);
-                const f32x4 f1 = *reinterpret_cast<const f32x4*>(cs + 32 * p + 16 + 4 * g);
+                const float* const csp = PRE ? psc + 2 * kCH : cs;
+                const f32x4 f0 = *reinterpret_cast<const f32x4*>(csp + 32 * p + 4 * g);
+                const f32x4 f1 = *reinterpret_cast<const f32x4*>(csp + 32 * p + 16 + 4 * g);
                 const float f[8] = {f0[0], f0[1], f0[2], f0[3], f1[0], f1[1], f1[2], f1[3]};
                 float x[8];
 #pragma unroll
@@ -767,20 +911,34 @@ bool hy_chunk_scan_ok(const void* proj, int ldp, int q_off, int k_off, int v_off
            hy_chunk_scan_pays(mode, T, B, H, D, Dv, longest);
 }
 
-template <int D, int MODE, bool STATE>
+template <int D, int MODE, bool STATE, bool PRE = false>
 static void chunk_scan_pass(const hy::ChunkScan& a, int segs, hipStream_t s) {
-    constexpr int lds = hy::ChunkLds<D, MODE>::SIZE;
+    constexpr int lds = hy::ChunkLds<D, MODE, PRE>::SIZE;
     static_assert(lds <= 160 * 1024, "LDS of one workgroup");
-    const auto kern = hy::chunk_scan_kernel<D, MODE, STATE>;
+    const auto kern = hy::chunk_scan_kernel<D, MODE, STATE, PRE>;
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     const int nslab = (a.Dv + 16 * hy::kCW - 1) / (16 * hy::kCW);
     kern<<<dim3((a.B * a.H + 7) / 8 * 8 * nslab, segs), 64 * hy::kCW, lds, s>>>(a);
 }
 template <int D, int MODE>
 static void chunk_scan_run(const hy::ChunkScan& a, hipStream_t s) {
-    if constexpr (MODE != hy::kScanDelta)
+    if constexpr (MODE != hy::kScanDelta) {
         if (a.segs > 1) chunk_scan_pass<D, MODE, true>(a, a.segs - 1, s);
+    } else if (a.tiles != nullptr) {
+        constexpr int lds = 4 * hy::kCH * D + 8192 + 4 * 1024;
+        const auto kern = hy::delta_tiles_kernel<D>;
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        kern<<<(unsigned)(hy::delta_slots(a.T, a.B) * a.H), 256, lds, s>>>(a);
+        return chunk_scan_pass<D, MODE, false, true>(a, a.segs, s);
+    }
     chunk_scan_pass<D, MODE, false>(a, a.segs, s);
+}
+
+// Bytes of scratch for the delta rule's tiles, or 0: made between the steps, as where no sequence has two chunks, and of launches whose tiles would take more
+// than 512 MB (a prompt portion of 32768 tokens and 16 heads takes 270).
+int64_t hy_delta_tiles_bytes(const void* proj, int ldp, int q_off, int k_off, int v_off, int T, int B, int H, int D, int Dv, int longest) {
+    const int64_t n = hy::delta_slots(T, B) * H * hy::kDeltaTiles;
+    return longest > hy::kCH && n <= (int64_t)512 << 20 && hy_chunk_scan_ok(proj, ldp, q_off, k_off, v_off, T, B, H, D, Dv, longest, hy::kScanDelta) ? n : 0;
 }
 
 // Segments that a sequence's chunks are dealt to, here and in gla_scan.hip: launches that leave half of the CUs or more without a
@@ -820,13 +978,13 @@ static void chunk_scan_d(int D, const hy::ChunkScan& a, hipStream_t s) {
 }
 
 // One decay per head and token (dts = H) or per head (dts = 0), with beta the delta correction (D <= 128); see
-// launch_hy_linear_scan.
+// launch_hy_linear_scan.  seg: hy_chunk_segment_floats, with beta hy_delta_tiles_bytes or nullptr.
 void launch_hy_chunk_scan(const uint16_t* proj, int ldp, int q_off, int k_off, int v_off, const float* qscale, const float* kscale,
                           float q_mul, const float* decay, int dts, const float* beta, const int32_t* q_start,
-                          const int32_t* pos0, const int32_t* slots, float* S, float* o, int B, int HK, int H, int D, int Dv, const float* vscale,
+                          const int32_t* pos0, const int32_t* slots, float* S, float* o, int T, int B, int HK, int H, int D, int Dv, const float* vscale,
                           int segs, float* seg, hipStream_t s) {
     hy::ChunkScan a{proj, ldp, q_off, k_off, v_off, qscale, kscale, vscale, decay, beta, dts, q_mul, nullptr, nullptr, nullptr,
-                    q_start, pos0, slots, nullptr, S, nullptr, o, B, HK, H, Dv, 1, nullptr, nullptr, nullptr};
+                    q_start, pos0, slots, nullptr, S, nullptr, o, B, HK, H, Dv, T, 1, nullptr, nullptr, nullptr, beta != nullptr ? reinterpret_cast<unsigned char*>(seg) : nullptr};
     if (beta == nullptr && segs > 1) chunk_scan_scratch(a, D, segs, seg);
     if (beta != nullptr) chunk_scan_d<hy::kScanDelta>(D, a, s);
     else chunk_scan_d<hy::kScanPlain>(D, a, s);
@@ -840,7 +998,7 @@ void launch_hy_chunk_mlstm(const uint16_t* proj, int ldp, const float* gate_pre,
     float *la = scratch, *lb = la + th, *em = lb + th, *n0 = em + th;
     hy::mlstm_gates_kernel<<<dim3(B, H), 256, 0, s>>>(gate_pre, q_start, pos0, slots, n, m, n0, la, lb, em, H, D, cap);
     hy::ChunkScan a{proj, ldp, 0, H * D, 2 * H * D, nullptr, nullptr, nullptr, nullptr, nullptr, H, 1.f / sqrtf((float)D), la, lb, em,
-                    q_start, pos0, slots, n0, S, n, o, B, H, H, Dv, 1, nullptr, nullptr, nullptr};
+                    q_start, pos0, slots, n0, S, n, o, B, H, H, Dv, T, 1, nullptr, nullptr, nullptr, nullptr};
     if (segs > 1) chunk_scan_scratch(a, D, segs, n0 + (int64_t)B * H * D);
     chunk_scan_d<hy::kScanMlstm>(D, a, s);
 }

@@ -431,7 +431,7 @@ __global__ void __launch_bounds__(256) linear_scan_kernel(
 
 bool hy_chunk_scan_ok(const void*, int, int, int, int, int, int, int, int, int, int, int);
 void launch_hy_chunk_scan(const uint16_t*, int, int, int, int, const float*, const float*, float, const float*, int,
-                          const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*, int, int, int, int, int, const float*,
+                          const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*, int, int, int, int, int, int, const float*,
                           int, float*, hipStream_t);
 
 bool hy_gla_scan_ok(const void*, const void*, int, int, int, int, int, int, int, int, int);
@@ -529,7 +529,7 @@ static bool linear_scan_d(bool pipe, const T* proj, int ldp, int q_off, int k_of
 // chd: decay holds one number per state row ([T, H, D]) instead of one per head ([T, H]).
 // fixed (not with chd): decay holds one number per head for all tokens ([H]).
 // longest: the most tokens that any sequence brings, as far as the caller knows (it only picks the kernel).
-// segs, seg: hy_chunk_segments and its scratch.
+// segs, seg: hy_chunk_segments and its scratch; with beta 1 and hy_delta_tiles_bytes of scratch, or nullptr.
 // Returns false when D has no instantiation (D > 256).
 bool launch_hy_linear_scan(const void* proj, int ldp, int q_off, int k_off, int v_off, const float* qscale,
                            const float* kscale, float q_mul, const float* decay, bool chd, bool fixed, const float* beta,
@@ -550,7 +550,7 @@ bool launch_hy_linear_scan(const void* proj, int ldp, int q_off, int k_off, int 
     }
     if (!chd && !f32 && hy_chunk_scan_ok(proj, ldp, q_off, k_off, v_off, T, B, H, D, Dv, longest, delta ? hy::kScanDelta : hy::kScanPlain)) {
         launch_hy_chunk_scan((const uint16_t*)proj, ldp, q_off, k_off, v_off, qscale, kscale, q_mul, decay, fixed ? 0 : H, beta,
-                             q_start, pos0, slots, S, o, B, HK, H, D, Dv, vscale, segs, seg, s);
+                             q_start, pos0, slots, S, o, T, B, HK, H, D, Dv, vscale, segs, seg, s);
         return true;
     }
     const int dts = fixed ? 0 : H;
