@@ -916,7 +916,8 @@ static void chunk_scan_pass(const hy::ChunkScan& a, int segs, hipStream_t s) {
     constexpr int lds = hy::ChunkLds<D, MODE, PRE>::SIZE;
     static_assert(lds <= 160 * 1024, "LDS of one workgroup");
     const auto kern = hy::chunk_scan_kernel<D, MODE, STATE, PRE>;
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    (void)set;
     const int nslab = (a.Dv + 16 * hy::kCW - 1) / (16 * hy::kCW);
     kern<<<dim3((a.B * a.H + 7) / 8 * 8 * nslab, segs), 64 * hy::kCW, lds, s>>>(a);
 }
@@ -927,7 +928,8 @@ static void chunk_scan_run(const hy::ChunkScan& a, hipStream_t s) {
     } else if (a.tiles != nullptr) {
         constexpr int lds = 4 * hy::kCH * D + 8192 + 4 * 1024;
         const auto kern = hy::delta_tiles_kernel<D>;
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        (void)set;
         kern<<<(unsigned)(hy::delta_slots(a.T, a.B) * a.H), 256, lds, s>>>(a);
         return chunk_scan_pass<D, MODE, false, true>(a, a.segs, s);
     }

@@ -67,7 +67,8 @@ def load() -> None:
 
 
 def _k():
-    load()
+    if not _loaded:
+        load()
     return torch.ops.chronos
 
 

@@ -20,10 +20,19 @@ Routing is by measured shape:
 from __future__ import annotations
 
 import os
+import sys
 from dataclasses import dataclass
 from typing import Callable, Optional
 
 import torch
+
+_pkg = sys.modules[__package__]
+
+
+def _k():
+    """The package's kernels.  (An import statement inside every function here cost a step of a hybrid decoder 30 us.)"""
+    return _pkg._k()
+
 
 # Largest M routed to the GEMV (gemv_ok).  Env CHRONOS_GEMV_MAX_M; scripts/single_stream.py A/Bs it (py_gemv_max_m).
 # M = 2 goes to the skinny MFMA GEMM: the two-row GEMV streams at 1-3.5 TB/s against 4-5.5 at M = 1 and the skinny
@@ -328,8 +337,6 @@ def product_f32(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
     plan = few_rows_plan(m, n, k) or mid_rows_plan(m, n, k)
     if plan is None or plan[0] not in _SLICED:
         return None
-    from . import _k
-
     skinny = plan[0] >= SK_BASE
     return _k().gemm_f32(x, w, plan[0] - SK_BASE * skinny, plan[1], skinny)
 
@@ -342,8 +349,6 @@ def product_slices(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
     plan = few_rows_plan(m, n, k)
     if plan is None or plan[1] == 1 or (plan[0] >= SK_BASE and plan[0] not in _UNEVEN):
         return None
-    from . import _k
-
     skinny = plan[0] >= SK_BASE
     return _k().gemm_slices(x, w, plan[0] - SK_BASE * skinny, plan[1], skinny)
 
@@ -515,8 +520,6 @@ def product_act(x: torch.Tensor, w: torch.Tensor, mode: int, limit: float = 0.0,
     if 64 < m < MANY_MIN or PP_MODE != "auto" or x.dim() != 2 or not _plain_rows(x, w) or _registered(m, n, k):
         return None
     if m <= 64:
-        from . import _k
-
         cfg = _few_more(m, n, k, 2 if mode == 3 else 1)
         return _k().gemm_few(x, w, cfg, mode, 0, 0, None, limit, slope, shift)[0] if cfg else None
     glu = mode == 3
@@ -527,8 +530,6 @@ def product_act(x: torch.Tensor, w: torch.Tensor, mode: int, limit: float = 0.0,
         pays = _plan_cache[key] = _many_act_pays(rows, n, k, glu)
     if not pays:
         return None
-    from . import _k
-
     return _k().gemm_act(x, w, mode, limit, slope, shift)
 
 
@@ -561,18 +562,20 @@ def product_rows(x: torch.Tensor, w: torch.Tensor, n0: int, nf: int, bias: Optio
     cfg = _few_more(x.shape[0], *w.shape, 0)
     if not cfg:
         return None
-    from . import _k
-
     return _k().gemm_few(x, w, cfg, 0, n0, nf, bias, 0.0, 0.0, 0.0)
+
+
+_Tensor, _WEIGHTS, _BF16 = torch.Tensor, (torch.Tensor, torch.nn.Parameter), torch.bfloat16
+_autocast, _grad, _functorch, _forward_ad = torch.is_autocast_enabled, torch.is_grad_enabled, torch._C._are_functorch_transforms_active, torch.autograd.forward_ad
 
 
 def _plain_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Operands that the kernels take as they lie, and nothing that has to see the product (gradients, transforms,
     autocast, subclasses)."""
-    return (type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter) and not torch.is_autocast_enabled("cuda") and x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16 and w.dim() == 2
-            and w.shape[1] == x.shape[-1] and w.device == x.device
-            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
-            and not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0
+    return (type(x) is _Tensor and type(w) in _WEIGHTS and not _autocast("cuda") and x.dtype is _BF16 and w.dtype is _BF16 and w.dim() == 2
+            and w.shape[1] == x.shape[-1] and w.is_cuda is x.is_cuda and w.get_device() == x.get_device()
+            and not (_grad() and (x.requires_grad or w.requires_grad))
+            and not _functorch() and _forward_ad._current_level < 0
             and x.is_contiguous() and w.is_contiguous() and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 
 
@@ -580,13 +583,12 @@ def pp_gemm(x: torch.Tensor, w: torch.Tensor, mode: int, plan: tuple[int, int], 
             eps: float = 1e-5):
     """One launch of gemm_pp.hip (or gemm_skinny.hip for a skinny plan): returns (y, partials) — partials only for
     the residual epilogue."""
-    from . import _k
-
-    k = x.shape[-1]
+    if x.dim() != 2:
+        x = x.reshape(-1, x.shape[-1])
     if plan[0] >= SK_BASE:
-        return _k().gemm_skinny(x.reshape(-1, k), w, mode, plan[0] - SK_BASE, plan[1], resid, part, eps)
-    y, pt = _k().gemm_pp(x.reshape(-1, k), w, mode, plan[0], plan[1], resid, part, eps, False)
-    return y, pt
+        return _k().gemm_skinny(x, w, mode, plan[0] - SK_BASE, plan[1], resid, part, eps)
+    return _k().gemm_pp(x, w, mode, plan[0], plan[1], resid, part, eps, False)
+
 
 # (M, N, K) -> bool predicate + kernel; extension point for further shape-specialised kernels
 _custom: list[tuple[Callable[[int, int, int], bool], Callable[[torch.Tensor, torch.Tensor], torch.Tensor]]] = []
@@ -670,8 +672,6 @@ def gemv_resid(x: torch.Tensor, w: torch.Tensor, resid: torch.Tensor) -> ResidOu
     """Producer (O / down projection, TP=1): the new residual stream s = bf16(bf16(x @ w.T) + resid) and the RMSNorm
     partial sums of s^2, in one launch — the GEMV at M <= 2, the batched GEMM's kResid epilogue above.  ``w`` may be
     an fp8 QTensor at the W8A16 GEMV shapes (resid_ok(..., fp8=True))."""
-    from . import _k
-
     m, k = x.numel() // x.shape[-1], x.shape[-1]
     if is_q(w):
         s = torch.empty(resid.shape, dtype=resid.dtype, device=resid.device)
@@ -709,16 +709,12 @@ def mfma_swiglu_ok(m: int, n: int, k: int) -> bool:
 
 
 def _gemv(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False) -> torch.Tensor:
-    from . import _k
-
     k = x.shape[-1]
     y = _k().gemv(x.reshape(-1, k), w, swiglu)
     return y.view(*x.shape[:-1], y.shape[-1])
 
 
 def mfma_gemm(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False, stages: int = 3) -> torch.Tensor:
-    from . import _k
-
     k = x.shape[-1]
     y = _k().gemm(x.reshape(-1, k), w, swiglu, stages)
     return y.view(*x.shape[:-1], y.shape[-1])
@@ -727,7 +723,7 @@ def mfma_gemm(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False, stages: in
 def gate_up_silu(x: torch.Tensor, w_gu: torch.Tensor) -> torch.Tensor:
     """silu(x @ gate.T) * (x @ up.T) with w_gu = [gate; up]: one fused launch (GEMV at M <= 2, the batched GEMM's
     SwiGLU epilogue above, with the folded input norm when x is a LazyNorm), else GEMM + silu_mul."""
-    from . import _k, silu_mul
+    from . import silu_mul
 
     if is_q(w_gu):  # fp8 weights: the W8A16 GEMV (folded norm fused when x is a LazyNorm), else W8A8
         m, n, k = (x.rows() if isinstance(x, LazyNorm) else x.numel() // x.shape[-1]), w_gu.shape[0], x.shape[-1]
@@ -760,10 +756,18 @@ def gate_up_silu(x: torch.Tensor, w_gu: torch.Tensor) -> torch.Tensor:
     return silu_mul(linear(x, w_gu))
 
 
+def _linear_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
+    """The rules' plan of a plain product whose operands _plain_rows takes, or None: one look-up for a shape that was here before."""
+    key = (m, n, k, "linear", PP_MODE, GEMV_MAX_M)
+    hit = _plan_cache.get(key, False)
+    if hit is False:
+        hit = (few_rows_plan(m, n, k) if m <= 64 else slab_rows_plan(m, n, k) if m >= MANY_MIN else None) or (mid_rows_plan(m, n, k) if 32 < m <= 512 else None)
+        _plan_cache[key] = hit
+    return hit
+
+
 def linear(x, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     if is_q(w):  # fp8 weights: the W8A16 GEMV (folded norm fused when x is a LazyNorm), else W8A8
-        from . import _k
-
         m, n, k = (x.rows() if isinstance(x, LazyNorm) else x.numel() // x.shape[-1]), w.shape[0], x.shape[-1]
         if isinstance(x, LazyNorm) and x.fusable() and m <= 2 and gemv_q_ok(m, n, k):
             return _k().gemv_normp(x.s, x.part, x.eps, w.q, False, w.s)
@@ -775,8 +779,6 @@ def linear(x, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tens
     if isinstance(x, LazyNorm):
         m, n, k = x.rows(), w.shape[0], x.shape[-1]
         if x.fusable() and out is None and gemv_ok(m, n, k):
-            from . import _k
-
             return _k().gemv_normp(x.s, x.part, x.eps, w, False)
         plan = pp_plan(m, n, k, PP_PLAIN) if x.fusable() and out is None else None
         if plan is not None:
@@ -788,15 +790,17 @@ def linear(x, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tens
         n = w.shape[0]
         few = None
         if out is None and m > 0 and _plain_rows(x, w):
-            few = (few_rows_plan(m, n, k) if m <= 64 else slab_rows_plan(m, n, k) if m >= MANY_MIN else None) or (mid_rows_plan(m, n, k) if 32 < m <= 512 else None)
+            few = _linear_plan(m, n, k)
+            if few is not None and not _custom and x.dim() == 2:   # (what follows, without the views)
+                if few[1] > 1 and few[0] < SK_BASE and few[0] != 88:
+                    return _k().gemm_split(x, w, few[0], few[1])
+                return pp_gemm(x, w, PP_PLAIN, few)[0]
         if few is None and gemv_ok(m, n, k):
             return _gemv(x, w)
         for pred, fn in _custom:
             if pred(m, n, k):
                 return fn(x, w)
         if few is not None and few[1] > 1 and few[0] < SK_BASE and few[0] != 88:   # a split without tickets
-            from . import _k
-
             return _k().gemm_split(x.reshape(-1, k), w, *few).view(*x.shape[:-1], n)
         plan = (few or pp_plan(m, n, k, PP_PLAIN)) if out is None else None
         if plan is not None:

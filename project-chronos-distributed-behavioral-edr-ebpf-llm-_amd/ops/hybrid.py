@@ -12,12 +12,14 @@ stream, norms, recurrent state, gates, router and attention scores are float32 i
 from __future__ import annotations
 
 import os
+import sys
 
 import torch
 
-from . import hybrid_ref as ref
+from . import gemm as _gemm, hybrid_ref as ref
 from .hybrid_ref import ACT_GELU, ACT_GLU, ACT_RELU2  # noqa: F401
 
+_pkg = sys.modules[__package__]
 _REF_ON_GPU = os.environ.get("CHRONOS_HYBRID_REF", "0") not in ("", "0")
 
 
@@ -39,7 +41,8 @@ def load() -> None:
 
 
 def _k():
-    load()
+    if not _lib_loaded:
+        load()
     return torch.ops.chronos
 
 
@@ -54,18 +57,14 @@ def matmul(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None) -
     if bias is not None:
         return torch.addmm(bias, x, w.t())
     if x.dtype == torch.bfloat16:
-        from . import linear
-
-        return linear(x, w)
+        return _pkg.linear(x, w)
     return torch.matmul(x, w.t())
 
 
 def matmul_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x @ w.T as float32: the product's sums themselves where the framework's kernels take it, else the rounded product's values."""
     if _gpu(x) and x.dtype == torch.bfloat16:
-        from .gemm import product_f32
-
-        y = product_f32(x, w)
+        y = _gemm.product_f32(x, w)
         if y is not None:
             return y
     return matmul(x, w).float()
@@ -75,9 +74,7 @@ def matmul_slices(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x @ w.T for add_layer_norm or scale_add_rms_norm, which also take a product of few rows as the float32 slices [S, T, n] of its split and
     sum and round them themselves, a launch less."""
     if _gpu(x) and x.dtype == torch.bfloat16:
-        from .gemm import product_slices
-
-        y = product_slices(x, w)
+        y = _gemm.product_slices(x, w)
         if y is not None:
             return y
     return matmul(x, w)
@@ -129,9 +126,7 @@ def matmul_rowdot(h, w, w_few, bias=None, joined=None):
     """(h @ w.T, rowdot(h, w_few, bias)); ``joined`` (whole, n0, nf): both matrices' rows one behind the other, which few rows of h take in
     one launch."""
     if joined is not None and _gpu(h) and h.dtype == torch.bfloat16:
-        from .gemm import product_rows
-
-        y = product_rows(h, *joined, bias)
+        y = _gemm.product_rows(h, *joined, bias)
         if y is not None:
             return y
     return matmul(h, w), rowdot(h, w_few, bias)
@@ -147,9 +142,7 @@ def act_inplace(x, kind: int):
 def matmul_act(x, w, kind: int):
     """act_inplace(x @ w.T, kind), in the product's epilogue where that is faster (the activation then reads the unrounded product)."""
     if _gpu(x) and x.dtype == torch.bfloat16 and kind in (ACT_RELU2, ACT_GELU):
-        from .gemm import product_act
-
-        y = product_act(x, w, 4 if kind == ACT_RELU2 else 5)
+        y = _gemm.product_act(x, w, 4 if kind == ACT_RELU2 else 5)
         if y is not None:
             return y
     return act_inplace(matmul(x, w), kind)
@@ -158,9 +151,7 @@ def matmul_act(x, w, kind: int):
 def matmul_glu(x, w, limit: float, slope: float, shift: float, act_dtype):
     """glu(x @ w.T, ...), w = [gate; up], in the product's epilogue where that is faster (the unit then reads the unrounded product)."""
     if _gpu(x) and x.dtype == torch.bfloat16 and act_dtype == torch.bfloat16:
-        from .gemm import product_act
-
-        y = product_act(x, w, 3, limit, slope, shift)
+        y = _gemm.product_act(x, w, 3, limit, slope, shift)
         if y is not None:
             return y
     return glu(matmul(x, w), limit, slope, shift, act_dtype)
