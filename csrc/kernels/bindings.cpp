@@ -733,13 +733,13 @@ std::tuple<Tensor, Tensor> gemm_few(const Tensor& x, const Tensor& w, int64_t cf
 }
 
 // The float32 slices [splitk, M, N] of a plain product of few rows whose K is split over workgroups, nothing kept between calls: gemm_lg.hip's
-// ring tiles of few rows, or (skinny) gemm_skinny.hip's uneven configs.  Their sum in order, rounded, is the product; one slice is the product unrounded.
+// ring tiles of few rows, gemm_slab.hip (88, two slices and more), or (skinny) gemm_skinny.hip's uneven configs.  Their sum in order, rounded, is the product; one slice is the product unrounded.
 Tensor gemm_slices(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk, bool skinny) {
     chk_bf16(x, "x");
     chk_bf16(w, "w");
     const int64_t K = x.size(-1), M = x.numel() / K, N = w.size(0);
     CHK(w.dim() == 2 && w.size(1) == K, "gemm_split: w must be [N, K]");
-    CHK(skinny ? cfg >= chronos::kSkinnyUneven && cfg < chronos::kSkinnyConfigs : cfg == 19 || cfg == 32 || cfg == 33 || cfg == 36 || (cfg >= 38 && cfg <= 39) || (cfg >= 72 && cfg <= 75) || cfg == 78 || cfg == 79, "gemm_split: cfg");
+    CHK(skinny ? cfg >= chronos::kSkinnyUneven && cfg < chronos::kSkinnyConfigs : cfg == 19 || cfg == 32 || cfg == 33 || cfg == 36 || (cfg >= 38 && cfg <= 39) || (cfg >= 72 && cfg <= 75) || cfg == 78 || cfg == 79 || (cfg == 88 && splitk > 1), "gemm_split: cfg");
     const int BM = skinny ? 16 * chronos::gemm_skinny_mt((int)cfg) : chronos::gemm_lg_xm((int)cfg);
     const int BN = skinny ? 16 * chronos::gemm_skinny_rt((int)cfg) : chronos::gemm_lg_wn((int)cfg);
     CHK((N + BN) * K * 2 < (1LL << 31) && (M + BM) * K * 2 < (1LL << 31), "gemm_split: operand > 2 GiB");

@@ -285,8 +285,9 @@ bool launch_gemm_slab(int mode, bool normp, const PPArgs& a, hipStream_t st) {
         if (mode != kPPPlain && mode != kPPResid) return false;
         normp ? slab_launch<kPPPart, true>(a, st) : slab_launch<kPPPart, false>(a, st);
         const int64_t n = (int64_t)a.M * a.N;
-        if (mode == kPPPlain) launch_gemm_slices(a.ws, a.y, n, a.splitk, st);
-        else slab_sum_resid_kernel<<<(unsigned)((n / 8 + 255) / 256), 256, 0, st>>>(a.ws, a.resid, a.y, a.part_out, n, a.splitk);
+        if (mode == kPPPlain) {
+            if (a.y != nullptr) launch_gemm_slices(a.ws, a.y, n, a.splitk, st);   // (else the slices are what is wanted)
+        } else slab_sum_resid_kernel<<<(unsigned)((n / 8 + 255) / 256), 256, 0, st>>>(a.ws, a.resid, a.y, a.part_out, n, a.splitk);
         return true;
     }
     switch (mode) {

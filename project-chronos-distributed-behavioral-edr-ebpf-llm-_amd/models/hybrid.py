@@ -1423,9 +1423,9 @@ class HybridDecoder:
                 self.layer_tap(ri, x)
 
     def last_product(self, x, w, bias=None):
-        """A sublayer's last product, in the form that its stream's join takes (see _join and matmul_slices)."""
+        """A sublayer's last product, in the form that its stream's join takes (see _join and matmul_parts)."""
         if bias is None and self.cfg.residual in ("out_norm", "post_norm"):
-            return hops.matmul_slices(x, w)
+            return hops.matmul_parts(x, w)
         return hops.matmul(x, w, bias)
 
     def _join(self, y, x, w):

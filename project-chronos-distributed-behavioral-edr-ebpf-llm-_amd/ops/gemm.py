@@ -353,6 +353,19 @@ def product_slices(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
     return _k().gemm_slices(x, w, plan[0] - SK_BASE * skinny, plan[1], skinny)
 
 
+def product_parts(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
+    """product_slices beyond 64 rows: the slices where linear()'s rules split K.  Product, its sum and the
+    join behind it -> product and join, us: 113 rows of 1024 x 2816 12.1 -> 9.7, of 2048 x 5632 18.3 -> 15.0, 200 of 2048 x 2048 14.8 -> 11.5, 700 of 4096 x 11008 77 -> 71, 1351 of 4096 x
+    14336 153 -> 149, 3000 of 2048 x 5632 88 -> 76; faster at all of 72 measured."""
+    (m, k), n = x.shape if x.dim() == 2 else (0, 0), w.shape[0]
+    if m <= 64 or n % 8 or n > 8192 or not _plain_rows(x, w) or _registered(m, n, k):
+        return None
+    plan = _linear_plan(m, n, k)
+    if plan is None or plan[1] == 1 or plan[0] >= SK_BASE:
+        return None
+    return _k().gemm_slices(x, w, plan[0], plan[1], False)
+
+
 # Many rows, shapes that the plan does not list: what a launch takes in us, fitted on a grid of M = 65 .. 8192, N = 512 .. 16384, K = 512 ..
 # 8192 (rms error 8 %).  88 (gemm_slab.hip): constant, per half tile of the last round, per 64-deep step of a round of
 # 256 x 256 tiles and of the halves, per M of results, per M of weights; 19 and 32 (128 x rows by 128 and 64 W rows): constant, per round of

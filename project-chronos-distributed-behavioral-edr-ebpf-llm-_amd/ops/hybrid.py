@@ -80,6 +80,14 @@ def matmul_slices(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return matmul(x, w)
 
 
+def matmul_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """matmul_slices for any number of rows."""
+    if _gpu(x) and x.dtype == torch.bfloat16 and x.shape[0] > 64:
+        y = _gemm.product_parts(x, w)
+        return matmul(x, w) if y is None else y
+    return matmul_slices(x, w)
+
+
 def embed_rows(ids, table, act_dtype, scale: float = 1.0, emit: bool = True):
     """(float32 residual rows times ``scale``, the same rows in the activation dtype or None when ``emit`` is off)."""
     if _gpu(table):
