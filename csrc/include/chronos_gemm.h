@@ -17,14 +17,15 @@ struct PPArgs {
     int M, N, K, F, nparts_in, splitk, kts;
     float eps;
     int gm;      // tile order: M-tiles per group (0 = every M-tile of a W panel consecutive); knob pp_gm
+    int turn;          // gemm_lg, ring tiles, one x tile: workgroups start their K at different stages (sums in another order)
     int handoff;       // gemm_lg split-K slab hand-off (knob lg_handoff): -1 auto, 0 fences, 1 write-through
     float limit, slope, shift;  // kPPGlu: min(g, limit) sigmoid(slope g) (clamp(u, -limit, limit) + shift)
-    float* yf;          // gemm_skinny, plain: outputs n0 .. n0 + nf go here, float32 [M, nf], plus bias; y is [M, n0] then
+    int act;            // gemm_lg, ring tiles: kPPRelu2 or kPPGelu on the plain product, kPPGlu in place of SwiGLU
+    float* yf;          // gemm_skinny, gemm_lg's ring tiles, plain: outputs n0 .. n0 + nf go here, float32 [M, nf], plus bias; y is [M, n0] then
     const float* bias;
     int n0, nf;
     const float* xsc;  // gemm_lg F8 (W8A8 e4m3fn bytes in x / w): per-token scales [M]
     const float* wsc;  // ... and per-output-channel scales [N]
-    int turn;          // gemm_lg, ring tiles, one x tile: workgroups start their K at different stages (sums in another order)
     int ablate;  // timing-only diagnostics (knob pp_ablate): 1 skip loop DMA, 2 skip LDS reads, 4 skip MFMA, 8 nt weights, 16/32 alias every W/x tile onto tile 0
 };
 
@@ -49,6 +50,8 @@ int gemm_lg_wn(int cfg);  // W rows per tile
 bool gemm_lg_splitk_ok(int cfg);  // false for 81-87, names of 88 that never took a split
 bool gemm_lg_sliced(int cfg, int mode);  // its split-K writes float32 slices [splitk, M, N] and needs no tickets (gemm_slab.hip)
 bool gemm_lg_ablations_built();  // the timing-only ablation ids 40-71 exist (CHRONOS_GEMM_ABLATIONS build)
+// plain ring tiles 19, 32, 38, 39, 72, 74, 75, 79, unsplit, with act (kPPGlu: glu) or with yf
+bool launch_gemm_ring(int cfg, bool glu, const PPArgs& a, hipStream_t st);
 bool launch_gemm_lg(int cfg, int mode, bool normp, const PPArgs& a, hipStream_t st);
 // config 88 without split-K or (plain, resid) with it, and the hybrid decoders' epilogues (csrc/kernels/gemm_slab.hip)
 bool launch_gemm_slab(int mode, bool normp, const PPArgs& a, hipStream_t st);
@@ -69,6 +72,7 @@ int gemm_skinny_mt(int cfg);
 int gemm_skinny_nw(int cfg);  // waves per workgroup
 // y [n] = the sum of S float32 slices [S, n], in their order
 void launch_gemm_slices(const float* ws, uint16_t* y, int64_t n, int S, hipStream_t st);
+void launch_gemm_slices_rows(const float* ws, uint16_t* y, float* yf, const float* bias, int M, int N, int n0, int nf, int S, hipStream_t st);
 void launch_gemm_slices_f32(const float* ws, float* y, int64_t n, int S, hipStream_t st);
 bool launch_gemm_skinny(int cfg, int mode, bool normp, const PPArgs& a, hipStream_t st);
 

@@ -19,6 +19,8 @@ struct GemvNorm {
     uint16_t* rout;        // producer: residual out [M, N]
     float* part_out;       // producer: partials [M, gridDim.x]
     const float* wscale;   // fp8-e4m3 weights (W8A16): per-output-row scale [N]; nullptr = bf16 weights
+    int act;               // launch_gemv_act
+    float limit, slope, shift;
 };
 
 struct GemvRope {
@@ -39,6 +41,7 @@ struct GemvRope {
 // wscale != nullptr: W is fp8-e4m3 bytes [N, K] with per-row scales (W8A16: bf16 activations, K % 1024 == 0, M <= 2)
 void launch_gemv_ex(const uint16_t* x, int M, int K, const uint16_t* W, int N, uint16_t* y, bool swiglu,
                     const GemvNorm* nrm, const GemvRope* rope, bool fp8, hipStream_t st, const float* wscale = nullptr);
+void launch_gemv_act(const uint16_t* x, int K, const uint16_t* W, int N, uint16_t* y, int mode, float limit, float slope, float shift, hipStream_t st);
 // producer: rout = bf16(bf16(x @ W^T) + rin), part_out[m, wg] = per-workgroup sum of rout^2; returns nparts
 int launch_gemv_resid(const uint16_t* x, int M, int K, const uint16_t* W, int N, const uint16_t* rin, uint16_t* rout,
                       float* part_out, hipStream_t st, const float* wscale = nullptr);

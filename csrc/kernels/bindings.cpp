@@ -766,6 +766,78 @@ Tensor gemm_slices(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk
     return ws;
 }
 
+// gemm_few on gemm_lg.hip's ring tiles: mode 0 with float32 outputs n0 .. n0 + nf of w's rows behind the n0 others, K split over workgroups or not; with an
+// activation (3: N % the tile's rows == 0) unsplit.
+std::tuple<Tensor, Tensor> gemm_ring(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk, int64_t mode, int64_t n0, int64_t nf,
+                                     const c10::optional<Tensor>& bias, double limit, double slope, double shift) {
+    chk_bf16(x, "x");
+    chk_bf16(w, "w");
+    CHK(x.dim() == 2 && w.dim() == 2 && w.size(1) == x.size(1), "gemm_ring: x [M, K], w [N, K]");
+    CHK(cfg == 19 || cfg == 32 || cfg == 38 || cfg == 39 || cfg == 72 || cfg == 74 || cfg == 75 || cfg == 79, "gemm_ring: cfg");
+    CHK(mode == 0 || (mode >= chronos::kPPGlu && mode <= chronos::kPPGelu), "gemm_ring: mode");
+    const int64_t K = x.size(1), M = x.size(0), rows = w.size(0);
+    const int BM = chronos::gemm_lg_xm((int)cfg), BN = chronos::gemm_lg_wn((int)cfg);
+    CHK(mode == 0 ? n0 > 0 && nf > 0 && n0 % 4 == 0 && n0 <= rows && nf <= rows - n0 : n0 == 0 && nf == 0, "gemm_ring: n0 % 4 == 0, n0 + nf <= rows; with an activation no float32 outputs");
+    const int64_t N = mode == 0 ? (n0 + nf + 3) / 4 * 4 : rows;
+    CHK(N <= rows && N % 4 == 0 && (mode != chronos::kPPGlu || N % BN == 0), "gemm_ring: rows in 4s (gated units: whole tiles)");
+    CHK((rows + BN) * K * 2 < (1LL << 31) && (M + BM) * K * 2 < (1LL << 31), "gemm_ring: operand > 2 GiB");
+    CHK(M >= 1 && K >= 64 && K % 64 == 0 && K <= (1 << 20), "gemm_ring: size");
+    CHK(splitk >= 1 && splitk <= 64 && (K / 64) % splitk == 0 && (mode == 0 || splitk == 1), "gemm_ring: splitk must divide K / 64 (activations: 1)");
+    CHK(((reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr())) & 15) == 0, "gemm_ring: alignment");
+    if (bias.has_value()) {
+        chk_gpu(*bias, "bias");
+        CHK(bias->scalar_type() == at::kFloat && bias->numel() == nf, "gemm_ring: bias [nf] f32");
+    }
+    c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+    chronos::PPArgs a{};
+    a.x = bf(x);
+    a.w = bf(w);
+    a.M = (int)M;
+    a.N = (int)N;
+    a.K = (int)K;
+    a.F = (int)(N / 2);
+    a.splitk = (int)splitk;
+    a.kts = (int)(K / 64 / splitk);
+    a.gm = chronos::knob("pp_gm", 8);
+    a.turn = 1;
+    a.act = (int)mode;
+    a.limit = (float)limit;
+    a.slope = (float)slope;
+    a.shift = (float)shift;
+    Tensor y = at::empty({M, mode == chronos::kPPGlu ? N / 2 : mode == 0 ? n0 : N}, x.options()), yf, ws;
+    a.y = bfm(y);
+    const float* b = bias.has_value() ? bias->data_ptr<float>() : nullptr;
+    if (mode == 0) yf = at::empty({M, nf}, x.options().dtype(at::kFloat));
+    if (splitk > 1) {
+        ws = at::empty({splitk, M, N}, x.options().dtype(at::kFloat));
+        a.ws = ws.data_ptr<float>();
+    } else if (mode == 0) {
+        a.yf = yf.data_ptr<float>();
+        a.bias = b;
+        a.n0 = (int)n0;
+        a.nf = (int)nf;
+    }
+    CHK(splitk > 1 ? chronos::launch_gemm_lg((int)cfg, 0, false, a, cur_stream()) : chronos::launch_gemm_ring((int)cfg, mode == chronos::kPPGlu, a, cur_stream()),
+        "gemm_ring: launch");
+    if (splitk > 1) chronos::launch_gemm_slices_rows(ws.data_ptr<float>(), bfm(y), yf.data_ptr<float>(), b, (int)M, (int)N, (int)n0, (int)nf, (int)splitk, cur_stream());
+    return {y, yf};
+}
+
+// One row's product with an activation (modes of gemm_few), K % 512 == 0
+Tensor gemv_act(const Tensor& x, const Tensor& w, int64_t mode, double limit, double slope, double shift) {
+    chk_bf16(x, "x");
+    chk_bf16(w, "w");
+    CHK(x.dim() == 2 && x.size(0) == 1 && w.dim() == 2 && w.size(1) == x.size(1), "gemv_act: x [1, K], w [N, K]");
+    CHK(mode >= chronos::kPPGlu && mode <= chronos::kPPGelu, "gemv_act: mode");
+    const int64_t K = x.size(1), N = w.size(0);
+    CHK(K >= 512 && K % 512 == 0 && N >= 16 && N % 16 == 0 && N < (1LL << 31) && K < (1LL << 31), "gemv_act: K % 512 == 0, N % 16 == 0");
+    CHK(((reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr())) & 15) == 0, "gemv_act: alignment");
+    c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+    Tensor y = at::empty({1, mode == chronos::kPPGlu ? N / 2 : N}, x.options());
+    chronos::launch_gemv_act(bf(x), (int)K, bf(w), (int)N, bfm(y), (int)mode, (float)limit, (float)slope, (float)shift, cur_stream());
+    return y;
+}
+
 Tensor gemm_split(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk) {
     CHK(splitk > 1, "gemm_split: splitk");
     const Tensor ws = gemm_slices(x, w, cfg, splitk, false);
@@ -1008,6 +1080,8 @@ TORCH_LIBRARY(chronos, m) {
     m.def("gemm(Tensor x, Tensor w, bool swiglu, int stages=3) -> Tensor");
     m.def("gemm_act(Tensor x, Tensor w, int mode, float limit, float slope, float shift) -> Tensor");
     m.def("gemm_few(Tensor x, Tensor w, int cfg, int mode, int n0, int nf, Tensor? bias, float limit, float slope, float shift) -> (Tensor, Tensor)");
+    m.def("gemm_ring(Tensor x, Tensor w, int cfg, int splitk, int mode, int n0, int nf, Tensor? bias, float limit, float slope, float shift) -> (Tensor, Tensor)");
+    m.def("gemv_act(Tensor x, Tensor w, int mode, float limit, float slope, float shift) -> Tensor");
     m.def("gemm_split(Tensor x, Tensor w, int cfg, int splitk) -> Tensor");
     m.def("gemm_slices(Tensor x, Tensor w, int cfg, int splitk, bool skinny) -> Tensor");
     m.def("gemm_f32(Tensor x, Tensor w, int cfg, int splitk, bool skinny) -> Tensor");
@@ -1058,6 +1132,8 @@ TORCH_LIBRARY_IMPL(chronos, CUDA, m) {
     m.impl("gemm", &gemm);
     m.impl("gemm_act", &gemm_act);
     m.impl("gemm_few", &gemm_few);
+    m.impl("gemm_ring", &gemm_ring);
+    m.impl("gemv_act", &gemv_act);
     m.impl("gemm_split", &gemm_split);
     m.impl("gemm_slices", &gemm_slices);
     m.impl("gemm_f32", &gemm_f32);

@@ -28,6 +28,7 @@
 //     rows and W rows in its L2.  Correctness never depends on placement.
 //
 // What bounds the large-M configs against hipBLASLt (ablations, PMC, microbenchmarks): profiles/r4_studies.md.
+#include "chronos_act.h"
 #include "chronos_hip.h"
 #include "chronos_gemm.h"
 #include "chronos_slab.h"
@@ -112,7 +113,10 @@ __device__ __forceinline__ int lg_swz64(int row) { return (4 - ((row >> 2) & 3))
 // gain at every one (8 rows, us, in turn over 1.2 GB, 300 MB, 150 MB of weights: 2048 x 1024 5.8 -> 5.6, 5.6 -> 5.0, 5.7 -> 5.1; 8192 x 2048 10.0 -> 9.5, 10.2 -> 8.5, 11.3 ->
 // 9.8; 32768 x 4096 59.6 -> 51.2, 64.3 -> 47.1, 65.1 -> 47.0).  Of 44 decode steps of hybrid decoders (2 - 64 rows, widths 1024 - 4096) the mark makes all up to 7 % faster or level but for
 // 6 to 16 rows of width 2048, up to 3 % slower (12 rows 280 -> 290): four such layers and the head together just about fill the memory-side cache.
-template <int WN, int XM, int RB, int ST, int MODE, bool NORMP, int NWX, int ABL = 0, int VAR = 0, bool F8 = false, bool ONCE = false>
+//
+// MORE: the hybrid decoders' activations and, behind the product's columns, float32 ones of a few rows (launch_gemm_ring); instances of their own: jumping over that
+// code cost the others' epilogues 0.9 us of cold instruction fetches.
+template <int WN, int XM, int RB, int ST, int MODE, bool NORMP, int NWX, int ABL = 0, int VAR = 0, bool F8 = false, bool ONCE = false, bool MORE = false>
 __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
     constexpr bool STG = VAR == 1, MAN = VAR == 2;
     // VAR 3 (M32): the slab schedule on v_mfma_f32_32x32x16_bf16 — 32 x 32 blocks, half the MFMA issues per k-step
@@ -230,7 +234,8 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
     // 26.7; 128256 x 4096, 64 rows 191 / 177, 32 rows 186 / 184; 6144 x 4096 in two slices, 32 rows 13.1 / 12.0; level at 4096 x 14336 in four slices.
     // From K = 4096 on: level at 2048 (64 rows of 8192: 13.8 / 13.9), at 1024 slower (a decode step of one row, its weights in the memory-side cache: 156 / 161).  With more x tiles neighbours share their W rows and lose them from the L2 (1024 rows of 6144 x 4096: 52.1 / 54.1).
     constexpr bool TURN = !SLAB && !F8 && (ONCE || XM > 128);
-    const int turn0 = TURN && a.turn ? ((int)(blockIdx.x >> 3) + 8 * (int)(blockIdx.x & 7)) % NS : 0;
+    const int place = (int)(blockIdx.x >> 3) + 8 * (int)(blockIdx.x & 7);
+    const int turn0 = TURN && a.turn ? place - (int)((uint32_t)place * (uint32_t)a.turn >> 22) * NS : 0;   // place % NS (lg_turn)
     auto issue = [&](int j) {
         unsigned char* st = smem + (j % ST) * STAGE;
         int stage = min(j, NS1);
@@ -1086,6 +1091,7 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
         }
     }
 
+    static_assert(!MORE || (!SLAB && !F8 && !NORMP && ABL == 0), "more in the epilogue: ring tiles, bf16, no folded norm");
     // ---- epilogue: lane holds D[n = wrow0[s] + 4*(lane>>4) + i][m = xrow0 + 16*u + (lane&15)]
     const float* inv = reinterpret_cast<const float*>(smem + EXTRA + 16);
     if constexpr (M32) {
@@ -1173,6 +1179,13 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
                         cu = *reinterpret_cast<const f32x4*>(a.wsc + a.F + f);
                     }
                     u16x4 o;
+                    if (MORE && a.act == kPPGlu) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const float gv = fminf(acc[s][u][i], a.limit), uv = fminf(fmaxf(acc[s + NT / 2][u][i], -a.limit), a.limit);
+                            o[i] = f2bf(gv * hy::sigmoid_act<uint16_t>(a.slope * gv) * (uv + a.shift));
+                        }
+                    } else
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const float gv = bf2f(f2bf(acc[s][u][i] * sc * cg[i]));
@@ -1211,23 +1224,42 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
                     f32x4 cw = {1.f, 1.f, 1.f, 1.f};
                     if constexpr (F8)
                         if (n < a.N) cw = *reinterpret_cast<const f32x4*>(a.wsc + n);
+                    int ld = a.N;
+                    if constexpr (MORE) {
+                        if (a.yf != nullptr) {
+                            ld = a.n0;
+                            if (n >= a.n0) {   // (n0 % 4 == 0)
+#pragma unroll
+                                for (int i = 0; i < 4; ++i)
+                                    if (n + i < a.n0 + a.nf)
+                                        a.yf[(int64_t)m * a.nf + n + i - a.n0] = acc[s][u][i] + (a.bias != nullptr ? a.bias[n + i - a.n0] : 0.f);
+                                continue;
+                            }
+                        } else if (a.act != 0) {
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) acc[s][u][i] = hy::act_apply(acc[s][u][i], a.act == kPPRelu2 ? hy::kActRelu2 : hy::kActGelu);
+                        }
+                    }
                     u16x4 o;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) o[i] = f2bf(acc[s][u][i] * sc * cw[i]);
-                    if (n < a.N) *reinterpret_cast<u16x4*>(a.y + (int64_t)m * a.N + n) = o;  // N % 4 == 0
+                    if (n < a.N) *reinterpret_cast<u16x4*>(a.y + (int64_t)m * ld + n) = o;  // N % 4 == 0
                 }
             }
         }
     }
 }
 
-template <int WN, int XM, int RB, int ST, int MODE, bool NORMP, int NWX, int ABL = 0, int VAR = 0, bool F8 = false>
+// 2^22 / NS rounded up: place * this >> 22 is place / NS for places up to 1079 (8192 workgroups) and NS from 2 to 2047; 0: no turning
+int lg_turn(int groups, int NS) { return groups <= 8 * 1024 && NS >= 2 && NS < 2048 ? ((1 << 22) + NS - 1) / NS : 0; }
+
+template <int WN, int XM, int RB, int ST, int MODE, bool NORMP, int NWX, int ABL = 0, int VAR = 0, bool F8 = false, bool MORE = false>
 void lg_launch(const PPArgs& a, hipStream_t st) {
     const int lds = ST * (WN + XM) * RB + 16 + XM * 4 + (F8 && ST == 2 ? (WN + XM) * 4 : 0);
     const int mt = (a.M + XM - 1) / XM;
     const int ntl = MODE == kSwiglu ? a.F / (WN / 2) : (a.N + WN - 1) / WN;
     PPArgs b = a;
-    b.turn = a.turn && mt == 1 && a.K >= 4096;
+    b.turn = a.turn && mt == 1 && a.K >= 4096 ? lg_turn(ntl * a.splitk, a.kts * (128 / RB)) : 0;
     auto go = [&](auto kern, bool& attr) {
         if (!attr) {
             hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -1238,12 +1270,12 @@ void lg_launch(const PPArgs& a, hipStream_t st) {
     if constexpr (XM <= 128 && ST > 2 && !F8 && ABL == 0 && WN / (1024 / RB) % (2 * NWX) == 0 && XM / (1024 / RB) % (2 * NWX) == 0) {
         if (mt == 1) {
             static bool attr = false;
-            go(gemm_lg_kernel<WN, XM, RB, ST, MODE, NORMP, NWX, ABL, VAR, F8, true>, attr);
+            go(gemm_lg_kernel<WN, XM, RB, ST, MODE, NORMP, NWX, ABL, VAR, F8, true, MORE>, attr);
             return;
         }
     }
     static bool attr = false;
-    go(gemm_lg_kernel<WN, XM, RB, ST, MODE, NORMP, NWX, ABL, VAR, F8>, attr);
+    go(gemm_lg_kernel<WN, XM, RB, ST, MODE, NORMP, NWX, ABL, VAR, F8, false, MORE>, attr);
 }
 
 // tile configs (ids continue gemm_pp's): {WN = W rows, XM = x rows, RB = LDS row bytes (BK = RB/2), ST = ring depth,
@@ -1420,6 +1452,27 @@ int gemm_lg_f8_wn(int cfg) {
 bool launch_gemm_lg_f8(int cfg, bool swiglu, const PPArgs& a, hipStream_t st) {
     if (a.M == 0) return true;
     return swiglu ? lg_f8_mode<kSwiglu>(cfg, a, st) : lg_f8_mode<kPlain>(cfg, a, st);
+}
+
+bool launch_gemm_ring(int cfg, bool glu, const PPArgs& a, hipStream_t st) {
+    if (a.M == 0) return true;
+    switch (cfg) {
+#define LG_MORE(ID, WN_, XM_, ST_, NWX_)                                                                        \
+    case ID:                                                                                                    \
+        if (glu) lg_launch<WN_, XM_, 128, ST_, kSwiglu, false, NWX_, 0, 0, false, true>(a, st);                 \
+        else lg_launch<WN_, XM_, 128, ST_, kPlain, false, NWX_, 0, 0, false, true>(a, st);                      \
+        return true;
+        LG_MORE(19, 128, 128, 4, 4)
+        LG_MORE(32, 64, 128, 4, 2)
+        LG_MORE(38, 128, 64, 6, 2)
+        LG_MORE(39, 64, 64, 6, 2)
+        LG_MORE(72, 64, 32, 8, 2)
+        LG_MORE(74, 64, 32, 4, 2)
+        LG_MORE(75, 128, 32, 4, 2)
+        LG_MORE(79, 64, 32, 12, 2)
+#undef LG_MORE
+        default: return false;
+    }
 }
 
 bool launch_gemm_lg(int cfg, int mode, bool normp, const PPArgs& a, hipStream_t st) {

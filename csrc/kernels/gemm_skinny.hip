@@ -350,8 +350,28 @@ __global__ void __launch_bounds__(256) skinny_sum_kernel(const float* __restrict
     }
 }
 
+// ... and of columns n0 .. n0 + nf, plus bias, to yf [M, nf] as float; y [M, n0], n0 and N multiples of 4
+__global__ void __launch_bounds__(256) skinny_sum_rows_kernel(const float* __restrict__ ws, uint16_t* __restrict__ y, float* __restrict__ yf,
+                                                              const float* __restrict__ bias, int M, int N, int n0, int nf, int S) {
+    const int c = ((int)blockIdx.x * 256 + threadIdx.x) * 4, m = blockIdx.y;
+    if (c >= N) return;
+    const float* p = ws + (int64_t)m * N + c;
+    f32x4 v = *reinterpret_cast<const f32x4*>(p);
+    for (int s = 1; s < S; ++s) v += *reinterpret_cast<const f32x4*>(p + (int64_t)s * M * N);
+    if (c < n0) {
+        *reinterpret_cast<u16x4*>(y + (int64_t)m * n0 + c) = u16x4{f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (c + i < n0 + nf) yf[(int64_t)m * nf + c + i - n0] = v[i] + (bias != nullptr ? bias[c + i - n0] : 0.f);
+}
+
 }  // namespace
 
+void launch_gemm_slices_rows(const float* ws, uint16_t* y, float* yf, const float* bias, int M, int N, int n0, int nf, int S, hipStream_t st) {
+    skinny_sum_rows_kernel<<<dim3((N / 4 + 255) / 256, M), 256, 0, st>>>(ws, y, yf, bias, M, N, n0, nf, S);
+}
 void launch_gemm_slices(const float* ws, uint16_t* y, int64_t n, int S, hipStream_t st) {   // n % 4 == 0
     skinny_sum_kernel<false><<<(unsigned)((n / 4 + 255) / 256), 256, 0, st>>>(ws, y, n, S);
 }

@@ -14,6 +14,8 @@
 //     which split K, meet in LDS.
 // One 256-thread workgroup owns R output rows.  Fused SwiGLU epilogue for the gate/up projection (w = [gate; up]):
 // the workgroup streams R gate rows and the matching R up rows and writes silu(g) * u directly.
+#include "chronos_act.h"
+#include "chronos_gemm.h"
 #include "chronos_hip.h"
 #include "chronos_gemv.h"
 
@@ -91,7 +93,10 @@ enum : int { kPlain = 0, kSwiglu = 1, kRope = 2, kRope8 = 3, kResid = 4 };
 // piece is then 16 elements, a chunk 1024 elements, and x comes as two 16-B pieces per chunk; every fused epilogue is
 // the same, the row sums scaled by their row's weight scale first.  Half the weight bytes of the bf16 kernel, no
 // activation quantisation launch (the W8A8 qgemv path needs one per projection).
-template <int M, int R, int MODE, bool NORMP, bool WQ = false>
+//
+// ACT: the hybrid decoders' activations on the sums themselves (nrm.act: kPPGlu in place of SwiGLU, kPPRelu2, kPPGelu), a launch of 4.6 us less in a step
+// of one row; instances of their own, the others have no register to spare.
+template <int M, int R, int MODE, bool NORMP, bool WQ = false, bool ACT = false>
 __global__ void __launch_bounds__(256) gemv_kernel(const uint16_t* __restrict__ x, int mrows, int K,
                                                    const uint16_t* __restrict__ W, uint16_t* __restrict__ y,
                                                    int nout, int half, GemvNorm nrm, GemvRope rp,
@@ -302,13 +307,18 @@ __global__ void __launch_bounds__(256) gemv_kernel(const uint16_t* __restrict__ 
             for (int t = threadIdx.x; t < R * M; t += 256) {
                 const int r = t / M, m = t % M;
                 if (m >= mrows) continue;
-                const float gv = totw(r * M + m);
-                if constexpr (SWIGLU) {
+                float gv = totw(r * M + m);
+                if constexpr (SWIGLU && ACT) {
+                    gv = fminf(gv, nrm.limit);
+                    const float u = fminf(fmaxf(totw((R + r) * M + m), -nrm.limit), nrm.limit);
+                    y[(int64_t)m * nout + n0 + r] = f2bf(gv * hy::sigmoid_act<uint16_t>(nrm.slope * gv) * (u + nrm.shift));
+                } else if constexpr (SWIGLU) {
                     const float u = totw((R + r) * M + m);
                     const float gb = bf2f(f2bf(gv)), ub = bf2f(f2bf(u));  // the unfused path rounds the GEMM outputs
                     const float sg = bf2f(f2bf(gb / (1.f + __expf(-gb))));
                     y[(int64_t)m * nout + n0 + r] = f2bf(sg * ub);
                 } else {
+                    if constexpr (ACT) gv = hy::act_apply(gv, nrm.act == kPPRelu2 ? hy::kActRelu2 : hy::kActGelu);
                     y[(int64_t)m * nout + n0 + r] = f2bf(gv);
                 }
             }
@@ -347,6 +357,15 @@ static int rows_knob(const char* name, int dflt) {
     return (v == 1 || v == 2 || v == 4 || v == 8 || v == 16) ? v : dflt;
 }
 
+// the decode gate: its state and the kernel's gn
+static int gate_rows(const int32_t*& gst) {
+    gst = g_gate_n > 0 && g_gate_n <= kGateMax ? g_gate_state : nullptr;
+    // early gate by default: a gated single-stream step (after the verdict closed or the row parked for a jump)
+    // costs 0.28 ms instead of 2.25 (the late check let every workgroup issue its first ring of weight loads, which
+    // at K = 4096 is the whole row), and the live step is no slower (3.60 vs 3.72 ms/token; profiles/r2_studies.md)
+    return gst ? (knob("gemv_early_gate", 1) ? -g_gate_n : g_gate_n) : 0;
+}
+
 template <int M, bool WQ = false>
 static void launch_m(const uint16_t* x, int mrows, int K, const uint16_t* W, int N, uint16_t* y, int mode,
                      const GemvNorm* nrm, const GemvRope* rp, hipStream_t st, const float* wscale = nullptr) {
@@ -360,11 +379,8 @@ static void launch_m(const uint16_t* x, int mrows, int K, const uint16_t* W, int
     na.wscale = wscale;
     const GemvRope ra = rp ? *rp : rz;
     const bool np = nrm && nrm->part;  // consumer of a kResid producer
-    const int32_t* gst = g_gate_n > 0 && g_gate_n <= kGateMax ? g_gate_state : nullptr;
-    // early gate by default: a gated single-stream step (after the verdict closed or the row parked for a jump)
-    // costs 0.28 ms instead of 2.25 (the late check let every workgroup issue its first ring of weight loads, which
-    // at K = 4096 is the whole row), and the live step is no slower (3.60 vs 3.72 ms/token; profiles/r2_studies.md)
-    const int gn = gst ? (knob("gemv_early_gate", 1) ? -g_gate_n : g_gate_n) : 0;
+    const int32_t* gst = nullptr;
+    const int gn = gate_rows(gst);
     // Persistent grid: the workgroups that fit on the device at once (occupancy x CUs), each looping over row groups
     // with the next group's weight ring prefetched.  A grid of 512 for every kernel (two per CU, what the 2-wave
     // gate_up fits) measured 2.88 ms/token in the single-stream decode step against 3.06 with one workgroup per group
@@ -475,6 +491,25 @@ void launch_gemv_ex(const uint16_t* x, int M, int K, const uint16_t* W, int N, u
     }
     if (M == 1) launch_m<1>(x, M, K, W, N, y, mode, nrm, rope, st);
     else launch_m<2>(x, M, K, W, N, y, mode, nrm, rope, st);
+}
+
+// One row with an activation (mode kPPGlu: N = 2 F rows, gate then up).
+void launch_gemv_act(const uint16_t* x, int K, const uint16_t* W, int N, uint16_t* y, int mode, float limit, float slope, float shift, hipStream_t st) {
+    GemvNorm na{};
+    na.act = mode;
+    na.limit = limit;
+    na.slope = slope;
+    na.shift = shift;
+    const bool glu = mode == kPPGlu;
+    const int32_t* gst = nullptr;
+    const int gn = gate_rows(gst);
+    const int groups = glu ? N / 2 / rows_swiglu<1>() : N / rows_plain<1>();
+    auto go = [&](auto kern) {
+        const int fit = resident_workgroups(kern, 256);
+        hipLaunchKernelGGL(kern, dim3(fit < groups ? fit : groups), dim3(256), 0, st, x, 1, K, W, y, glu ? N / 2 : N, glu ? N / 2 : 0, na, GemvRope{}, gst, gn, groups);
+    };
+    if (glu) go(gemv_kernel<1, rows_swiglu<1>(), kSwiglu, false, false, true>);
+    else go(gemv_kernel<1, rows_plain<1>(), kPlain, false, false, true>);
 }
 
 int gemv_resid_parts(int M, int N, bool wq) {

@@ -324,8 +324,9 @@ def mid_rows_plan(m: int, n: int, k: int) -> Optional[tuple[int, int]]:
     return out
 
 
-# Configs of gemm_slices (csrc/kernels/bindings.cpp)
+# Configs of gemm_slices and of gemm_ring (csrc/kernels/bindings.cpp)
 _SLICED = (19, 32, 33, 36, 38, 39, 72, 73, 74, 75, 78, 79, *_UNEVEN)
+_RING = (19, 32, 38, 39, 72, 74, 75, 79)
 
 
 def product_f32(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
@@ -525,15 +526,21 @@ def _many_act_pays(m: int, n: int, k: int, glu: bool) -> bool:
 
 def product_act(x: torch.Tensor, w: torch.Tensor, mode: int, limit: float = 0.0, slope: float = 0.0, shift: float = 0.0) -> Optional[torch.Tensor]:
     """x @ w.T with an activation in the epilogue (mode as in torch.ops.chronos.gemm_act: 3 a gated unit of w = [gate; up], 4 squared ReLU, 5
-    GELU), or None where that does not pay: with up to 64 rows by _FEW_MORE, from 128 on where the best product (many_rows_plan's or, below it,
-    as if it were) and a pass of its own are faster by their models.  On the grid of _MANY_88, against the faster of the library and this product with
+    GELU), or None where that does not pay: with up to 64 rows by _ring_more and _FEW_MORE, below 128 in the GEMV's or the ring tiles'
+    epilogue where linear() takes those unsplit, from 128 on where the best product (many_rows_plan's or, below it, as if it were) and a pass of its
+    own are faster by their models.  On the grid of _MANY_88, against the faster of the library and this product with
     its pass: gated units 1.12 times as fast (188 shapes; the worst 0.92), the others 1.15 (196; 0.90).  Both worst are long rounds that leave a
     third of the CUs idle (_third_idle); they stay, because the pass reads a rounded product: a step with it is further from float64 (0.0076 for 0.0067)."""
     m, (n, k) = x.numel() // max(1, x.shape[-1]), w.shape
-    if 64 < m < MANY_MIN or PP_MODE != "auto" or x.dim() != 2 or not _plain_rows(x, w) or _registered(m, n, k):
+    if PP_MODE != "auto" or x.dim() != 2 or not _plain_rows(x, w) or _registered(m, n, k):
         return None
-    if m <= 64:
+    if m < MANY_MIN:
         cfg = _few_more(m, n, k, 2 if mode == 3 else 1)
+        if m == 1 and not cfg and _linear_plan(1, n, k) is None and gemv_ok(1, n, k):
+            return _k().gemv_act(x, w, mode, limit, slope, shift)
+        plan = _linear_plan(m, n, k) if m > 64 or _ring_more(m, n, k) else None
+        if plan is not None and plan[0] in _RING and plan[1] == 1 and (mode != 3 or n % _PP_BN[plan[0]] == 0):
+            return _k().gemm_ring(x, w, plan[0], 1, mode, 0, 0, None, limit, slope, shift)[0]
         return _k().gemm_few(x, w, cfg, mode, 0, 0, None, limit, slope, shift)[0] if cfg else None
     glu = mode == 3
     rows = -(-m // 128) * 128
@@ -568,14 +575,30 @@ def _few_more(m: int, n: int, k: int, kind: int) -> int:
     return 0
 
 
+def _ring_more(m: int, n: int, k: int) -> bool:
+    """Whether up to 64 rows with more to do behind the product go to the ring tiles before gemm_few, whose workgroups of 32 weight rows are
+    more than a round of 256 from 8192 rows on, and don't take K round from places of their own over large weights.  Two launches, gemm_few -> ring, us:
+    gated units of 11264 x 2048, 4 rows 13.3, 15.0 -> 11.4, 16 rows 13.9, 16.8 -> 11.7, 64 rows 17.3, 24.0 -> 14.8; of 16384 x 1024, 16 rows
+    10.6, 10.2 -> 8.4; GELU after 14336 x 1024, 32 rows 10.8, 12.4 -> 8.7; 12304 x 4096 with float32 rows, 4 rows 25.9, 26.3 -> 18.0, 16 rows
+    25.2, 30.0 -> 18.8.  On this side: 8192 x 2048 with GELU 16 rows 10.6, ring 10.9, 64 rows 13.8, ring 14.5."""
+    return m > 1 and n * k > 8_000_000 and (n > 8192 or n * k > 24_000_000)
+
+
 def product_rows(x: torch.Tensor, w: torch.Tensor, n0: int, nf: int, bias: Optional[torch.Tensor]):
     """(x @ w[:n0].T, float32 x @ w[n0 : n0 + nf].T + bias) in one launch, or None where two are faster."""
-    if x.dim() != 2 or not 0 < x.shape[0] <= 64 or not _plain_rows(x, w) or _registered(x.shape[0], n0, w.shape[1]):
+    if x.dim() != 2 or not 0 < x.shape[0] <= 512 or not _plain_rows(x, w) or _registered(x.shape[0], n0, w.shape[1]):
         return None
-    cfg = _few_more(x.shape[0], *w.shape, 0)
-    if not cfg:
-        return None
-    return _k().gemm_few(x, w, cfg, 0, n0, nf, bias, 0.0, 0.0, 0.0)
+    m, (n, k) = x.shape[0], w.shape
+    # the ring tiles also wherever gemm_few has no config.  Two launches -> one, us: 12304 x 4096, 64 rows 32.4 -> 25.3, 200 rows 49.1 -> 39.9;
+    # 6160 x 2048, 100 rows 18.6 -> 12.7, 400 rows 26.5 -> 20.3; 3080 x 1024, 400 rows 13.0 -> 10.2
+    cfg = _few_more(m, n, k, 0)
+    plan = _linear_plan(m, n0, k) if not cfg or _ring_more(m, n, k) else None
+    if plan is not None and plan[0] in _RING:
+        # the rows behind are one tile more, which must not be a round more
+        bn, tiles = _PP_BN[plan[0]], -(-m // _PP_BM[plan[0]]) * plan[1]
+        if -(-(-(-(n0 + nf) // bn) * tiles) // 256) <= -(-(-(-n0 // bn) * tiles) // 256):
+            return _k().gemm_ring(x, w, plan[0], plan[1], 0, n0, nf, bias, 0.0, 0.0, 0.0)
+    return _k().gemm_few(x, w, cfg, 0, n0, nf, bias, 0.0, 0.0, 0.0) if cfg else None
 
 
 _Tensor, _WEIGHTS, _BF16 = torch.Tensor, (torch.Tensor, torch.nn.Parameter), torch.bfloat16
