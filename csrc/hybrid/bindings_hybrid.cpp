@@ -29,6 +29,7 @@ void launch_hy_mlstm_scan(const void*, int, const float*, const int32_t*, const 
                           float*, float*, float*, int, int, int, int, int, float, int, int, bool, hipStream_t);
 int hy_chunk_segments(int, int, int, int, int, int);
 int64_t hy_delta_tiles_bytes(const void*, int, int, int, int, int, int, int, int, int, int);
+int64_t hy_gla_tiles_bytes(const void*, const void*, int, int, int, int, int, int, int, int, int, int);
 bool hy_chunk_scan_pays(int, int, int, int, int, int, int);
 bool hy_gla_scan_pays(int, int, int);
 int64_t hy_chunk_segment_floats(int, int, int, int, int);
@@ -98,7 +99,7 @@ void launch_hy_delta_prep(const void*, int, const float*, const float*, float*, 
                           float, bool, hipStream_t);
 bool launch_hy_linear_scan(const void*, int, int, int, int, const float*, const float*, float, const float*, bool, bool,
                            const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*, int, int, int, int,
-                           int, int, const float*, int, int, float*, bool, hipStream_t);
+                           int, int, const float*, int, int, float*, void*, bool, hipStream_t);
 void launch_hy_moe_route_topk(const void*, const void*, const float*, float*, int32_t*, float*, int, int, int, int, bool,
                               hipStream_t);
 void launch_hy_moe_glu_grouped(const uint16_t*, const int32_t*, const float*, const uint16_t*, const uint16_t*, uint16_t*,
@@ -961,12 +962,18 @@ Tensor hy_linear_scan(const Tensor& proj, int64_t q_off, int64_t k_off, int64_t 
         const int64_t bytes = chronos::hy_delta_tiles_bytes(proj.data_ptr(), (int)C, (int)q_off, (int)k_off, (int)v_off, (int)T, (int)B, (int)H, (int)D, (int)Dv, mq);
         if (bytes > 0) seg = at::empty({bytes / 4}, S.options());
     }
+    Tensor tiles;
+    if (chd && !beta && !f32(proj)) {
+        const int64_t bytes = chronos::hy_gla_tiles_bytes(proj.data_ptr(), decay.data_ptr(), (int)C, (int)q_off, (int)k_off, (int)v_off, (int)T, (int)B, (int)H, (int)D, (int)Dv, mq);
+        if (bytes > 0) tiles = at::empty({bytes / 4}, S.options());
+    }
     const bool ok = chronos::launch_hy_linear_scan(
         proj.data_ptr(), (int)C, (int)q_off, (int)k_off, (int)v_off, qscale ? qscale->data_ptr<float>() : nullptr,
         kscale ? kscale->data_ptr<float>() : nullptr, (float)q_mul, decay.data_ptr<float>(), chd, fixed,
         beta ? beta->data_ptr<float>() : nullptr, q_start.data_ptr<int32_t>(), pos0.data_ptr<int32_t>(),
         slots.data_ptr<int32_t>(), S.data_ptr<float>(), o.data_ptr<float>(), (int)T, (int)B, (int)HK, (int)H, (int)D, (int)Dv,
-        vscale ? vscale->data_ptr<float>() : nullptr, mq, segs, seg.defined() ? seg.data_ptr<float>() : nullptr, f32(proj), stream());
+        vscale ? vscale->data_ptr<float>() : nullptr, mq, segs, seg.defined() ? seg.data_ptr<float>() : nullptr,
+        tiles.defined() ? tiles.data_ptr() : nullptr, f32(proj), stream());
     TORCH_CHECK(ok, "chronos hybrid op: linear_scan keeps a state column in registers, D <= 256 (got ", D, ")");
     return o;
 }

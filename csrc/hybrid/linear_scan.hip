@@ -436,7 +436,7 @@ void launch_hy_chunk_scan(const uint16_t*, int, int, int, int, const float*, con
 
 bool hy_gla_scan_ok(const void*, const void*, int, int, int, int, int, int, int, int, int);
 void launch_hy_gla_scan(const uint16_t*, int, int, int, int, const float*, const float*, float, const float*, const int32_t*,
-                        const int32_t*, const int32_t*, float*, float*, int, int, int, int, int, const float*, int, float*, hipStream_t);
+                        const int32_t*, const int32_t*, float*, float*, int, int, int, int, int, int, const float*, int, float*, void*, hipStream_t);
 
 bool hy_state_step_ok(const void*, const void*, const void*, int, int, int, int, int);
 void launch_hy_state_step(const uint16_t*, int, int, int, int, const float*, const float*, float, const float*, bool, int,
@@ -529,12 +529,13 @@ static bool linear_scan_d(bool pipe, const T* proj, int ldp, int q_off, int k_of
 // chd: decay holds one number per state row ([T, H, D]) instead of one per head ([T, H]).
 // fixed (not with chd): decay holds one number per head for all tokens ([H]).
 // longest: the most tokens that any sequence brings, as far as the caller knows (it only picks the kernel).
-// segs, seg: hy_chunk_segments and its scratch; with beta 1 and hy_delta_tiles_bytes of scratch, or nullptr.
+// segs, seg: hy_chunk_segments and its scratch; with beta 1 and hy_delta_tiles_bytes of scratch, or nullptr.  tiles: hy_gla_tiles_bytes of scratch, or
+// nullptr.
 // Returns false when D has no instantiation (D > 256).
 bool launch_hy_linear_scan(const void* proj, int ldp, int q_off, int k_off, int v_off, const float* qscale,
                            const float* kscale, float q_mul, const float* decay, bool chd, bool fixed, const float* beta,
                            const int32_t* q_start, const int32_t* pos0, const int32_t* slots, float* S, float* o, int T,
-                           int B, int HK, int H, int D, int Dv, const float* vscale, int longest, int segs, float* seg, bool f32, hipStream_t s) {
+                           int B, int HK, int H, int D, int Dv, const float* vscale, int longest, int segs, float* seg, void* tiles, bool f32, hipStream_t s) {
     if (B == 0) return true;
     const bool pipe = T > B;   // some sequence brings more than one token
     const bool delta = beta != nullptr;
@@ -545,7 +546,7 @@ bool launch_hy_linear_scan(const void* proj, int ldp, int q_off, int k_off, int 
     }
     if (chd && !delta && !f32 && hy_gla_scan_ok(proj, decay, ldp, q_off, k_off, v_off, T, B, D, Dv, longest)) {
         launch_hy_gla_scan((const uint16_t*)proj, ldp, q_off, k_off, v_off, qscale, kscale, q_mul, decay, q_start, pos0, slots, S, o,
-                           B, HK, H, D, Dv, vscale, segs, seg, s);
+                           T, B, HK, H, D, Dv, vscale, segs, seg, tiles, s);
         return true;
     }
     if (!chd && !f32 && hy_chunk_scan_ok(proj, ldp, q_off, k_off, v_off, T, B, H, D, Dv, longest, delta ? hy::kScanDelta : hy::kScanPlain)) {
