@@ -493,8 +493,7 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
             pt[p * 64 + lane] = v;
             if constexpr (MLSTM) {
                 float sum = (v[0] + v[1]) + (v[2] + v[3]);
-                sum += __shfl_xor(sum, 16, 64);
-                sum += __shfl_xor(sum, 32, 64);
+                sum = rows_sum(sum);
                 if (g == 0) psum[p * 16 + ln] = sum;
             }
         }
@@ -735,8 +734,7 @@ __global__ void __launch_bounds__(64 * kCW, 1) __attribute__((amdgpu_waves_per_e
             for (int j = 0; j < (D + 63) / 64; ++j) nl[j] = a.n0[(int64_t)group * D + min(lane + 64 * j, D - 1)];
         }
         auto over_rows = [](float x) {   // lanes of the same column hold a quarter of the rows each
-            x += __shfl_xor(x, 16, 64);
-            return x + __shfl_xor(x, 32, 64);
+            return rows_sum(x);
         };
         for (int64_t t = s0; t < te; ++t) {
             float d, w, rr = a.q_mul;

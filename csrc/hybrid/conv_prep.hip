@@ -103,7 +103,7 @@ __global__ void __launch_bounds__(256) conv_prep_vec_kernel(const T* __restrict_
             y[e] = j < a.H ? v : rnd<T>(v);
             ss += y[e] * y[e];
         }
-        for (int m = 1; m < lph; m <<= 1) ss += __shfl_xor(ss, m, 64);
+        ss = group_sum(ss, lph);
         const float inv = 1.f / sqrtf(ss / (float)a.D + a.eps);
         const int p = a.pos[t];
         if (on && j < a.H) {

@@ -468,8 +468,7 @@ __global__ void __launch_bounds__(256, 1) gla_scan_kernel(const GlaScan a) {
                         acc[r & 1] += bf2f(qs[row]) * S[i][r];
                     }
                 float x = acc[0] + acc[1];
-                x += __shfl_xor(x, 16, 64);
-                x += __shfl_xor(x, 32, 64);
+                x = rows_sum(x);
                 if (!STATE && g == 0) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x * ws[kGC + t]), ord, ocol + t * orow, 0, 0);
             }
             continue;
@@ -715,8 +714,7 @@ __global__ void __launch_bounds__(256 * GlaTile<D>::RW) __attribute__((amdgpu_wa
                         acc[r & 1] += bf2f(q[t * ld + row]) * S[i][r];
                     }
                 float x = acc[0] + acc[1];
-                x += __shfl_xor(x, 16, 64);
-                x += __shfl_xor(x, 32, 64);
+                x = rows_sum(x);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) last[r] = t == 4 * g + r ? x : last[r];
             }

@@ -204,8 +204,7 @@ __global__ void __launch_bounds__(64 * NW) latent_attention_mfma_kernel(
                 S[kt][i] = sv;
                 mx = fmaxf(mx, sv);
             }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = rows_max(mx);
         const float mn = fmaxf(mrow, mx);
         const float corr = (mn == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(mrow - mn);
         const float mref = (mn == -INFINITY) ? 0.f : mn;   // (all masked: every exponent is -inf, every weight 0)
@@ -218,8 +217,7 @@ __global__ void __launch_bounds__(64 * NW) latent_attention_mfma_kernel(
                 S[kt][i] = p;
                 sum += p;
             }
-        sum += __shfl_xor(sum, 16, 64);
-        sum += __shfl_xor(sum, 32, 64);
+        sum = rows_sum(sum);
         lrow = lrow * corr + sum;
         mrow = mn;
         // ---- weighted sum of the value columns: k index of step u = [tile 2u keys 4g..4g+3 | tile 2u+1 keys 4g..4g+3]

@@ -146,8 +146,7 @@ __global__ void __launch_bounds__(64 * NW) latent_expanded_kernel(const LatentEx
             float mx = -INFINITY;
 #pragma unroll
             for (int kt = 0; kt < 4; ++kt) mx = fmaxf(fmaxf(mx, fmaxf(S[j][kt][0], S[j][kt][1])), fmaxf(S[j][kt][2], S[j][kt][3]));
-            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            mx = rows_max(mx);
             const float mn = fmaxf(mrow[j], mx * scale2);
             const float corr = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(mrow[j] - mn);
             const float mref = mn == -INFINITY ? 0.f : mn;   // (all masked: every weight is 0)
@@ -160,8 +159,7 @@ __global__ void __launch_bounds__(64 * NW) latent_expanded_kernel(const LatentEx
                     sum += p;
                     pf[j][kt >> 1][4 * (kt & 1) + i] = (__bf16)p;
                 }
-            sum += __shfl_xor(sum, 16, 64);
-            sum += __shfl_xor(sum, 32, 64);
+            sum = rows_sum(sum);
             lrow[j] = lrow[j] * corr + sum;
             mrow[j] = mn;
             if (__builtin_amdgcn_ballot_w64(corr != 1.f) != 0) {   // (rarely, once the maxima have settled)

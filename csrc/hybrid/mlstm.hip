@@ -390,8 +390,7 @@ __global__ void __launch_bounds__(256) mlstm_out_vec_kernel(const float* __restr
     float ss = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
-#pragma unroll
-    for (int k = 1; k < LPR; k <<= 1) ss += __shfl_xor(ss, k, 64);
+    ss = group_sum(ss, LPR);
     const float inv = 1.f / sqrtf(ss / (float)Dv + eps);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {

@@ -67,14 +67,7 @@ __device__ __forceinline__ void select_softmax(const float* zr, const float* __r
                 bv = c[j]; be = e; bs = s[j];
             }
         }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const float ov = __shfl_xor(bv, o, 64), os = __shfl_xor(bs, o, 64);
-            const int oe = __shfl_xor(be, o, 64);
-            if (ov > bv || (ov == bv && oe < be)) {
-                bv = ov; be = oe; bs = os;
-            }
-        }
+        lanes_best(bv, be, bs);
         if (lane == 0) {
             idx[k] = be;
             wt[k] = bs;
@@ -152,14 +145,8 @@ __device__ __forceinline__ void select_topk(const float* zr, int32_t* __restrict
                 bv = c[j]; be = e;
             }
         }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const float ov = __shfl_xor(bv, o, 64);
-            const int oe = __shfl_xor(be, o, 64);
-            if (ov > bv || (ov == bv && oe < be)) {
-                bv = ov; be = oe;
-            }
-        }
+        float none = 0.f;
+        lanes_best(bv, be, none);
         if (k == 0) first = bv;  // the largest logit: the softmax's reference point
         const float ex = expf(bv - first);
         sum += ex;
@@ -223,14 +210,8 @@ __device__ __forceinline__ void select_group(const float* zr, int32_t* __restric
                 bv = c[j]; be = e;
             }
         }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const float ov = __shfl_xor(bv, o, 64);
-            const int oe = __shfl_xor(be, o, 64);
-            if (ov > bv || (ov == bv && oe < be)) {
-                bv = ov; be = oe;
-            }
-        }
+        float none = 0.f;
+        lanes_best(bv, be, none);
         sum += bv;
         if (k == lane) {
             mine = bv;

@@ -80,9 +80,7 @@ __global__ void __launch_bounds__(HPW * mix_threads(D)) state_mix_kernel(const S
     }
     auto total = [&](f32x4 x) {   // the sum over all rows of this lane's columns, in every lane
 #pragma unroll
-        for (int o = CL; o < 64; o <<= 1)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) x[e] += __shfl_xor(x[e], o, 64);
+        for (int e = 0; e < 4; ++e) x[e] = across_sum<CL>(x[e]);
         if (rl == 0) part[sub][wv][cl] = x;
         __syncthreads();
         x = part[sub][0][cl];
@@ -205,8 +203,7 @@ __global__ void __launch_bounds__(HPW * mix_threads(D)) state_mix_kernel(const S
         const f32x4 o = total(x[0] + x[1]) * rd;
         // the head's norm and gate: a row's columns lie over CL lanes (dead ones hold 0)
         float ss = o[0] * o[0] + o[1] * o[1] + o[2] * o[2] + o[3] * o[3];
-#pragma unroll
-        for (int k = 1; k < CL; k <<= 1) ss += __shfl_xor(ss, k, 64);
+        ss = group_sum(ss, CL);
         const float inv = 1.f / sqrtf(ss / (float)a.Dv + a.eps);
         if (wv == 0 && rl == 0 && live) {
             u16x4 out;

@@ -53,9 +53,7 @@ __global__ void __launch_bounds__(D >= 128 ? 2 * D : 256) state_step_kernel(cons
         S[i] = live && !fresh ? __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(Sp + (int64_t)(RI * i) * a.Dv)) : f32x4{0.f, 0.f, 0.f, 0.f};
     auto total = [&](f32x4 x) {   // the sum over all rows of this lane's columns, in every lane
 #pragma unroll
-        for (int o = CL; o < 64; o <<= 1)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) x[e] += __shfl_xor(x[e], o, 64);
+        for (int e = 0; e < 4; ++e) x[e] = across_sum<CL>(x[e]);
         if (rl == 0) part[wv][cl] = x;
         __syncthreads();
         x = part[0][cl];

@@ -144,7 +144,7 @@ __global__ void __launch_bounds__(256) window_prep_vec_kernel(
                 ld8f(nw + c, wf);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
-                for (int k = 1; k < LPH; k <<= 1) ss += __shfl_xor(ss, k, 64);
+                ss = group_sum(ss, LPH);
                 const float inv = 1.f / sqrtf(ss / (float)D + eps);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) v[e] = v[e] * inv * wf[e];

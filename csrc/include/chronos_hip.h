@@ -10,6 +10,8 @@
 #include <hip/hip_bf16.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace chronos {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -47,30 +49,95 @@ __device__ __forceinline__ f32x4 ld_wt(const float* p) {
     return v;
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+// Reductions across lanes on the vector ALUs: the halves and the 16-lane rows of a wave change places (v_permlane32_swap, v_permlane16_swap), within a
+// row lanes turn (row_ror).  A value that is the same in every 2 n lanes of a row is turned by n for lane ^ n.  Same operands, same bits as
+// shuffles, whose way through LDS takes some 100 cycles each.  All lanes of the wave are active.  Decode steps, us, shuffles -> this: one row of four
+// Llama-3-8B layers 525 -> 491 (every row of a GEMV ends in one), of a hybrid of width 1024 156 -> 153, 64 rows of one of 4096 818 -> 808; prompts of 4 x 2048
+// tokens with windowed attention 1706 -> 1683.
+template <typename Op> __device__ __forceinline__ float lanes_xor32(float v, Op&& op) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+template <typename Op> __device__ __forceinline__ float lanes_xor16(float v, Op&& op) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+template <typename Op> __device__ __forceinline__ float lanes_all(float v, Op&& op) {
+    v = lanes_xor16(lanes_xor32(v, op), op);
+#define CHRONOS_ROR(n) v = op(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + n, 0xf, 0xf, false)))
+    CHRONOS_ROR(8);
+    CHRONOS_ROR(4);
+    CHRONOS_ROR(2);
+    CHRONOS_ROR(1);
+#undef CHRONOS_ROR
     return v;
 }
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+struct LaneSum {
+    __device__ __forceinline__ float operator()(float a, float b) const { return a + b; }
+};
+struct LaneMax {
+    __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); }
+};
+__device__ __forceinline__ float wave_sum(float v) { return lanes_all(v, LaneSum{}); }
+__device__ __forceinline__ float wave_max(float v) { return lanes_all(v, LaneMax{}); }
+// over the four lanes that share lane % 16 (the rows of a matrix product's column)
+__device__ __forceinline__ float rows_sum(float v) { return lanes_xor32(lanes_xor16(v, LaneSum{}), LaneSum{}); }
+__device__ __forceinline__ float rows_max(float v) { return lanes_xor32(lanes_xor16(v, LaneMax{}), LaneMax{}); }
+
+// over groups of n neighbouring lanes, n a power of two (the lanes of a group all active): the quad, then the row's quads and halves mirrored, whose lanes hold
+// the same by then
+__device__ __forceinline__ float group_sum(float v, int n) {
+#define CHRONOS_DPP(c) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), c, 0xf, 0xf, false))
+    if (n > 1) CHRONOS_DPP(0xb1);    // quad_perm 1 0 3 2
+    if (n > 2) CHRONOS_DPP(0x4e);    // quad_perm 2 3 0 1
+    if (n > 4) CHRONOS_DPP(0x141);   // row_half_mirror
+    if (n > 8) CHRONOS_DPP(0x140);   // row_mirror
+#undef CHRONOS_DPP
+    if (n > 16) v = lanes_xor16(v, LaneSum{});
+    if (n > 32) v = lanes_xor32(v, LaneSum{});
     return v;
+}
+// over the lanes that share lane % n, n 16, 32 or 64
+template <int n> __device__ __forceinline__ float across_sum(float v) {
+    static_assert(n == 16 || n == 32 || n == 64, "rows of lanes");
+    if constexpr (n == 16) v = lanes_xor16(v, LaneSum{});
+    if constexpr (n <= 32) v = lanes_xor32(v, LaneSum{});
+    return v;
+}
+// The wave's best (largest value, lowest number of equal ones) in every lane, a value s beside it; no value is NaN
+__device__ __forceinline__ void lanes_best(float& v, int& e, float& s) {
+    auto better = [](float v1, int e1, float v0, int e0) { return v1 > v0 || (v1 == v0 && e1 < e0); };
+    auto pair = [&](const auto& pv, const auto& pe, const auto& ps) {
+        const bool second = better(__uint_as_float(pv[1]), (int)pe[1], __uint_as_float(pv[0]), (int)pe[0]);
+        v = __uint_as_float(second ? pv[1] : pv[0]);
+        e = (int)(second ? pe[1] : pe[0]);
+        s = __uint_as_float(second ? ps[1] : ps[0]);
+    };
+    auto swap32 = [](uint32_t x) { return __builtin_amdgcn_permlane32_swap(x, x, false, false); };
+    auto swap16 = [](uint32_t x) { return __builtin_amdgcn_permlane16_swap(x, x, false, false); };
+    pair(swap32(__float_as_uint(v)), swap32((uint32_t)e), swap32(__float_as_uint(s)));
+    pair(swap16(__float_as_uint(v)), swap16((uint32_t)e), swap16(__float_as_uint(s)));
+    auto turned = [&](auto ctrl) {
+        auto ror = [](int x) { return __builtin_amdgcn_update_dpp(0, x, decltype(ctrl)::value, 0xf, 0xf, false); };
+        const float ov = __int_as_float(ror(__float_as_int(v))), os = __int_as_float(ror(__float_as_int(s)));
+        const int oe = ror(e);
+        if (better(ov, oe, v, e)) v = ov, e = oe, s = os;
+    };
+    turned(std::integral_constant<int, 0x128>{});
+    turned(std::integral_constant<int, 0x124>{});
+    turned(std::integral_constant<int, 0x122>{});
+    turned(std::integral_constant<int, 0x121>{});
 }
 
-// Block-wide sum for blockDim.x <= 1024; `red` must hold >= 16 floats of LDS.
+// Block-wide sum for blockDim.x <= 1024, a multiple of 64; `red` must hold >= 16 floats of LDS.  Every wave adds the waves' sums itself.
 __device__ __forceinline__ float block_sum(float v, float* red) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
     v = wave_sum(v);
     if (lane == 0) red[w] = v;
     __syncthreads();
-    float t = (threadIdx.x < (unsigned)nw) ? red[threadIdx.x] : 0.f;
-    if (w == 0) t = wave_sum(t);
-    if (threadIdx.x == 0) red[0] = t;
+    const float t = wave_sum(lane < nw ? red[lane] : 0.f);
     __syncthreads();
-    float r = red[0];
-    __syncthreads();
-    return r;
+    return t;
 }
 
 // ---- fp8 e4m3 (OCP "fn" encoding on gfx950 — not MI300's fnuz) KV-cache helpers ---------------------------------

@@ -250,8 +250,7 @@ __global__ void __launch_bounds__(256, PF ? 2 : 1) paged_attn_kernel(
                     s[g][i] = v;
                     mx = fmaxf(mx, v);
                 }
-            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            mx = rows_max(mx);
             const float mnew = fmaxf(m[qt], mx);
             const float alpha = exp2f(m[qt] - mnew);
             m[qt] = mnew;
@@ -299,8 +298,7 @@ __global__ void __launch_bounds__(256, PF ? 2 : 1) paged_attn_kernel(
 #pragma unroll
     for (int qt = 0; qt < NQT; ++qt) {
         float lt = lsum[qt];
-        lt += __shfl_xor(lt, 16, 64);
-        lt += __shfl_xor(lt, 32, 64);
+        lt = rows_sum(lt);
         const int row = qt * 16 + r;
         if (h4 == 0) {
             sm[w * ROWS + row] = m[qt];
@@ -577,8 +575,7 @@ __global__ void __launch_bounds__(256, 1) split_decode_kernel(
                 sc[g][i] = v;
                 mx = fmaxf(mx, v);
             }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = rows_max(mx);
         const float mnew = fmaxf(m, mx);
         const float alpha = exp2f(m - mnew);
         m = mnew;
@@ -643,8 +640,7 @@ __global__ void __launch_bounds__(256, 1) split_decode_kernel(
     const float oscale = FP8 ? v_scale : 1.f;  // fp8: V's cache scale applied once to the merged output
     {
         float lt = lsum;
-        lt += __shfl_xor(lt, 16, 64);
-        lt += __shfl_xor(lt, 32, 64);
+        lt = rows_sum(lt);
         if (h4 == 0) {
             sm[w * ROWS + r] = m;
             sl[w * ROWS + r] = lt;
@@ -1018,8 +1014,7 @@ __global__ void __launch_bounds__(256, OCC) paged_decode_kernel(
             for (int g = 0; g < 2; ++g)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[g][i]);
-            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * scale_log2;
+            mx = rows_max(mx) * scale_log2;
             if (__any(mx > m + kRescaleThrD)) {
                 const float mnew = fmaxf(m, mx);
                 alpha = __builtin_amdgcn_exp2f(m - mnew);
@@ -1050,8 +1045,7 @@ __global__ void __launch_bounds__(256, OCC) paged_decode_kernel(
                 s[g][i] = v;
                 mx = fmaxf(mx, v);
             }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = rows_max(mx);
         const float mnew = fmaxf(m, mx);
         alpha = exp2f(m - mnew);
         m = mnew;
@@ -1092,8 +1086,7 @@ __global__ void __launch_bounds__(256, OCC) paged_decode_kernel(
     }
 
     float lt = lsum;
-    lt += __shfl_xor(lt, 16, 64);
-    lt += __shfl_xor(lt, 32, 64);
+    lt = rows_sum(lt);
     if (r < G && cmem) {
         // merge with the prefix part: out = (o 2^(m - M) + Op l_p 2^(m_p - M)) / (l 2^(m - M) + l_p 2^(m_p - M)),
         // M = max(m, lse_p), with the producer's Op = its O / l_p and lse_p = m_p + log2 l_p (scaled log2 units)
@@ -1235,8 +1228,7 @@ __global__ void __launch_bounds__(256) casc_prefix_kernel(
         for (int g = 0; g < 2; ++g)
 #pragma unroll
             for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sc[g][i]);
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * scale_log2;
+        mx = rows_max(mx) * scale_log2;
         const float mnew = fmaxf(m, mx);
         const float alpha = exp2f(m - mnew);
         m = mnew;
@@ -1258,8 +1250,7 @@ __global__ void __launch_bounds__(256) casc_prefix_kernel(
         }
     }
     float lt = lsum;
-    lt += __shfl_xor(lt, 16, 64);
-    lt += __shfl_xor(lt, 32, 64);
+    lt = rows_sum(lt);
     if (mem) {
         const int64_t row = (int64_t)seq * hq + head;
         const float inv = 1.f / lt;  // lt >= 1: the row's max key contributes 2^0

@@ -188,8 +188,7 @@ __global__ void __launch_bounds__(256, 2) attn_prefill_kernel(
                         sc[g][i] = v;
                         mx = fmaxf(mx, v);
                     }
-                mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-                mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+                mx = rows_max(mx);
                 const float mnew = fmaxf(m[mt], mx);
                 const float alpha = exp2f(m[mt] - mnew);
                 m[mt] = mnew;
@@ -220,8 +219,7 @@ __global__ void __launch_bounds__(256, 2) attn_prefill_kernel(
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
         float lt = lsum[mt];
-        lt += __shfl_xor(lt, 16, 64);
-        lt += __shfl_xor(lt, 32, 64);
+        lt = rows_sum(lt);
         const int R = w * 32 + mt * 16 + r;
         const int tr = rel0 + R / G, hd = h * G + R % G;
         if (tr >= qlen) continue;
@@ -534,7 +532,7 @@ __global__ void __launch_bounds__(256, 2) attn_prefill2_kernel(
             for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sc[kb][i]);
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * scale_log2;
+            mx = lanes_xor32(mx, LaneMax{}) * scale_log2;
         } else {
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb)
@@ -550,7 +548,7 @@ __global__ void __launch_bounds__(256, 2) attn_prefill2_kernel(
                     sc[kb][i] = v;
                     mx = fmaxf(mx, v);
                 }
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            mx = lanes_xor32(mx, LaneMax{});
         }
         // defer-max (cdna_hip_programming.md T13): O and l are rescaled only when some row's max grew more than
         // kRescaleThr (log2 units) past the max its running sums use — a wave-uniform branch, rare once the causal
@@ -902,7 +900,7 @@ __global__ void __launch_bounds__(256, 2) attn_prefill8_kernel(
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
             for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sc[kb][i]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * cl;
+        mx = lanes_xor32(mx, LaneMax{}) * cl;
         if constexpr (FOLD) {
             // mx is relative to m (the accumulators started at -m)
             if (s == 0 || __any(mx > kRescaleThr)) {

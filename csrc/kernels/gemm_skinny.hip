@@ -309,8 +309,7 @@ __global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a) {
                 *reinterpret_cast<u16x4*>(a.y + at) = o;
             }
             // the CPR consecutive lanes of a row hold its 16 RT outputs: butterfly in a fixed order
-#pragma unroll
-            for (int off = 1; off < CPR; off <<= 1) ss += __shfl_xor(ss, off, 64);
+            ss = group_sum(ss, CPR);
             if (c == 0 && live) a.part_out[(int64_t)r * (a.N / (16 * RT)) + g] = ss;
         } else {
             const int n = g * 16 * RT + 4 * c;
