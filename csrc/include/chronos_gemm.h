@@ -67,6 +67,21 @@ bool launch_gemm_lg_f8(int cfg, bool swiglu, const PPArgs& a, hipStream_t st);
 constexpr int kSkinnyConfigs = 18;
 constexpr int kSkinnyUneven = 12;  // from this config on: plain epilogue and activations only, K any multiple of 64 (the shares of slices
                                   // and waves differ by a unit), the split's sums in a second launch instead of tickets
+// The norm in front of a product of few rows, made by every workgroup itself: c = alpha x + (the S float32 slices ys [S, M, K] of a product, summed in
+// order and rounded, or its rows y), xn = c / rms(c) wn, the product's rows h = xn in bfloat16.  The first workgroup writes xn and h for
+// whoever else reads them; xn is not x, which the others still read.
+struct JoinRows {
+    const float* ys;
+    const uint16_t* y;
+    int S;
+    int64_t stride;
+    const float *x, *wn;
+    float* xn;
+    uint16_t* h;
+    float alpha, eps;
+};
+constexpr int kJoinMost = 4096;   // M K at most, K % 256 == 0
+bool launch_gemm_join(int cfg, int mode, const PPArgs& a, const JoinRows& j, hipStream_t st);
 int gemm_skinny_rt(int cfg);
 int gemm_skinny_mt(int cfg);
 int gemm_skinny_nw(int cfg);  // waves per workgroup

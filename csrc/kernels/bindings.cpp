@@ -732,6 +732,56 @@ std::tuple<Tensor, Tensor> gemm_few(const Tensor& x, const Tensor& w, int64_t cf
     return {y, yf};
 }
 
+// gemm_few, or the plain product, behind a post-norm join whose rows every workgroup makes itself (JoinRows): y [S, M, K] float32 slices or [M, K]
+// bfloat16, x [M, K] float32 (read), h [M, K] bfloat16 (written) -> (product, its float32 rows, the new x).
+std::tuple<Tensor, Tensor, Tensor> gemm_join(const Tensor& y, const Tensor& x, const Tensor& wn, double alpha, double eps, Tensor& h, const Tensor& w,
+                                             int64_t cfg, int64_t mode, int64_t n0, int64_t nf, const c10::optional<Tensor>& bias, double limit,
+                                             double slope, double shift) {
+    chk_bf16(w, "w");
+    chk_bf16(h, "h");
+    chk_gpu(x, "x");
+    chk_gpu(y, "y");
+    chk_gpu(wn, "wn");
+    CHK(x.dim() == 2 && x.scalar_type() == at::kFloat && wn.scalar_type() == at::kFloat && wn.numel() == x.size(1) && h.sizes() == x.sizes(), "gemm_join: x [M, K] f32, wn [K] f32, h [M, K]");
+    const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+    const bool slices = y.dim() == 3;
+    CHK(slices ? y.scalar_type() == at::kFloat && y.size(0) >= 1 && y.size(1) == M && y.size(2) == K : y.scalar_type() == at::kBFloat16 && y.sizes() == x.sizes(), "gemm_join: y [S, M, K] f32 or [M, K] bf16");
+    CHK(w.dim() == 2 && w.size(1) == K && M >= 1 && K >= 256 && K % 256 == 0 && M * K <= chronos::kJoinMost && N * K < (1LL << 40), "gemm_join: K % 256 == 0, M K at most kJoinMost");
+    CHK((cfg == 14 || cfg == 15) && (mode == 0 || (mode == chronos::kPPGlu && cfg == 15)), "gemm_join: cfg, mode");
+    CHK(N >= 1 && N % (16 * chronos::gemm_skinny_rt((int)cfg)) == 0, "gemm_join: N % (16 RT)");
+    CHK(mode == 0 ? n0 >= 0 && nf >= 0 && n0 % 4 == 0 && n0 + nf <= N : nf == 0, "gemm_join: n0 % 4 == 0, n0 + nf <= N; with an activation no float32 outputs");
+    CHK(((reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr()) | reinterpret_cast<uintptr_t>(y.data_ptr()) |
+          reinterpret_cast<uintptr_t>(wn.data_ptr()) | reinterpret_cast<uintptr_t>(h.data_ptr())) & 15) == 0, "gemm_join: alignment");
+    if (bias.has_value()) {
+        chk_gpu(*bias, "bias");
+        CHK(bias->scalar_type() == at::kFloat && bias->numel() == nf, "gemm_join: bias [nf] f32");
+    }
+    c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+    Tensor xn = at::empty_like(x), yf, out = at::empty({M, mode != 0 ? N / 2 : nf > 0 ? n0 : N}, h.options());
+    chronos::PPArgs a{};
+    a.w = bf(w);
+    a.y = bfm(out);
+    a.M = (int)M;
+    a.N = (int)N;
+    a.K = (int)K;
+    a.F = (int)(N / 2);
+    a.splitk = 1;
+    a.limit = (float)limit;
+    a.slope = (float)slope;
+    a.shift = (float)shift;
+    if (nf > 0) {
+        yf = at::empty({M, nf}, x.options());
+        a.yf = yf.data_ptr<float>();
+        a.bias = bias.has_value() ? bias->data_ptr<float>() : nullptr;
+        a.n0 = (int)n0;
+        a.nf = (int)nf;
+    }
+    const chronos::JoinRows j{slices ? y.data_ptr<float>() : nullptr, slices ? nullptr : bf(y), slices ? (int)y.size(0) : 1, M * K,
+                              x.data_ptr<float>(), wn.data_ptr<float>(), xn.data_ptr<float>(), bfm(h), (float)alpha, (float)eps};
+    CHK(chronos::launch_gemm_join((int)cfg, (int)mode, a, j, cur_stream()), "gemm_join: launch");
+    return {out, yf, xn};
+}
+
 // The float32 slices [splitk, M, N] of a plain product of few rows whose K is split over workgroups, nothing kept between calls: gemm_lg.hip's
 // ring tiles of few rows, gemm_slab.hip (88, two slices and more), or (skinny) gemm_skinny.hip's uneven configs.  Their sum in order, rounded, is the product; one slice is the product unrounded.
 Tensor gemm_slices(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk, bool skinny) {
@@ -1080,6 +1130,8 @@ TORCH_LIBRARY(chronos, m) {
     m.def("gemm(Tensor x, Tensor w, bool swiglu, int stages=3) -> Tensor");
     m.def("gemm_act(Tensor x, Tensor w, int mode, float limit, float slope, float shift) -> Tensor");
     m.def("gemm_few(Tensor x, Tensor w, int cfg, int mode, int n0, int nf, Tensor? bias, float limit, float slope, float shift) -> (Tensor, Tensor)");
+    m.def("gemm_join(Tensor y, Tensor x, Tensor wn, float alpha, float eps, Tensor(a!) h, Tensor w, int cfg, int mode, int n0, int nf, Tensor? bias, float limit, float slope, "
+          "float shift) -> (Tensor, Tensor, Tensor)");
     m.def("gemm_ring(Tensor x, Tensor w, int cfg, int splitk, int mode, int n0, int nf, Tensor? bias, float limit, float slope, float shift) -> (Tensor, Tensor)");
     m.def("gemv_act(Tensor x, Tensor w, int mode, float limit, float slope, float shift) -> Tensor");
     m.def("gemm_split(Tensor x, Tensor w, int cfg, int splitk) -> Tensor");
@@ -1132,6 +1184,7 @@ TORCH_LIBRARY_IMPL(chronos, CUDA, m) {
     m.impl("gemm", &gemm);
     m.impl("gemm_act", &gemm_act);
     m.impl("gemm_few", &gemm_few);
+    m.impl("gemm_join", &gemm_join);
     m.impl("gemm_ring", &gemm_ring);
     m.impl("gemv_act", &gemv_act);
     m.impl("gemm_split", &gemm_split);

@@ -24,6 +24,7 @@
 //     reproducible, graph == eager);
 //   * epilogue per (row m, 4 consecutive outputs): 8-byte stores, CPR consecutive lanes cover a row's 16 RT outputs.
 #include <algorithm>
+#include <type_traits>
 
 #include "chronos_act.h"
 #include "chronos_gemm.h"
@@ -36,8 +37,15 @@ enum : int { kPlain = kPPPlain, kSwiglu = kPPSwiglu, kResid = kPPResid, kGlu = k
 constexpr bool sk_pair(int mode) { return mode == kSwiglu || mode == kGlu; }   // w = [gate; up]
 constexpr int XL_MIN_MT = 2;  // x staged through LDS from MT = 2 (x bytes >= the weight bytes per wave)
 
-template <int RT, int MT, int D, int NW, int MODE, bool NORMP>
-__global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a) {
+struct NoJoin {};
+
+// Join (JoinRows): the rows come from a post-norm join that every workgroup makes itself, a launch less.  Bound by the chain of launches: a product of one
+// row that takes 3.5 to 6 us takes about 2 us more so, its join as a launch 3 to 3.5 (a decode step of one row, width 1024: 151 -> 144 us).
+
+template <int RT, int MT, int D, int NW, int MODE, bool NORMP, typename Join = NoJoin>
+__global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a, Join jn) {
+    constexpr bool JOIN = !std::is_same_v<Join, NoJoin>;
+    static_assert(!JOIN || (MT == 1 && !NORMP && (MODE == kPlain || MODE == kGlu)), "a join in front: up to 16 rows");
     static_assert(!sk_pair(MODE) || RT % 2 == 0, "swiglu: RT/2 gate tiles + RT/2 up tiles");
     constexpr int NT = 64 * NW;                        // threads
     constexpr int UNITS = RT * MT * 64;                // f32x4 accumulators per wave
@@ -80,7 +88,7 @@ __global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a) {
     const bf16x8* xp[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-        if constexpr (XL)  // pieces of 8 rows: xp[i] for i < 2 MT covers rows 8 i .. 8 i + 7
+        if constexpr (XL || JOIN)  // pieces of 8 rows: xp[i] for i < 2 MT covers rows 8 i .. 8 i + 7
             xp[mt] = nullptr;
         else
             xp[mt] = reinterpret_cast<const bf16x8*>(a.x + (int64_t)min(16 * mt + (lane & 15), M - 1) * K + kbase);
@@ -104,7 +112,7 @@ __global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a) {
             wr[d][rt][1] = __builtin_nontemporal_load(wp[rt] + off + 4);
         }
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
+        for (int mt = 0; mt < MT && !JOIN; ++mt) {
             if constexpr (XL) {  // the same registers, in the line layout: piece 2 mt + h
                 xr[d][mt][0] = xl[2 * mt][off];
                 xr[d][mt][1] = xl[2 * mt + 1][off];
@@ -114,9 +122,60 @@ __global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a) {
             }
         }
     };
+    // JOIN: the rows' 4 columns of thread tid in runs of 256, wave w runs w and NW + w; everything that they read is asked for before the weights
+    unsigned char* const hs = smem + NW * SZ * 16 + 16 * MT * 4 + 16;   // the product's rows [M, K]
+    constexpr int JR = JOIN ? kJoinMost / 256 / NW : 1;
+    f32x4 jc[JR], jw[JR], jv[JR];
+    if constexpr (JOIN) {
+#pragma unroll
+        for (int q = 0; q < JR; ++q) {
+            const int at = (q * NW + wave) * 256 + 4 * lane;
+            if ((q * NW + wave) * 256 >= M * K) break;   // (wave-uniform)
+            jc[q] = *reinterpret_cast<const f32x4*>(jn.x + at);
+            jw[q] = *reinterpret_cast<const f32x4*>(jn.wn + at % K);
+            if (jn.ys != nullptr) {
+                f32x4 v = *reinterpret_cast<const f32x4*>(jn.ys + at);
+#pragma unroll 4
+                for (int k = 1; k < jn.S; ++k) v += *reinterpret_cast<const f32x4*>(jn.ys + k * jn.stride + at);
+                jv[q] = v;
+            } else {
+                const u16x4 v = *reinterpret_cast<const u16x4*>(jn.y + at);
+                jv[q] = f32x4{bf2f(v[0]), bf2f(v[1]), bf2f(v[2]), bf2f(v[3])};
+            }
+        }
+    }
 #pragma unroll
     for (int d = 0; d < D; ++d)
         if (d < NU) load(d, d);
+
+    if constexpr (JOIN) {
+        float* const red = reinterpret_cast<float*>(smem);
+#pragma unroll
+        for (int q = 0; q < JR; ++q) {
+            if ((q * NW + wave) * 256 >= M * K) break;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) jc[q][e] = jc[q][e] * jn.alpha + bf2f(f2bf(jv[q][e]));   // (rows of y are bfloat16 already)
+            const float ss = wave_sum(jc[q][0] * jc[q][0] + jc[q][1] * jc[q][1] + jc[q][2] * jc[q][2] + jc[q][3] * jc[q][3]);
+            if (lane == 0) red[q * NW + wave] = ss;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < JR; ++q) {
+            const int at = (q * NW + wave) * 256 + 4 * lane;
+            if ((q * NW + wave) * 256 >= M * K) break;
+            const int runs = K / 256, r0 = (q * NW + wave) / runs * runs;
+            float sum = 0.f;
+            for (int k = 0; k < runs; ++k) sum += red[r0 + k];
+            const f32x4 v = jc[q] * (1.f / sqrtf(sum / (float)K + jn.eps)) * jw[q];
+            const u16x4 o = {f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
+            *reinterpret_cast<u16x4*>(hs + at * 2) = o;
+            if (blockIdx.x == 0) {
+                *reinterpret_cast<f32x4*>(jn.xn + at) = v;
+                *reinterpret_cast<u16x4*>(jn.h + at) = o;
+            }
+        }
+        __syncthreads();
+    }
 
     f32x4 acc[RT][MT];
 #pragma unroll
@@ -129,6 +188,11 @@ __global__ void __launch_bounds__(64 * NW) skinny_kernel(PPArgs a) {
         for (int d = 0; d < D; ++d) {
             const int u = u0 + d;
             if (u < NU) {
+                if constexpr (JOIN) {
+                    const unsigned char* const at = hs + (min(lane & 15, M - 1) * K + kbase + u * 64 * NW) * 2;
+                    xr[d][0][0] = *reinterpret_cast<const bf16x8*>(at);
+                    xr[d][0][1] = *reinterpret_cast<const bf16x8*>(at + 64);
+                }
                 if constexpr (XL) {
                     // line layout -> LDS (row t = 8 i + lane / 8, chunk lane % 8 in slot chunk ^ (t & 7)) -> MFMA layout
                     // (row 16 mt + lane % 16, chunk 4 h + lane / 16); LDS ops of a wave run in order, so the previous
@@ -392,7 +456,7 @@ void launch_cfg(const PPArgs& a, hipStream_t st) {
         attr = true;
     }
     const int G = sk_pair(MODE) ? a.F / (8 * RT) : a.N / (16 * RT);
-    hipLaunchKernelGGL(kern, dim3(G * a.splitk), dim3(64 * NW), lds, st, a);
+    hipLaunchKernelGGL(kern, dim3(G * a.splitk), dim3(64 * NW), lds, st, a, NoJoin{});
     if (a.splitk > 1 && a.cnt == nullptr && a.y != nullptr) launch_gemm_slices(a.ws, a.y, (int64_t)a.M * a.N, a.splitk, st);
 }
 
@@ -441,6 +505,26 @@ bool launch_mode(int cfg, const PPArgs& a, hipStream_t st) {
 }
 
 }  // namespace
+
+namespace {
+template <int RT, int D, int NW, int MODE>
+void launch_join(const PPArgs& a, const JoinRows& j, hipStream_t st) {
+    constexpr int UNITS = RT * 64, base = NW * (UNITS + UNITS / 16) * 16 + 16 * 4 + 16;
+    const auto kern = skinny_kernel<RT, 1, D, NW, MODE, false, JoinRows>;
+    static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, base + 2 * kJoinMost);
+    (void)set;
+    kern<<<sk_pair(MODE) ? a.F / (8 * RT) : a.N / (16 * RT), 64 * NW, base + a.M * a.K * 2, st>>>(a, j);
+}
+}  // namespace
+
+// configs 14 and 15, plain (with float32 rows behind or not) and gated units
+bool launch_gemm_join(int cfg, int mode, const PPArgs& a, const JoinRows& j, hipStream_t st) {
+    if (cfg == 14 && mode == kPlain) launch_join<1, 4, 8, kPlain>(a, j, st);
+    else if (cfg == 15 && mode == kPlain) launch_join<2, 4, 8, kPlain>(a, j, st);
+    else if (cfg == 15 && mode == kGlu) launch_join<2, 4, 8, kGlu>(a, j, st);
+    else return false;
+    return true;
+}
 
 int gemm_skinny_rt(int cfg) {
     switch (cfg) {

@@ -1291,10 +1291,14 @@ class HybridDecoder:
             for ri, li in enumerate(cfg.runs):   # the cache is keyed by run, the weights by layer
                 spec, lw = cfg.layers[li], w.layers[li]
                 y = MIXERS[spec.mixer.kind][0](self, ri, spec.mixer, lw.mix, h, meta, cache)
-                h = self._join(y, x, lw.norm1)
+                last = ri + 1 == len(cfg.runs)
+                x = h.stream() if type(h) is hops.JoinedRows else x
+                nxt = None if last else cfg.layers[cfg.runs[ri + 1]].mixer.kind   # what reads the join's rows
+                h = self._join(y, x, lw.norm1, nxt if spec.ff is None else spec.ff.kind)
                 if spec.ff is not None:
                     y = FEED_FORWARDS[spec.ff.kind][0](self, spec.ff, lw.ff, h)
-                    h = self._join(y, x, lw.norm2)
+                    x = h.stream() if type(h) is hops.JoinedRows else x
+                    h = self._join(y, x, lw.norm2, nxt)
                 if self.layer_tap is not None:
                     self.layer_tap(ri, x)
         if cfg.residual == "out_norm":
@@ -1428,14 +1432,18 @@ class HybridDecoder:
             return hops.matmul_parts(x, w)
         return hops.matmul(x, w, bias)
 
-    def _join(self, y, x, w):
+    def _join(self, y, x, w, reader=None):
         """The residual rule: folds the sublayer output y into the float32 stream x (in place) and returns the
-        stream in the activation dtype for the next sublayer."""
+        stream in the activation dtype for the next sublayer.  reader: its kind; for one whose first product takes a join of few
+        rows with it, a hops.JoinedRows, whose stream() is x from then on."""
         cfg = self.cfg
         if isinstance(y, (tuple, PairOut)):
             raise NotImplementedError("a feed-forward with a separate part needs the pre-norm or the sandwich stream, "
                                       "a parallel mixer the sandwich stream")
         if cfg.residual == "post_norm":
+            if reader in ("delta_rule", "gla", "window_attention", "glu") and self.layer_tap is None and self.act_dtype == torch.bfloat16 and \
+                    hops.JoinedRows.serves(y, x):
+                return hops.JoinedRows(y, x, w, cfg.residual_alpha, cfg.norm_eps)
             return hops.scale_add_rms_norm(y, x, w, cfg.residual_alpha, cfg.norm_eps, self.act_dtype)
         return hops.add_layer_norm(y, x, w, cfg.norm_eps, self.act_dtype)
 

@@ -601,6 +601,27 @@ def product_rows(x: torch.Tensor, w: torch.Tensor, n0: int, nf: int, bias: Optio
     return _k().gemm_few(x, w, cfg, 0, n0, nf, bias, 0.0, 0.0, 0.0) if cfg else None
 
 
+def join_rows_ok(m: int, k: int) -> bool:
+    """Sizes at which a product's workgroups make a join's m rows of k columns themselves.  A decode step of four layers, us, joins as launches of
+    their own -> in the products: one row of 1024 151 -> 144, of 2048 225 -> 214, of 4096 457 -> 446; 2 rows of 1024 155 -> 149; beyond, every workgroup's
+    reading outweighs the launch: 3 rows of 1024 156 -> 158, 4 157 -> 160, 2 of 2048 231 -> 233."""
+    return 0 < m and k % 256 == 0 and m * k <= (4096 if m == 1 else 2048)
+
+
+def join_config(h: torch.Tensor, w: torch.Tensor, kind: int) -> int:
+    """Config of gemm_join for the rows h that a post-norm join is to give, or 0 where the join and its product take two launches: kind 0 a product
+    with float32 rows behind, 1 a plain one, 2 a gated unit, each where gemm_few's configs of one x tile have it alone."""
+    m, (n, k) = h.shape[0], w.shape
+    if not join_rows_ok(m, k) or n % 32 or not _plain_rows(h, w) or _registered(m, n, k):
+        return 0
+    if kind == 1:
+        plan = _linear_plan(m, n, k)
+        cfg = plan[0] - SK_BASE if plan is not None and plan[1] == 1 else 0
+    else:
+        cfg = 0 if _ring_more(m, n, k) else _few_more(m, n, k, kind)
+    return cfg if cfg == 15 or (cfg == 14 and kind != 2) else 0
+
+
 _Tensor, _WEIGHTS, _BF16 = torch.Tensor, (torch.Tensor, torch.nn.Parameter), torch.bfloat16
 _autocast, _grad, _functorch, _forward_ad = torch.is_autocast_enabled, torch.is_grad_enabled, torch._C._are_functorch_transforms_active, torch.autograd.forward_ad
 

@@ -50,10 +50,49 @@ def _f32(act_dtype) -> bool:
     return act_dtype == torch.float32
 
 
+class JoinedRows:
+    """scale_add_rms_norm(y, x, w, ..) for the product behind it: a launch less where every workgroup of that product makes the rows itself.
+    ``stream()`` is the float32 residual behind the join, ``rows()`` its rows in the activation dtype; both join first, in x, if no product has."""
+
+    def __init__(self, y, x, w, alpha: float, eps: float):
+        self.y, self.x, self.w, self.alpha, self.eps, self.done = y, x, w, alpha, eps, False
+        self.h = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device)
+
+    @staticmethod
+    def serves(y, x) -> bool:
+        return _gpu(x) and type(y) is torch.Tensor and type(x) is torch.Tensor and x.dim() == 2 and _gemm.join_rows_ok(*x.shape) and \
+            y.is_contiguous() and x.is_contiguous() and (y.dtype == torch.float32 if y.dim() == 3 else y.dtype == torch.bfloat16 and y.shape == x.shape) and \
+            not (torch.is_grad_enabled() and (y.requires_grad or x.requires_grad))
+
+    def rows(self):
+        if not self.done:
+            self.h = scale_add_rms_norm(self.y, self.x, self.w, self.alpha, self.eps, torch.bfloat16)
+            self.done = True
+        return self.h
+
+    def stream(self):
+        self.rows()
+        return self.x
+
+    def product(self, w, kind: int, n0: int = 0, nf: int = 0, bias=None, limit: float = 0.0, slope: float = 0.0, shift: float = 0.0):
+        """(product, its float32 rows) as _gemm.join_config's kinds, or None."""
+        cfg = 0 if self.done else _gemm.join_config(self.h, w, kind)
+        if not cfg:
+            return None
+        out, few, self.x = _gemm._k().gemm_join(self.y, self.x, self.w, self.alpha, self.eps, self.h, w, cfg, 3 if kind == 2 else 0, n0, nf, bias, limit, slope, shift)
+        self.done = True
+        return out, few
+
+
 def matmul(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
     """x @ w.T (+ bias): the framework's routed projection GEMMs for bfloat16, the library's float32 GEMM otherwise.
     A biased projection is one library GEMM whose epilogue adds the bias (in the activation dtype, like w) to the
     float accumulator before the rounding."""
+    if type(x) is JoinedRows:
+        y = x.product(w, 1) if bias is None else None
+        if y is not None:
+            return y[0]
+        x = x.rows()
     if bias is not None:
         return torch.addmm(bias, x, w.t())
     if x.dtype == torch.bfloat16:
@@ -125,6 +164,8 @@ def add_layer_norm(y, x, w, eps: float, act_dtype):
 
 
 def rowdot(h, w, bias=None):
+    if type(h) is JoinedRows:
+        h = h.rows()
     if _gpu(h):
         return _k().hy_rowdot(h, w, bias)
     return ref.rowdot(h, w, bias)
@@ -133,6 +174,11 @@ def rowdot(h, w, bias=None):
 def matmul_rowdot(h, w, w_few, bias=None, joined=None):
     """(h @ w.T, rowdot(h, w_few, bias)); ``joined`` (whole, n0, nf): both matrices' rows one behind the other, which few rows of h take in
     one launch."""
+    if type(h) is JoinedRows:
+        y = h.product(joined[0], 0, joined[1], joined[2], bias) if joined is not None else None
+        if y is not None:
+            return y
+        h = h.rows()
     if joined is not None and _gpu(h) and h.dtype == torch.bfloat16:
         y = _gemm.product_rows(h, *joined, bias)
         if y is not None:
@@ -158,6 +204,11 @@ def matmul_act(x, w, kind: int):
 
 def matmul_glu(x, w, limit: float, slope: float, shift: float, act_dtype):
     """glu(x @ w.T, ...), w = [gate; up], in the product's epilogue where that is faster (the unit then reads the unrounded product)."""
+    if type(x) is JoinedRows:
+        y = x.product(w, 2, 0, 0, None, limit, slope, shift) if act_dtype == torch.bfloat16 else None
+        if y is not None:
+            return y[0]
+        x = x.rows()
     if _gpu(x) and x.dtype == torch.bfloat16 and act_dtype == torch.bfloat16:
         y = _gemm.product_act(x, w, 3, limit, slope, shift)
         if y is not None:
