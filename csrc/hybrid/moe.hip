@@ -13,6 +13,7 @@
 //
 // No step of either kernel depends on the host knowing the routing: both capture into a graph.
 #include "hybrid_common.h"
+#include "rowdot_tile.h"
 
 #include <type_traits>
 
@@ -311,6 +312,24 @@ __global__ void __launch_bounds__(64 * kRouteWaves) moe_route_token_kernel(const
     if (wave == 0) select_any<FORM>(z, idx + t * c.top, wt + t * c.top, c, sc, okg);
 }
 
+// Projection and choice of many tokens: a workgroup takes 16 tokens by all N <= 16 NT rows of w, its 8 waves then choose for two of them each; the
+// logits stay in LDS and are those of the projection by itself, bit for bit.  us, two launches -> this, softmax and top-k: 600 tokens of 1024 by 8 rows 8.0, 7.0 -> 7.4,
+// 5.8; 2446 of 2048 by 18 13.0, 11.5 -> 12.6, 10.2; 8192 of 2048 by 16 21.1, 17.1 -> 17.8, 14.2; of 4096 by 32 34.8, 31.0 -> 30.3, 27.6.  Beyond 32 rows the choices, two
+// after each other in a wave, take longer than the launch: 8192 of 4096 by 34 31.4, 27.8 -> 34.4, 31.5, by 64 43.8, 38.2 -> 48.3, 44.8; 1000 by 64 28.8, 27.3 -> 30.2, 27.2.
+template <int FORM, int NT>
+__global__ void __launch_bounds__(512) moe_route_tile_kernel(const uint16_t* __restrict__ h, const uint16_t* __restrict__ w, const float* __restrict__ bias,
+                                                             int32_t* __restrict__ idx, float* __restrict__ wt, int rows, int d, Choice c) {
+    __shared__ f32x4 red[8][NT][64];
+    __shared__ float z[16][16 * NT], sc[FORM == kGroups ? 8 : 1][16 * NT];
+    __shared__ int okg[FORM == kGroups ? 8 : 1][64];
+    const int64_t t0 = (int64_t)blockIdx.x * 16;
+    const int wv = threadIdx.x >> 6;
+    rowdot_tile<1, NT, 8>(h, w, bias, t0, 0, rows, d, c.N, red, [&](int64_t t, int r, float v) { z[t - t0][r] = v; });
+    __syncthreads();
+    for (int i = wv; i < 16 && t0 + i < rows; i += 8)
+        select_any<FORM>(z[i], idx + (t0 + i) * c.top, wt + (t0 + i) * c.top, c, sc[FORM == kGroups ? wv : 0], okg[FORM == kGroups ? wv : 0]);
+}
+
 // Gated experts: per token sum_k weight_k * W_down,e ( g sigmoid(slope g) (u + shift) ), g = min(W_gate,e h, limit),
 // u = clamp(W_up,e h, +-limit).  w_gu [E, 2F, d]: gate rows then up rows, or (tiled) in the grouped path's tile order.
 // LDS: h (d) | gate, up (2F) | out (d).
@@ -382,6 +401,13 @@ static void moe_route(const void* h, const void* w, const float* bias, float* z,
     if (T == 0) return;
     if (!f32 && hy_moe_route_one(T, c.N, d) && hy::aligned16(h, w)) {
         hy::moe_route_token_kernel<FORM><<<T, 64 * hy::kRouteWaves, 0, s>>>((const uint16_t*)h, (const uint16_t*)w, bias, idx, wt, d, c);
+        return;
+    }
+    if (!f32 && T > 512 && c.N > 0 && c.N <= 32 && d % 64 == 0 && hy::aligned16(h, w)) {
+        const uint16_t *hb = (const uint16_t*)h, *wb = (const uint16_t*)w;
+        const unsigned wgs = (T + 15) / 16;
+        if (c.N <= 16) hy::moe_route_tile_kernel<FORM, 1><<<wgs, 512, 0, s>>>(hb, wb, bias, idx, wt, T, d, c);
+        else hy::moe_route_tile_kernel<FORM, 2><<<wgs, 512, 0, s>>>(hb, wb, bias, idx, wt, T, d, c);
         return;
     }
     launch_hy_rowdot(h, w, bias, z, T, d, c.N, f32, s);
