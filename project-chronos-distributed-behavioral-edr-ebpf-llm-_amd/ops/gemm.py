@@ -608,11 +608,11 @@ def join_rows_ok(m: int, k: int) -> bool:
     return 0 < m and k % 256 == 0 and m * k <= (4096 if m == 1 else 2048)
 
 
-def join_config(h: torch.Tensor, w: torch.Tensor, kind: int) -> int:
+def join_config(h: torch.Tensor, w: torch.Tensor, kind: int, n0: int = 0) -> int:
     """Config of gemm_join for the rows h that a post-norm join is to give, or 0 where the join and its product take two launches: kind 0 a product
-    with float32 rows behind, 1 a plain one, 2 a gated unit, each where gemm_few's configs of one x tile have it alone."""
+    with float32 rows behind its first n0, 1 a plain one, 2 a gated unit, each where gemm_few's configs of one x tile have it alone."""
     m, (n, k) = h.shape[0], w.shape
-    if not join_rows_ok(m, k) or n % 32 or not _plain_rows(h, w) or _registered(m, n, k):
+    if not join_rows_ok(m, k) or n % 32 or not _plain_rows(h, w) or _registered(m, n0 or n, k):
         return 0
     if kind == 1:
         plan = _linear_plan(m, n, k)

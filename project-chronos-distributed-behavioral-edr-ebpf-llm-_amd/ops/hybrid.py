@@ -76,7 +76,7 @@ class JoinedRows:
 
     def product(self, w, kind: int, n0: int = 0, nf: int = 0, bias=None, limit: float = 0.0, slope: float = 0.0, shift: float = 0.0):
         """(product, its float32 rows) as _gemm.join_config's kinds, or None."""
-        cfg = 0 if self.done else _gemm.join_config(self.h, w, kind)
+        cfg = 0 if self.done else _gemm.join_config(self.h, w, kind, n0)
         if not cfg:
             return None
         out, few, self.x = _gemm._k().gemm_join(self.y, self.x, self.w, self.alpha, self.eps, self.h, w, cfg, 3 if kind == 2 else 0, n0, nf, bias, limit, slope, shift)

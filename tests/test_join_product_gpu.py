@@ -74,3 +74,21 @@ def test_model_steps(rows, monkeypatch):
     assert (sum(taken) == 7) == (rows <= 2) and (len(taken) == 0) == (rows > 2)   # eight joins, the last has no reader
     # bfloat16 activations whose last bits differ here and there
     assert float((got[0] - got[1]).norm() / got[1].norm()) < 0.01
+
+
+def test_registered_kernel_gets_its_product():
+    """A kernel registered for the product is called, whatever stands in front of it."""
+    from chronos.ops import gemm
+    from chronos.ops import hybrid as hops
+
+    hops.load()
+    y, x, wn, w, _ = _inputs(1, 1024, 1120, 2, 3)
+    calls = []
+    entry = (lambda m, n, k: (n, k) == (1080, 1024), lambda a, b: calls.append(tuple(b.shape)) or a @ b.t())
+    gemm._custom.append(entry)
+    try:
+        joined = hops.JoinedRows(y, x, wn, 2.0, 1e-6)
+        out, few = hops.matmul_rowdot(joined, w[:1080], w[1080:], None, (w, 1080, 40))
+    finally:
+        gemm._custom.remove(entry)
+    assert calls == [(1080, 1024)] and out.shape == (1, 1080) and few.shape == (1, 40) and joined.stream() is x
