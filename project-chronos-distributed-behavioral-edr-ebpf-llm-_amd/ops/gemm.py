@@ -585,15 +585,16 @@ def _ring_more(m: int, n: int, k: int) -> bool:
 
 
 def product_rows(x: torch.Tensor, w: torch.Tensor, n0: int, nf: int, bias: Optional[torch.Tensor]):
-    """(x @ w[:n0].T, float32 x @ w[n0 : n0 + nf].T + bias) in one launch, or None where two are faster."""
-    if x.dim() != 2 or not 0 < x.shape[0] <= 512 or not _plain_rows(x, w) or _registered(x.shape[0], n0, w.shape[1]):
+    """(x @ w[:n0].T, float32 x @ w[n0 : n0 + nf].T + bias) in one launch, or None where two are faster or one doesn't take these numbers of rows."""
+    if x.dim() != 2 or not 0 < x.shape[0] <= 512 or n0 % 4 or nf < 1 or not _plain_rows(x, w) or _registered(x.shape[0], n0, w.shape[1]):
         return None
     m, (n, k) = x.shape[0], w.shape
     # the ring tiles also wherever gemm_few has no config.  Two launches -> one, us: 12304 x 4096, 64 rows 32.4 -> 25.3, 200 rows 49.1 -> 39.9;
-    # 6160 x 2048, 100 rows 18.6 -> 12.7, 400 rows 26.5 -> 20.3; 3080 x 1024, 400 rows 13.0 -> 10.2
+    # 6160 x 2048, 100 rows 18.6 -> 12.7, 400 rows 26.5 -> 20.3; 3080 x 1024, 400 rows 13.0 -> 10.2.  512 rows are where this rule's
+    # measurements ended and no line of speed (2064 x 2048, 512 rows 17.8 -> 13.2, 600 17.6 -> 13.2, 1500 23.6 -> 17.9).
     cfg = _few_more(m, n, k, 0)
     plan = _linear_plan(m, n0, k) if not cfg or _ring_more(m, n, k) else None
-    if plan is not None and plan[0] in _RING:
+    if plan is not None and plan[0] in _RING and -(-(n0 + nf) // 4) * 4 <= n:   # (it stores in 4s)
         # the rows behind are one tile more, which must not be a round more
         bn, tiles = _PP_BN[plan[0]], -(-m // _PP_BM[plan[0]]) * plan[1]
         if -(-(-(-(n0 + nf) // bn) * tiles) // 256) <= -(-(-(-n0 // bn) * tiles) // 256):
@@ -612,7 +613,7 @@ def join_config(h: torch.Tensor, w: torch.Tensor, kind: int, n0: int = 0) -> int
     """Config of gemm_join for the rows h that a post-norm join is to give, or 0 where the join and its product take two launches: kind 0 a product
     with float32 rows behind its first n0, 1 a plain one, 2 a gated unit, each where gemm_few's configs of one x tile have it alone."""
     m, (n, k) = h.shape[0], w.shape
-    if not join_rows_ok(m, k) or n % 32 or not _plain_rows(h, w) or _registered(m, n0 or n, k):
+    if not join_rows_ok(m, k) or n % 32 or n0 % 4 or not _plain_rows(h, w) or _registered(m, n0 or n, k):
         return 0
     if kind == 1:
         plan = _linear_plan(m, n, k)

@@ -59,6 +59,31 @@ def test_registered_kernels_get_their_products(monkeypatch):
     assert None not in every()
 
 
+# rows behind the product that fill no 4 (the joined matrix ends with them, or has padding), no rows at all, a product off the 4s
+@pytest.mark.parametrize("m", [8, 100, 300])
+@pytest.mark.parametrize("rows,n0,nf,one", [(1030, 1024, 6, None), (1029, 1024, 5, None), (1056, 1024, 6, True), (1032, 1024, 6, True), (1056, 1024, 0, None),
+                                            (1024, 1002, 22, None)])
+def test_rows_behind_that_one_launch_does_not_take(monkeypatch, m, rows, n0, nf, one):
+    """... stay with two: what gemm_ring and gemm_few refuse (n0 in 4s, n0 + nf rows in 4s, rows behind there) does not reach them."""
+    import chronos.ops as ops
+
+    class Kernels:
+        def gemm_ring(self, x, w, cfg, split, mode, n0, nf, *more):
+            assert n0 % 4 == 0 and nf > 0 and (n0 + nf + 3) // 4 * 4 <= w.shape[0]
+            return "y", "f"
+
+        def gemm_few(self, x, w, cfg, mode, n0, nf, *more):
+            assert n0 % 4 == 0 and nf > 0 and n0 + nf <= w.shape[0] and w.shape[0] % 32 == 0
+            return "y", "f"
+
+    monkeypatch.setattr(ops, "_k", Kernels)
+    x, w = torch.zeros(m, 1024, dtype=torch.bfloat16), torch.zeros(rows, 1024, dtype=torch.bfloat16)
+    got = G.product_rows(x, w, n0, nf, None)
+    assert got is None if one is None or (m <= 64 and rows % 32) else got == ("y", "f")
+    h = torch.zeros(1, 1024, dtype=torch.bfloat16)
+    assert n0 % 4 == 0 or G.join_config(h, w, 0, n0) == 0
+
+
 def _operands(m, n, k):
     g = torch.Generator(device=DEV).manual_seed(m + n + k)
     return torch.randn(m, k, device=DEV, generator=g).bfloat16(), (torch.randn(n, k, device=DEV, generator=g) * k ** -0.5).bfloat16()

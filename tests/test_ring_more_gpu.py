@@ -67,6 +67,22 @@ def test_which_products(m, n, k, mode, takes):
     assert (G.product_rows(x, joined, n, 16, None) is not None) == (m > 1 or n * k < 30e6)
 
 
+@pytest.mark.parametrize("m", [8, 100, 400])
+@pytest.mark.parametrize("rows,n0,nf", [(1030, 1024, 6), (1029, 1024, 5), (1031, 1024, 6)])
+def test_joined_without_padding(m, rows, n0, nf):
+    """matmul_rowdot of a joined matrix that ends with its last row."""
+    from chronos.ops import hybrid as hops
+
+    hops.load()
+    g, x, w = _operands(m, rows, 1024)
+    bias = torch.randn(nf, device=DEV, generator=g)
+    y, yf = hops.matmul_rowdot(x, w[:n0], w[n0:n0 + nf].contiguous(), bias, (w, n0, nf))
+    want = x.double() @ w[:n0 + nf].double().t()
+    size = (x.double().abs() @ w[:n0 + nf].double().abs().t()) * 1024 * 2 ** -24          # float32 sums in any order
+    assert ((y.double() - want[:, :n0]).abs() <= want[:, :n0].abs() * 2 ** -8 + size[:, :n0]).all()
+    assert ((yf.double() - want[:, n0:] - bias.double()).abs() <= size[:, n0:] + 2 ** -22 * (want[:, n0:].abs() + bias.abs())).all()
+
+
 @pytest.mark.parametrize("bad", [dict(cfg=36), dict(mode=3, n=130), dict(mode=4, split=2), dict(n0=2), dict(nf=0), dict(n0=128, nf=40), dict(split=5), dict(mode=2)])
 def test_what_is_refused(bad):
     from chronos import ops
