@@ -10,7 +10,8 @@
 //             per-lane LDS-DMA source addresses; activation in the epilogue.
 //   down GEMM Y[row, :] = Z[row, :] W_down[e]^T.
 //   combine   out[t, :] = sum_k weight[t, k] * Y[row(t, k), :]  (+ weight * h[t, :] for an identity expert), summed
-//             in the order of k in float: the result does not depend on what else is in the batch.
+//             in the order of k in float.  A row's sums over d and F have one order, whatever the tile's size and however many items there are
+//             (moe_turn), so the result does not depend on what else is in the batch.
 //
 // Gated experts (act = gated unit): the up GEMM runs over W_gu [E, 2F, d] whose rows are PERMUTED at weight-packing
 // time (moe_glu_row_order) so that every 128-row tile holds 64 gate rows and their 64 up rows in the accumulator
@@ -242,6 +243,16 @@ __device__ __forceinline__ bool moe_place_tile(const int32_t* __restrict__ idx, 
     return there;
 }
 
+// The k-step that tiles over an expert's weight rows 256 tn256 .. start with where they are turned; they take the steps round from there.  It follows from the weights
+// alone and is the same for tiles of all sizes, so that a token's result does not depend on the batch.  All from the first, the
+// workgroups read the same columns of weight rows that lie a power of two apart, lines that share few of the memory's channels.  The whole feed-forward, weights
+// cold, us, from the first step -> turned: 32 experts of 4096 x 2048, top 4, GELU, 2 tokens 64 -> 56, 6 133 -> 112, 64 211 -> 171, 300 (64-row tiles) 224 -> 199, 450
+// and 1000 (128-row tiles) 280 -> 221, 366 -> 338, 1600, 2500 and 8192 (256) 353 -> 295, 507 -> 472, 1131 -> 1092; gated, 4 tokens 129 -> 113, 64 298 -> 251, 450 333 ->
+// 306, 2500 680 -> 648; 128 of 2048 x 1024, top 8, 4 tokens 66 -> 59, 128 196 -> 182, 2000 348 -> 336; 64 gated of 2048 x 1408, top 6, 8192 tokens 862 -> 870.
+// 2 steps per 256 rows and 9 per expert: of nine pairs the best in sum (4 and 9: 64 tokens 171, 1000 345, of 256-row tiles 2500 521 where this took 493; 16 and 9:
+// 172, 345, 514; 1 and 5: 174, 341, 512); 8 and 1, which give many tiles of neighbouring experts the same step, are as slow as none (64 tokens 208).
+__device__ __forceinline__ int moe_turn(int e, int tn256, int KT) { return (2 * tn256 + 9 * e) % KT; }
+
 // The wave's outputs: NS x NM accumulator tiles of 16 weight rows by 16 tokens, from weight row n0 and token row m0 on (item: the items of the lane's
 // tokens, -1: padding, not stored).  Lane l
 // holds D[n = 4 (l >> 4) + i][m = l & 15] of each = y[m][n .. n + 3].
@@ -283,10 +294,6 @@ __device__ __forceinline__ void moe_store(const f32x4 (&acc)[NS][NM], uint16_t* 
 // The tiles there are go to the XCDs in contiguous runs (their L2s then share rows of x and w); a launch of small tiles is
 // bound by the weights' bytes and spreads them over all.
 // ONCE: the weights' DMA is marked as read once (nt), which memory itself gives faster and which leaves nothing behind for a next call.
-// turned: a tile takes its k-steps round from one that its expert and its weight rows choose (so that a token's result does not depend on the
-// batch).  All from the first, the workgroups read the same columns of weight rows that lie a power of two apart, lines that share few of the
-// memory's channels.  32 experts of 4096 x 2048, the whole feed-forward, us: GELU, top 4, 6 tokens 114 -> 90, 64 tokens 218 -> 171, 300 (64-row
-// tiles) 237 -> 195, 450, 700 and 1000 (128-row tiles) 287 -> 220, 360 -> 305, 372 -> 343; gated, 64 tokens 222 -> 190, 300 244 -> 213, 450 273 -> 266, 1000 level.
 template <int TM, bool GATHER, int ACT, bool PLACE, bool ONCE>
 __global__ void __launch_bounds__(256, 2) moe_gemm_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
                                                           uint16_t* __restrict__ y, int32_t* __restrict__ meta,
@@ -345,7 +352,7 @@ __global__ void __launch_bounds__(256, 2) moe_gemm_kernel(const uint16_t* __rest
         items_of();
         __syncthreads();   // the ring's memory is read
     }
-    const int KT = K / BK, turn = turned ? (TM == 128 ? tn + 5 * e : 4 * tn + 9 * e) % KT : 0;
+    const int KT = K / BK, turn = turned ? moe_turn(e, tn / 2, KT) : 0;
     auto issue = [&](int kt) {
         unsigned char* st = smem + (kt % ST) * (C::W + C::X);
         kt += turn;
@@ -397,7 +404,8 @@ __global__ void __launch_bounds__(256, 2) moe_gemm_kernel(const uint16_t* __rest
 // its tiles on the slab loop of chronos_slab.h.  Bound by the matrix cores and the padding of every expert's last tile.
 // Results through the wave's 4 KiB of LDS, 16 rows at a time, so that a store instruction writes whole lines: 16 lanes a row (8 for a
 // gated unit's 64 columns); registers as in moe_store, row r's 16-byte piece c at c ^ (r % pieces).
-template <bool GATHER, int ACT>
+// TURNED (moe_turn): instances of their own (asked at run time, 16 gated experts of 2048 x 1024, 8192 tokens: 415 -> 436).
+template <bool GATHER, int ACT, bool TURNED>
 __global__ void __launch_bounds__(256, 1) moe_gemm256_kernel(const uint16_t* __restrict__ x, uint32_t xbytes,
                                                              const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
                                                              const int32_t* __restrict__ meta, int maxTiles, int top, int N,
@@ -409,10 +417,12 @@ __global__ void __launch_bounds__(256, 1) moe_gemm256_kernel(const uint16_t* __r
     const int32_t* row_item = meta + 1 + maxTiles;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wn = wave >> 1, wm = wave & 1, in = lane >> 3, pc = (lane & 7) ^ in;
+    int expert = 0;   // of the last tile that off was asked for
     auto off = [&](auto NMC, int id, int m, uint32_t (&wv)[8], auto& xv, const void*& wb) {
         constexpr int NM = decltype(NMC)::value;
         const int tile = id / nt, tn = id - tile * nt;
-        wb = w + (int64_t)__builtin_amdgcn_readfirstlane(meta[1 + tile]) * N * K;
+        expert = meta[1 + tile];
+        wb = w + (int64_t)__builtin_amdgcn_readfirstlane(expert) * N * K;
 #pragma unroll
         for (int i = 0; i < 8; ++i) wv[i] = moe_weight_offset(tn, 2 * wave + (i >> 2), i & 3, lane, N, K);
 #pragma unroll
@@ -471,7 +481,11 @@ __global__ void __launch_bounds__(256, 1) moe_gemm256_kernel(const uint16_t* __r
                     *reinterpret_cast<u16x8*>(y + (int64_t)(m0 + 16 * t + RPS * k + rr) * ld + n) = v[k];
         }
     };
-    slab_run<false>(smem, meta[0] * nt, 0, K / 64, x, (int)xbytes, (int)((uint32_t)N * K * 2), off, [](auto, int, int) {}, epi);
+    auto run = [&](const auto& turn) {
+        slab_run<false>(smem, meta[0] * nt, 0, K / 64, x, (int)xbytes, (int)((uint32_t)N * K * 2), off, [](auto, int, int) {}, epi, turn);
+    };
+    if constexpr (TURNED) run([&](int id) { return moe_turn(__builtin_amdgcn_readfirstlane(expert), id % nt, K / 64); });
+    else run(SlabFirst{});
 }
 
 // An index of E and above is an identity expert (its output is the token itself) where the experts' layer has such
@@ -569,18 +583,22 @@ constexpr int64_t kOnceBytes = 256 << 20;
 template <int TM, bool GATHER, int ACT, bool PLACE = false>
 static void moe_gemm(const uint16_t* x, int64_t rows, const uint16_t* w, uint16_t* y, int32_t* meta, int maxTiles, int top, int N, int K,
                      float limit, float slope, float shift, hipStream_t s, const int32_t* idx = nullptr, int items = 0, int E = 0) {
+    // weights that come from memory, all experts' and not the chosen ones', whose number is the batch's (below, out of a cache: 2 to 4 % slower turned, 16
+    // gated experts of 2048 x 1024 39.5 -> 40.7; few chosen of large ones: no slower, one token of 128 x 2048 x 1024 32.7, of 32 x 4096 x 2048 52 -> 51)
+    const bool turned = (int64_t)E * N * K * 2 >= kOnceBytes;
     if constexpr (TM == 256) {
-        const auto kern = hy::moe_gemm256_kernel<GATHER, ACT>;
-        constexpr int lds = kSlabLds;
-        static const hipError_t once = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        (void)once;
-        kern<<<kSlabCUs, 256, lds, s>>>(x, (uint32_t)(rows * K * 2), w, y, meta, maxTiles, top, N, K, limit, slope, shift);
+        auto go = [&](auto kern) {
+            static const hipError_t once = moe_lds(kern, kSlabLds);
+            (void)once;
+            kern<<<kSlabCUs, 256, kSlabLds, s>>>(x, (uint32_t)(rows * K * 2), w, y, meta, maxTiles, top, N, K, limit, slope, shift);
+        };
+        if (turned) go(hy::moe_gemm256_kernel<GATHER, ACT, true>);
+        else go(hy::moe_gemm256_kernel<GATHER, ACT, false>);
     } else {
         constexpr int lds = hy::Tile<TM>::lds;
-        // weights that come from memory (below, out of a cache: 2 to 4 % slower turned, 16 gated experts of 2048 x 1024 39.5 -> 40.7)
         const bool large = std::min<int64_t>(items, E) * N * K * 2 >= kOnceBytes;
         auto go = [&](auto kern) {
-            kern<<<maxTiles * (N / hy::Tile<TM>::TN), 256, lds, s>>>(x, w, y, meta, maxTiles, top, N, K, limit, slope, shift, idx, items, E, large);
+            kern<<<maxTiles * (N / hy::Tile<TM>::TN), 256, lds, s>>>(x, w, y, meta, maxTiles, top, N, K, limit, slope, shift, idx, items, E, turned);
         };
         if constexpr (TM <= 64)
             if (large && items <= (TM == 32 ? 20 : 52) * E) {

@@ -179,16 +179,22 @@ template <bool PAIR> struct SlabRow {   // byte offset of the wave's W block b; 
     constexpr int operator()(int b) const { return 128 * (!PAIR || b < 4 ? 16 * b : 128 + 16 * (b - 4)); }
 };
 
+struct SlabFirst {   // all tiles start with slab 0
+    __device__ __forceinline__ int operator()(int) const { return 0; }
+};
+
 // The tiles of one workgroup, one after the other without a pause of the slab pipeline: the pieces that a tile's last two slabs issue are
 // those of the next tile's first two, which land while this tile's results are stored.  Tile v of the launch goes to workgroup
 // v % gridDim.x (gridDim.x = slab_grid(T, tail)); xcd_remap gives neighbouring tiles to the same XCD.
 // NMX < 8: tiles of 256 W rows by 32 NMX x rows, all alike (T of them, no tail).
 //   off(NM, tile, m, wv, xv, wb): byte offsets of the lane's rows of slab 0 (x rows from row m of the tile on) and the W matrix
+//   turn(tile): the slab that a tile starts with, asked once off was for the same tile; it takes them round from there
 //   rows(NM, tile, m): called before a tile's first slab, for what its epilogue needs of its rows
 //   epi(NM, tile, m, acc): store the results (rows: the wave's 4 KiB of LDS)
-template <bool PAIR, int NMX = 8, class Off, class Rows, class Epi>
+template <bool PAIR, int NMX = 8, class Off, class Rows, class Epi, class Turn = SlabFirst>
 __device__ __forceinline__ void slab_run(unsigned char* smem, int T, int tail, int NS, const void* x, int xbytes, int wbytes, const Off& off,
-                                         const Rows& rows, const Epi& epi) {
+                                         const Rows& rows, const Epi& epi, const Turn& turn = {}) {
+    constexpr bool TURN = !std::is_same_v<Turn, SlabFirst>;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wn = wave >> 1, wm = wave & 1, ln = lane & 15, g = lane >> 4, G = gridDim.x;
     const int ch0 = (g ^ (ln & 7)) * 16, ch1 = ((4 + g) ^ (ln & 7)) * 16;   // (16-row blocks: the swizzle depends on ln only)
@@ -203,18 +209,24 @@ __device__ __forceinline__ void slab_run(unsigned char* smem, int T, int tail, i
         const uint32_t ldw = lds + wave * 8192, ldx = lds + kSlabImg + wave * (1024 * NM);
         uint32_t xv[NM], nwv[8], nxv[NM];
         const void* nwb = nullptr;
-        int v = first, dv = v, dj = 0;   // the tile in work; tile and slab whose pieces are issued
+        int v = first, dv = v, dj = 0;   // the tile in work; tile and slab (its number in the tile's order) whose pieces are issued
+        int t0 = 0;                      // TURN: that tile's first
         auto next = [&]() {
             if (++dj < NS) return;
             if (dv + G >= count) { dj = NS - 1; return; }   // (nobody reads these)
             dv += G;
             dj = 0;
+            if constexpr (TURN) t0 = __builtin_amdgcn_readfirstlane(turn(tile_of(dv)));   // (not sooner: what off asked memory for comes behind the pieces)
             wb = nwb;
 #pragma unroll
             for (int i = 0; i < 8; ++i) wv[i] = nwv[i];
 #pragma unroll
             for (int i = 0; i < NM; ++i) xv[i] = nxv[i];
             if (NS == 1 && dv + G < count) off(NMC, tile_of(dv + G), m_of(dv + G), nwv, nxv, nwb);   // (the next slab is the next tile's)
+        };
+        auto at = [&]() {   // where that slab lies in a row, bytes (an offset that went along with dj cost 35 moves a slab, 4 %)
+            const int j = TURN ? dj + t0 : dj;
+            return (TURN && j >= NS ? j - NS : j) * 128;
         };
         uint32_t pw = ldw, px = ldx;   // where the pieces of the slab in work go
         auto dst = [&](auto IC) {
@@ -223,8 +235,8 @@ __device__ __forceinline__ void slab_run(unsigned char* smem, int T, int tail, i
         };
         auto go = [&](auto IC) {
             constexpr int p = decltype(IC)::value;
-            if constexpr (p < NM) lg_dma_go(x, xbytes, xv[p], dj * 128);
-            else lg_dma_go(wb, wbytes, wv[p - NM], dj * 128);
+            if constexpr (p < NM) lg_dma_go(x, xbytes, xv[p], at());
+            else lg_dma_go(wb, wbytes, wv[p - NM], at());
         };
         auto all = [&](auto IC) {
             dst(IC);
@@ -235,6 +247,7 @@ __device__ __forceinline__ void slab_run(unsigned char* smem, int T, int tail, i
             if (u < count) off(NMC, tile_of(u), m_of(u), nwv, nxv, nwb);
         };
         off(NMC, tile_of(v), m_of(v), wv, xv, wb);
+        if constexpr (TURN) t0 = __builtin_amdgcn_readfirstlane(turn(tile_of(v)));
         lg_static_for(all, std::make_integer_sequence<int, 8 + NM>{});
         after(v + G);
         next();

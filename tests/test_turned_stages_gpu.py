@@ -44,24 +44,31 @@ def test_sums_of_up_to_eight_rows_keep_their_order(cfg, rows):
         assert torch.equal(y, all_rows[:m])
 
 
-# k-steps of the two products: 2 and 256 (fewer and more than the ring holds), 30 and 32; tiles of 32, 64 and 128 rows
+# k-steps of the two products: 2 and 256 (fewer and more than the ring holds), 30 and 32.  Batches of tiles of 32, 64, 128 and (not of 128 wide ones) 256 rows, placed in
+# the first product and by a launch, on both sides of where the chosen experts' weights are 256 MB
+@pytest.mark.parametrize("form", ["gelu", "glu"])
 @pytest.mark.parametrize("d,F", [(128, 16384), (1920, 2048)])
-@pytest.mark.parametrize("T", [5, 60, 300, 900])
-def test_turned_experts(d, F, T):
+def test_turned_experts(d, F, form):
     """moe_grouped.hip's tiles over experts' weights of 256 MB and more, against the PyTorch reference (tolerance of the other expert tests), and a
     token's result whatever else is in the batch."""
     from chronos.ops import hybrid as hops, hybrid_ref as ref
 
-    E, top, bf = 80, 8, torch.bfloat16
+    E, top, bf, T = 80, 8, torch.bfloat16, 4000
     assert E * F * d * 2 >= 1 << 28
     g = torch.Generator(device=DEV).manual_seed(T + d)
     rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
-    h, wt = rnd(T + 11, d).to(bf), torch.rand(T + 11, top, device=DEV, generator=g)
-    idx = torch.rand(T + 11, E, device=DEV, generator=g).topk(top, -1).indices.int()
-    idx[:10] = torch.arange(E, device=DEV).view(10, top)      # (every expert has an item, so both batches below take the same tiles)
-    wu, wd = (rnd(E, F, d) * d ** -0.5).to(bf), (rnd(E, d, F) * F ** -0.5).to(bf)
-    more = hops.moe_ffn(h, idx, wt, wu, wd, 1, bf)
-    want = ref.moe_ffn(h, idx, wt, wu, wd, 1, bf).float()
-    assert (more.float() - want).abs().max() <= 1.5e-2 * want.abs().max()
-    n = max(T, 10)
-    assert torch.equal(hops.moe_ffn(h[:n].contiguous(), idx[:n].contiguous(), wt[:n].contiguous(), wu, wd, 1, bf), more[:n])
+    h, wt = rnd(T, d).to(bf), torch.rand(T, top, device=DEV, generator=g)
+    idx = torch.rand(T, E, device=DEV, generator=g).topk(top, -1).indices.int()
+    wu, wd = (rnd(E, F * (2 if form == "glu" else 1), d) * d ** -0.5).to(bf), (rnd(E, d, F) * F ** -0.5).to(bf)
+    if form == "glu":
+        order = hops.moe_glu_row_order(F).to(DEV)
+        tiled = wu[:, order].contiguous()
+        run = lambda n: hops.moe_glu_ffn(h[:n].contiguous(), idx[:n].contiguous(), wt[:n].contiguous(), tiled, wd, 7.0, 1.702, 1.0, bf, True)  # noqa: E731
+        want = ref.moe_glu_ffn(h[:200], idx[:200], wt[:200], wu, wd, 7.0, 1.702, 1.0, bf).float()
+    else:
+        run = lambda n: hops.moe_ffn(h[:n].contiguous(), idx[:n].contiguous(), wt[:n].contiguous(), wu, wd, 1, bf)  # noqa: E731
+        want = ref.moe_ffn(h[:200], idx[:200], wt[:200], wu, wd, 1, bf).float()
+    whole = run(T)
+    assert (whole[:200].float() - want).abs().max() <= 1.5e-2 * want.abs().max()
+    for n in (1, 2, 3, 9, 10, 60, 130, 300, 450, 900, 1800, 2500):
+        assert torch.equal(run(n), whole[:n]), n
