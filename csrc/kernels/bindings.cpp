@@ -584,7 +584,7 @@ static int32_t* split_tickets(const Tensor& x, int64_t n, Tensor& own) {
 //   scale rsqrt(sum(part_in[m]) / K + eps).  cfg = tile config (gemm_pp_bm / gemm_pp_bn), splitk divides K / 64.
 std::tuple<Tensor, Tensor> gemm_pp(const Tensor& x, const Tensor& w, int64_t mode, int64_t cfg, int64_t splitk,
                                    const c10::optional<Tensor>& resid, const c10::optional<Tensor>& part_in,
-                                   double eps, bool prio) {
+                                   double eps, bool prio, bool in_order) {
     chk_bf16(x, "x");
     chk_bf16(w, "w");
     const int64_t K = x.size(-1), M = x.numel() / K, N = w.size(0);
@@ -621,9 +621,7 @@ std::tuple<Tensor, Tensor> gemm_pp(const Tensor& x, const Tensor& w, int64_t mod
     a.ablate = chronos::gemm_lg_ablations_built() ? chronos::knob("pp_ablate", 0) : 0;
     a.gm = chronos::knob("pp_gm", 8);  // +7-9 % at M = 16384 (profiles/r3_gemm_tile_order_m16384.jsonl)
     a.handoff = chronos::knob("lg_handoff", -1);
-    // up to 8 rows a layer's sums keep their order: steps of so few rows are the ones over long fp8 caches, whose bytes would follow a last bit of
-    // the stream; the vocabulary's logits are cached nowhere
-    a.turn = M > 8 || N > 65536;
+    a.turn = !in_order;
     Tensor y = at::empty({M, mode == 1 ? N / 2 : N}, x.options());
     a.y = bfm(y);
     Tensor part_out;
@@ -784,7 +782,7 @@ std::tuple<Tensor, Tensor, Tensor> gemm_join(const Tensor& y, const Tensor& x, c
 
 // The float32 slices [splitk, M, N] of a plain product of few rows whose K is split over workgroups, nothing kept between calls: gemm_lg.hip's
 // ring tiles of few rows, gemm_slab.hip (88, two slices and more), or (skinny) gemm_skinny.hip's uneven configs.  Their sum in order, rounded, is the product; one slice is the product unrounded.
-Tensor gemm_slices(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk, bool skinny) {
+Tensor gemm_slices(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk, bool skinny, bool in_order) {
     chk_bf16(x, "x");
     chk_bf16(w, "w");
     const int64_t K = x.size(-1), M = x.numel() / K, N = w.size(0);
@@ -808,7 +806,7 @@ Tensor gemm_slices(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk
     a.splitk = (int)splitk;
     a.kts = (int)(K / 64 / splitk);
     a.gm = chronos::knob("pp_gm", 8);
-    a.turn = 1;
+    a.turn = !in_order;
     Tensor ws = at::empty({splitk, M, N}, x.options().dtype(at::kFloat));
     a.ws = ws.data_ptr<float>();
     CHK(skinny ? chronos::launch_gemm_skinny((int)cfg, 0, false, a, cur_stream()) : chronos::launch_gemm_lg((int)cfg, 0, false, a, cur_stream()),
@@ -888,9 +886,9 @@ Tensor gemv_act(const Tensor& x, const Tensor& w, int64_t mode, double limit, do
     return y;
 }
 
-Tensor gemm_split(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk) {
+Tensor gemm_split(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk, bool in_order) {
     CHK(splitk > 1, "gemm_split: splitk");
-    const Tensor ws = gemm_slices(x, w, cfg, splitk, false);
+    const Tensor ws = gemm_slices(x, w, cfg, splitk, false, in_order);
     c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
     Tensor y = at::empty({ws.size(1), ws.size(2)}, x.options());
     chronos::launch_gemm_slices(ws.data_ptr<float>(), bfm(y), y.numel(), (int)splitk, cur_stream());
@@ -899,7 +897,7 @@ Tensor gemm_split(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk)
 
 // The same product as float32 [M, N]: its sums without the rounding
 Tensor gemm_f32(const Tensor& x, const Tensor& w, int64_t cfg, int64_t splitk, bool skinny) {
-    const Tensor ws = gemm_slices(x, w, cfg, splitk, skinny);
+    const Tensor ws = gemm_slices(x, w, cfg, splitk, skinny, false);
     if (splitk == 1) return ws[0];
     c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
     Tensor y = at::empty({ws.size(1), ws.size(2)}, ws.options());
@@ -1134,10 +1132,10 @@ TORCH_LIBRARY(chronos, m) {
           "float shift) -> (Tensor, Tensor, Tensor)");
     m.def("gemm_ring(Tensor x, Tensor w, int cfg, int splitk, int mode, int n0, int nf, Tensor? bias, float limit, float slope, float shift) -> (Tensor, Tensor)");
     m.def("gemv_act(Tensor x, Tensor w, int mode, float limit, float slope, float shift) -> Tensor");
-    m.def("gemm_split(Tensor x, Tensor w, int cfg, int splitk) -> Tensor");
-    m.def("gemm_slices(Tensor x, Tensor w, int cfg, int splitk, bool skinny) -> Tensor");
+    m.def("gemm_split(Tensor x, Tensor w, int cfg, int splitk, bool in_order=False) -> Tensor");
+    m.def("gemm_slices(Tensor x, Tensor w, int cfg, int splitk, bool skinny, bool in_order=False) -> Tensor");
     m.def("gemm_f32(Tensor x, Tensor w, int cfg, int splitk, bool skinny) -> Tensor");
-    m.def("gemm_pp(Tensor x, Tensor w, int mode, int cfg, int splitk, Tensor? resid, Tensor? part_in, float eps, bool prio) -> (Tensor, Tensor)");
+    m.def("gemm_pp(Tensor x, Tensor w, int mode, int cfg, int splitk, Tensor? resid, Tensor? part_in, float eps, bool prio, bool in_order=False) -> (Tensor, Tensor)");
     m.def("gemm_skinny(Tensor x, Tensor w, int mode, int cfg, int splitk, Tensor? resid, Tensor? part_in, float eps) "
           "-> (Tensor, Tensor)");
     m.def("gemv_resid(Tensor x, Tensor w, Tensor resid_in, Tensor(a!) resid_out, Tensor? ws=None) -> Tensor");

@@ -453,6 +453,9 @@ class KVCache:
         self.dtype = dtype
         per = hkv * block_size * cfg.head_dim
         tdt = torch.uint8 if dtype == "fp8" else torch.bfloat16  # fp8 = OCP e4m3fn bytes + per-layer scale
+        # one-byte pages: a last bit of a layer's products moves whole bytes behind it, so steps over them keep their sums' order (ops.linear's in_order);
+        # 8B layers take 1 us longer so in steps of 2 to 8 rows, 5 us in steps of 16
+        self.bytes = tdt == torch.uint8
         self.buf = torch.zeros(cfg.num_layers, 2, num_blocks, per, device=device, dtype=tdt)
         self.k_scale = [float(k_scale)] * cfg.num_layers
         self.v_scale = [float(v_scale)] * cfg.num_layers
@@ -638,8 +641,8 @@ class LlamaModel:
         T = st["T"]
         if (_FUSE_NORM and self.w.norms_folded and self.tp.world == 1 and x.is_cuda and st["sb"].cp is None
                 and (st["sb"].tiles is None or T > 2) and ops.resid_ok(T, w.shape[0], w.shape[1], ops.is_q(w))):
-            return ops.gemv_resid(x, w, st["resid"])
-        return ops.linear(x, w)
+            return ops.gemv_resid(x, w, st["resid"], st["in_order"])
+        return ops.linear(x, w, in_order=st["in_order"])
 
     def _attn_rows(self, li: int, qkv: torch.Tensor, sb: StepBatch, q_buf: torch.Tensor, kv: KVCache) -> torch.Tensor:
         """RoPE + paged-KV write + attention for the rows of one step batch (prefill tiles or decode rows)."""
@@ -688,7 +691,7 @@ class LlamaModel:
         else:
             # a LazyNorm input goes straight to the projection (the batched GEMM applies the folded norm as a row
             # scale; anything else materialises it)
-            qkv = ops.qlinear(*x, lw.wqkv.q, lw.wqkv.s) if q8 else ops.linear(x, lw.wqkv)
+            qkv = ops.qlinear(*x, lw.wqkv.q, lw.wqkv.s) if q8 else ops.linear(x, lw.wqkv, in_order=st["in_order"])
             if sb.dec is None:
                 attn = self._attn_rows(li, qkv, sb, st["q_buf"], kv)
             else:
@@ -704,7 +707,7 @@ class LlamaModel:
         x = st["x"]
         if self.w.fp8 and not st.get("w16"):
             return ops.qlinear(*ops.qgate_up_quant(*x, lw.w_gu.q, lw.w_gu.s), lw.w_down.q, lw.w_down.s)
-        return self._out_proj(ops.gate_up_silu(x, lw.w_gu), lw.w_down, st)
+        return self._out_proj(ops.gate_up_silu(x, lw.w_gu, st["in_order"]), lw.w_down, st)
 
     def _forward_sp(self, sb: StepBatch, kv: KVCache, logits_dtype) -> torch.Tensor:
         """TP prefill with sequence parallelism (SURVEY.md §2.5 "Sequence parallel"): every row-parallel output is
@@ -718,7 +721,7 @@ class LlamaModel:
         eps = cfg.rms_eps
         emb = ops.embedding(sb.ids, w.embed, w.vocab_start)
         resid = tp.reduce_scatter_rows(_pad_rows(emb, Tp))  # vocab-parallel embedding: partial rows -> shard
-        st = dict(sb=sb, T=T, resid=resid, q_buf=torch.empty(T, self.hq, cfg.head_dim, device=emb.device,
+        st = dict(sb=sb, T=T, resid=resid, in_order=kv.bytes, q_buf=torch.empty(T, self.hq, cfg.head_dim, device=emb.device,
                                                              dtype=emb.dtype))
         xs = ops.rmsnorm(resid, w.layers[0].attn_norm, eps)
         L = len(w.layers)
@@ -779,7 +782,7 @@ class LlamaModel:
         for p in self._decode_halves(sb):
             h = tp.all_reduce(ops.embedding(p.ids, w.embed, w.vocab_start))
             T = p.ids.numel()
-            st = dict(sb=p, T=T, resid=h, q_buf=torch.empty(T, self.hq, cfg.head_dim, device=h.device, dtype=h.dtype))
+            st = dict(sb=p, T=T, resid=h, in_order=kv.bytes, q_buf=torch.empty(T, self.hq, cfg.head_dim, device=h.device, dtype=h.dtype))
             st["x"] = self._norm(h, st, w.layers[0].attn_norm, first=True)
             states.append(st)
         L = len(w.layers)
@@ -844,7 +847,7 @@ class LlamaModel:
             ids = p.ids if p.dec is None else torch.cat([p.ids, p.dec.ids])
             h = tp.all_reduce(ops.embedding(ids, w.embed, w.vocab_start))
             T = ids.numel()
-            st = dict(sb=p, T=T, resid=h, q_buf=torch.empty(T, self.hq, cfg.head_dim, device=h.device, dtype=h.dtype),
+            st = dict(sb=p, T=T, resid=h, in_order=kv.bytes, q_buf=torch.empty(T, self.hq, cfg.head_dim, device=h.device, dtype=h.dtype),
                       w16=(w.fp8 and _W8A16_DECODE and T <= 2 and h.is_cuda and p.cp is None and p.dec is None
                            and cfg.hidden_size % 1024 == 0))
             st["x"] = self._norm(h, st, w.layers[0].attn_norm, first=True)

@@ -58,3 +58,21 @@ def test_fp8_model_and_engine_cpu():
     eng.run_until_idle()
     for r in reqs:
         assert {"risk_score", "verdict", "reason"} <= set(json.loads(r.text))
+
+
+def test_steps_over_fp8_pages_keep_their_sums_order(monkeypatch):
+    """Layer products in front of one-byte pages ask for sums in order, whatever the number of rows; those over bfloat16 pages, and the head, do not."""
+    from chronos import ops
+    from chronos.models.llama import build_model
+
+    m = build_model("tiny", "cpu")
+    asked = []
+    linear, gate = ops.linear, ops.gate_up_silu
+    monkeypatch.setattr(ops, "linear", lambda x, w, out=None, in_order=False: asked.append((w is m.w.lm_head, in_order)) or linear(x, w, out, in_order))
+    monkeypatch.setattr(ops, "gate_up_silu", lambda x, w, in_order=False: asked.append((False, in_order)) or gate(x, w, in_order))
+    for dtype in ("fp8", "bf16"):
+        for rows in (1, 3, 12):
+            del asked[:]
+            kv = m.make_cache(rows + 1, 16, rows, dtype)
+            m.forward(m.prefill_batch([[1]] * rows, [0] * rows, [[1 + i] for i in range(rows)]), kv)
+            assert len(asked) == 4 * m.cfg.num_layers + 1 and all(order == (dtype == "fp8" and not head) for head, order in asked)

@@ -1,47 +1,79 @@
-"""gemm_lg.hip's ring tiles of one x tile, whose workgroups start their K at different stages: every stage is taken once, whatever their number."""
+"""Tiles that take K round from a place of their own: gemm_lg.hip's ring tiles of one x tile (stages), moe_grouped.hip's over large weights (k-steps).  Every stage
+is taken once, whatever their number."""
 import pytest
 import torch
 
 DEV = "cuda"
 pytestmark = pytest.mark.gpu
 
+# ring tiles of at most 128 x rows whose pieces fill their waves, and those of 256 rows; 14, 18 and 12 take K in 32s
+RING = [(72, (2, 8, 9, 32)), (74, (2, 7, 31)), (75, (16, 31)), (79, (5, 32)), (38, (33, 64)), (39, (8, 64)), (32, (65, 128)), (19, (100,)), (15, (128,)), (29, (40, 128)),
+        (30, (129, 256)), (35, (200,)), (14, (137,)), (18, (256,)), (12, (250,))]
 
-# stages per slice (K / 64 / split): one, fewer than the ring holds, as many, one more, odd, many; N: a part tile, one round, more workgroups than
-# stages on every XCD, ragged
-@pytest.mark.parametrize("cfg,rows", [(72, (9, 32)), (75, (16, 31)), (79, (32,)), (38, (33, 64)), (39, (64,)), (32, (65, 128)), (19, (100,)), (15, (128,)), (29, (40, 128))])
-@pytest.mark.parametrize("k,split", [(64, 1), (192, 1), (512, 2), (576, 1), (832, 1), (4096, 1)])
-@pytest.mark.parametrize("n", [16, 4100, 70656])
+
+def _operands(m, n, k, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return g, torch.randn(m, k, device=DEV, generator=g).to(torch.bfloat16), (torch.randn(n, k, device=DEV, generator=g) * k ** -0.5).to(torch.bfloat16)
+
+
+# stages per slice (K / 64 / split): 64, 65, one, 9 (more and fewer than rings of 4 to 12 hold), 11, 43, 172; N: a part tile, ragged, more workgroups than stages
+@pytest.mark.parametrize("cfg,rows", RING)
+@pytest.mark.parametrize("k,split", [(4096, 1), (4160, 1), (4096, 64), (4608, 8), (5632, 8), (11008, 4), (11008, 1)])
+@pytest.mark.parametrize("n", [16, 4100, 20004])
 def test_turned_products(cfg, rows, k, split, n):
     from chronos import ops
 
     ops.load()
-    g = torch.Generator(device=DEV).manual_seed(cfg + k + n)
-    w = torch.randn(n, k, device=DEV, generator=g).to(torch.bfloat16)
     for m in rows:
-        x = torch.randn(m, k, device=DEV, generator=g).to(torch.bfloat16)
+        _, x, w = _operands(m, n, k, cfg + k + n)
         want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
         # float32 sums of exact products in any order: half a last place of the largest partial sum for each of k terms
-        if cfg in (72, 75, 79, 38, 39, 32, 19):
+        if cfg in (72, 74, 75, 79, 38, 39, 32, 19):
             y = torch.ops.chronos.gemm_slices(x, w, cfg, split, False)
             assert ((y.double().sum(0) - want).abs() <= size * k * 2 ** -24).all()
-        if split == 1 and n % 4 == 0:
+        if split == 1:
             y, _ = torch.ops.chronos.gemm_pp(x, w, 0, cfg, 1, None, None, 1e-5, False)
             assert ((y.double() - want).abs() <= want.abs() * 2 ** -8 + size * k * 2 ** -24).all()
 
 
-@pytest.mark.parametrize("cfg,rows", [(74, (2, 8)), (72, (3, 8))])
-def test_sums_of_up_to_eight_rows_keep_their_order(cfg, rows):
-    """A layer's product of up to 8 rows has the bits of the same rows among 64 on a kernel that is not turned (two x tiles)."""
+@pytest.mark.parametrize("cfg,rows", RING)
+@pytest.mark.parametrize("k", [4096, 4672])
+def test_turned_epilogues(cfg, rows, k):
+    """Gated units behind a folded norm, and residuals with their partial sums: as in order but for last bits of the sums."""
     from chronos import ops
 
     ops.load()
-    g = torch.Generator(device=DEV).manual_seed(cfg)
-    w = torch.randn(28672, 4096, device=DEV, generator=g).to(torch.bfloat16)
-    x = torch.randn(64, 4096, device=DEV, generator=g).to(torch.bfloat16)
-    all_rows, _ = torch.ops.chronos.gemm_pp(x, w, 0, cfg, 1, None, None, 1e-5, False)
+    n = 1536
     for m in rows:
-        y, _ = torch.ops.chronos.gemm_pp(x[:m].contiguous(), w, 0, cfg, 1, None, None, 1e-5, False)
-        assert torch.equal(y, all_rows[:m])
+        g, x, w = _operands(m, n, k, cfg + m)
+        r = torch.randn(m, n, device=DEV, generator=g).to(torch.bfloat16)
+        part = (x.float() ** 2).view(m, 64, -1).sum(-1)
+        for mode, res, pt in ((1, None, part), (0, None, part), (2, r, None)):
+            a, b = (torch.ops.chronos.gemm_pp(x, w, mode, cfg, 1, res, pt, 1e-5, False, in_order) for in_order in (False, True))
+            # sums of variance 1: float32 orders move them by less than 2e-5 (a sum with a normal number, a gated unit: 3 times that), so that values are the same or, where
+            # the sum lies that close to a boundary, a bfloat16 step apart, at most 2^-7 of the value.  Gated units round gate, sigmoid's product and up number: a step
+            # (2^-8 to 2^-7) of each, the gate's times the unit's relative slope 1 + g (1 - sigmoid(g)), 5 at g = -6: 8 steps of 2^-8 in all.  A residual's product is rounded by itself
+            # before the sum (of at most |r| + |sum|)
+            d, mag = (a[0].float() - b[0].float()).abs(), torch.maximum(a[0].float().abs(), b[0].float().abs())
+            mag = 4 * mag if mode == 1 else mag if mode == 0 else 2 * mag + r.float().abs()
+            assert (d <= mag * 2 ** -7 + 6e-5).all() and float((d > 0).float().mean()) < 0.05
+            if mode == 2:
+                assert ((a[1] - b[1]).abs() <= 0.02 * b[1].abs() + 1e-3).all()
+
+
+@pytest.mark.parametrize("cfg,rows", [(74, (2, 8)), (72, (3, 8, 30)), (38, (64,))])
+def test_sums_in_order(cfg, rows):
+    """in_order: a product's rows have the bits of the same rows among 128 on a kernel that is never turned (several x tiles); without it they are turned."""
+    from chronos import ops
+    from chronos.ops import gemm as G
+
+    ops.load()
+    _, x, w = _operands(128, 28672, 4096, cfg)
+    all_rows = G.pp_gemm(x, w, 0, (cfg, 1))[0]
+    for m in rows:
+        xs = x[:m].contiguous()
+        assert torch.equal(G.pp_gemm(xs, w, 0, (cfg, 1), in_order=True)[0], all_rows[:m])
+        assert not torch.equal(G.pp_gemm(xs, w, 0, (cfg, 1))[0], all_rows[:m])
 
 
 # k-steps of the two products: 2 and 256 (fewer and more than the ring holds), 30 and 32.  Batches of tiles of 32, 64, 128 and (not of 128 wide ones) 256 rows, placed in
