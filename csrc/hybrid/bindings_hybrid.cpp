@@ -1273,6 +1273,12 @@ TORCH_LIBRARY_FRAGMENT(chronos, m) {
     m.def("hy_head_few_rows(int T, int N, int H, int K) -> int", [](int64_t T, int64_t N, int64_t H, int64_t K) { return (int64_t)chronos::hy_head_few_rows((int)T, (int)N, (int)H, (int)K); });
     m.def("hy_moe_route_one(int T, int N, int d) -> bool", [](int64_t T, int64_t N, int64_t d) { return chronos::hy_moe_route_one((int)T, (int)N, (int)d); });
     m.def("hy_latent_nsplit(int wgs, int max_ctx, bool windowed, int rank) -> int", [](int64_t w, int64_t c, bool win, int64_t r) { return (int64_t)chronos::hy_latent_nsplit((int)w, (int)c, win, (int)r); });
+    m.def("hy_window_nsplit(int B, int max_q, int H, int G, int D, int Dv, int window, int keep, int max_ctx) -> int",
+          [](int64_t B, int64_t q, int64_t H, int64_t G, int64_t D, int64_t Dv, int64_t window, int64_t keep, int64_t ctx) {
+              need(B >= 1 && q >= 1 && G >= 1 && H % G == 0 && std::max({B, q, H, D, Dv, window, keep, ctx}) < (1LL << 20), "window_nsplit: sizes");
+              return (int64_t)chronos::hy_window_nsplit(false, (int)(H * D + G * (D + Dv)), (int)(B * q), (int)B, (int)q, (int)H, (int)G, (int)D, (int)Dv, (int)window, (int)keep,
+                                                        0, (int)ctx, 0, false);
+          });
     m.def("hy_moe_tile(int items, int E, int d, int F, int up) -> int", [](int64_t items, int64_t E, int64_t d, int64_t F, int64_t up) {
         need(items >= 0 && E >= 1 && d >= 1 && F >= 1 && up >= 1 && std::max({items, E, d, F, up}) < (1LL << 31), "moe_tile: sizes");
         return (int64_t)chronos::hy_moe_tile((int)items, (int)E, (int)d, (int)F, (int)up);

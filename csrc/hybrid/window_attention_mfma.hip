@@ -437,8 +437,11 @@ bool hy_window_mfma_ok(int ldq, int D, int Dv) { return !(D % 8 || Dv % 16 || D 
 // Splits of a row block's key tiles over workgroups (merged by a combine kernel) for launches that would leave most
 // of the chip idle — decode rows, a lone short portion: enough workgroups to cover the CUs twice (four times for few
 // rows with unit keys, whose workgroups need half the LDS), at least 2 key tiles per split, at most 16; of up to 16 rows a head, whose time is a
-// workgroup's chain of latencies, one tile per split up to ten (decode steps with two such layers, us, width 1024, two tiles -> one: one row at 100, 200 and 700
-// tokens 142.9 -> 140.0, 143.3 -> 140.7, 144.1 -> 143.0, 4 at 700 157.4 -> 155.1, 16 and 60 level; of all tiles of windows of 1024 one row 216.5 -> 219.6).  Prompt portions (more than 64
+// workgroup's chain of latencies, one tile per split from four tiles, where there are partials to combine anyway, to sixteen, beyond which some workgroups would have
+// two.  Decode steps with two such layers, us, two tiles -> one: width 1024, one row at 60 tokens (two and three tiles) 138.2 -> 139.4, 100 142.9 -> 140.2, 450
+// 143.9 -> 140.8, 700 and 1000 144.1 -> 142.6, 4 at 200 155.7 -> 152.9; width 2048, 200 and 700 tokens 212.1 -> 210.0, 215.8 -> 213.5.  The attention by itself,
+// 11 to 16 tiles 11.6 - 12.2 -> 10.9 - 11.7, in ten splits 12.2 - 12.7; 18 tiles in sixteen splits 13.7 for 12.5 (profiles/window_decode_splits.json, replayed by
+// tests/test_measured_rules.py).  Prompt portions (more than 64
 // rows) write and read far more partials than decode rows: only where a walk's tiles weigh more than all rows' partials, 1000 (token, head)
 // rows a tile, all of the step's tokens counted and not its longest portion's, which a mixed step's decode rows do not have.  us, split /
 // not: 8 heads, 2 of keys, 8 x 300 tokens (19200 rows, 5 tiles) 32 / 19, 21 x 117 (3) 26 / 12, 1 x 700 (5600, 11) 22 / 30; 300 tokens beside 8 decode
@@ -458,7 +461,7 @@ int hy_window_nsplit(bool f32, int ldq, int T, int B, int max_q, int H, int G, i
     const int tiles = span / hy::WKT + 1 + (window > 0 ? (std::min(keep, max_ctx) + hy::WKT - 1) / hy::WKT : 0) +
                       (window > 0 && pool > 0 ? (max_ctx / pool + hy::WKT - 1) / hy::WKT : 0);
     int want = (enough + wgs - 1) / wgs;
-    want = std::min(want, std::min(16, rows <= 16 ? std::max(tiles / 2, std::min(tiles, 10)) : rows <= 64 || (int64_t)T * H <= 1000LL * tiles ? tiles / 2 : 1));
+    want = std::min(want, std::min(16, rows <= 16 && tiles >= 4 && tiles <= 16 ? tiles : rows <= 64 || (int64_t)T * H <= 1000LL * tiles ? tiles / 2 : 1));
     return want < 1 ? 1 : want;
 }
 

@@ -155,6 +155,28 @@ def test_tiles_of_experts():
     assert _mean(before) >= 1.08 and _slower(before) <= 27 and min(before) >= 1 / 1.23
 
 
+def test_splits_of_windowed_decode_rows():
+    """A key tile per split or two: the pick is no slower than the other by more than 3 %, and than ten splits with some workgroups on two tiles."""
+    import torch
+
+    from chronos.ops import hybrid as hops
+
+    hops.load()
+    picks = set()
+    for H, G, window, keep, B, ctx, two, ten, one in _table("window_decode_splits.json")["rows"]:
+        tiles = min(ctx, window + 1) // 64 + 1 + (keep > 0) if window else ctx // 64 + 1
+        splits = torch.ops.chronos.hy_window_nsplit(B, 1, H, G, 128, 128, window, keep, ctx)
+        wgs = B * G
+        assert splits == max(1, min(-(-512 // wgs), 16, tiles if 4 <= tiles <= 16 else tiles // 2))
+        picks.add((tiles, splits))
+        us = one if 4 <= tiles <= 16 else two
+        # (17 to 21 tiles: one that is left over costs two per split a round; sixteen splits gain there and lose from 17 on)
+        assert us <= 1.035 * min(two, ten, one) or 16 < tiles <= 21, (H, G, window, B, ctx)
+    assert len(picks) >= 12
+    steps = _table("window_decode_splits.json")["steps"]["rows"]
+    assert all((one < two) == (tokens > 60) for width, B, tokens, two, one in steps if width == "1k")
+
+
 def _lines(key, pick, least):
     """Every measured pair of forms: what the rule picks is not slower than the other form by more than `least`."""
     for r in _rows(_table("decode_forms.json")[key]):

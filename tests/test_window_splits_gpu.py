@@ -6,8 +6,8 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-# lengths around a tile's edges, more tiles than single splits, splits without a key; windows and kept tokens in other tiles
-@pytest.mark.parametrize("lens", [[1], [64], [65], [200], [640], [641, 3], [700, 64, 129], [1500]])
+# lengths around a tile's edges, 3 and 4 tiles, 16 and 17, splits without a key; windows and kept tokens in other tiles
+@pytest.mark.parametrize("lens", [[1], [64], [65], [130], [191], [192], [200], [640], [641, 3], [700, 64, 129], [960], [1023], [1024, 30], [1500]])
 @pytest.mark.parametrize("window,keep", [(0, 0), (512, 4), (100, 70)])
 def test_decode_rows(lens, window, keep):
     from chronos.ops import hybrid as hops, hybrid_ref as ref
