@@ -37,6 +37,7 @@
 // with the tiles ahead 270.
 // One and two waves per workgroup: 436 and 302 us where four took 233 (of 171, before addresses, weights and stores lost
 // their branches).
+#include "chronos_lds.h"
 #include "chunk_common.h"
 
 #include <algorithm>
@@ -913,9 +914,8 @@ template <int D, int MODE, bool STATE, bool PRE = false>
 static void chunk_scan_pass(const hy::ChunkScan& a, int segs, hipStream_t s) {
     constexpr int lds = hy::ChunkLds<D, MODE, PRE>::SIZE;
     static_assert(lds <= 160 * 1024, "LDS of one workgroup");
-    const auto kern = hy::chunk_scan_kernel<D, MODE, STATE, PRE>;
-    static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    (void)set;
+    constexpr auto kern = hy::chunk_scan_kernel<D, MODE, STATE, PRE>;
+    lds_limit<kern>(lds);
     const int nslab = (a.Dv + 16 * hy::kCW - 1) / (16 * hy::kCW);
     kern<<<dim3((a.B * a.H + 7) / 8 * 8 * nslab, segs), 64 * hy::kCW, lds, s>>>(a);
 }
@@ -925,9 +925,8 @@ static void chunk_scan_run(const hy::ChunkScan& a, hipStream_t s) {
         if (a.segs > 1) chunk_scan_pass<D, MODE, true>(a, a.segs - 1, s);
     } else if (a.tiles != nullptr) {
         constexpr int lds = 4 * hy::kCH * D + 8192 + 4 * 1024;
-        const auto kern = hy::delta_tiles_kernel<D>;
-        static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        (void)set;
+        constexpr auto kern = hy::delta_tiles_kernel<D>;
+        lds_limit<kern>(lds);
         kern<<<(unsigned)(hy::delta_slots(a.T, a.B) * a.H), 256, lds, s>>>(a);
         return chunk_scan_pass<D, MODE, false, true>(a, a.segs, s);
     }

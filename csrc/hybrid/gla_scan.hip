@@ -20,6 +20,7 @@
 // token 988 us, this 375; one of 4000, 8 heads: 1684 and 694, in eight segments 172.  P on the vector ALUs from running products: 648 us, and the same
 // with F in float32: state 9.6e-8 of its norm off the float64 recurrence (token by token 8.7e-8, this 7.8e-8); with the stores of a
 // chunk waited for by the next: 482 us, with that 448, and the terms rounded in pairs 403 (382 as measured for the 375).
+#include "chronos_lds.h"
 #include "chunk_common.h"
 
 #include <type_traits>
@@ -776,14 +777,12 @@ static void gla_scan_pass(const hy::GlaScan& a, int segs, hipStream_t s) {
     if (a.tiles != nullptr) {
         using M = hy::GlaWalkLds<D>;
         static_assert(M::SIZE <= 160 * 1024 && D <= 64 * M::NW, "LDS of one workgroup, a row per thread");
-        static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(hy::gla_walk_kernel<D, STATE>), hipFuncAttributeMaxDynamicSharedMemorySize, M::SIZE);
-        (void)set;
+        lds_limit<hy::gla_walk_kernel<D, STATE>>(M::SIZE);
         return go(hy::gla_walk_kernel<D, STATE>, 64 * M::NW, M::SIZE);
     }
     constexpr int lds = hy::GlaLds<D>::SIZE;
     static_assert(lds <= 160 * 1024, "LDS of one workgroup");
-    static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(hy::gla_scan_kernel<D, STATE>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    (void)set;
+    lds_limit<hy::gla_scan_kernel<D, STATE>>(lds);
     go(hy::gla_scan_kernel<D, STATE>, 256, lds);
 }
 template <int D>

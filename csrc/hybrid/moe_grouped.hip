@@ -20,6 +20,7 @@
 // The tile loop is an LDS-DMA ring (16x16x32 bf16 MFMAs, XOR-swizzled images, one barrier per k-step with a counted vmcnt) at
 // two tile sizes, below, and for experts with many tokens the projections' slab walk (chronos_slab.h).  Needs d % 128 == 0 and F % 128 == 0.
 #include "hybrid_common.h"
+#include "chronos_lds.h"
 #include "chronos_slab.h"
 #include "moe_tile.h"
 
@@ -569,10 +570,6 @@ int64_t hy_moe_meta_ints(int items, int E, int tm) {
     return 1 + n + n * tm + items + (int64_t)moe_align_wgs(items) * E;
 }
 
-template <typename F> static hipError_t moe_lds(F kern, int lds) {
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-}
-
 // Weights of the experts chosen (one product's, at most) from which their reads are marked as read once: what the memory-side cache holds.  Below
 // it a decoder of few layers finds them there again.  The whole feed-forward, us, plain -> marked: GELU 4096 wide, 32 experts of 2048, top 4:
 // 4 tokens (268 MB each product) 101 -> 89, 16 204 -> 181, 64 (512 MB) 238 -> 210, 128 239 -> 212, 400 253 -> 231, but 2 tokens 54 -> 62; 2048 wide, 16
@@ -588,10 +585,10 @@ static void moe_gemm(const uint16_t* x, int64_t rows, const uint16_t* w, uint16_
     const bool turned = (int64_t)E * N * K * 2 >= kOnceBytes;
     if constexpr (TM == 256) {
         auto go = [&](auto kern) {
-            static const hipError_t once = moe_lds(kern, kSlabLds);
-            (void)once;
             kern<<<kSlabCUs, 256, kSlabLds, s>>>(x, (uint32_t)(rows * K * 2), w, y, meta, maxTiles, top, N, K, limit, slope, shift);
         };
+        lds_limit<hy::moe_gemm256_kernel<GATHER, ACT, true>>(kSlabLds);
+        lds_limit<hy::moe_gemm256_kernel<GATHER, ACT, false>>(kSlabLds);
         if (turned) go(hy::moe_gemm256_kernel<GATHER, ACT, true>);
         else go(hy::moe_gemm256_kernel<GATHER, ACT, false>);
     } else {
@@ -602,12 +599,10 @@ static void moe_gemm(const uint16_t* x, int64_t rows, const uint16_t* w, uint16_
         };
         if constexpr (TM <= 64)
             if (large && items <= (TM == 32 ? 20 : 52) * E) {
-                static const hipError_t once = moe_lds(hy::moe_gemm_kernel<TM, GATHER, ACT, PLACE, true>, lds);
-                (void)once;
+                lds_limit<hy::moe_gemm_kernel<TM, GATHER, ACT, PLACE, true>>(lds);
                 return go(hy::moe_gemm_kernel<TM, GATHER, ACT, PLACE, true>);
             }
-        static const hipError_t once = moe_lds(hy::moe_gemm_kernel<TM, GATHER, ACT, PLACE, false>, lds);
-        (void)once;
+        lds_limit<hy::moe_gemm_kernel<TM, GATHER, ACT, PLACE, false>>(lds);
         go(hy::moe_gemm_kernel<TM, GATHER, ACT, PLACE, false>);
     }
 }

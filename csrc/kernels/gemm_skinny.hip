@@ -29,6 +29,7 @@
 #include "chronos_act.h"
 #include "chronos_gemm.h"
 #include "chronos_hip.h"
+#include "chronos_lds.h"
 
 namespace chronos {
 namespace {
@@ -510,9 +511,8 @@ namespace {
 template <int RT, int D, int NW, int MODE>
 void launch_join(const PPArgs& a, const JoinRows& j, hipStream_t st) {
     constexpr int UNITS = RT * 64, base = NW * (UNITS + UNITS / 16) * 16 + 16 * 4 + 16;
-    const auto kern = skinny_kernel<RT, 1, D, NW, MODE, false, JoinRows>;
-    static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, base + 2 * kJoinMost);
-    (void)set;
+    constexpr auto kern = skinny_kernel<RT, 1, D, NW, MODE, false, JoinRows>;
+    lds_limit<kern>(base + 2 * kJoinMost);
     kern<<<sk_pair(MODE) ? a.F / (8 * RT) : a.N / (16 * RT), 64 * NW, base + a.M * a.K * 2, st>>>(a, j);
 }
 }  // namespace
