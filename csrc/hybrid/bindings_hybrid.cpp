@@ -28,8 +28,8 @@ void launch_hy_act(void*, int64_t, int, bool, hipStream_t);
 void launch_hy_mlstm_scan(const void*, int, const float*, const int32_t*, const int32_t*, const int32_t*, float*, float*,
                           float*, float*, float*, int, int, int, int, int, float, int, int, bool, hipStream_t);
 int hy_chunk_segments(int, int, int, int, int, int);
-int64_t hy_delta_tiles_bytes(const void*, int, int, int, int, int, int, int, int, int, int);
-int64_t hy_gla_tiles_bytes(const void*, const void*, int, int, int, int, int, int, int, int, int, int);
+int64_t hy_delta_tiles_bytes(const void*, int, int, int, int, int, int, int, int, int, int, int64_t);
+int64_t hy_gla_tiles_bytes(const void*, const void*, int, int, int, int, int, int, int, int, int, int, int64_t);
 bool hy_chunk_scan_pays(int, int, int, int, int, int, int);
 bool hy_gla_scan_pays(int, int, int);
 int64_t hy_chunk_segment_floats(int, int, int, int, int);
@@ -935,8 +935,9 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> hy_delta_prep(const Tensor& y, const 
 Tensor hy_linear_scan(const Tensor& proj, int64_t q_off, int64_t k_off, int64_t v_off, const c10::optional<Tensor>& qscale,
                       const c10::optional<Tensor>& kscale, double q_mul, const Tensor& decay,
                       const c10::optional<Tensor>& beta, const Tensor& q_start, const Tensor& pos0, const Tensor& slots,
-                      Tensor& S, int64_t HK, int64_t H, int64_t D, int64_t Dv, const c10::optional<Tensor>& vscale, int64_t max_q) {
+                      Tensor& S, int64_t HK, int64_t H, int64_t D, int64_t Dv, const c10::optional<Tensor>& vscale, int64_t max_q, int64_t tiles_mb) {
     c10::hip::HIPGuardMasqueradingAsCUDA g(proj.device());
+    need(tiles_mb >= 0 && tiles_mb < (1LL << 31), "linear_scan: tiles_mb");
     need(is_act(proj) && proj.dim() == 2 && proj.is_contiguous(), "linear_scan: proj [T, C]");
     const int64_t T = proj.size(0), C = proj.size(1), B = slots.numel();
     need(HK >= 1 && H % HK == 0 && D >= 1 && Dv >= 1, "linear_scan: head counts");
@@ -959,12 +960,12 @@ Tensor hy_linear_scan(const Tensor& proj, int64_t q_off, int64_t k_off, int64_t 
     Tensor seg;
     if (segs > 1) seg = at::empty({chronos::hy_chunk_segment_floats((int)B, (int)H, (int)D, (int)Dv, segs)}, S.options());
     if (beta && !chd && !f32(proj)) {
-        const int64_t bytes = chronos::hy_delta_tiles_bytes(proj.data_ptr(), (int)C, (int)q_off, (int)k_off, (int)v_off, (int)T, (int)B, (int)H, (int)D, (int)Dv, mq);
+        const int64_t bytes = chronos::hy_delta_tiles_bytes(proj.data_ptr(), (int)C, (int)q_off, (int)k_off, (int)v_off, (int)T, (int)B, (int)H, (int)D, (int)Dv, mq, tiles_mb << 20);
         if (bytes > 0) seg = at::empty({bytes / 4}, S.options());
     }
     Tensor tiles;
     if (chd && !beta && !f32(proj)) {
-        const int64_t bytes = chronos::hy_gla_tiles_bytes(proj.data_ptr(), decay.data_ptr(), (int)C, (int)q_off, (int)k_off, (int)v_off, (int)T, (int)B, (int)H, (int)D, (int)Dv, mq);
+        const int64_t bytes = chronos::hy_gla_tiles_bytes(proj.data_ptr(), decay.data_ptr(), (int)C, (int)q_off, (int)k_off, (int)v_off, (int)T, (int)B, (int)H, (int)D, (int)Dv, mq, tiles_mb << 20);
         if (bytes > 0) tiles = at::empty({bytes / 4}, S.options());
     }
     const bool ok = chronos::launch_hy_linear_scan(
@@ -1355,7 +1356,7 @@ TORCH_LIBRARY_FRAGMENT(chronos, m) {
     m.def("hy_delta_prep(Tensor y, Tensor ab, Tensor a_log, int HK, int H, int D, float q_mul) -> (Tensor, Tensor, Tensor, Tensor)");
     m.def("hy_linear_scan(Tensor proj, int q_off, int k_off, int v_off, Tensor? qscale, Tensor? kscale, float q_mul, "
           "Tensor decay, Tensor? beta, Tensor q_start, Tensor pos0, Tensor slots, Tensor(a!) S, int HK, int H, int D, "
-          "int Dv, Tensor? vscale, int max_q=0) -> Tensor");
+          "int Dv, Tensor? vscale, int max_q=0, int tiles_mb=512) -> Tensor");
     m.def("hy_moe_route_topk(Tensor h, Tensor w, Tensor bias, int top) -> (Tensor, Tensor)");
     m.def("hy_add_rms_norm(Tensor y, Tensor(a!) x, Tensor? w_out, float eps, bool out_f32, Tensor? y2, Tensor? gate2, "
           "Tensor? w_y, bool emit) -> Tensor");

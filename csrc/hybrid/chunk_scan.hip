@@ -934,10 +934,10 @@ static void chunk_scan_run(const hy::ChunkScan& a, hipStream_t s) {
 }
 
 // Bytes of scratch for the delta rule's tiles, or 0: made between the steps, as where no sequence has two chunks, and of launches whose tiles would take more
-// than 512 MB (a prompt portion of 32768 tokens and 16 heads takes 270).
-int64_t hy_delta_tiles_bytes(const void* proj, int ldp, int q_off, int k_off, int v_off, int T, int B, int H, int D, int Dv, int longest) {
+// than `most` (512 MB: a prompt portion of 32768 tokens and 16 heads takes 270).
+int64_t hy_delta_tiles_bytes(const void* proj, int ldp, int q_off, int k_off, int v_off, int T, int B, int H, int D, int Dv, int longest, int64_t most) {
     const int64_t n = hy::delta_slots(T, B) * H * hy::kDeltaTiles;
-    return longest > hy::kCH && n <= (int64_t)512 << 20 && hy_chunk_scan_ok(proj, ldp, q_off, k_off, v_off, T, B, H, D, Dv, longest, hy::kScanDelta) ? n : 0;
+    return longest > hy::kCH && n <= most && hy_chunk_scan_ok(proj, ldp, q_off, k_off, v_off, T, B, H, D, Dv, longest, hy::kScanDelta) ? n : 0;
 }
 
 // Segments that a sequence's chunks are dealt to, here and in gla_scan.hip: launches that leave half of the CUs or more without a

@@ -794,11 +794,11 @@ static void gla_scan_run(const hy::GlaScan& a, hipStream_t s) {
 
 // Bytes of scratch for the chunks' tiles, or 0: made between the steps, as where no sequence has more than five chunks (the launch more costs 2.5 us: 21
 // sequences of 64 tokens, 4 heads of 128 x 256, 21.8 us so, 23.5 with tiles ahead, of 117 38.6 and 33.4), and of launches whose tiles would take more than
-// 512 MB (a prompt portion of 16384 tokens and 16 heads of 128 takes 470).
-int64_t hy_gla_tiles_bytes(const void* proj, const void* decay, int ldp, int q_off, int k_off, int v_off, int T, int B, int H, int D, int Dv, int longest) {
+// `most` (512 MB: a prompt portion of 16384 tokens and 16 heads of 128 takes 470).
+int64_t hy_gla_tiles_bytes(const void* proj, const void* decay, int ldp, int q_off, int k_off, int v_off, int T, int B, int H, int D, int Dv, int longest, int64_t most) {
     const int size = D == 32 ? hy::GlaTile<32>::SIZE : D == 64 ? hy::GlaTile<64>::SIZE : D == 128 ? hy::GlaTile<128>::SIZE : hy::GlaTile<256>::SIZE;
     const int64_t n = hy::gla_slots(T, B) * H * size;
-    return longest > 5 * hy::kGC && n <= (int64_t)512 << 20 && hy_gla_scan_ok(proj, decay, ldp, q_off, k_off, v_off, T, B, D, Dv, longest) ? n : 0;
+    return longest > 5 * hy::kGC && n <= most && hy_gla_scan_ok(proj, decay, ldp, q_off, k_off, v_off, T, B, D, Dv, longest) ? n : 0;
 }
 
 void launch_hy_gla_scan(const uint16_t* proj, int ldp, int q_off, int k_off, int v_off, const float* qscale, const float* kscale,

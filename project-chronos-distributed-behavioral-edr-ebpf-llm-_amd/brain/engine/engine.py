@@ -70,7 +70,8 @@ class EngineConfig:
     max_model_len: int = 4096      # prompt + generated tokens per sequence
     kv_blocks: int = 0             # 0 = size from HBM (kv_fraction of free memory, capped at what max_slots can use)
     kv_fraction: float = 0.9
-    reserve_gb: float = 12.0       # activations / graph pools / grammar table headroom
+    reserve_gb: float = 12.0       # activations / graph pools / grammar table headroom; scratch of a hybrid prompt step among them, up to
+                                   # 512 MB for a recurrence's tiles (ops.hybrid.linear_scan's tiles_mb) beside the step's activations
     max_prefill_tokens: int = 16384
     default_num_predict: int = 128
     max_out: int = 512             # hard cap on generated tokens per request

@@ -397,12 +397,13 @@ def low_rank_decay(a, w, b, inv_tau: float):
 
 
 def linear_scan(proj, q_off: int, k_off: int, v_off: int, qscale, kscale, q_mul: float, decay, beta, q_start, pos0,
-                slots, S, HK: int, H: int, D: int, Dv: int, vscale=None, max_q: int = 0):
+                slots, S, HK: int, H: int, D: int, Dv: int, vscale=None, max_q: int = 0, tiles_mb: int = 512):
     """``max_q``: the most tokens any sequence brings in this step (picks the kernel, any value gives the same
-    results up to rounding; 0 = unknown)."""
+    results up to rounding; 0 = unknown).  ``tiles_mb``: scratch that the call may take for its chunks' tiles, for as long as it runs (28 to 32 KB per chunk and head;
+    chunks whose tiles need more make them on their way)."""
     if _gpu(proj):
         return _k().hy_linear_scan(proj, q_off, k_off, v_off, qscale, kscale, q_mul, decay, beta, q_start, pos0, slots,
-                                   S, HK, H, D, Dv, vscale, max_q)
+                                   S, HK, H, D, Dv, vscale, max_q, tiles_mb)
     return ref.linear_scan(proj, q_off, k_off, v_off, qscale, kscale, q_mul, decay, beta, q_start, pos0, slots, S, HK,
                            H, D, Dv, vscale)
 
