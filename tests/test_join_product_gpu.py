@@ -37,22 +37,44 @@ def test_join_in_front(m, k, S):
         assert torch.equal(out, want) and (not nf or torch.equal(few, wfew))
 
 
+def _decode_rows(model, rows, ctx, vocab):
+    """A step of one token a row behind ctx cached ones, and pages that hold them."""
+    from chronos import ops
+    from chronos.models.llama import StepBatch
+
+    per = ctx // 16 + 1
+    i32 = dict(dtype=torch.int32, device=DEV)
+    pos, ar = torch.full((rows,), ctx, **i32), torch.arange(rows + 1, **i32)
+    ids = torch.randint(0, vocab, (rows,), generator=torch.Generator().manual_seed(6)).int().to(DEV)
+    sb = StepBatch(ids, pos, ar[:rows], torch.arange(1, 1 + rows * per, **i32).view(rows, per), ar, pos + 1, torch.arange(rows, device=DEV), None, rows, 1,
+                   ops.pick_nsplit(rows * model.hkv, ctx + 1), slots=ar[:rows].clone(), max_q=1)
+    cache, g = model.make_cache(1 + rows * per, 16, rows), torch.Generator(device=DEV).manual_seed(9)
+    for name in ("S", "n", "m", "lat", "kc", "vc", "kp", "vp", "hist"):
+        for t in getattr(cache, name).values():
+            t.normal_(0.0, 0.5, generator=g)
+    return sb, cache
+
+
 @pytest.mark.parametrize("rows", [1, 2, 3])
 def test_model_steps(rows, monkeypatch):
     """Decode steps of a design with all three readers, with the joins in their products and with every join a launch: the same to rounding."""
+    from chronos import ops
     from chronos.models import kalesun
     from chronos.models.hybrid import HybridDecoder
     from chronos.ops import hybrid as hops
     from chronos.utils import design_bench as db
-    from perf import cases
 
+    ops.load()
     hops.load()
-    case = dict(kind="hybrid_decode", design="kalesun", size="1k", rows=rows, ctx=70)
-    cfg = cases._hybrid_config(case)
-    dev = torch.device("cuda:0")
-    weights = cases._packed(cfg, kalesun, cases._hybrid_tensors(cfg, kalesun, dev, 3), dev)
-    model = HybridDecoder(cfg, weights, dev, 8192, torch.bfloat16)
-    assert db.KALESUN_SIZES["1k"]["width"] == 1024
+    ops.device_init()
+    size = db.KALESUN_SIZES["1k"]
+    design = db.kalesun_config(size)
+    for layer in design["layers"]:   # (a router's choice may turn on a last bit)
+        if layer["mlp"]["kind"] == "moe":
+            layer["mlp"] = dict(kind="dense", ff=size["ff"], limit=7.0)
+    cfg = kalesun.config_from_dict(design)
+    model = HybridDecoder(cfg, kalesun.pack_weights(cfg, kalesun.random_tensors(cfg, 3), DEV, torch.bfloat16), torch.device(DEV, 0), 8192, torch.bfloat16)
+    assert size["width"] == 1024
     got, taken = [], []
     product = hops.JoinedRows.product
 
@@ -65,10 +87,7 @@ def test_model_steps(rows, monkeypatch):
     for joined in (True, False):
         if not joined:
             monkeypatch.setattr(hops.JoinedRows, "serves", staticmethod(lambda y, x: False))
-        sb, nb = cases._decode_batch(cases._lens(case), cfg.vocab_size, model.hkv, dev, 5, True)
-        cache = model.make_cache(nb, 16, rows)
-        for t in cases._cache_tensors(cache):
-            t.normal_(0.0, 0.5, generator=torch.Generator(device=dev).manual_seed(9))
+        sb, cache = _decode_rows(model, rows, 70, cfg.vocab_size)
         with torch.no_grad():
             got.append(model.forward(sb, cache).double())
     assert (sum(taken) == 7) == (rows <= 2) and (len(taken) == 0) == (rows > 2)   # eight joins, the last has no reader
