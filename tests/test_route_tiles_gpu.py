@@ -36,3 +36,22 @@ def test_like_two_launches(T, d, N, top, form):
     assert float((~same).float().mean()) < 2e-3 and bool(same[7]) and torch.equal(idx[5], idx[3])
     assert float((wt[same] - wwant[same]).abs().max()) < 1e-5
     assert int(idx.min()) >= 0 and int(idx.max()) < N
+
+
+@pytest.mark.parametrize("T,d,N,top", [(513, 64, 1, 1), (4999, 1024, 16, 16), (700, 320, 17, 17), (8191, 2048, 32, 32)])
+def test_logits_are_the_projections(T, d, N, top):
+    """The choices follow from the logits that the projection by itself gives, ties and near ties included: not one differs."""
+    from chronos.ops import hybrid as hops
+
+    hops.load()
+    g = torch.Generator(device=DEV).manual_seed(T - N)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
+    h, w, b = rnd(T, d).bfloat16(), (rnd(N, d) * 0.02 * d ** -0.5).bfloat16(), rnd(N) * 0.02
+    if N > 4:
+        w[3], b[3] = w[1], b[1]
+    z = hops.rowdot(h, w, b)
+    val, want = torch.sort(z, dim=1, descending=True, stable=True)   # (equal ones: the lower row first)
+    idx, wt = hops.moe_route_topk(h, w, b, top)
+    assert torch.equal(idx.long(), want[:, :top])
+    # exponentials of float32 differences, N of them added up and divided by: N + 4 roundings of 2^-24 and expf's two
+    assert float((wt.double() - torch.softmax(val[:, :top].double(), 1)).abs().max()) < (N + 8) * 2.0 ** -24
