@@ -211,13 +211,14 @@ Tensor hy_layer_norm(const Tensor& x, const Tensor& w, double eps, bool out_f32,
 }
 
 // y as float32 slices [S, T, D] of a bfloat16 product: the output of a join, checked
-static Tensor join_slices(const Tensor& y, const Tensor& x, const Tensor& w, bool out_f32) {
+// (w: laid out again where it starts off the 16 bytes, which a join of y's rows takes as it lies)
+static Tensor join_slices(const Tensor& y, const Tensor& x, Tensor& w, bool out_f32) {
     flt(y, "join: float32 slices");
     need(!out_f32 && y.is_contiguous() && x.is_contiguous() && x.dim() == 2 && y.size(1) == x.size(0) && y.size(2) == x.size(1) && y.size(0) >= 1 && y.size(0) <= 64,
          "join: slices [S, T, D], 1 <= S <= 64, of a bfloat16 stream");
     need(x.size(1) % 8 == 0 && x.size(1) <= 8192 && w.numel() == x.size(1), "join: slices of rows of up to 8192 columns, a multiple of 8");
-    need(((reinterpret_cast<uintptr_t>(y.data_ptr()) | reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr())) & 15) == 0,
-         "join: slices need 16-byte aligned operands");
+    need(((reinterpret_cast<uintptr_t>(y.data_ptr()) | reinterpret_cast<uintptr_t>(x.data_ptr())) & 15) == 0, "join: slices need 16-byte aligned operands");
+    if ((reinterpret_cast<uintptr_t>(w.data_ptr()) & 15) != 0) w = w.clone();
     return at::empty_like(x, x.options().dtype(at::kBFloat16));
 }
 
@@ -226,8 +227,8 @@ Tensor hy_add_layer_norm(const Tensor& y, Tensor& x, const Tensor& w, double eps
     flt(x, "add_layer_norm: float32 residual");
     flt(w, "add_layer_norm: float32 weight");
     if (y.dim() == 3) {
-        Tensor h = join_slices(y, x, w, out_f32);
-        chronos::launch_hy_layer_norm_slices(y.data_ptr<float>(), (int)y.size(0), x.data_ptr<float>(), w.data_ptr<float>(),
+        Tensor wa = w, h = join_slices(y, x, wa, out_f32);
+        chronos::launch_hy_layer_norm_slices(y.data_ptr<float>(), (int)y.size(0), x.data_ptr<float>(), wa.data_ptr<float>(),
                                              reinterpret_cast<uint16_t*>(h.data_ptr()), (int)x.size(0), (int)x.size(1), (float)eps, stream());
         return h;
     }
@@ -565,8 +566,8 @@ Tensor hy_scale_add_rms_norm(const Tensor& y, Tensor& x, const Tensor& w, double
     flt(x, "scale_add_rms_norm: float32 residual");
     flt(w, "scale_add_rms_norm: float32 weight");
     if (y.dim() == 3) {
-        Tensor h = join_slices(y, x, w, out_f32);
-        chronos::launch_hy_rms_norm_slices(y.data_ptr<float>(), (int)y.size(0), x.data_ptr<float>(), w.data_ptr<float>(),
+        Tensor wa = w, h = join_slices(y, x, wa, out_f32);
+        chronos::launch_hy_rms_norm_slices(y.data_ptr<float>(), (int)y.size(0), x.data_ptr<float>(), wa.data_ptr<float>(),
                                            reinterpret_cast<uint16_t*>(h.data_ptr()), (int)x.size(0), (int)x.size(1), (float)alpha, (float)eps, stream());
         return h;
     }

@@ -749,12 +749,14 @@ std::tuple<Tensor, Tensor, Tensor> gemm_join(const Tensor& y, const Tensor& x, c
     CHK(N >= 1 && N % (16 * chronos::gemm_skinny_rt((int)cfg)) == 0, "gemm_join: N % (16 RT)");
     CHK(mode == 0 ? n0 >= 0 && nf >= 0 && n0 % 4 == 0 && n0 + nf <= N : nf == 0, "gemm_join: n0 % 4 == 0, n0 + nf <= N; with an activation no float32 outputs");
     CHK(((reinterpret_cast<uintptr_t>(x.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr()) | reinterpret_cast<uintptr_t>(y.data_ptr()) |
-          reinterpret_cast<uintptr_t>(wn.data_ptr()) | reinterpret_cast<uintptr_t>(h.data_ptr())) & 15) == 0, "gemm_join: alignment");
+          reinterpret_cast<uintptr_t>(h.data_ptr())) & 15) == 0, "gemm_join: alignment");
     if (bias.has_value()) {
         chk_gpu(*bias, "bias");
         CHK(bias->scalar_type() == at::kFloat && bias->numel() == nf, "gemm_join: bias [nf] f32");
     }
     c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+    // (a join by itself takes a weight that starts off the 16 bytes)
+    const Tensor wa = (reinterpret_cast<uintptr_t>(wn.data_ptr()) & 15) == 0 ? wn : wn.clone();
     Tensor xn = at::empty_like(x), yf, out = at::empty({M, mode != 0 ? N / 2 : nf > 0 ? n0 : N}, h.options());
     chronos::PPArgs a{};
     a.w = bf(w);
@@ -775,7 +777,7 @@ std::tuple<Tensor, Tensor, Tensor> gemm_join(const Tensor& y, const Tensor& x, c
         a.nf = (int)nf;
     }
     const chronos::JoinRows j{slices ? y.data_ptr<float>() : nullptr, slices ? nullptr : bf(y), slices ? (int)y.size(0) : 1, M * K,
-                              x.data_ptr<float>(), wn.data_ptr<float>(), xn.data_ptr<float>(), bfm(h), (float)alpha, (float)eps};
+                              x.data_ptr<float>(), wa.data_ptr<float>(), xn.data_ptr<float>(), bfm(h), (float)alpha, (float)eps};
     CHK(chronos::launch_gemm_join((int)cfg, (int)mode, a, j, cur_stream()), "gemm_join: launch");
     return {out, yf, xn};
 }

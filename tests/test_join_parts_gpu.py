@@ -41,3 +41,26 @@ def test_what_has_no_parts():
         assert hops.matmul_parts(x, w).dtype == BF
     with pytest.raises(RuntimeError):
         torch.ops.chronos.gemm_slices(x, w, 88, 1, False)     # (one slice of the slab walk is its plain product)
+
+
+@pytest.mark.parametrize("m,n,k", [(16, 1024, 2816), (200, 1024, 2816), (1, 1024, 1024)])
+def test_weight_off_the_16_bytes(m, n, k):
+    """A norm's weight that lies behind others in one buffer: joins took it with a product's rows, and do with its slices and in the product behind them."""
+    from chronos.ops import hybrid as hops
+
+    hops.load()
+    g = torch.Generator(device=DEV).manual_seed(m + n)
+    x, w = torch.randn(m, k, device=DEV, generator=g).to(BF), (torch.randn(n, k, device=DEV, generator=g) * k ** -0.5).to(BF)
+    flat = torch.randn(n + 1, device=DEV, generator=g)
+    x0, off, on = torch.randn(m, n, device=DEV, generator=g), flat[1:], flat[1:].clone()
+    assert off.data_ptr() % 16 == 4
+    y = hops.matmul_parts(x, w)
+    assert (y.dim() == 3) == (m > 1)
+    if m > 1:   # (slices: one kernel for both)
+        for join in (lambda r, v: hops.add_layer_norm(y, r, v, 1e-5, BF), lambda r, v: hops.scale_add_rms_norm(y, r, v, 1.7, 1e-6, BF)):
+            r1, r2 = x0.clone(), x0.clone()
+            assert torch.equal(join(r1, off), join(r2, on)) and torch.equal(r1, r2)
+    else:
+        got = [hops.JoinedRows(y, x0.clone(), v, 1.7, 1e-6) for v in (off, on)]
+        a, b = (j.product(w, 1)[0] for j in got)
+        assert torch.equal(a, b) and torch.equal(got[0].stream(), got[1].stream())
