@@ -230,7 +230,7 @@ __global__ void __launch_bounds__(128 * NWX, 1) gemm_lg_kernel(PPArgs a) {
     // TURN: every workgroup takes its stages round from one of its own, an XCD's neighbours one stage apart and the XCDs eight.  All from
     // the first, they read the same columns of rows that lie a power of two apart, lines that share few of the memory's and the
     // L2s' channels.  One x tile, weights cold, us, from the first stage / turned: 28672 x 4096, 64 rows 49.4 / 40.2 (128-row tiles) and 53.1 / 50.0, 16
-    // rows 41.3 / 37.8, 128 rows 55.6 / 49.1, 256 rows 72.6 / 66.3; 32768 x 4096, 64 rows 60.6 / 44.2, 32 rows 48.3 / 42.1; 2 to 8 rows 38.6 / 37.2; 14336 x 4096, 64 rows 29.0 /
+    // rows 41.3 / 37.8, 2 to 8 rows 38.6 / 37.2, 128 rows 55.6 / 49.1, 256 rows 72.6 / 66.3; 32768 x 4096, 64 rows 60.6 / 44.2, 32 rows 48.3 / 42.1; 14336 x 4096, 64 rows 29.0 /
     // 26.7; 128256 x 4096, 64 rows 191 / 177, 32 rows 186 / 184; 6144 x 4096 in two slices, 32 rows 13.1 / 12.0; level at 4096 x 14336 in four slices, and
     // at the vocabulary by 2 to 8 rows (156 / 154).  Not for callers that ask for sums in order (a.turn).
     // From K = 4096 on: level at 2048 (64 rows of 8192: 13.8 / 13.9), at 1024 slower (a decode step of one row, its weights in the memory-side cache: 156 / 161).  With more x tiles neighbours share their W rows and lose them from the L2 (1024 rows of 6144 x 4096: 52.1 / 54.1).
